@@ -39,6 +39,12 @@ int ls_model_create(const char* class_name, const char* weight_path, int max_bat
 int ls_model_destroy(ls_model* model);
 /* LSModel::Infer, model_base.h:69 */
 int ls_model_infer(ls_model* model);
+/* LSModel::Infer on token ids int32 [batch, seq_len] in host memory of any kind (the reference's
+ * pybind classes copy them themselves, pywrapper/wrapper.cc:116-156): sets input 0 to a buffer of
+ * the model's own and its shape.  host_out: NULL, or -- QuantBert -- pinned host memory (hipHostMalloc)
+ * for output 0, written as float32 (host_f16 != 0: fp16) by the time the call returns. */
+int ls_model_infer_host(ls_model* model, const int* ids, int batch, int seq_len, void* host_out,
+                        int host_f16);
 /* model_base.h:72-79 */
 int ls_model_set_input_ptr(ls_model* model, int index, void* input_ptr);
 int ls_model_set_input_shape(ls_model* model, int index, const int* shape, int ndim);

@@ -34,6 +34,9 @@ int quantize_transpose(const T* input, int8_t* output, int rows, int cols, float
 // stored uint8 (= code + 127) kernels -> int8 codes (optionally transposed) / T values
 // p[0..n) = value by a kernel (graph-capture safe, unlike hipMemsetAsync here)
 int fill_i32(int* p, int value, int n, hipStream_t s);
+// copies to or from pinned host memory made by a kernel: n 4-byte words / n fp16 values as floats
+int copy_words(const void* in, void* out, long n, hipStream_t s);
+int widen_f16(const __half* in, float* out, long n, hipStream_t s);
 int stored_u8_to_i8(const uint8_t* input, int8_t* output, int rows, int cols, bool transpose,
                     hipStream_t s);
 template <typename T>

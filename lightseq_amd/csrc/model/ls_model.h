@@ -63,6 +63,11 @@ class LSModel {
   }
   virtual DataType get_output_dtype(int index) { return slot_of(outputs_, index, "output").dtype; }
 
+  // Infer() on token ids [batch, seq_len] in host memory.  host_out: null, or pinned host memory
+  // that receives output 0 as float32 (host_f16: as fp16), for models whose output is fp16; it
+  // is written when the call returns.
+  virtual void InferHost(const int* ids, int batch, int seq_len, void* host_out, bool host_f16) = 0;
+
   virtual void benchmark_mode(bool is_benchmark) = 0;
 
   // Not in the reference: the HIP stream the model launches on (for event timing).

@@ -72,6 +72,13 @@ int ls_model_infer(ls_model* model) {
   return guarded([&] { model->impl->Infer(); });
 }
 
+int ls_model_infer_host(ls_model* model, const int* ids, int batch, int seq_len, void* host_out,
+                        int host_f16) {
+  NEED_MODEL(model);
+  if (!ids) return lsh::lsh_fail(LSH_ERR_INVALID, "ls_model_infer_host: null ids");
+  return guarded([&] { model->impl->InferHost(ids, batch, seq_len, host_out, host_f16 != 0); });
+}
+
 int ls_model_set_input_ptr(ls_model* model, int index, void* input_ptr) {
   NEED_MODEL(model);
   return guarded([&] { model->impl->set_input_ptr(index, input_ptr); });

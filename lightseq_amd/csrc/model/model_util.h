@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <cstring>
 #include <list>
 #include <map>
 #include <stdexcept>
@@ -68,6 +69,28 @@ class DeviceBuffer {
   }
   T* p_ = nullptr;
   size_t n_ = 0;
+};
+
+// Token ids that arrive in host memory: a pinned buffer of the model's largest input, from which a
+// kernel brings them to the GPU.  The buffer is free again once the model's stream has been
+// synchronised, which every call does before it returns.
+class HostIds {
+ public:
+  HostIds() = default;
+  HostIds(const HostIds&) = delete;
+  HostIds& operator=(const HostIds&) = delete;
+  ~HostIds() {
+    if (p_) (void)hipHostFree(p_);
+  }
+  // `ids` (n of them, n <= capacity) on their way to `dst`
+  void upload(const int* ids, size_t n, int* dst, size_t capacity, hipStream_t s) {
+    if (!p_) CHECK_GPU_ERROR(hipHostMalloc(reinterpret_cast<void**>(&p_), capacity * sizeof(int)));
+    std::memcpy(p_, ids, n * sizeof(int));
+    LSH_CALL(lsh::copy_words(p_, dst, (long)n, s));
+  }
+
+ private:
+  int* p_ = nullptr;
 };
 
 // A HIP stream of the default priority that is destroyed with its owner.

@@ -1,5 +1,7 @@
 #include "quant_bert.h"
 
+#include <algorithm>
+
 namespace lightseq {
 namespace hip {
 
@@ -33,18 +35,37 @@ QuantBert::~QuantBert() {
   encoder_.reset();  // before the buffers and the stream it uses (members, released after this)
 }
 
-void QuantBert::Infer() {
+void QuantBert::Infer() { infer(nullptr, false); }
+
+void QuantBert::infer(void* host_out, bool host_f16) {
   if (input_shapes_[0].size() != 2) throw std::runtime_error("token_ids must be 2-D");
   int batch_size = input_shapes_[0][0], seq_len = input_shapes_[0][1];
-  encoder_->run_one_infer(batch_size, seq_len);
-  CHECK_GPU_ERROR(hipStreamSynchronize(stream_));
-  if (encoder_->finish_infer()) {  // a route gave up and was switched off: once more without it
+  auto run = [&] {
     encoder_->run_one_infer(batch_size, seq_len);
+    if (host_out) {
+      const long n = (long)batch_size * seq_len * tw_._hidden_size;
+      if (host_f16) LSH_CALL(lsh::copy_words(encoder_->_p_d_output, host_out, n / 2, stream_));
+      else LSH_CALL(lsh::widen_f16(encoder_->_p_d_output, static_cast<float*>(host_out), n, stream_));
+    }
     CHECK_GPU_ERROR(hipStreamSynchronize(stream_));
+  };
+  run();
+  if (encoder_->finish_infer()) {  // a route gave up and was switched off: once more without it
+    run();
     encoder_->finish_infer();
   }
   encoder_->collect_profile();
   set_output_shape(0, {batch_size, seq_len, tw_._hidden_size});
+}
+
+void QuantBert::InferHost(const int* ids, int batch, int seq_len, void* host_out, bool host_f16) {
+  // more ids than the input holds: Infer() names the limit that was passed
+  const size_t n = (size_t)std::max(batch, 0) * (size_t)std::max(seq_len, 0);
+  if (ids && n > 0 && n <= d_input_.size())
+    h_ids_.upload(ids, n, d_input_.get(), d_input_.size(), stream_);
+  set_input_ptr(0, d_input_.get());
+  set_input_shape(0, {batch, seq_len});
+  infer(host_out, host_f16);
 }
 
 LSMODEL_REGISTER(QuantBert)

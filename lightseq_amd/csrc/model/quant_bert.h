@@ -17,6 +17,7 @@ class QuantBert : public LSModel {
   ~QuantBert();
 
   void Infer() override;
+  void InferHost(const int* ids, int batch, int seq_len, void* host_out, bool host_f16) override;
   void benchmark_mode(bool) override {}
   void* get_stream() override { return stream_.get(); }
 
@@ -24,8 +25,10 @@ class QuantBert : public LSModel {
   const QuantBertWeight& weight() const { return tw_; }
 
  private:
+  void infer(void* host_out, bool host_f16);
   // owners first: released after the encoder, also when the constructor throws half way
   StreamOwner stream_;
+  HostIds h_ids_;
   DeviceBuffer<int> d_input_, d_padding_mask_;
   DeviceBuffer<__half> d_encoder_output_;
   std::shared_ptr<QuantBertEncoder> encoder_;

@@ -1,5 +1,7 @@
 #include "quant_gpt.h"
 
+#include <algorithm>
+
 namespace lightseq {
 namespace hip {
 
@@ -47,6 +49,17 @@ void QuantGpt::Infer() {
   } else {
     throw std::runtime_error("Unsupported sampling_method");
   }
+}
+
+void QuantGpt::InferHost(const int* ids, int batch, int seq_len, void* host_out, bool) {
+  if (host_out) throw std::runtime_error("this model has no fp16 output to hand over");
+  // more ids than the input holds: Infer() names the limit that was passed
+  const size_t n = (size_t)std::max(batch, 0) * (size_t)std::max(seq_len, 0);
+  if (ids && n > 0 && n <= d_input_.size())
+    h_ids_.upload(ids, n, d_input_.get(), d_input_.size(), stream_);
+  set_input_ptr(0, d_input_.get());
+  set_input_shape(0, {batch, seq_len});
+  Infer();
 }
 
 LSMODEL_REGISTER(QuantGpt)

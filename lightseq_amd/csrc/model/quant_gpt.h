@@ -18,6 +18,7 @@ class QuantGpt : public LSModel {
   ~QuantGpt();
 
   void Infer() override;
+  void InferHost(const int* ids, int batch, int seq_len, void* host_out, bool host_f16) override;
   void benchmark_mode(bool is_benchmark) override { encoder_->benchmark_mode(is_benchmark); }
   void* get_stream() override { return stream_.get(); }
 
@@ -28,6 +29,7 @@ class QuantGpt : public LSModel {
   bool is_ppl() const { return tw_._sampling_method == "ppl"; }
   // owners first: released after the encoder, also when the constructor throws half way
   StreamOwner stream_;
+  HostIds h_ids_;
   DeviceBuffer<int> d_input_, d_sample_id;
   DeviceBuffer<float> d_ppl;
   std::shared_ptr<QuantGptEncoder> encoder_;

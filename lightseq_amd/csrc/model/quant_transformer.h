@@ -20,6 +20,7 @@ class QuantTransformer : public LSModel {
   ~QuantTransformer();
 
   void Infer() override;
+  void InferHost(const int* ids, int batch, int seq_len, void* host_out, bool host_f16) override;
   void benchmark_mode(bool is_benchmark) override;
   void* get_stream() override { return stream_.get(); }
 
@@ -34,6 +35,7 @@ class QuantTransformer : public LSModel {
   // owners first: the stream and the buffers outlive the encoder and decoder that use them,
   // and are released when the constructor throws half way (unsupported files are common)
   StreamOwner stream_;
+  HostIds h_ids_;
   DeviceBuffer<int> d_input_, d_padding_mask_, d_output_;
   DeviceBuffer<__half> d_encoder_output_;
   std::shared_ptr<QuantBertEncoder> encoder_;
