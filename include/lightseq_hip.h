@@ -438,6 +438,30 @@ int lsh_build_act_lut(int8_t* lut, const void* bias_f16, int n, float dequant_sc
                       float quant_scale, float clip_max, int act, lsh_stream_t stream);
 int lsh_gemm_i8_lut_i8o(const int8_t* A, const int8_t* W, int8_t* C, const int8_t* lut, int m,
                         int n, int k, float alpha, lsh_stream_t stream);
+/* Products on blocked operands: blocks of 16 rows x 64 bytes (1 KB) in the lane order of the
+ * 16x16x64 int8 matrix instruction, [rows / 16][row_bytes / 64], rows rounded up to 16 (the
+ * layout of lsh_tile_weight_16x64).  lsh_block_rows converts `rows` rows of `row_bytes` bytes
+ * (a multiple of 64) from row-major into it (back != 0: out of it); the padding rows become
+ * zeros.  A [m, k] and W [n, k] are blocked, k % 64 == 0, n % 4 == 0; C is row-major, but for the
+ * table form, whose int8 output is blocked (n % 64 == 0).  ksplit: as lsh_gemm_i8_i32o_splitk.
+ * The same numbers as the row-major products.  No counterpart in the reference. */
+int lsh_block_rows(const void* in, void* out, int rows, int row_bytes, int back, lsh_stream_t stream);
+int lsh_gemm_i8_blocked_i8o(const int8_t* A, const int8_t* W, int8_t* C, int m, int n, int k,
+                            float alpha, lsh_stream_t stream);
+int lsh_gemm_i8_blocked_i32o(const int8_t* A, const int8_t* W, int32_t* C, int m, int n, int k,
+                             int ksplit, lsh_stream_t stream);
+int lsh_gemm_i8_blocked_lut_i8o(const int8_t* A, const int8_t* W, int8_t* C, const int8_t* lut,
+                                int m, int n, int k, float alpha, lsh_stream_t stream);
+int lsh_gemm_i8_blocked_decself_qkv_i8o_f16(const int8_t* A, const int8_t* W, const void* qkv_bias,
+                                            int8_t* new_q, int8_t* new_k, int8_t* new_v,
+                                            int step_token_num, int hidden, int k, int head_num,
+                                            int max_step, int step_id, float alpha,
+                                            float dequant_scale, float quant_scale,
+                                            lsh_stream_t stream);
+int lsh_gemm_i8_blocked_encdec_q_f16(const int8_t* A, const int8_t* W, const void* q_bias,
+                                     void* new_q, int step_token_num, int hidden, int k,
+                                     int beam_size, int head_num, float alpha, float dequant_scale,
+                                     lsh_stream_t stream);
 /* The int32 product with K split into `ksplit` equal ranges computed by different workgroups
  * (for shapes whose tile count would leave compute units idle, e.g. the second FFN product):
  * range p writes the plane C + p * m * n, so C needs ksplit * m * n elements; the planes are

@@ -131,7 +131,24 @@ __global__ void __launch_bounds__(64 * NW, D <= 64 ? 2 : 1)
 encself_attn_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
                     const __half* __restrict__ v, const int* __restrict__ pad_mask,
                     __half* __restrict__ ctx, int8_t* __restrict__ ctx_q, float quant_scale, int S,
-                    int head_num, float alpha, float dq, int key_len) {
+                    int head_num, float alpha, float dq, int key_len,
+                    const int* __restrict__ seq) {
+  const int bh = blockIdx.y;
+  const int b = bh / head_num, head = bh % head_num;
+  // Packed rows (MODE 3 with an EncPack plan, ctx_q then a blocked matrix): the sequence is rows
+  // row0 .. row0 + S, whatever the padded length S0 is.  Everything else: rows b * S0 ..
+  const int S0 = S;
+  long row0 = (long)b * S;
+  if (MODE == kAttnEncI8 && seq != nullptr) {
+    row0 = seq[2 * b];
+    S = seq[2 * b + 1];
+    const int pad_row = seq[2 * (gridDim.y / head_num)];
+    // the context of the padding's row, once per head
+    if (b == 0 && blockIdx.x == 0 && pad_row >= 0 && threadIdx.x < D / 16)
+      *reinterpret_cast<uint4*>(ctx_q + blocked_offset(pad_row, head * D + threadIdx.x * 16, head_num * D)) =
+          make_uint4(0, 0, 0, 0);
+    if ((int)blockIdx.x * (32 * NW) >= S) return;
+  }
   // number of keys: the layer mode (MODE 2) may attend over another sequence (cross
   // attention, cached decoding); everywhere else keys and queries are the same S positions
   const int Sk = MODE == kAttnLayer ? key_len : S;
@@ -147,8 +164,6 @@ encself_attn_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, g = lane >> 5;
-  const int bh = blockIdx.y;
-  const int b = bh / head_num, head = bh % head_num;
   constexpr int NT = 64 * NW;  // threads; 32 queries per wavefront
   const int qi = blockIdx.x * (32 * NW) + wave * 32 + l32;
   const _Float16* qb = reinterpret_cast<const _Float16*>(q) + (long)bh * S * D;
@@ -157,7 +172,7 @@ encself_attn_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
 
   // MODE 3: int8 codes [tokens, 3 * hidden] and the fp16 bias [3 * hidden]
   const int hidden3 = 3 * head_num * D;
-  const int8_t* codes = reinterpret_cast<const int8_t*>(q) + (long)b * S * hidden3 + head * D;
+  const int8_t* codes = reinterpret_cast<const int8_t*>(q) + row0 * hidden3 + head * D;
   const _Float16* bias = reinterpret_cast<const _Float16*>(k) + head * D;
 
   v8h qreg[D / 16];
@@ -193,8 +208,8 @@ encself_attn_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
         wv[i][r] = *reinterpret_cast<const uint2*>(codes + (long)min(kg * 4 + r, S - 1) * hidden3 +
                                                    2 * hid + ch * 8);
     }
-    const int pm0 = pad_mask[(long)b * S + min(lane, S - 1)];
-    const int pm1 = pad_mask[(long)b * S + min(lane + 64, S - 1)];
+    const int pm0 = pad_mask[(long)b * S0 + min(lane, S - 1)];
+    const int pm1 = pad_mask[(long)b * S0 + min(lane + 64, S - 1)];
     __builtin_amdgcn_sched_barrier(0);
     // queries: lane half g converts chunk kp * 32 + g * 16 .. + 16, then the halves swap their
     // second part (see the general path below)
@@ -242,10 +257,11 @@ encself_attn_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
     const uint64_t pad_q = __ballot(wave < 2 ? padk0 : padk1);
     const bool q_pad = qi >= S || ((pad_q >> ((wave & 1) * 32 + l32)) & 1) != 0;
     __syncthreads();
-    const long tok = (long)b * S + qi;
+    const long tok = row0 + qi;
     attend_block128<D>(Ks, Vt, qreg, padk0, padk1, q_pad, qi < S, alpha, quant_scale,
                        ctx ? ctx + ((long)bh * S + qi) * D : nullptr,
-                       ctx_q ? ctx_q + tok * (head_num * D) + head * D : nullptr, l32, g);
+                       ctx_q ? ctx_q + code_offset(tok, head * D, head_num * D, seq != nullptr) : nullptr,
+                       l32, g, seq != nullptr ? 256 : 16);
     return;
   } else if (MODE == kAttnEncI8) {
 #pragma unroll
@@ -279,7 +295,7 @@ encself_attn_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
   }
   const bool q_pad = qi >= S || (MODE == kAttnLayer ? false
                                  : GPT              ? qi >= pad_mask[b]
-                                                    : pad_mask[(long)b * S + qi] != 0);
+                                                    : pad_mask[(long)b * S0 + qi] != 0);
 
   float m = kFloatInfNeg, sum = 0.f;
   v16f sc[4];
@@ -374,7 +390,7 @@ encself_attn_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
           } else if (GPT) {
             msk[tid] = (key0 + tid < S) ? 0 : 1;
           } else {
-            msk[tid] = (key0 + tid < S) ? pad_mask[(long)b * S + key0 + tid] : 1;
+            msk[tid] = (key0 + tid < S) ? pad_mask[(long)b * S0 + key0 + tid] : 1;
           }
         }
         __syncthreads();
@@ -490,7 +506,7 @@ encself_attn_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
   }
 
   if (qi >= S) return;
-  const long tok = (long)b * S + qi;
+  const long tok = row0 + qi;
   const int hidden = head_num * D;
 #pragma unroll
   for (int db = 0; db < D / 32; ++db) {
@@ -512,7 +528,8 @@ encself_attn_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
       if (ctx_q != nullptr) {
         // a padded query gives zeros, whose code is 0
         const uint32_t w4 = float2int8_pack4(o[0], o[1], o[2], o[3], quant_scale);
-        *reinterpret_cast<uint32_t*>(ctx_q + tok * hidden + head * D + dd) = q_pad ? 0u : w4;
+        *reinterpret_cast<uint32_t*>(ctx_q + code_offset(tok, head * D + dd, hidden, seq != nullptr)) =
+            q_pad ? 0u : w4;
       }
     }
   }
@@ -524,17 +541,18 @@ template <int MODE>
 static bool launch_attn(int dim_per_head, int seq_len, int batch_heads, hipStream_t s,
                         const __half* q, const __half* k, const __half* v, const int* pad_mask,
                         __half* ctx, int8_t* ctx_q, float quant_scale, int head_num, float alpha,
-                        float dq, int key_len = -1) {
+                        float dq, int key_len = -1, const int* seq = nullptr) {
   if (key_len < 0) key_len = seq_len;  // self attention: as many keys as queries
 #define LSH_ATTN(DD, NWV)                                                                      \
   if (key_len <= 128)                                                                          \
     encself_attn_kernel<DD, MODE, NWV, true>                                                   \
         <<<dim3((seq_len + 32 * NWV - 1) / (32 * NWV), batch_heads), 64 * NWV, 0, s>>>(        \
-            q, k, v, pad_mask, ctx, ctx_q, quant_scale, seq_len, head_num, alpha, dq, key_len); \
+            q, k, v, pad_mask, ctx, ctx_q, quant_scale, seq_len, head_num, alpha, dq, key_len,  \
+            seq);                                                                              \
   else                                                                                         \
     encself_attn_kernel<DD, MODE, NWV, false>                                                  \
       <<<dim3((seq_len + 32 * NWV - 1) / (32 * NWV), batch_heads), 64 * NWV, 0, s>>>(          \
-          q, k, v, pad_mask, ctx, ctx_q, quant_scale, seq_len, head_num, alpha, dq, key_len)
+          q, k, v, pad_mask, ctx, ctx_q, quant_scale, seq_len, head_num, alpha, dq, key_len, seq)
   const bool wide = seq_len > 64;
   switch (dim_per_head) {
     case 32:
@@ -590,6 +608,25 @@ int encself_attention_i8qkv(const int8_t* qkv, const __half* qkv_bias, float deq
     return lsh_fail(LSH_ERR_UNSUPPORTED,
                         "encself_attention_i8qkv: dim_per_head must be 32, 64 or 128");
   return lsh_check_launch("encself_attn_kernel<i8 qkv>");
+}
+
+int encself_attention_packed(const int8_t* qkv, const __half* qkv_bias, float dequant_scale,
+                             const int* pad_mask, int8_t* ctx_q, float quant_scale, int batch,
+                             int seq_len, int head_num, int dim_per_head, hipStream_t s,
+                             const EncPack& pack) {
+  if (batch <= 0 || seq_len <= 0 || head_num <= 0 || !qkv || !qkv_bias || !pad_mask || !ctx_q ||
+      !pack.seq || (head_num * dim_per_head) % 64 != 0)
+    return lsh_fail(LSH_ERR_INVALID, "encself_attention_packed: bad arguments");
+  if (seq_len > 1024)
+    return lsh_fail(LSH_ERR_UNSUPPORTED, "encself_attention_packed: seq_len > 1024");
+  const float alpha = __half2float(__float2half_rn(sqrtf(1.f / (float)dim_per_head)));
+  if (!launch_attn<kAttnEncI8>(dim_per_head, seq_len, batch * head_num, s,
+                               reinterpret_cast<const __half*>(qkv), qkv_bias, nullptr, pad_mask,
+                               nullptr, ctx_q, quant_scale, head_num, alpha, dequant_scale, -1,
+                               pack.seq))
+    return lsh_fail(LSH_ERR_UNSUPPORTED,
+                    "encself_attention_packed: dim_per_head must be 32, 64 or 128");
+  return lsh_check_launch("encself_attn_kernel<packed>");
 }
 
 int gpt_prefill_attention_f16(const __half* q_codes, const __half* k_codes, const __half* v,

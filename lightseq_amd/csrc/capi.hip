@@ -468,6 +468,38 @@ int lsh_gemm_i8_lut_i8o(const int8_t* A, const int8_t* W, int8_t* C, const int8_
                         int n, int k, float alpha, lsh_stream_t stream) {
   return gemm_i8_lut_i8o(A, W, C, lut, m, n, k, alpha, HS(stream));
 }
+int lsh_block_rows(const void* in, void* out, int rows, int row_bytes, int back, lsh_stream_t stream) {
+  return block_rows(in, out, rows, row_bytes, back != 0, HS(stream));
+}
+int lsh_gemm_i8_blocked_i8o(const int8_t* A, const int8_t* W, int8_t* C, int m, int n, int k,
+                            float alpha, lsh_stream_t stream) {
+  return gemm_blk_i8o(A, W, C, m, n, k, alpha, HS(stream));
+}
+int lsh_gemm_i8_blocked_i32o(const int8_t* A, const int8_t* W, int32_t* C, int m, int n, int k,
+                             int ksplit, lsh_stream_t stream) {
+  return gemm_blk_i32o(A, W, C, m, n, k, ksplit, HS(stream));
+}
+int lsh_gemm_i8_blocked_lut_i8o(const int8_t* A, const int8_t* W, int8_t* C, const int8_t* lut,
+                                int m, int n, int k, float alpha, lsh_stream_t stream) {
+  return gemm_blk_lut(A, W, C, lut, m, n, k, alpha, HS(stream));
+}
+int lsh_gemm_i8_blocked_decself_qkv_i8o_f16(const int8_t* A, const int8_t* W, const void* qkv_bias,
+                                            int8_t* new_q, int8_t* new_k, int8_t* new_v,
+                                            int step_token_num, int hidden, int k, int head_num,
+                                            int max_step, int step_id, float alpha,
+                                            float dequant_scale, float quant_scale,
+                                            lsh_stream_t stream) {
+  return gemm_blk_decself_qkv(A, W, H(qkv_bias), new_q, new_k, new_v, step_token_num, hidden, k,
+                              head_num, max_step, step_id, alpha, dequant_scale, quant_scale,
+                              HS(stream));
+}
+int lsh_gemm_i8_blocked_encdec_q_f16(const int8_t* A, const int8_t* W, const void* q_bias,
+                                     void* new_q, int step_token_num, int hidden, int k,
+                                     int beam_size, int head_num, float alpha, float dequant_scale,
+                                     lsh_stream_t stream) {
+  return gemm_blk_encdec_q(A, W, H(q_bias), static_cast<__half*>(new_q), step_token_num, hidden, k, beam_size, head_num,
+                           alpha, dequant_scale, HS(stream));
+}
 int lsh_gemm_i8_i32o_splitk(const int8_t* A, const int8_t* W, int32_t* C, int m, int n, int k,
                             int ksplit, int* used, lsh_stream_t stream) {
   return gemm_i8_i32o_splitk(A, W, C, m, n, k, ksplit, used, HS(stream));

@@ -1,0 +1,265 @@
+// int8 and fp16 products on blocked operands (tile_common.h names the layout): what the models and
+// layers run.  Weights are blocked once at load; activations are written blocked by the kernel
+// that produces them (layer norm, attention, the table epilogue), so no product waits for a
+// rearrangement.
+//
+// Two kernels: gemm_kw_kernel (gemm_kw.h) for outputs of up to a few rounds of small tiles, and
+// the LDS tile loop of gemm_tile.h for the large ones.  The dispatch estimates both.
+#include "gemm_dec_epi.h"
+#include "gemm_kw.h"
+#include "ls_launch.h"
+
+#include <hip/hip_ext.h>
+
+#include <algorithm>
+#include <mutex>
+
+namespace lsh {
+
+// one output tile per workgroup, both operands blocked
+template <typename Epi, int WGM, int WGN, int MB, int NB, int NST>
+__global__ void __launch_bounds__(64 * WGM * WGN)
+gemm_blk_tile_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, Epi epi, int M,
+                     int N, int K, int tiles_m, int tiles_n) {
+  extern __shared__ __align__(16) int8_t smem[];
+  asm volatile("" : "+s"(tiles_m) : "s"(A), "s"(W));
+  constexpr int TM = WGM * MB * 32;
+  int tm, tn;
+  tile_of(blockIdx.x, tiles_m * tiles_n, tiles_m, tiles_n, tm, tn);
+  tile_gemm<Epi, WGM, WGN, MB, NB, NST, false, true>(A, W, epi, tm * TM, M, N, K, tn, smem);
+}
+
+namespace {
+
+template <auto Kern>
+int raise_lds(size_t smem) {
+  static std::mutex mu;
+  static unsigned long long done = 0;  // bit per device index
+  int dev = 0;
+  if (int rc = lsh_check_hip(hipGetDevice(&dev), "hipGetDevice(gemm_blk)")) return rc;
+  if (dev < 0 || dev >= 64) return lsh_fail(LSH_ERR_UNSUPPORTED, "blocked gemm: device index out of range");
+  std::lock_guard<std::mutex> lock(mu);
+  if (!(done >> dev & 1ull)) {
+    if (smem > 64 * 1024)
+      if (int rc = lsh_check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(Kern),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem),
+                                 "hipFuncSetAttribute(gemm_blk)"))
+        return rc;
+    done |= 1ull << dev;
+  }
+  return LSH_OK;
+}
+
+template <auto Kern, typename... Args>
+int launch_blk(dim3 grid, int threads, size_t smem, hipStream_t s, Args... args) {
+  if (int rc = raise_lds<Kern>(smem)) return rc;
+  hipEvent_t e0, e1;
+  if (gemm_take_timing_events(&e0, &e1))
+    hipExtLaunchKernelGGL(Kern, grid, dim3(threads), (unsigned)smem, s, e0, e1, 0, args...);
+  else
+    Kern<<<grid, threads, smem, s>>>(args...);
+  return lsh_check_launch("blocked gemm");
+}
+
+template <typename Tr, typename Epi, int MB, int NB>
+int launch_kw(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K, int ksplit,
+              hipStream_t s) {
+  const int tm = (M + 16 * MB - 1) / (16 * MB), tn = (N + 16 * NB - 1) / (16 * NB);
+  const dim3 grid(tm * tn, ksplit);
+  constexpr size_t smem = kw_lds_bytes<Epi, MB, NB>();
+  const int slices = K / 64 / ksplit;
+  if (slices % 16 == 0)
+    return launch_blk<gemm_kw_kernel<Tr, Epi, MB, NB, 4>>(grid, 256, smem, s, A, W, epi, M, N, K, slices, tm, tn);
+  if (slices % 12 == 0)
+    return launch_blk<gemm_kw_kernel<Tr, Epi, MB, NB, 3>>(grid, 256, smem, s, A, W, epi, M, N, K, slices, tm, tn);
+  return launch_blk<gemm_kw_kernel<Tr, Epi, MB, NB, 1>>(grid, 256, smem, s, A, W, epi, M, N, K, slices, tm, tn);
+}
+
+// The LDS tile kernel: 8 wavefronts for the tall tiles, 4 for 128 x 128 and 128 x 64 (two or three
+// workgroups then share a compute unit and one's epilogue runs under the other's K loop).
+constexpr TileCost kLdsCost[] = {{128, 64, 2.5f, 2.45f, 0.2f, 2.6f, 0.6f},
+                                 {128, 128, 2.9f, 3.6f, 0.6f, 4.9f, 0.9f},
+                                 {256, 128, 3.1f, 5.4f, 1.5f, 9.0f, 1.3f},
+                                 {256, 192, 3.6f, 7.1f, 3.0f, 9.5f, 1.7f},
+                                 {256, 256, 4.1f, 9.2f, 4.0f, 12.0f, 2.4f}};
+struct LdsTile {
+  int tm = 0, tn = 0;
+  float us = 0;
+};
+LdsTile choose_lds_tile(int M, int N, int K, int cus, bool table) {
+  LdsTile best;
+  if (K % kBK != 0 || K / kBK < 3 || N % 16 != 0) return best;
+  for (const auto& c : kLdsCost) {
+    const float us = tile_us(c, M, N, K, 1, cus, table);
+    if (best.tm == 0 || us < best.us) best = LdsTile{c.tm, c.tn, us};
+  }
+  return best;
+}
+
+template <typename Tr, typename Epi, bool TILES>
+int dispatch_blk(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K, hipStream_t s,
+                 int ksplit = 1) {
+  if (M <= 0 || N <= 0 || K <= 0 || !A || !W)
+    return lsh_fail(LSH_ERR_INVALID, "blocked gemm: bad arguments");
+  if (K % 64 != 0 || N % 4 != 0)
+    return lsh_fail(LSH_ERR_UNSUPPORTED, "blocked gemm: needs K bytes % 64 == 0 and N % 4 == 0");
+  if (((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W)) & 15u) != 0 || !epi.aligned())
+    return lsh_fail(LSH_ERR_INVALID, "blocked gemm: operands must be 16-byte aligned");
+  const unsigned long long lim = 0xffffffffull;
+  if ((unsigned long long)(M + 15) / 16 * 16 * K >= lim || (unsigned long long)(N + 15) / 16 * 16 * K >= lim ||
+      (long)((M + 15) / 16) * ((N + 15) / 16) >= (1L << 24))
+    return lsh_fail(LSH_ERR_UNSUPPORTED, "blocked gemm: operand or output too large");
+  if (ksplit < 1 || K % (64 * ksplit) != 0)
+    return lsh_fail(LSH_ERR_INVALID, "blocked gemm: K does not split into whole 64-byte slices");
+  const int cus = cu_count();
+  const KwTile kw = kw_choose_tile(M, N, K / ksplit, ksplit, cus, Epi::kTable);
+  if constexpr (TILES) {
+    if (ksplit == 1) {
+      const LdsTile t = choose_lds_tile(M, N, K, cus, Epi::kTable);
+      if (t.tm != 0 && t.us < kw.us) {
+        const int tm = (M + t.tm - 1) / t.tm, tn = (N + t.tn - 1) / t.tn;
+        const dim3 grid(tm * tn);
+        if (t.tn == 256)
+          return launch_blk<gemm_blk_tile_kernel<Epi, 2, 4, 4, 2, 2>>(grid, 512, 2 * 512 * kBK, s, A, W, epi, M, N,
+                                                                      K, tm, tn);
+        if (t.tn == 192)
+          return launch_blk<gemm_blk_tile_kernel<Epi, 4, 2, 2, 3, 2>>(grid, 512, 2 * 448 * kBK, s, A, W, epi, M, N,
+                                                                      K, tm, tn);
+        if (t.tm == 256)
+          return launch_blk<gemm_blk_tile_kernel<Epi, 4, 2, 2, 2, 3>>(grid, 512, 3 * 384 * kBK, s, A, W, epi, M, N,
+                                                                      K, tm, tn);
+        if (t.tn == 128)
+          return launch_blk<gemm_blk_tile_kernel<Epi, 2, 2, 2, 2, 2>>(grid, 256, 2 * 256 * kBK, s, A, W, epi, M, N,
+                                                                      K, tm, tn);
+        // long K loops: a third stage instead of a third workgroup per compute unit
+        if (K >= 2048)
+          return launch_blk<gemm_blk_tile_kernel<Epi, 4, 1, 1, 2, 3>>(grid, 256, 3 * 192 * kBK, s, A, W, epi, M, N,
+                                                                      K, tm, tn);
+        return launch_blk<gemm_blk_tile_kernel<Epi, 4, 1, 1, 2, 2>>(grid, 256, 2 * 192 * kBK, s, A, W, epi, M, N, K,
+                                                                    tm, tn);
+      }
+    }
+  }
+  if (kw.mb == 1) return launch_kw<Tr, Epi, 1, 1>(A, W, epi, M, N, K, ksplit, s);
+  if (kw.mb == 2) return launch_kw<Tr, Epi, 2, 2>(A, W, epi, M, N, K, ksplit, s);
+  if (kw.nb == 2) return launch_kw<Tr, Epi, 4, 2>(A, W, epi, M, N, K, ksplit, s);
+  return launch_kw<Tr, Epi, 4, 4>(A, W, epi, M, N, K, ksplit, s);
+}
+
+}  // namespace
+
+const char* gemm_blk_kernel_name(int M, int N, int K, bool table) {
+  const LdsTile t = choose_lds_tile(M, N, K, cu_count(), table);
+  return t.tm != 0 && t.us < kw_choose_tile(M, N, K, 1, cu_count(), table).us ? "gemm_blk_tile_kernel"
+                                                                              : "gemm_kw_kernel";
+}
+
+int gemm_blk_i8o(const int8_t* A, const int8_t* W, int8_t* C, int M, int N, int K, float alpha,
+                 hipStream_t s) {
+  return dispatch_blk<KwI8, EpiI8, true>(A, W, EpiI8{C, alpha}, M, N, K, s);
+}
+
+int gemm_blk_i32o(const int8_t* A, const int8_t* W, int32_t* C, int M, int N, int K, int ksplit,
+                  hipStream_t s) {
+  return dispatch_blk<KwI8, EpiI32, true>(A, W, EpiI32{C}, M, N, K, s, ksplit);
+}
+
+// Range of K per workgroup for the few rows of a generation step: as many int32 planes (summed by
+// the layer norm that reads them) as make the launch one round of the chip, four at most -- the
+// same rule as for row-major operands.
+int gemm_blk_preferred_ksplit(int M, int N, int K) {
+  int best = 1;
+  float best_us = kw_choose_tile(M, N, K, 1, cu_count(), false).us;
+  for (int ks = 2; ks <= 4; ks *= 2) {
+    if (M > 64 || K % (1024 * ks) != 0) break;
+    // a plane more for the layer norm to fetch: 0.2 us
+    const float us = kw_choose_tile(M, N, K / ks, ks, cu_count(), false).us + 0.2f * ks;
+    if (us < best_us) {
+      best = ks;
+      best_us = us;
+    }
+  }
+  return best;
+}
+
+int gemm_blk_lut(const int8_t* A, const int8_t* W, int8_t* C, const int8_t* lut, int M, int N, int K,
+                 float alpha, hipStream_t s) {
+  if (!lut) return lsh_fail(LSH_ERR_INVALID, "blocked gemm (table epilogue): null table");
+  if (N % 64 != 0)
+    return lsh_fail(LSH_ERR_UNSUPPORTED, "blocked gemm (table epilogue): the output needs N % 64 == 0");
+  return dispatch_blk<KwI8, EpiLutBlk, true>(A, W, EpiLutBlk{C, lut, alpha}, M, N, K, s);
+}
+
+int gemm_blk_decself_qkv(const int8_t* A, const int8_t* W, const __half* qkv_bias, int8_t* new_q,
+                         int8_t* new_k, int8_t* new_v, int step_token_num, int hidden, int K,
+                         int head_num, int max_step, int step_id, float alpha, float dequant_scale,
+                         float quant_scale, hipStream_t s) {
+  if (!qkv_bias || !new_q || !new_k || !new_v || head_num <= 0 || hidden <= 0 ||
+      hidden % head_num != 0 || max_step <= 0)
+    return lsh_fail(LSH_ERR_INVALID, "blocked gemm (decoder qkv): bad arguments");
+  if (step_id < 0 || step_id >= max_step)
+    return lsh_fail(LSH_ERR_INVALID, "blocked gemm (decoder qkv): step_id outside the cache");
+  const int d = hidden / head_num;
+  if (d % 4 != 0 || hidden >= (1 << 22) || (long)hidden * max_step >= (1L << 31))
+    return lsh_fail(LSH_ERR_UNSUPPORTED, "blocked gemm (decoder qkv): needs dim_per_head % 4 == 0");
+  return dispatch_blk<KwI8, EpiDecQkvI8, false>(
+      A, W,
+      EpiDecQkvI8{new_q, new_k, new_v, qkv_bias, alpha, dequant_scale, quant_scale, hidden, head_num,
+                  d, max_step, step_id, 1.0f / (float)hidden, 1.0f / (float)d},
+      step_token_num, 3 * hidden, K, s);
+}
+
+int gemm_blk_encdec_q(const int8_t* A, const int8_t* W, const __half* q_bias, __half* new_q,
+                      int step_token_num, int hidden, int K, int beam_size, int head_num, float alpha,
+                      float dequant_scale, hipStream_t s) {
+  if (!q_bias || !new_q || head_num <= 0 || hidden <= 0 || hidden % head_num != 0 ||
+      beam_size <= 0 || step_token_num <= 0 || step_token_num % beam_size != 0)
+    return lsh_fail(LSH_ERR_INVALID, "blocked gemm (cross-attention q): bad arguments");
+  const int d = hidden / head_num;
+  if (d % 4 != 0 || step_token_num >= (1 << 22))
+    return lsh_fail(LSH_ERR_UNSUPPORTED, "blocked gemm (cross-attention q): needs dim_per_head % 4 == 0");
+  return dispatch_blk<KwI8, EpiEncdecQF16, false>(
+      A, W,
+      EpiEncdecQF16{new_q, q_bias, alpha, dequant_scale, beam_size, head_num, d,
+                    1.0f / (float)beam_size, 1.0f / (float)d},
+      step_token_num, hidden, K, s);
+}
+
+// [rows, K bytes] row-major -> blocked (rows beyond the matrix: zeros), or back.  A thread moves
+// 16 bytes.
+template <bool BACK>
+__global__ void __launch_bounds__(256)
+block_rows_kernel(const int8_t* __restrict__ in, int8_t* __restrict__ out, long chunks, int rows, int K) {
+  const long chunk = (long)blockIdx.x * 256 + threadIdx.x;
+  if (chunk >= chunks) return;
+  const int lane = (int)(chunk & 63);
+  const long blk = chunk >> 6;
+  const int ks = (int)(blk % (K / 64));
+  const long row = blk / (K / 64) * 16 + (lane & 15);
+  const int k = ks * 64 + (lane >> 4) * 16;
+  if (BACK) {
+    if (row < rows)
+      *reinterpret_cast<v4i*>(out + row * K + k) = *reinterpret_cast<const v4i*>(in + chunk * 16);
+  } else {
+    v4i v = (v4i)0;
+    if (row < rows) v = *reinterpret_cast<const v4i*>(in + row * K + k);
+    *reinterpret_cast<v4i*>(out + chunk * 16) = v;
+  }
+}
+
+int block_rows(const void* in, void* out, int rows, int row_bytes, bool back, hipStream_t s) {
+  if (!in || !out || in == out || rows <= 0 || row_bytes <= 0 || row_bytes % 64 != 0 ||
+      ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15u) != 0)
+    return lsh_fail(LSH_ERR_INVALID, "block_rows: needs row bytes % 64 == 0 and aligned pointers");
+  const long chunks = (long)((rows + 15) / 16) * row_bytes;
+  const unsigned grid = (unsigned)((chunks + 255) / 256);
+  if (back)
+    block_rows_kernel<true><<<grid, 256, 0, s>>>(static_cast<const int8_t*>(in), static_cast<int8_t*>(out),
+                                                 chunks, rows, row_bytes);
+  else
+    block_rows_kernel<false><<<grid, 256, 0, s>>>(static_cast<const int8_t*>(in), static_cast<int8_t*>(out),
+                                                  chunks, rows, row_bytes);
+  return lsh_check_launch("block_rows_kernel");
+}
+
+}  // namespace lsh

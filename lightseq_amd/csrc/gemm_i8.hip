@@ -37,6 +37,7 @@
 #include "ls_device.h"
 #include "ls_launch.h"
 #include "tile_common.h"
+#include "gemm_dec_epi.h"
 #include "gemm_tile.h"
 
 #include <hip/hip_ext.h>
@@ -50,166 +51,6 @@
 namespace lsh {
 
 constexpr int kBM = 128, kBN = 128;
-
-// n / d for 0 <= n < 2^24, d > 0, with inv = 1.0f / d from the host: the float product is
-// within one of the quotient, the remainder decides.  A handful of instructions where the
-// integer division is about forty -- in kernels whose length is their instruction count.
-__device__ __forceinline__ int div_by(int n, int d, float inv) {
-  int q = (int)((float)n * inv);
-  const int r = n - q * d;
-  if (r >= d) ++q;
-  if (r < 0) --q;
-  return q;
-}
-
-// Decode-step QKV product followed by ker_arrange_decself_qkv_i8I_i8O
-// (inference/kernels/transformerKernels_int8.cc.cu:1432-1513; call sites
-// model/quant_decoder.cc.cu:660-674, model/quant_gpt_encoder.cc.cu:640-653): the int8 code
-// of the product is dequantised, biased and requantised with the cache scale; columns
-// [0, H) go to new_q [M, H], [H, 2H) and [2H, 3H) to slot step_id of the K and V caches
-// [M, heads, max_step, d].  Same float arithmetic as the stand-alone kernel (no fused
-// multiply-add).
-struct EpiDecQkvI8 {
-  int8_t *new_q, *new_k, *new_v;
-  const __half* bias;
-  float alpha, dequant_scale, quant_scale;
-  int hidden, head_num, dim_per_head, max_step, step_id;
-  float inv_hidden, inv_dim;  // 1 / hidden, 1 / dim_per_head (for store1)
-  // the 16 bias values of columns n .. n + 15: they do not depend on the product, so the
-  // decode-step kernel requests them with its first weights
-  struct Pre {
-    half8_t b0, b1;
-  };
-  __device__ __forceinline__ Pre prefetch(int n) const {
-    return Pre{*reinterpret_cast<const half8_t*>(bias + n),
-               *reinterpret_cast<const half8_t*>(bias + n + 8)};
-  }
-  __device__ __forceinline__ void store16(long m, int n, int N, const v16i& c, bool full) const {
-    store16_pre(m, n, N, c, full, prefetch(n));
-  }
-  __device__ __forceinline__ void store16_pre(long m, int n, int N, const v16i& c, bool,
-                                              const Pre& pre) const {
-#pragma clang fp contract(off)
-    const int part = n / hidden, i = n - part * hidden;
-    const half8_t b0 = pre.b0, b1 = pre.b1;
-    int q[16];
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const float b = __half2float(k < 8 ? b0.v[k] : b1.v[k - 8]);
-      const float val = (float)requant_acc(c[k], alpha) * dequant_scale + b;
-      q[k] = float2int8(val, quant_scale);
-    }
-    int8_t* dst;
-    if (part == 0) {
-      dst = new_q + m * hidden + i;
-    } else {
-      const int head = i / dim_per_head, dim = i - head * dim_per_head;
-      dst = (part == 1 ? new_k : new_v) +
-            ((m * head_num + head) * max_step + step_id) * dim_per_head + dim;
-    }
-    uint4 o;
-    o.x = pack4_i8(q[0], q[1], q[2], q[3]);
-    o.y = pack4_i8(q[4], q[5], q[6], q[7]);
-    o.z = pack4_i8(q[8], q[9], q[10], q[11]);
-    o.w = pack4_i8(q[12], q[13], q[14], q[15]);
-    *reinterpret_cast<uint4*>(dst) = o;
-    (void)N;
-  }
-  // one element; its bias value is requested with the first weights
-  struct Pre1 {
-    __half b;
-  };
-  __device__ __forceinline__ Pre1 prefetch1(int n) const { return Pre1{bias[n]}; }
-  // what the elements of one column share: the 16 columns of a block lie in one part and one
-  // head (dim_per_head % 16 == 0), so the divisions run on the block's first column, the same
-  // in every lane, once per block; an element's address is base + row * row_stride + add.
-  // 32-bit offsets: this form serves the decode-step kernels only (at most 64 rows; the
-  // launcher refuses caches of 2^31 bytes and more for them)
-  struct Blk1 {
-    int8_t* base;
-    int row_stride, add;
-  };
-  __device__ __forceinline__ Blk1 block1(int n) const {
-    const int nb = __builtin_amdgcn_readfirstlane(n & ~15);
-    const int part = div_by(nb, hidden, inv_hidden), ib = nb - part * hidden;
-    const int head = div_by(ib, dim_per_head, inv_dim), dim = ib - head * dim_per_head + (n & 15);
-    if (part == 0) return Blk1{new_q, hidden, ib + (n & 15)};
-    return Blk1{part == 1 ? new_k : new_v, head_num * max_step * dim_per_head,
-                (head * max_step + step_id) * dim_per_head + dim};
-  }
-  __device__ __forceinline__ void store1(long m, Blk1 blk, int N, int acc, Pre1 pre,
-                                         const int8_t*, int) const {
-#pragma clang fp contract(off)
-    const float val = (float)requant_acc_fast(acc, alpha) * dequant_scale + __half2float(pre.b);
-    blk.base[(unsigned)((int)m * blk.row_stride + blk.add)] =
-        (int8_t)float2int8(val, quant_scale);
-    (void)N;
-  }
-  bool vec_ok(int) const { return true; }
-  static const char* name() { return "EpiDecQkvI8"; }
-};
-
-// Decode-step cross-attention query product followed by ker_arrange_encdec_q_i8I
-// (inference/kernels/transformerKernels_int8.cc.cu:1596-1645; call site
-// model/quant_decoder.cc.cu:745-760): code -> half(code * dq) + bias (a half add) -> fp16 q
-// [batch, heads, beam, d].
-struct EpiEncdecQF16 {
-  __half* new_q;
-  const __half* bias;
-  float alpha, dequant_scale;
-  int beam_size, head_num, dim_per_head;
-  float inv_beam, inv_dim;  // 1 / beam_size, 1 / dim_per_head (for store1)
-  struct Pre {  // the bias of columns n .. n + 15, requested ahead of the product
-    half8_t b0, b1;
-  };
-  __device__ __forceinline__ Pre prefetch(int n) const {
-    return Pre{*reinterpret_cast<const half8_t*>(bias + n),
-               *reinterpret_cast<const half8_t*>(bias + n + 8)};
-  }
-  __device__ __forceinline__ void store16(long m, int n, int N, const v16i& c, bool full) const {
-    store16_pre(m, n, N, c, full, prefetch(n));
-  }
-  __device__ __forceinline__ void store16_pre(long m, int n, int N, const v16i& c, bool,
-                                              const Pre& pre) const {
-    const int head = n / dim_per_head, dim = n - head * dim_per_head;
-    const long batch_id = m / beam_size, beam_id = m - batch_id * beam_size;
-    __half* dst = new_q + ((batch_id * head_num + head) * beam_size + beam_id) * dim_per_head + dim;
-    const half8_t b0 = pre.b0, b1 = pre.b1;
-    half8_t lo, hi;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      lo.v[k] = __float2half_rn(dequant_add_bias_h(requant_acc(c[k], alpha), dequant_scale,
-                                                   __half2float(b0.v[k])));
-      hi.v[k] = __float2half_rn(dequant_add_bias_h(requant_acc(c[8 + k], alpha), dequant_scale,
-                                                   __half2float(b1.v[k])));
-    }
-    *reinterpret_cast<half8_t*>(dst) = lo;
-    *reinterpret_cast<half8_t*>(dst + 8) = hi;
-    (void)N;
-  }
-  struct Pre1 {
-    __half b;
-  };
-  __device__ __forceinline__ Pre1 prefetch1(int n) const { return Pre1{bias[n]}; }
-  struct Blk1 {
-    int add;  // the column's share of the offset: head * beam_size * dim_per_head + dim
-  };
-  __device__ __forceinline__ Blk1 block1(int n) const {
-    const int nb = __builtin_amdgcn_readfirstlane(n & ~15);
-    const int head = div_by(nb, dim_per_head, inv_dim), dim = nb - head * dim_per_head + (n & 15);
-    return Blk1{head * beam_size * dim_per_head + dim};
-  }
-  __device__ __forceinline__ void store1(long m, Blk1 blk, int N, int acc, Pre1 pre,
-                                         const int8_t*, int) const {
-    const int batch_id = div_by((int)m, beam_size, inv_beam), beam_id = (int)m - batch_id * beam_size;
-    new_q[(unsigned)((batch_id * head_num * beam_size + beam_id) * dim_per_head + blk.add)] =
-        __float2half_rn(dequant_add_bias_h(requant_acc_fast(acc, alpha), dequant_scale,
-                                           __half2float(pre.b)));
-    (void)N;
-  }
-  bool vec_ok(int) const { return true; }
-  static const char* name() { return "EpiEncdecQF16"; }
-};
 
 // The same with the scale read from device memory (the csrc layers keep their clip values
 // and the alpha derived from them on the device: csrc/kernels/cuda/cublas_wrappers.cpp:134
@@ -382,32 +223,6 @@ __device__ __forceinline__ void store_tile_acc(const Epi& epi, const v16i (&acc)
       }
     }
   }
-}
-
-// linear work index -> tile.  Workgroups (and the persistent kernel's work items) are
-// dealt round-robin to the 8 XCDs; renumber so that each XCD (own L2) works on a
-// contiguous run of tiles, walked in column-major order of 8-tile-tall groups so that a
-// run shares W columns and A rows.
-// Work-item counts stay below 2^24 (checked by the dispatcher): with both operands masked to
-// 24 bits the compiler divides through a float reciprocal, a dozen instructions instead of
-// the forty of a full 32-bit division -- this arithmetic runs before the first load of a
-// launch and sits in the kernel four times.
-__device__ __forceinline__ int div24(int a, int b) {
-  return (int)(((unsigned)a & 0xffffffu) / ((unsigned)b & 0xffffffu));
-}
-__device__ __forceinline__ void tile_of(int t, int nblk, int tiles_m, int tiles_n, int& tile_m,
-                                        int& tile_n) {
-  const int per = nblk / 8, rem = nblk % 8;
-  const int xcd = t % 8, loc = t / 8;
-  const int pid = xcd * per + (xcd < rem ? xcd : rem) + loc;
-  constexpr int GROUP = 8;
-  const int group_sz = GROUP * tiles_n;
-  const int grp = div24(pid, group_sz);
-  const int in_grp = pid - grp * group_sz;
-  const int first_m = grp * GROUP;
-  const int gm = min(tiles_m - first_m, GROUP);
-  tile_n = div24(in_grp, gm);
-  tile_m = first_m + (in_grp - tile_n * gm);
 }
 
 // ---------------------------------------------------------------------------------
@@ -914,7 +729,7 @@ __global__ void __launch_bounds__(256)
 gemm_i8_skinny_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, Epi epi, int M,
                       int N, int K, int, int, bool vec_store, int ksplit) {
   __shared__ int red[4][MBLK][16][64];  // [wavefront][m block][register][lane]
-  constexpr bool kLut = std::is_same<Epi, EpiLutI8>::value;
+  constexpr bool kLut = is_lut<Epi>;
   __shared__ __align__(16) int8_t tab[kLut ? 32 * 256 : 16];  // table rows of the 32 columns
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, g = lane >> 5;
@@ -1022,7 +837,7 @@ gemm_i8_skinny16_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__
                         int N, int K, int kw, int, bool vec_store, int) {
   // NB 16-column blocks per workgroup: 2, or 1 where that still fits one round of the chip
   __shared__ int red[4][MB][NB][4][64];  // [wavefront][row block][column block][register][lane]
-  constexpr bool kLut = std::is_same<Epi, EpiLutI8>::value;
+  constexpr bool kLut = is_lut<Epi>;
   __shared__ __align__(16) int8_t tab[kLut ? 16 * NB * 256 : 16];  // table rows of the columns
   asm volatile("" ::"s"(A), "s"(W));  // one batch of kernel-argument loads, not two in a row
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1278,6 +1093,13 @@ void route_epoch_bump() { g_route_epoch.fetch_add(1, std::memory_order_acq_rel);
 void gemm_i8_time_next_launch(hipEvent_t start, hipEvent_t stop) {
   g_ev_start = start;
   g_ev_stop = stop;
+}
+
+bool gemm_take_timing_events(hipEvent_t* start, hipEvent_t* stop) {
+  *start = g_ev_start;
+  *stop = g_ev_stop;
+  g_ev_start = g_ev_stop = nullptr;
+  return *start != nullptr;
 }
 
 // Compute units of the current device (256 on MI355X), read once per device: the choices below
@@ -1536,7 +1358,7 @@ static int dispatch(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int
       }
     }
   }
-  if constexpr (std::is_same<Epi, EpiLutI8>::value) {
+  if constexpr (is_lut<Epi>) {
     // the tabulated epilogue: 128 x 64 tiles, 2 stages + 16 KB of table rows in LDS
     if (stream && ksplit == 1 && K / kBK >= 2) {
       const int tn64 = (N + kSBN - 1) / kSBN;

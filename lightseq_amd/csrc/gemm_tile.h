@@ -9,6 +9,13 @@
 
 namespace lsh {
 
+// Where the table kernels of gemm_kw.h find code `code` of column `col` in the column's 256 bytes of
+// LDS: the 16-byte chunks are permuted by the column, so that the lanes of one lookup, whose
+// columns differ, spread over the banks.
+__device__ __forceinline__ int kw_table_index(int code, int col) {
+  return (code + 128) ^ ((col & 15) << 4);
+}
+
 // ---------------------------------------------------------------------------------
 // Epilogues.  store16(m, n, N, c, full): c[0..15] are C[m, n .. n+15]; `full` means all
 // 16 columns exist and the vector path may be used.
@@ -39,7 +46,15 @@ struct EpiI32 {
                                          int) const {
     C[m * N + blk.n] = acc;
   }
-  bool vec_ok(int N) const { return N % 4 == 0 && (reinterpret_cast<uintptr_t>(C) & 15u) == 0; }
+  // four neighbouring elements (gemm_kw.h)
+  static constexpr bool kTable = false, kBlockedOut = false;
+  struct Col {};
+  __device__ __forceinline__ Col column(int, int) const { return Col{}; }
+  __device__ __forceinline__ void store4(int m, int n, int N, Col, const v4i& c) const {
+    *reinterpret_cast<v4i*>(C + (long)m * N + n) = c;
+  }
+  bool aligned() const { return C != nullptr && (reinterpret_cast<uintptr_t>(C) & 15u) == 0; }
+  bool vec_ok(int N) const { return N % 4 == 0 && aligned(); }
   static const char* name() { return "EpiI32"; }
 };
 
@@ -81,7 +96,15 @@ struct EpiI8 {
                                          int) const {
     C[m * N + blk.n] = (int8_t)requant_acc_fast(acc, alpha);
   }
-  bool vec_ok(int N) const { return N % 16 == 0 && (reinterpret_cast<uintptr_t>(C) & 15u) == 0; }
+  static constexpr bool kTable = false, kBlockedOut = false;
+  struct Col {};
+  __device__ __forceinline__ Col column(int, int) const { return Col{}; }
+  __device__ __forceinline__ void store4(int m, int n, int N, Col, const v4i& c) const {
+    *reinterpret_cast<uint32_t*>(C + (long)m * N + n) =
+        requant_acc_pack4(c[0], c[1], c[2], c[3], alpha);
+  }
+  bool aligned() const { return C != nullptr && (reinterpret_cast<uintptr_t>(C) & 15u) == 0; }
+  bool vec_ok(int N) const { return N % 16 == 0 && aligned(); }
   static const char* name() { return "EpiI8"; }
 };
 
@@ -93,7 +116,8 @@ struct EpiI8 {
 // element -- more than the matrix cores spend on a K = 768 product -- while the lookup is
 // one byte load per element from a table that stays in L2 (768 KB for N = 3072); the lanes
 // of one load instruction read two table rows, i.e. a handful of cache lines.
-struct EpiLutI8 {
+template <bool BLK>
+struct EpiLut {
   int8_t* C;
   const int8_t* lut;
   float alpha;
@@ -114,7 +138,9 @@ struct EpiLutI8 {
 #pragma unroll
     for (int i = 0; i < 16; ++i)
       q[i] = tab[(n_local + i) * 256 + requant_acc_fast(c[i], alpha) + 128];
-    store16_i8(C + m * N + n, n, N, q, full);
+    // blocked output: the 16 columns are one 16-byte chunk, and the lanes of consecutive rows
+    // write consecutive chunks
+    store16_i8(C + (BLK ? blocked_offset(m, n, N) : m * N + n), n, N, q, full);
   }
   // one element, the table rows of the workgroup's columns staged in LDS (n_local: the
   // element's column among them)
@@ -128,13 +154,59 @@ struct EpiLutI8 {
                                          const int8_t* tab, int n_local) const {
     C[m * N + blk.n] = tab[n_local * 256 + requant_acc_fast(acc, alpha) + 128];
   }
-  bool vec_ok(int N) const { return N % 16 == 0 && (reinterpret_cast<uintptr_t>(C) & 15u) == 0; }
+  static constexpr bool kTable = true, kBlockedOut = BLK;
+  __device__ __forceinline__ const int8_t* table() const { return lut; }
+  struct Col {};
+  __device__ __forceinline__ Col column(int, int) const { return Col{}; }
+  __device__ __forceinline__ void store4(int m, int n, int N, Col, const v4i& c,
+                                         const int8_t* tab) const {
+    int q[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      q[i] = tab[i * 256 + kw_table_index(requant_acc_fast(c[i], alpha), n + i)];
+    *reinterpret_cast<uint32_t*>(C + (BLK ? blocked_offset(m, n, N) : (long)m * N + n)) =
+        pack4_i8(q[0], q[1], q[2], q[3]);
+  }
+  bool aligned() const { return C != nullptr && (reinterpret_cast<uintptr_t>(C) & 15u) == 0; }
+  bool vec_ok(int N) const { return N % 16 == 0 && aligned(); }
   static const char* name() { return "EpiLutI8"; }
 };
+typedef EpiLut<false> EpiLutI8;
+typedef EpiLut<true> EpiLutBlk;
+template <typename Epi>
+constexpr bool is_lut = std::is_same<Epi, EpiLutI8>::value || std::is_same<Epi, EpiLutBlk>::value;
 
 template <typename Epi>
-__device__ __forceinline__ const int8_t* epi_lut(const Epi&) { return nullptr; }
-__device__ __forceinline__ const int8_t* epi_lut(const EpiLutI8& e) { return e.lut; }
+__device__ __forceinline__ const int8_t* epi_lut(const Epi& e) {
+  if constexpr (is_lut<Epi>) return e.lut;
+  else return nullptr;
+}
+
+// linear work index -> tile.  Workgroups (and the persistent kernel's work items) are
+// dealt round-robin to the 8 XCDs; renumber so that each XCD (own L2) works on a
+// contiguous run of tiles, walked in column-major order of 8-tile-tall groups so that a
+// run shares W columns and A rows.
+// Work-item counts stay below 2^24 (checked by the dispatcher): with both operands masked to
+// 24 bits the compiler divides through a float reciprocal, a dozen instructions instead of
+// the forty of a full 32-bit division -- this arithmetic runs before the first load of a
+// launch and sits in the kernel four times.
+__device__ __forceinline__ int div24(int a, int b) {
+  return (int)(((unsigned)a & 0xffffffu) / ((unsigned)b & 0xffffffu));
+}
+__device__ __forceinline__ void tile_of(int t, int nblk, int tiles_m, int tiles_n, int& tile_m,
+                                        int& tile_n) {
+  const int per = nblk / 8, rem = nblk % 8;
+  const int xcd = t % 8, loc = t / 8;
+  const int pid = xcd * per + (xcd < rem ? xcd : rem) + loc;
+  constexpr int GROUP = 8;
+  const int group_sz = GROUP * tiles_n;
+  const int grp = div24(pid, group_sz);
+  const int in_grp = pid - grp * group_sz;
+  const int first_m = grp * GROUP;
+  const int gm = min(tiles_m - first_m, GROUP);
+  tile_n = div24(in_grp, gm);
+  tile_m = first_m + (in_grp - tile_n * gm);
+}
 
 // ---------------------------------------------------------------------------------
 // One output tile of TM x TN = (WGM * MB * 32) x (WGN * NB * 32) on WGM * WGN wavefronts: rows
@@ -149,18 +221,19 @@ __device__ __forceinline__ const int8_t* epi_lut(const EpiLutI8& e) { return e.l
 // of them); the caller separates two calls by a barrier of its own.
 // Preconditions: K % 128 == 0, K / 128 >= NST, N % 16 == 0, 32-bit operand offsets, operands
 // 16-byte aligned.  A_FROM_L2: the rows of A were written by other compute units of this XCD
-// during this launch (read past the vector cache).
+// during this launch (read past the vector cache).  BLOCKED: both operands in the blocked layout.
 // ---------------------------------------------------------------------------------
 template <typename Epi, int NST>
 constexpr int tile_gemm_barriers(int nk) {
-  return nk + (std::is_same<Epi, EpiLutI8>::value ? 1 : 0);
+  return nk + (is_lut<Epi> ? 1 : 0);
 }
 
-template <typename Epi, int WGM, int WGN, int MB, int NB, int NST, bool A_FROM_L2 = false>
+template <typename Epi, int WGM, int WGN, int MB, int NB, int NST, bool A_FROM_L2 = false,
+          bool BLOCKED = false>
 __device__ __forceinline__ void tile_gemm(const int8_t* __restrict__ A,
                                           const int8_t* __restrict__ W, const Epi& epi, int row0,
                                           int row_end, int N, int K, int tn, int8_t* smem) {
-  constexpr bool LUT = std::is_same<Epi, EpiLutI8>::value;
+  constexpr bool LUT = is_lut<Epi>;
   // The operand order of the MFMA decides what a lane's 16 accumulators are: weight rows first,
   // 16 adjacent columns of one output row (one 16-byte store of int8 codes); activations first,
   // 16 rows of one column -- the layout for int32 output, whose stores then cover whole lines.
@@ -170,6 +243,7 @@ __device__ __forceinline__ void tile_gemm(const int8_t* __restrict__ A,
   constexpr int STAGE = (TM + TN) * kBK;
   constexpr int NA = TM / 8 / NWV, NW = TN / 8 / NWV, PER = NA + NW;  // 1-KB loads per wavefront
   constexpr int NTAB = TN / 4 / NWV;  // table loads per wavefront
+  constexpr int KSTEP = BLOCKED ? 2048 : kBK;  // bytes from one K step of a row to the next
   static_assert(TM % (8 * NWV) == 0 && TN % (8 * NWV) == 0, "stage rows split over the wavefronts");
   static_assert((NST - 1) * PER < 64, "vmcnt range");
   static_assert(!LUT || (TM >= TN && TN % (4 * NWV) == 0), "table fits a freed stage");
@@ -183,12 +257,26 @@ __device__ __forceinline__ void tile_gemm(const int8_t* __restrict__ A,
     const int row = (wave + NWV * i) * 8 + (lane >> 3);
     const int c = (lane & 7) ^ key_act(row);
     a_src[i] = (uint32_t)min(row0 + row, row_end - 1) * (uint32_t)K + c * 16;
+    if (BLOCKED) {
+      // one 1-KB block of 16 rows x 64 bytes per load, as it lies in memory: it is in fragment
+      // order already, and 16 lanes of a fragment read are 256 contiguous bytes of LDS
+      const int q = wave + NWV * i;
+      a_src[i] = (uint32_t)min((row0 >> 4) + (q >> 1), (row_end - 1) >> 4) * 16u * (uint32_t)K +
+                 (q & 1) * 1024 + lane * 16;
+    }
   }
 #pragma unroll
   for (int i = 0; i < NW; ++i) {
     const int row = (wave + NWV * i) * 8 + (lane >> 3);
     const int c = (lane & 7) ^ key_wgt(row);
     w_src[i] = (uint32_t)min(tn * TN + row, N - 1) * (uint32_t)K + c * 16;
+    if (BLOCKED) {
+      // the two halves of an odd block's rows change places: 16 lanes in sigma order read eight
+      // rows of an even and the same eight of the odd block, which must not share their banks
+      const int q = wave + NWV * i;
+      w_src[i] = (uint32_t)min(tn * (TN / 16) + (q >> 1), (N - 1) >> 4) * 16u * (uint32_t)K +
+                 (q & 1) * 1024 + (lane ^ ((q >> 1) & 1) * 8) * 16;
+    }
   }
   const uint32_t lds0 = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)smem);
   auto dma1 = [&](const int8_t* base, uint32_t voff, uint32_t lds) {
@@ -209,12 +297,12 @@ __device__ __forceinline__ void tile_gemm(const int8_t* __restrict__ A,
     const uint32_t base = lds0 + slot * STAGE;
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
-      if (A_FROM_L2) dma1_l2(A + kt * kBK, a_src[i], base + (wave + NWV * i) * 1024);
-      else dma1(A + kt * kBK, a_src[i], base + (wave + NWV * i) * 1024);
+      if (A_FROM_L2) dma1_l2(A + kt * KSTEP, a_src[i], base + (wave + NWV * i) * 1024);
+      else dma1(A + kt * KSTEP, a_src[i], base + (wave + NWV * i) * 1024);
     }
 #pragma unroll
     for (int i = 0; i < NW; ++i)
-      dma1(W + kt * kBK, w_src[i], base + TM * kBK + (wave + NWV * i) * 1024);
+      dma1(W + kt * KSTEP, w_src[i], base + TM * kBK + (wave + NWV * i) * 1024);
   };
   // LDS byte offset of this lane's fragment chunk for K slice 0; slice ks is at (offset ^ (ks << 5)):
   // chunk index 2 * ks + g, swizzled by the row key, and 2 * ks only touches bits 1-2 of it
@@ -222,23 +310,28 @@ __device__ __forceinline__ void tile_gemm(const int8_t* __restrict__ A,
 #pragma unroll
   for (int i = 0; i < MB; ++i) {
     const int row = wm * (MB * 32) + i * 32 + l32;
-    a_base[i] = row * kBK + ((g ^ key_act(row)) << 4);
+    a_base[i] = BLOCKED ? (row >> 4) * 2048 + g * 256 + (row & 15) * 16
+                        : row * kBK + ((g ^ key_act(row)) << 4);
   }
 #pragma unroll
   for (int j = 0; j < NB; ++j) {
     const int row = wn * (NB * 32) + j * 32 + sigma(l32);
-    w_base[j] = TM * kBK + row * kBK + ((g ^ key_wgt(row)) << 4);
+    w_base[j] = TM * kBK + (BLOCKED ? (row >> 4) * 2048 + g * 256 + ((row & 15) ^ ((row >> 4) & 1) * 8) * 16
+                                    : row * kBK + ((g ^ key_wgt(row)) << 4));
   }
+  auto slice_at = [&](int base, int ks) {
+    return BLOCKED ? base + (ks >> 1) * 1024 + (ks & 1) * 512 : base ^ (ks << 5);
+  };
   struct Frag {
     v4i a[MB], w[NB];
   };
   auto load_frag = [&](Frag& f, const int8_t* stage, int ks) {
 #pragma unroll
     for (int i = 0; i < MB; ++i)
-      f.a[i] = *reinterpret_cast<const v4i*>(stage + (a_base[i] ^ (ks << 5)));
+      f.a[i] = *reinterpret_cast<const v4i*>(stage + slice_at(a_base[i], ks));
 #pragma unroll
     for (int j = 0; j < NB; ++j)
-      f.w[j] = *reinterpret_cast<const v4i*>(stage + (w_base[j] ^ (ks << 5)));
+      f.w[j] = *reinterpret_cast<const v4i*>(stage + slice_at(w_base[j], ks));
   };
   v16i acc[MB][NB];
 #pragma unroll

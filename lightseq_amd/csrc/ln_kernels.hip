@@ -15,8 +15,6 @@
 #include "ls_launch.h"
 #include "ln_rows8.h"
 
-#include <hip/hip_ext.h>
-
 #include <type_traits>
 
 namespace lsh {
@@ -129,15 +127,18 @@ ln_rows8_kernel(const AccT* __restrict__ gemm_out, T* residual, T* out_t,
                 int8_t* __restrict__ out_q, const T* __restrict__ scale,
                 const T* __restrict__ bias, const T* __restrict__ residual_bias,
                 const T* __restrict__ colsum, int tokens, int hidden, float dequant_scale,
-                float quant_scale, int is_post_ln, int nparts, long part_stride) {
+                float quant_scale, int is_post_ln, int nparts, long part_stride, int blocked,
+                const int* __restrict__ row_map) {
   constexpr int RPW = kWave / LPR;
   const int lane = threadIdx.x & 63;
   const int row = (blockIdx.x * 4 + (threadIdx.x >> 6)) * RPW + lane / LPR;
+  int in_row = -1;
+  if (MODE == kLnResOut && row_map != nullptr) in_row = row_map[min(row, tokens - 1)];
   // dead rows keep the shuffles convergent
   ln_rows8_row<T, AccT, MODE, LPR, ITER>(row, row < tokens, lane % LPR, gemm_out, residual, out_t,
                                          out_q, scale, bias, residual_bias, colsum, hidden,
                                          dequant_scale, quant_scale, is_post_ln, nparts,
-                                         part_stride);
+                                         part_stride, nullptr, 0, blocked, in_row);
 }
 
 // ---------------------------------------------------------------------------------
@@ -306,7 +307,7 @@ __device__ __forceinline__ void
 ln_row_wg_finish(const float (&x)[4], bool on, int e, long base, const float (&g)[4],
                  const float (&b)[4], const float (&rb)[4], T* residual, T* out_t,
                  int8_t* __restrict__ out_q, int hidden, float quant_scale, int is_post_ln,
-                 float (*red)[4]) {
+                 float (*red)[4], int blocked) {
   const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int wpr = (int)blockDim.x >> 6;  // wavefronts of the row
   auto row_total = [&](float v, float* r) {
@@ -338,7 +339,7 @@ ln_row_wg_finish(const float (&x)[4], bool on, int e, long base, const float (&g
   if (MODE == kLnResOut) {
     st4(out_t, base + e, o);
   } else {
-    *reinterpret_cast<uint32_t*>(out_q + base + e) =
+    *reinterpret_cast<uint32_t*>(out_q + code_offset((int)blockIdx.x, e, hidden, blocked)) =
         pack4_i8(float2int8(o[0], quant_scale), float2int8(o[1], quant_scale),
                  float2int8(o[2], quant_scale), float2int8(o[3], quant_scale));
     float w[4];
@@ -366,7 +367,7 @@ ln_row_wg_kernel(const AccT* __restrict__ gemm_out, T* residual, T* out_t,
                  int8_t* __restrict__ out_q, const T* __restrict__ scale,
                  const T* __restrict__ bias, const T* __restrict__ residual_bias,
                  const T* __restrict__ colsum, int hidden, float dequant_scale,
-                 float quant_scale, int is_post_ln, int nparts, long part_stride) {
+                 float quant_scale, int is_post_ln, int nparts, long part_stride, int blocked) {
   __shared__ float red[2][4];
   const int e0 = (int)threadIdx.x * 4;
   const bool on = e0 < hidden;
@@ -435,7 +436,7 @@ ln_row_wg_kernel(const AccT* __restrict__ gemm_out, T* residual, T* out_t,
     if (!on) x[k] = 0.f;
   }
   ln_row_wg_finish<T, MODE>(x, on, e, base, g, b, rb, residual, out_t, out_q, hidden, quant_scale,
-                            is_post_ln, red);
+                            is_post_ln, red, blocked);
 }
 
 // The workgroup-per-row kernel is chosen by the caller, never by the row count: the two
@@ -469,7 +470,7 @@ dec_emb_ln_row_wg_kernel(const int8_t* __restrict__ token_emb, const T* __restri
                          int8_t* __restrict__ out_q, const T* __restrict__ scale,
                          const T* __restrict__ bias, const T* __restrict__ residual_bias,
                          int hidden, int vocab, int step, int max_step, float emb_scale,
-                         float quant_scale, int is_post_ln) {
+                         float quant_scale, int is_post_ln, int blocked) {
 #pragma clang fp contract(off)
   __shared__ float red[2][4];
   const int e0 = (int)threadIdx.x * 4;
@@ -496,7 +497,7 @@ dec_emb_ln_row_wg_kernel(const int8_t* __restrict__ token_emb, const T* __restri
     x[k] = on ? TT<T>::safe(TT<T>::rnd(v)) : 0.f;
   }
   ln_row_wg_finish<T, kLnFirst>(x, on, e, base, g, b, rb, residual, nullptr, out_q, hidden,
-                                quant_scale, is_post_ln, red);
+                                quant_scale, is_post_ln, red, blocked);
 }
 
 template <typename T>
@@ -504,12 +505,12 @@ int dec_emb_norm_layer_i8O(const int8_t* token_emb, const T* pos_emb, const int*
                            T* residual, int8_t* out_q, const T* scale, const T* bias,
                            const T* residual_bias, int rows, int hidden, int vocab, int step,
                            int max_step, float dequant_scale, bool scaled, float quant_scale,
-                           bool is_post_ln, hipStream_t s) {
+                           bool is_post_ln, hipStream_t s, bool blocked) {
   if (!token_emb || !pos_emb || !tokens || !residual || !out_q || !scale || !bias || rows <= 0 ||
       hidden <= 0 || vocab <= 0 || max_step <= 0)
     return lsh_fail(LSH_ERR_INVALID, "dec_emb_norm_layer_i8O: bad arguments");
   if (step < 0 || step >= max_step) return lsh_fail(LSH_ERR_INVALID, "violate step < max_step");
-  if (hidden % 4 != 0 || hidden > 1024 || !aligned16(token_emb) || !aligned16(pos_emb) ||
+  if (hidden % 4 != 0 || hidden > 1024 || (blocked && hidden % 64 != 0) || !aligned16(token_emb) || !aligned16(pos_emb) ||
       !aligned16(residual) || !aligned16(out_q) || !aligned16(scale) || !aligned16(bias) ||
       !aligned16(residual_bias))
     return lsh_fail(LSH_ERR_UNSUPPORTED,
@@ -520,17 +521,17 @@ int dec_emb_norm_layer_i8O(const int8_t* token_emb, const T* pos_emb, const int*
   dec_emb_ln_row_wg_kernel<T><<<rows, tpr, 0, s>>>(token_emb, pos_emb, tokens, residual, out_q,
                                                    scale, bias, residual_bias, hidden, vocab, step,
                                                    max_step, emb_scale, quant_scale,
-                                                   is_post_ln ? 1 : 0);
+                                                   is_post_ln ? 1 : 0, blocked ? 1 : 0);
   return lsh_check_launch("dec_emb_ln_row_wg_kernel");
 }
 template int dec_emb_norm_layer_i8O<__half>(const int8_t*, const __half*, const int*, __half*,
                                             int8_t*, const __half*, const __half*, const __half*,
                                             int, int, int, int, int, float, bool, float, bool,
-                                            hipStream_t);
+                                            hipStream_t, bool);
 template int dec_emb_norm_layer_i8O<float>(const int8_t*, const float*, const int*, float*,
                                            int8_t*, const float*, const float*, const float*, int,
                                            int, int, int, int, float, bool, float, bool,
-                                           hipStream_t);
+                                           hipStream_t, bool);
 
 // The same for a generation step of the GPT model: the embedding of one token per sequence at
 // position `pos` (a padding token gives zeros), the token counted into real_seq_len and
@@ -542,7 +543,7 @@ gpt_emb_ln_row_wg_kernel(const int8_t* __restrict__ token_emb, const T* __restri
                          int8_t* __restrict__ out_q, const T* __restrict__ scale,
                          const T* __restrict__ bias, const T* __restrict__ residual_bias,
                          int* real_seq_len, int* zero_flag, int padding_id, int hidden, int vocab,
-                         int pos, float emb_scale, float quant_scale, int is_post_ln) {
+                         int pos, float emb_scale, float quant_scale, int is_post_ln, int blocked) {
 #pragma clang fp contract(off)
   __shared__ float red[2][4];
   const int e0 = (int)threadIdx.x * 4;
@@ -574,7 +575,7 @@ gpt_emb_ln_row_wg_kernel(const int8_t* __restrict__ token_emb, const T* __restri
     x[k] = on ? TT<T>::safe(TT<T>::rnd(v)) : 0.f;
   }
   ln_row_wg_finish<T, kLnFirst>(x, on, e, base, g, b, rb, residual, nullptr, out_q, hidden,
-                                quant_scale, is_post_ln, red);
+                                quant_scale, is_post_ln, red, blocked);
 }
 
 template <typename T>
@@ -583,13 +584,13 @@ int gpt_emb_step_norm_layer_i8O(const int8_t* token_emb, const T* pos_emb, const
                                 const T* residual_bias, int* real_seq_len, int* zero_flag,
                                 int batch_size, int hidden, int vocab, int padding_id, int pos,
                                 int max_step, float dequant_scale, float quant_scale,
-                                bool is_post_ln, hipStream_t s) {
+                                bool is_post_ln, hipStream_t s, bool blocked) {
   if (!token_emb || !pos_emb || !token_id || !residual || !out_q || !scale || !bias ||
       !real_seq_len || batch_size <= 0 || hidden <= 0 || vocab <= 0)
     return lsh_fail(LSH_ERR_INVALID, "gpt_emb_step_norm_layer_i8O: bad arguments");
   if (pos < 0 || pos >= max_step)
     return lsh_fail(LSH_ERR_INVALID, "gpt_emb_step_norm_layer_i8O: position outside the table");
-  if (hidden % 4 != 0 || hidden > 1024 || !aligned16(token_emb) || !aligned16(pos_emb) ||
+  if (hidden % 4 != 0 || hidden > 1024 || (blocked && hidden % 64 != 0) || !aligned16(token_emb) || !aligned16(pos_emb) ||
       !aligned16(residual) || !aligned16(out_q) || !aligned16(scale) || !aligned16(bias) ||
       !aligned16(residual_bias))
     return lsh_fail(LSH_ERR_UNSUPPORTED,
@@ -598,23 +599,25 @@ int gpt_emb_step_norm_layer_i8O(const int8_t* token_emb, const T* pos_emb, const
   const int tpr = ((hidden / 4 + 63) / 64) * 64;
   gpt_emb_ln_row_wg_kernel<T><<<batch_size, tpr, 0, s>>>(
       token_emb, pos_emb, token_id, residual, out_q, scale, bias, residual_bias, real_seq_len,
-      zero_flag, padding_id, hidden, vocab, pos, dequant_scale, quant_scale, is_post_ln ? 1 : 0);
+      zero_flag, padding_id, hidden, vocab, pos, dequant_scale, quant_scale, is_post_ln ? 1 : 0,
+      blocked ? 1 : 0);
   return lsh_check_launch("gpt_emb_ln_row_wg_kernel");
 }
 template int gpt_emb_step_norm_layer_i8O<__half>(const int8_t*, const __half*, const int*,
                                                  __half*, int8_t*, const __half*, const __half*,
                                                  const __half*, int*, int*, int, int, int, int,
-                                                 int, int, float, float, bool, hipStream_t);
+                                                 int, int, float, float, bool, hipStream_t, bool);
 template int gpt_emb_step_norm_layer_i8O<float>(const int8_t*, const float*, const int*, float*,
                                                 int8_t*, const float*, const float*, const float*,
                                                 int*, int*, int, int, int, int, int, int, float,
-                                                float, bool, hipStream_t);
+                                                float, bool, hipStream_t, bool);
 
 template <typename T, typename AccT, int MODE>
 static int launch_ln(const AccT* gemm_out, T* residual, T* out_t, int8_t* out_q, const T* scale,
                      const T* bias, const T* residual_bias, const T* colsum, int tokens,
                      int hidden, float dequant_scale, float quant_scale, int is_post_ln,
-                     hipStream_t stream, int nparts = 1, long part_stride = 0) {
+                     hipStream_t stream, int nparts = 1, long part_stride = 0, bool blocked = false,
+                     const int* row_map = nullptr) {
   if (tokens <= 0 || hidden <= 0) return lsh_fail(LSH_ERR_INVALID, "layer norm: empty shape");
   if (nparts < 1 || (nparts > 1 && (sizeof(AccT) != 4 || part_stride % 4 != 0)))
     return lsh_fail(LSH_ERR_INVALID, "layer norm: bad accumulator planes");
@@ -622,11 +625,15 @@ static int launch_ln(const AccT* gemm_out, T* residual, T* out_t, int8_t* out_q,
                       aligned16(residual) && aligned16(out_t) && aligned16(out_q) &&
                       aligned16(scale) && aligned16(bias) && aligned16(residual_bias) &&
                       aligned16(colsum);
-  if (vec_ok && hidden <= 1024 && g_ln_few_rows) {
+  if ((blocked && hidden % 64 != 0) || ((blocked || row_map) && !vec_ok))
+    return lsh_fail(LSH_ERR_UNSUPPORTED, "layer norm: blocked codes and row maps need hidden % 64 == 0, "
+                                         "hidden <= 2048 and aligned operands");
+  const int blk = blocked ? 1 : 0;
+  if (vec_ok && hidden <= 1024 && g_ln_few_rows && !row_map) {
     const int tpr = ((hidden / 4 + 63) / 64) * 64;  // threads of a row: whole wavefronts
     ln_row_wg_kernel<T, AccT, MODE><<<tokens, tpr, 0, stream>>>(
         gemm_out, residual, out_t, out_q, scale, bias, residual_bias, colsum, hidden,
-        dequant_scale, quant_scale, is_post_ln, nparts, part_stride);
+        dequant_scale, quant_scale, is_post_ln, nparts, part_stride, blk);
     return lsh_check_launch("ln_row_wg_kernel");
   }
   if (vec_ok && hidden % 8 == 0) {
@@ -635,7 +642,7 @@ static int launch_ln(const AccT* gemm_out, T* residual, T* out_t, int8_t* out_q,
   ln_rows8_kernel<T, AccT, MODE, LPR, IT>                                                        \
       <<<(tokens + 4 * (64 / LPR) - 1) / (4 * (64 / LPR)), 256, 0, stream>>>(                    \
           gemm_out, residual, out_t, out_q, scale, bias, residual_bias, colsum, tokens, hidden,  \
-          dequant_scale, quant_scale, is_post_ln, nparts, part_stride)
+          dequant_scale, quant_scale, is_post_ln, nparts, part_stride, blk, row_map)
     if (hidden <= 256) LSH_LN8_CASE(32, 1);
     else if (hidden <= 512) LSH_LN8_CASE(32, 2);
     else if (hidden <= 768) LSH_LN8_CASE(32, 3);
@@ -683,12 +690,6 @@ int tile_weight_16x64(const int8_t* w, int8_t* tiled, int N, int K, hipStream_t 
   return lsh_check_launch("tile_weight_16x64_kernel");
 }
 
-static thread_local hipEvent_t g_gln_ev_start = nullptr, g_gln_ev_stop = nullptr;
-void gemm_ln_time_next_launch(hipEvent_t start, hipEvent_t stop) {
-  g_gln_ev_start = start;
-  g_gln_ev_stop = stop;
-}
-
 bool gemm_ln_fused_supported(int hidden, int K) {
   return hidden == K && (hidden == 512 || hidden == 768 || hidden == 1024);
 }
@@ -707,14 +708,11 @@ int gemm_i8_residual_ln_i8O(const int8_t* A, const int8_t* w_tiled, float alpha,
       !aligned16(residual_bias) || !aligned16(output) || !aligned16(residual))
     return lsh_fail(LSH_ERR_INVALID, "gemm_i8_residual_ln_i8O: pointers must be 16-byte aligned");
   const int grid = (batch_tokens + 15) / 16;
-  // kernel-exact begin / end timestamps when the caller asked for them
-  hipEvent_t e0 = g_gln_ev_start, e1 = g_gln_ev_stop;
-  g_gln_ev_start = g_gln_ev_stop = nullptr;
   const int post = is_post_ln ? 1 : 0;
 #define LSH_GLN(NT, KS, LPR, IT)                                                               \
-  hipExtLaunchKernelGGL((gemm_ln_rows16_kernel<T, NT, KS, LPR, IT>), dim3(grid), dim3(512), 0,  \
-                        stream, e0, e1, 0, A, w_tiled, alpha, residual, output, scale, bias,    \
-                        residual_bias, batch_tokens, dequant_scale, quant_scale, post)
+  gemm_ln_rows16_kernel<T, NT, KS, LPR, IT><<<grid, 512, 0, stream>>>(                          \
+      A, w_tiled, alpha, residual, output, scale, bias, residual_bias, batch_tokens,            \
+      dequant_scale, quant_scale, post)
   if (hidden_size == 512) LSH_GLN(4, 8, 32, 2);
   else if (hidden_size == 768) LSH_GLN(6, 12, 32, 3);
   else LSH_GLN(8, 16, 64, 2);
@@ -731,50 +729,53 @@ template int gemm_i8_residual_ln_i8O<float>(const int8_t*, const int8_t*, float,
 template <typename T>
 int norm_layer_resual_i8O(int token_num, int hidden_size, hipStream_t stream, T* input,
                           int8_t* output, const T* scale, const T* bias, const T* residual_bias,
-                          float quant_scale, bool is_post_ln) {
+                          float quant_scale, bool is_post_ln, bool blocked) {
   if (!input || !output || !scale || !bias || !residual_bias)
     return lsh_fail(LSH_ERR_INVALID, "ker_norm_layer_resual_i8O: null pointer");
   return launch_ln<T, int8_t, kLnFirst>(nullptr, input, nullptr, output, scale, bias,
                                         residual_bias, nullptr, token_num, hidden_size, 0.f,
-                                        quant_scale, is_post_ln, stream);
+                                        quant_scale, is_post_ln, stream, 1, 0, blocked);
 }
 
 template <typename T, typename AccT>
 int residual_bias_ln_i8O(const AccT* input, const T* scale, const T* bias, const T* residual_bias,
                          int8_t* output, T* residual, int batch_tokens, int hidden_size,
                          float dequant_scale, float quant_scale, hipStream_t stream,
-                         bool is_post_ln, const T* colsum, int nparts, long part_stride) {
+                         bool is_post_ln, const T* colsum, int nparts, long part_stride,
+                         bool blocked) {
   if (!input || !output || !scale || !bias || !residual)
     return lsh_fail(LSH_ERR_INVALID, "ker_residual_bias_ln_*_i8O: null pointer");
   return launch_ln<T, AccT, kLnResQuant>(input, residual, nullptr, output, scale, bias,
                                          residual_bias, colsum, batch_tokens, hidden_size,
                                          dequant_scale, quant_scale, is_post_ln, stream, nparts,
-                                         part_stride);
+                                         part_stride, blocked);
 }
 
 template <typename T>
 int residual_bias_ln_i32I(const int32_t* input, const T* scale, const T* bias, const T* residual,
                           T* output, int batch_tokens, int hidden_size, float dequant_scale,
-                          hipStream_t stream, const T* colsum, int nparts, long part_stride) {
+                          hipStream_t stream, const T* colsum, int nparts, long part_stride,
+                          const int* row_map) {
   if (!input || !output || !scale || !bias || !residual)
     return lsh_fail(LSH_ERR_INVALID, "ker_residual_bias_ln_i32I: null pointer");
   // the kernel only reads `residual`; output may alias it (the reference calls it in place)
   return launch_ln<T, int32_t, kLnResOut>(input, const_cast<T*>(residual), output, nullptr, scale,
                                           bias, nullptr, colsum, batch_tokens, hidden_size,
-                                          dequant_scale, 0.f, 0, stream, nparts, part_stride);
+                                          dequant_scale, 0.f, 0, stream, nparts, part_stride, false,
+                                          row_map);
 }
 
 #define LSH_INST(T)                                                                              \
   template int norm_layer_resual_i8O<T>(int, int, hipStream_t, T*, int8_t*, const T*, const T*,  \
-                                        const T*, float, bool);                                  \
+                                        const T*, float, bool, bool);                            \
   template int residual_bias_ln_i8O<T, int8_t>(const int8_t*, const T*, const T*, const T*,      \
                                                int8_t*, T*, int, int, float, float, hipStream_t, \
-                                               bool, const T*, int, long);                       \
+                                               bool, const T*, int, long, bool);                 \
   template int residual_bias_ln_i8O<T, int32_t>(const int32_t*, const T*, const T*, const T*,    \
                                                 int8_t*, T*, int, int, float, float,             \
-                                                hipStream_t, bool, const T*, int, long);         \
+                                                hipStream_t, bool, const T*, int, long, bool);   \
   template int residual_bias_ln_i32I<T>(const int32_t*, const T*, const T*, const T*, T*, int,   \
-                                        int, float, hipStream_t, const T*, int, long);
+                                        int, float, hipStream_t, const T*, int, long, const int*);
 LSH_INST(float)
 LSH_INST(__half)
 #undef LSH_INST

@@ -126,11 +126,14 @@ ln_rows8_row(int row, bool live, int sub, const AccT* __restrict__ gemm_out, T* 
              int8_t* __restrict__ out_q, const T* __restrict__ scale, const T* __restrict__ bias,
              const T* __restrict__ residual_bias, const T* __restrict__ colsum, int hidden,
              float dequant_scale, float quant_scale, int is_post_ln, int nparts, long part_stride,
-             const half8_t* pre_res = nullptr, int dead_row = 0) {
+             const half8_t* pre_res = nullptr, int dead_row = 0, int blocked = 0, int in_row = -1) {
   // pre_res (fp16 only): the lane's ITER residual chunks, already loaded by the caller.
   // dead_row: the row whose addresses a lane without a row reads (and drops); a caller that
   // hands over a staged tile names a row of the tile.
-  const long base = (long)(live ? row : dead_row) * hidden;
+  // blocked: out_q is a blocked matrix.  in_row: the row of gemm_out and residual that row `row` of
+  // out_t is made from, where that is another one (kLnResOut).
+  const long base = (long)(live ? (in_row >= 0 ? in_row : row) : dead_row) * hidden;
+  const long out_base = (long)row * hidden;
 
   float x[ITER][8];
   // Every load of the row -- parameters, residual, accumulator, column sums -- is requested
@@ -247,14 +250,14 @@ ln_rows8_row(int row, bool live, int sub, const AccT* __restrict__ gemm_out, T* 
       for (int k = 0; k < 8; ++k)
         o[k] = (x[it][k] - mean) * rstd * TT<T>::safe(gs[it][k]) + TT<T>::safe(bs[it][k]);
       if (MODE == kLnResOut) {
-        st8(out_t, base + e, o);
+        st8(out_t, out_base + e, o);
       } else {
         uint2 packed;
         packed.x = pack4_i8(float2int8(o[0], quant_scale), float2int8(o[1], quant_scale),
                             float2int8(o[2], quant_scale), float2int8(o[3], quant_scale));
         packed.y = pack4_i8(float2int8(o[4], quant_scale), float2int8(o[5], quant_scale),
                             float2int8(o[6], quant_scale), float2int8(o[7], quant_scale));
-        *reinterpret_cast<uint2*>(out_q + base + e) = packed;
+        *reinterpret_cast<uint2*>(out_q + code_offset(row, e, hidden, blocked)) = packed;
         float w[8];
 #pragma unroll
         for (int k = 0; k < 8; ++k) {

@@ -136,6 +136,20 @@ __device__ __forceinline__ int unpack_i8(uint32_t w, int i) {
   return (int)(int8_t)((w >> (8 * i)) & 0xff);
 }
 
+// Blocked layout of a matrix with K bytes per row (int8: K columns, fp16: K / 2), K % 64 == 0:
+// blocks of 16 rows x 64 bytes, 1 KB each, [rows / 16][K / 64]; inside a block the four 16-byte
+// quarters of the 64 bytes one after the other, each with its 16 rows: byte lane * 16 of a block
+// is what lane `lane` of a wavefront holds of a 16x16x64 (int8) or 16x16x32 (fp16) MFMA fragment.
+// A matrix occupies whole blocks (rows rounded up to 16).
+__host__ __device__ __forceinline__ long blocked_offset(long row, int k, int K) {
+  return ((row >> 4) * (K >> 6) + (k >> 6)) * 1024 + ((k >> 4) & 3) * 256 + (row & 15) * 16 +
+         (k & 15);
+}
+// where the code of (row, column k) of an int8 matrix of `hidden` columns goes: blocked or row-major
+__device__ __forceinline__ long code_offset(long row, int k, int hidden, int blocked) {
+  return blocked ? blocked_offset(row, k, hidden) : row * hidden + k;
+}
+
 // ---- vector views ------------------------------------------------------------
 struct __align__(8) half4_t {
   __half v[4];

@@ -57,7 +57,7 @@ int bias_relu_i8I_i8O(int tokens, hipStream_t s, const int8_t* input, int8_t* ou
 template <typename T>
 int norm_layer_resual_i8O(int token_num, int hidden_size, hipStream_t stream, T* input,
                           int8_t* output, const T* scale, const T* bias, const T* residual_bias,
-                          float quant_scale, bool is_post_ln);
+                          float quant_scale, bool is_post_ln, bool blocked = false);
 // launch_dec_emb_i8I (vocabulary-major table) followed by norm_layer_resual_i8O under an
 // LnFewRowsScope, in one launch: residual receives what the layer norm leaves there, out_q its
 // int8 codes.  hidden % 4 == 0, hidden <= 1024.
@@ -67,23 +67,25 @@ int gpt_emb_step_norm_layer_i8O(const int8_t* token_emb, const T* pos_emb, const
                                 const T* residual_bias, int* real_seq_len, int* zero_flag,
                                 int batch_size, int hidden, int vocab, int padding_id, int pos,
                                 int max_step, float dequant_scale, float quant_scale,
-                                bool is_post_ln, hipStream_t s);
+                                bool is_post_ln, hipStream_t s, bool blocked = false);
 template <typename T>
 int dec_emb_norm_layer_i8O(const int8_t* token_emb, const T* pos_emb, const int* tokens,
                            T* residual, int8_t* out_q, const T* scale, const T* bias,
                            const T* residual_bias, int rows, int hidden, int vocab, int step,
                            int max_step, float dequant_scale, bool scaled, float quant_scale,
-                           bool is_post_ln, hipStream_t s);
+                           bool is_post_ln, hipStream_t s, bool blocked = false);
 template <typename T, typename AccT>
 int residual_bias_ln_i8O(const AccT* input, const T* scale, const T* bias, const T* residual_bias,
                          int8_t* output, T* residual, int batch_tokens, int hidden_size,
                          float dequant_scale, float quant_scale, hipStream_t stream,
-                         bool is_post_ln, const T* colsum, int nparts = 1, long part_stride = 0);
+                         bool is_post_ln, const T* colsum, int nparts = 1, long part_stride = 0,
+                         bool blocked = false);
+// row_map (optional): row r of output is made from row row_map[r] of input and residual
 template <typename T>
 int residual_bias_ln_i32I(const int32_t* input, const T* scale, const T* bias, const T* residual,
                           T* output, int batch_tokens, int hidden_size, float dequant_scale,
                           hipStream_t stream, const T* colsum, int nparts = 1,
-                          long part_stride = 0);
+                          long part_stride = 0, const int* row_map = nullptr);
 // `nparts` > 1: `input` holds that many int32 accumulator planes `part_stride` elements apart
 // (split-K GEMM output, gemm_i8_i32o_splitk) which are summed before the dequantisation.
 //
@@ -130,8 +132,6 @@ int enc_emb_i8I(const int8_t* token_emb, const T* pos_emb, const int* tokens, T*
 // [N, K] int8 -> the 16-row x 64-byte MFMA-ordered tiling the fused kernel streams
 int tile_weight_16x64(const int8_t* w, int8_t* tiled, int N, int K, hipStream_t s);
 bool gemm_ln_fused_supported(int hidden, int K);
-// the next fused launch of this thread records its own begin / end timestamps into the events
-void gemm_ln_time_next_launch(hipEvent_t start, hipEvent_t stop);
 // output / residual as residual_bias_ln_i8O would leave them after gemm_i8_i8o(A, W, alpha)
 template <typename T>
 int gemm_i8_residual_ln_i8O(const int8_t* A, const int8_t* w_tiled, float alpha, const T* scale,
@@ -166,6 +166,37 @@ int qkv_attention_i8(const int8_t* x, const int8_t* qkv_weight, const __half* qk
                      const int* pad_mask, int8_t* ctx_q, float requant_alpha, float dequant_scale,
                      float quant_scale, int batch, int seq_len, int head_num, int dim_per_head,
                      hipStream_t s, const int* plan = nullptr);
+
+// ---- sequences without their padding (enc_pack_kernels.hip) ---------------------------------
+// The rows of a batch that are computed: the tokens of every sequence up to its last one that is
+// not padding, one sequence after the other, and one row that stands for all the padding behind
+// them (its embedding is zero and so is its context, so every padded row of a stack comes out
+// the same).  EncPack is the device memory of one plan.
+struct EncPack {
+  int* seq;      // [2 * batch + 1]: first row and length of a sequence; the padding's row, or -1
+  int* row_map;  // [batch * seq_len]: the row that position (b, s) is computed in
+  int* items;    // [batch * heads]: work items of the fused QKV + attention kernel, or null
+};
+bool enc_pack_supported(int batch, int seq_len, int head_num);
+// Fills the plan from the token ids.  host_rows (optional, pinned): receives `ticket` << 32 | number
+// of rows, for a host that waits for this plan.
+int enc_pack_plan(const int* tokens, int padding_id, const EncPack& pack, int batch, int seq_len,
+                  int head_num, unsigned long long* host_rows, unsigned ticket, hipStream_t s);
+// launch_enc_emb_i8I into the rows of the plan; pad_mask keeps its [batch, seq_len] form
+int enc_emb_packed(const int8_t* token_emb, const __half* pos_emb, const int* tokens, __half* output,
+                   int* pad_mask, int padding_id, const EncPack& pack, int batch, int seq_len,
+                   int hidden, hipStream_t s, float dequant_scale, bool scaled, int vocab_size);
+// qkv_attention_i8 on packed rows with blocked x, qkv_weight and ctx_q
+int qkv_attention_packed(const int8_t* x, const int8_t* qkv_weight, const __half* qkv_bias,
+                         const int* pad_mask, int8_t* ctx_q, float requant_alpha,
+                         float dequant_scale, float quant_scale, int batch, int seq_len, int head_num,
+                         int dim_per_head, hipStream_t s, const EncPack& pack);
+// encself_attention_i8qkv on packed rows (row-major QKV codes) with a blocked ctx_q
+int encself_attention_packed(const int8_t* qkv, const __half* qkv_bias, float dequant_scale,
+                             const int* pad_mask, int8_t* ctx_q, float quant_scale, int batch,
+                             int seq_len, int head_num, int dim_per_head, hipStream_t s,
+                             const EncPack& pack);
+
 // The plan of such launches (batch * head_num ints, made once per padding mask): workgroups take
 // their (sequence, head) pairs longest sequence first, paired on a compute unit with the
 // shortest, and leave out the 32-token blocks that hold nothing but padding.  Same bytes on
@@ -235,6 +266,30 @@ const char* gemm_i8_act_epilogue_name(int act);
 // The next int8 GEMM launched from this thread records kernel-exact begin / end
 // timestamps into the two events (hipExtLaunchKernelGGL), then the hook clears itself.
 void gemm_i8_time_next_launch(hipEvent_t start, hipEvent_t stop);
+// hands over (and clears) what it was given; false when nothing was
+bool gemm_take_timing_events(hipEvent_t* start, hipEvent_t* stop);
+
+// ---- products on blocked operands (gemm_blocked.hip) ----------------------------------------
+// A [M, K] and W [N, K] int8 in the blocked layout (blocked_offset in ls_device.h), both allocated
+// in whole blocks of 16 rows.  K % 64 == 0, N % 4 == 0.  C is row-major but for gemm_blk_lut,
+// whose int8 output is blocked again (N % 64 == 0).
+int block_rows(const void* in, void* out, int rows, int row_bytes, bool back, hipStream_t s);
+int gemm_blk_i8o(const int8_t* A, const int8_t* W, int8_t* C, int M, int N, int K, float alpha,
+                 hipStream_t s);
+int gemm_blk_i32o(const int8_t* A, const int8_t* W, int32_t* C, int M, int N, int K, int ksplit,
+                  hipStream_t s);
+int gemm_blk_preferred_ksplit(int M, int N, int K);
+int gemm_blk_lut(const int8_t* A, const int8_t* W, int8_t* C, const int8_t* lut, int M, int N, int K,
+                 float alpha, hipStream_t s);
+int gemm_blk_decself_qkv(const int8_t* A, const int8_t* W, const __half* qkv_bias, int8_t* new_q,
+                         int8_t* new_k, int8_t* new_v, int step_token_num, int hidden, int K,
+                         int head_num, int max_step, int step_id, float alpha, float dequant_scale,
+                         float quant_scale, hipStream_t s);
+int gemm_blk_encdec_q(const int8_t* A, const int8_t* W, const __half* q_bias, __half* new_q,
+                      int step_token_num, int hidden, int K, int beam_size, int head_num, float alpha,
+                      float dequant_scale, hipStream_t s);
+// the kernel the dispatch picks (profiles)
+const char* gemm_blk_kernel_name(int M, int N, int K, bool table);
 // Counts the changes of the process-wide route switches below (tile kernel, decode-step
 // kernel, fused decode attention, activation table kernel).  Whoever keeps launches recorded
 // (the models' step graphs) compares it with the value it recorded under and drops what it

@@ -93,6 +93,18 @@ class HostIds {
   int* p_ = nullptr;
 };
 
+// A pointer that is set for the length of a call.
+class HostIdsScope {
+ public:
+  HostIdsScope(const int*& slot, const int* ids) : slot_(slot) { slot_ = ids; }
+  ~HostIdsScope() { slot_ = nullptr; }
+  HostIdsScope(const HostIdsScope&) = delete;
+  HostIdsScope& operator=(const HostIdsScope&) = delete;
+
+ private:
+  const int*& slot_;
+};
+
 // A HIP stream of the default priority that is destroyed with its owner.
 class StreamOwner {
  public:
@@ -313,6 +325,21 @@ inline DeviceBuffer<int8_t> upload_kernel(const std::vector<uint8_t>& w, int row
   LSH_CALL(lsh::stored_u8_to_i8(raw.get(), q.get(), rows, cols, transpose, s));
   CHECK_GPU_ERROR(hipStreamSynchronize(s));
   return q;
+}
+
+// row-major int8 [n, k] -> blocked; the row-major copy is released
+inline DeviceBuffer<int8_t> block_weight(DeviceBuffer<int8_t>& w, int n, int k, hipStream_t s) {
+  DeviceBuffer<int8_t> b((size_t)(n + 15) / 16 * 16 * k);
+  LSH_CALL(lsh::block_rows(w.get(), b.get(), n, k, false, s));
+  CHECK_GPU_ERROR(hipStreamSynchronize(s));
+  w = DeviceBuffer<int8_t>();
+  return b;
+}
+inline DeviceBuffer<int8_t> unblock_weight(const DeviceBuffer<int8_t>& b, int n, int k, hipStream_t s) {
+  DeviceBuffer<int8_t> w((size_t)n * k);
+  LSH_CALL(lsh::block_rows(b.get(), w.get(), n, k, true, s));
+  CHECK_GPU_ERROR(hipStreamSynchronize(s));
+  return w;
 }
 
 }  // namespace hip

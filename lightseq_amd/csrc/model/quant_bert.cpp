@@ -41,7 +41,7 @@ void QuantBert::infer(void* host_out, bool host_f16) {
   if (input_shapes_[0].size() != 2) throw std::runtime_error("token_ids must be 2-D");
   int batch_size = input_shapes_[0][0], seq_len = input_shapes_[0][1];
   auto run = [&] {
-    encoder_->run_one_infer(batch_size, seq_len);
+    encoder_->run_one_infer(batch_size, seq_len, host_ids_);
     if (host_out) {
       const long n = (long)batch_size * seq_len * tw_._hidden_size;
       if (host_f16) LSH_CALL(lsh::copy_words(encoder_->_p_d_output, host_out, n / 2, stream_));
@@ -65,6 +65,7 @@ void QuantBert::InferHost(const int* ids, int batch, int seq_len, void* host_out
     h_ids_.upload(ids, n, d_input_.get(), d_input_.size(), stream_);
   set_input_ptr(0, d_input_.get());
   set_input_shape(0, {batch, seq_len});
+  HostIdsScope scope(host_ids_, ids);
   infer(host_out, host_f16);
 }
 

@@ -29,6 +29,7 @@ class QuantBert : public LSModel {
   // owners first: released after the encoder, also when the constructor throws half way
   StreamOwner stream_;
   HostIds h_ids_;
+  const int* host_ids_ = nullptr;  // the ids of an InferHost() call under way
   DeviceBuffer<int> d_input_, d_padding_mask_;
   DeviceBuffer<__half> d_encoder_output_;
   std::shared_ptr<QuantBertEncoder> encoder_;

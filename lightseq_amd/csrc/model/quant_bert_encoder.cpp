@@ -43,7 +43,14 @@ std::string QuantBertEncoder::check() {
 
 void QuantBertEncoder::init_buffer() {
   const int H = _tw._hidden_size, I = _tw._inner_size;
-  const long tokens = (long)_max_batch_size * _tw._max_step;
+  // blocked matrices occupy whole blocks of 16 rows
+  const long tokens = ((long)_max_batch_size * _tw._max_step + 15) / 16 * 16;
+  _blockable = H % 64 == 0 && I % 64 == 0;
+  _pack_seq.alloc(2 * (size_t)_max_batch_size + 1);
+  _pack_map.alloc(tokens);
+  _residual.alloc((size_t)tokens * H);
+  CHECK_GPU_ERROR(hipHostMalloc(reinterpret_cast<void**>(&_h_pack_rows), sizeof(unsigned long long)));
+  *_h_pack_rows = 0;
   _qkv_buf.alloc((size_t)(3 * _max_batch_dim));
   const size_t wide = (size_t)tokens * std::max(I, 3 * H);
   _int8_ffn_in_buf.alloc(wide);
@@ -77,12 +84,15 @@ void QuantBertEncoder::init_buffer() {
     d.b_ffn2 = upload_half(w.ffn_second_bias, _stream);
     d.w_qkv = upload_kernel(w.multihead_project_kernel_qkv, H, 3 * H, true, _stream);
     d.w_out = upload_kernel(w.multihead_project_kernel_output, H, H, true, _stream);
-    if (gemm_ln_fused_supported(H, H)) {
-      d.w_out_tiled.alloc((size_t)H * H);
-      LSH_CALL(tile_weight_16x64(d.w_out.get(), d.w_out_tiled.get(), H, H, _stream));
-    }
     d.w_ffn1 = upload_kernel(w.ffn_first_kernel, H, I, true, _stream);
     d.w_ffn2 = upload_kernel(w.ffn_second_kernel, I, H, true, _stream);
+    if (_blockable) {
+      // the blocked form is the one kept; ensure_row_major_weights() brings the other back
+      d.qkv_blk = block_weight(d.w_qkv, 3 * H, H, _stream);
+      d.out_blk = block_weight(d.w_out, H, H, _stream);
+      d.ffn1_blk = block_weight(d.w_ffn1, I, H, _stream);
+      d.ffn2_blk = block_weight(d.w_ffn2, H, I, _stream);
+    }
     {
       // table of the FFN1 epilogue (dequantise, bias, activation, requantise) per output code
       const float* c = &_enc_clip_max[l * _tw._clip_stride];
@@ -123,16 +133,16 @@ void QuantBertEncoder::reset_profile() {
 
 void QuantBertEncoder::prof_begin(int site, int m, int n, int k, const char* epilogue) {
   if (!_profiling) return;
-  const bool fused_ln = std::string(epilogue) == "fused_ln";
   const bool fused_qa = std::string(epilogue) == "fused_qkv_attn";
   const bool segment = std::string(epilogue) == "ffn_segment";
+  const bool blocked = std::string(epilogue) == "blocked";
   SiteProfile& p = _profile[site];
   if (p.m != m || p.n != n || p.k != k || p.kernel.empty() || p.route != epilogue) {
     p.m = m; p.n = n; p.k = k;
     p.route = epilogue;
-    p.kernel = fused_ln   ? "gemm_ln_rows16_kernel"
-               : fused_qa ? "qkv_attn_kernel"
+    p.kernel = fused_qa   ? "qkv_attn_kernel"
                : segment  ? "ffn_segment_kernel"
+               : blocked  ? gemm_blk_kernel_name(m, n, k, site == 2)
                           : gemm_i8_kernel_name(m, n, k, epilogue);
   }
   Pending pe;
@@ -146,8 +156,7 @@ void QuantBertEncoder::prof_begin(int site, int m, int n, int k, const char* epi
     }
   }
   // the launcher records the kernel's own begin / end timestamps into the events
-  if (fused_ln) gemm_ln_time_next_launch(pe.e0, pe.e1);
-  else if (fused_qa) qkv_attention_time_next_launch(pe.e0, pe.e1);
+  if (fused_qa) qkv_attention_time_next_launch(pe.e0, pe.e1);
   else if (segment) ffn_segment_time_next_launch(pe.e0, pe.e1);
   else gemm_i8_time_next_launch(pe.e0, pe.e1);
   _pending.push_back(pe);
@@ -166,6 +175,7 @@ void QuantBertEncoder::collect_profile() {
 }
 
 QuantBertEncoder::~QuantBertEncoder() {
+  if (_h_pack_rows) (void)hipHostFree(_h_pack_rows);
   ffn_segment_release(this);
   if (_h_seg_error) (void)hipHostFree(_h_seg_error);
 }
@@ -190,7 +200,122 @@ void QuantBertEncoder::tap(int8_t* dst, const int8_t* src, size_t n) {
     CHECK_GPU_ERROR(hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToDevice, _stream));
 }
 
-void QuantBertEncoder::run_one_infer(int batch_size, int batch_seq_len) {
+// Everything but the taps' bisection and the opt-in feed-forward segment, which work on row-major
+// tensors of the padded shape.
+bool QuantBertEncoder::packed_route() const {
+  const bool tapped = taps.ln1_q || taps.qkv_q || taps.ctx_q || taps.out_q || taps.ln2_q || taps.ffn1_q ||
+                      taps.act_q || taps.ffn2_acc || taps.res_attn || taps.res_ffn;
+  return _fuse && _blockable && !tapped && !ffn_segment_enabled() && qkv_attention_plan_enabled() &&
+         enc_pack_supported(_batch_size, _batch_seq_len, _tw._head_num);
+}
+
+void QuantBertEncoder::ensure_row_major_weights() {
+  const int H = _tw._hidden_size, I = _tw._inner_size;
+  if (!_blockable || _layers.empty() || _layers[0].w_qkv.get()) return;
+  for (Layer& d : _layers) {
+    d.w_qkv = unblock_weight(d.qkv_blk, 3 * H, H, _stream);
+    d.w_out = unblock_weight(d.out_blk, H, H, _stream);
+    d.w_ffn1 = unblock_weight(d.ffn1_blk, I, H, _stream);
+    d.w_ffn2 = unblock_weight(d.ffn2_blk, H, I, _stream);
+  }
+}
+
+// Rows of the plan: counted from the ids where the caller has them, otherwise as the plan kernel
+// reports them.  That kernel is the first of the call, so while this waits the launches behind
+// it (embedding, first layer norm, first attention) keep the GPU busy.
+int QuantBertEncoder::packed_rows(const int* host_token_ids) {
+  if (host_token_ids) {
+    int rows = 0;
+    bool padded = false;
+    for (int b = 0; b < _batch_size; ++b) {
+      const int* row = host_token_ids + (size_t)b * _batch_seq_len;
+      int len = _batch_seq_len;
+      while (len > 0 && row[len - 1] == _tw._padding_id) --len;
+      rows += len;
+      padded |= len < _batch_seq_len;
+    }
+    return rows + (padded ? 1 : 0);
+  }
+  const volatile unsigned long long* p = _h_pack_rows;
+  for (long spin = 0; spin < (1L << 22); ++spin)
+    if ((unsigned)(*p >> 32) == _pack_ticket) return (int)(unsigned)*p;
+  CHECK_GPU_ERROR(hipStreamSynchronize(_stream));
+  if ((unsigned)(*p >> 32) != _pack_ticket) throw std::runtime_error("the packing plan did not run");
+  return (int)(unsigned)*p;
+}
+
+void QuantBertEncoder::run_packed(const int* host_token_ids) {
+  const int H = _tw._hidden_size, I = _tw._inner_size, B = _batch_size, S = _batch_seq_len;
+  const int h = _tw._head_num, dph = _tw._dim_per_head, post = _tw._is_post_ln;
+  const float Q = _quant_range;
+  const bool qkv_fused = qkv_attention_fused_supported(B, S, h, dph);
+  const EncPack pack{_pack_seq.get(), _pack_map.get(), qkv_fused ? _qa_plan.get() : nullptr};
+  LSH_CALL(enc_pack_plan(_p_d_token_id, _tw._padding_id, pack, B, S, h,
+                         host_token_ids ? nullptr : _h_pack_rows, ++_pack_ticket, _stream));
+  LSH_CALL(enc_emb_packed(_int8_emb.get(), _pos_emb.get(), _p_d_token_id, _residual.get(),
+                          _p_d_padding_mask, _tw._padding_id, pack, B, S, H, _stream,
+                          _src_emb_clip_max / Q, _tw._scale_embedding, _tw._src_vocab_size));
+  int8_t *a = _int8_ffn_in_buf.get(), *b = _int8_ffn_out_buf.get();
+  __half* res = _residual.get();
+  // until the number of rows is known, launches cover the most there can be
+  int M = host_token_ids ? packed_rows(host_token_ids) : _batch_token_num;
+  bool known = host_token_ids != nullptr;
+  auto rows = [&] {
+    if (!known) M = packed_rows(nullptr);
+    known = true;
+    return M;
+  };
+  for (_layer_id = 0; _layer_id < _tw._n_enc_layer; _layer_id++) {
+    const Layer& w = _layers[_layer_id];
+    const float* c = &_enc_clip_max[_layer_id * _tw._clip_stride];
+    if (_layer_id == 0)
+      LSH_CALL(norm_layer_resual_i8O<__half>(M, H, _stream, res, a, w.ln1_scale.get(), w.ln1_bias.get(),
+                                             w.b_out.get(), Q / c[4], post, true));
+    // QKV product and attention: one kernel per (sequence, head) for short sequences, else the
+    // product's codes and an attention that dequantises them
+    int8_t* ctx = b;
+    if (qkv_fused) {
+      prof_begin(0, _batch_token_num, 3 * H, H, "fused_qkv_attn");
+      LSH_CALL(qkv_attention_packed(a, w.qkv_blk.get(), w.b_qkv.get(), _p_d_padding_mask, ctx,
+                                    c[0] * c[4] / (c[8] * Q), c[8] / Q, Q / c[5], B, S, h, dph, _stream,
+                                    pack));
+      std::swap(a, b);
+    } else {
+      prof_begin(0, rows(), 3 * H, H, "blocked");
+      LSH_CALL(gemm_blk_i8o(a, w.qkv_blk.get(), b, rows(), 3 * H, H, c[0] * c[4] / (c[8] * Q), _stream));
+      ctx = a;
+      LSH_CALL(encself_attention_packed(b, w.b_qkv.get(), c[8] / Q, _p_d_padding_mask, ctx, Q / c[5], B, S,
+                                        h, dph, _stream, pack));
+    }
+    // `a` holds the context
+    prof_begin(1, rows(), H, H, "blocked");
+    LSH_CALL(gemm_blk_i8o(a, w.out_blk.get(), b, M, H, H, c[1] * c[5] / (c[9] * Q), _stream));
+    LSH_CALL((residual_bias_ln_i8O<__half, int8_t>(b, w.ln2_scale.get(), w.ln2_bias.get(), w.b_ffn2.get(),
+                                                   a, res, M, H, c[9] / Q, Q / c[6], _stream, post, nullptr,
+                                                   1, 0, true)));
+    prof_begin(2, M, I, H, "blocked");
+    LSH_CALL(gemm_blk_lut(a, w.ffn1_blk.get(), b, w.ffn1_act_lut.get(), M, I, H,
+                          c[2] * c[6] / (c[10] * Q), _stream));
+    prof_begin(3, M, H, I, "blocked");
+    LSH_CALL(gemm_blk_i32o(b, w.ffn2_blk.get(), _int32_ffn_out_buf.get(), M, H, I, 1, _stream));
+    const float dequant_scale = _tw._use_gelu ? c[3] * c[7] / (Q * Q) : c[3] * c[7] / (2 * Q * Q);
+    const __half* colsum = w.ffn2_colsum.get();  // nullptr for GELU models
+    if (_layer_id == _tw._n_enc_layer - 1) {
+      // every position of the padded shape from the row it was computed in
+      LSH_CALL(residual_bias_ln_i32I<__half>(_int32_ffn_out_buf.get(), _final_ln_scale.get(),
+                                             _final_ln_bias.get(), res, _p_d_output, _batch_token_num, H,
+                                             dequant_scale, _stream, colsum, 1, 0, pack.row_map));
+    } else {
+      const Layer& nx = _layers[_layer_id + 1];
+      const float clip_next = _enc_clip_max[(_layer_id + 1) * _tw._clip_stride + 4];
+      LSH_CALL((residual_bias_ln_i8O<__half, int32_t>(
+          _int32_ffn_out_buf.get(), nx.ln1_scale.get(), nx.ln1_bias.get(), nx.b_out.get(), a, res, M, H,
+          dequant_scale, Q / clip_next, _stream, post, colsum, 1, 0, true)));
+    }
+  }
+}
+
+void QuantBertEncoder::run_one_infer(int batch_size, int batch_seq_len, const int* host_token_ids) {
   if (batch_size > _max_batch_size)
     throw std::runtime_error("batch size of input greater than max_batch_size");
   if (batch_seq_len > _tw._max_step)
@@ -199,6 +324,12 @@ void QuantBertEncoder::run_one_infer(int batch_size, int batch_seq_len) {
   _batch_size = batch_size;
   _batch_seq_len = batch_seq_len;
   _batch_token_num = batch_size * batch_seq_len;
+  if (packed_route()) {
+    _seg_active = false;
+    run_packed(host_token_ids);
+    return;
+  }
+  ensure_row_major_weights();
 
   LSH_CALL(enc_emb_i8I<__half>(_int8_emb.get(), _pos_emb.get(), _p_d_token_id, _p_d_output,
                                _p_d_padding_mask, _tw._padding_id, batch_size, batch_seq_len,
@@ -279,32 +410,18 @@ void QuantBertEncoder::self_attention() {
   }
   tap(taps.ctx_q, _int8_ffn_in_buf.get(), (size_t)M * H);
 
-  const bool tap_out = (taps.out_q || taps.res_attn) && taps.tap_layer == _layer_id;
-  if (_fuse && !tap_out && w.w_out_tiled.get() != nullptr) {
-    // out-projection + dequant + residual + LayerNorm + quant in one kernel: the int8 product
-    // never reaches memory.  Same bytes as the pair below; reads _int8_ffn_in_buf (context codes)
-    // and must not overwrite it, so the LayerNorm output goes to _int8_ffn_out_buf and the two
-    // buffers swap roles.
-    prof_begin(1, M, H, H, "fused_ln");
-    LSH_CALL(gemm_i8_residual_ln_i8O<__half>(
-        _int8_ffn_in_buf.get(), w.w_out_tiled.get(), c[1] * c[5] / (c[9] * Q), w.ln2_scale.get(),
-        w.ln2_bias.get(), w.b_ffn2.get(), _int8_ffn_out_buf.get(), _p_d_output, M, H, H, c[9] / Q,
-        Q / c[6], _stream, _tw._is_post_ln));
-    std::swap(_int8_ffn_in_buf, _int8_ffn_out_buf);
-  } else {
-    prof_begin(1, M, H, H, "EpiI8");
-    LSH_CALL(gemm_i8_i8o(_int8_ffn_in_buf.get(), w.w_out.get(), _int8_ffn_out_buf.get(), M, H, H,
-                         c[1] * c[5] / (c[9] * Q), _stream));
-    tap(taps.out_q, _int8_ffn_out_buf.get(), (size_t)M * H);
+  prof_begin(1, M, H, H, "EpiI8");
+  LSH_CALL(gemm_i8_i8o(_int8_ffn_in_buf.get(), w.w_out.get(), _int8_ffn_out_buf.get(), M, H, H,
+                       c[1] * c[5] / (c[9] * Q), _stream));
+  tap(taps.out_q, _int8_ffn_out_buf.get(), (size_t)M * H);
 
-    if (taps.res_attn && taps.tap_layer == _layer_id)
-      CHECK_GPU_ERROR(hipMemcpyAsync(taps.res_attn, _p_d_output, (size_t)M * H * sizeof(__half),
-                                     hipMemcpyDeviceToDevice, _stream));
-    LSH_CALL((residual_bias_ln_i8O<__half, int8_t>(
-        _int8_ffn_out_buf.get(), w.ln2_scale.get(), w.ln2_bias.get(), w.b_ffn2.get(),
-        _int8_ffn_in_buf.get(), _p_d_output, M, H, c[9] / Q, Q / c[6], _stream, _tw._is_post_ln,
-        nullptr)));
-  }
+  if (taps.res_attn && taps.tap_layer == _layer_id)
+    CHECK_GPU_ERROR(hipMemcpyAsync(taps.res_attn, _p_d_output, (size_t)M * H * sizeof(__half),
+                                   hipMemcpyDeviceToDevice, _stream));
+  LSH_CALL((residual_bias_ln_i8O<__half, int8_t>(
+      _int8_ffn_out_buf.get(), w.ln2_scale.get(), w.ln2_bias.get(), w.b_ffn2.get(),
+      _int8_ffn_in_buf.get(), _p_d_output, M, H, c[9] / Q, Q / c[6], _stream, _tw._is_post_ln,
+      nullptr)));
   tap(taps.ln2_q, _int8_ffn_in_buf.get(), (size_t)M * H);
 }
 

@@ -24,7 +24,8 @@ class QuantBertEncoder {
   ~QuantBertEncoder();
   void init_buffer();
   std::string check();
-  void run_one_infer(int batch_size, int batch_seq_len);
+  // host_token_ids (optional): the same ids in host memory, where the caller has them
+  void run_one_infer(int batch_size, int batch_seq_len, const int* host_token_ids = nullptr);
   // After the stream has been synchronised: true when the run has to be repeated (a kernel that
   // waits for workgroups of its own launch gave up; the encoder has switched that route off).
   bool finish_infer();
@@ -62,6 +63,11 @@ class QuantBertEncoder {
  private:
   void self_attention();
   void ffn_add_norm();
+  // the route of every call without taps: blocked operands, no rows for padding
+  bool packed_route() const;
+  void run_packed(const int* host_token_ids);
+  int packed_rows(const int* host_token_ids);
+  void ensure_row_major_weights();
   void tap(int8_t* dst, const int8_t* src, size_t n);
   // event bracket around one GEMM launch of `site` (0 qkv, 1 out, 2 ffn1, 3 ffn2)
   void prof_begin(int site, int m, int n, int k, const char* epilogue);
@@ -94,12 +100,19 @@ class QuantBertEncoder {
   DeviceBuffer<int32_t> _int32_ffn_out_buf;
   DeviceBuffer<int> _qa_plan;      // plan of the fused QKV + attention launches of a call
   const int* _qa_plan_cur = nullptr;  // ... when this call has one
+  // packed route
+  bool _blockable = false;  // widths that block (multiples of 64)
+  DeviceBuffer<int> _pack_seq, _pack_map;
+  DeviceBuffer<__half> _residual;  // residual stream of the packed rows
+  unsigned long long* _h_pack_rows = nullptr;  // pinned: ticket << 32 | rows of the plan
+  unsigned _pack_ticket = 0;
   // weights
   DeviceBuffer<int8_t> _int8_emb;                       // [vocab, H]
   DeviceBuffer<__half> _pos_emb, _final_ln_scale, _final_ln_bias;
   struct Layer {
-    DeviceBuffer<int8_t> w_qkv, w_out, w_ffn1, w_ffn2;  // [N, K] int8
-    DeviceBuffer<int8_t> w_out_tiled;  // w_out in 16 x 64 MFMA tiles (fused out-projection + LN)
+    // [N, K] int8: row-major where the widths do not block or a route with taps has asked for it
+    DeviceBuffer<int8_t> w_qkv, w_out, w_ffn1, w_ffn2;
+    DeviceBuffer<int8_t> qkv_blk, out_blk, ffn1_blk, ffn2_blk;  // ... blocked
     DeviceBuffer<int8_t> ffn1_act_lut;  // [inner, 256]: bias + activation + requant per code
     DeviceBuffer<__half> ln1_scale, ln1_bias, b_qkv, b_out, ln2_scale, ln2_bias, b_ffn1, b_ffn2,
         ffn2_colsum;

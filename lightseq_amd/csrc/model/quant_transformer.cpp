@@ -50,7 +50,7 @@ void QuantTransformer::Infer() {
   if (input_shapes_[0].size() != 2) throw std::runtime_error("source_ids must be 2-D");
   int batch_size = input_shapes_[0][0], seq_len = input_shapes_[0][1];
   if (tw_._multilg_type != 0) throw std::runtime_error("multilingle not supported");
-  encoder_->run_one_infer(batch_size, seq_len);
+  encoder_->run_one_infer(batch_size, seq_len, host_ids_);
   if (enc_out_tap_)
     CHECK_GPU_ERROR(hipMemcpyAsync(enc_out_tap_, d_encoder_output_.get(),
                                    (size_t)batch_size * seq_len * tw_._hidden_size * sizeof(__half),
@@ -58,7 +58,7 @@ void QuantTransformer::Infer() {
   decoder_->run_one_infer(batch_size, seq_len);
   CHECK_GPU_ERROR(hipStreamSynchronize(stream_));
   if (encoder_->finish_infer()) {  // an encoder route gave up and was switched off: once more
-    encoder_->run_one_infer(batch_size, seq_len);
+    encoder_->run_one_infer(batch_size, seq_len, host_ids_);
     decoder_->run_one_infer(batch_size, seq_len);
     CHECK_GPU_ERROR(hipStreamSynchronize(stream_));
     encoder_->finish_infer();
@@ -82,6 +82,7 @@ void QuantTransformer::InferHost(const int* ids, int batch, int seq_len, void* h
     h_ids_.upload(ids, n, d_input_.get(), d_input_.size(), stream_);
   set_input_ptr(0, d_input_.get());
   set_input_shape(0, {batch, seq_len});
+  HostIdsScope scope(host_ids_, ids);
   Infer();
 }
 

@@ -36,6 +36,7 @@ class QuantTransformer : public LSModel {
   // and are released when the constructor throws half way (unsupported files are common)
   StreamOwner stream_;
   HostIds h_ids_;
+  const int* host_ids_ = nullptr;  // the ids of an InferHost() call under way
   DeviceBuffer<int> d_input_, d_padding_mask_, d_output_;
   DeviceBuffer<__half> d_encoder_output_;
   std::shared_ptr<QuantBertEncoder> encoder_;

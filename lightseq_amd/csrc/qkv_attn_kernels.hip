@@ -40,11 +40,15 @@ constexpr int kQaNst = 2;
 // the pair of its index and the blocks up to the sequence length of the call.
 constexpr int kQaItemHeadShift = 16, kQaItemBlocksShift = 28;
 
+// PK: x, the weights and ctx_q are blocked matrices and the rows are those of an EncPack plan (`seq`:
+// first row and length of a sequence, the padding's row at seq[2 * batch]), whose items `plan` is.
+template <bool PK>
 __global__ void __launch_bounds__(256, 2)
 qkv_attn_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W,
                 const _Float16* __restrict__ bias, const int* __restrict__ pad_mask,
                 const int* __restrict__ plan, int8_t* __restrict__ ctx_q, float requant_alpha,
-                float dq, float quant_scale, float alpha, int S, int batch, int head_num, int K) {
+                float dq, float quant_scale, float alpha, int S, int batch, int head_num, int K,
+                const int* __restrict__ seq) {
   constexpr int D = kQaD, WGN = 2, MB = 2, NB = 3, NWV = 4, TM = kQaTM, TN = kQaTN;
   constexpr int STAGE = kQaStage, NST = kQaNst;
   constexpr int NA = TM / 8 / NWV, NW = TN / 8 / NWV;  // 1-KB loads per wavefront
@@ -74,7 +78,21 @@ qkv_attn_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W,
   const int hidden = head_num * D;
   const int nk = K / kBK;
   const int qi = wave * 32 + l32;  // the lane's query in the attention (wavefront w: block w)
-  int8_t* out_row = ctx_q + ((long)b * S + qi) * hidden + head * D;
+  int row0 = b * S, len = S;
+  if constexpr (PK) {
+    row0 = __builtin_amdgcn_readfirstlane(seq[2 * b]);
+    len = __builtin_amdgcn_readfirstlane(seq[2 * b + 1]);
+    const int pad_row = __builtin_amdgcn_readfirstlane(seq[2 * batch]);
+    // the context of the padding's row, once per head
+    if (b == 0 && pad_row >= 0 && tid < 4)
+      *reinterpret_cast<uint4*>(ctx_q + blocked_offset(pad_row, head * D + tid * 16, hidden)) =
+          make_uint4(0, 0, 0, 0);
+    if (nblk == 0) return;
+  }
+  // where the lane's context codes go: 16-byte chunk c at c * out_chunk
+  const int out_chunk = PK ? 256 : 16;
+  int8_t* out_row = PK ? ctx_q + blocked_offset(row0 + qi, head * D, hidden)
+                       : ctx_q + ((long)b * S + qi) * hidden + head * D;
   if (nblk == 0) {
     // nothing but padding: the context of a padded query is zero
     if (qi < S) {
@@ -86,8 +104,8 @@ qkv_attn_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W,
   }
 
   // padding flags of keys `lane` and `64 + lane` (requested first, used after the product)
-  const int pm0 = pad_mask[(long)b * S + min(lane, S - 1)];
-  const int pm1 = pad_mask[(long)b * S + min(lane + 64, S - 1)];
+  const int pm0 = pad_mask[(long)b * S + min(lane, len - 1)];
+  const int pm1 = pad_mask[(long)b * S + min(lane + 64, len - 1)];
 
   // Rows of the tile beyond block nblk are padding: they are not loaded, multiplied, converted
   // or attended.  Wavefront (wm, wn) owns the row blocks wm and wm + 2, so that the blocks that
@@ -99,7 +117,14 @@ qkv_attn_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W,
     const int row = (wave + NWV * i) * 8 + (lane >> 3);  // row block i of the tile
     const int c = (lane & 7) ^ key_act(row);
     // tokens past the end of the sequence read its last token and are zeroed in step 2
-    a_src[i] = (uint32_t)(b * S + min(row, S - 1)) * (uint32_t)K + c * 16;
+    a_src[i] = (uint32_t)(row0 + min(row, len - 1)) * (uint32_t)K + c * 16;
+    if constexpr (PK) {
+      // 16 tokens x 64 bytes per load, in fragment order (tile_gemm); the sequence starts at any
+      // row of a block, so the 16 rows lie in two
+      const int q = wave + NWV * i;
+      a_src[i] = (uint32_t)blocked_offset(row0 + min((q >> 1) * 16 + (lane & 15), len - 1),
+                                          (q & 1) * 64 + (lane >> 4) * 16, K);
+    }
   }
 #pragma unroll
   for (int i = 0; i < NW; ++i) {
@@ -107,7 +132,13 @@ qkv_attn_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W,
     const int c = (lane & 7) ^ key_wgt(row);
     // tile column `row`: part row / 64 (q, k, v), dimension row % 64 of this head
     w_src[i] = (uint32_t)((row >> 6) * hidden + head * D + (row & 63)) * (uint32_t)K + c * 16;
+    if constexpr (PK) {
+      const int q = wave + NWV * i, rb = q >> 1;  // rows 16 rb .. of the tile
+      w_src[i] = (uint32_t)((rb >> 2) * hidden + head * D + (rb & 3) * 16) * (uint32_t)K + (q & 1) * 1024 +
+                 (lane ^ (rb & 1) * 8) * 16;
+    }
   }
+  constexpr int KSTEP = PK ? 2048 : kBK;
   const uint32_t lds0 = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)smem);
   auto dma1 = [&](const int8_t* base, uint32_t voff, uint32_t lds) {
     lds = __builtin_amdgcn_readfirstlane(lds);
@@ -119,23 +150,28 @@ qkv_attn_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W,
     const uint32_t base = lds0 + slot * STAGE;
 #pragma unroll
     for (int i = 0; i < NA; ++i)
-      if (i < nblk) dma1(A + kt * kBK, a_src[i], base + (wave + NWV * i) * 1024);
+      if (i < nblk) dma1(A + kt * KSTEP, a_src[i], base + (wave + NWV * i) * 1024);
 #pragma unroll
     for (int i = 0; i < NW; ++i)
-      dma1(W + kt * kBK, w_src[i], base + TM * kBK + (wave + NWV * i) * 1024);
+      dma1(W + kt * KSTEP, w_src[i], base + TM * kBK + (wave + NWV * i) * 1024);
   };
   // LDS byte offset of this lane's fragment chunk for K slice 0; slice ks is at (offset ^ (ks << 5))
   int a_base[MB], w_base[NB];
 #pragma unroll
   for (int i = 0; i < MB; ++i) {
     const int row = (wm + 2 * i) * 32 + l32;
-    a_base[i] = row * kBK + ((g ^ key_act(row)) << 4);
+    a_base[i] = PK ? (row >> 4) * 2048 + g * 256 + (row & 15) * 16
+                   : row * kBK + ((g ^ key_act(row)) << 4);
   }
 #pragma unroll
   for (int j = 0; j < NB; ++j) {
     const int row = wn * (NB * 32) + j * 32 + sigma(l32);
-    w_base[j] = TM * kBK + row * kBK + ((g ^ key_wgt(row)) << 4);
+    w_base[j] = TM * kBK + (PK ? (row >> 4) * 2048 + g * 256 + ((row & 15) ^ ((row >> 4) & 1) * 8) * 16
+                               : row * kBK + ((g ^ key_wgt(row)) << 4));
   }
+  auto slice_at = [&](int base, int ks) {
+    return PK ? base + (ks >> 1) * 1024 + (ks & 1) * 512 : base ^ (ks << 5);
+  };
   struct Frag {
     v4i a[MB], w[NB];
   };
@@ -148,11 +184,11 @@ qkv_attn_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W,
     auto load_frag = [&](Frag& f, const int8_t* stage, int ks) {
 #pragma unroll
       for (int i = 0; i < LB; ++i)
-        f.a[i] = *reinterpret_cast<const v4i*>(stage + (a_base[i] ^ (ks << 5)));
+        f.a[i] = *reinterpret_cast<const v4i*>(stage + slice_at(a_base[i], ks));
       if (LB > 0) {
 #pragma unroll
         for (int j = 0; j < NB; ++j)
-          f.w[j] = *reinterpret_cast<const v4i*>(stage + (w_base[j] ^ (ks << 5)));
+          f.w[j] = *reinterpret_cast<const v4i*>(stage + slice_at(w_base[j], ks));
       }
     };
     // the first products of the tile start from a zero that is an operand of the instruction,
@@ -240,7 +276,7 @@ qkv_attn_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W,
       v8h lo, hi;
       requant_dequant16_bias(acc[i][j], requant_alpha, bias + part * hidden + head * D + d0, dq, lo,
                              hi);
-      if (t >= S) lo = hi = (v8h)(_Float16)0;
+      if (t >= len) lo = hi = (v8h)(_Float16)0;
       if (part == 2) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -258,8 +294,8 @@ qkv_attn_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W,
 
   // ---- step 3: attention; wavefront w owns queries 32 w .. 32 w + 31 ----
   if (wave >= nblk) {
-    // queries that are all padding: zeros
-    if (qi < S) {
+    // queries that are all padding: zeros (they have no row of their own on packed rows)
+    if (!PK && qi < S) {
       uint4* o = reinterpret_cast<uint4*>(out_row + g * 32);
       o[0] = make_uint4(0, 0, 0, 0);
       o[1] = make_uint4(0, 0, 0, 0);
@@ -270,21 +306,21 @@ qkv_attn_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W,
 #pragma unroll
   for (int ks = 0; ks < D / 16; ++ks)
     qreg[ks] = *reinterpret_cast<const v8h*>(&Qs[qi * KSTR + ks * 16 + g * 8]);
-  const bool padk0 = pm0 != 0 || lane >= S, padk1 = pm1 != 0 || lane + 64 >= S;
+  const bool padk0 = pm0 != 0 || lane >= len, padk1 = pm1 != 0 || lane + 64 >= len;
   const uint64_t pad_q = __ballot(wave < 2 ? padk0 : padk1);
-  const bool q_pad = qi >= S || ((pad_q >> ((wave & 1) * 32 + l32)) & 1) != 0;
+  const bool q_pad = qi >= len || ((pad_q >> ((wave & 1) * 32 + l32)) & 1) != 0;
   if (nblk >= 4)
-    attend_block128<D, 4>(Ks, Vt, qreg, padk0, padk1, q_pad, qi < S, alpha, quant_scale, nullptr,
-                          out_row, l32, g);
+    attend_block128<D, 4>(Ks, Vt, qreg, padk0, padk1, q_pad, qi < len, alpha, quant_scale, nullptr,
+                          out_row, l32, g, out_chunk);
   else if (nblk == 3)
-    attend_block128<D, 3>(Ks, Vt, qreg, padk0, padk1, q_pad, qi < S, alpha, quant_scale, nullptr,
-                          out_row, l32, g);
+    attend_block128<D, 3>(Ks, Vt, qreg, padk0, padk1, q_pad, qi < len, alpha, quant_scale, nullptr,
+                          out_row, l32, g, out_chunk);
   else if (nblk == 2)
-    attend_block128<D, 2>(Ks, Vt, qreg, padk0, padk1, q_pad, qi < S, alpha, quant_scale, nullptr,
-                          out_row, l32, g);
+    attend_block128<D, 2>(Ks, Vt, qreg, padk0, padk1, q_pad, qi < len, alpha, quant_scale, nullptr,
+                          out_row, l32, g, out_chunk);
   else
-    attend_block128<D, 1>(Ks, Vt, qreg, padk0, padk1, q_pad, qi < S, alpha, quant_scale, nullptr,
-                          out_row, l32, g);
+    attend_block128<D, 1>(Ks, Vt, qreg, padk0, padk1, q_pad, qi < len, alpha, quant_scale, nullptr,
+                          out_row, l32, g, out_chunk);
 }
 
 // ---------------------------------------------------------------------------------
@@ -380,10 +416,11 @@ int qkv_attention_plan(const int* pad_mask, int* plan, int batch, int seq_len, i
   return lsh_check_launch("qkv_attn_plan_kernel");
 }
 
-int qkv_attention_i8(const int8_t* x, const int8_t* qkv_weight, const __half* qkv_bias,
+template <bool PK>
+static int launch_qkv_attention(const int8_t* x, const int8_t* qkv_weight, const __half* qkv_bias,
                      const int* pad_mask, int8_t* ctx_q, float requant_alpha, float dequant_scale,
                      float quant_scale, int batch, int seq_len, int head_num, int dim_per_head,
-                     hipStream_t s, const int* plan) {
+                     hipStream_t s, const int* plan, const int* seq) {
   if (!x || !qkv_weight || !qkv_bias || !pad_mask || !ctx_q || batch <= 0 || seq_len <= 0 ||
       head_num <= 0)
     return lsh_fail(LSH_ERR_INVALID, "qkv_attention_i8: bad arguments");
@@ -402,7 +439,7 @@ int qkv_attention_i8(const int8_t* x, const int8_t* qkv_weight, const __half* qk
     if (lsh_check_hip(hipGetDevice(&dev), "hipGetDevice")) return LSH_ERR_HIP;
     std::lock_guard<std::mutex> lock(mu);
     if (dev >= 64 || !((raised >> dev) & 1)) {
-      if (lsh_check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(qkv_attn_kernel),
+      if (lsh_check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(PK ? qkv_attn_kernel<true> : qkv_attn_kernel<false>),
                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem),
                         "hipFuncSetAttribute(qkv_attn_kernel)"))
         return LSH_ERR_HIP;
@@ -415,12 +452,32 @@ int qkv_attention_i8(const int8_t* x, const int8_t* qkv_weight, const __half* qk
   g_qa_ev_start = g_qa_ev_stop = nullptr;
   if (plan != nullptr && !qkv_attention_plan_supported(batch, seq_len, head_num))
     return lsh_fail(LSH_ERR_INVALID, "qkv_attention_i8: this shape has no plan");
-  hipExtLaunchKernelGGL(qkv_attn_kernel, dim3(batch * head_num), dim3(256), smem, s, e0, e1, 0, x,
+  hipExtLaunchKernelGGL(qkv_attn_kernel<PK>, dim3(batch * head_num), dim3(256), smem, s, e0, e1, 0, x,
                         qkv_weight, reinterpret_cast<const _Float16*>(qkv_bias), pad_mask, plan,
                         ctx_q,
                         requant_alpha, dequant_scale, quant_scale, alpha, seq_len, batch, head_num,
-                        hidden);
+                        hidden, seq);
   return lsh_check_launch("qkv_attn_kernel");
+}
+
+int qkv_attention_i8(const int8_t* x, const int8_t* qkv_weight, const __half* qkv_bias,
+                     const int* pad_mask, int8_t* ctx_q, float requant_alpha, float dequant_scale,
+                     float quant_scale, int batch, int seq_len, int head_num, int dim_per_head,
+                     hipStream_t s, const int* plan) {
+  return launch_qkv_attention<false>(x, qkv_weight, qkv_bias, pad_mask, ctx_q, requant_alpha,
+                                     dequant_scale, quant_scale, batch, seq_len, head_num,
+                                     dim_per_head, s, plan, nullptr);
+}
+
+int qkv_attention_packed(const int8_t* x, const int8_t* qkv_weight, const __half* qkv_bias,
+                         const int* pad_mask, int8_t* ctx_q, float requant_alpha,
+                         float dequant_scale, float quant_scale, int batch, int seq_len, int head_num,
+                         int dim_per_head, hipStream_t s, const EncPack& pack) {
+  if (!pack.seq || !pack.items)
+    return lsh_fail(LSH_ERR_INVALID, "qkv_attention_packed: needs a plan with items");
+  return launch_qkv_attention<true>(x, qkv_weight, qkv_bias, pad_mask, ctx_q, requant_alpha,
+                                    dequant_scale, quant_scale, batch, seq_len, head_num, dim_per_head,
+                                    s, pack.items, pack.seq);
 }
 
 }  // namespace lsh

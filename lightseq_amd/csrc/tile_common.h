@@ -162,7 +162,7 @@ __device__ __forceinline__ uint32_t float2int8_pack4(float x0, float x1, float x
 // at: a masked key's probability is exactly zero, so leaving its block out changes nothing).
 // qreg[ks]: d = ks * 16 + g * 8 .. + 8 of the lane's query.  q_pad: the query is padding (its
 // context is zero).  out_h / out_q: where the D context values of the lane's query go (fp16 /
-// int8 codes), or null; nothing is stored when `live` is false.
+// int8 codes, whose 16-byte chunks are out_chunk bytes apart), or null; nothing is stored when `live` is false.
 constexpr int attn_kstr(int D) { return D + 8; }  // halfs per K row in LDS
 constexpr int kAttnVstr = 128 + 4;                // halfs per V^T row in LDS
 
@@ -171,7 +171,7 @@ __device__ __forceinline__ void attend_block128(const _Float16* Ks, const _Float
                                                 const v8h (&qreg)[D / 16], bool padk0, bool padk1,
                                                 bool q_pad, bool live, float alpha,
                                                 float quant_scale, __half* out_h, int8_t* out_q,
-                                                int l32, int g) {
+                                                int l32, int g, int out_chunk = 16) {
   constexpr int KSTR = attn_kstr(D), VSTR = kAttnVstr;
   v16f sc[NKB];
   {
@@ -294,7 +294,7 @@ __device__ __forceinline__ void attend_block128(const _Float16* Ks, const _Float
       if (out_q != nullptr) {
         // a padded query gives zeros, whose code is 0
         const uint32_t w4 = float2int8_pack4(o[0], o[1], o[2], o[3], quant_scale);
-        *reinterpret_cast<uint32_t*>(out_q + dd) = q_pad ? 0u : w4;
+        *reinterpret_cast<uint32_t*>(out_q + (dd >> 4) * out_chunk + (dd & 15)) = q_pad ? 0u : w4;
       }
     }
   }

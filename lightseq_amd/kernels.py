@@ -813,6 +813,46 @@ def gemm_i8_lut_i8o(a, w, c, lut, m, n, k, alpha):
     call("lsh_gemm_i8_lut_i8o", ptr(a), ptr(w), ptr(c), ptr(lut), m, n, k, alpha, current_stream())
 
 
+def block_rows(x, back_rows=None):
+    """A 2-D tensor (row bytes a multiple of 64) in the blocked layout, as a flat int8 tensor of
+    whole 16-row blocks; with ``back_rows = (rows, columns, dtype)`` the other way round."""
+    if back_rows is None:
+        _dev(x)
+        rows, nbytes = x.shape[0], x.shape[1] * x.element_size()
+        out = torch.empty((rows + 15) // 16 * 16 * nbytes, dtype=torch.int8, device=x.device)
+    else:
+        rows, cols, dtype = back_rows
+        out = torch.empty(rows, cols, dtype=dtype, device=x.device)
+        nbytes = cols * out.element_size()
+    call("lsh_block_rows", ptr(x), ptr(out), rows, nbytes, int(back_rows is not None), current_stream())
+    return out
+
+
+def gemm_i8_blocked_i8o(a, w, c, m, n, k, alpha):
+    call("lsh_gemm_i8_blocked_i8o", ptr(a), ptr(w), ptr(c), m, n, k, alpha, current_stream())
+
+
+def gemm_i8_blocked_i32o(a, w, c, m, n, k, ksplit=1):
+    call("lsh_gemm_i8_blocked_i32o", ptr(a), ptr(w), ptr(c), m, n, k, ksplit, current_stream())
+
+
+def gemm_i8_blocked_lut_i8o(a, w, c, lut, m, n, k, alpha):
+    call("lsh_gemm_i8_blocked_lut_i8o", ptr(a), ptr(w), ptr(c), ptr(lut), m, n, k, alpha, current_stream())
+
+
+def gemm_i8_blocked_decself_qkv_i8o(a, w, qkv_bias, new_q, new_k, new_v, step_token_num, hidden, k,
+                                    head_num, max_step, step_id, alpha, dequant_scale, quant_scale):
+    call("lsh_gemm_i8_blocked_decself_qkv_i8o_f16", ptr(a), ptr(w), ptr(qkv_bias), ptr(new_q), ptr(new_k),
+         ptr(new_v), step_token_num, hidden, k, head_num, max_step, step_id, alpha, dequant_scale,
+         quant_scale, current_stream())
+
+
+def gemm_i8_blocked_encdec_q(a, w, q_bias, new_q, step_token_num, hidden, k, beam_size, head_num,
+                                 alpha, dequant_scale):
+    call("lsh_gemm_i8_blocked_encdec_q_f16", ptr(a), ptr(w), ptr(q_bias), ptr(new_q), step_token_num, hidden,
+         k, beam_size, head_num, alpha, dequant_scale, current_stream())
+
+
 class FfnSegmentSync:
     """Barrier counters, error word and launch count of ``ffn_segment_i8`` (one per caller)."""
 

@@ -60,6 +60,12 @@ _SIGNATURES = {
     "lsh_gemm_i8_encdec_q_f16": (False, "pppp" + "iiiii" + "ff" + "s"),
     "lsh_gpt_emb_step_norm_layer_i8O_f16": (False, "pppppppppp" + "iiiiii" + "ffi" + "s"),
     "lsh_dec_emb_norm_layer_i8O_f16": (False, "pppppppp" + "iiiii" + "fifi" + "s"),
+    "lsh_block_rows": (False, "ppiiis"),
+    "lsh_gemm_i8_blocked_i8o": (False, "pppiiifs"),
+    "lsh_gemm_i8_blocked_i32o": (False, "pppiiiis"),
+    "lsh_gemm_i8_blocked_lut_i8o": (False, "pppp" + "iiif" + "s"),
+    "lsh_gemm_i8_blocked_decself_qkv_i8o_f16": (False, "pppppp" + "iiiiii" + "fff" + "s"),
+    "lsh_gemm_i8_blocked_encdec_q_f16": (False, "pppp" + "iiiii" + "ff" + "s"),
     "lsh_gemm_i8_i32o_splitk": (False, "ppp" + "iiii" + "p" + "s"),
     "lsh_gemm_i8_preferred_ksplit": (False, "iii"),
     "lsh_layer_norm_row_kernel": (False, "i"),
