@@ -520,7 +520,7 @@ constexpr int kNoCand = 0x7fffffff;
 
 template <typename T>
 __global__ void __launch_bounds__(1024)
-beam_topk_kernel(const int8_t* __restrict__ logits, const T* __restrict__ logit_bias,
+beam_topk_kernel(const int8_t* __restrict__ logits, long ldl, const T* __restrict__ logit_bias,
                  const float* __restrict__ seq_probs, const float* __restrict__ seq_score,
                  const int* __restrict__ alive_seq, float dq, float* __restrict__ top_score,
                  int* __restrict__ top_idx, int vocab, int max_step, float length_norm,
@@ -542,7 +542,7 @@ beam_topk_kernel(const int8_t* __restrict__ logits, const T* __restrict__ logit_
     }
     return;
   }
-  const int8_t* lr = logits + (long)row * vocab;
+  const int8_t* lr = logits + row * ldl;
   const RowStats st = row_stats(lr, logit_bias, vocab, dq, 0, 0, red);
   const float base = seq_probs[row] - logf(st.sum_exp) - st.max_logit;
   ScoreIdx prev;
@@ -583,7 +583,7 @@ beam_topk_kernel(const int8_t* __restrict__ logits, const T* __restrict__ logit_
 // difference of the log-sum-exp, shared by all candidates of the row).
 template <typename T, bool VEC>
 __global__ void __launch_bounds__(1024)
-beam_topk_reg_kernel(const int8_t* __restrict__ logits, const T* __restrict__ logit_bias,
+beam_topk_reg_kernel(const int8_t* __restrict__ logits, long ldl, const T* __restrict__ logit_bias,
                      const float* __restrict__ seq_probs, const float* __restrict__ seq_score,
                      const int* __restrict__ alive_seq, float dq, float* __restrict__ top_score,
                      int* __restrict__ top_idx, int vocab, int max_step, float length_norm,
@@ -606,7 +606,7 @@ beam_topk_reg_kernel(const int8_t* __restrict__ logits, const T* __restrict__ lo
     }
     return;
   }
-  const int8_t* lr = logits + (long)row * vocab;
+  const int8_t* lr = logits + row * ldl;
   float lg[NI];
   auto id_of = [&](int i) { return VEC ? (i >> 4) * 16384 + 16 * t + (i & 15) : t + 1024 * i; };
   if (VEC) {
@@ -748,7 +748,7 @@ constexpr int kBeamPartIds = 8192;  // ids of a part, at most (a multiple of 16:
 
 template <typename T>
 __global__ void __launch_bounds__(512)
-beam_topk_part_kernel(const int8_t* __restrict__ logits, const T* __restrict__ logit_bias,
+beam_topk_part_kernel(const int8_t* __restrict__ logits, long ldl, const T* __restrict__ logit_bias,
                       const float* __restrict__ seq_probs, const float* __restrict__ seq_score,
                       const int* __restrict__ alive_seq, float dq, float* __restrict__ top_score,
                       int* __restrict__ top_idx, int vocab, int max_step, float length_norm,
@@ -778,7 +778,7 @@ beam_topk_part_kernel(const int8_t* __restrict__ logits, const T* __restrict__ l
   float all[4][16];
 #pragma unroll
   for (int p = 0; p < 4; ++p)
-    beam_part_load(logits + (long)row * vocab, logit_bias, p * kBeamPartIds,
+    beam_part_load(logits + row * ldl, logit_bias, p * kBeamPartIds,
                    min((p + 1) * kBeamPartIds, vocab), dq, all[p]);
   float tmax = kFloatInfNeg;
 #pragma unroll
@@ -1037,7 +1037,7 @@ int beam_search_step_i8I(const int8_t* logits, const T* logit_bias, float* seq_p
                          float* top_score, int* top_idx, int* parent, int* num_finished,
                          float dequant_scale, int vocab_size, int max_step, float length_norm,
                          int cur_step, int batch_size, int beam_size, int end_id, hipStream_t s,
-                         float* part_ws, size_t part_ws_words) {
+                         float* part_ws, size_t part_ws_words, int logits_stride) {
   if (!logits || !logit_bias || !seq_probs || !seq_score || !old_alive_seq || !new_alive_seq ||
       !top_score || !top_idx || !parent || !num_finished || vocab_size <= 0 || batch_size <= 0 ||
       max_step <= 0 || cur_step < 0 || cur_step + 1 >= max_step)
@@ -1048,7 +1048,9 @@ int beam_search_step_i8I(const int8_t* logits, const T* logit_bias, float* seq_p
     return lsh_fail(LSH_ERR_INVALID, "beam_search_step: the sequence buffers must differ");
   if ((long)beam_size * vocab_size > 0x7ffffffe)
     return lsh_fail(LSH_ERR_UNSUPPORTED, "beam_search_step: beam_size * vocab_size overflows");
-  const bool vec = vocab_size % 16 == 0 &&
+  const long ldl = logits_stride ? logits_stride : vocab_size;
+  if (ldl < vocab_size) return lsh_fail(LSH_ERR_INVALID, "beam_search_step: rows overlap");
+  const bool vec = vocab_size % 16 == 0 && ldl % 16 == 0 &&
                    ((reinterpret_cast<uintptr_t>(logits) | reinterpret_cast<uintptr_t>(logit_bias)) &
                     15u) == 0;
   const int rows = batch_size * beam_size;
@@ -1061,22 +1063,22 @@ int beam_search_step_i8I(const int8_t* logits, const T* logit_bias, float* seq_p
     float* p_score = part_ws;
     int* p_idx = reinterpret_cast<int*>(p_score + (size_t)rows * parts * beam_size);
     beam_topk_part_kernel<T><<<dim3(parts, rows), 512, 0, s>>>(
-        logits, logit_bias, seq_probs, seq_score, old_alive_seq, dequant_scale, p_score, p_idx,
+        logits, ldl, logit_bias, seq_probs, seq_score, old_alive_seq, dequant_scale, p_score, p_idx,
         vocab_size, max_step, length_norm, cur_step, beam_size, end_id, num_finished);
     if (int rc = lsh_check_launch("beam_topk_part_kernel")) return rc;
     top_score = p_score;
     top_idx = p_idx;
   } else if (vocab_size <= 32 * 1024 && vec)
     beam_topk_reg_kernel<T, true><<<batch_size * beam_size, 1024, 0, s>>>(
-        logits, logit_bias, seq_probs, seq_score, old_alive_seq, dequant_scale, top_score,
+        logits, ldl, logit_bias, seq_probs, seq_score, old_alive_seq, dequant_scale, top_score,
         top_idx, vocab_size, max_step, length_norm, cur_step, beam_size, end_id, num_finished);
   else if (vocab_size <= 32 * 1024)
     beam_topk_reg_kernel<T, false><<<batch_size * beam_size, 1024, 0, s>>>(
-        logits, logit_bias, seq_probs, seq_score, old_alive_seq, dequant_scale, top_score,
+        logits, ldl, logit_bias, seq_probs, seq_score, old_alive_seq, dequant_scale, top_score,
         top_idx, vocab_size, max_step, length_norm, cur_step, beam_size, end_id, num_finished);
   else
     beam_topk_kernel<T><<<batch_size * beam_size, 1024, 0, s>>>(
-        logits, logit_bias, seq_probs, seq_score, old_alive_seq, dequant_scale, top_score,
+        logits, ldl, logit_bias, seq_probs, seq_score, old_alive_seq, dequant_scale, top_score,
         top_idx, vocab_size, max_step, length_norm, cur_step, beam_size, end_id, num_finished);
   if (int rc = lsh_check_launch("beam_topk_kernel")) return rc;
   beam_merge_kernel<<<batch_size < 1024 ? batch_size : 1024, 64, 0, s>>>(top_score, top_idx, old_alive_seq, new_alive_seq,
@@ -1087,10 +1089,10 @@ int beam_search_step_i8I(const int8_t* logits, const T* logit_bias, float* seq_p
 }
 template int beam_search_step_i8I<float>(const int8_t*, const float*, float*, float*, const int*,
                                          int*, float*, int*, int*, int*, float, int, int, float,
-                                         int, int, int, int, hipStream_t, float*, size_t);
+                                         int, int, int, int, hipStream_t, float*, size_t, int);
 template int beam_search_step_i8I<__half>(const int8_t*, const __half*, float*, float*, const int*,
                                           int*, float*, int*, int*, int*, float, int, int, float,
-                                          int, int, int, int, hipStream_t, float*, size_t);
+                                          int, int, int, int, hipStream_t, float*, size_t, int);
 
 // ---------------------------------------------------------------------------------
 // The search step for callers that cannot allocate device memory (code under HIP graph

@@ -974,13 +974,13 @@ int lsh_gpt_greedy_step(const int8_t* logits, int* ids, int* last_ids, int vocab
                         int max_step, int cur_len, int batch_size, int* unfinished, int eos_id,
                         lsh_stream_t stream) {
   return gpt_greedy_step(logits, ids, last_ids, vocab_size, max_step, cur_len, batch_size,
-                         unfinished, eos_id, HS(stream));
+                         unfinished, eos_id, HS(stream), vocab_size);
 }
 int lsh_gpt_sample_step(const int8_t* logits, int* ids, int* last_ids, int vocab_size,
                         int max_step, int cur_len, int batch_size, int* unfinished, int eos_id,
                         int k, float p, float dequant_scale, void* state, lsh_stream_t stream) {
   return gpt_sample_step(logits, ids, last_ids, vocab_size, max_step, cur_len, batch_size,
-                         unfinished, eos_id, k, p, dequant_scale, state, HS(stream));
+                         unfinished, eos_id, k, p, dequant_scale, state, HS(stream), vocab_size);
 }
 
 }  // extern "C"

@@ -49,13 +49,14 @@ __host__ __device__ constexpr long decself_group_floats(int step_num) {
 }
 
 // q: the D query codes; kb / vb: the pair's cache rows [max_step][D]; out: where the D context
-// codes go (nothing is stored unless `live`).  lds: decself_group_floats() floats of the group.
+// codes go (nothing is stored unless `live`), 16 codes together and `out_chunk` bytes from one 16 to
+// the next (16: row-major, 256: a blocked matrix, see blocked_offset).  lds: decself_group_floats() floats of the group.
 // wid: wavefront within the group, lane: lane within the wavefront.
 template <int D, int NWV, int UN>
 __device__ __forceinline__ void decself_attend_row_rounds(const int8_t* q, const int8_t* kb,
                                                           const int8_t* vb, int8_t* out, bool live,
-                                                   int step_num, float attn_scale, float dq,
-                                                   float quant_scale, float* lds, int wid,
+                                                   int out_chunk, int step_num, float attn_scale,
+                                                   float dq, float quant_scale, float* lds, int wid,
                                                    int lane) {
 #pragma clang fp contract(off)
   constexpr int CH = D / 16;    // lanes per cache row
@@ -163,7 +164,7 @@ __device__ __forceinline__ void decself_attend_row_rounds(const int8_t* q, const
     for (int st = 1; st < NWV; st *= 2)
 #pragma unroll
       for (int i = 0; i < NWV; i += 2 * st) t[i] += t[i + st];
-    if (live) out[tid] = (int8_t)float2int8(t[0], quant_scale);
+    if (live) out[(tid >> 4) * out_chunk + (tid & 15)] = (int8_t)float2int8(t[0], quant_scale);
   }
 }
 
@@ -203,7 +204,7 @@ __device__ __forceinline__ float byte_to_float(uint32_t w) {
 template <int D, int NWV, int UN>
 __device__ __forceinline__ void decself_attend_row_once_body(uint4 qv, const uint4 (&kv)[UN],
                                                              const uint4 (&vv)[UN], int8_t* out,
-                                                             bool live, int step_num,
+                                                             bool live, int out_chunk, int step_num,
                                                              float attn_scale, float dq,
                                                              float quant_scale, float* lds, int wid,
                                                              int lane);
@@ -232,14 +233,15 @@ __device__ __forceinline__ void decself_attend_load_rows(const int8_t* kb, const
 template <int D, int NWV, int UN>
 __device__ __forceinline__ void decself_attend_row_once(const int8_t* q, const int8_t* kb,
                                                         const int8_t* vb, int8_t* out, bool live,
-                                                        int step_num, float attn_scale, float dq,
+                                                        int out_chunk, int step_num,
+                                                        float attn_scale, float dq,
                                                         float quant_scale, float* lds, int wid,
                                                         int lane) {
   constexpr int CH = D / 16;
   const uint4 qv = *reinterpret_cast<const uint4*>(q + (lane % CH) * 16);
   uint4 kv[UN], vv[UN];
   decself_attend_load_rows<D, NWV, UN>(kb, vb, step_num, wid, lane, kv, vv);
-  decself_attend_row_once_body<D, NWV, UN>(qv, kv, vv, out, live, step_num, attn_scale, dq,
+  decself_attend_row_once_body<D, NWV, UN>(qv, kv, vv, out, live, out_chunk, step_num, attn_scale, dq,
                                            quant_scale, lds, wid, lane);
 }
 
@@ -248,7 +250,7 @@ __device__ __forceinline__ void decself_attend_row_once(const int8_t* q, const i
 template <int D, int NWV, int UN>
 __device__ __forceinline__ void decself_attend_row_once_body(uint4 qv, const uint4 (&kv)[UN],
                                                              const uint4 (&vv)[UN], int8_t* out,
-                                                             bool live, int step_num,
+                                                             bool live, int out_chunk, int step_num,
                                                              float attn_scale, float dq,
                                                              float quant_scale, float* lds, int wid,
                                                              int lane) {
@@ -343,7 +345,7 @@ __device__ __forceinline__ void decself_attend_row_once_body(uint4 qv, const uin
     for (int st = 1; st < 4 * NWV; st *= 2)
 #pragma unroll
       for (int i = 0; i < 4 * NWV; i += 2 * st) t[i] += t[i + st];
-    if (live) out[tid] = (int8_t)float2int8(t[0], quant_scale);
+    if (live) out[(tid >> 4) * out_chunk + (tid & 15)] = (int8_t)float2int8(t[0], quant_scale);
   }
 }
 
@@ -352,14 +354,14 @@ __device__ __forceinline__ void decself_attend_row_once_body(uint4 qv, const uin
 template <int D, int NWV, int UN>
 __device__ __forceinline__ void decself_attend_row(const int8_t* q, const int8_t* kb,
                                                    const int8_t* vb, int8_t* out, bool live,
-                                                   int step_num, float attn_scale, float dq,
-                                                   float quant_scale, float* lds, int wid,
+                                                   int out_chunk, int step_num, float attn_scale,
+                                                   float dq, float quant_scale, float* lds, int wid,
                                                    int lane) {
   if (step_num <= UN * NWV * (64 / (D / 16)))
-    decself_attend_row_once<D, NWV, UN>(q, kb, vb, out, live, step_num, attn_scale, dq,
+    decself_attend_row_once<D, NWV, UN>(q, kb, vb, out, live, out_chunk, step_num, attn_scale, dq,
                                         quant_scale, lds, wid, lane);
   else
-    decself_attend_row_rounds<D, NWV, UN>(q, kb, vb, out, live, step_num, attn_scale, dq,
+    decself_attend_row_rounds<D, NWV, UN>(q, kb, vb, out, live, out_chunk, step_num, attn_scale, dq,
                                           quant_scale, lds, wid, lane);
 }
 

@@ -143,7 +143,8 @@ __global__ void __launch_bounds__(256)
 decself_attn_kernel(int32_t* __restrict__ scores, const int8_t* __restrict__ q,
                     const int8_t* __restrict__ k_cache, const int8_t* __restrict__ v_cache,
                     int8_t* __restrict__ new_v, long bh_total, int step_num, int max_step,
-                    int head_num, int d, float attn_scale, float dq, float quant_scale) {
+                    int head_num, int d, float attn_scale, float dq, float quant_scale,
+                    int blocked) {
 #pragma clang fp contract(off)
   extern __shared__ float probs_all[];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -189,7 +190,7 @@ decself_attn_kernel(int32_t* __restrict__ scores, const int8_t* __restrict__ q,
   for (int dd = lane; dd < d; dd += 64) {
     float acc = 0.f;
     for (int j = 0; j < step_num; ++j) acc += (float)vb[(long)j * d + dd] * probs[j] * dq;
-    new_v[row * ((long)head_num * d) + (long)head * d + dd] = (int8_t)float2int8(acc, quant_scale);
+    new_v[code_offset(row, head * d + dd, head_num * d, blocked)] = (int8_t)float2int8(acc, quant_scale);
   }
 }
 
@@ -206,7 +207,7 @@ __global__ void __launch_bounds__(64 * NWV)
 decself_attn_wg_kernel(const int8_t* __restrict__ q, const int8_t* __restrict__ k_cache,
                        const int8_t* __restrict__ v_cache, int8_t* __restrict__ new_v,
                        int step_num, int max_step, int head_num, float attn_scale, float dq,
-                       float quant_scale) {
+                       float quant_scale, int blocked) {
   extern __shared__ __align__(16) float lds_f[];
   // grid: x = head, y = row (no division before the first load)
   const int head = (int)blockIdx.x;
@@ -214,8 +215,8 @@ decself_attn_wg_kernel(const int8_t* __restrict__ q, const int8_t* __restrict__ 
   const long bh = row * head_num + head;
   decself_attend_row<D, NWV, UN>(q + bh * D, k_cache + bh * (long)max_step * D,
                                  v_cache + bh * (long)max_step * D,
-                                 new_v + row * ((long)head_num * D) + (long)head * D, true, step_num,
-                                 attn_scale, dq, quant_scale, lds_f, threadIdx.x >> 6,
+                                 new_v + code_offset(row, head * D, head_num * D, blocked), true,
+                                 blocked ? 256 : 16, step_num, attn_scale, dq, quant_scale, lds_f, threadIdx.x >> 6,
                                  threadIdx.x & 63);
 }
 
@@ -226,17 +227,22 @@ template <int D, int UN>
 __global__ void __launch_bounds__(256)
 decself_attn_pack_kernel(const int8_t* __restrict__ q, const int8_t* __restrict__ k_cache,
                          const int8_t* __restrict__ v_cache, int8_t* __restrict__ new_v,
-                         long bh_total, int step_num, int max_step, float attn_scale, float dq,
-                         float quant_scale) {
+                         long bh_total, int step_num, int max_step, int head_num, float attn_scale,
+                         float dq, float quant_scale, int blocked) {
   extern __shared__ __align__(16) float lds_f[];
   const int wave = threadIdx.x >> 6;
   const long bh_raw = (long)blockIdx.x * 4 + wave;
   const bool live = bh_raw < bh_total;
   const long bh = live ? bh_raw : bh_total - 1;
-  // new_v is [rows, heads * D] and a pair's D codes sit at bh * D of it
+  // new_v is [rows, heads * D]: row-major, a pair's D codes sit at bh * D of it
+  long at = bh * D;
+  if (blocked) {
+    const int row = (int)(bh / head_num);
+    at = blocked_offset(row, ((int)bh - row * head_num) * D, head_num * D);
+  }
   decself_attend_row_once<D, 1, UN>(q + bh * D, k_cache + bh * (long)max_step * D,
-                                    v_cache + bh * (long)max_step * D, new_v + bh * D, live,
-                                    step_num, attn_scale, dq, quant_scale,
+                                    v_cache + bh * (long)max_step * D, new_v + at, live,
+                                    blocked ? 256 : 16, step_num, attn_scale, dq, quant_scale,
                                     lds_f + wave * decself_group_floats<D, 1>(step_num), 0,
                                     threadIdx.x & 63);
 }
@@ -259,7 +265,7 @@ int decself_scores_i8(const int8_t* q, const int8_t* k_cache, int32_t* scores, i
   if (int rc = decself_check(batch_head_num, step_num, max_step, 1, dim_per_head)) return rc;
   decself_attn_kernel<0><<<(batch_head_num + 3) / 4, 256, 0, s>>>(
       scores, q, k_cache, nullptr, nullptr, batch_head_num, step_num, max_step, 1, dim_per_head,
-      0.f, 0.f, 0.f);
+      0.f, 0.f, 0.f, 0);
   return lsh_check_launch("decself_attn_kernel<0>");
 }
 
@@ -272,16 +278,18 @@ int fuse_softmax_new_value_i32I_i8O(const int32_t* correlation, const int8_t* v,
   if (int rc = decself_check(batch_head_num, step_num, max_step, head_num, dim_per_head)) return rc;
   decself_attn_kernel<1><<<(batch_head_num + 3) / 4, 256, decself_lds(step_num), s>>>(
       const_cast<int32_t*>(correlation), nullptr, nullptr, v, new_v, batch_head_num, step_num,
-      max_step, head_num, dim_per_head, attn_scale, dequant_scale, quant_scale);
+      max_step, head_num, dim_per_head, attn_scale, dequant_scale, quant_scale, 0);
   return lsh_check_launch("decself_attn_kernel<1>");
 }
 
 int decself_attention_i8(const int8_t* q, const int8_t* k_cache, const int8_t* v_cache,
                          int8_t* new_v, int batch_head_num, int step_num, int max_step,
                          int head_num, int dim_per_head, float attn_scale, float dequant_scale,
-                         float quant_scale, hipStream_t s) {
+                         float quant_scale, hipStream_t s, bool blocked) {
   if (!q || !k_cache || !v_cache || !new_v)
     return lsh_fail(LSH_ERR_INVALID, "decself_attention: null pointer");
+  if (blocked && (dim_per_head % 16 != 0 || head_num * dim_per_head % 64 != 0))
+    return lsh_fail(LSH_ERR_UNSUPPORTED, "decself_attention: blocked output of this width");
   if (int rc = decself_check(batch_head_num, step_num, max_step, head_num, dim_per_head)) return rc;
   const bool aligned = ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k_cache) |
                          reinterpret_cast<uintptr_t>(v_cache)) & 15u) == 0;
@@ -301,13 +309,13 @@ int decself_attention_i8(const int8_t* q, const int8_t* k_cache, const int8_t* v
   if (step_num <= 4 * kpw)                                                                       \
     decself_attn_pack_kernel<D, 4>                                                               \
         <<<(batch_head_num + 3) / 4, 256, 4 * decself_group_floats<D, 1>(step_num) * sizeof(float), \
-           s>>>(q, k_cache, v_cache, new_v, batch_head_num, step_num, max_step, attn_scale,      \
-                dequant_scale, quant_scale);                                                     \
+           s>>>(q, k_cache, v_cache, new_v, batch_head_num, step_num, max_step, head_num,        \
+                attn_scale, dequant_scale, quant_scale, blocked);                                                     \
   else                                                                                           \
     decself_attn_pack_kernel<D, 8>                                                               \
         <<<(batch_head_num + 3) / 4, 256, 4 * decself_group_floats<D, 1>(step_num) * sizeof(float), \
-           s>>>(q, k_cache, v_cache, new_v, batch_head_num, step_num, max_step, attn_scale,      \
-                dequant_scale, quant_scale)
+           s>>>(q, k_cache, v_cache, new_v, batch_head_num, step_num, max_step, head_num,        \
+                attn_scale, dequant_scale, quant_scale, blocked)
       if (dim_per_head == 32) { LSH_DECSELF_PACK(32); }
       else if (dim_per_head == 64) { LSH_DECSELF_PACK(64); }
       else { LSH_DECSELF_PACK(128); }
@@ -322,7 +330,7 @@ int decself_attention_i8(const int8_t* q, const int8_t* k_cache, const int8_t* v
   decself_attn_wg_kernel<D, 8, UN>                                                              \
       <<<grid, 512, decself_group_floats<D, 8>(step_num) * sizeof(float), s>>>(                 \
           q, k_cache, v_cache, new_v, step_num, max_step, head_num, attn_scale, dequant_scale,  \
-          quant_scale)
+          quant_scale, blocked)
 #define LSH_DECSELF(D)                                                                          \
   if (wide) {                                                                                   \
     if (un8 <= 3) LSH_DECSELF_WIDE(D, 3);                                                       \
@@ -334,7 +342,7 @@ int decself_attention_i8(const int8_t* q, const int8_t* k_cache, const int8_t* v
     decself_attn_wg_kernel<D, 4, 4>                                                             \
         <<<grid, 256, decself_group_floats<D, 4>(step_num) * sizeof(float), s>>>(               \
         q, k_cache, v_cache, new_v, step_num, max_step, head_num, attn_scale, dequant_scale,    \
-        quant_scale)
+        quant_scale, blocked)
     if (dim_per_head == 32) { LSH_DECSELF(32); }
     else if (dim_per_head == 64) { LSH_DECSELF(64); }
     else { LSH_DECSELF(128); }
@@ -344,7 +352,7 @@ int decself_attention_i8(const int8_t* q, const int8_t* k_cache, const int8_t* v
   }
   decself_attn_kernel<2><<<(batch_head_num + 3) / 4, 256, decself_lds(step_num), s>>>(
       nullptr, q, k_cache, v_cache, new_v, batch_head_num, step_num, max_step, head_num,
-      dim_per_head, attn_scale, dequant_scale, quant_scale);
+      dim_per_head, attn_scale, dequant_scale, quant_scale, blocked);
   return lsh_check_launch("decself_attn_kernel<2>");
 }
 
@@ -487,7 +495,7 @@ encdec_attn_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
                    const __half* __restrict__ v, const int* __restrict__ pad_mask,
                    __half* __restrict__ ctx, int8_t* __restrict__ ctx_q, float quant_scale,
                    long waves_total, int beam_size, int head_num, int seq_len, int d,
-                   float alpha_h) {
+                   float alpha_h, int blocked) {
 #pragma clang fp contract(off)
   extern __shared__ float probs_all[];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -535,7 +543,7 @@ encdec_attn_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
     const float c = TT<__half>::rnd(acc);
     if (ctx) ctx[w * d + dd] = __float2half_rn(c);
     if (ctx_q)
-      ctx_q[row * ((long)head_num * d) + (long)head * d + dd] = (int8_t)float2int8(c, quant_scale);
+      ctx_q[code_offset(row, head * d + dd, head_num * d, blocked)] = (int8_t)float2int8(c, quant_scale);
   }
 }
 
@@ -550,7 +558,7 @@ encdec_attn_vec_kernel(const __half* __restrict__ q, const __half* __restrict__ 
                        const __half* __restrict__ v, const int* __restrict__ pad_mask,
                        __half* __restrict__ ctx, int8_t* __restrict__ ctx_q, float quant_scale,
                        long waves_total, int beam_size, int head_num, int seq_len,
-                       float alpha_h) {
+                       float alpha_h, int blocked) {
 #pragma clang fp contract(off)
   extern __shared__ float probs_all[];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -617,7 +625,7 @@ encdec_attn_vec_kernel(const __half* __restrict__ q, const __half* __restrict__ 
     const float c = TT<__half>::rnd(acc);
     if (ctx) ctx[w * D + dd] = __float2half_rn(c);
     if (ctx_q)
-      ctx_q[row * ((long)head_num * D) + (long)head * D + dd] = (int8_t)float2int8(c, quant_scale);
+      ctx_q[code_offset(row, head * D + dd, head_num * D, blocked)] = (int8_t)float2int8(c, quant_scale);
   }
 }
 
@@ -653,7 +661,7 @@ __global__ void __launch_bounds__(QPROD ? 512 : 256)
 encdec_attn_short_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
                          const __half* __restrict__ v, const int* __restrict__ pad_mask,
                          __half* __restrict__ ctx, int8_t* __restrict__ ctx_q, float quant_scale,
-                         int beam_size, int head_num, int seq_len, float alpha_h,
+                         int beam_size, int head_num, int seq_len, float alpha_h, int blocked,
                          EncdecQProd qp = EncdecQProd{}) {
 #pragma clang fp contract(off)
   constexpr int CH = D / 8;     // lanes per row
@@ -685,15 +693,17 @@ encdec_attn_short_kernel(const __half* __restrict__ q, const __half* __restrict_
       const int KS = qp.hidden >> 6;  // 64-byte K slices (<= 16)
       const int m = lane & 15, kq = lane >> 4;
       // matrix row m: beam m of the sentence (rows beyond the beams repeat the last one)
-      const int8_t* xp = qp.x + (b * beam_size + min(m, beam_size - 1)) * (long)qp.hidden + kq * 16;
+      const long xr = b * beam_size + min(m, beam_size - 1);
+      const int8_t* xp = qp.x + code_offset(xr, kq * 16, qp.hidden, blocked);
       // the row operand: column 16 pw + m of the head
-      const int8_t* wp = qp.W + ((long)head * D + pw * 16 + m) * (long)qp.hidden + kq * 16;
+      const int8_t* wp = qp.W + code_offset((long)head * D + pw * 16 + m, kq * 16, qp.hidden, blocked);
+      const int slice = blocked ? 1024 : 64;  // from one 64-byte slice of a row to the next
       const uint2 braw = *reinterpret_cast<const uint2*>(qp.bias + head * D + pw * 16 + 4 * kq);
       v4i xf[16], wf[16];
 #pragma unroll
-      for (int sl = 0; sl < 16; ++sl) wf[sl] = *reinterpret_cast<const v4i*>(wp + min(sl, KS - 1) * 64);
+      for (int sl = 0; sl < 16; ++sl) wf[sl] = *reinterpret_cast<const v4i*>(wp + min(sl, KS - 1) * slice);
 #pragma unroll
-      for (int sl = 0; sl < 16; ++sl) xf[sl] = *reinterpret_cast<const v4i*>(xp + min(sl, KS - 1) * 64);
+      for (int sl = 0; sl < 16; ++sl) xf[sl] = *reinterpret_cast<const v4i*>(xp + min(sl, KS - 1) * slice);
       __builtin_amdgcn_sched_barrier(0);  // every request of the kernel is out before a product
       v4i acc = (v4i)0;
 #pragma unroll
@@ -801,7 +811,7 @@ encdec_attn_short_kernel(const __half* __restrict__ q, const __half* __restrict_
     const float cv = TT<__half>::rnd(t);
     if (ctx) ctx[w * D + dd] = __float2half_rn(cv);
     if (ctx_q)
-      ctx_q[row * ((long)head_num * D) + (long)head * D + dd] = (int8_t)float2int8(cv, quant_scale);
+      ctx_q[code_offset(row, head * D + dd, head_num * D, blocked)] = (int8_t)float2int8(cv, quant_scale);
   }
 }
 
@@ -817,7 +827,7 @@ int encdec_q_attention_f16(const int8_t* x, const int8_t* q_weight, const __half
                            const __half* k, const __half* v, const int* pad_mask, int8_t* ctx_q,
                            float quant_scale, int batch_size, int beam_size, int head_num,
                            int batch_seq_len, int hidden, float alpha, float dequant_scale,
-                           hipStream_t s) {
+                           hipStream_t s, bool blocked) {
   if (!x || !q_weight || !q_bias || !k || !v || !pad_mask || !ctx_q || batch_size <= 0)
     return lsh_fail(LSH_ERR_INVALID, "encdec_q_attention: bad arguments");
   if (!encdec_q_attention_supported(beam_size, head_num, hidden, batch_seq_len) ||
@@ -838,7 +848,7 @@ int encdec_q_attention_f16(const int8_t* x, const int8_t* q_weight, const __half
 #define LSH_ENCDEC_Q(UN)                                                                     \
   encdec_attn_short_kernel<64, UN, true><<<grid, 512, 0, s>>>(                               \
       nullptr, k, v, pad_mask, nullptr, ctx_q, quant_scale, beam_size, head_num, batch_seq_len, \
-      alpha_h, qp)
+      alpha_h, blocked, qp)
   if (un <= 4) LSH_ENCDEC_Q(4);
   else if (un <= 8) LSH_ENCDEC_Q(8);
   else LSH_ENCDEC_Q(16);
@@ -849,10 +859,12 @@ int encdec_q_attention_f16(const int8_t* x, const int8_t* q_weight, const __half
 int encdec_attention_f16(const __half* q, const __half* k, const __half* v, const int* pad_mask,
                          __half* ctx, int8_t* ctx_q, float quant_scale, int batch_size,
                          int beam_size, int head_num, int batch_seq_len, int dim_per_head,
-                         hipStream_t s) {
+                         hipStream_t s, bool blocked) {
   if (!q || !k || !v || !pad_mask || (!ctx && !ctx_q) || batch_size <= 0 || beam_size <= 0 ||
       head_num <= 0 || batch_seq_len <= 0 || dim_per_head <= 0)
     return lsh_fail(LSH_ERR_INVALID, "encdec_attention: bad arguments");
+  if (blocked && (dim_per_head % 16 != 0 || head_num * dim_per_head % 64 != 0))
+    return lsh_fail(LSH_ERR_UNSUPPORTED, "encdec_attention: blocked output of this width");
   if (batch_seq_len > 4096)
     return lsh_fail(LSH_ERR_UNSUPPORTED, "encdec_attention: source length above 4096");
   const long waves = (long)batch_size * head_num * beam_size;
@@ -870,7 +882,8 @@ int encdec_attention_f16(const __half* q, const __half* k, const __half* v, cons
     const int un = (batch_seq_len + kpw - 1) / kpw;
 #define LSH_ENCDEC_SHORT(D, UN)                                                                   \
   encdec_attn_short_kernel<D, UN><<<grid, 256, 0, s>>>(q, k, v, pad_mask, ctx, ctx_q, quant_scale, \
-                                                       beam_size, head_num, batch_seq_len, alpha_h)
+                                                       beam_size, head_num, batch_seq_len, alpha_h, \
+                                                       blocked)
 #define LSH_ENCDEC_SHORT_D(D)                \
   if (un <= 4) LSH_ENCDEC_SHORT(D, 4);       \
   else if (un <= 8) LSH_ENCDEC_SHORT(D, 8);  \
@@ -886,7 +899,7 @@ int encdec_attention_f16(const __half* q, const __half* k, const __half* v, cons
 #define LSH_ENCDEC(D)                                                                           \
   encdec_attn_vec_kernel<D><<<(int)((waves + 3) / 4), 256, lds, s>>>(                           \
       q, k, v, pad_mask, ctx, ctx_q, quant_scale, waves, beam_size, head_num, batch_seq_len,    \
-      alpha_h)
+      alpha_h, blocked)
     if (dim_per_head == 32) LSH_ENCDEC(32);
     else if (dim_per_head == 64) LSH_ENCDEC(64);
     else LSH_ENCDEC(128);
@@ -895,7 +908,7 @@ int encdec_attention_f16(const __half* q, const __half* k, const __half* v, cons
   }
   encdec_attn_kernel<<<(int)((waves + 3) / 4), 256, lds, s>>>(
       q, k, v, pad_mask, ctx, ctx_q, quant_scale, waves, beam_size, head_num, batch_seq_len,
-      dim_per_head, alpha_h);
+      dim_per_head, alpha_h, blocked);
   return lsh_check_launch("encdec_attn_kernel");
 }
 

@@ -42,7 +42,7 @@ decself_qkv_attn_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__
                         int8_t* v_cache, int8_t* __restrict__ ctx, int rows, int hidden,
                         int head_num, int max_step, int step_id, float alpha, float dequant_scale,
                         float cache_quant_scale, float attn_scale, float cache_dequant_scale,
-                        float ctx_quant_scale) {
+                        float ctx_quant_scale, int blocked_ctx) {
   static_assert(NWV * RG == 8, "8 wavefronts: RG groups of NWV");
   constexpr int D = kDqaD, COLS = kDqaCols;
   extern __shared__ float lds_f[];
@@ -139,8 +139,8 @@ decself_qkv_attn_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__
     const long bh = (long)row * head_num + head;
     decself_attend_row<D, NWV, UN>(new_q + bh * D, k_cache + bh * (long)max_step * D,
                                    v_cache + bh * (long)max_step * D,
-                                   ctx + (long)row * hidden + head * D, row0 + g < rows, step_num,
-                                   attn_scale, cache_dequant_scale, ctx_quant_scale,
+                                   ctx + code_offset(row, head * D, hidden, blocked_ctx), row0 + g < rows,
+                                   blocked_ctx ? 256 : 16, step_num, attn_scale, cache_dequant_scale, ctx_quant_scale,
                                    lds_f + g * gfl, wid, lane);
   }
 }
@@ -160,7 +160,7 @@ decself_qkv_attn_early_kernel(const int8_t* __restrict__ x, const int8_t* __rest
                               int8_t* v_cache, int8_t* __restrict__ ctx, int rows, int hidden,
                               int head_num, int max_step, int step_id, float alpha,
                               float dequant_scale, float cache_quant_scale, float attn_scale,
-                              float cache_dequant_scale, float ctx_quant_scale) {
+                              float cache_dequant_scale, float ctx_quant_scale, int blocked_ctx) {
   constexpr int D = kDqaD, COLS = kDqaCols, NWV = 8;
   constexpr int CH = D / 16, KPW = 64 / CH;
   extern __shared__ float lds_f[];
@@ -269,8 +269,9 @@ decself_qkv_attn_early_kernel(const int8_t* __restrict__ x, const int8_t* __rest
         vv[u] = nv;
       }
     }
-    decself_attend_row_once_body<D, NWV, UN>(qv, kv, vv, ctx + (long)row * hidden + head * D,
-                                             true, step_num, attn_scale, cache_dequant_scale,
+    decself_attend_row_once_body<D, NWV, UN>(qv, kv, vv,
+                                             ctx + code_offset(row, head * D, hidden, blocked_ctx),
+                                             true, blocked_ctx ? 256 : 16, step_num, attn_scale, cache_dequant_scale,
                                              ctx_quant_scale, lds_f, wave, lane);
   }
 }
@@ -291,13 +292,13 @@ bool decself_qkv_attention_supported(int rows, int hidden, int head_num, int max
 // [3 * hidden]; new_q int8 [rows, hidden]; caches int8 [rows, heads, max_step, 64]; ctx int8
 // [rows, hidden].  alpha, dequant_scale, cache_quant_scale: the three scales of
 // gemm_i8_decself_qkv_i8o; attn_scale, cache_dequant_scale, ctx_quant_scale: those of
-// decself_attention_i8 (step_num = step_id + 1).
+// decself_attention_i8 (step_num = step_id + 1).  blocked_ctx: ctx is a blocked matrix.
 int decself_qkv_attention_i8(const int8_t* x, const int8_t* qkv_weight, const __half* qkv_bias,
                              int8_t* new_q, int8_t* k_cache, int8_t* v_cache, int8_t* ctx,
                              int rows, int hidden, int head_num, int max_step, int step_id,
                              float alpha, float dequant_scale, float cache_quant_scale,
                              float attn_scale, float cache_dequant_scale, float ctx_quant_scale,
-                             hipStream_t s) {
+                             hipStream_t s, bool blocked_ctx) {
   if (!x || !qkv_weight || !qkv_bias || !new_q || !k_cache || !v_cache || !ctx)
     return lsh_fail(LSH_ERR_INVALID, "decself_qkv_attention_i8: null pointer");
   if (!decself_qkv_attention_supported(rows, hidden, head_num, max_step))
@@ -321,7 +322,7 @@ int decself_qkv_attention_i8(const int8_t* x, const int8_t* qkv_weight, const __
     decself_qkv_attn_kernel<NWV, UN, RG><<<grid, 512, lds, s>>>(                                   \
         x, qkv_weight, qkv_bias, new_q, k_cache, v_cache, ctx, rows, hidden, head_num, max_step,   \
         step_id, alpha, dequant_scale, cache_quant_scale, attn_scale, cache_dequant_scale,         \
-        ctx_quant_scale);                                                                          \
+        ctx_quant_scale, blocked_ctx);                                                             \
   } while (0)
 #define LSH_DQA_EARLY(UN)                                                                          \
   do {                                                                                             \
@@ -330,7 +331,7 @@ int decself_qkv_attention_i8(const int8_t* x, const int8_t* qkv_weight, const __
     decself_qkv_attn_early_kernel<UN><<<rows * head_num, 512, lds, s>>>(                           \
         x, qkv_weight, qkv_bias, new_q, k_cache, v_cache, ctx, rows, hidden, head_num, max_step,   \
         step_id, alpha, dequant_scale, cache_quant_scale, attn_scale, cache_dequant_scale,         \
-        ctx_quant_scale);                                                                          \
+        ctx_quant_scale, blocked_ctx);                                                             \
   } while (0)
   if (step_num <= 64) LSH_DQA(1, 4, 8);
   else if (step_num <= 128) LSH_DQA(4, 2, 2);

@@ -68,11 +68,13 @@ int launch_kw(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K, in
   const dim3 grid(tm * tn, ksplit);
   constexpr size_t smem = kw_lds_bytes<Epi, MB, NB>();
   const int slices = K / 64 / ksplit;
-  if (slices % 16 == 0)
-    return launch_blk<gemm_kw_kernel<Tr, Epi, MB, NB, 4>>(grid, 256, smem, s, A, W, epi, M, N, K, slices, tm, tn);
-  if (slices % 12 == 0)
-    return launch_blk<gemm_kw_kernel<Tr, Epi, MB, NB, 3>>(grid, 256, smem, s, A, W, epi, M, N, K, slices, tm, tn);
-  return launch_blk<gemm_kw_kernel<Tr, Epi, MB, NB, 1>>(grid, 256, smem, s, A, W, epi, M, N, K, slices, tm, tn);
+#define LSH_KW(D)                                                                                   \
+  return launch_blk<gemm_kw_kernel<Tr, Epi, MB, NB, D>>(grid, 256, smem, s, A, W, epi, M, N, K, slices, tm, tn)
+  if (slices % 16 == 0) LSH_KW(4);
+  if (slices % 12 == 0) LSH_KW(3);
+  if (slices % 8 == 0) LSH_KW(2);
+  LSH_KW(1);
+#undef LSH_KW
 }
 
 // The LDS tile kernel: 8 wavefronts for the tall tiles, 4 for 128 x 128 and 128 x 64 (two or three
@@ -164,16 +166,17 @@ int gemm_blk_i32o(const int8_t* A, const int8_t* W, int32_t* C, int M, int N, in
   return dispatch_blk<KwI8, EpiI32, true>(A, W, EpiI32{C}, M, N, K, s, ksplit);
 }
 
-// Range of K per workgroup for the few rows of a generation step: as many int32 planes (summed by
-// the layer norm that reads them) as make the launch one round of the chip, four at most -- the
-// same rule as for row-major operands.
+// Ranges of K (int32 planes, summed by the layer norm that reads them) for the few rows of a
+// generation step, four at most: as many as make the estimate smallest, 0.1 us of it for a
+// plane more to fetch.  16 x 1024 x 4096 with weights from memory: 4.6 us in one range, 3.5 in
+// four.
 int gemm_blk_preferred_ksplit(int M, int N, int K) {
   int best = 1;
+  if (M > kKwColdRows) return best;
   float best_us = kw_choose_tile(M, N, K, 1, cu_count(), false).us;
-  for (int ks = 2; ks <= 4; ks *= 2) {
-    if (M > 64 || K % (1024 * ks) != 0) break;
-    // a plane more for the layer norm to fetch: 0.2 us
-    const float us = kw_choose_tile(M, N, K / ks, ks, cu_count(), false).us + 0.2f * ks;
+  for (int ks = 2; ks <= 4; ++ks) {
+    if (K % (512 * ks) != 0) continue;
+    const float us = kw_choose_tile(M, N, K / ks, ks, cu_count(), false).us + 0.1f * ks;
     if (us < best_us) {
       best = ks;
       best_us = us;

@@ -203,11 +203,21 @@ struct KwTile {
   int mb, nb;
   float us;
 };
+// Few rows: a generation step, whose weights come from the memory and not from the L2.  A compute
+// unit draws about 37 KB/us of them (16 x 1024 x 4096: 64 KB of weights per tile 4.6 us, 16 KB
+// 3.5 us), so a tile's weights are priced at that rate where it is more than the fitted slope.
+constexpr int kKwColdRows = 64;
+inline TileCost kw_cold_cost(TileCost c) {
+  const float slope = (float)c.tn / 36.f;  // us per 1024 bytes of K
+  c.b = c.b * 1.35f < slope ? slope / 1.35f : c.b;
+  c.s1 = c.s1 < slope ? slope : c.s1;
+  return c;
+}
 // K: the bytes of one of `ksplit` ranges
 inline KwTile kw_choose_tile(int M, int N, int K, int ksplit, int cus, bool table) {
   KwTile best{0, 0, 0.f};
   for (const auto& c : kKwCost) {
-    const float us = tile_us(c, M, N, K, ksplit, cus, table);
+    const float us = tile_us(M <= kKwColdRows ? kw_cold_cost(c) : c, M, N, K, ksplit, cus, table);
     if (best.mb == 0 || us < best.us) best = KwTile{c.tm / 16, c.tn / 16, us};
   }
   return best;

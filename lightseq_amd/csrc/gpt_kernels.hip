@@ -502,16 +502,16 @@ int topk_sample_i8I(int batch_size, int batch_seq_len, int logits_seq_len, hipSt
   return lsh_check_launch("topk_sample_tail_kernel");
 }
 
-// the model's step: ids [batch, max_step] in place, logits [batch, vocab] of the last
-// position; writes column cur_len, the step's input ids and the unfinished flag
+// the model's step: ids [batch, max_step] in place, logits of the last position, rows ldl codes
+// apart; writes column cur_len, the step's input ids and the unfinished flag
 __global__ void __launch_bounds__(1024)
-gpt_greedy_step_kernel(const int8_t* __restrict__ logits, int* ids, int* __restrict__ last_ids,
-                       int vocab, int max_step, int cur_len, int* unfinished, int eos_id) {
+gpt_greedy_step_kernel(const int8_t* __restrict__ logits, long ldl, int* ids,
+                       int* __restrict__ last_ids, int vocab, int max_step, int cur_len, int* unfinished, int eos_id) {
   __shared__ int red[32];
   const int b = blockIdx.x;
   const bool ended = ids[(long)b * max_step + cur_len - 1] == eos_id;
   int tok = eos_id;
-  if (!ended) tok = block_argmax_i8(logits + (long)b * vocab, vocab, red);
+  if (!ended) tok = block_argmax_i8(logits + b * ldl, vocab, red);
   if (threadIdx.x == 0) {
     if (!ended && tok != eos_id) unfinished[0] = 1;
     ids[(long)b * max_step + cur_len] = tok;
@@ -520,14 +520,15 @@ gpt_greedy_step_kernel(const int8_t* __restrict__ logits, int* ids, int* __restr
 }
 
 int gpt_greedy_step(const int8_t* logits, int* ids, int* last_ids, int vocab_size, int max_step,
-                    int cur_len, int batch_size, int* unfinished, int eos_id, hipStream_t s) {
+                    int cur_len, int batch_size, int* unfinished, int eos_id, hipStream_t s,
+                    int logits_stride) {
   if (!logits || !ids || !last_ids || !unfinished || batch_size <= 0 || vocab_size <= 0 ||
-      cur_len <= 0 || cur_len >= max_step)
+      logits_stride < vocab_size || cur_len <= 0 || cur_len >= max_step)
     return lsh_fail(LSH_ERR_INVALID, "gpt_greedy_step: bad arguments");
   if (vocab_size > (1 << 20))
     return lsh_fail(LSH_ERR_UNSUPPORTED, "gpt_greedy_step: vocabulary above 2^20 ids");
-  gpt_greedy_step_kernel<<<batch_size, 1024, 0, s>>>(logits, ids, last_ids, vocab_size, max_step,
-                                                     cur_len, unfinished, eos_id);
+  gpt_greedy_step_kernel<<<batch_size, 1024, 0, s>>>(logits, logits_stride, ids, last_ids,
+                                                     vocab_size, max_step, cur_len, unfinished, eos_id);
   return lsh_check_launch("gpt_greedy_step_kernel");
 }
 
@@ -733,14 +734,14 @@ int topp_sample_i8I(int batch_size, int batch_seq_len, int logits_seq_len, hipSt
 
 // the model's step with random sampling: as gpt_greedy_step_kernel
 __global__ void __launch_bounds__(kSampleThreads)
-gpt_sample_step_kernel(const int8_t* __restrict__ logits, int* ids, int* __restrict__ last_ids,
-                       int vocab, int max_step, int cur_len, int* unfinished, int eos_id, int k,
+gpt_sample_step_kernel(const int8_t* __restrict__ logits, long ldl, int* ids,
+                       int* __restrict__ last_ids, int vocab, int max_step, int cur_len, int* unfinished, int eos_id, int k,
                        float p, float scale, SampleState* st) {
   __shared__ SampleShared sh;
   const int b = blockIdx.x;
   const bool ended = ids[(long)b * max_step + cur_len - 1] == eos_id;
   int tok = eos_id;
-  if (!ended) tok = sample_row(logits + (long)b * vocab, vocab, k, p, scale, st + b, sh);
+  if (!ended) tok = sample_row(logits + b * ldl, vocab, k, p, scale, st + b, sh);
   if (threadIdx.x == 0) {
     if (!ended && tok != eos_id) unfinished[0] = 1;
     ids[(long)b * max_step + cur_len] = tok;
@@ -750,9 +751,9 @@ gpt_sample_step_kernel(const int8_t* __restrict__ logits, int* ids, int* __restr
 
 int gpt_sample_step(const int8_t* logits, int* ids, int* last_ids, int vocab_size, int max_step,
                     int cur_len, int batch_size, int* unfinished, int eos_id, int k, float p,
-                    float dequant_scale, void* state, hipStream_t s) {
+                    float dequant_scale, void* state, hipStream_t s, int logits_stride) {
   if (!logits || !ids || !last_ids || !unfinished || !state || batch_size <= 0 ||
-      vocab_size <= 0 || cur_len <= 0 || cur_len >= max_step || !(dequant_scale > 0.f) ||
+      vocab_size <= 0 || logits_stride < vocab_size || cur_len <= 0 || cur_len >= max_step || !(dequant_scale > 0.f) ||
       (reinterpret_cast<uintptr_t>(state) & 15u) != 0)
     return lsh_fail(LSH_ERR_INVALID, "gpt_sample_step: bad arguments");
   if (k != 0 && k != 2 && k != 4 && k != 8 && k != 16 && k != 32)
@@ -762,7 +763,7 @@ int gpt_sample_step(const int8_t* logits, int* ids, int* last_ids, int vocab_siz
   if (vocab_size > (1 << kSampleIdBits))
     return lsh_fail(LSH_ERR_UNSUPPORTED, "gpt_sample_step: vocabulary above 2^20 ids");
   gpt_sample_step_kernel<<<batch_size, kSampleThreads, 0, s>>>(
-      logits, ids, last_ids, vocab_size, max_step, cur_len, unfinished, eos_id, k, p,
+      logits, logits_stride, ids, last_ids, vocab_size, max_step, cur_len, unfinished, eos_id, k, p,
       dequant_scale, static_cast<SampleState*>(state));
   return lsh_check_launch("gpt_sample_step_kernel");
 }
@@ -774,26 +775,71 @@ int gpt_sample_step(const int8_t* logits, int* ids, int* last_ids, int vocab_siz
 // position) pair gets its own workgroup and a second kernel adds a sequence's terms in order;
 // without one a workgroup per sequence walks its positions.  Both give the same bits.
 // ---------------------------------------------------------------------------------
-// -log p(next token) / (len - 1) of position s of sequence b, the same in every thread
-__device__ __forceinline__ float ppl_term(const int8_t* __restrict__ logits,
-                                          const int* __restrict__ input_ids, int b, int s, int len,
-                                          int vocab, int seq_len, float dq, float* red) {
+// -log p(next token) / (len - 1) of position s of sequence b, the same in every thread.  lr: the
+// position's logits.  ALIGNED rows (16-byte aligned, as the model's padded rows are) are read as
+// 16-byte pieces, four per thread requested together and kept in registers from the maximum to
+// the sum (up to 65536 ids; the pieces are read again beyond that); what bounds it then is the
+// exp and four more instructions per id: 3072 rows of 50257 ids in 163 us with byte loads, see
+// below for what it takes now.
+constexpr int kPplPieces = 4;
+template <bool ALIGNED>
+__device__ __forceinline__ float ppl_term(const int8_t* __restrict__ lr, int target, int len,
+                                          int vocab, float dq, float* red) {
 #pragma clang fp contract(off)
-  const long tok = (long)b * seq_len + s;
-  const int8_t* lr = logits + tok * vocab;
-  float mx = kFloatInfNeg;
-  for (int v = threadIdx.x; v < vocab; v += blockDim.x) mx = fmaxf(mx, (float)lr[v] * dq);
-  mx = block_max(mx, red);
-  float se = 0.f;
-  for (int v = threadIdx.x; v < vocab; v += blockDim.x)
-    se += __expf(fmaxf((float)lr[v] * dq - mx, kLogitThreshMin));
+  float mx, se = 0.f;
+  if constexpr (ALIGNED) {
+    const int t = threadIdx.x, n = blockDim.x;
+    const int full = vocab >> 4;  // whole pieces; the last vocab % 16 ids go one per thread
+    // bytes whose unsigned order is that of code * dq
+    const uint32_t flip = dq < 0.f ? 0x7f7f7f7fu : 0x80808080u;
+    uint4 w[kPplPieces];
+    const int ev = (full << 4) + t;
+    const bool tail = ev < vocab;
+    const int tc = lr[tail ? ev : 0];
+    unsigned um = tail ? ((unsigned)tc ^ flip) & 0xffu : 0u;
+    auto fetch = [&](int p0) {
+#pragma unroll
+      for (int u = 0; u < kPplPieces; ++u)
+        w[u] = *reinterpret_cast<const uint4*>(lr + (long)max(min(p0 + u * n + t, full - 1), 0) * 16);
+    };
+    for (int p0 = 0; p0 < full; p0 += kPplPieces * n) {
+      fetch(p0);
+#pragma unroll
+      for (int u = 0; u < kPplPieces; ++u) {
+        if (p0 + u * n + t >= full) continue;
+        const uint32_t ws[4] = {w[u].x ^ flip, w[u].y ^ flip, w[u].z ^ flip, w[u].w ^ flip};
+#pragma unroll
+        for (int e = 0; e < 16; ++e) um = max(um, __builtin_amdgcn_ubfe(ws[e >> 2], 8 * (e & 3), 8));
+      }
+    }
+    const int mi = (int)block_max((float)um, red);
+    mx = (float)(dq < 0.f ? 127 - mi : mi - 128) * dq;
+    for (int p0 = 0; p0 < full; p0 += kPplPieces * n) {
+      if (full > kPplPieces * n) fetch(p0);
+#pragma unroll
+      for (int u = 0; u < kPplPieces; ++u) {
+        if (p0 + u * n + t >= full) continue;
+        const uint32_t ws[4] = {w[u].x, w[u].y, w[u].z, w[u].w};
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          se += __expf(fmaxf((float)unpack_i8(ws[e >> 2], e & 3) * dq - mx, kLogitThreshMin));
+      }
+    }
+    if (tail) se += __expf(fmaxf((float)tc * dq - mx, kLogitThreshMin));
+  } else {
+    mx = kFloatInfNeg;
+    for (int v = threadIdx.x; v < vocab; v += blockDim.x) mx = fmaxf(mx, (float)lr[v] * dq);
+    mx = block_max(mx, red);
+    for (int v = threadIdx.x; v < vocab; v += blockDim.x)
+      se += __expf(fmaxf((float)lr[v] * dq - mx, kLogitThreshMin));
+  }
   se = block_sum(se, red);
-  int target = input_ids[tok + 1];
   target = min(max(target, 0), vocab - 1);
   const float log_prob = ((float)lr[target] * dq - mx - logf(se)) / (float)(len - 1);
   return -log_prob;
 }
 
+template <bool ALIGNED>
 __global__ void __launch_bounds__(1024)
 ppl_kernel(const int8_t* __restrict__ logits, const int* __restrict__ input_ids,
            const int* __restrict__ real_seq_len, float* ppl, int vocab, int seq_len, float dq) {
@@ -801,52 +847,76 @@ ppl_kernel(const int8_t* __restrict__ logits, const int* __restrict__ input_ids,
   const int b = blockIdx.x;
   const int len = real_seq_len[b];
   float total = 0.f;
-  for (int s = 0; s < seq_len && s < len - 1; ++s)
-    total += ppl_term(logits, input_ids, b, s, len, vocab, seq_len, dq, red);
+  for (int s = 0; s < seq_len && s < len - 1; ++s) {
+    const long tok = (long)b * seq_len + s;
+    total += ppl_term<ALIGNED>(logits + tok * vocab, input_ids[tok + 1], len, vocab, dq, red);
+  }
   if (threadIdx.x == 0) ppl[b] += total;
 }
 
-// grid (seq_len, batch): terms[b * seq_len + s]
+// grid (seq_len, batch): terms[b * seq_len + s]; the logits' rows are ldl codes apart
+template <bool ALIGNED>
 __global__ void __launch_bounds__(1024)
-ppl_terms_kernel(const int8_t* __restrict__ logits, const int* __restrict__ input_ids,
+ppl_terms_kernel(const int8_t* __restrict__ logits, long ldl, const int* __restrict__ input_ids,
                  const int* __restrict__ real_seq_len, float* __restrict__ terms, int vocab,
                  int seq_len, float dq) {
   __shared__ float red[16];
   const int b = blockIdx.y, s = blockIdx.x;
   const int len = real_seq_len[b];
   if (s >= len - 1) return;  // (uniform: no term, nothing read by the sum)
-  const float t = ppl_term(logits, input_ids, b, s, len, vocab, seq_len, dq, red);
-  if (threadIdx.x == 0) terms[(long)b * seq_len + s] = t;
+  const long tok = (long)b * seq_len + s;
+  const float t = ppl_term<ALIGNED>(logits + tok * ldl, input_ids[tok + 1], len, vocab, dq, red);
+  if (threadIdx.x == 0) terms[tok] = t;
 }
 
-__global__ void ppl_sum_kernel(const float* __restrict__ terms,
-                               const int* __restrict__ real_seq_len, float* ppl, int batch,
-                               int seq_len) {
+// One wavefront per sequence: 64 terms are fetched together, lane 0's chain of additions takes
+// them from the other lanes in ascending order (a thread that fetched its own terms one by one
+// waited for the memory between any two additions: 27.6 us for 384 terms).
+__global__ void __launch_bounds__(64)
+ppl_sum_kernel(const float* __restrict__ terms, const int* __restrict__ real_seq_len, float* ppl,
+               int seq_len) {
 #pragma clang fp contract(off)
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= batch) return;
-  const int len = real_seq_len[b];
+  const int b = blockIdx.x, lane = threadIdx.x;
+  const int n = min(seq_len, real_seq_len[b] - 1);
   float total = 0.f;
-  for (int s = 0; s < seq_len && s < len - 1; ++s) total += terms[(long)b * seq_len + s];
-  ppl[b] += total;
+  for (int s0 = 0; s0 < n; s0 += 64) {
+    const float t = s0 + lane < n ? terms[(long)b * seq_len + s0 + lane] : 0.f;
+    const int m = min(n - s0, 64);
+    for (int i = 0; i < m; ++i)
+      total += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, t), i));
+  }
+  if (lane == 0) ppl[b] += total;
 }
 
 int ppl_i8I(int batch_size, int batch_seq_len, hipStream_t s, const int8_t* logits,
             const int* input_ids, const int* real_seq_len, float* ppl, int vocab_size,
-            float dequant_scale, float* workspace) {
+            float dequant_scale, float* workspace, int logits_stride) {
   if (!logits || !input_ids || !real_seq_len || !ppl || batch_size <= 0 || batch_seq_len <= 0 ||
       vocab_size <= 0)
     return lsh_fail(LSH_ERR_INVALID, "ker_ppl_i8I: bad arguments");
+  const int ldl = logits_stride ? logits_stride : vocab_size;
+  if (ldl < vocab_size) return lsh_fail(LSH_ERR_INVALID, "ker_ppl_i8I: rows overlap");
+  const bool aligned = (reinterpret_cast<uintptr_t>(logits) & 15u) == 0 && ldl % 16 == 0;
   if (workspace != nullptr && batch_size <= 65535) {
-    ppl_terms_kernel<<<dim3(batch_seq_len, batch_size), 1024, 0, s>>>(
-        logits, input_ids, real_seq_len, workspace, vocab_size, batch_seq_len, dequant_scale);
+    const dim3 grid(batch_seq_len, batch_size);
+    if (aligned)
+      ppl_terms_kernel<true><<<grid, 1024, 0, s>>>(logits, ldl, input_ids, real_seq_len, workspace,
+                                                   vocab_size, batch_seq_len, dequant_scale);
+    else
+      ppl_terms_kernel<false><<<grid, 1024, 0, s>>>(logits, ldl, input_ids, real_seq_len, workspace,
+                                                    vocab_size, batch_seq_len, dequant_scale);
     if (int rc = lsh_check_launch("ppl_terms_kernel")) return rc;
-    ppl_sum_kernel<<<(batch_size + 63) / 64, 64, 0, s>>>(workspace, real_seq_len, ppl, batch_size,
-                                                         batch_seq_len);
+    ppl_sum_kernel<<<batch_size, 64, 0, s>>>(workspace, real_seq_len, ppl, batch_seq_len);
     return lsh_check_launch("ppl_sum_kernel");
   }
-  ppl_kernel<<<batch_size, 1024, 0, s>>>(logits, input_ids, real_seq_len, ppl, vocab_size,
-                                         batch_seq_len, dequant_scale);
+  if (logits_stride && logits_stride != vocab_size)
+    return lsh_fail(LSH_ERR_UNSUPPORTED, "ker_ppl_i8I: padded rows need the workspace");
+  if (aligned)
+    ppl_kernel<true><<<batch_size, 1024, 0, s>>>(logits, input_ids, real_seq_len, ppl, vocab_size,
+                                                 batch_seq_len, dequant_scale);
+  else
+    ppl_kernel<false><<<batch_size, 1024, 0, s>>>(logits, input_ids, real_seq_len, ppl, vocab_size,
+                                                  batch_seq_len, dequant_scale);
   return lsh_check_launch("ppl_kernel");
 }
 

@@ -151,7 +151,8 @@ __global__ void __launch_bounds__(256, 2)
 gpt_prefill_attn_i8_kernel(const int8_t* __restrict__ q_codes, const int8_t* __restrict__ k_cache,
                            const int8_t* __restrict__ v_cache, const int* __restrict__ real_seq_len,
                            int8_t* __restrict__ ctx_q, float quant_scale, float v_quant_scale,
-                           int S, int head_num, int max_step, float alpha, float dq, int BH) {
+                           int S, int head_num, int max_step, float alpha, float dq, int BH,
+                           int blocked) {
   constexpr int D = 64, VSTR = kPfVstr;
   extern __shared__ __align__(16) int8_t smem[];
   const int nkb_max = (S + 127) / 128;
@@ -331,7 +332,7 @@ gpt_prefill_attn_i8_kernel(const int8_t* __restrict__ q_codes, const int8_t* __r
       for (int j = 0; j < 4; ++j) o[j] = round_h(acc[db][4 * vg + j]);
       const uint32_t w4 = float2int8_pack4(o[0], o[1], o[2], o[3], quant_scale);
       // a padded query gives zeros, whose code is 0
-      *reinterpret_cast<uint32_t*>(ctx_q + tok * hidden + head * D + dd) = q_pad ? 0u : w4;
+      *reinterpret_cast<uint32_t*>(ctx_q + code_offset(tok, head * D + dd, hidden, blocked)) = q_pad ? 0u : w4;
     }
   }
 }
@@ -339,7 +340,8 @@ gpt_prefill_attn_i8_kernel(const int8_t* __restrict__ q_codes, const int8_t* __r
 int gpt_prefill_attention_i8(const int8_t* q_codes, const int8_t* k_cache, const int8_t* v_cache,
                              const int* real_seq_len, int8_t* ctx_q, float quant_scale,
                              float dequant_scale, float v_quant_scale, int batch, int seq_len,
-                             int head_num, int dim_per_head, int max_step, hipStream_t s) {
+                             int head_num, int dim_per_head, int max_step, hipStream_t s,
+                             bool blocked) {
   if (batch <= 0 || seq_len <= 0 || head_num <= 0 || !q_codes || !k_cache || !v_cache ||
       !real_seq_len || !ctx_q || seq_len > max_step || !(v_quant_scale > 0.f))
     return lsh_fail(LSH_ERR_INVALID, "gpt_prefill_attention_i8: bad arguments");
@@ -373,7 +375,7 @@ int gpt_prefill_attention_i8(const int8_t* q_codes, const int8_t* k_cache, const
   const float alpha = __half2float(__float2half_rn(sqrtf(1.f / (float)dim_per_head)));
   gpt_prefill_attn_i8_kernel<<<(int)(BH * nqb), 256, gpt_prefill_lds_bytes(seq_len), s>>>(
       q_codes, k_cache, v_cache, real_seq_len, ctx_q, quant_scale, v_quant_scale, seq_len, head_num,
-      max_step, alpha, dequant_scale, (int)BH);
+      max_step, alpha, dequant_scale, (int)BH, blocked);
   return lsh_check_launch("gpt_prefill_attn_i8_kernel");
 }
 

@@ -246,7 +246,7 @@ int decself_qkv_attention_i8(const int8_t* x, const int8_t* qkv_weight, const __
                              int rows, int hidden, int head_num, int max_step, int step_id,
                              float alpha, float dequant_scale, float cache_quant_scale,
                              float attn_scale, float cache_dequant_scale, float ctx_quant_scale,
-                             hipStream_t s);
+                             hipStream_t s, bool blocked_ctx = false);
 // Decode-step cross-attention query product with ker_arrange_encdec_q_i8I as its epilogue:
 // fp16 q [batch, heads, beam, d].
 int gemm_i8_encdec_q_f16(const int8_t* A, const int8_t* W, const __half* q_bias, __half* new_q,
@@ -353,10 +353,11 @@ int fuse_softmax_new_value_i32I_i8O(const int32_t* correlation, const int8_t* v,
                                     int batch_head_num, int step_num, int max_step, int head_num,
                                     int dim_per_head, float attn_scale, float dequant_scale,
                                     float quant_scale, hipStream_t s);
+// (blocked: the context codes are written as a blocked matrix)
 int decself_attention_i8(const int8_t* q, const int8_t* k_cache, const int8_t* v_cache,
                          int8_t* new_v, int batch_head_num, int step_num, int max_step,
                          int head_num, int dim_per_head, float attn_scale, float dequant_scale,
-                         float quant_scale, hipStream_t s);
+                         float quant_scale, hipStream_t s, bool blocked = false);
 template <typename T>
 int arrange_encdec_q_i8I(int step_token_num, int hidden_size, hipStream_t s, const int8_t* ori_q,
                          const T* q_bias, T* new_q, int beam_size, int dim_per_head, int head_num,
@@ -371,13 +372,14 @@ int correlation_softmax_encdec(int batch_size, int head_num_per_seq, int batch_s
 int encdec_attention_f16(const __half* q, const __half* k, const __half* v, const int* pad_mask,
                          __half* ctx, int8_t* ctx_q, float quant_scale, int batch_size,
                          int beam_size, int head_num, int batch_seq_len, int dim_per_head,
-                         hipStream_t s);
+                         hipStream_t s, bool blocked = false);
+// blocked: x, q_weight and ctx_q are blocked matrices
 bool encdec_q_attention_supported(int beam_size, int head_num, int hidden, int batch_seq_len);
 int encdec_q_attention_f16(const int8_t* x, const int8_t* q_weight, const __half* q_bias,
                            const __half* k, const __half* v, const int* pad_mask, int8_t* ctx_q,
                            float quant_scale, int batch_size, int beam_size, int head_num,
                            int batch_seq_len, int hidden, float alpha, float dequant_scale,
-                           hipStream_t s);
+                           hipStream_t s, bool blocked = false);
 
 // ---- beam search (beam_kernels.hip) -------------------------------------------------------
 template <typename T>
@@ -416,7 +418,7 @@ int beam_search_step_i8I(const int8_t* logits, const T* logit_bias, float* seq_p
                          float* top_score, int* top_idx, int* parent, int* num_finished,
                          float dequant_scale, int vocab_size, int max_step, float length_norm,
                          int cur_step, int batch_size, int beam_size, int end_id, hipStream_t s,
-                         float* part_ws = nullptr, size_t part_ws_words = 0);
+                         float* part_ws = nullptr, size_t part_ws_words = 0, int logits_stride = 0);
 // 4-byte words of the optional workspace `part_ws` with which the per-row top-k of the step is
 // dealt to several workgroups per row (0: this shape runs one workgroup per row either way)
 size_t beam_search_step_workspace_words(int batch_size, int beam_size, int vocab_size);
@@ -460,7 +462,8 @@ int gpt_arrange_qkv_prefill_i8(int batch_token_num, int hidden_size, hipStream_t
 int gpt_prefill_attention_i8(const int8_t* q_codes, const int8_t* k_cache, const int8_t* v_cache,
                              const int* real_seq_len, int8_t* ctx_q, float quant_scale,
                              float dequant_scale, float v_quant_scale, int batch, int seq_len,
-                             int head_num, int dim_per_head, int max_step, hipStream_t s);
+                             int head_num, int dim_per_head, int max_step, hipStream_t s,
+                             bool blocked = false);
 template <typename T>
 int correlation_softmax_gpt_i32I(int batch_size, int batch_seq_len, int head_num, hipStream_t s,
                                  const int32_t* correlation, T* output, const int* real_seq_len,
@@ -496,22 +499,24 @@ template <typename T>
 int dec_topk_sample_i8I(int batch_size, int batch_seq_len, int max_step, int logits_seq_len,
                         hipStream_t s, const int8_t* logits, const T* logit_bias, int* ids,
                         int vocab_size, int k, int* unfinished, void* state, int eos_id,
-                        float dequant_scale);
+                        float dequant_scale, int logits_stride = 0);
 template <typename T>
 int dec_topp_sample_i8I(int batch_size, int batch_seq_len, int max_step, int logits_seq_len,
                         hipStream_t s, const int8_t* logits, const T* logit_bias, int* ids,
                         int vocab_size, float p, int* unfinished, void* state, int eos_id,
-                        float dequant_scale);
+                        float dequant_scale, int logits_stride = 0);
 // the model's step with random sampling (k in {2,..,32}: top-k; k == 0: top-p with p)
 int gpt_sample_step(const int8_t* logits, int* ids, int* last_ids, int vocab_size, int max_step,
                     int cur_len, int batch_size, int* unfinished, int eos_id, int k, float p,
-                    float dequant_scale, void* state, hipStream_t s);
+                    float dequant_scale, void* state, hipStream_t s, int logits_stride);
 int gpt_greedy_step(const int8_t* logits, int* ids, int* last_ids, int vocab_size, int max_step,
-                    int cur_len, int batch_size, int* unfinished, int eos_id, hipStream_t s);
+                    int cur_len, int batch_size, int* unfinished, int eos_id, hipStream_t s,
+                    int logits_stride);
 int ppl_i8I(int batch_size, int batch_seq_len, hipStream_t s, const int8_t* logits,
             const int* input_ids, const int* real_seq_len, float* ppl, int vocab_size,
-            float dequant_scale, float* workspace = nullptr);  // workspace: batch * seq_len floats
-                                                               // -> one workgroup per position
+            float dequant_scale, float* workspace = nullptr, int logits_stride = 0);
+// workspace: batch * seq_len floats -> one workgroup per position; it also allows rows of logits
+// that lie logits_stride codes apart (0: vocab_size)
 
 // ---- operator kernels of the csrc layer path (layer_ops.hip); clip values are device
 // ---- scalars of type T, dropout ratios must be 0 -------------------------------------

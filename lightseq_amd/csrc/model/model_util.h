@@ -171,6 +171,12 @@ class StepTaps {
   bool wants(int layer, int step, const char* name) const {
     return !_dst.empty() && step == _step && (layer < 0 || layer == _layer) && _dst.count(name);
   }
+  // an int8 matrix, copied row-major whichever way the model holds it
+  void copy_codes(int layer, int step, const char* name, const int8_t* src, int rows, int cols,
+                  bool blocked, hipStream_t stream) const {
+    if (!blocked) return copy(layer, step, name, src, (size_t)rows * cols, stream);
+    if (wants(layer, step, name)) LSH_CALL(lsh::block_rows(src, _dst.at(name), rows, cols, true, stream));
+  }
   void copy(int layer, int step, const char* name, const void* src, size_t bytes,
             hipStream_t stream) const {
     if (!wants(layer, step, name)) return;
@@ -341,6 +347,62 @@ inline DeviceBuffer<int8_t> unblock_weight(const DeviceBuffer<int8_t>& b, int n,
   CHECK_GPU_ERROR(hipStreamSynchronize(s));
   return w;
 }
+
+// [n, k] row-major -> a blocked copy whose rows are padded with zeros to a multiple of 64
+inline DeviceBuffer<int8_t> block_weight_padded(const DeviceBuffer<int8_t>& w, int n, int k, hipStream_t s) {
+  const size_t bytes = (size_t)((n + 63) & ~63) * k;
+  DeviceBuffer<int8_t> b(bytes);
+  CHECK_GPU_ERROR(hipMemsetAsync(b.get(), 0, bytes, s));
+  LSH_CALL(lsh::block_rows(w.get(), b.get(), n, k, false, s));
+  CHECK_GPU_ERROR(hipStreamSynchronize(s));
+  return b;
+}
+
+// The products of a layer stack whose int8 matrices are all blocked (hidden and inner size
+// multiples of 64) or all row-major.
+struct LayerProducts {
+  bool blocked = false;
+  static bool can_block(int hidden, int inner, int dim_per_head) {
+    return hidden % 64 == 0 && inner % 64 == 0 && dim_per_head % 16 == 0;
+  }
+  // rows an activation matrix needs room for
+  size_t rows(size_t n) const { return (n + 15) & ~(size_t)15; }
+  DeviceBuffer<int8_t> weight(const std::vector<uint8_t>& w, int k, int n, hipStream_t s) const {
+    DeviceBuffer<int8_t> q = upload_kernel(w, k, n, true, s);
+    return blocked ? block_weight(q, n, k, s) : std::move(q);
+  }
+  void i8o(const int8_t* x, const int8_t* w, int8_t* out, int m, int n, int k, float alpha,
+           hipStream_t s) const {
+    LSH_CALL(blocked ? lsh::gemm_blk_i8o(x, w, out, m, n, k, alpha, s)
+                     : lsh::gemm_i8_i8o(x, w, out, m, n, k, alpha, s));
+  }
+  void lut(const int8_t* x, const int8_t* w, int8_t* out, const int8_t* table, int m, int n, int k,
+           float alpha, hipStream_t s) const {
+    LSH_CALL(blocked ? lsh::gemm_blk_lut(x, w, out, table, m, n, k, alpha, s)
+                     : lsh::gemm_i8_lut_i8o(x, w, out, table, m, n, k, alpha, s));
+  }
+  // int32 accumulators in up to max_planes planes of [m, n]; returns their number
+  int i32o(const int8_t* x, const int8_t* w, int32_t* out, int m, int n, int k, int max_planes,
+           hipStream_t s) const {
+    if (blocked) {
+      const int planes = std::min(max_planes, lsh::gemm_blk_preferred_ksplit(m, n, k));
+      LSH_CALL(lsh::gemm_blk_i32o(x, w, out, m, n, k, planes, s));
+      return planes;
+    }
+    int planes = 1;
+    LSH_CALL(lsh::gemm_i8_i32o_splitk(x, w, out, m, n, k,
+                                      std::min(max_planes, lsh::gemm_i8_preferred_ksplit(m, n, k)),
+                                      &planes, s));
+    return planes;
+  }
+  void decself_qkv(const int8_t* x, const int8_t* w, const __half* bias, int8_t* q, int8_t* k_cache,
+                   int8_t* v_cache, int rows, int hidden, int head_num, int max_step, int step,
+                   float alpha, float dequant_scale, float quant_scale, hipStream_t s) const {
+    LSH_CALL((blocked ? lsh::gemm_blk_decself_qkv : lsh::gemm_i8_decself_qkv_i8o)(
+        x, w, bias, q, k_cache, v_cache, rows, hidden, hidden, head_num, max_step, step, alpha,
+        dequant_scale, quant_scale, s));
+  }
+};
 
 }  // namespace hip
 }  // namespace lightseq

@@ -84,11 +84,13 @@ void QuantDecoder::init_buffer() {
   _encoder_out_buf.alloc(tokens * (size_t)L * 2 * H);
   _cur_step_query.alloc(rows * H);
   _query_buf1.alloc(rows * H);
-  const size_t wide = rows * (size_t)std::max(I, 3 * H);
+  _ops.blocked = LayerProducts::can_block(H, I, _tw._dim_per_head);
+  _logits_stride = _ops.blocked ? (V + 63) & ~63 : V;
+  const size_t wide = _ops.rows(rows) * (size_t)std::max(I, 3 * H);
   _buf_a.alloc(wide);
   _buf_b.alloc(wide);
   _buf_q.alloc(wide);
-  _logits.alloc(rows * (size_t)V);
+  _logits.alloc(rows * (size_t)_logits_stride);
   // up to 8 accumulator planes of the split-K second FFN product
   _int32_ffn_out_buf.alloc(rows * H * 8);
   for (int i = 0; i < 2; ++i) {
@@ -121,8 +123,10 @@ void QuantDecoder::init_buffer() {
   CHECK_GPU_ERROR(hipStreamSynchronize(_stream));  // start_id_vec dies below
 
   // ---- embedding block ----
-  // stored [H, vocab]; one [vocab, H] copy serves the row lookup and the logits GEMM
+  // stored [H, vocab]; a [vocab, H] copy serves the row lookup and, where products run on
+  // row-major operands, the logits; a blocked one padded to whole tiles serves them otherwise
   _int8_trg_emb = upload_kernel(_tw.trg_token_embedding, H, V, true, _stream);
+  if (_ops.blocked) _emb_blk = block_weight_padded(_int8_trg_emb, V, H, _stream);
   _pos_emb = upload_half(_tw.trg_position_embedding, _stream);
   _out_ln_scale = upload_half(_tw.trg_norm_scale, _stream);
   _out_ln_bias = upload_half(_tw.trg_norm_bias, _stream);
@@ -167,11 +171,11 @@ void QuantDecoder::init_buffer() {
     d.ffn_ln_bias = upload_half(w.ffn_norm_bias, _stream);
     d.b_ffn1 = upload_half(w.ffn_first_bias, _stream);
     d.b_ffn2 = upload_half(w.ffn_second_bias, _stream);
-    d.w_self_qkv = upload_kernel(w.self_project_kernel_qkv, H, 3 * H, true, _stream);
-    d.w_self_out = upload_kernel(w.self_project_kernel_output, H, H, true, _stream);
-    d.w_encdec_q = upload_kernel(w.encdec_project_kernel_q, H, H, true, _stream);
-    d.w_encdec_out = upload_kernel(w.encdec_project_kernel_output, H, H, true, _stream);
-    d.w_ffn1 = upload_kernel(w.ffn_first_kernel, H, I, true, _stream);
+    d.w_self_qkv = _ops.weight(w.self_project_kernel_qkv, H, 3 * H, _stream);
+    d.w_self_out = _ops.weight(w.self_project_kernel_output, H, H, _stream);
+    d.w_encdec_q = _ops.weight(w.encdec_project_kernel_q, H, H, _stream);
+    d.w_encdec_out = _ops.weight(w.encdec_project_kernel_output, H, H, _stream);
+    d.w_ffn1 = _ops.weight(w.ffn_first_kernel, H, I, _stream);
     {
       const float* c = &_dec_clip_max[l * 19];
       d.ffn1_act_lut.alloc((size_t)I * 256);
@@ -179,7 +183,7 @@ void QuantDecoder::init_buffer() {
                              _quant_range / c[11], c[11],
                              _tw._use_gelu ? kActGelu : kActReluNarrow, _stream));
     }
-    d.w_ffn2 = upload_kernel(w.ffn_second_kernel, I, H, true, _stream);
+    d.w_ffn2 = _ops.weight(w.ffn_second_kernel, I, H, _stream);
     if (!_tw._use_gelu) {
       // ReLU offset trick (:332-354): column sums of the fp16-rounded dequantised FFN2
       // kernel times clip/2
@@ -326,6 +330,12 @@ bool QuantDecoder::run_step() {
 // and the cache reorder (kernels and device-to-device copies only, so that it can be captured)
 void QuantDecoder::enqueue_step() {
   LnFewRowsScope few_rows;  // every step of every batch size: layer norms by the row kernel
+  // The opt-in launch reads row-major operands.  With taps set the two launches run, so that q
+  // and the caches are copied before the attention as the tap names promise; the bytes are the
+  // same either way.
+  _qkv_attn = !step_taps.any() && decself_qkv_attention_enabled() && _tw._dim_per_head == 64 &&
+              decself_qkv_attention_supported(_step_token_num, _tw._hidden_size, _tw._head_num,
+                                              _tw._max_step);
   embedding();
   for (_layer_id = 0; _layer_id < _tw._n_dec_layer; _layer_id++) {
     self_attention();
@@ -333,14 +343,14 @@ void QuantDecoder::enqueue_step() {
     ffn_add_norm();
   }
   /* --- Project hidden states to vocab logits (:527-532) --- */
-  LSH_CALL(gemm_i8_i8o(_buf_a.get(), _int8_trg_emb.get(), _logits.get(), _step_token_num,
-                       _tw._trg_vocab_size, _tw._hidden_size,
-                       _output_ln_clip_max * _trg_emb_clip_max / (_logits_clip_max * _quant_range),
-                       _stream));
+  _ops.i8o(_buf_a.get(), (_ops.blocked ? _emb_blk : _int8_trg_emb).get(), _logits.get(),
+           _step_token_num, _logits_stride, _tw._hidden_size,
+           _output_ln_clip_max * _trg_emb_clip_max / (_logits_clip_max * _quant_range), _stream);
   if (_rec_logits && _cur_step < _rec_max_steps)
-    CHECK_GPU_ERROR(hipMemcpyAsync(
-        _rec_logits + (size_t)_cur_step * _step_token_num * _tw._trg_vocab_size, _logits.get(),
-        (size_t)_step_token_num * _tw._trg_vocab_size, hipMemcpyDeviceToDevice, _stream));
+    CHECK_GPU_ERROR(hipMemcpy2DAsync(
+        _rec_logits + (size_t)_cur_step * _step_token_num * _tw._trg_vocab_size,
+        _tw._trg_vocab_size, _logits.get(), _logits_stride, _tw._trg_vocab_size, _step_token_num,
+        hipMemcpyDeviceToDevice, _stream));
   if (step_runs_beam_search())
     beam_search();
   else
@@ -355,6 +365,8 @@ void QuantDecoder::enqueue_step() {
 //   res_in, res_self, res_encdec, res_out: the fp16 residual stream [rows, hidden] at the start of
 //   the layer, after the first, the second and the last layer norm
 #define TAP(name, ptr, bytes) step_taps.copy(_layer_id, _cur_step, name, ptr, bytes, _stream)
+#define TAP_CODES(name, ptr, cols) \
+  step_taps.copy_codes(_layer_id, _cur_step, name, ptr, _step_token_num, cols, _ops.blocked, _stream)
 
 // hidden sizes the fused embedding + first layer norm covers
 bool QuantDecoder::emb_ln_fused() const {
@@ -371,7 +383,7 @@ void QuantDecoder::embedding() {
 
 void QuantDecoder::self_attention() {
   const int H = _tw._hidden_size, M = _step_token_num;
-  const Layer& w = _layers[_layer_id];
+  Layer& w = _layers[_layer_id];
   const float* c = &_dec_clip_max[_layer_id * 19];
   const float Q = _quant_range;
   int8_t* k_cache = _self_k_cache[_cache_cur].get() + (size_t)_layer_id * _layer_size_self_k;
@@ -384,60 +396,59 @@ void QuantDecoder::self_attention() {
           _int8_trg_emb.get(), _pos_emb.get(), _alive_seq[_alive_cur].get(),
           _cur_step_query.get(), _buf_a.get(), w.self_ln_scale.get(), w.self_ln_bias.get(),
           w.b_self_out.get(), M, H, _tw._trg_vocab_size, _cur_step, _tw._max_step,
-          _trg_emb_clip_max / _quant_range, true, Q / c[6], _tw._is_post_ln, _stream));
+          _trg_emb_clip_max / _quant_range, true, Q / c[6], _tw._is_post_ln, _stream,
+          _ops.blocked && !_qkv_attn));
     } else {
       LSH_CALL(norm_layer_resual_i8O<__half>(M, H, _stream, _cur_step_query.get(), _buf_a.get(),
                                              w.self_ln_scale.get(), w.self_ln_bias.get(),
-                                             w.b_self_out.get(), Q / c[6], _tw._is_post_ln));
+                                             w.b_self_out.get(), Q / c[6], _tw._is_post_ln,
+                                             _ops.blocked && !_qkv_attn));
     }
   }
   const size_t mh = (size_t)M * H;
-  TAP("self_ln_q", _buf_a.get(), mh);
+  TAP_CODES("self_ln_q", _buf_a.get(), H);
   TAP("res_in", _cur_step_query.get(), mh * sizeof(__half));
   const float attn_scale =
       __half2float(__float2half_rn(sqrtf(1.f / (float)_tw._dim_per_head)));
-  // With taps set the two launches run, so that q and the caches are copied before the
-  // attention as the tap names promise; the bytes are the same either way.
-  if (!step_taps.any() && decself_qkv_attention_enabled() && _tw._dim_per_head == 64 &&
-      decself_qkv_attention_supported(M, H, _tw._head_num, _tw._max_step)) {
-    LSH_CALL(decself_qkv_attention_i8(_buf_a.get(), w.w_self_qkv.get(), w.b_self_qkv.get(),
-                                      _buf_q.get(), k_cache, v_cache, _buf_b.get(), M, H,
-                                      _tw._head_num, _tw._max_step, _cur_step,
-                                      c[0] * c[6] / (c[12] * Q), c[12] / Q, Q / c[18], attn_scale,
-                                      c[18] / Q, Q / c[7], _stream));
+  if (_qkv_attn) {
+    if (_ops.blocked && !w.w_self_qkv_rows.get())
+      w.w_self_qkv_rows = unblock_weight(w.w_self_qkv, 3 * H, H, _stream);
+    LSH_CALL(decself_qkv_attention_i8(
+        _buf_a.get(), (_ops.blocked ? w.w_self_qkv_rows : w.w_self_qkv).get(), w.b_self_qkv.get(),
+        _buf_q.get(), k_cache, v_cache, _buf_b.get(), M, H, _tw._head_num, _tw._max_step, _cur_step,
+        c[0] * c[6] / (c[12] * Q), c[12] / Q, Q / c[18], attn_scale, c[18] / Q, Q / c[7], _stream,
+        _ops.blocked));
   } else {
-  // QKV product; its epilogue is ker_arrange_decself_qkv_i8I_i8O: q -> _buf_q, k / v -> slot
-  // _cur_step of the caches (all three with the cache clip)
-  if (_tw._dim_per_head % 16 == 0) {
-    LSH_CALL(gemm_i8_decself_qkv_i8o(_buf_a.get(), w.w_self_qkv.get(), w.b_self_qkv.get(),
-                                     _buf_q.get(), k_cache, v_cache, M, H, H, _tw._head_num,
-                                     _tw._max_step, _cur_step, c[0] * c[6] / (c[12] * Q),
-                                     c[12] / Q, Q / c[18], _stream));
-  } else {
-    LSH_CALL(gemm_i8_i8o(_buf_a.get(), w.w_self_qkv.get(), _buf_b.get(), M, 3 * H, H,
-                         c[0] * c[6] / (c[12] * Q), _stream));
-    LSH_CALL(arrange_decself_qkv_i8I_i8O<__half>(M, H, _stream, _buf_b.get(), w.b_self_qkv.get(),
-                                                 _buf_q.get(), k_cache, v_cache, _tw._head_num,
-                                                 _tw._dim_per_head, _tw._max_step, _cur_step,
-                                                 c[12] / Q, Q / c[18]));
+    // QKV product; its epilogue is ker_arrange_decself_qkv_i8I_i8O: q -> _buf_q, k / v -> slot
+    // _cur_step of the caches (all three with the cache clip)
+    if (_tw._dim_per_head % 16 == 0) {
+      _ops.decself_qkv(_buf_a.get(), w.w_self_qkv.get(), w.b_self_qkv.get(), _buf_q.get(), k_cache,
+                       v_cache, M, H, _tw._head_num, _tw._max_step, _cur_step,
+                       c[0] * c[6] / (c[12] * Q), c[12] / Q, Q / c[18], _stream);
+    } else {
+      LSH_CALL(gemm_i8_i8o(_buf_a.get(), w.w_self_qkv.get(), _buf_b.get(), M, 3 * H, H,
+                           c[0] * c[6] / (c[12] * Q), _stream));
+      LSH_CALL(arrange_decself_qkv_i8I_i8O<__half>(
+          M, H, _stream, _buf_b.get(), w.b_self_qkv.get(), _buf_q.get(), k_cache, v_cache,
+          _tw._head_num, _tw._dim_per_head, _tw._max_step, _cur_step, c[12] / Q, Q / c[18]));
+    }
+    TAP("self_q", _buf_q.get(), mh);
+    TAP("self_k_cache", k_cache, mh * _tw._max_step);
+    TAP("self_v_cache", v_cache, mh * _tw._max_step);
+    // int8 q.K -> softmax -> new value, one kernel
+    LSH_CALL(decself_attention_i8(_buf_q.get(), k_cache, v_cache, _buf_b.get(), M * _tw._head_num,
+                                  _cur_step + 1, _tw._max_step, _tw._head_num, _tw._dim_per_head,
+                                  attn_scale, c[18] / Q, Q / c[7], _stream, _ops.blocked));
   }
-  TAP("self_q", _buf_q.get(), mh);
-  TAP("self_k_cache", k_cache, mh * _tw._max_step);
-  TAP("self_v_cache", v_cache, mh * _tw._max_step);
-  // int8 q.K -> softmax -> new value, one kernel
-  LSH_CALL(decself_attention_i8(_buf_q.get(), k_cache, v_cache, _buf_b.get(), M * _tw._head_num,
-                                _cur_step + 1, _tw._max_step, _tw._head_num, _tw._dim_per_head,
-                                attn_scale, c[18] / Q, Q / c[7], _stream));
-  }
-  TAP("self_ctx_q", _buf_b.get(), mh);
-  LSH_CALL(gemm_i8_i8o(_buf_b.get(), w.w_self_out.get(), _buf_a.get(), M, H, H,
-                       c[1] * c[7] / (c[13] * Q), _stream));
+  TAP_CODES("self_ctx_q", _buf_b.get(), H);
+  _ops.i8o(_buf_b.get(), w.w_self_out.get(), _buf_a.get(), M, H, H, c[1] * c[7] / (c[13] * Q),
+           _stream);
   TAP("self_out_q", _buf_a.get(), mh);
   LSH_CALL((residual_bias_ln_i8O<__half, int8_t>(
       _buf_a.get(), w.encdec_ln_scale.get(), w.encdec_ln_bias.get(), w.b_encdec_out.get(),
       _buf_b.get(), _cur_step_query.get(), M, H, c[13] / Q, Q / c[8], _stream, _tw._is_post_ln,
-      nullptr)));
-  TAP("encdec_ln_q", _buf_b.get(), mh);
+      nullptr, 1, 0, _ops.blocked)));
+  TAP_CODES("encdec_ln_q", _buf_b.get(), H);
   TAP("res_self", _cur_step_query.get(), mh * sizeof(__half));
 }
 
@@ -453,25 +464,25 @@ void QuantDecoder::encdec_attention() {
   // the rows of _buf_b).  With taps set the launches below run.
   if (!step_taps.any() && _tw._dim_per_head == 64 &&
       encdec_q_attention_supported(_tw._beam_size, _tw._head_num, H, _batch_seq_len)) {
-    int8_t* ctx_q = _buf_a.get() + mh;
+    int8_t* ctx_q = _buf_a.get() + _ops.rows(M) * H;
     LSH_CALL(encdec_q_attention_f16(
         _buf_b.get(), w.w_encdec_q.get(), w.b_encdec_q.get(),
         _encdec_k.get() + (size_t)_layer_id * _layer_size_encdec_k,
         _encdec_v.get() + (size_t)_layer_id * _layer_size_encdec_k, _p_d_padding_mask, ctx_q,
         Q / c[9], _batch_size, _tw._beam_size, _tw._head_num, _batch_seq_len, H,
-        c[2] * c[8] / (c[14] * Q), c[14] / Q, _stream));
-    LSH_CALL(gemm_i8_i8o(ctx_q, w.w_encdec_out.get(), _buf_a.get(), M, H, H,
-                         c[3] * c[9] / (c[15] * Q), _stream));
+        c[2] * c[8] / (c[14] * Q), c[14] / Q, _stream, _ops.blocked));
+    _ops.i8o(ctx_q, w.w_encdec_out.get(), _buf_a.get(), M, H, H, c[3] * c[9] / (c[15] * Q), _stream);
     LSH_CALL((residual_bias_ln_i8O<__half, int8_t>(
         _buf_a.get(), w.ffn_ln_scale.get(), w.ffn_ln_bias.get(), w.b_ffn2.get(), _buf_b.get(),
-        _cur_step_query.get(), M, H, c[15] / Q, Q / c[10], _stream, _tw._is_post_ln, nullptr)));
+        _cur_step_query.get(), M, H, c[15] / Q, Q / c[10], _stream, _tw._is_post_ln, nullptr, 1, 0,
+        _ops.blocked)));
     return;
   }
   // q product; its epilogue is ker_arrange_encdec_q_i8I (fp16 q [batch, heads, beam, d])
   if (_tw._dim_per_head % 16 == 0) {
-    LSH_CALL(gemm_i8_encdec_q_f16(_buf_b.get(), w.w_encdec_q.get(), w.b_encdec_q.get(),
-                                  _query_buf1.get(), M, H, H, _tw._beam_size, _tw._head_num,
-                                  c[2] * c[8] / (c[14] * Q), c[14] / Q, _stream));
+    LSH_CALL((_ops.blocked ? gemm_blk_encdec_q : gemm_i8_encdec_q_f16)(
+        _buf_b.get(), w.w_encdec_q.get(), w.b_encdec_q.get(), _query_buf1.get(), M, H, H,
+        _tw._beam_size, _tw._head_num, c[2] * c[8] / (c[14] * Q), c[14] / Q, _stream));
   } else {
     LSH_CALL(gemm_i8_i8o(_buf_b.get(), w.w_encdec_q.get(), _buf_a.get(), M, H, H,
                          c[2] * c[8] / (c[14] * Q), _stream));
@@ -489,15 +500,16 @@ void QuantDecoder::encdec_attention() {
       _query_buf1.get(), _encdec_k.get() + (size_t)_layer_id * _layer_size_encdec_k,
       _encdec_v.get() + (size_t)_layer_id * _layer_size_encdec_k, _p_d_padding_mask, nullptr,
       _buf_b.get(), Q / c[9], _batch_size, _tw._beam_size, _tw._head_num, _batch_seq_len,
-      _tw._dim_per_head, _stream));
-  TAP("encdec_ctx_q", _buf_b.get(), mh);
-  LSH_CALL(gemm_i8_i8o(_buf_b.get(), w.w_encdec_out.get(), _buf_a.get(), M, H, H,
-                       c[3] * c[9] / (c[15] * Q), _stream));
+      _tw._dim_per_head, _stream, _ops.blocked));
+  TAP_CODES("encdec_ctx_q", _buf_b.get(), H);
+  _ops.i8o(_buf_b.get(), w.w_encdec_out.get(), _buf_a.get(), M, H, H, c[3] * c[9] / (c[15] * Q),
+           _stream);
   TAP("encdec_out_q", _buf_a.get(), mh);
   LSH_CALL((residual_bias_ln_i8O<__half, int8_t>(
       _buf_a.get(), w.ffn_ln_scale.get(), w.ffn_ln_bias.get(), w.b_ffn2.get(), _buf_b.get(),
-      _cur_step_query.get(), M, H, c[15] / Q, Q / c[10], _stream, _tw._is_post_ln, nullptr)));
-  TAP("ffn_ln_q", _buf_b.get(), mh);
+      _cur_step_query.get(), M, H, c[15] / Q, Q / c[10], _stream, _tw._is_post_ln, nullptr, 1, 0,
+        _ops.blocked)));
+  TAP_CODES("ffn_ln_q", _buf_b.get(), H);
   TAP("res_encdec", _cur_step_query.get(), mh * sizeof(__half));
 }
 
@@ -508,15 +520,13 @@ void QuantDecoder::ffn_add_norm() {
   const float Q = _quant_range;
 
   // FFN1 GEMM with the bias + activation + requantisation in its epilogue
-  LSH_CALL(gemm_i8_lut_i8o(_buf_b.get(), w.w_ffn1.get(), _buf_a.get(), w.ffn1_act_lut.get(), M, I,
-                           H, c[4] * c[10] / (c[16] * Q), _stream));
-  TAP("ffn1_act_q", _buf_a.get(), (size_t)M * I);
-  int nparts = 1;
+  _ops.lut(_buf_b.get(), w.w_ffn1.get(), _buf_a.get(), w.ffn1_act_lut.get(), M, I, H,
+           c[4] * c[10] / (c[16] * Q), _stream);
+  TAP_CODES("ffn1_act_q", _buf_a.get(), I);
   // a tapped accumulator is one plane (the planes of a split product sum to it exactly)
   const bool tap_acc = step_taps.wants(_layer_id, _cur_step, "ffn2_acc");
-  LSH_CALL(gemm_i8_i32o_splitk(_buf_a.get(), w.w_ffn2.get(), _int32_ffn_out_buf.get(), M, H, I,
-                               tap_acc ? 1 : gemm_i8_preferred_ksplit(M, H, I), &nparts,
-                               _stream));
+  const int nparts = _ops.i32o(_buf_a.get(), w.w_ffn2.get(), _int32_ffn_out_buf.get(), M, H, I,
+                               tap_acc ? 1 : 8, _stream);
   TAP("ffn2_acc", _int32_ffn_out_buf.get(), (size_t)M * H * sizeof(int32_t));
 
   const float dequant_scale =
@@ -538,12 +548,14 @@ void QuantDecoder::ffn_add_norm() {
   LSH_CALL((residual_bias_ln_i8O<__half, int32_t>(
       _int32_ffn_out_buf.get(), scale_ptr, bias_ptr, res_bias_ptr, _buf_a.get(),
       _cur_step_query.get(), M, H, dequant_scale, Q / clip_max, _stream, _tw._is_post_ln,
-      w.ffn2_colsum.get(), nparts, (long)M * H)));
-  TAP("next_ln_q", _buf_a.get(), (size_t)M * H);
+      w.ffn2_colsum.get(), nparts, (long)M * H,
+      _ops.blocked && (!_qkv_attn || _layer_id == _tw._n_dec_layer - 1))));
+  TAP_CODES("next_ln_q", _buf_a.get(), H);
   TAP("res_out", _cur_step_query.get(), (size_t)M * H * sizeof(__half));
 }
 
 #undef TAP
+#undef TAP_CODES
 
 // QuantDecoder::sample and ::topk_greedy_search after its first step
 // (inference/model/quant_decoder.cc.cu:952-984, 1108-1131): one token per row, in place
@@ -555,13 +567,13 @@ void QuantDecoder::sample_tokens() {
     LSH_CALL(dec_topp_sample_i8I<__half>(_step_token_num, _cur_step + 1, _tw._max_step, 1, _stream,
                                          _logits.get(), _logit_bias.get(), alive,
                                          _tw._trg_vocab_size, _tw._topp, _sample_unfinished.get(),
-                                         _sample_state.get(), _tw._end_id, dq));
+                                         _sample_state.get(), _tw._end_id, dq, _logits_stride));
   } else {
     const int k = _tw._sampling_method == "topk" ? _tw._topk : 1;
     LSH_CALL(dec_topk_sample_i8I<__half>(_step_token_num, _cur_step + 1, _tw._max_step, 1, _stream,
                                          _logits.get(), _logit_bias.get(), alive,
                                          _tw._trg_vocab_size, k, _sample_unfinished.get(),
-                                         _sample_state.get(), _tw._end_id, dq));
+                                         _sample_state.get(), _tw._end_id, dq, _logits_stride));
   }
   if (_rec_alive && _cur_step < _rec_max_steps)
     CHECK_GPU_ERROR(hipMemcpyAsync(
@@ -577,7 +589,7 @@ void QuantDecoder::beam_search() {
       alive_new, _top_score.get(), _top_idx.get(), _parent.get(), _num_finished.get(),
       _logits_clip_max / _quant_range, _tw._trg_vocab_size, _tw._max_step,
       _h_length_norm[_cur_step], _cur_step, _batch_size, _tw._beam_size, _tw._end_id, _stream,
-      _topk_part_ws.get(), _topk_part_ws.size()));
+      _topk_part_ws.get(), _topk_part_ws.size(), _logits_stride));
   if (_rec_alive && _cur_step < _rec_max_steps)
     CHECK_GPU_ERROR(hipMemcpyAsync(
         _rec_alive + (size_t)_cur_step * _step_token_num * _tw._max_step, alive_new,

@@ -112,11 +112,17 @@ class QuantDecoder {
   DeviceBuffer<int> _sample_unfinished;           // the flag of a sampling step
   DeviceBuffer<unsigned long long> _sample_state;  // lsh_rng_state_t per row (16 bytes each)
   // weights
-  DeviceBuffer<int8_t> _int8_trg_emb;  // [vocab, H]: embedding rows and logits kernel
+  // [vocab, H]: embedding rows, and the logits kernel where operands are row-major; blocked and
+  // padded to whole tiles otherwise
+  DeviceBuffer<int8_t> _int8_trg_emb, _emb_blk;
+  LayerProducts _ops;
+  int _logits_stride = 0;  // codes from one row of logits to the next
+  bool _qkv_attn = false;  // this step runs the opt-in launch of QKV product and attention
   DeviceBuffer<__half> _pos_emb, _out_ln_scale, _out_ln_bias, _kv_kernel /*[n_layer*2*H, H]*/,
       _kv_bias, _logit_bias;
   struct Layer {
     DeviceBuffer<int8_t> w_self_qkv, w_self_out, w_encdec_q, w_encdec_out, w_ffn1, w_ffn2;
+    DeviceBuffer<int8_t> w_self_qkv_rows;  // row-major, made when the opt-in launch first asks
     DeviceBuffer<int8_t> ffn1_act_lut;  // [inner, 256]: bias + activation + requant per code
     DeviceBuffer<__half> self_ln_scale, self_ln_bias, b_self_qkv, b_self_out, encdec_ln_scale,
         encdec_ln_bias, b_encdec_q, b_encdec_out, ffn_ln_scale, ffn_ln_bias, b_ffn1, b_ffn2,

@@ -66,15 +66,17 @@ void QuantGptEncoder::init_buffer() {
   set_seed(0);
   CHECK_GPU_ERROR(hipHostMalloc(reinterpret_cast<void**>(&_h_unfinished), sizeof(int)));
   *_h_unfinished = 0;
+  _ops.blocked = LayerProducts::can_block(H, I, _tw._dim_per_head);
+  _logits_stride = _ops.blocked ? (V + 63) & ~63 : V;
   _query.alloc((size_t)_max_batch_dim);
   _qkv_buf.alloc((size_t)(3 * _max_batch_dim));
-  const size_t wide = tokens * (size_t)std::max(I, 3 * H);
+  const size_t wide = _ops.rows(tokens) * (size_t)std::max(I, 3 * H);
   _buf_a.alloc(wide);
   _buf_b.alloc(wide);
   _buf_q.alloc(wide);
-  _hid_last.alloc((size_t)_max_batch_size * H);
+  for (auto& h : _hid_last) h.alloc(_ops.rows(_max_batch_size) * H);
   // perplexity needs the logits of every position, sampling only of the last one
-  _logits.alloc((_tw._sampling_method == "ppl" ? tokens : (size_t)_max_batch_size) * V);
+  _logits.alloc((_tw._sampling_method == "ppl" ? tokens : (size_t)_max_batch_size) * _logits_stride);
   // room for the accumulator planes of the split-K second FFN product
   _int32_ffn_out_buf.alloc(std::max(tokens * H * 4, (size_t)64 * H * 8));
   _self_k_cache.alloc((size_t)L * _max_batch_dim);
@@ -82,8 +84,10 @@ void QuantGptEncoder::init_buffer() {
   CHECK_GPU_ERROR(hipMemsetAsync(_self_k_cache.get(), 0, _self_k_cache.size(), _stream));
   CHECK_GPU_ERROR(hipMemsetAsync(_self_v_cache.get(), 0, _self_v_cache.size(), _stream));
 
-  // stored [H, vocab]; one [vocab, H] copy serves the row lookup and the logits GEMM
+  // stored [H, vocab]; a [vocab, H] copy serves the row lookup and, where products run on
+  // row-major operands, the logits; a blocked one padded to whole tiles serves them otherwise
   _int8_emb = upload_kernel(_tw.token_embedding, H, V, true, _stream);
+  if (_ops.blocked) _emb_blk = block_weight_padded(_int8_emb, V, H, _stream);
   _pos_emb = upload_half(_tw.position_embedding, _stream);
   _out_ln_scale = upload_half(_tw.norm_scale, _stream);
   _out_ln_bias = upload_half(_tw.norm_bias, _stream);
@@ -100,16 +104,16 @@ void QuantGptEncoder::init_buffer() {
     d.ln2_bias = upload_half(w.ffn_norm_bias, _stream);
     d.b_ffn1 = upload_half(w.ffn_first_bias, _stream);
     d.b_ffn2 = upload_half(w.ffn_second_bias, _stream);
-    d.w_qkv = upload_kernel(w.multihead_project_kernel_qkv, H, 3 * H, true, _stream);
-    d.w_out = upload_kernel(w.multihead_project_kernel_output, H, H, true, _stream);
-    d.w_ffn1 = upload_kernel(w.ffn_first_kernel, H, I, true, _stream);
+    d.w_qkv = _ops.weight(w.multihead_project_kernel_qkv, H, 3 * H, _stream);
+    d.w_out = _ops.weight(w.multihead_project_kernel_output, H, H, _stream);
+    d.w_ffn1 = _ops.weight(w.ffn_first_kernel, H, I, _stream);
     {
       const float* c = &_enc_clip_max[l * 12];
       d.ffn1_act_lut.alloc((size_t)I * 256);
       LSH_CALL(build_act_lut(d.ffn1_act_lut.get(), d.b_ffn1.get(), I, c[10] / _quant_range,
                              _quant_range / c[7], c[7], kActGelu, _stream));
     }
-    d.w_ffn2 = upload_kernel(w.ffn_second_kernel, I, H, true, _stream);
+    d.w_ffn2 = _ops.weight(w.ffn_second_kernel, I, H, _stream);
   }
   CHECK_GPU_ERROR(hipStreamSynchronize(_stream));
 }
@@ -122,23 +126,21 @@ void QuantGptEncoder::init_buffer() {
 //   max_step, d] after the append;  res_in, res_attn, res_out: the fp16 residual stream [batch,
 //   hidden] at the start of the layer, after the first and after the last layer norm
 #define TAP(name, ptr, bytes) step_taps.copy(_layer_id, _tap_step, name, ptr, bytes, _stream)
+#define TAP_CODES(name, ptr, rows, cols) \
+  step_taps.copy_codes(_layer_id, _tap_step, name, ptr, rows, cols, _ops.blocked, _stream)
 
-void QuantGptEncoder::ffn_add_norm(int rows, int8_t* in, int8_t* tmp) {
+void QuantGptEncoder::ffn_add_norm(int rows, int8_t* in, int8_t* tmp, bool blocked_out) {
   const int H = _tw._hidden_size, I = _tw._inner_size;
   const Layer& w = _layers[_layer_id];
   const float* c = &_enc_clip_max[_layer_id * 12];
   const float Q = _quant_range;
-  LSH_CALL(gemm_i8_lut_i8o(in, w.w_ffn1.get(), tmp, w.ffn1_act_lut.get(), rows, I, H,
-                           c[2] * c[6] / (c[10] * Q), _stream));
-  TAP("act_q", tmp, (size_t)rows * I);
-  int nparts = 1;
+  _ops.lut(in, w.w_ffn1.get(), tmp, w.ffn1_act_lut.get(), rows, I, H, c[2] * c[6] / (c[10] * Q),
+           _stream);
+  TAP_CODES("act_q", tmp, rows, I);
   // a tapped accumulator is one plane (the planes of a split product sum to it exactly)
   const bool tap_acc = step_taps.wants(_layer_id, _tap_step, "ffn2_acc");
-  LSH_CALL(gemm_i8_i32o_splitk(tmp, w.w_ffn2.get(), _int32_ffn_out_buf.get(), rows, H, I,
-                               tap_acc      ? 1
-                               : rows <= 64 ? gemm_i8_preferred_ksplit(rows, H, I)
-                                            : std::min(4, gemm_i8_preferred_ksplit(rows, H, I)),
-                               &nparts, _stream));
+  const int nparts = _ops.i32o(tmp, w.w_ffn2.get(), _int32_ffn_out_buf.get(), rows, H, I,
+                               tap_acc ? 1 : rows <= 64 ? 8 : 4, _stream);
   TAP("ffn2_acc", _int32_ffn_out_buf.get(), (size_t)rows * H * sizeof(int32_t));
   const float dequant_scale = c[3] * c[7] / (Q * Q);
   const __half *scale_ptr, *bias_ptr, *res_bias_ptr;
@@ -157,14 +159,14 @@ void QuantGptEncoder::ffn_add_norm(int rows, int8_t* in, int8_t* tmp) {
   }
   LSH_CALL((residual_bias_ln_i8O<__half, int32_t>(
       _int32_ffn_out_buf.get(), scale_ptr, bias_ptr, res_bias_ptr, in, _query.get(), rows, H,
-      dequant_scale, Q / clip_max, _stream, false, nullptr, nparts, (long)rows * H)));
-  TAP("next_ln_q", in, (size_t)rows * H);
+      dequant_scale, Q / clip_max, _stream, false, nullptr, nparts, (long)rows * H, blocked_out)));
+  TAP_CODES("next_ln_q", in, rows, H);
   TAP("res_out", _query.get(), (size_t)rows * H * sizeof(__half));
 }
 
 // all prompt positions at once (:253-291 / :299-341); leaves the int8 LayerNorm output of
-// the last layer in _buf_a
-void QuantGptEncoder::prompt_pass(const int* ids) {
+// the last layer in _buf_a, row-major where the caller picks positions from it
+void QuantGptEncoder::prompt_pass(const int* ids, bool row_major_out) {
   const int H = _tw._hidden_size, M = _batch_token_num;
   const float Q = _quant_range;
   CHECK_GPU_ERROR(hipMemsetAsync(_real_seq_len.get(), 0, sizeof(int) * _batch_size, _stream));
@@ -184,8 +186,9 @@ void QuantGptEncoder::prompt_pass(const int* ids) {
     const float* c = &_enc_clip_max[_layer_id * 12];
     if (_layer_id == 0)
       LSH_CALL(norm_layer_resual_i8O<__half>(M, H, _stream, _query.get(), a, w.ln1_scale.get(),
-                                             w.ln1_bias.get(), w.b_out.get(), Q / c[4], false));
-    LSH_CALL(gemm_i8_i8o(a, w.w_qkv.get(), b, M, 3 * H, H, c[0] * c[4] / (c[8] * Q), _stream));
+                                             w.ln1_bias.get(), w.b_out.get(), Q / c[4], false,
+                                             _ops.blocked));
+    _ops.i8o(a, w.w_qkv.get(), b, M, 3 * H, H, c[0] * c[4] / (c[8] * Q), _stream);
     int8_t* k_cache = _self_k_cache.get() + (size_t)_layer_id * _max_batch_dim;
     int8_t* v_cache = _self_v_cache.get() + (size_t)_layer_id * _max_batch_dim;
     if (on_codes) {
@@ -197,20 +200,23 @@ void QuantGptEncoder::prompt_pass(const int* ids) {
                                           _tw._max_step, c[8] / Q, Q / c[11]));
       LSH_CALL(gpt_prefill_attention_i8(q8, k_cache, v_cache, _real_seq_len.get(), a, Q / c[5],
                                         c[11] / Q, Q / c[11], _batch_size, _batch_seq_len,
-                                        _tw._head_num, _tw._dim_per_head, _tw._max_step, _stream));
+                                        _tw._head_num, _tw._dim_per_head, _tw._max_step, _stream,
+                                        _ops.blocked));
     } else {
       LSH_CALL(gpt_arrange_qkv_prefill_f16(M, H, _stream, b, w.b_qkv.get(), qc, kc, vd, k_cache,
                                            v_cache, _batch_seq_len, _tw._dim_per_head,
                                            _tw._head_num, _tw._max_step, c[8] / Q, Q / c[11]));
-      LSH_CALL(gpt_prefill_attention_f16(qc, kc, vd, _real_seq_len.get(), nullptr, a, Q / c[5],
-                                         c[11] / Q, _batch_size, _batch_seq_len, _tw._head_num,
-                                         _tw._dim_per_head, _stream));
+      LSH_CALL(gpt_prefill_attention_f16(qc, kc, vd, _real_seq_len.get(), nullptr,
+                                         _ops.blocked ? b : a, Q / c[5], c[11] / Q, _batch_size,
+                                         _batch_seq_len, _tw._head_num, _tw._dim_per_head, _stream));
+      if (_ops.blocked) LSH_CALL(block_rows(b, a, M, H, false, _stream));
     }
-    LSH_CALL(gemm_i8_i8o(a, w.w_out.get(), b, M, H, H, c[1] * c[5] / (c[9] * Q), _stream));
+    _ops.i8o(a, w.w_out.get(), b, M, H, H, c[1] * c[5] / (c[9] * Q), _stream);
     LSH_CALL((residual_bias_ln_i8O<__half, int8_t>(b, w.ln2_scale.get(), w.ln2_bias.get(),
                                                    w.b_ffn2.get(), a, _query.get(), M, H,
-                                                   c[9] / Q, Q / c[6], _stream, false, nullptr)));
-    ffn_add_norm(M, a, b);
+                                                   c[9] / Q, Q / c[6], _stream, false, nullptr, 1,
+                                                   0, _ops.blocked)));
+    ffn_add_norm(M, a, b, _ops.blocked && !(row_major_out && _layer_id == _tw._n_enc_layer - 1));
   }
 }
 
@@ -224,6 +230,11 @@ const int8_t* QuantGptEncoder::step_pass() {
   _tap_step = _steps_run;
   // the step's embedding and the first layer norm are one launch where the row kernel covers
   // the width (the same bytes); with taps set the two launches run
+  // the opt-in launch of the QKV product and the attention reads row-major operands
+  const bool qkv_attn = !step_taps.any() && decself_qkv_attention_enabled() &&
+                        _tw._dim_per_head == 64 &&
+                        decself_qkv_attention_supported(B, H, _tw._head_num, _tw._max_step);
+  const bool ln1_blocked = _ops.blocked && !qkv_attn;
   const bool emb_ln_fused = !step_taps.any() && H % 4 == 0 && H <= 1024 && _tw._n_enc_layer > 0;
   if (emb_ln_fused) {
     const Layer& w0 = _layers[0];
@@ -231,7 +242,7 @@ const int8_t* QuantGptEncoder::step_pass() {
         _int8_emb.get(), _pos_emb.get(), _last_ids.get(), _query.get(), a, w0.ln1_scale.get(),
         w0.ln1_bias.get(), w0.b_out.get(), _real_seq_len.get(), _unfinished.get(), B, H,
         _tw._src_vocab_size, _tw._padding_id, _batch_seq_len - 1, _tw._max_step,
-        _src_emb_clip_max / Q, Q / _enc_clip_max[4], false, _stream));
+        _src_emb_clip_max / Q, Q / _enc_clip_max[4], false, _stream, ln1_blocked));
   } else {
     LSH_CALL(gpt_embedding_i8I<__half>(B, 1, H, _stream, _int8_emb.get(), _pos_emb.get(),
                                        _last_ids.get(), _query.get(), _real_seq_len.get(),
@@ -240,55 +251,48 @@ const int8_t* QuantGptEncoder::step_pass() {
   }
   const size_t bh = (size_t)B * H;
   for (_layer_id = 0; _layer_id < _tw._n_enc_layer; _layer_id++) {
-    const Layer& w = _layers[_layer_id];
+    Layer& w = _layers[_layer_id];
     const float* c = &_enc_clip_max[_layer_id * 12];
     int8_t* k_cache = _self_k_cache.get() + (size_t)_layer_id * _max_batch_dim;
     int8_t* v_cache = _self_v_cache.get() + (size_t)_layer_id * _max_batch_dim;
     if (_layer_id == 0 && !emb_ln_fused)
       LSH_CALL(norm_layer_resual_i8O<__half>(B, H, _stream, _query.get(), a, w.ln1_scale.get(),
-                                             w.ln1_bias.get(), w.b_out.get(), Q / c[4], false));
-    TAP("ln1_q", a, bh);
+                                             w.ln1_bias.get(), w.b_out.get(), Q / c[4], false, ln1_blocked));
+    TAP_CODES("ln1_q", a, B, H);
     TAP("res_in", _query.get(), bh * sizeof(__half));
     // With taps set the two launches run, so that q and the caches are copied before the
     // attention as the tap names promise.
-    if (!step_taps.any() && decself_qkv_attention_enabled() && _tw._dim_per_head == 64 &&
-        decself_qkv_attention_supported(B, H, _tw._head_num, _tw._max_step)) {
-      LSH_CALL(decself_qkv_attention_i8(a, w.w_qkv.get(), w.b_qkv.get(), _buf_q.get(), k_cache,
-                                        v_cache, b, B, H, _tw._head_num, _tw._max_step,
-                                        _batch_seq_len - 1, c[0] * c[4] / (c[8] * Q), c[8] / Q,
-                                        Q / c[11], _atten_scaler, c[11] / Q, Q / c[5], _stream));
+    if (qkv_attn) {
+      if (_ops.blocked && !w.w_qkv_rows.get()) w.w_qkv_rows = unblock_weight(w.w_qkv, 3 * H, H, _stream);
+      LSH_CALL(decself_qkv_attention_i8(
+          a, (_ops.blocked ? w.w_qkv_rows : w.w_qkv).get(), w.b_qkv.get(), _buf_q.get(), k_cache,
+          v_cache, b, B, H, _tw._head_num, _tw._max_step, _batch_seq_len - 1,
+          c[0] * c[4] / (c[8] * Q), c[8] / Q, Q / c[11], _atten_scaler, c[11] / Q, Q / c[5], _stream,
+          _ops.blocked));
     } else {
-    // QKV product; its epilogue is ker_arrange_decself_qkv_i8I_i8O: q -> _buf_q, k / v appended
-    // to the caches at the token's position
-    if (_tw._dim_per_head % 16 == 0) {
-      LSH_CALL(gemm_i8_decself_qkv_i8o(a, w.w_qkv.get(), w.b_qkv.get(), _buf_q.get(), k_cache,
-                                       v_cache, B, H, H, _tw._head_num, _tw._max_step,
-                                       _batch_seq_len - 1, c[0] * c[4] / (c[8] * Q), c[8] / Q,
-                                       Q / c[11], _stream));
-    } else {
-      LSH_CALL(gemm_i8_i8o(a, w.w_qkv.get(), b, B, 3 * H, H, c[0] * c[4] / (c[8] * Q), _stream));
-      LSH_CALL(arrange_decself_qkv_i8I_i8O<__half>(B, H, _stream, b, w.b_qkv.get(), _buf_q.get(),
-                                                   k_cache, v_cache, _tw._head_num,
-                                                   _tw._dim_per_head, _tw._max_step,
-                                                   _batch_seq_len - 1, c[8] / Q, Q / c[11]));
+      // QKV product; its epilogue is ker_arrange_decself_qkv_i8I_i8O: q -> _buf_q, k / v appended
+      // to the caches at the token's position
+      _ops.decself_qkv(a, w.w_qkv.get(), w.b_qkv.get(), _buf_q.get(), k_cache, v_cache, B, H,
+                       _tw._head_num, _tw._max_step, _batch_seq_len - 1, c[0] * c[4] / (c[8] * Q),
+                       c[8] / Q, Q / c[11], _stream);
+      TAP("self_q", _buf_q.get(), bh);
+      TAP("k_cache", k_cache, bh * _tw._max_step);
+      TAP("v_cache", v_cache, bh * _tw._max_step);
+      LSH_CALL(decself_attention_i8(_buf_q.get(), k_cache, v_cache, b, B * _tw._head_num,
+                                    _batch_seq_len, _tw._max_step, _tw._head_num,
+                                    _tw._dim_per_head, _atten_scaler, c[11] / Q, Q / c[5], _stream,
+                                    _ops.blocked));
     }
-    TAP("self_q", _buf_q.get(), bh);
-    TAP("k_cache", k_cache, bh * _tw._max_step);
-    TAP("v_cache", v_cache, bh * _tw._max_step);
-    LSH_CALL(decself_attention_i8(_buf_q.get(), k_cache, v_cache, b, B * _tw._head_num,
-                                  _batch_seq_len,
-                                  _tw._max_step, _tw._head_num, _tw._dim_per_head, _atten_scaler,
-                                  c[11] / Q, Q / c[5], _stream));
-    }
-    TAP("ctx_q", b, bh);
-    LSH_CALL(gemm_i8_i8o(b, w.w_out.get(), a, B, H, H, c[1] * c[5] / (c[9] * Q), _stream));
+    TAP_CODES("ctx_q", b, B, H);
+    _ops.i8o(b, w.w_out.get(), a, B, H, H, c[1] * c[5] / (c[9] * Q), _stream);
     TAP("out_q", a, bh);
     LSH_CALL((residual_bias_ln_i8O<__half, int8_t>(a, w.ln2_scale.get(), w.ln2_bias.get(),
                                                    w.b_ffn2.get(), b, _query.get(), B, H,
-                                                   c[9] / Q, Q / c[6], _stream, false, nullptr)));
-    TAP("ln2_q", b, bh);
+                                                   c[9] / Q, Q / c[6], _stream, false, nullptr, 1,
+                                                   0, _ops.blocked)));
+    TAP_CODES("ln2_q", b, B, H);
     TAP("res_attn", _query.get(), bh * sizeof(__half));
-    ffn_add_norm(B, b, a);
+    ffn_add_norm(B, b, a, _layer_id == _tw._n_enc_layer - 1 ? _ops.blocked : ln1_blocked);
     std::swap(a, b);  // `a` names the buffer holding the layer's int8 LayerNorm output
   }
   _tap_step = -2;
@@ -296,28 +300,35 @@ const int8_t* QuantGptEncoder::step_pass() {
 }
 
 #undef TAP
+#undef TAP_CODES
+
+// int8 logits of `rows` hidden rows, _logits_stride codes from one row to the next (:399-404)
+void QuantGptEncoder::logits_product(const int8_t* hidden, int rows) {
+  _ops.i8o(hidden, (_ops.blocked ? _emb_blk : _int8_emb).get(), _logits.get(), rows, _logits_stride,
+           _tw._hidden_size,
+           _output_ln_clip_max * _src_emb_clip_max / (_logits_clip_max * _quant_range), _stream);
+}
 
 // logits of the last position + greedy choice, enqueued only (:399-487)
 void QuantGptEncoder::enqueue_sampling(const int8_t* hidden, bool clear_flag) {
-  const int H = _tw._hidden_size, V = _tw._src_vocab_size, B = _batch_size;
-  LSH_CALL(gemm_i8_i8o(hidden, _int8_emb.get(), _logits.get(), B, V, H,
-                       _output_ln_clip_max * _src_emb_clip_max / (_logits_clip_max * _quant_range),
-                       _stream));
+  const int V = _tw._src_vocab_size, B = _batch_size;
+  logits_product(hidden, B);
   if (_rec_logits && _steps_run < _rec_max_steps)
-    CHECK_GPU_ERROR(hipMemcpyAsync(_rec_logits + (size_t)_steps_run * B * V, _logits.get(),
-                                   (size_t)B * V, hipMemcpyDeviceToDevice, _stream));
+    CHECK_GPU_ERROR(hipMemcpy2DAsync(_rec_logits + (size_t)_steps_run * B * V, V, _logits.get(),
+                                     _logits_stride, V, B, hipMemcpyDeviceToDevice, _stream));
   // (after a cached step the flag was cleared by the step's embedding launch)
   if (clear_flag) LSH_CALL(fill_i32(_unfinished.get(), 0, 1, _stream));
   const bool topp = _tw._sampling_method == "topp";
   if (!topp && _tw._topk == 1) {
     LSH_CALL(gpt_greedy_step(_logits.get(), _ids.get(), _last_ids.get(), V, _tw._max_step,
-                             _batch_seq_len, B, _unfinished.get(), _tw._eos_id, _stream));
+                             _batch_seq_len, B, _unfinished.get(), _tw._eos_id, _stream,
+                             _logits_stride));
   } else {
     // ker_topk_sample_i8I<k> / ker_topp_sample_i8I (:405-430, :448-473)
     LSH_CALL(gpt_sample_step(_logits.get(), _ids.get(), _last_ids.get(), V, _tw._max_step,
                              _batch_seq_len, B, _unfinished.get(), _tw._eos_id,
                              topp ? 0 : _tw._topk, _tw._topp, _logits_clip_max / _quant_range,
-                             _sample_state.get(), _stream));
+                             _sample_state.get(), _stream, _logits_stride));
   }
 }
 
@@ -360,16 +371,18 @@ int QuantGptEncoder::run_one_sample(int batch_size, int batch_seq_len) {
   CHECK_GPU_ERROR(hipMemcpy2DAsync(_ids.get(), sizeof(int) * _tw._max_step, _p_d_token_id,
                                    sizeof(int) * batch_seq_len, sizeof(int) * batch_seq_len,
                                    batch_size, hipMemcpyDeviceToDevice, _stream));
-  prompt_pass(_p_d_token_id);
+  prompt_pass(_p_d_token_id, true);
   // hidden states of the last prompt position of every sequence
-  CHECK_GPU_ERROR(hipMemcpy2DAsync(_hid_last.get(), H,
+  CHECK_GPU_ERROR(hipMemcpy2DAsync(_hid_last[0].get(), H,
                                    _buf_a.get() + (size_t)(batch_seq_len - 1) * H,
                                    (size_t)batch_seq_len * H, H, batch_size,
                                    hipMemcpyDeviceToDevice, _stream));
+  if (_ops.blocked)
+    LSH_CALL(block_rows(_hid_last[0].get(), _hid_last[1].get(), batch_size, H, false, _stream));
   int loop_steps = 0;
   if (_batch_seq_len < _tw._max_step) {
     // (:347-353) after the prompt pass the run ends when nothing is unfinished
-    enqueue_sampling(_hid_last.get(), true);
+    enqueue_sampling(_hid_last[_ops.blocked].get(), true);
     const bool go_on = !(finish_token() == 0 || _batch_seq_len >= _batch_max_seq_len);
     _phases.mark(1, _stream);
     if (go_on) {
@@ -406,17 +419,15 @@ void QuantGptEncoder::run_one_infer(int batch_size, int batch_seq_len) {
   _batch_size = batch_size;
   _batch_seq_len = batch_seq_len;
   _batch_token_num = batch_size * batch_seq_len;
-  const int H = _tw._hidden_size, V = _tw._src_vocab_size;
+  const int V = _tw._src_vocab_size;
   CHECK_GPU_ERROR(hipMemsetAsync(_p_d_ppl, 0, sizeof(float) * batch_size, _stream));
-  prompt_pass(_p_d_token_id);
+  prompt_pass(_p_d_token_id, false);
   /* compute_ppl (:781-797) */
-  LSH_CALL(gemm_i8_i8o(_buf_a.get(), _int8_emb.get(), _logits.get(), _batch_token_num, V, H,
-                       _output_ln_clip_max * _src_emb_clip_max / (_logits_clip_max * _quant_range),
-                       _stream));
+  logits_product(_buf_a.get(), _batch_token_num);
   // the FFN2 accumulator buffer (tokens * hidden int32, idle by now) holds the per-position terms
   LSH_CALL(ppl_i8I(batch_size, batch_seq_len, _stream, _logits.get(), _p_d_token_id,
                    _real_seq_len.get(), _p_d_ppl, V, _logits_clip_max / _quant_range,
-                   reinterpret_cast<float*>(_int32_ffn_out_buf.get())));
+                   reinterpret_cast<float*>(_int32_ffn_out_buf.get()), _logits_stride));
 }
 
 }  // namespace hip

@@ -60,9 +60,10 @@ class QuantGptEncoder {
   int* _p_d_sample_id;
 
  private:
-  void prompt_pass(const int* ids);
+  void prompt_pass(const int* ids, bool row_major_out);
   const int8_t* step_pass();
-  void ffn_add_norm(int rows, int8_t* in, int8_t* tmp);
+  void ffn_add_norm(int rows, int8_t* in, int8_t* tmp, bool blocked_out);
+  void logits_product(const int8_t* hidden, int rows);
   void enqueue_sampling(const int8_t* hidden, bool clear_flag);
   int finish_token();
 
@@ -89,13 +90,17 @@ class QuantGptEncoder {
   DeviceBuffer<int> _real_seq_len, _ids, _last_ids, _unfinished;
   DeviceBuffer<long long> _sample_state;  // lsh_rng_state_t [max_batch_size]
   DeviceBuffer<__half> _query, _qkv_buf;  // q codes | k codes | v, each max_batch_dim
-  DeviceBuffer<int8_t> _buf_a, _buf_b, _buf_q, _hid_last, _logits;
+  DeviceBuffer<int8_t> _buf_a, _buf_b, _buf_q, _logits;
+  DeviceBuffer<int8_t> _hid_last[2];  // row-major, and as the logits product reads it
   DeviceBuffer<int32_t> _int32_ffn_out_buf;
   DeviceBuffer<int8_t> _self_k_cache, _self_v_cache;  // [n_layer][max_batch_dim]
-  DeviceBuffer<int8_t> _int8_emb;                     // [vocab, H]
+  DeviceBuffer<int8_t> _int8_emb, _emb_blk;           // [vocab, H]; blocked, padded
+  LayerProducts _ops;
+  int _logits_stride = 0;  // codes from one row of logits to the next
   DeviceBuffer<__half> _pos_emb, _out_ln_scale, _out_ln_bias;
   struct Layer {
     DeviceBuffer<int8_t> w_qkv, w_out, w_ffn1, w_ffn2;
+    DeviceBuffer<int8_t> w_qkv_rows;    // row-major, made when the opt-in launch first asks
     DeviceBuffer<int8_t> ffn1_act_lut;  // [inner, 256]: bias + GELU + requant per code
     DeviceBuffer<__half> ln1_scale, ln1_bias, b_qkv, b_out, ln2_scale, ln2_bias, b_ffn1, b_ffn2;
   };

@@ -116,7 +116,7 @@ __device__ int dec_sample_row(const int8_t* __restrict__ lr, const T* __restrict
 
 template <typename T>
 __global__ void __launch_bounds__(kSampleThreads)
-dec_sample_kernel(const int8_t* __restrict__ logits, const T* __restrict__ bias, int* ids,
+dec_sample_kernel(const int8_t* __restrict__ logits, long ldl, const T* __restrict__ bias, int* ids,
                   int vocab, int max_step, int cur_len, int logits_seq_len, int* unfinished,
                   int eos_id, int k, float p, float scale, SampleState* st) {
   __shared__ SampleShared sh;
@@ -126,7 +126,7 @@ dec_sample_kernel(const int8_t* __restrict__ logits, const T* __restrict__ bias,
     if (threadIdx.x == 0) ids[last + 1] = eos_id;
     return;
   }
-  const int8_t* lr = logits + ((long)b * logits_seq_len + logits_seq_len - 1) * vocab;
+  const int8_t* lr = logits + ((long)b * logits_seq_len + logits_seq_len - 1) * ldl;
   const int tok = dec_sample_row<T>(lr, bias, vocab, k, p, scale, st ? st + b : nullptr, sh);
   if (threadIdx.x == 0) {
     if (tok != eos_id) unfinished[0] = 1;
@@ -137,18 +137,19 @@ dec_sample_kernel(const int8_t* __restrict__ logits, const T* __restrict__ bias,
 template <typename T>
 int dec_sample(const char* who, int rows, int cur_len, int max_step, int logits_seq_len,
                hipStream_t s, const int8_t* logits, const T* bias, int* ids, int vocab, int k,
-               float p, int* unfinished, void* state, int eos_id, float scale) {
+               float p, int* unfinished, void* state, int eos_id, float scale, int ldl) {
+  if (ldl == 0) ldl = vocab;
   const std::string w(who);
   if (!logits || !bias || !ids || !unfinished || rows <= 0 || cur_len <= 0 ||
-      cur_len >= max_step || logits_seq_len <= 0 || vocab <= 0)
+      cur_len >= max_step || logits_seq_len <= 0 || vocab <= 0 || ldl < vocab)
     return lsh_fail(LSH_ERR_INVALID, (w + ": bad arguments").c_str());
   if (k != 1 && (!state || (reinterpret_cast<uintptr_t>(state) & 15u) != 0))
     return lsh_fail(LSH_ERR_INVALID,
                     (w + ": random sampling needs the generator state array (lsh_rng_setup)").c_str());
   if (vocab > (1 << kSampleIdBits))
     return lsh_fail(LSH_ERR_UNSUPPORTED, (w + ": vocabulary above 2^20 ids").c_str());
-  dec_sample_kernel<T><<<rows, kSampleThreads, 0, s>>>(logits, bias, ids, vocab, max_step, cur_len,
-                                                       logits_seq_len, unfinished, eos_id, k, p,
+  dec_sample_kernel<T><<<rows, kSampleThreads, 0, s>>>(logits, ldl, bias, ids, vocab, max_step,
+                                                       cur_len, logits_seq_len, unfinished, eos_id, k, p,
                                                        scale, static_cast<SampleState*>(state));
   return lsh_check_launch("dec_sample_kernel");
 }
@@ -159,31 +160,31 @@ template <typename T>
 int dec_topk_sample_i8I(int batch_size, int batch_seq_len, int max_step, int logits_seq_len,
                         hipStream_t s, const int8_t* logits, const T* logit_bias, int* ids,
                         int vocab_size, int k, int* unfinished, void* state, int eos_id,
-                        float dequant_scale) {
+                        float dequant_scale, int logits_stride) {
   if (k != 1 && k != 2 && k != 4 && k != 8 && k != 16 && k != 32)
     return lsh_fail(LSH_ERR_INVALID, "topk argument should be in [1,2,4,8,16,32]");
   return dec_sample<T>("ker_topk_sample_i8I", batch_size, batch_seq_len, max_step, logits_seq_len,
                        s, logits, logit_bias, ids, vocab_size, k, 0.f, unfinished, state, eos_id,
-                       dequant_scale);
+                       dequant_scale, logits_stride);
 }
 
 template <typename T>
 int dec_topp_sample_i8I(int batch_size, int batch_seq_len, int max_step, int logits_seq_len,
                         hipStream_t s, const int8_t* logits, const T* logit_bias, int* ids,
                         int vocab_size, float p, int* unfinished, void* state, int eos_id,
-                        float dequant_scale) {
+                        float dequant_scale, int logits_stride) {
   if (!(p > 0.f) || p > 1.f)
     return lsh_fail(LSH_ERR_INVALID, "ker_topp_sample_i8I: topp outside (0, 1]");
   return dec_sample<T>("ker_topp_sample_i8I", batch_size, batch_seq_len, max_step, logits_seq_len,
                        s, logits, logit_bias, ids, vocab_size, 0, p, unfinished, state, eos_id,
-                       dequant_scale);
+                       dequant_scale, logits_stride);
 }
 
 #define LSH_INST(T)                                                                              \
   template int dec_topk_sample_i8I<T>(int, int, int, int, hipStream_t, const int8_t*, const T*,  \
-                                      int*, int, int, int*, void*, int, float);                  \
+                                      int*, int, int, int*, void*, int, float, int);             \
   template int dec_topp_sample_i8I<T>(int, int, int, int, hipStream_t, const int8_t*, const T*,  \
-                                      int*, int, float, int*, void*, int, float);
+                                      int*, int, float, int*, void*, int, float, int);
 LSH_INST(float)
 LSH_INST(__half)
 #undef LSH_INST
