@@ -7,6 +7,7 @@
 // all cross-lane traffic is wave reductions, and sums run in a fixed order so that a
 // step is reproducible bit for bit.
 #include "dec_attend.h"
+#include "ln_step.h"
 #include "ls_device.h"
 #include "ls_launch.h"
 
@@ -648,15 +649,19 @@ encdec_attn_vec_kernel(const __half* __restrict__ q, const __half* __restrict__ 
 // requests the keys, values and mask of beam b; after the barrier the product wavefronts are
 // done and wavefront b goes on with beam b.  Two short instruction streams side by side
 // instead of one long one, and the two memory streams travel together.
+// LN_ROWS > 0 (beam_size <= LN_ROWS): the product wavefronts also make the sentence's rows, by the
+// layer norm that precedes the product (ln_step.h; `x` is not read).  A workgroup normalises its
+// own sentence's beams only, so this holds for any batch; the launch it replaces took 3 us.
 struct EncdecQProd {
   const int8_t* x;
   const int8_t* W;
   const __half* bias;
   int hidden;
   float alpha, dequant_scale;
+  LnStep ln;
 };
 
-template <int D, int UN, bool QPROD = false>
+template <int D, int UN, bool QPROD = false, int LN_ROWS = 0>
 __global__ void __launch_bounds__(QPROD ? 512 : 256)
 encdec_attn_short_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
                          const __half* __restrict__ v, const int* __restrict__ pad_mask,
@@ -668,6 +673,8 @@ encdec_attn_short_kernel(const __half* __restrict__ q, const __half* __restrict_
   constexpr int KPW = 64 / CH;  // rows per load instruction of the wavefront
   __shared__ float part_all[4][4][D];
   __shared__ __align__(16) __half q_lds[QPROD ? 4 * D : 8];
+  __shared__ __align__(16) int8_t codes[LN_ROWS ? 16 * 1024 : 16];
+  __shared__ __align__(16) float red_ln[LN_ROWS ? 2 * LN_ROWS * 4 : 4];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   // grid: x = head, y = sentence, z = groups of 4 beams; wavefront = beam
   const int head = (int)blockIdx.x, beam = (int)blockIdx.z * 4 + wid;
@@ -699,9 +706,21 @@ encdec_attn_short_kernel(const __half* __restrict__ q, const __half* __restrict_
       const int8_t* wp = qp.W + code_offset((long)head * D + pw * 16 + m, kq * 16, qp.hidden, blocked);
       const int slice = blocked ? 1024 : 64;  // from one 64-byte slice of a row to the next
       const uint2 braw = *reinterpret_cast<const uint2*>(qp.bias + head * D + pw * 16 + 4 * kq);
+      LnStepRows<false, LN_ROWS ? LN_ROWS : 1> ln;
+      if constexpr (LN_ROWS) {
+        ln.load(qp.ln, (int)threadIdx.x - 256, b * beam_size, beam_size, qp.hidden);
+        __builtin_amdgcn_sched_barrier(0);
+      }
       v4i xf[16], wf[16];
 #pragma unroll
       for (int sl = 0; sl < 16; ++sl) wf[sl] = *reinterpret_cast<const v4i*>(wp + min(sl, KS - 1) * slice);
+      if constexpr (LN_ROWS) {
+        __builtin_amdgcn_sched_barrier(0);
+        ln.finish(qp.ln, (int)threadIdx.x - 256, b * beam_size, beam_size, qp.hidden, codes, red_ln,
+                  head == 0);
+        __syncthreads();
+        xp = codes + lane * 16;
+      }
 #pragma unroll
       for (int sl = 0; sl < 16; ++sl) xf[sl] = *reinterpret_cast<const v4i*>(xp + min(sl, KS - 1) * slice);
       __builtin_amdgcn_sched_barrier(0);  // every request of the kernel is out before a product
@@ -726,6 +745,8 @@ encdec_attn_short_kernel(const __half* __restrict__ q, const __half* __restrict_
         *reinterpret_cast<uint2*>(q_lds + m * D + pw * 16 + 4 * kq) = out.u;
       }
       __syncthreads();
+      if constexpr (LN_ROWS)
+        if (head == 0) ln.store(qp.ln, (int)threadIdx.x - 256, b * beam_size, beam_size, qp.hidden);
       return;
     }
   }
@@ -742,6 +763,11 @@ encdec_attn_short_kernel(const __half* __restrict__ q, const __half* __restrict_
   for (int u = 0; u < UN; ++u) {
     const int j = min(u * KPW + grp, seq_len - 1);
     vv[u].u = *reinterpret_cast<const uint4*>(vb + (long)j * D);
+  }
+  if constexpr (LN_ROWS) {  // the layer norm's barriers
+    __syncthreads();
+    __syncthreads();
+    __syncthreads();
   }
   if constexpr (QPROD) {
     __syncthreads();
@@ -827,8 +853,8 @@ int encdec_q_attention_f16(const int8_t* x, const int8_t* q_weight, const __half
                            const __half* k, const __half* v, const int* pad_mask, int8_t* ctx_q,
                            float quant_scale, int batch_size, int beam_size, int head_num,
                            int batch_seq_len, int hidden, float alpha, float dequant_scale,
-                           hipStream_t s, bool blocked) {
-  if (!x || !q_weight || !q_bias || !k || !v || !pad_mask || !ctx_q || batch_size <= 0)
+                           hipStream_t s, bool blocked, const LnStep* ln) {
+  if ((!x && !ln) || !q_weight || !q_bias || !k || !v || !pad_mask || !ctx_q || batch_size <= 0)
     return lsh_fail(LSH_ERR_INVALID, "encdec_q_attention: bad arguments");
   if (!encdec_q_attention_supported(beam_size, head_num, hidden, batch_seq_len) ||
       batch_size > 65535 ||
@@ -839,20 +865,35 @@ int encdec_q_attention_f16(const int8_t* x, const int8_t* q_weight, const __half
                     "encdec_q_attention: needs heads of 64, hidden <= 1024, at most 4 beams, a "
                     "source of at most 128 tokens, 16-byte aligned operands");
   const long rows = (long)batch_size * beam_size;
-  if (x < ctx_q + rows * hidden && ctx_q < x + rows * hidden)
+  if (!ln && x < ctx_q + rows * hidden && ctx_q < x + rows * hidden)
     return lsh_fail(LSH_ERR_INVALID, "encdec_q_attention: ctx_q overlaps x");
   const float alpha_h = __half2float(__float2half_rn(sqrtf(1.f / 64.f)));
   const dim3 grid(head_num, batch_size, 1);
-  const EncdecQProd qp{x, q_weight, q_bias, hidden, alpha, dequant_scale};
+  if (ln) {
+    const uintptr_t all = reinterpret_cast<uintptr_t>(ln->acc) | reinterpret_cast<uintptr_t>(ln->res_in) |
+                          reinterpret_cast<uintptr_t>(ln->res_out) | reinterpret_cast<uintptr_t>(ln->scale) |
+                          reinterpret_cast<uintptr_t>(ln->bias) | reinterpret_cast<uintptr_t>(ln->res_bias) |
+                          reinterpret_cast<uintptr_t>(ln->colsum);
+    if (!blocked || hidden % 256 != 0 || ln->planes != 0 || !ln->acc || !ln->res_in || !ln->res_out ||
+        ln->res_in == ln->res_out || !ln->scale || !ln->bias || (all & 15u) != 0)
+      return lsh_fail(LSH_ERR_UNSUPPORTED, "encdec_q_attention: layer norm not covered");
+  }
+  const EncdecQProd qp{x, q_weight, q_bias, hidden, alpha, dequant_scale, ln ? *ln : LnStep{}};
   const int un = (batch_seq_len + 7) / 8;
-#define LSH_ENCDEC_Q(UN)                                                                     \
-  encdec_attn_short_kernel<64, UN, true><<<grid, 512, 0, s>>>(                               \
+#define LSH_ENCDEC_Q_LN(UN, LN)                                                              \
+  encdec_attn_short_kernel<64, UN, true, LN><<<grid, 512, 0, s>>>(                               \
       nullptr, k, v, pad_mask, nullptr, ctx_q, quant_scale, beam_size, head_num, batch_seq_len, \
       alpha_h, blocked, qp)
-  if (un <= 4) LSH_ENCDEC_Q(4);
-  else if (un <= 8) LSH_ENCDEC_Q(8);
-  else LSH_ENCDEC_Q(16);
+#define LSH_ENCDEC_Q(UN)                                 \
+  if (!ln) LSH_ENCDEC_Q_LN(UN, 0);                       \
+  else if (beam_size == 1) LSH_ENCDEC_Q_LN(UN, 1);       \
+  else if (beam_size == 2) LSH_ENCDEC_Q_LN(UN, 2);       \
+  else LSH_ENCDEC_Q_LN(UN, 4)
+  if (un <= 4) { LSH_ENCDEC_Q(4); }
+  else if (un <= 8) { LSH_ENCDEC_Q(8); }
+  else { LSH_ENCDEC_Q(16); }
 #undef LSH_ENCDEC_Q
+#undef LSH_ENCDEC_Q_LN
   return lsh_check_launch("encdec_attn_short_kernel<q product>");
 }
 

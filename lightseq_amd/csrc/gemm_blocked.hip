@@ -7,6 +7,7 @@
 // the LDS tile loop of gemm_tile.h for the large ones.  The dispatch estimates both.
 #include "gemm_dec_epi.h"
 #include "gemm_kw.h"
+#include "ln_step.h"
 #include "ls_launch.h"
 
 #include <hip/hip_ext.h>
@@ -27,6 +28,60 @@ gemm_blk_tile_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W,
   int tm, tn;
   tile_of(blockIdx.x, tiles_m * tiles_n, tiles_m, tiles_n, tm, tn);
   tile_gemm<Epi, WGM, WGN, MB, NB, NST, false, true>(A, W, epi, tm * TM, M, N, K, tn, smem);
+}
+
+// A product of one to four rows that makes its rows itself (ln_step.h): 16 columns per workgroup,
+// a quarter of K per wavefront (D slices), its weights requested right behind the inputs of
+// the layer norm and in flight while it runs.  Everything after the codes is gemm_kw_kernel's.
+// us per generation step of a GPT-2 medium shape, batch 1: 573 -> 457.
+template <typename Epi, bool I32, int ROWS, int D>
+__global__ void __launch_bounds__(256)
+ln_gemm_kernel(const LnStep ln, const int8_t* __restrict__ W, Epi epi, int M, int N, int K) {
+  extern __shared__ __align__(16) int8_t smem[];
+  __shared__ __align__(16) float red_ln[2 * ROWS * 4];
+  int8_t* codes = smem;           // [16 rows, K] blocked
+  int8_t* part = smem + 16 * K;   // partial sums, then the table rows: as in gemm_kw_kernel
+  int8_t* tab = part + 4 * 68 * 16;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, kq = lane >> 4;
+  const int n0 = blockIdx.x * 16;
+  // every argument in one batch of scalar loads
+  asm volatile("" ::"s"(W), "s"(M), "s"(N), "s"(K), "s"(epi.alpha));
+  LnStepRows<I32, ROWS, D> rows;
+  rows.load(ln, tid, 0, M, K);
+  __builtin_amdgcn_sched_barrier(0);
+  const int8_t* wp = W + ((long)blockIdx.x * (K >> 6) + wave * D) * 1024 + lane * 16;
+  v4i fw[D];
+#pragma unroll
+  for (int u = 0; u < D; ++u) fw[u] = *reinterpret_cast<const v4i*>(wp + u * 1024);
+  v4i table = (v4i)0;  // through registers: the layer norm would wait for a DMA
+  if constexpr (Epi::kTable)
+    table = *reinterpret_cast<const v4i*>(epi.table() + min(n0 + (tid >> 4), N - 1) * 256 +
+                                          (((tid ^ (tid >> 4)) & 15) << 4));
+  const int quad = tid & 3, row = tid >> 2;
+  const int n = n0 + 4 * quad;
+  const typename Epi::Col col = epi.column(min(n, N - 4), N);
+  __builtin_amdgcn_sched_barrier(0);
+  rows.finish(ln, tid, 0, M, K, codes, red_ln, blockIdx.x == 0);
+  if constexpr (Epi::kTable) *reinterpret_cast<v4i*>(tab + tid * 16) = table;
+  __syncthreads();
+  v4i acc = (v4i)0;
+#pragma unroll
+  for (int u = 0; u < D; ++u) {
+    asm volatile("" : "+v"(fw[u]));
+    const v4i a = *reinterpret_cast<const v4i*>(codes + (wave * D + u) * 1024 + lane * 16);
+    acc = KwI8::mma(fw[u], a, acc);
+  }
+  v4i* cells = reinterpret_cast<v4i*>(part);
+  cells[wave * 68 + kq * 17 + l16] = acc;
+  __syncthreads();
+  if (blockIdx.x == 0) rows.store(ln, tid, 0, M, K);
+  if (row >= M || n >= N) return;
+  const int cell = quad * 17 + row;
+  const v4i c = (cells[cell] + cells[68 + cell]) + (cells[2 * 68 + cell] + cells[3 * 68 + cell]);
+  if constexpr (Epi::kTable) epi.store4(row, n, N, col, c, tab + 4 * quad * 256);
+  else epi.store4(row, n, N, col, c);
 }
 
 namespace {
@@ -98,6 +153,35 @@ LdsTile choose_lds_tile(int M, int N, int K, int cus, bool table) {
   return best;
 }
 
+template <typename Epi, bool I32, int ROWS>
+int launch_ln_rows(const LnStep& ln, const int8_t* W, Epi epi, int M, int N, int K, hipStream_t s) {
+  const dim3 grid((N + 15) / 16);
+  const size_t smem = 16 * (size_t)K + 4 * 68 * 16 + (Epi::kTable ? 16 * 256 : 0);
+  switch (K >> 8) {
+    case 1: return launch_blk<ln_gemm_kernel<Epi, I32, ROWS, 1>>(grid, 256, smem, s, ln, W, epi, M, N, K);
+    case 2: return launch_blk<ln_gemm_kernel<Epi, I32, ROWS, 2>>(grid, 256, smem, s, ln, W, epi, M, N, K);
+    case 3: return launch_blk<ln_gemm_kernel<Epi, I32, ROWS, 3>>(grid, 256, smem, s, ln, W, epi, M, N, K);
+    default: return launch_blk<ln_gemm_kernel<Epi, I32, ROWS, 4>>(grid, 256, smem, s, ln, W, epi, M, N, K);
+  }
+}
+template <typename Epi, bool I32>
+int launch_ln_gemm(const LnStep& ln, const int8_t* W, Epi epi, int M, int N, int K, hipStream_t s) {
+  if (!ln_step_supported(M, K) || N % 4 != 0 || ln.planes > 4 || (ln.planes != 0) != I32)
+    return lsh_fail(LSH_ERR_UNSUPPORTED, "layer norm + product: shape not covered");
+  if (!ln.acc || !ln.res_in || !ln.res_out || ln.res_in == ln.res_out || !ln.scale || !ln.bias || !W ||
+      !epi.aligned())
+    return lsh_fail(LSH_ERR_INVALID, "layer norm + product: bad operands");
+  const uintptr_t all = reinterpret_cast<uintptr_t>(ln.acc) | reinterpret_cast<uintptr_t>(ln.res_in) |
+                        reinterpret_cast<uintptr_t>(ln.res_out) | reinterpret_cast<uintptr_t>(ln.scale) |
+                        reinterpret_cast<uintptr_t>(ln.bias) | reinterpret_cast<uintptr_t>(ln.res_bias) |
+                        reinterpret_cast<uintptr_t>(ln.colsum) | reinterpret_cast<uintptr_t>(W);
+  if ((all & 15u) != 0 || ln.plane_stride % 4 != 0)
+    return lsh_fail(LSH_ERR_INVALID, "layer norm + product: operands must be 16-byte aligned");
+  if (M == 1) return launch_ln_rows<Epi, I32, 1>(ln, W, epi, M, N, K, s);
+  if (M == 2) return launch_ln_rows<Epi, I32, 2>(ln, W, epi, M, N, K, s);
+  return launch_ln_rows<Epi, I32, 4>(ln, W, epi, M, N, K, s);
+}
+
 template <typename Tr, typename Epi, bool TILES>
 int dispatch_blk(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K, hipStream_t s,
                  int ksplit = 1) {
@@ -150,6 +234,12 @@ int dispatch_blk(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K,
 
 }  // namespace
 
+// Every workgroup repeats the rows' arithmetic, 0.35 us a row: beyond four rows it costs what the
+// launch costs that it replaces.
+bool ln_step_supported(int rows, int hidden) {
+  return rows >= 1 && rows <= 4 && hidden % 256 == 0 && hidden >= 256 && hidden <= 1024;
+}
+
 const char* gemm_blk_kernel_name(int M, int N, int K, bool table) {
   const LdsTile t = choose_lds_tile(M, N, K, cu_count(), table);
   return t.tm != 0 && t.us < kw_choose_tile(M, N, K, 1, cu_count(), table).us ? "gemm_blk_tile_kernel"
@@ -186,17 +276,18 @@ int gemm_blk_preferred_ksplit(int M, int N, int K) {
 }
 
 int gemm_blk_lut(const int8_t* A, const int8_t* W, int8_t* C, const int8_t* lut, int M, int N, int K,
-                 float alpha, hipStream_t s) {
+                 float alpha, hipStream_t s, const LnStep* ln) {
   if (!lut) return lsh_fail(LSH_ERR_INVALID, "blocked gemm (table epilogue): null table");
   if (N % 64 != 0)
     return lsh_fail(LSH_ERR_UNSUPPORTED, "blocked gemm (table epilogue): the output needs N % 64 == 0");
+  if (ln) return launch_ln_gemm<EpiLutBlk, false>(*ln, W, EpiLutBlk{C, lut, alpha}, M, N, K, s);
   return dispatch_blk<KwI8, EpiLutBlk, true>(A, W, EpiLutBlk{C, lut, alpha}, M, N, K, s);
 }
 
 int gemm_blk_decself_qkv(const int8_t* A, const int8_t* W, const __half* qkv_bias, int8_t* new_q,
                          int8_t* new_k, int8_t* new_v, int step_token_num, int hidden, int K,
                          int head_num, int max_step, int step_id, float alpha, float dequant_scale,
-                         float quant_scale, hipStream_t s) {
+                         float quant_scale, hipStream_t s, const LnStep* ln) {
   if (!qkv_bias || !new_q || !new_k || !new_v || head_num <= 0 || hidden <= 0 ||
       hidden % head_num != 0 || max_step <= 0)
     return lsh_fail(LSH_ERR_INVALID, "blocked gemm (decoder qkv): bad arguments");
@@ -205,27 +296,25 @@ int gemm_blk_decself_qkv(const int8_t* A, const int8_t* W, const __half* qkv_bia
   const int d = hidden / head_num;
   if (d % 4 != 0 || hidden >= (1 << 22) || (long)hidden * max_step >= (1L << 31))
     return lsh_fail(LSH_ERR_UNSUPPORTED, "blocked gemm (decoder qkv): needs dim_per_head % 4 == 0");
-  return dispatch_blk<KwI8, EpiDecQkvI8, false>(
-      A, W,
-      EpiDecQkvI8{new_q, new_k, new_v, qkv_bias, alpha, dequant_scale, quant_scale, hidden, head_num,
-                  d, max_step, step_id, 1.0f / (float)hidden, 1.0f / (float)d},
-      step_token_num, 3 * hidden, K, s);
+  const EpiDecQkvI8 epi{new_q, new_k, new_v, qkv_bias, alpha, dequant_scale, quant_scale, hidden, head_num,
+                        d, max_step, step_id, 1.0f / (float)hidden, 1.0f / (float)d};
+  if (ln) return launch_ln_gemm<EpiDecQkvI8, true>(*ln, W, epi, step_token_num, 3 * hidden, K, s);
+  return dispatch_blk<KwI8, EpiDecQkvI8, false>(A, W, epi, step_token_num, 3 * hidden, K, s);
 }
 
 int gemm_blk_encdec_q(const int8_t* A, const int8_t* W, const __half* q_bias, __half* new_q,
                       int step_token_num, int hidden, int K, int beam_size, int head_num, float alpha,
-                      float dequant_scale, hipStream_t s) {
+                      float dequant_scale, hipStream_t s, const LnStep* ln) {
   if (!q_bias || !new_q || head_num <= 0 || hidden <= 0 || hidden % head_num != 0 ||
       beam_size <= 0 || step_token_num <= 0 || step_token_num % beam_size != 0)
     return lsh_fail(LSH_ERR_INVALID, "blocked gemm (cross-attention q): bad arguments");
   const int d = hidden / head_num;
   if (d % 4 != 0 || step_token_num >= (1 << 22))
     return lsh_fail(LSH_ERR_UNSUPPORTED, "blocked gemm (cross-attention q): needs dim_per_head % 4 == 0");
-  return dispatch_blk<KwI8, EpiEncdecQF16, false>(
-      A, W,
-      EpiEncdecQF16{new_q, q_bias, alpha, dequant_scale, beam_size, head_num, d,
-                    1.0f / (float)beam_size, 1.0f / (float)d},
-      step_token_num, hidden, K, s);
+  const EpiEncdecQF16 epi{new_q, q_bias, alpha, dequant_scale, beam_size, head_num, d,
+                          1.0f / (float)beam_size, 1.0f / (float)d};
+  if (ln) return launch_ln_gemm<EpiEncdecQF16, false>(*ln, W, epi, step_token_num, hidden, K, s);
+  return dispatch_blk<KwI8, EpiEncdecQF16, false>(A, W, epi, step_token_num, hidden, K, s);
 }
 
 // [rows, K bytes] row-major -> blocked (rows beyond the matrix: zeros), or back.  A thread moves

@@ -279,15 +279,33 @@ int gemm_blk_i8o(const int8_t* A, const int8_t* W, int8_t* C, int M, int N, int 
 int gemm_blk_i32o(const int8_t* A, const int8_t* W, int32_t* C, int M, int N, int K, int ksplit,
                   hipStream_t s);
 int gemm_blk_preferred_ksplit(int M, int N, int K);
+
+// residual_bias_ln_i8O of a few rows, made by the product (or the cross-attention launch) that
+// reads its codes instead of a launch of its own (ln_step.h): the same codes and the same
+// residual stream, which goes to another buffer because other workgroups still read res_in.
+struct LnStep {
+  const void* acc;    // planes == 0: int8 [rows, hidden]; else int32 planes of [rows, hidden]
+  int planes;         // at most 4
+  long plane_stride;  // elements
+  const __half* res_in;
+  __half* res_out;
+  const __half *scale, *bias, *res_bias, *colsum;  // the last two may be null
+  float dequant_scale, quant_scale;
+  int is_post_ln;
+};
+// rows and widths for which a product takes an LnStep instead of A
+bool ln_step_supported(int rows, int hidden);
+
+// (ln: A is not read, it may be null)
 int gemm_blk_lut(const int8_t* A, const int8_t* W, int8_t* C, const int8_t* lut, int M, int N, int K,
-                 float alpha, hipStream_t s);
+                 float alpha, hipStream_t s, const LnStep* ln = nullptr);
 int gemm_blk_decself_qkv(const int8_t* A, const int8_t* W, const __half* qkv_bias, int8_t* new_q,
                          int8_t* new_k, int8_t* new_v, int step_token_num, int hidden, int K,
                          int head_num, int max_step, int step_id, float alpha, float dequant_scale,
-                         float quant_scale, hipStream_t s);
+                         float quant_scale, hipStream_t s, const LnStep* ln = nullptr);
 int gemm_blk_encdec_q(const int8_t* A, const int8_t* W, const __half* q_bias, __half* new_q,
                       int step_token_num, int hidden, int K, int beam_size, int head_num, float alpha,
-                      float dequant_scale, hipStream_t s);
+                      float dequant_scale, hipStream_t s, const LnStep* ln = nullptr);
 // the kernel the dispatch picks (profiles)
 const char* gemm_blk_kernel_name(int M, int N, int K, bool table);
 // Counts the changes of the process-wide route switches below (tile kernel, decode-step
@@ -373,13 +391,14 @@ int encdec_attention_f16(const __half* q, const __half* k, const __half* v, cons
                          __half* ctx, int8_t* ctx_q, float quant_scale, int batch_size,
                          int beam_size, int head_num, int batch_seq_len, int dim_per_head,
                          hipStream_t s, bool blocked = false);
-// blocked: x, q_weight and ctx_q are blocked matrices
+// blocked: x, q_weight and ctx_q are blocked matrices; ln (with blocked, hidden % 256 == 0): the rows
+// are made by this layer norm, x is not read
 bool encdec_q_attention_supported(int beam_size, int head_num, int hidden, int batch_seq_len);
 int encdec_q_attention_f16(const int8_t* x, const int8_t* q_weight, const __half* q_bias,
                            const __half* k, const __half* v, const int* pad_mask, int8_t* ctx_q,
                            float quant_scale, int batch_size, int beam_size, int head_num,
                            int batch_seq_len, int hidden, float alpha, float dequant_scale,
-                           hipStream_t s, bool blocked = false);
+                           hipStream_t s, bool blocked = false, const LnStep* ln = nullptr);
 
 // ---- beam search (beam_kernels.hip) -------------------------------------------------------
 template <typename T>

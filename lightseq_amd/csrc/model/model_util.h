@@ -365,6 +365,8 @@ struct LayerProducts {
   static bool can_block(int hidden, int inner, int dim_per_head) {
     return hidden % 64 == 0 && inner % 64 == 0 && dim_per_head % 16 == 0;
   }
+  // Where a step's layer norms are made by the products that read them (LnStep).
+  bool ln_in_product(int rows, int hidden) const { return blocked && lsh::ln_step_supported(rows, hidden); }
   // rows an activation matrix needs room for
   size_t rows(size_t n) const { return (n + 15) & ~(size_t)15; }
   DeviceBuffer<int8_t> weight(const std::vector<uint8_t>& w, int k, int n, hipStream_t s) const {
@@ -377,8 +379,8 @@ struct LayerProducts {
                      : lsh::gemm_i8_i8o(x, w, out, m, n, k, alpha, s));
   }
   void lut(const int8_t* x, const int8_t* w, int8_t* out, const int8_t* table, int m, int n, int k,
-           float alpha, hipStream_t s) const {
-    LSH_CALL(blocked ? lsh::gemm_blk_lut(x, w, out, table, m, n, k, alpha, s)
+           float alpha, hipStream_t s, const lsh::LnStep* ln = nullptr) const {
+    LSH_CALL(blocked ? lsh::gemm_blk_lut(x, w, out, table, m, n, k, alpha, s, ln)
                      : lsh::gemm_i8_lut_i8o(x, w, out, table, m, n, k, alpha, s));
   }
   // int32 accumulators in up to max_planes planes of [m, n]; returns their number
@@ -397,10 +399,22 @@ struct LayerProducts {
   }
   void decself_qkv(const int8_t* x, const int8_t* w, const __half* bias, int8_t* q, int8_t* k_cache,
                    int8_t* v_cache, int rows, int hidden, int head_num, int max_step, int step,
-                   float alpha, float dequant_scale, float quant_scale, hipStream_t s) const {
-    LSH_CALL((blocked ? lsh::gemm_blk_decself_qkv : lsh::gemm_i8_decself_qkv_i8o)(
-        x, w, bias, q, k_cache, v_cache, rows, hidden, hidden, head_num, max_step, step, alpha,
-        dequant_scale, quant_scale, s));
+                   float alpha, float dequant_scale, float quant_scale, hipStream_t s,
+                   const lsh::LnStep* ln = nullptr) const {
+    LSH_CALL(blocked ? lsh::gemm_blk_decself_qkv(x, w, bias, q, k_cache, v_cache, rows, hidden, hidden,
+                                                 head_num, max_step, step, alpha, dequant_scale,
+                                                 quant_scale, s, ln)
+                     : lsh::gemm_i8_decself_qkv_i8o(x, w, bias, q, k_cache, v_cache, rows, hidden,
+                                                    hidden, head_num, max_step, step, alpha,
+                                                    dequant_scale, quant_scale, s));
+  }
+  void encdec_q(const int8_t* x, const int8_t* w, const __half* bias, __half* q, int rows, int hidden,
+                int beam_size, int head_num, float alpha, float dequant_scale, hipStream_t s,
+                const lsh::LnStep* ln = nullptr) const {
+    LSH_CALL(blocked ? lsh::gemm_blk_encdec_q(x, w, bias, q, rows, hidden, hidden, beam_size, head_num,
+                                              alpha, dequant_scale, s, ln)
+                     : lsh::gemm_i8_encdec_q_f16(x, w, bias, q, rows, hidden, hidden, beam_size,
+                                                 head_num, alpha, dequant_scale, s));
   }
 };
 

@@ -82,7 +82,7 @@ void QuantDecoder::init_buffer() {
   _encdec_k.alloc((size_t)L * _layer_size_encdec_k);
   _encdec_v.alloc((size_t)L * _layer_size_encdec_k);
   _encoder_out_buf.alloc(tokens * (size_t)L * 2 * H);
-  _cur_step_query.alloc(rows * H);
+  for (auto& q : _cur_step_query) q.alloc(rows * H);
   _query_buf1.alloc(rows * H);
   _ops.blocked = LayerProducts::can_block(H, I, _tw._dim_per_head);
   _logits_stride = _ops.blocked ? (V + 63) & ~63 : V;
@@ -336,6 +336,11 @@ void QuantDecoder::enqueue_step() {
   _qkv_attn = !step_taps.any() && decself_qkv_attention_enabled() && _tw._dim_per_head == 64 &&
               decself_qkv_attention_supported(_step_token_num, _tw._hidden_size, _tw._head_num,
                                               _tw._max_step);
+  // few rows: the layer norms inside the stack are made by the products that read them; that in
+  // front of the cross attention by its launch, whatever the number of rows
+  _ln_in_product = !step_taps.any() && !_qkv_attn && _ops.ln_in_product(_step_token_num, _tw._hidden_size);
+  _ln_in_encdec = !step_taps.any() && _ops.blocked && _tw._hidden_size % 256 == 0;
+  _res = 0;
   embedding();
   for (_layer_id = 0; _layer_id < _tw._n_dec_layer; _layer_id++) {
     self_attention();
@@ -376,7 +381,7 @@ bool QuantDecoder::emb_ln_fused() const {
 void QuantDecoder::embedding() {
   if (emb_ln_fused()) return;  // done by the first layer's launch
   LSH_CALL(dec_emb_i8I<__half>(_int8_trg_emb.get(), _pos_emb.get(), _alive_seq[_alive_cur].get(),
-                               _cur_step_query.get(), _batch_size, _tw._beam_size,
+                               _cur_step_query[_res].get(), _batch_size, _tw._beam_size,
                                _tw._hidden_size, _tw._trg_vocab_size, _cur_step, _tw._max_step,
                                _stream, _trg_emb_clip_max / _quant_range, true, true));
 }
@@ -394,12 +399,12 @@ void QuantDecoder::self_attention() {
       // the step's embedding and the first layer norm in one launch (the bytes of the pair)
       LSH_CALL(dec_emb_norm_layer_i8O<__half>(
           _int8_trg_emb.get(), _pos_emb.get(), _alive_seq[_alive_cur].get(),
-          _cur_step_query.get(), _buf_a.get(), w.self_ln_scale.get(), w.self_ln_bias.get(),
+          _cur_step_query[_res].get(), _buf_a.get(), w.self_ln_scale.get(), w.self_ln_bias.get(),
           w.b_self_out.get(), M, H, _tw._trg_vocab_size, _cur_step, _tw._max_step,
           _trg_emb_clip_max / _quant_range, true, Q / c[6], _tw._is_post_ln, _stream,
           _ops.blocked && !_qkv_attn));
     } else {
-      LSH_CALL(norm_layer_resual_i8O<__half>(M, H, _stream, _cur_step_query.get(), _buf_a.get(),
+      LSH_CALL(norm_layer_resual_i8O<__half>(M, H, _stream, _cur_step_query[_res].get(), _buf_a.get(),
                                              w.self_ln_scale.get(), w.self_ln_bias.get(),
                                              w.b_self_out.get(), Q / c[6], _tw._is_post_ln,
                                              _ops.blocked && !_qkv_attn));
@@ -407,7 +412,7 @@ void QuantDecoder::self_attention() {
   }
   const size_t mh = (size_t)M * H;
   TAP_CODES("self_ln_q", _buf_a.get(), H);
-  TAP("res_in", _cur_step_query.get(), mh * sizeof(__half));
+  TAP("res_in", _cur_step_query[_res].get(), mh * sizeof(__half));
   const float attn_scale =
       __half2float(__float2half_rn(sqrtf(1.f / (float)_tw._dim_per_head)));
   if (_qkv_attn) {
@@ -424,7 +429,8 @@ void QuantDecoder::self_attention() {
     if (_tw._dim_per_head % 16 == 0) {
       _ops.decself_qkv(_buf_a.get(), w.w_self_qkv.get(), w.b_self_qkv.get(), _buf_q.get(), k_cache,
                        v_cache, M, H, _tw._head_num, _tw._max_step, _cur_step,
-                       c[0] * c[6] / (c[12] * Q), c[12] / Q, Q / c[18], _stream);
+                       c[0] * c[6] / (c[12] * Q), c[12] / Q, Q / c[18], _stream,
+                       _ln_in_product && _layer_id > 0 ? &_ln : nullptr);
     } else {
       LSH_CALL(gemm_i8_i8o(_buf_a.get(), w.w_self_qkv.get(), _buf_b.get(), M, 3 * H, H,
                            c[0] * c[6] / (c[12] * Q), _stream));
@@ -444,12 +450,26 @@ void QuantDecoder::self_attention() {
   _ops.i8o(_buf_b.get(), w.w_self_out.get(), _buf_a.get(), M, H, H, c[1] * c[7] / (c[13] * Q),
            _stream);
   TAP("self_out_q", _buf_a.get(), mh);
+  if (encdec_q_fused() ? _ln_in_encdec : _ln_in_product && _tw._dim_per_head % 16 == 0) {
+    _ln = LnStep{_buf_a.get(), 0, 0, _cur_step_query[_res].get(), _cur_step_query[_res ^ 1].get(),
+                 w.encdec_ln_scale.get(), w.encdec_ln_bias.get(), w.b_encdec_out.get(), nullptr,
+                 c[13] / Q, Q / c[8], _tw._is_post_ln};
+    _res ^= 1;
+    return;
+  }
   LSH_CALL((residual_bias_ln_i8O<__half, int8_t>(
       _buf_a.get(), w.encdec_ln_scale.get(), w.encdec_ln_bias.get(), w.b_encdec_out.get(),
-      _buf_b.get(), _cur_step_query.get(), M, H, c[13] / Q, Q / c[8], _stream, _tw._is_post_ln,
+      _buf_b.get(), _cur_step_query[_res].get(), M, H, c[13] / Q, Q / c[8], _stream, _tw._is_post_ln,
       nullptr, 1, 0, _ops.blocked)));
   TAP_CODES("encdec_ln_q", _buf_b.get(), H);
-  TAP("res_self", _cur_step_query.get(), mh * sizeof(__half));
+  TAP("res_self", _cur_step_query[_res].get(), mh * sizeof(__half));
+}
+
+// Short sources, heads of 64: the query product and the cross attention are one launch (the same
+// bytes).  With taps set they are two.
+bool QuantDecoder::encdec_q_fused() const {
+  return !step_taps.any() && _tw._dim_per_head == 64 &&
+         encdec_q_attention_supported(_tw._beam_size, _tw._head_num, _tw._hidden_size, _batch_seq_len);
 }
 
 void QuantDecoder::encdec_attention() {
@@ -459,30 +479,25 @@ void QuantDecoder::encdec_attention() {
   const float Q = _quant_range;
 
   const size_t mh = (size_t)M * H;
-  // Short sources, heads of 64: the q product and the attention are one launch (the same
-  // bytes; the context goes to the second part of _buf_a because other workgroups still read
-  // the rows of _buf_b).  With taps set the launches below run.
-  if (!step_taps.any() && _tw._dim_per_head == 64 &&
-      encdec_q_attention_supported(_tw._beam_size, _tw._head_num, H, _batch_seq_len)) {
+  if (encdec_q_fused()) {
+    // the context goes to the second part of _buf_a because other workgroups still read the
+    // rows (_buf_b, or the first part)
     int8_t* ctx_q = _buf_a.get() + _ops.rows(M) * H;
     LSH_CALL(encdec_q_attention_f16(
         _buf_b.get(), w.w_encdec_q.get(), w.b_encdec_q.get(),
         _encdec_k.get() + (size_t)_layer_id * _layer_size_encdec_k,
         _encdec_v.get() + (size_t)_layer_id * _layer_size_encdec_k, _p_d_padding_mask, ctx_q,
         Q / c[9], _batch_size, _tw._beam_size, _tw._head_num, _batch_seq_len, H,
-        c[2] * c[8] / (c[14] * Q), c[14] / Q, _stream, _ops.blocked));
+        c[2] * c[8] / (c[14] * Q), c[14] / Q, _stream, _ops.blocked, _ln_in_encdec ? &_ln : nullptr));
     _ops.i8o(ctx_q, w.w_encdec_out.get(), _buf_a.get(), M, H, H, c[3] * c[9] / (c[15] * Q), _stream);
-    LSH_CALL((residual_bias_ln_i8O<__half, int8_t>(
-        _buf_a.get(), w.ffn_ln_scale.get(), w.ffn_ln_bias.get(), w.b_ffn2.get(), _buf_b.get(),
-        _cur_step_query.get(), M, H, c[15] / Q, Q / c[10], _stream, _tw._is_post_ln, nullptr, 1, 0,
-        _ops.blocked)));
+    encdec_norm();
     return;
   }
   // q product; its epilogue is ker_arrange_encdec_q_i8I (fp16 q [batch, heads, beam, d])
   if (_tw._dim_per_head % 16 == 0) {
-    LSH_CALL((_ops.blocked ? gemm_blk_encdec_q : gemm_i8_encdec_q_f16)(
-        _buf_b.get(), w.w_encdec_q.get(), w.b_encdec_q.get(), _query_buf1.get(), M, H, H,
-        _tw._beam_size, _tw._head_num, c[2] * c[8] / (c[14] * Q), c[14] / Q, _stream));
+    _ops.encdec_q(_buf_b.get(), w.w_encdec_q.get(), w.b_encdec_q.get(), _query_buf1.get(), M, H,
+                  _tw._beam_size, _tw._head_num, c[2] * c[8] / (c[14] * Q), c[14] / Q, _stream,
+                  _ln_in_product ? &_ln : nullptr);
   } else {
     LSH_CALL(gemm_i8_i8o(_buf_b.get(), w.w_encdec_q.get(), _buf_a.get(), M, H, H,
                          c[2] * c[8] / (c[14] * Q), _stream));
@@ -504,13 +519,29 @@ void QuantDecoder::encdec_attention() {
   TAP_CODES("encdec_ctx_q", _buf_b.get(), H);
   _ops.i8o(_buf_b.get(), w.w_encdec_out.get(), _buf_a.get(), M, H, H, c[3] * c[9] / (c[15] * Q),
            _stream);
-  TAP("encdec_out_q", _buf_a.get(), mh);
+  encdec_norm();
+}
+
+// the layer norm behind the cross attention
+void QuantDecoder::encdec_norm() {
+  const int H = _tw._hidden_size, M = _step_token_num;
+  const Layer& w = _layers[_layer_id];
+  const float* c = &_dec_clip_max[_layer_id * 19];
+  const float Q = _quant_range;
+  TAP("encdec_out_q", _buf_a.get(), (size_t)M * H);
+  if (_ln_in_product) {
+    _ln = LnStep{_buf_a.get(), 0, 0, _cur_step_query[_res].get(), _cur_step_query[_res ^ 1].get(),
+                 w.ffn_ln_scale.get(), w.ffn_ln_bias.get(), w.b_ffn2.get(), nullptr, c[15] / Q,
+                 Q / c[10], _tw._is_post_ln};
+    _res ^= 1;
+    return;
+  }
   LSH_CALL((residual_bias_ln_i8O<__half, int8_t>(
       _buf_a.get(), w.ffn_ln_scale.get(), w.ffn_ln_bias.get(), w.b_ffn2.get(), _buf_b.get(),
-      _cur_step_query.get(), M, H, c[15] / Q, Q / c[10], _stream, _tw._is_post_ln, nullptr, 1, 0,
-        _ops.blocked)));
+      _cur_step_query[_res].get(), M, H, c[15] / Q, Q / c[10], _stream, _tw._is_post_ln, nullptr, 1, 0,
+      _ops.blocked)));
   TAP_CODES("ffn_ln_q", _buf_b.get(), H);
-  TAP("res_encdec", _cur_step_query.get(), mh * sizeof(__half));
+  TAP("res_encdec", _cur_step_query[_res].get(), (size_t)M * H * sizeof(__half));
 }
 
 void QuantDecoder::ffn_add_norm() {
@@ -520,12 +551,14 @@ void QuantDecoder::ffn_add_norm() {
   const float Q = _quant_range;
 
   // FFN1 GEMM with the bias + activation + requantisation in its epilogue
-  _ops.lut(_buf_b.get(), w.w_ffn1.get(), _buf_a.get(), w.ffn1_act_lut.get(), M, I, H,
-           c[4] * c[10] / (c[16] * Q), _stream);
-  TAP_CODES("ffn1_act_q", _buf_a.get(), I);
+  // (with the layer norm inside the product _buf_a is its input)
+  int8_t* act = (_ln_in_product ? _buf_b : _buf_a).get();
+  _ops.lut(_buf_b.get(), w.w_ffn1.get(), act, w.ffn1_act_lut.get(), M, I, H,
+           c[4] * c[10] / (c[16] * Q), _stream, _ln_in_product ? &_ln : nullptr);
+  TAP_CODES("ffn1_act_q", act, I);
   // a tapped accumulator is one plane (the planes of a split product sum to it exactly)
   const bool tap_acc = step_taps.wants(_layer_id, _cur_step, "ffn2_acc");
-  const int nparts = _ops.i32o(_buf_a.get(), w.w_ffn2.get(), _int32_ffn_out_buf.get(), M, H, I,
+  const int nparts = _ops.i32o(act, w.w_ffn2.get(), _int32_ffn_out_buf.get(), M, H, I,
                                tap_acc ? 1 : 8, _stream);
   TAP("ffn2_acc", _int32_ffn_out_buf.get(), (size_t)M * H * sizeof(int32_t));
 
@@ -545,13 +578,20 @@ void QuantDecoder::ffn_add_norm() {
     res_bias_ptr = nx.b_self_out.get();
     clip_max = _dec_clip_max[(_layer_id + 1) * 19 + 6];
   }
+  if (_ln_in_product && _layer_id != _tw._n_dec_layer - 1) {
+    _ln = LnStep{_int32_ffn_out_buf.get(), nparts, (long)M * H, _cur_step_query[_res].get(),
+                 _cur_step_query[_res ^ 1].get(), scale_ptr, bias_ptr, res_bias_ptr,
+                 w.ffn2_colsum.get(), dequant_scale, Q / clip_max, _tw._is_post_ln};
+    _res ^= 1;
+    return;
+  }
   LSH_CALL((residual_bias_ln_i8O<__half, int32_t>(
       _int32_ffn_out_buf.get(), scale_ptr, bias_ptr, res_bias_ptr, _buf_a.get(),
-      _cur_step_query.get(), M, H, dequant_scale, Q / clip_max, _stream, _tw._is_post_ln,
+      _cur_step_query[_res].get(), M, H, dequant_scale, Q / clip_max, _stream, _tw._is_post_ln,
       w.ffn2_colsum.get(), nparts, (long)M * H,
       _ops.blocked && (!_qkv_attn || _layer_id == _tw._n_dec_layer - 1))));
   TAP_CODES("next_ln_q", _buf_a.get(), H);
-  TAP("res_out", _cur_step_query.get(), (size_t)M * H * sizeof(__half));
+  TAP("res_out", _cur_step_query[_res].get(), (size_t)M * H * sizeof(__half));
 }
 
 #undef TAP

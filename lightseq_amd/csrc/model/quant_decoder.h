@@ -68,7 +68,9 @@ class QuantDecoder {
   void embedding();
   bool emb_ln_fused() const;
   void self_attention();
+  bool encdec_q_fused() const;
   void encdec_attention();
+  void encdec_norm();
   void ffn_add_norm();
   void enqueue_step();
   void beam_search();
@@ -100,7 +102,10 @@ class QuantDecoder {
   // activations and state
   DeviceBuffer<__half> _encdec_k, _encdec_v;      // [n_layer][max_batch*max_step*H]
   DeviceBuffer<__half> _encoder_out_buf;          // [tokens, n_layer*2*H]
-  DeviceBuffer<__half> _cur_step_query, _query_buf1;
+  // the residual stream: a launch that makes a layer norm for itself writes the other buffer
+  DeviceBuffer<__half> _cur_step_query[2];
+  int _res = 0;
+  DeviceBuffer<__half> _query_buf1;
   DeviceBuffer<int8_t> _buf_a, _buf_b, _buf_q, _logits;
   DeviceBuffer<int32_t> _int32_ffn_out_buf;
   DeviceBuffer<int8_t> _self_k_cache[2], _self_v_cache[2];  // [n_layer][rows*max_step*H]
@@ -117,6 +122,8 @@ class QuantDecoder {
   DeviceBuffer<int8_t> _int8_trg_emb, _emb_blk;
   LayerProducts _ops;
   int _logits_stride = 0;  // codes from one row of logits to the next
+  lsh::LnStep _ln{};  // the layer norm that the next launch makes for itself
+  bool _ln_in_product = false, _ln_in_encdec = false;
   bool _qkv_attn = false;  // this step runs the opt-in launch of QKV product and attention
   DeviceBuffer<__half> _pos_emb, _out_ln_scale, _out_ln_bias, _kv_kernel /*[n_layer*2*H, H]*/,
       _kv_bias, _logit_bias;

@@ -68,7 +68,8 @@ void QuantGptEncoder::init_buffer() {
   *_h_unfinished = 0;
   _ops.blocked = LayerProducts::can_block(H, I, _tw._dim_per_head);
   _logits_stride = _ops.blocked ? (V + 63) & ~63 : V;
-  _query.alloc((size_t)_max_batch_dim);
+  _query[0].alloc((size_t)_max_batch_dim);
+  _query[1].alloc((size_t)_max_batch_size * H);
   _qkv_buf.alloc((size_t)(3 * _max_batch_dim));
   const size_t wide = _ops.rows(tokens) * (size_t)std::max(I, 3 * H);
   _buf_a.alloc(wide);
@@ -119,7 +120,9 @@ void QuantGptEncoder::init_buffer() {
 }
 
 // FFN block and the LayerNorm that follows it (:646-776).  `in` holds the int8
-// LayerNorm output and receives the next one; `tmp` is scratch of the same size.
+// LayerNorm output and receives the next one; `tmp` is scratch of the same size.  ln_in: the first
+// product makes its rows by this layer norm; ln_out: receives the one that follows, which then
+// the next layer's first product makes.
 // Step taps (debug): name -> what is copied, of the tapped layer at the tapped cached step.
 //   ln1_q, self_q, ctx_q, out_q, ln2_q, next_ln_q: int8 [batch, hidden];  act_q: int8 [batch, inner]
 //   ffn2_acc: int32 [batch, hidden];  k_cache, v_cache: the layer's int8 caches [batch, heads,
@@ -129,13 +132,14 @@ void QuantGptEncoder::init_buffer() {
 #define TAP_CODES(name, ptr, rows, cols) \
   step_taps.copy_codes(_layer_id, _tap_step, name, ptr, rows, cols, _ops.blocked, _stream)
 
-void QuantGptEncoder::ffn_add_norm(int rows, int8_t* in, int8_t* tmp, bool blocked_out) {
+void QuantGptEncoder::ffn_add_norm(int rows, int8_t* in, int8_t* tmp, bool blocked_out,
+                                   const LnStep* ln_in, LnStep* ln_out) {
   const int H = _tw._hidden_size, I = _tw._inner_size;
   const Layer& w = _layers[_layer_id];
   const float* c = &_enc_clip_max[_layer_id * 12];
   const float Q = _quant_range;
   _ops.lut(in, w.w_ffn1.get(), tmp, w.ffn1_act_lut.get(), rows, I, H, c[2] * c[6] / (c[10] * Q),
-           _stream);
+           _stream, ln_in);
   TAP_CODES("act_q", tmp, rows, I);
   // a tapped accumulator is one plane (the planes of a split product sum to it exactly)
   const bool tap_acc = step_taps.wants(_layer_id, _tap_step, "ffn2_acc");
@@ -157,11 +161,18 @@ void QuantGptEncoder::ffn_add_norm(int rows, int8_t* in, int8_t* tmp, bool block
     res_bias_ptr = nx.b_out.get();
     clip_max = _enc_clip_max[(_layer_id + 1) * 12 + 4];
   }
+  if (ln_out && _layer_id != _tw._n_enc_layer - 1) {
+    *ln_out = LnStep{_int32_ffn_out_buf.get(), nparts, (long)rows * H, _query[_res].get(),
+                     _query[_res ^ 1].get(), scale_ptr, bias_ptr, res_bias_ptr, nullptr, dequant_scale,
+                     Q / clip_max, 0};
+    _res ^= 1;
+    return;
+  }
   LSH_CALL((residual_bias_ln_i8O<__half, int32_t>(
-      _int32_ffn_out_buf.get(), scale_ptr, bias_ptr, res_bias_ptr, in, _query.get(), rows, H,
+      _int32_ffn_out_buf.get(), scale_ptr, bias_ptr, res_bias_ptr, in, _query[_res].get(), rows, H,
       dequant_scale, Q / clip_max, _stream, false, nullptr, nparts, (long)rows * H, blocked_out)));
   TAP_CODES("next_ln_q", in, rows, H);
-  TAP("res_out", _query.get(), (size_t)rows * H * sizeof(__half));
+  TAP("res_out", _query[_res].get(), (size_t)rows * H * sizeof(__half));
 }
 
 // all prompt positions at once (:253-291 / :299-341); leaves the int8 LayerNorm output of
@@ -169,9 +180,10 @@ void QuantGptEncoder::ffn_add_norm(int rows, int8_t* in, int8_t* tmp, bool block
 void QuantGptEncoder::prompt_pass(const int* ids, bool row_major_out) {
   const int H = _tw._hidden_size, M = _batch_token_num;
   const float Q = _quant_range;
+  _res = 0;
   CHECK_GPU_ERROR(hipMemsetAsync(_real_seq_len.get(), 0, sizeof(int) * _batch_size, _stream));
   LSH_CALL(gpt_embedding_i8I<__half>(_batch_size, _batch_seq_len, H, _stream, _int8_emb.get(),
-                                     _pos_emb.get(), ids, _query.get(), _real_seq_len.get(),
+                                     _pos_emb.get(), ids, _query[_res].get(), _real_seq_len.get(),
                                      _tw._padding_id, 0, _src_emb_clip_max / Q,
                                      _tw._src_vocab_size, _tw._max_step));
   int8_t *a = _buf_a.get(), *b = _buf_b.get();
@@ -185,7 +197,7 @@ void QuantGptEncoder::prompt_pass(const int* ids, bool row_major_out) {
     const Layer& w = _layers[_layer_id];
     const float* c = &_enc_clip_max[_layer_id * 12];
     if (_layer_id == 0)
-      LSH_CALL(norm_layer_resual_i8O<__half>(M, H, _stream, _query.get(), a, w.ln1_scale.get(),
+      LSH_CALL(norm_layer_resual_i8O<__half>(M, H, _stream, _query[_res].get(), a, w.ln1_scale.get(),
                                              w.ln1_bias.get(), w.b_out.get(), Q / c[4], false,
                                              _ops.blocked));
     _ops.i8o(a, w.w_qkv.get(), b, M, 3 * H, H, c[0] * c[4] / (c[8] * Q), _stream);
@@ -213,10 +225,11 @@ void QuantGptEncoder::prompt_pass(const int* ids, bool row_major_out) {
     }
     _ops.i8o(a, w.w_out.get(), b, M, H, H, c[1] * c[5] / (c[9] * Q), _stream);
     LSH_CALL((residual_bias_ln_i8O<__half, int8_t>(b, w.ln2_scale.get(), w.ln2_bias.get(),
-                                                   w.b_ffn2.get(), a, _query.get(), M, H,
+                                                   w.b_ffn2.get(), a, _query[_res].get(), M, H,
                                                    c[9] / Q, Q / c[6], _stream, false, nullptr, 1,
                                                    0, _ops.blocked)));
-    ffn_add_norm(M, a, b, _ops.blocked && !(row_major_out && _layer_id == _tw._n_enc_layer - 1));
+    ffn_add_norm(M, a, b, _ops.blocked && !(row_major_out && _layer_id == _tw._n_enc_layer - 1),
+                 nullptr, nullptr);
   }
 }
 
@@ -235,17 +248,22 @@ const int8_t* QuantGptEncoder::step_pass() {
                         _tw._dim_per_head == 64 &&
                         decself_qkv_attention_supported(B, H, _tw._head_num, _tw._max_step);
   const bool ln1_blocked = _ops.blocked && !qkv_attn;
+  // few rows: the layer norms between two layers and between the two halves of a layer are made
+  // by the products that read them
+  const bool ln_in_product = !step_taps.any() && !qkv_attn && _ops.ln_in_product(B, H);
+  LnStep ln{}, ln_next{};
+  _res = 0;
   const bool emb_ln_fused = !step_taps.any() && H % 4 == 0 && H <= 1024 && _tw._n_enc_layer > 0;
   if (emb_ln_fused) {
     const Layer& w0 = _layers[0];
     LSH_CALL(gpt_emb_step_norm_layer_i8O<__half>(
-        _int8_emb.get(), _pos_emb.get(), _last_ids.get(), _query.get(), a, w0.ln1_scale.get(),
+        _int8_emb.get(), _pos_emb.get(), _last_ids.get(), _query[_res].get(), a, w0.ln1_scale.get(),
         w0.ln1_bias.get(), w0.b_out.get(), _real_seq_len.get(), _unfinished.get(), B, H,
         _tw._src_vocab_size, _tw._padding_id, _batch_seq_len - 1, _tw._max_step,
         _src_emb_clip_max / Q, Q / _enc_clip_max[4], false, _stream, ln1_blocked));
   } else {
     LSH_CALL(gpt_embedding_i8I<__half>(B, 1, H, _stream, _int8_emb.get(), _pos_emb.get(),
-                                       _last_ids.get(), _query.get(), _real_seq_len.get(),
+                                       _last_ids.get(), _query[_res].get(), _real_seq_len.get(),
                                        _tw._padding_id, _batch_seq_len - 1, _src_emb_clip_max / Q,
                                        _tw._src_vocab_size, _tw._max_step, _unfinished.get()));
   }
@@ -256,10 +274,10 @@ const int8_t* QuantGptEncoder::step_pass() {
     int8_t* k_cache = _self_k_cache.get() + (size_t)_layer_id * _max_batch_dim;
     int8_t* v_cache = _self_v_cache.get() + (size_t)_layer_id * _max_batch_dim;
     if (_layer_id == 0 && !emb_ln_fused)
-      LSH_CALL(norm_layer_resual_i8O<__half>(B, H, _stream, _query.get(), a, w.ln1_scale.get(),
+      LSH_CALL(norm_layer_resual_i8O<__half>(B, H, _stream, _query[_res].get(), a, w.ln1_scale.get(),
                                              w.ln1_bias.get(), w.b_out.get(), Q / c[4], false, ln1_blocked));
     TAP_CODES("ln1_q", a, B, H);
-    TAP("res_in", _query.get(), bh * sizeof(__half));
+    TAP("res_in", _query[_res].get(), bh * sizeof(__half));
     // With taps set the two launches run, so that q and the caches are copied before the
     // attention as the tap names promise.
     if (qkv_attn) {
@@ -274,7 +292,8 @@ const int8_t* QuantGptEncoder::step_pass() {
       // to the caches at the token's position
       _ops.decself_qkv(a, w.w_qkv.get(), w.b_qkv.get(), _buf_q.get(), k_cache, v_cache, B, H,
                        _tw._head_num, _tw._max_step, _batch_seq_len - 1, c[0] * c[4] / (c[8] * Q),
-                       c[8] / Q, Q / c[11], _stream);
+                       c[8] / Q, Q / c[11], _stream,
+                       ln_in_product && _layer_id > 0 ? &ln_next : nullptr);
       TAP("self_q", _buf_q.get(), bh);
       TAP("k_cache", k_cache, bh * _tw._max_step);
       TAP("v_cache", v_cache, bh * _tw._max_step);
@@ -286,13 +305,21 @@ const int8_t* QuantGptEncoder::step_pass() {
     TAP_CODES("ctx_q", b, B, H);
     _ops.i8o(b, w.w_out.get(), a, B, H, H, c[1] * c[5] / (c[9] * Q), _stream);
     TAP("out_q", a, bh);
+    if (ln_in_product) {
+      ln = LnStep{a, 0, 0, _query[_res].get(), _query[_res ^ 1].get(), w.ln2_scale.get(),
+                  w.ln2_bias.get(), w.b_ffn2.get(), nullptr, c[9] / Q, Q / c[6], 0};
+      _res ^= 1;
+      ffn_add_norm(B, a, b, true, &ln, &ln_next);
+      continue;
+    }
     LSH_CALL((residual_bias_ln_i8O<__half, int8_t>(a, w.ln2_scale.get(), w.ln2_bias.get(),
-                                                   w.b_ffn2.get(), b, _query.get(), B, H,
+                                                   w.b_ffn2.get(), b, _query[_res].get(), B, H,
                                                    c[9] / Q, Q / c[6], _stream, false, nullptr, 1,
                                                    0, _ops.blocked)));
     TAP_CODES("ln2_q", b, B, H);
-    TAP("res_attn", _query.get(), bh * sizeof(__half));
-    ffn_add_norm(B, b, a, _layer_id == _tw._n_enc_layer - 1 ? _ops.blocked : ln1_blocked);
+    TAP("res_attn", _query[_res].get(), bh * sizeof(__half));
+    ffn_add_norm(B, b, a, _layer_id == _tw._n_enc_layer - 1 ? _ops.blocked : ln1_blocked, nullptr,
+                 nullptr);
     std::swap(a, b);  // `a` names the buffer holding the layer's int8 LayerNorm output
   }
   _tap_step = -2;

@@ -62,7 +62,8 @@ class QuantGptEncoder {
  private:
   void prompt_pass(const int* ids, bool row_major_out);
   const int8_t* step_pass();
-  void ffn_add_norm(int rows, int8_t* in, int8_t* tmp, bool blocked_out);
+  void ffn_add_norm(int rows, int8_t* in, int8_t* tmp, bool blocked_out, const lsh::LnStep* ln_in,
+                    lsh::LnStep* ln_out);
   void logits_product(const int8_t* hidden, int rows);
   void enqueue_sampling(const int8_t* hidden, bool clear_flag);
   int finish_token();
@@ -89,7 +90,11 @@ class QuantGptEncoder {
 
   DeviceBuffer<int> _real_seq_len, _ids, _last_ids, _unfinished;
   DeviceBuffer<long long> _sample_state;  // lsh_rng_state_t [max_batch_size]
-  DeviceBuffer<__half> _query, _qkv_buf;  // q codes | k codes | v, each max_batch_dim
+  // the residual stream; the second one holds a few rows of a step whose layer norms are made by
+  // the products (each writes the other buffer)
+  DeviceBuffer<__half> _query[2];
+  int _res = 0;
+  DeviceBuffer<__half> _qkv_buf;  // q codes | k codes | v, each max_batch_dim
   DeviceBuffer<int8_t> _buf_a, _buf_b, _buf_q, _logits;
   DeviceBuffer<int8_t> _hid_last[2];  // row-major, and as the logits product reads it
   DeviceBuffer<int32_t> _int32_ffn_out_buf;
