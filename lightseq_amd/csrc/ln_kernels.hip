@@ -456,6 +456,12 @@ bool ln_set_few_rows(bool on) {
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+__device__ __forceinline__ void publish_notice(const StepNotice& n) {
+  if (n.slot != nullptr && blockIdx.x == 0 && threadIdx.x == 0)
+    __hip_atomic_store(n.slot, ((unsigned long long)n.tag << 32) | (unsigned)*n.word,
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // The decoder's target embedding (inference/kernels/embKernels_int8.cc.cu:158-200) and the first
 // layer norm of the stack (ker_norm_layer_resual_i8O) in one launch, for the decode steps: a
 // row's embedding -- int8 table row (vocabulary-major) * scale + position row, rounded to the
@@ -470,8 +476,9 @@ dec_emb_ln_row_wg_kernel(const int8_t* __restrict__ token_emb, const T* __restri
                          int8_t* __restrict__ out_q, const T* __restrict__ scale,
                          const T* __restrict__ bias, const T* __restrict__ residual_bias,
                          int hidden, int vocab, int step, int max_step, float emb_scale,
-                         float quant_scale, int is_post_ln, int blocked) {
+                         float quant_scale, int is_post_ln, int blocked, StepNotice notice) {
 #pragma clang fp contract(off)
+  publish_notice(notice);
   __shared__ float red[2][4];
   const int e0 = (int)threadIdx.x * 4;
   const bool on = e0 < hidden;
@@ -505,7 +512,7 @@ int dec_emb_norm_layer_i8O(const int8_t* token_emb, const T* pos_emb, const int*
                            T* residual, int8_t* out_q, const T* scale, const T* bias,
                            const T* residual_bias, int rows, int hidden, int vocab, int step,
                            int max_step, float dequant_scale, bool scaled, float quant_scale,
-                           bool is_post_ln, hipStream_t s, bool blocked) {
+                           bool is_post_ln, hipStream_t s, bool blocked, StepNotice notice) {
   if (!token_emb || !pos_emb || !tokens || !residual || !out_q || !scale || !bias || rows <= 0 ||
       hidden <= 0 || vocab <= 0 || max_step <= 0)
     return lsh_fail(LSH_ERR_INVALID, "dec_emb_norm_layer_i8O: bad arguments");
@@ -521,17 +528,17 @@ int dec_emb_norm_layer_i8O(const int8_t* token_emb, const T* pos_emb, const int*
   dec_emb_ln_row_wg_kernel<T><<<rows, tpr, 0, s>>>(token_emb, pos_emb, tokens, residual, out_q,
                                                    scale, bias, residual_bias, hidden, vocab, step,
                                                    max_step, emb_scale, quant_scale,
-                                                   is_post_ln ? 1 : 0, blocked ? 1 : 0);
+                                                   is_post_ln ? 1 : 0, blocked ? 1 : 0, notice);
   return lsh_check_launch("dec_emb_ln_row_wg_kernel");
 }
 template int dec_emb_norm_layer_i8O<__half>(const int8_t*, const __half*, const int*, __half*,
                                             int8_t*, const __half*, const __half*, const __half*,
                                             int, int, int, int, int, float, bool, float, bool,
-                                            hipStream_t, bool);
+                                            hipStream_t, bool, StepNotice);
 template int dec_emb_norm_layer_i8O<float>(const int8_t*, const float*, const int*, float*,
                                            int8_t*, const float*, const float*, const float*, int,
                                            int, int, int, int, float, bool, float, bool,
-                                           hipStream_t, bool);
+                                           hipStream_t, bool, StepNotice);
 
 // The same for a generation step of the GPT model: the embedding of one token per sequence at
 // position `pos` (a padding token gives zeros), the token counted into real_seq_len and
@@ -543,8 +550,10 @@ gpt_emb_ln_row_wg_kernel(const int8_t* __restrict__ token_emb, const T* __restri
                          int8_t* __restrict__ out_q, const T* __restrict__ scale,
                          const T* __restrict__ bias, const T* __restrict__ residual_bias,
                          int* real_seq_len, int* zero_flag, int padding_id, int hidden, int vocab,
-                         int pos, float emb_scale, float quant_scale, int is_post_ln, int blocked) {
+                         int pos, float emb_scale, float quant_scale, int is_post_ln, int blocked,
+                         StepNotice notice) {
 #pragma clang fp contract(off)
+  publish_notice(notice);
   __shared__ float red[2][4];
   const int e0 = (int)threadIdx.x * 4;
   const bool on = e0 < hidden;
@@ -584,7 +593,7 @@ int gpt_emb_step_norm_layer_i8O(const int8_t* token_emb, const T* pos_emb, const
                                 const T* residual_bias, int* real_seq_len, int* zero_flag,
                                 int batch_size, int hidden, int vocab, int padding_id, int pos,
                                 int max_step, float dequant_scale, float quant_scale,
-                                bool is_post_ln, hipStream_t s, bool blocked) {
+                                bool is_post_ln, hipStream_t s, bool blocked, StepNotice notice) {
   if (!token_emb || !pos_emb || !token_id || !residual || !out_q || !scale || !bias ||
       !real_seq_len || batch_size <= 0 || hidden <= 0 || vocab <= 0)
     return lsh_fail(LSH_ERR_INVALID, "gpt_emb_step_norm_layer_i8O: bad arguments");
@@ -600,17 +609,17 @@ int gpt_emb_step_norm_layer_i8O(const int8_t* token_emb, const T* pos_emb, const
   gpt_emb_ln_row_wg_kernel<T><<<batch_size, tpr, 0, s>>>(
       token_emb, pos_emb, token_id, residual, out_q, scale, bias, residual_bias, real_seq_len,
       zero_flag, padding_id, hidden, vocab, pos, dequant_scale, quant_scale, is_post_ln ? 1 : 0,
-      blocked ? 1 : 0);
+      blocked ? 1 : 0, notice);
   return lsh_check_launch("gpt_emb_ln_row_wg_kernel");
 }
 template int gpt_emb_step_norm_layer_i8O<__half>(const int8_t*, const __half*, const int*,
                                                  __half*, int8_t*, const __half*, const __half*,
                                                  const __half*, int*, int*, int, int, int, int,
-                                                 int, int, float, float, bool, hipStream_t, bool);
+                                                 int, int, float, float, bool, hipStream_t, bool, StepNotice);
 template int gpt_emb_step_norm_layer_i8O<float>(const int8_t*, const float*, const int*, float*,
                                                 int8_t*, const float*, const float*, const float*,
                                                 int*, int*, int, int, int, int, int, int, float,
-                                                float, bool, hipStream_t, bool);
+                                                float, bool, hipStream_t, bool, StepNotice);
 
 template <typename T, typename AccT, int MODE>
 static int launch_ln(const AccT* gemm_out, T* residual, T* out_t, int8_t* out_q, const T* scale,

@@ -12,6 +12,7 @@
 #include <map>
 #include <stdexcept>
 #include <string>
+#include <thread>
 #include <unordered_map>
 #include <unordered_set>
 #include <vector>
@@ -187,6 +188,51 @@ class StepTaps {
  private:
   int _layer = -1, _step = -1;
   std::map<std::string, void*> _dst;
+};
+
+// The host's side of StepNotice.  A generation loop has to know after every step whether it goes on;
+// a copy of the word and a stream synchronisation leave the device idle for 25 - 35 us (the
+// wait, then the first launches of the next step).  Instead the loop enqueues the next step's
+// first launches, the first of which publishes the word, and waits for the word alone: the
+// device works meanwhile.  A step enqueued too far writes nothing that a finished run reads.
+class HostNotice {
+ public:
+  HostNotice() {}
+  HostNotice(const HostNotice&) = delete;
+  HostNotice& operator=(const HostNotice&) = delete;
+  ~HostNotice() {
+    if (slot_) (void)hipHostFree(slot_);
+  }
+  lsh::StepNotice next(const int* word) {
+    if (!slot_) {
+      CHECK_GPU_ERROR(hipHostMalloc(reinterpret_cast<void**>(&slot_), sizeof(*slot_)));
+      *slot_ = 0;
+    }
+    return lsh::StepNotice{word, slot_, ++tag_};
+  }
+  // the word of the last next(): a bounded wait on the slot, then on the stream
+  int wait(hipStream_t stream) const {
+    unsigned long long v = 0;
+    auto there = [&] {
+      v = __atomic_load_n(slot_, __ATOMIC_ACQUIRE);
+      return (unsigned)(v >> 32) == tag_;
+    };
+    for (int i = 0; i < 20000; ++i) {
+      if (there()) return (int)(unsigned)v;
+      __builtin_ia32_pause();
+    }
+    for (int i = 0; i < 200000; ++i) {
+      if (there()) return (int)(unsigned)v;
+      std::this_thread::yield();
+    }
+    CHECK_GPU_ERROR(hipStreamSynchronize(stream));
+    if (!there()) throw std::runtime_error("generation step: no word from the device");
+    return (int)(unsigned)v;
+  }
+
+ private:
+  unsigned long long* slot_ = nullptr;  // pinned
+  unsigned tag_ = 0;
 };
 
 // HIP graphs of a generation step.  A step is a fixed sequence of launches whose arguments

@@ -250,9 +250,36 @@ void QuantDecoder::run_one_infer(int batch_size, int batch_seq_len) {
 
   /* ---step2. autoregressive decoding--- */
   _phases.mark(1, _stream);
-  for (_cur_step = 0; _cur_step < _batch_max_decode_length - 1; _cur_step++) {
-    bool early_stop = run_step();
-    if (!_is_benchmark && early_stop) break;
+  const int limit = _batch_max_decode_length - 1;
+  if (!_is_benchmark && !_use_graphs && !_rec_logits && !_rec_alive && !step_taps.any() &&
+      emb_ln_fused()) {
+    // Whether a step is needed is known while the device works at its first layer: 7 to 10
+    // launches cover the way of the word to the host and of a launch to the device.
+    const int L = _tw._n_dec_layer, ahead = std::min(1, L);
+    for (_cur_step = 0; _cur_step < limit; _cur_step++) {
+      if (_cur_step == 0) {
+        step_begin(StepNotice{});
+        step_layers(0, ahead);
+      }
+      step_layers(ahead, L);
+      step_end();
+      const bool search = step_runs_beam_search();
+      step_done(search);
+      if (_cur_step + 1 == limit) {
+        if (finished(search, read_finished(search))) break;
+        continue;
+      }
+      ++_cur_step;
+      step_begin(_notice.next(search ? _num_finished.get() : _sample_unfinished.get()));
+      step_layers(0, ahead);
+      --_cur_step;
+      if (finished(search, _notice.wait(_stream))) break;
+    }
+  } else {
+    for (_cur_step = 0; _cur_step < limit; _cur_step++) {
+      const bool early_stop = run_step();
+      if (early_stop) break;
+    }
   }
   _phases.mark(2, _stream);
   _phases.set_loop_steps(_steps_run);
@@ -304,31 +331,40 @@ bool QuantDecoder::run_step() {
                        ((uint64_t)_cur_step << 8) | (uint64_t)(_alive_cur << 1 | _cache_cur);
   _graphs.run(key, _stream,
               _use_graphs && !_is_sampling && !_rec_logits && !_rec_alive && !step_taps.any(),
-              [&] { enqueue_step(); });
-  ++_steps_run;
-  if (!search) {
-    // (:979-984, 1126-1131) the sequences stay in their buffer, the caches are not reordered
-    if (_is_benchmark) return false;
-    CHECK_GPU_ERROR(hipMemcpyAsync(_h_num_finished, _sample_unfinished.get(), sizeof(int),
-                                   hipMemcpyDeviceToHost, _stream));
-    CHECK_GPU_ERROR(hipStreamSynchronize(_stream));
-    return *_h_num_finished != 1;
-  }
-  _alive_cur ^= 1;
-  if (_cur_step > 0) _cache_cur ^= 1;
-  if (!_is_benchmark) {
-    // the one device-to-host word of a step: all beams finished -> stop early
-    CHECK_GPU_ERROR(hipMemcpyAsync(_h_num_finished, _num_finished.get(), sizeof(int),
-                                   hipMemcpyDeviceToHost, _stream));
-    CHECK_GPU_ERROR(hipStreamSynchronize(_stream));
-    if (*_h_num_finished == _step_token_num) return true;
-  }
-  return false;
+              [&] {
+                step_begin(StepNotice{});
+                step_layers(0, _tw._n_dec_layer);
+                step_end();
+              });
+  step_done(search);
+  return !_is_benchmark && finished(search, read_finished(search));
 }
 
-// everything a step puts on the stream: embedding, the layer stack, the logits, the search
-// and the cache reorder (kernels and device-to-device copies only, so that it can be captured)
-void QuantDecoder::enqueue_step() {
+// host side of an enqueued step (a step that samples keeps its sequences in their buffer and does
+// not reorder the caches; :979-984, 1126-1131)
+void QuantDecoder::step_done(bool search) {
+  ++_steps_run;
+  if (!search) return;
+  _alive_cur ^= 1;
+  if (_cur_step > 0) _cache_cur ^= 1;
+}
+
+// the one device-to-host word of a step: all beams finished -> stop early
+int QuantDecoder::read_finished(bool search) {
+  CHECK_GPU_ERROR(hipMemcpyAsync(_h_num_finished,
+                                 search ? _num_finished.get() : _sample_unfinished.get(), sizeof(int),
+                                 hipMemcpyDeviceToHost, _stream));
+  CHECK_GPU_ERROR(hipStreamSynchronize(_stream));
+  return *_h_num_finished;
+}
+bool QuantDecoder::finished(bool search, int word) const {
+  return search ? word == _step_token_num : word != 1;
+}
+
+// What a step puts on the stream: embedding (step_begin), the layers from..to - 1 (step_layers),
+// the logits, the search and the cache reorder (step_end) -- kernels and device-to-device copies
+// only, so that it can be captured.
+void QuantDecoder::step_begin(StepNotice notice) {
   LnFewRowsScope few_rows;  // every step of every batch size: layer norms by the row kernel
   // The opt-in launch reads row-major operands.  With taps set the two launches run, so that q
   // and the caches are copied before the attention as the tap names promise; the bytes are the
@@ -341,12 +377,19 @@ void QuantDecoder::enqueue_step() {
   _ln_in_product = !step_taps.any() && !_qkv_attn && _ops.ln_in_product(_step_token_num, _tw._hidden_size);
   _ln_in_encdec = !step_taps.any() && _ops.blocked && _tw._hidden_size % 256 == 0;
   _res = 0;
-  embedding();
-  for (_layer_id = 0; _layer_id < _tw._n_dec_layer; _layer_id++) {
+  embedding(notice);
+}
+
+void QuantDecoder::step_layers(int from, int to) {
+  LnFewRowsScope few_rows;
+  for (_layer_id = from; _layer_id < to; _layer_id++) {
     self_attention();
     encdec_attention();
     ffn_add_norm();
   }
+}
+
+void QuantDecoder::step_end() {
   /* --- Project hidden states to vocab logits (:527-532) --- */
   _ops.i8o(_buf_a.get(), (_ops.blocked ? _emb_blk : _int8_trg_emb).get(), _logits.get(),
            _step_token_num, _logits_stride, _tw._hidden_size,
@@ -378,12 +421,28 @@ bool QuantDecoder::emb_ln_fused() const {
   return _tw._hidden_size % 4 == 0 && _tw._hidden_size <= 1024;
 }
 
-void QuantDecoder::embedding() {
-  if (emb_ln_fused()) return;  // done by the first layer's launch
+void QuantDecoder::embedding(StepNotice notice) {
+  if (_layers.empty()) return;
+  const int H = _tw._hidden_size, M = _step_token_num;
+  const Layer& w = _layers[0];
+  const float quant_scale = _quant_range / _dec_clip_max[6];
+  const bool blocked = _ops.blocked && !_qkv_attn;
+  if (emb_ln_fused()) {
+    // the step's embedding and the first layer norm in one launch (the bytes of the pair)
+    LSH_CALL(dec_emb_norm_layer_i8O<__half>(
+        _int8_trg_emb.get(), _pos_emb.get(), _alive_seq[_alive_cur].get(),
+        _cur_step_query[_res].get(), _buf_a.get(), w.self_ln_scale.get(), w.self_ln_bias.get(),
+        w.b_self_out.get(), M, H, _tw._trg_vocab_size, _cur_step, _tw._max_step,
+        _trg_emb_clip_max / _quant_range, true, quant_scale, _tw._is_post_ln, _stream, blocked, notice));
+    return;
+  }
   LSH_CALL(dec_emb_i8I<__half>(_int8_trg_emb.get(), _pos_emb.get(), _alive_seq[_alive_cur].get(),
-                               _cur_step_query[_res].get(), _batch_size, _tw._beam_size,
-                               _tw._hidden_size, _tw._trg_vocab_size, _cur_step, _tw._max_step,
-                               _stream, _trg_emb_clip_max / _quant_range, true, true));
+                               _cur_step_query[_res].get(), _batch_size, _tw._beam_size, H,
+                               _tw._trg_vocab_size, _cur_step, _tw._max_step, _stream,
+                               _trg_emb_clip_max / _quant_range, true, true));
+  LSH_CALL(norm_layer_resual_i8O<__half>(M, H, _stream, _cur_step_query[_res].get(), _buf_a.get(),
+                                         w.self_ln_scale.get(), w.self_ln_bias.get(),
+                                         w.b_self_out.get(), quant_scale, _tw._is_post_ln, blocked));
 }
 
 void QuantDecoder::self_attention() {
@@ -394,22 +453,6 @@ void QuantDecoder::self_attention() {
   int8_t* k_cache = _self_k_cache[_cache_cur].get() + (size_t)_layer_id * _layer_size_self_k;
   int8_t* v_cache = _self_v_cache[_cache_cur].get() + (size_t)_layer_id * _layer_size_self_k;
 
-  if (_layer_id == 0) {
-    if (emb_ln_fused()) {
-      // the step's embedding and the first layer norm in one launch (the bytes of the pair)
-      LSH_CALL(dec_emb_norm_layer_i8O<__half>(
-          _int8_trg_emb.get(), _pos_emb.get(), _alive_seq[_alive_cur].get(),
-          _cur_step_query[_res].get(), _buf_a.get(), w.self_ln_scale.get(), w.self_ln_bias.get(),
-          w.b_self_out.get(), M, H, _tw._trg_vocab_size, _cur_step, _tw._max_step,
-          _trg_emb_clip_max / _quant_range, true, Q / c[6], _tw._is_post_ln, _stream,
-          _ops.blocked && !_qkv_attn));
-    } else {
-      LSH_CALL(norm_layer_resual_i8O<__half>(M, H, _stream, _cur_step_query[_res].get(), _buf_a.get(),
-                                             w.self_ln_scale.get(), w.self_ln_bias.get(),
-                                             w.b_self_out.get(), Q / c[6], _tw._is_post_ln,
-                                             _ops.blocked && !_qkv_attn));
-    }
-  }
   const size_t mh = (size_t)M * H;
   TAP_CODES("self_ln_q", _buf_a.get(), H);
   TAP("res_in", _cur_step_query[_res].get(), mh * sizeof(__half));

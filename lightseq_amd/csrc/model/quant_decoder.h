@@ -65,14 +65,19 @@ class QuantDecoder {
  private:
   void project_encoder_output();
   bool run_step();
-  void embedding();
+  void embedding(lsh::StepNotice notice);
   bool emb_ln_fused() const;
   void self_attention();
   bool encdec_q_fused() const;
   void encdec_attention();
   void encdec_norm();
   void ffn_add_norm();
-  void enqueue_step();
+  void step_begin(lsh::StepNotice notice);
+  void step_layers(int from, int to);
+  void step_end();
+  void step_done(bool search);
+  int read_finished(bool search);
+  bool finished(bool search, int word) const;
   void beam_search();
   void sample_tokens();
   bool step_runs_beam_search() const;
@@ -94,6 +99,7 @@ class QuantDecoder {
   std::vector<float> _h_alive_seq_probs, _h_length_norm;
   int* _h_num_finished = nullptr;  // pinned; also receives the unfinished word of a sampling step
   bool _is_sampling = false;
+  HostNotice _notice;
 
   int8_t* _rec_logits = nullptr;
   int* _rec_alive = nullptr;

@@ -181,6 +181,7 @@ void QuantGptEncoder::prompt_pass(const int* ids, bool row_major_out) {
   const int H = _tw._hidden_size, M = _batch_token_num;
   const float Q = _quant_range;
   _res = 0;
+  _tap_step = -2;
   CHECK_GPU_ERROR(hipMemsetAsync(_real_seq_len.get(), 0, sizeof(int) * _batch_size, _stream));
   LSH_CALL(gpt_embedding_i8I<__half>(_batch_size, _batch_seq_len, H, _stream, _int8_emb.get(),
                                      _pos_emb.get(), ids, _query[_res].get(), _real_seq_len.get(),
@@ -233,47 +234,62 @@ void QuantGptEncoder::prompt_pass(const int* ids, bool row_major_out) {
   }
 }
 
-// one cached step for the tokens in _last_ids at position _batch_seq_len - 1 (:363-377);
-// returns the buffer that holds the int8 LayerNorm output of the last layer [batch, hidden]
-const int8_t* QuantGptEncoder::step_pass() {
+// One cached step for the tokens in _last_ids at position _batch_seq_len - 1 (:363-377): the
+// embedding, then the layers from..to - 1; after the last layer _step.a holds its int8
+// LayerNorm output [batch, hidden].
+void QuantGptEncoder::step_begin(StepNotice notice) {
   LnFewRowsScope few_rows;  // every step of every batch size: layer norms by the row kernel
   const int H = _tw._hidden_size, B = _batch_size;
   const float Q = _quant_range;
-  int8_t *a = _buf_a.get(), *b = _buf_b.get();
+  _step.a = _buf_a.get();
+  _step.b = _buf_b.get();
   _tap_step = _steps_run;
-  // the step's embedding and the first layer norm are one launch where the row kernel covers
-  // the width (the same bytes); with taps set the two launches run
   // the opt-in launch of the QKV product and the attention reads row-major operands
-  const bool qkv_attn = !step_taps.any() && decself_qkv_attention_enabled() &&
-                        _tw._dim_per_head == 64 &&
-                        decself_qkv_attention_supported(B, H, _tw._head_num, _tw._max_step);
-  const bool ln1_blocked = _ops.blocked && !qkv_attn;
+  _step.qkv_attn = !step_taps.any() && decself_qkv_attention_enabled() && _tw._dim_per_head == 64 &&
+                   decself_qkv_attention_supported(B, H, _tw._head_num, _tw._max_step);
+  _step.ln1_blocked = _ops.blocked && !_step.qkv_attn;
   // few rows: the layer norms between two layers and between the two halves of a layer are made
   // by the products that read them
-  const bool ln_in_product = !step_taps.any() && !qkv_attn && _ops.ln_in_product(B, H);
-  LnStep ln{}, ln_next{};
+  _step.ln_in_product = !step_taps.any() && !_step.qkv_attn && _ops.ln_in_product(B, H);
   _res = 0;
-  const bool emb_ln_fused = !step_taps.any() && H % 4 == 0 && H <= 1024 && _tw._n_enc_layer > 0;
-  if (emb_ln_fused) {
+  if (emb_ln_fused()) {
     const Layer& w0 = _layers[0];
     LSH_CALL(gpt_emb_step_norm_layer_i8O<__half>(
-        _int8_emb.get(), _pos_emb.get(), _last_ids.get(), _query[_res].get(), a, w0.ln1_scale.get(),
-        w0.ln1_bias.get(), w0.b_out.get(), _real_seq_len.get(), _unfinished.get(), B, H,
-        _tw._src_vocab_size, _tw._padding_id, _batch_seq_len - 1, _tw._max_step,
-        _src_emb_clip_max / Q, Q / _enc_clip_max[4], false, _stream, ln1_blocked));
+        _int8_emb.get(), _pos_emb.get(), _last_ids.get(), _query[_res].get(), _step.a,
+        w0.ln1_scale.get(), w0.ln1_bias.get(), w0.b_out.get(), _real_seq_len.get(),
+        _unfinished.get(), B, H, _tw._src_vocab_size, _tw._padding_id, _batch_seq_len - 1,
+        _tw._max_step, _src_emb_clip_max / Q, Q / _enc_clip_max[4], false, _stream,
+        _step.ln1_blocked, notice));
   } else {
     LSH_CALL(gpt_embedding_i8I<__half>(B, 1, H, _stream, _int8_emb.get(), _pos_emb.get(),
                                        _last_ids.get(), _query[_res].get(), _real_seq_len.get(),
                                        _tw._padding_id, _batch_seq_len - 1, _src_emb_clip_max / Q,
                                        _tw._src_vocab_size, _tw._max_step, _unfinished.get()));
   }
+}
+
+// the step's embedding and the first layer norm are one launch where the row kernel covers the
+// width (the same bytes); with taps set the two launches run
+bool QuantGptEncoder::emb_ln_fused() const {
+  return !step_taps.any() && _tw._hidden_size % 4 == 0 && _tw._hidden_size <= 1024 &&
+         _tw._n_enc_layer > 0;
+}
+
+void QuantGptEncoder::step_layers(int from, int to) {
+  LnFewRowsScope few_rows;
+  const int H = _tw._hidden_size, B = _batch_size;
+  const float Q = _quant_range;
+  int8_t *&a = _step.a, *&b = _step.b;
+  const bool qkv_attn = _step.qkv_attn, ln1_blocked = _step.ln1_blocked,
+             ln_in_product = _step.ln_in_product;
+  LnStep ln{}, &ln_next = _step.ln_next;
   const size_t bh = (size_t)B * H;
-  for (_layer_id = 0; _layer_id < _tw._n_enc_layer; _layer_id++) {
+  for (_layer_id = from; _layer_id < to; _layer_id++) {
     Layer& w = _layers[_layer_id];
     const float* c = &_enc_clip_max[_layer_id * 12];
     int8_t* k_cache = _self_k_cache.get() + (size_t)_layer_id * _max_batch_dim;
     int8_t* v_cache = _self_v_cache.get() + (size_t)_layer_id * _max_batch_dim;
-    if (_layer_id == 0 && !emb_ln_fused)
+    if (_layer_id == 0 && !emb_ln_fused())
       LSH_CALL(norm_layer_resual_i8O<__half>(B, H, _stream, _query[_res].get(), a, w.ln1_scale.get(),
                                              w.ln1_bias.get(), w.b_out.get(), Q / c[4], false, ln1_blocked));
     TAP_CODES("ln1_q", a, B, H);
@@ -322,8 +338,7 @@ const int8_t* QuantGptEncoder::step_pass() {
                  nullptr);
     std::swap(a, b);  // `a` names the buffer holding the layer's int8 LayerNorm output
   }
-  _tap_step = -2;
-  return a;
+  if (to == _tw._n_enc_layer) _tap_step = -2;
 }
 
 #undef TAP
@@ -364,14 +379,15 @@ void QuantGptEncoder::set_seed(unsigned long long seed) {
   LSH_CALL(sample_state_setup(_sample_state.get(), _max_batch_size, seed, _stream));
 }
 
-// host side of a sampled token: counters and the unfinished flag (one word back from the device)
-int QuantGptEncoder::finish_token() {
-  const int B = _batch_size;
-  const bool first = _steps_run == 0;
+// host side of a sampled token: the counters
+void QuantGptEncoder::count_token() {
   ++_steps_run;
   _batch_seq_len++;
-  _batch_token_num += B;
-  if (_is_benchmark && !first) return 1;  // nothing stops a benchmark run but the length
+  _batch_token_num += _batch_size;
+}
+
+// the unfinished flag of the step just enqueued (one word back from the device)
+int QuantGptEncoder::read_unfinished() {
   CHECK_GPU_ERROR(hipMemcpyAsync(_h_unfinished, _unfinished.get(), sizeof(int),
                                  hipMemcpyDeviceToHost, _stream));
   CHECK_GPU_ERROR(hipStreamSynchronize(_stream));
@@ -410,17 +426,37 @@ int QuantGptEncoder::run_one_sample(int batch_size, int batch_seq_len) {
   if (_batch_seq_len < _tw._max_step) {
     // (:347-353) after the prompt pass the run ends when nothing is unfinished
     enqueue_sampling(_hid_last[_ops.blocked].get(), true);
-    const bool go_on = !(finish_token() == 0 || _batch_seq_len >= _batch_max_seq_len);
-    _phases.mark(1, _stream);
-    if (go_on) {
+    count_token();
+    const int L = _tw._n_enc_layer;
+    if (!_is_benchmark && !_use_graphs && !_rec_logits && emb_ln_fused()) {
+      // Whether a step is needed is known while the device works at its first layers: two, that
+      // is 25 to 40 us, cover the way of the word to the host and of a launch to the device.
+      const int ahead = std::min(2, L);
+      _phases.mark(1, _stream);
       while (_batch_seq_len < _batch_max_seq_len) {
+        step_begin(_notice.next(_unfinished.get()));
+        step_layers(0, ahead);
+        if (_notice.wait(_stream) == 0) break;
+        ++loop_steps;
+        step_layers(ahead, L);
+        enqueue_sampling(_step.a, false);
+        count_token();
+      }
+    } else {
+      const bool go_on = !(read_unfinished() == 0 || _batch_seq_len >= _batch_max_seq_len);
+      _phases.mark(1, _stream);
+      while (go_on && _batch_seq_len < _batch_max_seq_len) {
         ++loop_steps;
         // the launches of a step depend on the batch size and the position only
         const uint64_t key = ((uint64_t)_batch_size << 32) | (uint32_t)_batch_seq_len;
-        _graphs.run(key, _stream, _use_graphs && !_rec_logits && !step_taps.any(),
-                    [&] { enqueue_sampling(step_pass(), false); });
-        int unfinished = finish_token();
-        if (!unfinished && !_is_benchmark) break;
+        _graphs.run(key, _stream, _use_graphs && !_rec_logits && !step_taps.any(), [&] {
+          step_begin(StepNotice{});
+          step_layers(0, L);
+          enqueue_sampling(_step.a, false);
+        });
+        count_token();
+        // nothing stops a benchmark run but the length
+        if (!_is_benchmark && read_unfinished() == 0) break;
       }
     }
   } else {

@@ -61,12 +61,15 @@ class QuantGptEncoder {
 
  private:
   void prompt_pass(const int* ids, bool row_major_out);
-  const int8_t* step_pass();
+  void step_begin(lsh::StepNotice notice);
+  bool emb_ln_fused() const;
+  void step_layers(int from, int to);
   void ffn_add_norm(int rows, int8_t* in, int8_t* tmp, bool blocked_out, const lsh::LnStep* ln_in,
                     lsh::LnStep* ln_out);
   void logits_product(const int8_t* hidden, int rows);
   void enqueue_sampling(const int8_t* hidden, bool clear_flag);
-  int finish_token();
+  void count_token();
+  int read_unfinished();
 
   const int _max_batch_size;
   const QuantGptWeight& _tw;
@@ -84,6 +87,12 @@ class QuantGptEncoder {
   PhaseEvents _phases;
   long _max_batch_dim;
   int* _h_unfinished = nullptr;  // pinned
+  HostNotice _notice;
+  struct {                       // the step being enqueued
+    int8_t *a, *b;               // a: input, then output of a layer
+    bool qkv_attn, ln1_blocked, ln_in_product;
+    lsh::LnStep ln_next;         // what the next layer's first product makes for itself
+  } _step{};
   int8_t* _rec_logits = nullptr;
   int _tap_step = -2;  // the cached step being enqueued (tokens sampled so far), -2 outside one
   int _rec_max_steps = 0;
