@@ -326,6 +326,23 @@ int ls_quant_linear_layer_fw_fp16(int layer_id, const void* inputs, const void* 
 /* Releases a layer and its buffers (the reference keeps them until the process ends). */
 int ls_destroy_layer(const char* layer_name, int layer_id);
 
+/* A forward pass in one call: stream, parameters, shape and the caller's own padding mask (1 for
+ * padding) of element type mask_type -- 0: the additive fp16 mask of the fw functions; 1: float,
+ * 2: fp16, 3: 8-bit (bool), 4: int32, 5: int64.  enc_output of the decoder layer: token s of
+ * sentence b at b * enc_stride_batch + s * enc_stride_seq (elements, multiples of 8; hidden values
+ * contiguous); layer 0 reads it where it makes the cross-attention keys and values (step <= 0).
+ * The five cache pointers are those of ls_transformer_decoder_layer_fw_fp16. */
+int ls_encoder_layer_call_fp16(int layer_id, const void* weights, const void* input, const void* padding_mask,
+                               int mask_type, void* output, int batch_size, int seq_len,
+                               int training_mode, int quant_mode, lsh_stream_t stream);
+int ls_decoder_layer_call_fp16(int layer_id, const void* weights, const void* dec_input,
+                               const void* enc_output, int64_t enc_stride_batch,
+                               int64_t enc_stride_seq, const void* padding_mask, int mask_type,
+                               void* dec_output, int batch_size, int trg_seq_len, int src_seq_len,
+                               int step, const void* new_k, const void* new_v, const void* old_k,
+                               const void* old_v, const void* encdec_kv, int training_mode,
+                               int quant_mode, lsh_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

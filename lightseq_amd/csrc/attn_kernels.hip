@@ -11,6 +11,7 @@
 #include <type_traits>
 
 #include "ls_device.h"
+#include "layer_device.h"
 #include "ls_launch.h"
 #include "tile_common.h"
 
@@ -132,7 +133,7 @@ encself_attn_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
                     const __half* __restrict__ v, const int* __restrict__ pad_mask,
                     __half* __restrict__ ctx, int8_t* __restrict__ ctx_q, float quant_scale, int S,
                     int head_num, float alpha, float dq, int key_len,
-                    const int* __restrict__ seq) {
+                    const int* __restrict__ seq, const __half* __restrict__ q_cmax, int k_pad) {
   const int bh = blockIdx.y;
   const int b = bh / head_num, head = bh % head_num;
   // Packed rows (MODE 3 with an EncPack plan, ctx_q then a blocked matrix): the sequence is rows
@@ -354,6 +355,52 @@ encself_attn_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
               }
             }
           }
+        } else if constexpr (ONE && MODE == kAttnLayer) {
+          // keys, values and mask are requested together before any of them is stored (one trip
+          // to memory instead of one per loop iteration: 14 -> 12 us); rows past the end
+          // read the last one and become zeros
+          constexpr int KCH = 128 * CH / NT, NP = 32 * CH, VP = (NP + NT - 1) / NT;
+          v8h kr[KCH], vr[VP][4];
+#pragma unroll
+          for (int i = 0; i < KCH; ++i) {
+            const int c = tid + i * NT;
+            kr[i] = *reinterpret_cast<const v8h*>(kbase + (long)min(c / CH, Sk - 1) * D + (c % CH) * 8);
+          }
+#pragma unroll
+          for (int i = 0; i < VP; ++i) {
+            const int p = min(tid + i * NT, NP - 1);
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              vr[i][r] = *reinterpret_cast<const v8h*>(
+                  vbase + (long)min(p / CH * 4 + r, Sk - 1) * D + (p % CH) * 8);
+          }
+          __half am = __float2half_rn(0.f);
+          if (pad_mask != nullptr)
+            am = reinterpret_cast<const __half*>(pad_mask)[(long)b * Sk + min(tid, Sk - 1)];
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int i = 0; i < KCH; ++i) {
+            const int c = tid + i * NT;
+            *reinterpret_cast<v8h*>(&Ks[c / CH * KSTR + (c % CH) * 8]) =
+                c / CH < Sk ? kr[i] : (v8h)(_Float16)0;
+          }
+#pragma unroll
+          for (int i = 0; i < VP; ++i) {
+            const int p = tid + i * NT, kg = p / CH, ch = p % CH;
+            if (p < NP) {
+#pragma unroll
+              for (int r = 0; r < 4; ++r)
+                if (kg * 4 + r >= Sk) vr[i][r] = (v8h)(_Float16)0;
+#pragma unroll
+              for (int e = 0; e < 8; ++e)
+                *reinterpret_cast<v4h*>(&Vt[(ch * 8 + e) * VSTR + kg * 4]) =
+                    (v4h){vr[i][0][e], vr[i][1][e], vr[i][2][e], vr[i][3][e]};
+            }
+          }
+          if (tid < 128) {
+            msk[tid] = tid < Sk ? 0 : 1;
+            addm[tid] = tid < Sk ? __half2float(am) : 0.f;
+          }
         } else {
           for (int c = tid; c < 128 * CH; c += NT) {
             const int row = c / CH, ch = c % CH;
@@ -380,7 +427,7 @@ encself_attn_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
             }
           }
         }
-        if (tid < 128) {
+        if (!(ONE && MODE == kAttnLayer) && tid < 128) {
           if (MODE == kAttnLayer) {
             msk[tid] = (key0 + tid < Sk) ? 0 : 1;
             addm[tid] = (key0 + tid < Sk && pad_mask != nullptr)
@@ -396,6 +443,11 @@ encself_attn_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
         __syncthreads();
 #pragma unroll
         for (int sb = 0; sb < 4; ++sb) {
+          if (MODE == kAttnLayer && key0 + sb * 32 >= Sk) {  // no key in this block of 32
+#pragma unroll
+            for (int i = 0; i < 16; ++i) sc[sb][i] = kFloatInfNeg;
+            continue;
+          }
           v16f c;
 #pragma unroll
           for (int i = 0; i < 16; ++i) c[i] = 0.f;
@@ -468,6 +520,7 @@ encself_attn_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
         constexpr bool REUSE = decltype(reuse_tag)::value;
 #pragma unroll
         for (int sb = 0; sb < 4; ++sb) {
+          if (MODE == kAttnLayer && kb * 128 + sb * 32 >= Sk) continue;
 #pragma unroll
           for (int t = 0; t < 2; ++t) {
             v8h pb;
@@ -508,6 +561,7 @@ encself_attn_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
   if (qi >= S) return;
   const long tok = row0 + qi;
   const int hidden = head_num * D;
+  const Quantiser codes_of = Quantiser::of(MODE == kAttnLayer && q_cmax != nullptr ? cm(q_cmax) : 1.f);
 #pragma unroll
   for (int db = 0; db < D / 32; ++db) {
 #pragma unroll
@@ -525,7 +579,11 @@ encself_attn_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
         else
           *reinterpret_cast<half4_t*>(ctx + ((long)bh * S + qi) * D + dd) = t;
       }
-      if (ctx_q != nullptr) {
+      if (MODE == kAttnLayer) {
+        if (ctx_q != nullptr)
+          *reinterpret_cast<uint32_t*>(ctx_q + blocked_offset(tok, head * D + dd, k_pad)) =
+              pack4_i8(codes_of.code(o[0]), codes_of.code(o[1]), codes_of.code(o[2]), codes_of.code(o[3]));
+      } else if (ctx_q != nullptr) {
         // a padded query gives zeros, whose code is 0
         const uint32_t w4 = float2int8_pack4(o[0], o[1], o[2], o[3], quant_scale);
         *reinterpret_cast<uint32_t*>(ctx_q + code_offset(tok, head * D + dd, hidden, seq != nullptr)) =
@@ -541,18 +599,20 @@ template <int MODE>
 static bool launch_attn(int dim_per_head, int seq_len, int batch_heads, hipStream_t s,
                         const __half* q, const __half* k, const __half* v, const int* pad_mask,
                         __half* ctx, int8_t* ctx_q, float quant_scale, int head_num, float alpha,
-                        float dq, int key_len = -1, const int* seq = nullptr) {
+                        float dq, int key_len = -1, const int* seq = nullptr,
+                        const __half* q_cmax = nullptr, int k_pad = 0) {
   if (key_len < 0) key_len = seq_len;  // self attention: as many keys as queries
 #define LSH_ATTN(DD, NWV)                                                                      \
   if (key_len <= 128)                                                                          \
     encself_attn_kernel<DD, MODE, NWV, true>                                                   \
         <<<dim3((seq_len + 32 * NWV - 1) / (32 * NWV), batch_heads), 64 * NWV, 0, s>>>(        \
             q, k, v, pad_mask, ctx, ctx_q, quant_scale, seq_len, head_num, alpha, dq, key_len,  \
-            seq);                                                                              \
+            seq, q_cmax, k_pad);                                                               \
   else                                                                                         \
     encself_attn_kernel<DD, MODE, NWV, false>                                                  \
       <<<dim3((seq_len + 32 * NWV - 1) / (32 * NWV), batch_heads), 64 * NWV, 0, s>>>(          \
-          q, k, v, pad_mask, ctx, ctx_q, quant_scale, seq_len, head_num, alpha, dq, key_len, seq)
+          q, k, v, pad_mask, ctx, ctx_q, quant_scale, seq_len, head_num, alpha, dq, key_len, seq, \
+          q_cmax, k_pad)
   const bool wide = seq_len > 64;
   switch (dim_per_head) {
     case 32:
@@ -684,6 +744,214 @@ int layer_cross_attention_f16(const __half* q, const __half* k, const __half* v,
   const float causal = mask_future ? 1.f : 0.f;
   if (!launch_attn<kAttnLayer>(dim_per_head, seq_len, batch * head_num, s, q, k, v, m, ctx,
                                nullptr, 0.f, head_num, alpha, causal, key_len))
+    return lsh_fail(LSH_ERR_UNSUPPORTED, "layer_attention: dim_per_head must be 32, 64 or 128");
+  return lsh_check_launch("encself_attn_kernel<layer>");
+}
+
+// ---------------------------------------------------------------------------------
+// A few queries per (batch, head) pair: the self attention of a cached decoding step (one query
+// per row), the cross attention of its beams, short sequences.  The kernel above gives a pair a
+// workgroup and stages keys and values in LDS through two barriers, which for one query is 14 us
+// of a launch.
+// Here a wavefront owns 32 queries of a pair and is a workgroup by itself: the keys come from memory
+// as MFMA fragments, the values as rows, all requested before the first product; only the values
+// change places in 4.5 KB of LDS that no other wavefront sees, so there is no barrier.  Same
+// products, same order of every sum and same rounding as above, hence the same bits.
+// 64 rows x 16 heads x 32 keys: 14 -> 6.7 us.
+// NKB: blocks of 32 keys (at most 128 keys).
+template <int D, int NKB>
+__global__ void __launch_bounds__(64)
+layer_attn_few_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
+                      const __half* __restrict__ v, const __half* __restrict__ add_mask,
+                      int8_t* __restrict__ codes, const __half* __restrict__ q_cmax, int k_pad, int q_blocks,
+                      int q_len, int head_num, int key_len, float alpha, int causal) {
+  constexpr int CH = D / 8, VS = 36;  // 16-byte chunks of a row; halfs per dimension in LDS
+  constexpr int VP = 8 * CH / 64 > 0 ? 8 * CH / 64 : 1;  // patches of 4 keys x 8 dims per lane and block
+  __shared__ __align__(16) _Float16 Vt[D * VS];
+  __shared__ __align__(16) float addm[NKB * 32];
+  const int lane = threadIdx.x;
+  const int bh = (int)blockIdx.x / q_blocks, q0 = ((int)blockIdx.x - bh * q_blocks) * 32;
+  const int b = bh / head_num, head = bh - b * head_num;
+  const int l32 = lane & 31, g = lane >> 5;
+  const int qi = q0 + l32;
+  const _Float16* qb = reinterpret_cast<const _Float16*>(q) + (long)bh * q_len * D;
+  const _Float16* kb = reinterpret_cast<const _Float16*>(k) + (long)bh * key_len * D;
+  const _Float16* vb = reinterpret_cast<const _Float16*>(v) + (long)bh * key_len * D;
+  v8h qreg[D / 16], kf[NKB][D / 16], vr[NKB][VP][4];
+#pragma unroll
+  for (int ks = 0; ks < D / 16; ++ks)
+    qreg[ks] = *reinterpret_cast<const v8h*>(qb + (long)min(qi, q_len - 1) * D + ks * 16 + g * 8);
+#pragma unroll
+  for (int sb = 0; sb < NKB; ++sb)
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks)
+      kf[sb][ks] = *reinterpret_cast<const v8h*>(kb + (long)min(sb * 32 + l32, key_len - 1) * D + ks * 16 + g * 8);
+  uint32_t am[(NKB + 1) / 2];
+  // (without a mask any values are read and dropped: a load inside a branch is followed by its wait)
+  const __half* mp = add_mask ? add_mask + (long)b * key_len : reinterpret_cast<const __half*>(kb);
+#pragma unroll
+  for (int i = 0; i < (NKB + 1) / 2; ++i) am[i] = __half_as_ushort(mp[min(i * 64 + lane, key_len - 1)]);
+#pragma unroll
+  for (int sb = 0; sb < NKB; ++sb)
+#pragma unroll
+    for (int i = 0; i < VP; ++i) {
+      const int p = (lane + 64 * i) % (8 * CH), kg = p / CH, ch = p % CH;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        vr[sb][i][r] = *reinterpret_cast<const v8h*>(vb + (long)min(sb * 32 + kg * 4 + r, key_len - 1) * D + ch * 8);
+    }
+  const Quantiser codes_of = Quantiser::of(cm(q_cmax));
+  __builtin_amdgcn_sched_barrier(0);
+  auto wave_sync = [&]() {  // LDS written by this wavefront, read by this wavefront
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+#pragma unroll
+  for (int i = 0; i < (NKB + 1) / 2; ++i) {
+    asm volatile("" : "+v"(am[i]));
+    const float x = __half2float(__ushort_as_half((unsigned short)am[i]));
+    if (i * 64 + lane < NKB * 32) addm[i * 64 + lane] = add_mask ? x : 0.f;
+  }
+  wave_sync();
+  const int last_key = min(key_len - 1, causal ? qi : key_len - 1);
+  float m = kFloatInfNeg;
+  v16f sc[NKB];
+#pragma unroll
+  for (int sb = 0; sb < NKB; ++sb) {
+    v16f c = (v16f)0.f;
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks)
+      c = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[sb][ks], qreg[ks], c, 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int key0 = sb * 32 + 8 * j + 4 * g;
+      const float4 am4 = *reinterpret_cast<const float4*>(&addm[key0]);
+      const float a4[4] = {am4.x, am4.y, am4.z, am4.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float t = round_h(alpha * c[4 * j + i]) + a4[i];
+        // (no short circuit: branches around a few instructions cost more than they skip)
+        const bool hidden = (key0 + i > last_key) | !(t > 0.5f * kFloatInfNeg);
+        sc[sb][4 * j + i] = hidden ? kFloatInfNeg : t;
+        m = fmaxf(m, sc[sb][4 * j + i]);
+      }
+    }
+  }
+  m = fmaxf(m, __shfl_xor(m, 32, 64));
+  const float nm = -(m == kFloatInfNeg ? 0.f : m) * 1.44269504088896340736f;
+  float sum = 0.f;
+#pragma unroll
+  for (int sb = 0; sb < NKB; ++sb)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      sc[sb][i] = __builtin_amdgcn_exp2f(fmaf(sc[sb][i], 1.44269504088896340736f, nm));
+      sum += sc[sb][i];
+    }
+  sum += __shfl_xor(sum, 32, 64);
+  float rs = __builtin_amdgcn_rcpf(sum);
+  rs = sum > 0.f ? fmaf(fmaf(-sum, rs, 1.f), rs, rs) : 0.f;  // no visible key: all zero
+  v16f acc[D / 32];
+#pragma unroll
+  for (int db = 0; db < D / 32; ++db) acc[db] = (v16f)0.f;
+#pragma unroll
+  for (int sb = 0; sb < NKB; ++sb) {
+    if (sb > 0) wave_sync();  // the last block's values have been read
+#pragma unroll
+    for (int i = 0; i < VP; ++i) {
+      const int p = (lane + 64 * i) % (8 * CH), kg = p / CH, ch = p % CH;
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        *reinterpret_cast<v4h*>(&Vt[(ch * 8 + e) * VS + kg * 4]) =
+            (v4h){vr[sb][i][0][e], vr[sb][i][1][e], vr[sb][i][2][e], vr[sb][i][3][e]};
+    }
+    wave_sync();
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      v8h pb;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float e = sc[sb][8 * t + j];
+        float qt = e * rs;
+        qt = fmaf(fmaf(-sum, qt, e), rs, qt);
+        asm volatile("" : "+v"(qt));  // a value of its own (see above)
+        pb[j] = (_Float16)qt;
+      }
+#pragma unroll
+      for (int db = 0; db < D / 32; ++db) {
+        const _Float16* vrow = &Vt[(db * 32 + l32) * VS + 16 * t + 4 * g];
+        const v4h lo = *reinterpret_cast<const v4h*>(vrow), hi = *reinterpret_cast<const v4h*>(vrow + 8);
+        const v8h a = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pb, acc[db], 0, 0, 0);
+      }
+    }
+  }
+  if (qi >= q_len) return;
+  const long row = (long)b * q_len + qi;
+#pragma unroll
+  for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+    for (int vg = 0; vg < 4; ++vg) {
+      const int dd = db * 32 + 8 * vg + 4 * g;
+      int c[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) c[j] = codes_of.code(round_h(acc[db][4 * vg + j]));
+      *reinterpret_cast<uint32_t*>(codes + blocked_offset(row, head * D + dd, k_pad)) =
+          pack4_i8(c[0], c[1], c[2], c[3]);
+    }
+}
+
+template <int D>
+static void launch_attn_few(const __half* q, const __half* k, const __half* v, const __half* add_mask,
+                            int8_t* codes, const __half* cmax, int k_pad, int pairs, int q_len, int head_num,
+                            int key_len, float alpha, bool causal, hipStream_t s) {
+  const int q_blocks = (q_len + 31) / 32;
+#define LSH_FEW(NKB)                                                                                    \
+  layer_attn_few_kernel<D, NKB><<<pairs * q_blocks, 64, 0, s>>>(q, k, v, add_mask, codes, cmax, k_pad,  \
+                                                                q_blocks, q_len, head_num, key_len,     \
+                                                                alpha, causal ? 1 : 0)
+  if (key_len <= 32) LSH_FEW(1);
+  else if (key_len <= 64) LSH_FEW(2);
+  else if (key_len <= 96) LSH_FEW(3);
+  else LSH_FEW(4);
+#undef LSH_FEW
+}
+
+constexpr int kAttnFewQueries = 128;
+
+int layer_attention_codes(const __half* q, const __half* k, const __half* v, const __half* add_mask,
+                          int8_t* codes, const __half* cmax, int k_pad, int batch, int seq_len, int key_len,
+                          int head_num, int dim_per_head, bool mask_future, hipStream_t s) {
+  if (batch <= 0 || seq_len <= 0 || key_len <= 0 || head_num <= 0 || !q || !k || !v || !codes || !cmax ||
+      k_pad % 64 != 0 || k_pad < head_num * dim_per_head || (mask_future && seq_len != key_len))
+    return lsh_fail(LSH_ERR_INVALID, "layer_attention_codes: bad arguments");
+  if (seq_len > 1024 || key_len > 1024)
+    return lsh_fail(LSH_ERR_UNSUPPORTED, "layer_attention: seq_len > 1024");
+  if (((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v) |
+        reinterpret_cast<uintptr_t>(codes)) & 15u) != 0)
+    return lsh_fail(LSH_ERR_INVALID, "layer_attention: pointers must be 16-byte aligned");
+  const float alpha = __half2float(
+      __float2half_rn(1.0f / __half2float(__float2half_rn(sqrtf((float)dim_per_head)))));
+  // Few queries: the fragments of a pair's keys and values fit a wavefront's registers up to 128 keys
+  // of 64 dimensions (64 of 128).
+  const long pairs = (long)batch * head_num;
+  if (seq_len <= kAttnFewQueries && pairs < (1L << 30) && key_len * dim_per_head <= 128 * 64 && key_len <= 128) {
+    if (dim_per_head == 32)
+      launch_attn_few<32>(q, k, v, add_mask, codes, cmax, k_pad, (int)pairs, seq_len, head_num, key_len, alpha,
+                          mask_future, s);
+    else if (dim_per_head == 64)
+      launch_attn_few<64>(q, k, v, add_mask, codes, cmax, k_pad, (int)pairs, seq_len, head_num, key_len, alpha,
+                          mask_future, s);
+    else if (dim_per_head == 128)
+      launch_attn_few<128>(q, k, v, add_mask, codes, cmax, k_pad, (int)pairs, seq_len, head_num, key_len, alpha,
+                           mask_future, s);
+    else
+      return lsh_fail(LSH_ERR_UNSUPPORTED, "layer_attention: dim_per_head must be 32, 64 or 128");
+    return lsh_check_launch("layer_attn_few_kernel");
+  }
+  if (!launch_attn<kAttnLayer>(dim_per_head, seq_len, batch * head_num, s, q, k, v,
+                               reinterpret_cast<const int*>(add_mask), nullptr, codes, 0.f, head_num, alpha,
+                               mask_future ? 1.f : 0.f, key_len, nullptr, cmax, k_pad))
     return lsh_fail(LSH_ERR_UNSUPPORTED, "layer_attention: dim_per_head must be 32, 64 or 128");
   return lsh_check_launch("encself_attn_kernel<layer>");
 }

@@ -1,0 +1,209 @@
+// The kernels and the dispatch of products on blocked operands, shared by the files that bring
+// epilogues (gemm_blocked.hip: the models', layer_gemm.hip: the layers').
+#pragma once
+#include "gemm_kw.h"
+#include "ls_launch.h"
+
+#include <hip/hip_ext.h>
+
+#include <algorithm>
+#include <mutex>
+
+namespace lsh {
+
+// one output tile per workgroup, both operands blocked
+template <typename Tr, typename Epi, int WGM, int WGN, int MB, int NB, int NST>
+__global__ void __launch_bounds__(64 * WGM * WGN)
+gemm_blk_tile_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, Epi epi, int M,
+                     int N, int K, int tiles_m, int tiles_n) {
+  extern __shared__ __align__(16) int8_t smem[];
+  asm volatile("" : "+s"(tiles_m) : "s"(A), "s"(W));
+  constexpr int TM = WGM * MB * 32;
+  int tm, tn;
+  tile_of(blockIdx.x, tiles_m * tiles_n, tiles_m, tiles_n, tm, tn);
+  tile_gemm<Epi, WGM, WGN, MB, NB, NST, false, true, typename Tr::Acc16>(A, W, epi, tm * TM, M, N, K, tn, smem);
+}
+
+template <auto Kern>
+int raise_lds(size_t smem) {
+  static std::mutex mu;
+  static unsigned long long done = 0;  // bit per device index
+  int dev = 0;
+  if (int rc = lsh_check_hip(hipGetDevice(&dev), "hipGetDevice(gemm_blk)")) return rc;
+  if (dev < 0 || dev >= 64) return lsh_fail(LSH_ERR_UNSUPPORTED, "blocked gemm: device index out of range");
+  std::lock_guard<std::mutex> lock(mu);
+  if (!(done >> dev & 1ull)) {
+    if (smem > 64 * 1024)
+      if (int rc = lsh_check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(Kern),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem),
+                                 "hipFuncSetAttribute(gemm_blk)"))
+        return rc;
+    done |= 1ull << dev;
+  }
+  return LSH_OK;
+}
+
+template <auto Kern, typename... Args>
+int launch_blk(dim3 grid, int threads, size_t smem, hipStream_t s, Args... args) {
+  if (int rc = raise_lds<Kern>(smem)) return rc;
+  hipEvent_t e0, e1;
+  if (gemm_take_timing_events(&e0, &e1))
+    hipExtLaunchKernelGGL(Kern, grid, dim3(threads), (unsigned)smem, s, e0, e1, 0, args...);
+  else
+    Kern<<<grid, threads, smem, s>>>(args...);
+  return lsh_check_launch("blocked gemm");
+}
+
+template <typename Tr, typename Epi, int MB, int NB>
+int launch_kw(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K, int ksplit,
+              hipStream_t s) {
+  const int tm = (M + 16 * MB - 1) / (16 * MB), tn = (N + 16 * NB - 1) / (16 * NB);
+  const dim3 grid(tm * tn, ksplit);
+  constexpr size_t smem = kw_lds_bytes<Epi, MB, NB>();
+  const int slices = K / 64 / ksplit;
+#define LSH_KW(D)                                                                                   \
+  return launch_blk<gemm_kw_kernel<Tr, Epi, MB, NB, D>>(grid, 256, smem, s, A, W, epi, M, N, K, slices, tm, tn)
+  if (slices % 16 == 0) LSH_KW(4);
+  if (slices % 12 == 0) LSH_KW(3);
+  if (slices % 8 == 0) LSH_KW(2);
+  LSH_KW(1);
+#undef LSH_KW
+}
+
+// The LDS tile kernel: 8 wavefronts for the tall tiles, 4 for 128 x 128 and 128 x 64 (two or three
+// workgroups then share a compute unit and one's epilogue runs under the other's K loop).
+constexpr TileCost kLdsCost[] = {{128, 64, 2.5f, 2.45f, 0.2f, 2.6f, 0.6f},
+                                 {128, 128, 2.9f, 3.6f, 0.6f, 4.9f, 0.9f},
+                                 {256, 128, 3.1f, 5.4f, 1.5f, 9.0f, 1.3f},
+                                 {256, 192, 3.6f, 7.1f, 3.0f, 9.5f, 1.7f},
+                                 {256, 256, 4.1f, 9.2f, 4.0f, 12.0f, 2.4f}};
+struct LdsTile {
+  int tm = 0, tn = 0;
+  float us = 0;
+};
+inline LdsTile choose_lds_tile(int M, int N, int K, int cus, bool table) {
+  LdsTile best;
+  if (K % kBK != 0 || K / kBK < 3 || N % 16 != 0) return best;
+  for (const auto& c : kLdsCost) {
+    const float us = tile_us(c, M, N, K, 1, cus, table);
+    if (best.tm == 0 || us < best.us) best = LdsTile{c.tm, c.tn, us};
+  }
+  return best;
+}
+
+inline int check_blk(const int8_t* A, const int8_t* W, bool aligned, int M, int N, int K) {
+  if (M <= 0 || N <= 0 || K <= 0 || !A || !W)
+    return lsh_fail(LSH_ERR_INVALID, "blocked gemm: bad arguments");
+  if (K % 64 != 0 || N % 4 != 0)
+    return lsh_fail(LSH_ERR_UNSUPPORTED, "blocked gemm: needs K bytes % 64 == 0 and N % 4 == 0");
+  if (((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W)) & 15u) != 0 || !aligned)
+    return lsh_fail(LSH_ERR_INVALID, "blocked gemm: operands must be 16-byte aligned");
+  const unsigned long long lim = 0xffffffffull;
+  if ((unsigned long long)(M + 15) / 16 * 16 * K >= lim || (unsigned long long)(N + 15) / 16 * 16 * K >= lim ||
+      (long)((M + 15) / 16) * ((N + 15) / 16) >= (1L << 24))
+    return lsh_fail(LSH_ERR_UNSUPPORTED, "blocked gemm: operand or output too large");
+  return LSH_OK;
+}
+
+template <typename Tr, typename Epi, bool TILES>
+int dispatch_blk(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K, hipStream_t s,
+                 int ksplit = 1) {
+  if (int rc = check_blk(A, W, epi.aligned(), M, N, K)) return rc;
+  if (ksplit < 1 || K % (64 * ksplit) != 0)
+    return lsh_fail(LSH_ERR_INVALID, "blocked gemm: K does not split into whole 64-byte slices");
+  const int cus = cu_count();
+  const KwTile kw = kw_choose_tile(M, N, K / ksplit, ksplit, cus, Epi::kTable);
+  if constexpr (TILES) {
+    if (ksplit == 1) {
+      const LdsTile t = choose_lds_tile(M, N, K, cus, Epi::kTable);
+      if (t.tm != 0 && t.us < kw.us) {
+        const int tm = (M + t.tm - 1) / t.tm, tn = (N + t.tn - 1) / t.tn;
+        const dim3 grid(tm * tn);
+        if (t.tn == 256)
+          return launch_blk<gemm_blk_tile_kernel<Tr, Epi, 2, 4, 4, 2, 2>>(grid, 512, 2 * 512 * kBK, s, A, W, epi, M, N,
+                                                                      K, tm, tn);
+        if (t.tn == 192)
+          return launch_blk<gemm_blk_tile_kernel<Tr, Epi, 4, 2, 2, 3, 2>>(grid, 512, 2 * 448 * kBK, s, A, W, epi, M, N,
+                                                                      K, tm, tn);
+        if (t.tm == 256)
+          return launch_blk<gemm_blk_tile_kernel<Tr, Epi, 4, 2, 2, 2, 3>>(grid, 512, 3 * 384 * kBK, s, A, W, epi, M, N,
+                                                                      K, tm, tn);
+        if (t.tn == 128)
+          return launch_blk<gemm_blk_tile_kernel<Tr, Epi, 2, 2, 2, 2, 2>>(grid, 256, 2 * 256 * kBK, s, A, W, epi, M, N,
+                                                                      K, tm, tn);
+        // long K loops: a third stage instead of a third workgroup per compute unit
+        if (K >= 2048)
+          return launch_blk<gemm_blk_tile_kernel<Tr, Epi, 4, 1, 1, 2, 3>>(grid, 256, 3 * 192 * kBK, s, A, W, epi, M, N,
+                                                                      K, tm, tn);
+        return launch_blk<gemm_blk_tile_kernel<Tr, Epi, 4, 1, 1, 2, 2>>(grid, 256, 2 * 192 * kBK, s, A, W, epi, M, N, K,
+                                                                    tm, tn);
+      }
+    }
+  }
+  if (kw.mb == 1) return launch_kw<Tr, Epi, 1, 1>(A, W, epi, M, N, K, ksplit, s);
+  if (kw.mb == 2) return launch_kw<Tr, Epi, 2, 2>(A, W, epi, M, N, K, ksplit, s);
+  if (kw.nb == 2) return launch_kw<Tr, Epi, 4, 2>(A, W, epi, M, N, K, ksplit, s);
+  return launch_kw<Tr, Epi, 4, 4>(A, W, epi, M, N, K, ksplit, s);
+}
+
+
+// fp16 products: every output one chain in ascending K (gemm_seq_kernel).  The estimates, in us with k
+// = K in units of 1000 bytes, are fits to a sweep of hidden 512, 768 and 1024 (K of one and of
+// four times that) over M from 4 to 8192; the smallest one is within 15 % of the fastest there.
+struct SeqTile {
+  int kind;  // 0: a wavefront per 16 x 16, 1: per 32 x 32; 2 - 4: LDS tiles 64 x 64, 128 x 64, 128 x 128
+  float us;
+};
+inline SeqTile choose_seq(int M, int N, int K) {
+  const float k = (float)K / 1000.f;
+  auto tiles = [&](int tm, int tn) { return (float)((long)((M + tm - 1) / tm) * ((N + tn - 1) / tn)); };
+  auto lds = [&](float t, float first, float more) {
+    return 2.f + first * k + (t > 256.f ? (t / 256.f - 1.f) * (1.f + more * k) : 0.f);
+  };
+  SeqTile best{0, std::max(std::max(2.8f, 0.9f + 0.5f * k), 2.f + 0.00095f * tiles(16, 16) * k)};
+  auto take = [&](int kind, float us) {
+    if (us < best.us) best = SeqTile{kind, us};
+  };
+  take(1, std::max(1.f + 1.2f * k, 2.f + 0.0022f * tiles(32, 32) * k));
+  if (K % kBK == 0 && K / kBK >= 3 && N % 16 == 0) {
+    take(2, lds(tiles(64, 64), 1.9f, 1.4f));
+    take(3, lds(tiles(128, 64), 3.7f, 1.8f));
+    take(4, lds(tiles(128, 128), 4.5f, 2.2f));
+  }
+  return best;
+}
+
+template <typename Epi, int MB, int D>
+int launch_seq(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K, hipStream_t s) {
+  const int tm = (M + 16 * MB - 1) / (16 * MB), tn = (N + 16 * MB - 1) / (16 * MB);
+  return launch_blk<gemm_seq_kernel<KwF16, Epi, 1, 1, MB, MB, D>>(dim3(tm * tn), 64, 0, s, A, W, epi, M, N, K,
+                                                                  K / 64, tm, tn);
+}
+template <typename Epi, int WGM, int WGN, int MB, int NB, int NST>
+int launch_f16_tile(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K, hipStream_t s) {
+  constexpr int TM = WGM * MB * 32, TN = WGN * NB * 32;
+  const int tm = (M + TM - 1) / TM, tn = (N + TN - 1) / TN;
+  return launch_blk<gemm_blk_tile_kernel<KwF16, Epi, WGM, WGN, MB, NB, NST>>(
+      dim3(tm * tn), 64 * WGM * WGN, NST * (TM + TN) * kBK, s, A, W, epi, M, N, K, tm, tn);
+}
+
+// K in bytes
+template <typename Epi>
+int dispatch_f16(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K, hipStream_t s) {
+  if (int rc = check_blk(A, W, epi.aligned(), M, N, K)) return rc;
+  const int slices = K / 64;
+  switch (choose_seq(M, N, K).kind) {
+    case 0:
+      if (slices % 16 == 0) return launch_seq<Epi, 1, 16>(A, W, epi, M, N, K, s);
+      if (slices % 8 == 0) return launch_seq<Epi, 1, 8>(A, W, epi, M, N, K, s);
+      return launch_seq<Epi, 1, 1>(A, W, epi, M, N, K, s);
+    case 1:
+      if (slices % 4 == 0) return launch_seq<Epi, 2, 4>(A, W, epi, M, N, K, s);
+      return launch_seq<Epi, 2, 1>(A, W, epi, M, N, K, s);
+    case 2: return launch_f16_tile<Epi, 2, 2, 1, 1, 3>(A, W, epi, M, N, K, s);
+    case 3: return launch_f16_tile<Epi, 4, 1, 1, 2, 2>(A, W, epi, M, N, K, s);
+    default: return launch_f16_tile<Epi, 2, 2, 2, 2, 2>(A, W, epi, M, N, K, s);
+  }
+}
+
+}  // namespace lsh

@@ -5,30 +5,11 @@
 //
 // Two kernels: gemm_kw_kernel (gemm_kw.h) for outputs of up to a few rounds of small tiles, and
 // the LDS tile loop of gemm_tile.h for the large ones.  The dispatch estimates both.
+#include "gemm_blk_dispatch.h"
 #include "gemm_dec_epi.h"
-#include "gemm_kw.h"
 #include "ln_step.h"
-#include "ls_launch.h"
-
-#include <hip/hip_ext.h>
-
-#include <algorithm>
-#include <mutex>
 
 namespace lsh {
-
-// one output tile per workgroup, both operands blocked
-template <typename Epi, int WGM, int WGN, int MB, int NB, int NST>
-__global__ void __launch_bounds__(64 * WGM * WGN)
-gemm_blk_tile_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, Epi epi, int M,
-                     int N, int K, int tiles_m, int tiles_n) {
-  extern __shared__ __align__(16) int8_t smem[];
-  asm volatile("" : "+s"(tiles_m) : "s"(A), "s"(W));
-  constexpr int TM = WGM * MB * 32;
-  int tm, tn;
-  tile_of(blockIdx.x, tiles_m * tiles_n, tiles_m, tiles_n, tm, tn);
-  tile_gemm<Epi, WGM, WGN, MB, NB, NST, false, true>(A, W, epi, tm * TM, M, N, K, tn, smem);
-}
 
 // A product of one to four rows that makes its rows itself (ln_step.h): 16 columns per workgroup,
 // a quarter of K per wavefront (D slices), its weights requested right behind the inputs of
@@ -86,73 +67,6 @@ ln_gemm_kernel(const LnStep ln, const int8_t* __restrict__ W, Epi epi, int M, in
 
 namespace {
 
-template <auto Kern>
-int raise_lds(size_t smem) {
-  static std::mutex mu;
-  static unsigned long long done = 0;  // bit per device index
-  int dev = 0;
-  if (int rc = lsh_check_hip(hipGetDevice(&dev), "hipGetDevice(gemm_blk)")) return rc;
-  if (dev < 0 || dev >= 64) return lsh_fail(LSH_ERR_UNSUPPORTED, "blocked gemm: device index out of range");
-  std::lock_guard<std::mutex> lock(mu);
-  if (!(done >> dev & 1ull)) {
-    if (smem > 64 * 1024)
-      if (int rc = lsh_check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(Kern),
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem),
-                                 "hipFuncSetAttribute(gemm_blk)"))
-        return rc;
-    done |= 1ull << dev;
-  }
-  return LSH_OK;
-}
-
-template <auto Kern, typename... Args>
-int launch_blk(dim3 grid, int threads, size_t smem, hipStream_t s, Args... args) {
-  if (int rc = raise_lds<Kern>(smem)) return rc;
-  hipEvent_t e0, e1;
-  if (gemm_take_timing_events(&e0, &e1))
-    hipExtLaunchKernelGGL(Kern, grid, dim3(threads), (unsigned)smem, s, e0, e1, 0, args...);
-  else
-    Kern<<<grid, threads, smem, s>>>(args...);
-  return lsh_check_launch("blocked gemm");
-}
-
-template <typename Tr, typename Epi, int MB, int NB>
-int launch_kw(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K, int ksplit,
-              hipStream_t s) {
-  const int tm = (M + 16 * MB - 1) / (16 * MB), tn = (N + 16 * NB - 1) / (16 * NB);
-  const dim3 grid(tm * tn, ksplit);
-  constexpr size_t smem = kw_lds_bytes<Epi, MB, NB>();
-  const int slices = K / 64 / ksplit;
-#define LSH_KW(D)                                                                                   \
-  return launch_blk<gemm_kw_kernel<Tr, Epi, MB, NB, D>>(grid, 256, smem, s, A, W, epi, M, N, K, slices, tm, tn)
-  if (slices % 16 == 0) LSH_KW(4);
-  if (slices % 12 == 0) LSH_KW(3);
-  if (slices % 8 == 0) LSH_KW(2);
-  LSH_KW(1);
-#undef LSH_KW
-}
-
-// The LDS tile kernel: 8 wavefronts for the tall tiles, 4 for 128 x 128 and 128 x 64 (two or three
-// workgroups then share a compute unit and one's epilogue runs under the other's K loop).
-constexpr TileCost kLdsCost[] = {{128, 64, 2.5f, 2.45f, 0.2f, 2.6f, 0.6f},
-                                 {128, 128, 2.9f, 3.6f, 0.6f, 4.9f, 0.9f},
-                                 {256, 128, 3.1f, 5.4f, 1.5f, 9.0f, 1.3f},
-                                 {256, 192, 3.6f, 7.1f, 3.0f, 9.5f, 1.7f},
-                                 {256, 256, 4.1f, 9.2f, 4.0f, 12.0f, 2.4f}};
-struct LdsTile {
-  int tm = 0, tn = 0;
-  float us = 0;
-};
-LdsTile choose_lds_tile(int M, int N, int K, int cus, bool table) {
-  LdsTile best;
-  if (K % kBK != 0 || K / kBK < 3 || N % 16 != 0) return best;
-  for (const auto& c : kLdsCost) {
-    const float us = tile_us(c, M, N, K, 1, cus, table);
-    if (best.tm == 0 || us < best.us) best = LdsTile{c.tm, c.tn, us};
-  }
-  return best;
-}
-
 template <typename Epi, bool I32, int ROWS>
 int launch_ln_rows(const LnStep& ln, const int8_t* W, Epi epi, int M, int N, int K, hipStream_t s) {
   const dim3 grid((N + 15) / 16);
@@ -180,56 +94,6 @@ int launch_ln_gemm(const LnStep& ln, const int8_t* W, Epi epi, int M, int N, int
   if (M == 1) return launch_ln_rows<Epi, I32, 1>(ln, W, epi, M, N, K, s);
   if (M == 2) return launch_ln_rows<Epi, I32, 2>(ln, W, epi, M, N, K, s);
   return launch_ln_rows<Epi, I32, 4>(ln, W, epi, M, N, K, s);
-}
-
-template <typename Tr, typename Epi, bool TILES>
-int dispatch_blk(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K, hipStream_t s,
-                 int ksplit = 1) {
-  if (M <= 0 || N <= 0 || K <= 0 || !A || !W)
-    return lsh_fail(LSH_ERR_INVALID, "blocked gemm: bad arguments");
-  if (K % 64 != 0 || N % 4 != 0)
-    return lsh_fail(LSH_ERR_UNSUPPORTED, "blocked gemm: needs K bytes % 64 == 0 and N % 4 == 0");
-  if (((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W)) & 15u) != 0 || !epi.aligned())
-    return lsh_fail(LSH_ERR_INVALID, "blocked gemm: operands must be 16-byte aligned");
-  const unsigned long long lim = 0xffffffffull;
-  if ((unsigned long long)(M + 15) / 16 * 16 * K >= lim || (unsigned long long)(N + 15) / 16 * 16 * K >= lim ||
-      (long)((M + 15) / 16) * ((N + 15) / 16) >= (1L << 24))
-    return lsh_fail(LSH_ERR_UNSUPPORTED, "blocked gemm: operand or output too large");
-  if (ksplit < 1 || K % (64 * ksplit) != 0)
-    return lsh_fail(LSH_ERR_INVALID, "blocked gemm: K does not split into whole 64-byte slices");
-  const int cus = cu_count();
-  const KwTile kw = kw_choose_tile(M, N, K / ksplit, ksplit, cus, Epi::kTable);
-  if constexpr (TILES) {
-    if (ksplit == 1) {
-      const LdsTile t = choose_lds_tile(M, N, K, cus, Epi::kTable);
-      if (t.tm != 0 && t.us < kw.us) {
-        const int tm = (M + t.tm - 1) / t.tm, tn = (N + t.tn - 1) / t.tn;
-        const dim3 grid(tm * tn);
-        if (t.tn == 256)
-          return launch_blk<gemm_blk_tile_kernel<Epi, 2, 4, 4, 2, 2>>(grid, 512, 2 * 512 * kBK, s, A, W, epi, M, N,
-                                                                      K, tm, tn);
-        if (t.tn == 192)
-          return launch_blk<gemm_blk_tile_kernel<Epi, 4, 2, 2, 3, 2>>(grid, 512, 2 * 448 * kBK, s, A, W, epi, M, N,
-                                                                      K, tm, tn);
-        if (t.tm == 256)
-          return launch_blk<gemm_blk_tile_kernel<Epi, 4, 2, 2, 2, 3>>(grid, 512, 3 * 384 * kBK, s, A, W, epi, M, N,
-                                                                      K, tm, tn);
-        if (t.tn == 128)
-          return launch_blk<gemm_blk_tile_kernel<Epi, 2, 2, 2, 2, 2>>(grid, 256, 2 * 256 * kBK, s, A, W, epi, M, N,
-                                                                      K, tm, tn);
-        // long K loops: a third stage instead of a third workgroup per compute unit
-        if (K >= 2048)
-          return launch_blk<gemm_blk_tile_kernel<Epi, 4, 1, 1, 2, 3>>(grid, 256, 3 * 192 * kBK, s, A, W, epi, M, N,
-                                                                      K, tm, tn);
-        return launch_blk<gemm_blk_tile_kernel<Epi, 4, 1, 1, 2, 2>>(grid, 256, 2 * 192 * kBK, s, A, W, epi, M, N, K,
-                                                                    tm, tn);
-      }
-    }
-  }
-  if (kw.mb == 1) return launch_kw<Tr, Epi, 1, 1>(A, W, epi, M, N, K, ksplit, s);
-  if (kw.mb == 2) return launch_kw<Tr, Epi, 2, 2>(A, W, epi, M, N, K, ksplit, s);
-  if (kw.nb == 2) return launch_kw<Tr, Epi, 4, 2>(A, W, epi, M, N, K, ksplit, s);
-  return launch_kw<Tr, Epi, 4, 4>(A, W, epi, M, N, K, ksplit, s);
 }
 
 }  // namespace

@@ -29,12 +29,14 @@ namespace lsh {
 typedef float v4f __attribute__((ext_vector_type(4)));
 
 struct KwI8 {
+  typedef v16i Acc16;  // of the LDS tile loop: sixteen neighbouring columns
   typedef v4i Acc;  // four neighbouring columns of one row
   static __device__ __forceinline__ Acc mma(const v4i& w, const v4i& a, const Acc& c) {
     return __builtin_amdgcn_mfma_i32_16x16x64_i8(w, a, c, 0, 0, 0);
   }
 };
 struct KwF16 {
+  typedef v16f Acc16;
   typedef v4f Acc;
   static __device__ __forceinline__ Acc mma(const v4i& w, const v4i& a, const Acc& c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, w),
@@ -44,6 +46,9 @@ struct KwF16 {
 
 // Epilogues: Col column(n, N) is what the columns n .. n + 3 need (requested before the first
 // product; n is clamped to N - 4), store4(m, n, N, col, acc) finishes four elements of row m.
+// kClips (optional): the epilogue needs values of device memory for all of its elements.  request()
+// loads them ahead of the first product and nothing waits for them there; finish(raw) returns
+// the epilogue that has them.
 // kTable: 256 bytes per column are staged in LDS from table() and handed to store4 as `tab`, the
 // table of column n (kw_table_index says where a code is).
 // kBlockedOut: the output is a blocked int8 matrix; the lanes of a wavefront then take the 256
@@ -93,6 +98,7 @@ gemm_kw_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, Epi e
   constexpr int PER = (16 * MB + ROWS - 1) / ROWS;
   const int n = n0 + 4 * quad;
   const typename Epi::Col col = epi.column(min(n, N - 4), N);
+  const auto raw = epi_request(epi);
 
   // this wavefront's slices
   const int first = (int)blockIdx.y * slices;
@@ -158,6 +164,7 @@ gemm_kw_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, Epi e
   if constexpr (Epi::kTable) wait_vmcnt<0>();
   __syncthreads();
   if (n >= N) return;
+  const auto fin = epi_finish(epi, raw);
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
     const int row = row0 + j * ROWS;
@@ -167,8 +174,84 @@ gemm_kw_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, Epi e
       const Acc c = (red[cell] + red[MB * NB * 68 + cell]) +
                     (red[2 * MB * NB * 68 + cell] + red[3 * MB * NB * 68 + cell]);
       const int mo = m + (int)blockIdx.y * M;
-      if constexpr (Epi::kTable) epi.store4(mo, n, N, col, c, tab + 4 * quad * 256);
-      else epi.store4(mo, n, N, col, c);
+      if constexpr (Epi::kTable) fin.store4(mo, n, N, col, c, tab + 4 * quad * 256);
+      else fin.store4(mo, n, N, col, c);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------
+// The same without the split of K, for fp16: every output is one chain of products in ascending K.
+// v_mfma_f32_16x16x32_f16 adds its 32 products in the order in which two v_mfma_f32_32x32x16_f16
+// do (checked bit for bit over random operands of several ranges), so this kernel, the LDS tile
+// loop and the row-major kernel all give the same bits; partial sums of K ranges do not, and in a
+// stack of quantised layers one unit of fp16 in a few outputs grows into percents of the result.
+// WM x WN wavefronts side by side, MB x NB blocks of 16 x 16 each; D slices in flight (slices % D
+// == 0); fragments of the wavefronts of a workgroup meet in the vector cache.
+// ---------------------------------------------------------------------------------
+template <typename Tr, typename Epi, int WM, int WN, int MB, int NB, int D>
+__global__ void __launch_bounds__(64 * WM * WN)
+gemm_seq_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, Epi epi, int M, int N, int K,
+                int slices, int tiles_m, int tiles_n) {
+  typedef typename Tr::Acc Acc;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l16 = lane & 15, kq = lane >> 4;
+  int tile_m, tile_n;
+  tile_of((int)blockIdx.x, (int)gridDim.x, tiles_m, tiles_n, tile_m, tile_n);
+  const int m0 = (tile_m * WM + wave / WN) * (16 * MB), n0 = (tile_n * WN + wave % WN) * (16 * NB);
+  if (m0 >= M || n0 >= N) return;  // (no barriers)
+  typename Epi::Col col[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) col[b] = epi.column(min(n0 + 16 * b + 4 * kq, N - 4), N);
+  uint32_t a_off[MB], w_off[NB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+    a_off[i] = (uint32_t)min(m0 + 16 * i, (M - 1) & ~15) * (uint32_t)K + lane * 16;
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+    w_off[b] = (uint32_t)min(n0 + 16 * b, (N - 1) & ~15) * (uint32_t)K + lane * 16;
+  v4i fa[D][MB], fw[D][NB];
+  auto load = [&](int u, int s) {
+    const int8_t* a = A + s * 1024;
+    const int8_t* w = W + s * 1024;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) fw[u][b] = *reinterpret_cast<const v4i*>(w + w_off[b]);
+#pragma unroll
+    for (int i = 0; i < MB; ++i) fa[u][i] = *reinterpret_cast<const v4i*>(a + a_off[i]);
+  };
+  Acc acc[MB][NB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int b = 0; b < NB; ++b) acc[i][b] = (Acc)0;
+  auto mma = [&](int u) {
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int b = 0; b < NB; ++b) acc[i][b] = Tr::mma(fw[u][b], fa[u][i], acc[i][b]);
+  };
+#pragma unroll
+  for (int u = 0; u < D; ++u) load(u, u);
+  __builtin_amdgcn_sched_barrier(0);
+  for (int s = D; s < slices; s += D) {
+#pragma unroll
+    for (int u = 0; u < D; ++u) {
+      mma(u);
+      load(u, s + u);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < D; ++u) mma(u);
+#pragma unroll
+  for (int i = 0; i < MB; ++i) {
+    const int m = m0 + 16 * i + l16;
+    if (m >= M) continue;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const int n = n0 + 16 * b + 4 * kq;
+      if (n < N) epi.store4(m, n, N, col[b], acc[i][b]);
     }
   }
 }

@@ -223,16 +223,41 @@ __device__ __forceinline__ void tile_of(int t, int nblk, int tiles_m, int tiles_
 // 16-byte aligned.  A_FROM_L2: the rows of A were written by other compute units of this XCD
 // during this launch (read past the vector cache).  BLOCKED: both operands in the blocked layout.
 // ---------------------------------------------------------------------------------
+template <typename Epi, typename = void>
+struct EpiHasClips : std::false_type {};
+template <typename Epi>
+struct EpiHasClips<Epi, std::enable_if_t<Epi::kClips>> : std::true_type {};
+struct EpiNoRaw {};
+template <typename Epi>
+__device__ __forceinline__ auto epi_request(const Epi& e) {
+  if constexpr (EpiHasClips<Epi>::value) return e.request();
+  else return EpiNoRaw{};
+}
+template <typename Epi, typename Raw>
+__device__ __forceinline__ Epi epi_finish(const Epi& e, const Raw& raw) {
+  if constexpr (EpiHasClips<Epi>::value) return e.finish(raw);
+  else return e;
+}
+
+// 32 x 32 products over 32 bytes of K: int8, or fp16 (the lanes hold the operands alike)
+__device__ __forceinline__ v16i mma32(const v4i& w, const v4i& a, const v16i& c) {
+  return __builtin_amdgcn_mfma_i32_32x32x32_i8(w, a, c, 0, 0, 0);
+}
+__device__ __forceinline__ v16f mma32(const v4i& w, const v4i& a, const v16f& c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, w), __builtin_bit_cast(v8h, a),
+                                                c, 0, 0, 0);
+}
 template <typename Epi, int NST>
 constexpr int tile_gemm_barriers(int nk) {
   return nk + (is_lut<Epi> ? 1 : 0);
 }
 
 template <typename Epi, int WGM, int WGN, int MB, int NB, int NST, bool A_FROM_L2 = false,
-          bool BLOCKED = false>
+          bool BLOCKED = false, typename Acc16 = v16i>
 __device__ __forceinline__ void tile_gemm(const int8_t* __restrict__ A,
-                                          const int8_t* __restrict__ W, const Epi& epi, int row0,
+                                          const int8_t* __restrict__ W, const Epi& epi_arg, int row0,
                                           int row_end, int N, int K, int tn, int8_t* smem) {
+  const auto raw = epi_request(epi_arg);
   constexpr bool LUT = is_lut<Epi>;
   // The operand order of the MFMA decides what a lane's 16 accumulators are: weight rows first,
   // 16 adjacent columns of one output row (one 16-byte store of int8 codes); activations first,
@@ -333,19 +358,17 @@ __device__ __forceinline__ void tile_gemm(const int8_t* __restrict__ A,
     for (int j = 0; j < NB; ++j)
       f.w[j] = *reinterpret_cast<const v4i*>(stage + slice_at(w_base[j], ks));
   };
-  v16i acc[MB][NB];
+  Acc16 acc[MB][NB];
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
-    for (int j = 0; j < NB; ++j) acc[i][j] = (v16i)0;
+    for (int j = 0; j < NB; ++j) acc[i][j] = (Acc16)0;
   auto mma = [&](const Frag& f) {
 #pragma unroll
     for (int i = 0; i < MB; ++i)
 #pragma unroll
       for (int j = 0; j < NB; ++j)
-        acc[i][j] = ROWS_IN_REGS
-                        ? __builtin_amdgcn_mfma_i32_32x32x32_i8(f.a[i], f.w[j], acc[i][j], 0, 0, 0)
-                        : __builtin_amdgcn_mfma_i32_32x32x32_i8(f.w[j], f.a[i], acc[i][j], 0, 0, 0);
+        acc[i][j] = ROWS_IN_REGS ? mma32(f.a[i], f.w[j], acc[i][j]) : mma32(f.w[j], f.a[i], acc[i][j]);
   };
   // issue order of one slice: an LDS read of the next slice after each of the first MFMAs
   auto pattern = [&]() {
@@ -404,7 +427,7 @@ __device__ __forceinline__ void tile_gemm(const int8_t* __restrict__ A,
       for (int i = 0; i < NTAB; ++i) {
         const int q = wave + NWV * i;
         const long off = min(first + q * 1024 + lane * 16, last);  // rows beyond N: never stored
-        dma1(reinterpret_cast<const int8_t*>(epi_lut(epi)), (uint32_t)off,
+        dma1(reinterpret_cast<const int8_t*>(epi_lut(epi_arg)), (uint32_t)off,
              lds0 + slot * STAGE + q * 1024);
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -420,6 +443,7 @@ __device__ __forceinline__ void tile_gemm(const int8_t* __restrict__ A,
     wait_vmcnt<0>();
     __builtin_amdgcn_s_barrier();
   }
+  const Epi epi = epi_finish(epi_arg, raw);
   if constexpr (ROWS_IN_REGS) {
     // int32 output: a lane holds column sigma(l32) of its block and the rows 8 (k / 4) + 4 g +
     // k % 4 in register k, so a store instruction writes two whole 128-byte lines (32 lanes, 32

@@ -1,0 +1,315 @@
+// What a quantised layer needs ahead of and between its products (layer_gemm.hip), in as few
+// launches as there are dependencies: one that prepares everything the forward pass starts from,
+// and the layer norm between two products.
+#include "layer_device.h"
+#include "ls_launch.h"
+
+#include <algorithm>
+
+namespace lsh {
+
+namespace {
+
+// ---- one launch for all of a layer's preparations -------------------------------------------
+// The parameters belong to the caller and may have changed since the last call, so every forward
+// pass quantises the weights (2 bytes read and 1 written per parameter: 10 MB for a
+// Transformer-base layer).  As one launch per matrix that was 4 us each, six to nine times per
+// layer; the sections below -- weights, the input, the mask, the copy of a decoding step's caches
+// -- do not depend on one another, so they are ranges of workgroups of one grid and the
+// launch lasts as long as the memory takes: Transformer-base encoder layer 4.9 us in all.
+//
+// Sections that write blocked matrices work on units of 16 rows x 512 columns: a wavefront reads
+// 128-byte pieces of 16 rows and writes 1 KB, the 16 rows x 64 bytes block; what a unit reads is
+// requested before any of it is converted.
+constexpr int kUnitK = 512;
+
+__device__ __forceinline__ const __half* unit_row(const LayerPrepSection& s, int row) {
+  const int r = min(row, s.rows - 1);
+  if (s.n1 == 1) return s.src + (long)r * s.stride0;
+  return s.src + (long)(r / s.n1) * s.stride0 + (long)(r % s.n1) * s.stride1;
+}
+
+__device__ __forceinline__ void unit_codes(const LayerPrepSection& s, int block) {
+  const int per_row = (s.K + kUnitK - 1) / kUnitK;
+  const int rb = block / per_row, kc = block - rb * per_row;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int row = rb * 16 + (lane & 15);
+  const int k0 = kc * kUnitK + wave * 64 + (lane >> 4) * 16;
+  const __half* src = unit_row(s, row);
+  half8_t x[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      x[i][h] = *reinterpret_cast<const half8_t*>(src + min(k0 + i * 256 + h * 8, s.K - 8));  // K % 8 == 0
+  const Quantiser of = Quantiser::of(cm(s.cmax));
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int k = k0 + i * 256;
+    if (k >= s.k_pad) break;
+    uint32_t w[4];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      int q[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) q[e] = of.code(__half2float(x[i][h].v[e]));
+      const bool on = row < s.rows && k + h * 8 < s.K;
+      w[2 * h] = on ? pack4_i8(q[0], q[1], q[2], q[3]) : 0u;
+      w[2 * h + 1] = on ? pack4_i8(q[4], q[5], q[6], q[7]) : 0u;
+    }
+    *reinterpret_cast<uint4*>(static_cast<int8_t*>(s.dst) + blocked_offset(row, k, s.k_pad)) =
+        make_uint4(w[0], w[1], w[2], w[3]);
+  }
+}
+
+// fp16 -> blocked fp16 (64 bytes of K are 32 halfs), fake-quantised where `cmax` is set
+__device__ __forceinline__ void unit_halfs(const LayerPrepSection& s, int block) {
+  const int per_row = (s.K + kUnitK - 1) / kUnitK;
+  const int rb = block / per_row, kc = block - rb * per_row;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int row = rb * 16 + (lane & 15);
+  const int k0 = kc * kUnitK + wave * 32 + (lane >> 4) * 8;
+  const __half* src = unit_row(s, row);
+  half8_t x[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) x[i] = *reinterpret_cast<const half8_t*>(src + min(k0 + i * 128, s.K - 8));
+  const Quantiser of = Quantiser::of(s.cmax ? cm(s.cmax) : 1.f);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int k = k0 + i * 128;
+    if (k >= s.k_pad) break;
+    if (s.cmax) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[i].v[e] = __float2half_rn(of.fake(__half2float(x[i].v[e])));
+    }
+    if (row >= s.rows || k >= s.K) x[i] = half8_t{};
+    *reinterpret_cast<half8_t*>(static_cast<char*>(s.dst) + blocked_offset(row, 2 * k, 2 * s.k_pad)) = x[i];
+  }
+}
+
+// Layer norm of one row by a wavefront (opb_layer_norm: var = E[x^2] - E[x]^2 + 1e-8), the row kept
+// in registers where it is at most 512 IT elements; the codes of the fp16 result, blocked.
+template <int IT>
+__device__ __forceinline__ void ln_row(const __half* inp, __half* out, int8_t* codes, const __half* gamma,
+                                       const __half* beta, const __half* cmax, int row, int hidden, int k_pad) {
+  const int lane = threadIdx.x & 63;
+  const long base = (long)row * hidden;
+  half8_t raw[IT], g[IT], b[IT];
+#pragma unroll
+  for (int it = 0; it < IT; ++it) {
+    const int e = min(lane * 8 + it * 512, hidden - 8);
+    raw[it] = *reinterpret_cast<const half8_t*>(inp + base + e);
+    g[it] = *reinterpret_cast<const half8_t*>(gamma + e);
+    b[it] = *reinterpret_cast<const half8_t*>(beta + e);
+  }
+  const Quantiser of = Quantiser::of(codes ? cm(cmax) : 1.f);
+  float s = 0.f, s2 = 0.f;
+#pragma unroll
+  for (int it = 0; it < IT; ++it)
+    if (lane * 8 + it * 512 < hidden) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const float x = __half2float(raw[it].v[k]);
+        s += x;
+        s2 += x * x;
+      }
+    }
+  const float mean = wave_sum(s) / (float)hidden;
+  const float var = wave_sum(s2) / (float)hidden - mean * mean + kLnEps;
+  const float rstd = rsqrtf(var);
+#pragma unroll
+  for (int it = 0; it < IT; ++it) {
+    const int e = lane * 8 + it * 512;
+    if (e >= hidden) continue;
+    half8_t o;
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      o.v[k] = __float2half_rn((__half2float(raw[it].v[k]) - mean) * rstd * __half2float(g[it].v[k]) +
+                               __half2float(b[it].v[k]));
+    if (out) *reinterpret_cast<half8_t*>(out + base + e) = o;
+    if (codes) {
+      int q[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) q[k] = of.code(__half2float(o.v[k]));
+      *reinterpret_cast<uint2*>(codes + blocked_offset(row, e, k_pad)) =
+          make_uint2(pack4_i8(q[0], q[1], q[2], q[3]), pack4_i8(q[4], q[5], q[6], q[7]));
+    }
+  }
+}
+__device__ __forceinline__ void ln_row_any(const __half* inp, __half* out, int8_t* codes, const __half* gamma,
+                                           const __half* beta, const __half* cmax, int row, int hidden,
+                                           int k_pad) {
+  if (hidden <= 512) ln_row<1>(inp, out, codes, gamma, beta, cmax, row, hidden, k_pad);
+  else if (hidden <= 1024) ln_row<2>(inp, out, codes, gamma, beta, cmax, row, hidden, k_pad);
+  else if (hidden <= 2048) ln_row<4>(inp, out, codes, gamma, beta, cmax, row, hidden, k_pad);
+  else ln_row<8>(inp, out, codes, gamma, beta, cmax, row, hidden, k_pad);
+}
+
+// the additive fp16 mask of the layers, half(value * -1e8), from whatever the caller's mask is made of
+__device__ __forceinline__ float mask_value(const void* p, int kind, long i) {
+  switch (kind) {
+    case kMaskF32: return static_cast<const float*>(p)[i];
+    case kMaskF16: return __half2float(static_cast<const __half*>(p)[i]);
+    case kMaskU8: return (float)static_cast<const unsigned char*>(p)[i];
+    case kMaskI32: return (float)static_cast<const int*>(p)[i];
+    default: return (float)static_cast<const long long*>(p)[i];
+  }
+}
+
+__global__ void __launch_bounds__(256)
+layer_prep_kernel(const LayerPrepArgs a) {
+  // the section that the workgroup belongs to: the first blocks are read together and compared, a
+  // walk would be as many trips to the kernel arguments
+  int i = 0, first = 0;
+#pragma unroll
+  for (int j = 1; j < kLayerPrepMost; ++j)
+    if ((int)blockIdx.x >= a.first[j]) {
+      i = j;
+      first = a.first[j];
+    }
+  const int block = (int)blockIdx.x - first;
+  const LayerPrepSection& s = a.s[i];
+  switch (s.kind) {
+    case kPrepCodes: unit_codes(s, block); break;
+    case kPrepHalfs: unit_halfs(s, block); break;
+    case kPrepNorm: {
+      const int row = block * 4 + (int)(threadIdx.x >> 6);
+      if (row < s.rows)
+        ln_row_any(s.src, nullptr, static_cast<int8_t*>(s.dst), s.gamma, s.beta, s.cmax, row, s.K, s.k_pad);
+      break;
+    }
+    case kPrepMask: {
+      const long j = (long)block * 256 + threadIdx.x;
+      if (j < s.rows)
+        static_cast<__half*>(s.dst)[j] = __float2half_rn(mask_value(s.src, s.n1, j) * -1e8f);
+      break;
+    }
+    default: {  // kPrepGrow: [rows, K] -> the first K of rows of stride1 elements, 2048 elements per block
+      const long j = ((long)block * 256 + threadIdx.x) * 8;
+      if (j < (long)s.rows * s.K) {
+        const long r = j / s.K, c = j - r * s.K;
+        *reinterpret_cast<half8_t*>(static_cast<__half*>(s.dst) + r * s.stride1 + c) =
+            *reinterpret_cast<const half8_t*>(s.src + j);
+      }
+    }
+  }
+}
+
+__global__ void __launch_bounds__(256)
+layer_norm_codes_kernel(const __half* inp, __half* out, int8_t* codes, const __half* __restrict__ gamma,
+                        const __half* __restrict__ beta, const __half* __restrict__ cmax, int rows,
+                        int hidden, int k_pad) {
+  const int row = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
+  if (row < rows) ln_row_any(inp, out, codes, gamma, beta, cmax, row, hidden, k_pad);
+}
+
+}  // namespace
+
+int LayerPrep::add(const LayerPrepSection& s) {
+  if (_args.n >= kLayerPrepMost) return lsh_fail(LSH_ERR_UNSUPPORTED, "layer_prep: too many sections");
+  _args.s[_args.n++] = s;
+  return LSH_OK;
+}
+
+static int prep_units(int rows, int K) { return (rows + 15) / 16 * ((K + kUnitK - 1) / kUnitK); }
+
+int LayerPrep::codes(const __half* src, int8_t* dst, const __half* cmax, int rows, int K, int k_pad) {
+  if (!src || !dst || !cmax || rows <= 0 || K <= 0 || K % 8 != 0 || k_pad < K || k_pad % 64 != 0)
+    return lsh_fail(LSH_ERR_INVALID, "layer_prep: bad matrix");
+  LayerPrepSection s{};
+  s.kind = kPrepCodes;
+  s.blocks = prep_units(rows, K);
+  s.src = src;
+  s.dst = dst;
+  s.cmax = cmax;
+  s.rows = rows;
+  s.K = K;
+  s.k_pad = k_pad;
+  s.n1 = 1;
+  s.stride0 = K;
+  return add(s);
+}
+int LayerPrep::halfs(const __half* src, __half* dst, const __half* cmax, int rows, int K, int k_pad, int n1,
+                     long stride0, long stride1) {
+  if (!src || !dst || rows <= 0 || K <= 0 || K % 8 != 0 || k_pad < K || k_pad % 32 != 0 || n1 <= 0)
+    return lsh_fail(LSH_ERR_INVALID, "layer_prep: bad fp16 matrix");
+  LayerPrepSection s{};
+  s.kind = kPrepHalfs;
+  s.blocks = prep_units(rows, K);
+  s.src = src;
+  s.dst = dst;
+  s.cmax = cmax;
+  s.rows = rows;
+  s.K = K;
+  s.k_pad = k_pad;
+  s.n1 = n1;
+  s.stride0 = stride0;
+  s.stride1 = stride1;
+  return add(s);
+}
+int LayerPrep::norm(const __half* src, int8_t* dst, const __half* gamma, const __half* beta,
+                    const __half* cmax, int rows, int hidden, int k_pad) {
+  if (!src || !dst || !gamma || !beta || !cmax || rows <= 0 || hidden <= 0 || hidden % 8 != 0 || hidden > 4096)
+    return lsh_fail(LSH_ERR_INVALID, "layer_prep: bad layer norm");
+  LayerPrepSection s{};
+  s.kind = kPrepNorm;
+  s.blocks = (rows + 3) / 4;
+  s.src = src;
+  s.dst = dst;
+  s.gamma = gamma;
+  s.beta = beta;
+  s.cmax = cmax;
+  s.rows = rows;
+  s.K = hidden;
+  s.k_pad = k_pad;
+  return add(s);
+}
+int LayerPrep::mask(const void* src, int kind, __half* dst, int count) {
+  if (!src || !dst || count <= 0 || kind < kMaskF32 || kind > kMaskI64)
+    return lsh_fail(LSH_ERR_INVALID, "layer_prep: bad mask");
+  LayerPrepSection s{};
+  s.kind = kPrepMask;
+  s.blocks = (count + 255) / 256;
+  s.src = static_cast<const __half*>(src);
+  s.dst = dst;
+  s.rows = count;
+  s.n1 = kind;
+  return add(s);
+}
+int LayerPrep::grow(const __half* src, __half* dst, int rows, int K, long dst_stride) {
+  if (!src || !dst || rows <= 0 || K <= 0 || K % 8 != 0 || dst_stride < K || dst_stride % 8 != 0)
+    return lsh_fail(LSH_ERR_INVALID, "layer_prep: bad cache copy");
+  LayerPrepSection s{};
+  s.kind = kPrepGrow;
+  s.blocks = (int)(((long)rows * K / 8 + 255) / 256);
+  s.src = src;
+  s.dst = dst;
+  s.rows = rows;
+  s.K = K;
+  s.stride1 = dst_stride;
+  return add(s);
+}
+int LayerPrep::launch(hipStream_t s) const {
+  LayerPrepArgs args = _args;
+  long blocks = 0;
+  for (int i = 0; i < kLayerPrepMost; ++i) {
+    args.first[i] = i < args.n ? (int)std::min(blocks, 0x7fffffffL) : 0x7fffffff;
+    if (i < args.n) blocks += args.s[i].blocks;
+  }
+  if (blocks <= 0) return LSH_OK;
+  if (blocks >= (1L << 30)) return lsh_fail(LSH_ERR_UNSUPPORTED, "layer_prep: too many workgroups");
+  layer_prep_kernel<<<(unsigned)blocks, 256, 0, s>>>(args);
+  return lsh_check_launch("layer_prep_kernel");
+}
+
+int layer_norm_codes(const __half* inp, __half* out, int8_t* codes, const __half* gamma, const __half* beta,
+                     const __half* cmax, int rows, int hidden, int k_pad, hipStream_t s) {
+  if (!inp || (!out && !codes) || !gamma || !beta || (codes && !cmax) || rows <= 0 || hidden <= 0 ||
+      hidden % 8 != 0 || hidden > 4096)
+    return lsh_fail(LSH_ERR_INVALID, "layer_norm_codes: bad arguments");
+  layer_norm_codes_kernel<<<(rows + 3) / 4, 256, 0, s>>>(inp, out, codes, gamma, beta, cmax, rows, hidden,
+                                                         k_pad);
+  return lsh_check_launch("layer_norm_codes_kernel");
+}
+
+}  // namespace lsh

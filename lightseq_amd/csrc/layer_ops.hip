@@ -7,16 +7,12 @@
 // layer's parameter blob), so no kernel needs a host copy of them.  Row kernels
 // (layer norm, softmax) give one 64-lane wavefront to a row and reduce with cross-lane
 // shuffles.  Dropout ratios must be 0 (inference); the mask outputs are still written.
-#include "ls_device.h"
+#include "layer_device.h"
 #include "ls_launch.h"
 
 namespace lsh {
 
 namespace {
-
-constexpr float kQ = 127.0f;               // kernels.h:20
-constexpr float kLnEps = 1e-8f;            // normalize_kernels.cu:12
-constexpr float kSoftmaxEps = 1e-8f;       // softmax_kernels.cu:11
 
 template <typename T>
 struct Vec {
@@ -77,57 +73,6 @@ __device__ __forceinline__ void or_mask(uint8_t* p, long i, const int (&m)[N]) {
     w |= (uint32_t)m[0] | ((uint32_t)m[1] << 8) | ((uint32_t)m[2] << 16) | ((uint32_t)m[3] << 24);
     *reinterpret_cast<uint32_t*>(p + i) = w;
   }
-}
-
-// kernels.h:425-435
-__device__ __forceinline__ int clip_mask_bits(float v, float cmax, int bit, bool symmetry = true) {
-  if (v >= cmax) return 1 << (bit - 1);
-  if (symmetry && v <= -cmax) return 1 << bit;
-  return 0;
-}
-// kernels.h:463-471
-__device__ __forceinline__ int quantize_b(float x, float cmax, int& mask, int bit) {
-  mask = clip_mask_bits(x, cmax, bit);
-  const float scale = cmax / kQ;
-  const float q = floorf(x / scale + 0.5f);
-  return (int)fminf(fmaxf(q, -kQ), kQ);
-}
-// kernels.h:473-488
-__device__ __forceinline__ float fake_quantize_b(float x, float cmax, int& mask, int bit,
-                                                 bool symmetry) {
-  mask = clip_mask_bits(x, cmax, bit, symmetry);
-  float scale = cmax / kQ;
-  if (!symmetry) scale /= 2;
-  float f = x / scale;
-  if (!symmetry) f -= kQ;
-  float q = fminf(fmaxf(floorf(f + 0.5f), -kQ), kQ);
-  return symmetry ? q * scale : (q + kQ) * scale;
-}
-// kernels.h:497-501
-__device__ __forceinline__ float dequantize_b(int q, float cmax) {
-  const float r = (float)q * (cmax / kQ);
-  return fminf(fmaxf(r, -cmax), cmax);
-}
-// dequantise + bias as T adds them (half: rounded operand, half add)
-template <typename T>
-__device__ __forceinline__ float deq_bias(int q, float cmax, float bias) {
-  return TT<T>::rnd(TT<T>::rnd(dequantize_b(q, cmax)) + bias);
-}
-template <typename T>
-__device__ __forceinline__ float cm(const T* p, int i = 0) {
-  return TT<T>::ld(p, i);
-}
-
-// dropout_kernels.cu:25-59: float GELU/ReLU for T=float, the half2 forms for T=half
-template <typename T, int ACT>
-__device__ __forceinline__ float act_b(float x) {
-  if (ACT == 1) return fmaxf(x, 0.f);
-  if (sizeof(T) == 2) {
-    const float p3 = TT<T>::rnd(x * TT<T>::rnd(x * x));
-    const float cdf = 0.5f * (1.0f + tanhf(0.7978845608028654f * (x + 0.044715f * p3)));
-    return TT<T>::rnd(x * TT<T>::rnd(cdf));
-  }
-  return gelu_tanh(x);
 }
 
 inline int grid_for(long nvec) { return (int)((nvec + 255) / 256); }

@@ -74,7 +74,51 @@ int ls_transformer_encoder_layer_fw_fp16(int layer_id, const void* input, const 
     layer->SetTrainingMode(training_mode != 0);
     layer->SetQuantMode(quant_mode != 0);
     layer->Forward(reinterpret_cast<const __half*>(input),
-                   reinterpret_cast<const __half*>(input_mask), reinterpret_cast<__half*>(output));
+                   input_mask, lsh::kMaskNone, reinterpret_cast<__half*>(output));
+  });
+}
+
+int ls_encoder_layer_call_fp16(int layer_id, const void* weights, const void* input, const void* padding_mask,
+                               int mask_type, void* output, int batch_size, int seq_len,
+                               int training_mode, int quant_mode, lsh_stream_t stream) {
+  return guarded([&] {
+    if (mask_type < lsh::kMaskNone || mask_type > lsh::kMaskI64)
+      throw std::runtime_error("encoder_layer_call: unknown mask type");
+    auto layer = find_layer(s_transformer_encoder_layers, layer_id, "Encoder layer");
+    Context::Instance().set_stream(reinterpret_cast<hipStream_t>(stream));
+    layer->assign_weight_ptr(reinterpret_cast<const __half*>(weights));
+    layer->set_cur_batch_shape(batch_size, seq_len);
+    layer->SetTrainingMode(training_mode != 0);
+    layer->SetQuantMode(quant_mode != 0);
+    layer->Forward(reinterpret_cast<const __half*>(input), padding_mask, mask_type,
+                   reinterpret_cast<__half*>(output));
+  });
+}
+
+int ls_decoder_layer_call_fp16(int layer_id, const void* weights, const void* dec_input,
+                               const void* enc_output, int64_t enc_stride_batch,
+                               int64_t enc_stride_seq, const void* padding_mask, int mask_type,
+                               void* dec_output, int batch_size, int trg_seq_len, int src_seq_len,
+                               int step, const void* new_k, const void* new_v, const void* old_k,
+                               const void* old_v, const void* encdec_kv, int training_mode,
+                               int quant_mode, lsh_stream_t stream) {
+  return guarded([&] {
+    if (mask_type < lsh::kMaskNone || mask_type > lsh::kMaskI64)
+      throw std::runtime_error("decoder_layer_call: unknown mask type");
+    auto layer = find_layer(s_transformer_decoder_layers, layer_id, "Decoder layer");
+    std::vector<__half*> cache;
+    if (step >= 0)
+      for (const void* p : {new_k, new_v, old_k, old_v, encdec_kv})
+        cache.push_back(const_cast<__half*>(reinterpret_cast<const __half*>(p)));
+    Context::Instance().set_stream(reinterpret_cast<hipStream_t>(stream));
+    layer->assign_weight_ptr(reinterpret_cast<const __half*>(weights));
+    layer->set_cur_batch_shape(batch_size, trg_seq_len, src_seq_len, step);
+    layer->SetTrainingMode(training_mode != 0);
+    layer->SetQuantMode(quant_mode != 0);
+    layer->Forward(reinterpret_cast<const __half*>(dec_input),
+                   reinterpret_cast<const __half*>(enc_output), (long)enc_stride_batch,
+                   (long)enc_stride_seq, padding_mask, mask_type, reinterpret_cast<__half*>(dec_output),
+                   cache);
   });
 }
 
@@ -111,8 +155,8 @@ int ls_transformer_decoder_layer_fw_fp16(int layer_id, const void* dec_input,
     layer->SetTrainingMode(training_mode != 0);
     layer->SetQuantMode(quant_mode != 0);
     layer->Forward(reinterpret_cast<const __half*>(dec_input),
-                   reinterpret_cast<const __half*>(enc_output),
-                   reinterpret_cast<const __half*>(enc_mask),
+                   reinterpret_cast<const __half*>(enc_output), (long)src_seq_len * layer->hidden_size(),
+                   layer->hidden_size(), enc_mask, lsh::kMaskNone,
                    reinterpret_cast<__half*>(dec_output), cache_vec);
   });
 }

@@ -1,8 +1,7 @@
 // Forward pass of the quantised decoder layer
-// (lightseq/csrc/layers/transformer_decoder_layer.cpp:91-547), built from this library's
-// operator kernels.  What differs from the reference's sequence is only where kernels are
-// fused: each attention core (scores, masked softmax, context, head merge) is one kernel, and
-// the int8 GEMMs read their scale from device memory in the epilogue.
+// (lightseq/csrc/layers/transformer_decoder_layer.cpp:91-547): one launch of preparations, six
+// products with the operators between them as epilogues, the two attention cores, the layer
+// norms between the blocks; layer 0 makes the cross-attention keys and values of the stack first.
 #include "transformer_decoder_layer.h"
 
 #include <algorithm>
@@ -19,7 +18,7 @@ int TransformerDecoderLayer<T>::_shared_nlayer = 0;
 template <typename T>
 DeviceBuffer<T> TransformerDecoderLayer<T>::_shared_encdec_kv;
 template <typename T>
-DeviceBuffer<T> TransformerDecoderLayer<T>::_shared_kv_tmp;
+DeviceBuffer<T> TransformerDecoderLayer<T>::_shared_enc_out;
 template <typename T>
 DeviceBuffer<T> TransformerDecoderLayer<T>::_shared_kv_weight;
 template <typename T>
@@ -37,7 +36,9 @@ TransformerDecoderLayer<T>::TransformerDecoderLayer(
       _heads(num_heads),
       _intermediate_size(intermediate_size),
       _is_pre_ln(pre_or_postLayerNorm),
-      _activation_fn(activation_fn) {
+      _activation_fn(activation_fn),
+      _kh((hidden_size + 63) & ~63),
+      _ki((intermediate_size + 63) & ~63) {
   (void)attn_prob_dropout_ratio;  // ratios only matter in training mode, which Forward rejects
   (void)activation_dropout_ratio;
   (void)hidden_output_dropout_ratio;
@@ -58,19 +59,20 @@ TransformerDecoderLayer<T>::TransformerDecoderLayer(
 
   const size_t tok = (size_t)max_batch_tokens, hs = (size_t)hidden_size,
                ims = (size_t)intermediate_size;
-  if (_is_pre_ln) _ln_out.alloc(tok * hs);
+  const size_t rows = (tok + 15) & ~(size_t)15;
   _qkv.alloc(3 * tok * hs);
-  _attn_o_inp.alloc(tok * hs);
   _encdec_inp.alloc(tok * hs);
-  _encdec_q.alloc(tok * hs);
   _ffn_inp.alloc(tok * hs);
-  _ff2_inp.alloc(tok * ims);
-  _fake_weight.alloc(hs * ims);
-  _vars.alloc(tok);
-  _qin.alloc(tok * std::max(hs, ims));
-  _qout.alloc(tok * std::max(3 * hs, ims));
-  _qweight.alloc(std::max(3 * hs * hs, hs * ims));
-  _igemm_alpha.alloc(tok);
+  _mask.alloc(tok);
+  alloc_blocked(_qin, rows, hs, _kh);
+  alloc_blocked(_act, rows, ims, _ki);
+  const size_t square = (hs + 15) / 16 * 16 * _kh;
+  _wqkv.alloc((3 * hs + 15) / 16 * 16 * _kh);
+  _wself_out.alloc(square);
+  _wq.alloc(square);
+  _wcross_out.alloc(square);
+  _winter.alloc((ims + 15) / 16 * 16 * _kh);
+  _woutput.alloc((hs + 15) / 16 * 16 * _ki);
   ++_shared_nlayer;  // transformer_decoder_layer.cpp:64
 }
 
@@ -80,7 +82,7 @@ TransformerDecoderLayer<T>::~TransformerDecoderLayer() {
   // one process can build a second stack after destroying the first.
   if (--_shared_nlayer == 0) {
     _shared_encdec_kv = DeviceBuffer<T>();
-    _shared_kv_tmp = DeviceBuffer<T>();
+    _shared_enc_out = DeviceBuffer<T>();
     _shared_kv_weight = DeviceBuffer<T>();
     _shared_infer_encdec_kv_ptr = nullptr;
   }
@@ -168,147 +170,12 @@ void TransformerDecoderLayer<T>::SetTrainingMode(bool training) { _training = tr
 template <typename T>
 void TransformerDecoderLayer<T>::SetQuantMode(bool enable_quant) { _enable_quant = enable_quant; }
 
-template <typename T>
-void TransformerDecoderLayer<T>::quant_linear(const T* inp, const T* w, const T* cmax,
-                                              int out_features, int in_features) {
-  const int tok = _batch_tokens;
-  LSH_CALL(opb_quantize<T>(_qin.get(), nullptr, _igemm_alpha.get(), inp, cmax,
-                           (long)tok * in_features, tok, 2, _stream));
-  LSH_CALL(opb_quantize<T>(_qweight.get(), nullptr, nullptr, w, cmax + 1,
-                           (long)out_features * in_features, 0, 4, _stream));
-  LSH_CALL(gemm_i8_i8o_dev_alpha(_qin.get(), _qweight.get(), _qout.get(), tok, out_features,
-                                 in_features, _igemm_alpha.get(), _stream));
-}
-
-// transformer_decoder_layer.cpp:91-233
-template <typename T>
-void TransformerDecoderLayer<T>::self_attn_layer_fw(const T* input_ptr, T* output_ptr,
-                                                    const std::vector<T*>& cache) {
-  const int tok = _batch_tokens, hs = _hidden_size, hd = hs / _heads;
-  const int from_len = _predict ? 1 : _trg_seq_len;
-  const int to_len = _predict ? _step + 1 : _trg_seq_len;
-  const int batch_size = _predict ? _batch_size * _trg_seq_len : _batch_size;
-  if (_is_pre_ln)
-    LSH_CALL(opb_layer_norm<T>(_ln_out.get(), nullptr, nullptr, _vars.get(), nullptr, input_ptr,
-                               _attn_nw_ptr, _attn_nb_ptr, nullptr, tok, hs, _stream));
-  quant_linear(_is_pre_ln ? _ln_out.get() : input_ptr, _attn_qkvw_ptr, _attn_qkv_cmax_ptr, 3 * hs,
-               hs);
-  // k and v leave this kernel as the cache will hold them: fake-quantised (:134-138)
-  LSH_CALL(opb_quant_bias_add_transform_20314<T>(_qkv.get(), nullptr, _qout.get(), _attn_qkvb_ptr,
-                                                 _attn_qkv_cmax_ptr + 2, batch_size, from_len, 3,
-                                                 _heads, hd, _stream, _attn_qkv_cache_cmax_ptr));
-  const size_t batch_dim = (size_t)tok * hs;
-  const T* q_tf = _qkv.get();
-  const T* k_tf = q_tf + batch_dim;
-  const T* v_tf = k_tf + batch_dim;
-  if (_predict) {  // :173-180: new cache = previous cache ++ this step's k / v
-    LSH_CALL(opb_concat3_dim1<T>(cache[2], k_tf, cache[0], batch_size * _heads, hd, _step, 1,
-                                 _stream));
-    LSH_CALL(opb_concat3_dim1<T>(cache[3], v_tf, cache[1], batch_size * _heads, hd, _step, 1,
-                                 _stream));
-    k_tf = cache[0];
-    v_tf = cache[1];
-  }
-  // scores, softmax (future positions masked outside a decoding step), context, head merge
-  LSH_CALL(layer_cross_attention_f16(q_tf, k_tf, v_tf, nullptr, _attn_o_inp.get(), batch_size,
-                                     from_len, to_len, _heads, hd, !_predict, _stream));
-
-  quant_linear(_attn_o_inp.get(), _attn_ow_ptr, _attn_out_cmax_ptr, hs, hs);
-  LSH_CALL(opb_quant_dropout_res_bias<T>(output_ptr, nullptr, _qout.get(), _attn_out_cmax_ptr + 2,
-                                         _attn_ob_ptr, input_ptr, (long)tok * hs, hs, 0.f,
-                                         _stream));
-  if (!_is_pre_ln)
-    LSH_CALL(opb_layer_norm<T>(output_ptr, nullptr, nullptr, _vars.get(), nullptr, output_ptr,
-                               _attn_nw_ptr, _attn_nb_ptr, nullptr, tok, hs, _stream));
-}
-
-// transformer_decoder_layer.cpp:236-262: k and v of the encoder output for every decoder
-// layer in one fp16 product with fake-quantised weights (the input is not quantised)
-template <typename T>
-void TransformerDecoderLayer<T>::encdec_kv_fw(const T* enc_output_ptr) {
-  if (!enc_output_ptr) throw std::runtime_error("Forward: null encoder output");
-  if (!_encdec_attn_kvw_ptr)
-    throw std::runtime_error("Forward: layer 0 holds no cross-attention k/v weights");
-  const size_t hs = _hidden_size;
-  const int nl = _shared_nlayer, src_tok = _batch_size * _src_seq_len;
-  const size_t kv_elems = (size_t)nl * 2 * _max_batch_tokens * hs;
-  if (_shared_kv_tmp.size() != kv_elems) _shared_kv_tmp.alloc(kv_elems);
-  if (!_predict && _shared_encdec_kv.size() != kv_elems) _shared_encdec_kv.alloc(kv_elems);
-  if (_shared_kv_weight.size() != (size_t)nl * 2 * hs * hs)
-    _shared_kv_weight.alloc((size_t)nl * 2 * hs * hs);
-  LSH_CALL(opb_fake_quantize<T>(nullptr, nullptr, _shared_kv_weight.get(), _encdec_attn_kvw_ptr,
-                                _encdec_kv_cmax_ptr + 1, (long)nl * 2 * hs * hs, 4, true,
-                                _stream));
-  LSH_CALL(gemm_f16_nt(enc_output_ptr, _shared_kv_weight.get(), _shared_kv_tmp.get(), src_tok,
-                       nl * 2 * (int)hs, (int)hs, _stream));
-  // [batch, src_len, layers * 2, heads, head_dim] -> [layers * 2, batch, heads, src_len, head_dim]
-  LSH_CALL(opb_bias_add_transform_20314<T>(
-      _predict ? _shared_infer_encdec_kv_ptr : _shared_encdec_kv.get(), _shared_kv_tmp.get(),
-      _encdec_attn_kvb_ptr, _batch_size, _src_seq_len, nl * 2, _heads, (int)hs / _heads, _stream));
-}
-
-// transformer_decoder_layer.cpp:278-412
-template <typename T>
-void TransformerDecoderLayer<T>::encdec_attn_layer_fw(const T* input_ptr, const T* enc_mask_ptr,
-                                                      T* output_ptr) {
-  const int tok = _batch_tokens, hs = _hidden_size, hd = hs / _heads;
-  if (_is_pre_ln)
-    LSH_CALL(opb_layer_norm<T>(_ln_out.get(), nullptr, nullptr, _vars.get(), nullptr, input_ptr,
-                               _encdec_attn_nw_ptr, _encdec_attn_nb_ptr, nullptr, tok, hs,
-                               _stream));
-  quant_linear(_is_pre_ln ? _ln_out.get() : input_ptr, _encdec_attn_qw_ptr, _encdec_qkv_cmax_ptr,
-               hs, hs);
-  LSH_CALL(opb_quant_bias_add_transform_20314<T>(
-      _encdec_q.get(), nullptr, _qout.get(), _encdec_attn_qb_ptr, _encdec_qkv_cmax_ptr + 2,
-      _batch_size, _trg_seq_len, 1, _heads, hd, _stream, nullptr));
-
-  const T* kv = _predict ? _shared_infer_encdec_kv_ptr : _shared_encdec_kv.get();
-  if (!kv) throw std::runtime_error("Forward: layer 0 has not produced the cross-attention k/v");
-  const size_t src_dim = (size_t)_batch_size * _src_seq_len * hs;
-  const T* k = kv + (size_t)_layer_id * 2 * src_dim;
-  LSH_CALL(layer_cross_attention_f16(_encdec_q.get(), k, k + src_dim, enc_mask_ptr,
-                                     _attn_o_inp.get(), _batch_size, _trg_seq_len, _src_seq_len,
-                                     _heads, hd, false, _stream));
-
-  quant_linear(_attn_o_inp.get(), _encdec_attn_ow_ptr, _encdec_out_cmax_ptr, hs, hs);
-  LSH_CALL(opb_quant_dropout_res_bias<T>(output_ptr, nullptr, _qout.get(),
-                                         _encdec_out_cmax_ptr + 2, _encdec_attn_ob_ptr, input_ptr,
-                                         (long)tok * hs, hs, 0.f, _stream));
-  if (!_is_pre_ln)
-    LSH_CALL(opb_layer_norm<T>(output_ptr, nullptr, nullptr, _vars.get(), nullptr, output_ptr,
-                               _encdec_attn_nw_ptr, _encdec_attn_nb_ptr, nullptr, tok, hs,
-                               _stream));
-}
-
-// transformer_decoder_layer.cpp:415-483
-template <typename T>
-void TransformerDecoderLayer<T>::ffn_layer_fw(T* inp_ptr, T* out_ptr) {
-  const int tok = _batch_tokens, hs = _hidden_size, ims = _intermediate_size;
-  if (_is_pre_ln)
-    LSH_CALL(opb_layer_norm<T>(_ln_out.get(), nullptr, nullptr, _vars.get(), nullptr, inp_ptr,
-                               _ffn_nw_ptr, _ffn_nb_ptr, nullptr, tok, hs, _stream));
-  quant_linear(_is_pre_ln ? _ln_out.get() : inp_ptr, _inter_w_ptr, _inter_cmax_ptr, ims, hs);
-  // dropout.h:118-122: ReLU output goes through the unsigned (symmetry = false) quantiser
-  const bool relu = _activation_fn == "relu";
-  LSH_CALL(opb_quant_dropout_act_bias<T>(relu ? 1 : 0, nullptr, _ff2_inp.get(), nullptr, nullptr,
-                                         nullptr, _qout.get(), _inter_b_ptr, _inter_cmax_ptr + 2,
-                                         _output_cmax_ptr, (long)tok * ims, ims, 0.f, !relu,
-                                         _stream));
-  LSH_CALL(opb_fake_quantize<T>(nullptr, nullptr, _fake_weight.get(), _output_w_ptr,
-                                _output_cmax_ptr + 1, (long)ims * hs, 4, true, _stream));
-  LSH_CALL(gemm_f16_nt(_ff2_inp.get(), _fake_weight.get(), out_ptr, tok, hs, ims, _stream));
-  LSH_CALL(opb_dropout_res_bias<T>(out_ptr, out_ptr, nullptr, _output_b_ptr, inp_ptr,
-                                   (long)tok * hs, hs, 0.f, _stream));
-  if (!_is_pre_ln)
-    LSH_CALL(opb_layer_norm<T>(out_ptr, nullptr, nullptr, _vars.get(), nullptr, out_ptr,
-                               _ffn_nw_ptr, _ffn_nb_ptr, nullptr, tok, hs, _stream));
-}
-
 // transformer_decoder_layer.cpp:508-547
 template <typename T>
 void TransformerDecoderLayer<T>::Forward(const T* dec_input_ptr, const T* enc_output_ptr,
-                                         const T* enc_mask_ptr, T* dec_output_ptr,
-                                         const std::vector<T*>& cache) {
+                                         long enc_stride_b, long enc_stride_s,
+                                         const void* enc_mask_ptr, int mask_kind,
+                                         T* dec_output_ptr, const std::vector<T*>& cache) {
   if (!dec_input_ptr || !dec_output_ptr) throw std::runtime_error("Forward: null input or output");
   if (!_attn_qkvw_ptr) throw std::runtime_error("Forward: no parameter blob assigned");
   if (_batch_tokens == 0) throw std::runtime_error("Forward: set_cur_batch_shape not called");
@@ -325,17 +192,103 @@ void TransformerDecoderLayer<T>::Forward(const T* dec_input_ptr, const T* enc_ou
   }
   _stream = Context::Instance().get_stream();
 
-  if (_layer_id == 0) {
-    if (_predict) {
-      _shared_infer_encdec_kv_ptr = cache[4];
-      if (_step == 0) encdec_kv_fw(enc_output_ptr);
-    } else {
-      encdec_kv_fw(enc_output_ptr);
-    }
+  const int tok = _batch_tokens, hs = _hidden_size, ims = _intermediate_size, hd = hs / _heads;
+  const bool relu = _activation_fn == "relu";
+  const int src_tok = _batch_size * _src_seq_len;
+
+  LayerPrep prep;
+  LSH_CALL(prep.codes(_attn_qkvw_ptr, _wqkv.get(), _attn_qkv_cmax_ptr + 1, 3 * hs, hs, _kh));
+  LSH_CALL(prep.codes(_attn_ow_ptr, _wself_out.get(), _attn_out_cmax_ptr + 1, hs, hs, _kh));
+  LSH_CALL(prep.codes(_encdec_attn_qw_ptr, _wq.get(), _encdec_qkv_cmax_ptr + 1, hs, hs, _kh));
+  LSH_CALL(prep.codes(_encdec_attn_ow_ptr, _wcross_out.get(), _encdec_out_cmax_ptr + 1, hs, hs, _kh));
+  LSH_CALL(prep.codes(_inter_w_ptr, _winter.get(), _inter_cmax_ptr + 1, ims, hs, _kh));
+  LSH_CALL(prep.halfs(_output_w_ptr, _woutput.get(), _output_cmax_ptr + 1, hs, ims, _ki, 1, ims, 0));
+  if (_is_pre_ln)
+    LSH_CALL(prep.norm(dec_input_ptr, _qin.get(), _attn_nw_ptr, _attn_nb_ptr, _attn_qkv_cmax_ptr, tok, hs, _kh));
+  else
+    LSH_CALL(prep.codes(dec_input_ptr, _qin.get(), _attn_qkv_cmax_ptr, tok, hs, _kh));
+  const T* mask = static_cast<const T*>(enc_mask_ptr);
+  if (mask && mask_kind != kMaskNone) {
+    LSH_CALL(prep.mask(enc_mask_ptr, mask_kind, _mask.get(), src_tok));
+    mask = _mask.get();
   }
-  self_attn_layer_fw(dec_input_ptr, _encdec_inp.get(), cache);
-  encdec_attn_layer_fw(_encdec_inp.get(), enc_mask_ptr, _ffn_inp.get());
-  ffn_layer_fw(_ffn_inp.get(), dec_output_ptr);
+  const int self_batch = _predict ? _batch_size * _trg_seq_len : _batch_size;
+  if (_predict && _step > 0)  // :173-180: new cache = previous cache ++ this step's k / v
+    for (int i = 0; i < 2; ++i)
+      LSH_CALL(prep.grow(cache[2 + i], cache[i], self_batch * _heads, _step * hd, (long)(_step + 1) * hd));
+  const int nl = _shared_nlayer;
+  if (_layer_id == 0 && _predict) _shared_infer_encdec_kv_ptr = cache[4];
+  if (makes_encdec_kv()) {
+    // :236-262: fake-quantised weights, the encoder output as it is
+    if (!enc_output_ptr) throw std::runtime_error("Forward: null encoder output");
+    if (!_encdec_attn_kvw_ptr)
+      throw std::runtime_error("Forward: layer 0 holds no cross-attention k/v weights");
+    const size_t enc_elems = (((size_t)_max_batch_tokens + 15) & ~(size_t)15) * _kh;
+    if (_shared_enc_out.size() != enc_elems) _shared_enc_out.alloc(enc_elems);
+    const size_t kv_elems = (size_t)nl * 2 * _max_batch_tokens * hs;
+    if (!_predict && _shared_encdec_kv.size() != kv_elems) _shared_encdec_kv.alloc(kv_elems);
+    const size_t w_elems = ((size_t)nl * 2 * hs + 15) / 16 * 16 * _kh;
+    if (_shared_kv_weight.size() != w_elems) _shared_kv_weight.alloc(w_elems);
+    LSH_CALL(prep.halfs(_encdec_attn_kvw_ptr, _shared_kv_weight.get(), _encdec_kv_cmax_ptr + 1, nl * 2 * hs,
+                        hs, _kh, 1, hs, 0));
+    LSH_CALL(prep.halfs(enc_output_ptr, _shared_enc_out.get(), nullptr, src_tok, hs, _kh, _src_seq_len,
+                        enc_stride_b, enc_stride_s));
+  }
+  LSH_CALL(prep.launch(_stream));
+
+  const size_t src_dim = (size_t)src_tok * hs;
+  T* kv = _predict ? _shared_infer_encdec_kv_ptr : _shared_encdec_kv.get();
+  if (makes_encdec_kv())
+    LSH_CALL(gemm_blk_kv_f16(_shared_enc_out.get(), _shared_kv_weight.get(), src_tok, nl, hs, _kh,
+                             _encdec_attn_kvb_ptr, _src_seq_len, _heads, kv, kv + src_dim,
+                             (long)(2 * src_dim), _stream));
+  if (!kv) throw std::runtime_error("Forward: layer 0 has not produced the cross-attention k/v");
+
+  // self attention (:91-233); k and v leave the product as the cache will hold them: fake-quantised
+  // (:134-138)
+  const int from_len = _predict ? 1 : _trg_seq_len, to_len = _predict ? _step + 1 : _trg_seq_len;
+  const size_t batch_dim = (size_t)tok * hs;
+  T* q = _qkv.get();
+  T* const self[3] = {q, _predict ? cache[0] : q + batch_dim, _predict ? cache[1] : q + 2 * batch_dim};
+  const int self_at = _predict ? _step : 0;
+  const int len[3] = {from_len, to_len, to_len}, at[3] = {0, self_at, self_at};
+  LSH_CALL(layer_gemm_heads(_qin.get(), _wqkv.get(), tok, 3, hs, _kh, _attn_qkvb_ptr, _attn_qkv_cmax_ptr,
+                            _attn_qkv_cache_cmax_ptr, from_len, _heads, self, len, at, _stream));
+  LSH_CALL(layer_attention_codes(self[0], self[1], self[2], nullptr, _qin.get(), _attn_out_cmax_ptr, _kh,
+                                 self_batch, from_len, to_len, _heads, hd, !_predict, _stream));
+  LSH_CALL(layer_gemm_residual(_qin.get(), _wself_out.get(), tok, hs, _kh, _attn_ob_ptr, _attn_out_cmax_ptr,
+                               dec_input_ptr, _encdec_inp.get(), _stream));
+
+  // cross attention (:278-412); a norm between two blocks closes the first (post) or opens the
+  // second (pre)
+  T* x = _encdec_inp.get();
+  LSH_CALL(layer_norm_codes(x, _is_pre_ln ? nullptr : x, _qin.get(),
+                            _is_pre_ln ? _encdec_attn_nw_ptr : _attn_nw_ptr,
+                            _is_pre_ln ? _encdec_attn_nb_ptr : _attn_nb_ptr, _encdec_qkv_cmax_ptr, tok, hs,
+                            _kh, _stream));
+  T* const cross[1] = {q};
+  LSH_CALL(layer_gemm_heads(_qin.get(), _wq.get(), tok, 1, hs, _kh, _encdec_attn_qb_ptr,
+                            _encdec_qkv_cmax_ptr, nullptr, _trg_seq_len, _heads, cross, &_trg_seq_len, at,
+                            _stream));
+  const T* k = kv + (size_t)_layer_id * 2 * src_dim;
+  LSH_CALL(layer_attention_codes(q, k, k + src_dim, mask, _qin.get(), _encdec_out_cmax_ptr, _kh, _batch_size,
+                                 _trg_seq_len, _src_seq_len, _heads, hd, false, _stream));
+  LSH_CALL(layer_gemm_residual(_qin.get(), _wcross_out.get(), tok, hs, _kh, _encdec_attn_ob_ptr,
+                               _encdec_out_cmax_ptr, x, _ffn_inp.get(), _stream));
+
+  // feed forward (:415-483); dropout.h:118-122: ReLU output goes through the unsigned quantiser
+  x = _ffn_inp.get();
+  LSH_CALL(layer_norm_codes(x, _is_pre_ln ? nullptr : x, _qin.get(),
+                            _is_pre_ln ? _ffn_nw_ptr : _encdec_attn_nw_ptr,
+                            _is_pre_ln ? _ffn_nb_ptr : _encdec_attn_nb_ptr, _inter_cmax_ptr, tok, hs, _kh,
+                            _stream));
+  LSH_CALL(layer_gemm_act(_qin.get(), _winter.get(), tok, ims, _kh, _inter_b_ptr, _inter_cmax_ptr,
+                          _output_cmax_ptr, relu, _act.get(), _ki, _stream));
+  LSH_CALL(layer_gemm_ffn2(_act.get(), _woutput.get(), tok, hs, _ki, _output_b_ptr, x, dec_output_ptr,
+                           _stream));
+  if (!_is_pre_ln)
+    LSH_CALL(layer_norm_codes(dec_output_ptr, dec_output_ptr, nullptr, _ffn_nw_ptr, _ffn_nb_ptr, nullptr,
+                              tok, hs, _kh, _stream));
 }
 
 template class TransformerDecoderLayer<__half>;

@@ -28,8 +28,12 @@ class TransformerDecoderLayer {
   // step + 1, head_dim] (written), [2] / [3] the previous step's k / v [.., step, head_dim]
   // (read; null at step 0), [4] (layer 0 only) cross-attention k, v of all layers
   // [layers * 2, batch, heads, src_seq_len, head_dim] (written at step 0, read afterwards).
-  void Forward(const T* dec_input_ptr, const T* enc_output_ptr, const T* enc_mask_ptr,
-               T* dec_output_ptr, const std::vector<T*>& cache);
+  // enc_output_ptr: token s of sequence b at b * enc_stride_b + s * enc_stride_s (elements); read
+  // by layer 0 where it makes the cross-attention keys and values.  mask_kind: as for the
+  // encoder layer.
+  void Forward(const T* dec_input_ptr, const T* enc_output_ptr, long enc_stride_b, long enc_stride_s,
+               const void* enc_mask_ptr, int mask_kind, T* dec_output_ptr, const std::vector<T*>& cache);
+  int hidden_size() const { return _hidden_size; }
 
   // step < 0: the whole target sequence with future positions masked; step >= 0: one
   // decoding step, trg_seq_len is then the beam size (transformer_decoder_layer.h:67-92)
@@ -46,13 +50,7 @@ class TransformerDecoderLayer {
   static int shared_layer_count() { return _shared_nlayer; }
 
  private:
-  void encdec_kv_fw(const T* enc_output_ptr);
-  void self_attn_layer_fw(const T* input_ptr, T* output_ptr, const std::vector<T*>& cache);
-  void encdec_attn_layer_fw(const T* input_ptr, const T* enc_mask_ptr, T* output_ptr);
-  void ffn_layer_fw(T* inp_ptr, T* out_ptr);
-  // int8 product of an activation and a weight matrix, both quantised here:
-  // qout[tokens, out] = sat(alpha * quantize(inp) x quantize(w)^T), cmax = {input, weight, output}
-  void quant_linear(const T* inp, const T* w, const T* cmax, int out_features, int in_features);
+  bool makes_encdec_kv() const { return _layer_id == 0 && _step <= 0; }
 
   const int _layer_id;
   const int _max_batch_tokens, _max_seq_len, _hidden_size, _heads, _intermediate_size;
@@ -66,13 +64,13 @@ class TransformerDecoderLayer {
 
   // decoder layers of the process share the cross-attention k/v (computed by layer 0)
   static int _shared_nlayer;
-  static DeviceBuffer<T> _shared_encdec_kv, _shared_kv_tmp, _shared_kv_weight;
+  static DeviceBuffer<T> _shared_encdec_kv, _shared_enc_out, _shared_kv_weight;
   static T* _shared_infer_encdec_kv_ptr;
 
-  DeviceBuffer<T> _ln_out, _qkv, _attn_o_inp, _encdec_inp, _encdec_q, _ffn_inp, _ff2_inp,
-      _fake_weight, _vars;
-  DeviceBuffer<int8_t> _qin, _qout, _qweight;
-  DeviceBuffer<float> _igemm_alpha;
+  // matrices of codes are blocked, their rows padded to 64 bytes
+  const int _kh, _ki;  // padded hidden and intermediate size
+  DeviceBuffer<T> _qkv, _encdec_inp, _ffn_inp, _mask, _act, _woutput;
+  DeviceBuffer<int8_t> _qin, _wqkv, _wself_out, _wq, _wcross_out, _winter;
 
   const T* _attn_qkvw_ptr = nullptr;
   const T* _attn_qkvb_ptr = nullptr;

@@ -1,8 +1,7 @@
 // Forward pass of the quantised encoder layer
-// (lightseq/csrc/layers/transformer_encoder_layer.cpp:66-293), built from this library's
-// operator kernels.  What differs from the reference's sequence is only where kernels are
-// fused: the attention core (scores, masked softmax, context, head merge) is one kernel,
-// and the int8 GEMMs read their scale from device memory in the epilogue.
+// (lightseq/csrc/layers/transformer_encoder_layer.cpp:66-293) in seven launches (eight with a
+// closing layer norm): the preparations, four products with the operators between them as
+// epilogues, the attention core, the layer norm between the halves.
 #include "transformer_encoder_layer.h"
 
 #include <algorithm>
@@ -28,7 +27,9 @@ TransformerEncoderLayer<T>::TransformerEncoderLayer(
       _intermediate_size(intermediate_size),
       _is_pre_ln(pre_or_postLayerNorm),
       _activation_fn(activation_fn),
-      _mask_future_tokens(mask_future_tokens) {
+      _mask_future_tokens(mask_future_tokens),
+      _kh((hidden_size + 63) & ~63),
+      _ki((intermediate_size + 63) & ~63) {
   (void)attn_prob_dropout_ratio;  // ratios only matter in training mode, which Forward rejects
   (void)activation_dropout_ratio;
   (void)hidden_output_dropout_ratio;
@@ -48,17 +49,16 @@ TransformerEncoderLayer<T>::TransformerEncoderLayer(
 
   const size_t tok = (size_t)max_batch_tokens, hs = (size_t)hidden_size,
                ims = (size_t)intermediate_size;
-  if (_is_pre_ln) _ln_out.alloc(tok * hs);
+  const size_t rows = (tok + 15) & ~(size_t)15;
   _qkv.alloc(3 * tok * hs);
-  _attn_o_inp.alloc(tok * hs);
   _ffn_inp.alloc(tok * hs);
-  _ff2_inp.alloc(tok * ims);
-  _fake_weight.alloc(hs * ims);
-  _vars.alloc(tok);
-  _qin.alloc(tok * std::max(hs, ims));
-  _qout.alloc(tok * std::max(3 * hs, ims));
-  _qweight.alloc(std::max(3 * hs * hs, hs * ims));
-  _igemm_alpha.alloc(tok);
+  _mask.alloc(tok);
+  alloc_blocked(_qin, rows, hs, _kh);
+  alloc_blocked(_act, rows, ims, _ki);
+  _wqkv.alloc((3 * hs + 15) / 16 * 16 * _kh);
+  _wout.alloc((hs + 15) / 16 * 16 * _kh);
+  _winter.alloc((ims + 15) / 16 * 16 * _kh);
+  _woutput.alloc((hs + 15) / 16 * 16 * _ki);
 }
 
 template <typename T>
@@ -113,83 +113,10 @@ void TransformerEncoderLayer<T>::SetTrainingMode(bool training) { _training = tr
 template <typename T>
 void TransformerEncoderLayer<T>::SetQuantMode(bool enable_quant) { _enable_quant = enable_quant; }
 
-// transformer_encoder_layer.cpp:66-185
-template <typename T>
-void TransformerEncoderLayer<T>::attn_layer_fw(const T* input_ptr, const T* input_mask_ptr,
-                                               T* output_ptr) {
-  const int tok = _batch_tokens, hs = _hidden_size;
-  if (_is_pre_ln)
-    LSH_CALL(opb_layer_norm<T>(_ln_out.get(), nullptr, nullptr, _vars.get(), nullptr, input_ptr,
-                               _attn_nw_ptr, _attn_nb_ptr, nullptr, tok, hs, _stream));
-  const T* gemmQKV_inp_ptr = _is_pre_ln ? _ln_out.get() : input_ptr;
-
-  LSH_CALL(opb_quantize<T>(_qin.get(), nullptr, _igemm_alpha.get(), gemmQKV_inp_ptr,
-                           _attn_qkv_cmax_ptr, (long)tok * hs, tok, 2, _stream));
-  LSH_CALL(opb_quantize<T>(_qweight.get(), nullptr, nullptr, _attn_qkvw_ptr,
-                           _attn_qkv_cmax_ptr + 1, 3L * hs * hs, 0, 4, _stream));
-  LSH_CALL(gemm_i8_i8o_dev_alpha(_qin.get(), _qweight.get(), _qout.get(), tok, 3 * hs, hs,
-                                 _igemm_alpha.get(), _stream));
-  const T* cache_cmax = _mask_future_tokens ? _attn_qkv_cache_cmax_ptr : nullptr;
-  LSH_CALL(opb_quant_bias_add_transform_20314<T>(_qkv.get(), nullptr, _qout.get(), _attn_qkvb_ptr,
-                                                 _attn_qkv_cmax_ptr + 2, _batch_size, _seq_len, 3,
-                                                 _heads, hs / _heads, _stream, cache_cmax));
-
-  // scores, masked softmax, context and head merge in one kernel (:121-148)
-  const size_t batch_dim = (size_t)tok * hs;
-  const T* q = _qkv.get();
-  LSH_CALL(layer_attention_f16(q, q + batch_dim, q + 2 * batch_dim, input_mask_ptr,
-                               _attn_o_inp.get(), _batch_size, _seq_len, _heads, hs / _heads,
-                               _mask_future_tokens, _stream));
-
-  LSH_CALL(opb_quantize<T>(_qin.get(), nullptr, _igemm_alpha.get(), _attn_o_inp.get(),
-                           _attn_out_cmax_ptr, (long)tok * hs, tok, 2, _stream));
-  LSH_CALL(opb_quantize<T>(_qweight.get(), nullptr, nullptr, _attn_ow_ptr, _attn_out_cmax_ptr + 1,
-                           (long)hs * hs, 0, 4, _stream));
-  LSH_CALL(gemm_i8_i8o_dev_alpha(_qin.get(), _qweight.get(), _qout.get(), tok, hs, hs,
-                                 _igemm_alpha.get(), _stream));
-  LSH_CALL(opb_quant_dropout_res_bias<T>(output_ptr, nullptr, _qout.get(), _attn_out_cmax_ptr + 2,
-                                         _attn_ob_ptr, input_ptr, (long)tok * hs, hs, 0.f,
-                                         _stream));
-  if (!_is_pre_ln)
-    LSH_CALL(opb_layer_norm<T>(output_ptr, nullptr, nullptr, _vars.get(), nullptr, output_ptr,
-                               _attn_nw_ptr, _attn_nb_ptr, nullptr, tok, hs, _stream));
-}
-
-// transformer_encoder_layer.cpp:188-250
-template <typename T>
-void TransformerEncoderLayer<T>::ffn_layer_fw(T* inp_ptr, T* out_ptr) {
-  const int tok = _batch_tokens, hs = _hidden_size, ims = _intermediate_size;
-  const T* ff1_inp = inp_ptr;
-  if (_is_pre_ln) {
-    LSH_CALL(opb_layer_norm<T>(_ln_out.get(), nullptr, nullptr, _vars.get(), nullptr, inp_ptr,
-                               _ffn_nw_ptr, _ffn_nb_ptr, nullptr, tok, hs, _stream));
-    ff1_inp = _ln_out.get();
-  }
-  LSH_CALL(opb_quantize<T>(_qin.get(), nullptr, _igemm_alpha.get(), ff1_inp, _inter_cmax_ptr,
-                           (long)tok * hs, tok, 2, _stream));
-  LSH_CALL(opb_quantize<T>(_qweight.get(), nullptr, nullptr, _inter_w_ptr, _inter_cmax_ptr + 1,
-                           (long)ims * hs, 0, 4, _stream));
-  LSH_CALL(gemm_i8_i8o_dev_alpha(_qin.get(), _qweight.get(), _qout.get(), tok, ims, hs,
-                                 _igemm_alpha.get(), _stream));
-  // dropout.h:118-122: ReLU output goes through the unsigned (symmetry = false) quantiser
-  const bool relu = _activation_fn == "relu";
-  LSH_CALL(opb_quant_dropout_act_bias<T>(relu ? 1 : 0, nullptr, _ff2_inp.get(), nullptr, nullptr,
-                                         nullptr, _qout.get(), _inter_b_ptr, _inter_cmax_ptr + 2,
-                                         _output_cmax_ptr, (long)tok * ims, ims, 0.f, !relu,
-                                         _stream));
-  LSH_CALL(opb_fake_quantize<T>(nullptr, nullptr, _fake_weight.get(), _output_w_ptr,
-                                _output_cmax_ptr + 1, (long)ims * hs, 4, true, _stream));
-  LSH_CALL(gemm_f16_nt(_ff2_inp.get(), _fake_weight.get(), out_ptr, tok, hs, ims, _stream));
-  LSH_CALL(opb_dropout_res_bias<T>(out_ptr, out_ptr, nullptr, _output_b_ptr, inp_ptr,
-                                   (long)tok * hs, hs, 0.f, _stream));
-  if (!_is_pre_ln)
-    LSH_CALL(opb_layer_norm<T>(out_ptr, nullptr, nullptr, _vars.get(), nullptr, out_ptr,
-                               _ffn_nw_ptr, _ffn_nb_ptr, nullptr, tok, hs, _stream));
-}
-
 // transformer_encoder_layer.cpp:277-293
 template <typename T>
-void TransformerEncoderLayer<T>::Forward(const T* input_ptr, const T* input_mask_ptr, T* out_ptr) {
+void TransformerEncoderLayer<T>::Forward(const T* input_ptr, const void* input_mask_ptr, int mask_kind,
+                                         T* out_ptr) {
   if (!input_ptr || !out_ptr) throw std::runtime_error("Forward: null input or output");
   if (!_attn_qkvw_ptr) throw std::runtime_error("Forward: no parameter blob assigned");
   if (_batch_tokens == 0) throw std::runtime_error("Forward: set_cur_batch_shape not called");
@@ -198,8 +125,49 @@ void TransformerEncoderLayer<T>::Forward(const T* input_ptr, const T* input_mask
   if (!_enable_quant)
     throw std::runtime_error("Forward: only the quantised path of the layer is provided");
   _stream = Context::Instance().get_stream();
-  attn_layer_fw(input_ptr, input_mask_ptr, _ffn_inp.get());
-  ffn_layer_fw(_ffn_inp.get(), out_ptr);
+  const int tok = _batch_tokens, hs = _hidden_size, ims = _intermediate_size, hd = hs / _heads;
+  const bool relu = _activation_fn == "relu";
+
+  LayerPrep prep;
+  LSH_CALL(prep.codes(_attn_qkvw_ptr, _wqkv.get(), _attn_qkv_cmax_ptr + 1, 3 * hs, hs, _kh));
+  LSH_CALL(prep.codes(_attn_ow_ptr, _wout.get(), _attn_out_cmax_ptr + 1, hs, hs, _kh));
+  LSH_CALL(prep.codes(_inter_w_ptr, _winter.get(), _inter_cmax_ptr + 1, ims, hs, _kh));
+  LSH_CALL(prep.halfs(_output_w_ptr, _woutput.get(), _output_cmax_ptr + 1, hs, ims, _ki, 1, ims, 0));
+  if (_is_pre_ln)
+    LSH_CALL(prep.norm(input_ptr, _qin.get(), _attn_nw_ptr, _attn_nb_ptr, _attn_qkv_cmax_ptr, tok, hs, _kh));
+  else
+    LSH_CALL(prep.codes(input_ptr, _qin.get(), _attn_qkv_cmax_ptr, tok, hs, _kh));
+  const T* mask = static_cast<const T*>(input_mask_ptr);
+  if (mask && mask_kind != kMaskNone) {
+    LSH_CALL(prep.mask(input_mask_ptr, mask_kind, _mask.get(), tok));
+    mask = _mask.get();
+  }
+  LSH_CALL(prep.launch(_stream));
+
+  // attention (:66-185)
+  const size_t batch_dim = (size_t)tok * hs;
+  T* const heads[3] = {_qkv.get(), _qkv.get() + batch_dim, _qkv.get() + 2 * batch_dim};
+  const int len[3] = {_seq_len, _seq_len, _seq_len}, at[3] = {0, 0, 0};
+  LSH_CALL(layer_gemm_heads(_qin.get(), _wqkv.get(), tok, 3, hs, _kh, _attn_qkvb_ptr, _attn_qkv_cmax_ptr,
+                            _mask_future_tokens ? _attn_qkv_cache_cmax_ptr : nullptr, _seq_len, _heads,
+                            heads, len, at, _stream));
+  LSH_CALL(layer_attention_codes(heads[0], heads[1], heads[2], mask, _qin.get(), _attn_out_cmax_ptr, _kh,
+                                 _batch_size, _seq_len, _seq_len, _heads, hd, _mask_future_tokens, _stream));
+  LSH_CALL(layer_gemm_residual(_qin.get(), _wout.get(), tok, hs, _kh, _attn_ob_ptr, _attn_out_cmax_ptr,
+                               input_ptr, _ffn_inp.get(), _stream));
+
+  // feed forward (:188-250); dropout.h:118-122: ReLU output goes through the unsigned quantiser.
+  // The norm between the halves closes the first (post) or opens the second (pre).
+  LSH_CALL(layer_norm_codes(_ffn_inp.get(), _is_pre_ln ? nullptr : _ffn_inp.get(), _qin.get(),
+                            _is_pre_ln ? _ffn_nw_ptr : _attn_nw_ptr, _is_pre_ln ? _ffn_nb_ptr : _attn_nb_ptr,
+                            _inter_cmax_ptr, tok, hs, _kh, _stream));
+  LSH_CALL(layer_gemm_act(_qin.get(), _winter.get(), tok, ims, _kh, _inter_b_ptr, _inter_cmax_ptr,
+                          _output_cmax_ptr, relu, _act.get(), _ki, _stream));
+  LSH_CALL(layer_gemm_ffn2(_act.get(), _woutput.get(), tok, hs, _ki, _output_b_ptr, _ffn_inp.get(), out_ptr,
+                           _stream));
+  if (!_is_pre_ln)
+    LSH_CALL(layer_norm_codes(out_ptr, out_ptr, nullptr, _ffn_nw_ptr, _ffn_nb_ptr, nullptr, tok, hs, _kh,
+                              _stream));
 }
 
 template class TransformerEncoderLayer<__half>;

@@ -20,7 +20,9 @@ class TransformerEncoderLayer {
                           bool pre_or_postLayerNorm, std::string activation_fn,
                           bool mask_future_tokens = false);
 
-  void Forward(const T* input_ptr, const T* input_mask_ptr, T* out_ptr);
+  // mask_kind: kMaskNone, the mask is the additive T mask of the reference (0 for tokens); else the
+  // caller's padding mask of that element type (1 for padding), null for none
+  void Forward(const T* input_ptr, const void* input_mask_ptr, int mask_kind, T* out_ptr);
 
   void set_cur_batch_shape(int batch_size, int seq_len);
   void SetTrainingMode(bool training);
@@ -33,9 +35,6 @@ class TransformerEncoderLayer {
   size_t param_count() const;
 
  private:
-  void attn_layer_fw(const T* input_ptr, const T* input_mask_ptr, T* output_ptr);
-  void ffn_layer_fw(T* inp_ptr, T* out_ptr);
-
   const int _layer_id;
   const int _max_batch_tokens, _max_seq_len, _hidden_size, _heads, _intermediate_size;
   const bool _is_pre_ln;
@@ -46,10 +45,11 @@ class TransformerEncoderLayer {
   bool _enable_quant = false;
   hipStream_t _stream = nullptr;
 
-  // local device memory, sized once at the maximum shapes
-  DeviceBuffer<T> _ln_out, _qkv, _attn_o_inp, _ffn_inp, _ff2_inp, _fake_weight, _vars;
-  DeviceBuffer<int8_t> _qin, _qout, _qweight;
-  DeviceBuffer<float> _igemm_alpha;
+  // local device memory, sized once at the maximum shapes; matrices of codes are blocked, their
+  // rows padded to 64 bytes
+  const int _kh, _ki;  // padded hidden and intermediate size
+  DeviceBuffer<T> _qkv, _ffn_inp, _mask, _act, _woutput;
+  DeviceBuffer<int8_t> _qin, _wqkv, _wout, _winter;
 
   const T* _attn_qkvw_ptr = nullptr;
   const T* _attn_qkvb_ptr = nullptr;

@@ -622,4 +622,69 @@ inline float length_norm(int length, float alpha) {
   return std::pow((5.f + length) / 6.f, -alpha);
 }
 
+// ---- the fused launches of the quantised layers (layer_gemm.hip, layer_fused.hip) ------------
+// Products on blocked int8 operands; clip values are device scalars {input, weight, output}.
+// Part p of the columns goes to base[p], fp16 [b][head][len[p]][d] from position at[p] on.
+int layer_gemm_heads(const int8_t* A, const int8_t* W, int rows, int parts, int hidden, int K,
+                     const __half* bias, const __half* cmax, const __half* cache_cmax, int seq, int heads,
+                     __half* const* base, const int* len, const int* at, hipStream_t s);
+int layer_gemm_residual(const int8_t* A, const int8_t* W, int rows, int N, int K, const __half* bias,
+                        const __half* cmax, const __half* residual, __half* out, hipStream_t s);
+// out: the next product's input, blocked fp16 with rows of out_k halfs
+int layer_gemm_act(const int8_t* A, const int8_t* W, int rows, int N, int K, const __half* bias,
+                   const __half* cmax, const __half* in_cmax, bool relu, __half* out, int out_k,
+                   hipStream_t s);
+// fp16 product of blocked operands, K halfs
+int layer_gemm_ffn2(const __half* A, const __half* W, int rows, int N, int K, const __half* bias,
+                    const __half* residual, __half* out, hipStream_t s);
+// fp16 product of blocked operands (K halfs, K % 32 == 0): keys and values of `layers` decoder layers
+int gemm_blk_kv_f16(const __half* A, const __half* W, int rows, int layers, int hidden, int K,
+                    const __half* bias, int seq, int heads, __half* k, __half* v, long layer_stride,
+                    hipStream_t s);
+
+enum { kMaskNone = 0, kMaskF32, kMaskF16, kMaskU8, kMaskI32, kMaskI64 };  // what a padding mask is made of
+enum { kPrepCodes, kPrepHalfs, kPrepNorm, kPrepMask, kPrepGrow };
+constexpr int kLayerPrepMost = 14;
+struct LayerPrepSection {
+  int kind, blocks;
+  const __half* src;
+  void* dst;
+  const __half *cmax, *gamma, *beta;
+  int rows, K, k_pad, n1;
+  long stride0, stride1;
+};
+struct LayerPrepArgs {
+  int first[kLayerPrepMost];  // first workgroup of each section
+  int n;
+  LayerPrepSection s[kLayerPrepMost];
+};
+// Everything a layer's forward pass starts from, collected and done in one launch.
+class LayerPrep {
+ public:
+  // fp16 [rows, K] -> blocked int8 codes [rows, k_pad] (the rest zeros)
+  int codes(const __half* src, int8_t* dst, const __half* cmax, int rows, int K, int k_pad);
+  // fp16 -> blocked fp16 [rows, k_pad], fake-quantised with cmax if it is set; row r is read at
+  // (r / n1) stride0 + (r % n1) stride1
+  int halfs(const __half* src, __half* dst, const __half* cmax, int rows, int K, int k_pad, int n1,
+            long stride0, long stride1);
+  // layer norm, then codes
+  int norm(const __half* src, int8_t* dst, const __half* gamma, const __half* beta, const __half* cmax,
+           int rows, int hidden, int k_pad);
+  int mask(const void* src, int kind, __half* dst, int count);
+  // rows of K elements to the beginning of rows of dst_stride elements
+  int grow(const __half* src, __half* dst, int rows, int K, long dst_stride);
+  int launch(hipStream_t s) const;
+
+ private:
+  int add(const LayerPrepSection& s);
+  LayerPrepArgs _args{};
+};
+// layer norm of fp16 rows to fp16 (out may be inp, or null) and / or to blocked codes
+int layer_norm_codes(const __half* inp, __half* out, int8_t* codes, const __half* gamma, const __half* beta,
+                     const __half* cmax, int rows, int hidden, int k_pad, hipStream_t s);
+// the layers' attention, its context as blocked codes [batch * seq_len, k_pad] (cmax: device scalar)
+int layer_attention_codes(const __half* q, const __half* k, const __half* v, const __half* add_mask,
+                          int8_t* codes, const __half* cmax, int k_pad, int batch, int seq_len, int key_len,
+                          int head_num, int dim_per_head, bool mask_future, hipStream_t s);
+
 }  // namespace lsh

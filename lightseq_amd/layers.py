@@ -9,7 +9,6 @@ the module in ``eval()`` mode).  torch owns the parameter and activation memory;
 computes with the library's HIP kernels on torch's current stream.
 """
 import copy
-import ctypes
 import itertools
 import math
 from dataclasses import dataclass
@@ -24,6 +23,20 @@ ACT_CLIP_MAX = 16.0
 WEIGHT_CLIP_MAX = 1.0
 
 _layer_ids = itertools.count()
+
+# element types of a padding mask that the layer call reads as they are
+_MASK_TYPES = {torch.float32: 1, torch.float16: 2, torch.bool: 3, torch.uint8: 3, torch.int32: 4,
+               torch.int64: 5}
+
+
+def _padding_mask(mask, device):
+    """(tensor, type) for the layer call: the mask itself, or the additive fp16 one made of it."""
+    kind = _MASK_TYPES.get(mask.dtype)
+    if kind is None:
+        mask, kind = (mask * -1e8).to(torch.half), 0
+    if mask.device != device:
+        mask = mask.to(device)
+    return mask.contiguous(), kind
 
 
 def calc_offset(sizes):
@@ -133,7 +146,7 @@ class LSTransformerEncoderLayer(nn.Module):
         if not hidden_states.is_cuda:
             raise ValueError("the layer runs on the GPU only (no CPU fallback exists)")
         hidden_states = hidden_states.contiguous().to(torch.half)
-        mask = (encoder_padding_mask * -1e8).to(torch.half).contiguous()
+        mask, mask_type = _padding_mask(encoder_padding_mask, hidden_states.device)
         para = self.para if self.para.dtype == torch.half else self._half_para()
         bs, sl, dim = hidden_states.size()
         if bs * sl > self.config.max_batch_tokens:
@@ -145,13 +158,10 @@ class LSTransformerEncoderLayer(nn.Module):
             assert bs == 1 and sl == mask.size(0)
         else:
             assert bs == mask.size(0) and sl == mask.size(1)
-        call("ls_layer_set_stream", current_stream())
-        call("ls_assign_layer_weight_grad_fp16", ptr(para), None, b"TransformerEncoderLayer",
-             self.layer_id)
         output = torch.empty_like(hidden_states)
-        call("ls_transformer_encoder_layer_fw_fp16", self.layer_id, ptr(hidden_states), ptr(mask),
-             ptr(output), bs, sl, int(self.training), int(self.config.pre_layer_norm),
-             int(self.quant_mode))
+        call("ls_encoder_layer_call_fp16", self.layer_id, ptr(para), ptr(hidden_states), ptr(mask),
+             mask_type, ptr(output), bs, sl, int(self.training), int(self.quant_mode),
+             current_stream())
         return output.to(self.para.dtype)
 
     def _half_para(self):
@@ -299,8 +309,8 @@ class LSTransformerDecoderLayer(nn.Module):
         if not decoder_states.is_cuda:
             raise ValueError("the layer runs on the GPU only (no CPU fallback exists)")
         decoder_states = decoder_states.contiguous().to(torch.half)
-        encoder_out = encoder_out.transpose(0, 1).contiguous().to(torch.half)
-        mask = (encoder_padding_mask * -1e8).to(torch.half).contiguous()
+        src_len, batch = encoder_out.shape[:2]
+        mask, mask_type = _padding_mask(encoder_padding_mask, decoder_states.device)
         para = self.para if self.para.dtype == torch.half else self._half_para()
         cfg = self.config
         step, cache_list = -1, None
@@ -315,13 +325,13 @@ class LSTransformerDecoderLayer(nn.Module):
             encdec_kv = None
             if cfg.layer_id == 0:
                 if step == 0:
-                    cache["encdec_kv"] = torch.zeros(
-                        (cfg.nlayer * 2, encoder_out.shape[0], encoder_out.shape[1] * self.hs),
+                    cache["encdec_kv"] = torch.empty(
+                        (cfg.nlayer * 2, batch, src_len * self.hs),
                         dtype=torch.half, device=decoder_states.device)
                 encdec_kv = cache["encdec_kv"]
             shape = (batch_beams, cfg.nhead, step + 1, self.hs // cfg.nhead)
-            new_k = torch.zeros(shape, dtype=torch.half, device=decoder_states.device)
-            new_v = torch.zeros(shape, dtype=torch.half, device=decoder_states.device)
+            new_k = torch.empty(shape, dtype=torch.half, device=decoder_states.device)
+            new_v = torch.empty(shape, dtype=torch.half, device=decoder_states.device)
             cache_list = [new_k, new_v] + old + [encdec_kv]
             cache["dec_self_k"], cache["dec_self_v"] = new_k, new_v
         bs, sl, dim = decoder_states.size()
@@ -331,27 +341,29 @@ class LSTransformerDecoderLayer(nn.Module):
         if sl > cfg.max_seq_len:
             raise ValueError(f"Sequence length {sl} exceeds the limit {cfg.max_seq_len}.")
         if mask.dim() == 1:
-            assert encoder_out.size(0) == 1 and encoder_out.size(1) == mask.size(0)
+            assert batch == 1 and src_len == mask.size(0)
         else:
-            assert encoder_out.size(0) == mask.size(0) and encoder_out.size(1) == mask.size(1)
-        batch = encoder_out.size(0)
+            assert batch == mask.size(0) and src_len == mask.size(1)
         if cache is None:
             assert bs == batch
             trg_len = sl
         else:
             assert bs % batch == 0 and sl == 1
             trg_len = bs // batch  # the beam size
-        call("ls_layer_set_stream", current_stream())
-        call("ls_assign_layer_weight_grad_fp16", ptr(para), None, b"TransformerDecoderLayer",
-             cfg.layer_id)
+        # layer 0 makes the cross-attention keys and values of the stack, outside a decoding step
+        # and in the first one; it reads the encoder output where it lies
+        enc = encoder_out
+        if cfg.layer_id == 0 and step <= 0:
+            if (enc.dtype != torch.half or enc.stride(2) != 1 or enc.stride(0) % 8 or enc.stride(1) % 8
+                    or enc.data_ptr() % 16):
+                enc = enc.to(torch.half).contiguous()
         output = torch.empty_like(decoder_states)
-        cache_ptrs = None
-        if cache_list is not None:
-            cache_ptrs = (ctypes.c_void_p * 5)(*[ptr(t) for t in cache_list])
+        pointers = [ptr(t) for t in cache_list] if cache_list is not None else [None] * 5
         training = self.training and cache is None
-        call("ls_transformer_decoder_layer_fw_fp16", cfg.layer_id, ptr(decoder_states),
-             ptr(encoder_out), ptr(mask), ptr(output), batch, trg_len, encoder_out.size(1), step,
-             cache_ptrs, int(training), int(cfg.pre_layer_norm), int(self.quant_mode))
+        call("ls_decoder_layer_call_fp16", cfg.layer_id, ptr(para), ptr(decoder_states),
+             enc.data_ptr(), enc.stride(1), enc.stride(0), ptr(mask), mask_type, ptr(output), batch,
+             trg_len, src_len, step, *pointers, int(training), int(self.quant_mode),
+             current_stream())
         return output.to(self.para.dtype)
 
     def _half_para(self):

@@ -169,6 +169,8 @@ _SIGNATURES = {
     "ls_create_quant_linear_layer_fp16": (False, "iiii"),
     "ls_quant_linear_layer_fw_fp16": (False, "i" + "pppp" + "iii"),
     "ls_destroy_layer": (False, "c" + "i"),
+    "ls_encoder_layer_call_fp16": (False, "i" + "pppipii" + "ii" + "s"),
+    "ls_decoder_layer_call_fp16": (False, "i" + "ppp" + "ll" + "pip" + "iiii" + "ppppp" + "ii" + "s"),
 }
 
 _lib = None
