@@ -81,10 +81,10 @@ void QuantDecoder::init_buffer() {
 
   _encdec_k.alloc((size_t)L * _layer_size_encdec_k);
   _encdec_v.alloc((size_t)L * _layer_size_encdec_k);
-  _encoder_out_buf.alloc(tokens * (size_t)L * 2 * H);
   for (auto& q : _cur_step_query) q.alloc(rows * H);
   _query_buf1.alloc(rows * H);
   _ops.blocked = LayerProducts::can_block(H, I, _tw._dim_per_head);
+  _encoder_out_buf.alloc(_ops.blocked ? _ops.rows(tokens) * H : tokens * (size_t)L * 2 * H);
   _logits_stride = _ops.blocked ? (V + 63) & ~63 : V;
   const size_t wide = _ops.rows(rows) * (size_t)std::max(I, 3 * H);
   _buf_a.alloc(wide);
@@ -150,6 +150,12 @@ void QuantDecoder::init_buffer() {
       }
     _kv_kernel.alloc(t.size());
     _kv_kernel.upload(t.data(), t.size(), _stream);
+    if (_ops.blocked) {  // (kv_dim is a multiple of 16: whole blocks)
+      DeviceBuffer<__half> b(t.size());
+      LSH_CALL(block_rows(_kv_kernel.get(), b.get(), (int)kv_dim, 2 * H, false, _stream));
+      CHECK_GPU_ERROR(hipStreamSynchronize(_stream));
+      _kv_kernel = std::move(b);
+    }
     CHECK_GPU_ERROR(hipStreamSynchronize(_stream));
   }
 
@@ -313,6 +319,15 @@ void QuantDecoder::run_one_infer(int batch_size, int batch_seq_len) {
 void QuantDecoder::project_encoder_output() {
   const int H = _tw._hidden_size, L = _tw._n_dec_layer;
   const int kv_dim = H * 2 * L;
+  if (_ops.blocked) {
+    // one product whose epilogue adds the bias and leaves keys and values where the layers read
+    // them (16 x 64 tokens, 6 layers of 1024: 145 + 17 us as product and rearrangement, 45 now)
+    LSH_CALL(block_rows(_p_d_encoder_output, _encoder_out_buf.get(), _batch_token_num, 2 * H, false, _stream));
+    LSH_CALL(gemm_blk_kv_f16(_encoder_out_buf.get(), _kv_kernel.get(), _batch_token_num, L, H, H,
+                             _kv_bias.get(), _batch_seq_len, _tw._head_num, _encdec_k.get(),
+                             _encdec_v.get(), _layer_size_encdec_k, _stream));
+    return;
+  }
   LSH_CALL(gemm_f16_nt(_p_d_encoder_output, _kv_kernel.get(), _encoder_out_buf.get(),
                        _batch_token_num, kv_dim, H, _stream));
   // _encoder_out_buf: [batch_size, batch_seq_len, layer_num, 2, hidden_size]

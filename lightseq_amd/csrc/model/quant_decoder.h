@@ -107,7 +107,8 @@ class QuantDecoder {
 
   // activations and state
   DeviceBuffer<__half> _encdec_k, _encdec_v;      // [n_layer][max_batch*max_step*H]
-  DeviceBuffer<__half> _encoder_out_buf;          // [tokens, n_layer*2*H]
+  // the encoder output, blocked; or where operands are row-major its product [tokens, n_layer*2*H]
+  DeviceBuffer<__half> _encoder_out_buf;
   // the residual stream: a launch that makes a layer norm for itself writes the other buffer
   DeviceBuffer<__half> _cur_step_query[2];
   int _res = 0;
