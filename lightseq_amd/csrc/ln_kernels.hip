@@ -121,8 +121,14 @@ ln_rows_kernel(const AccT* __restrict__ gemm_out, T* residual, T* out_t,
   }
 }
 
-template <typename T, typename AccT, int MODE, int LPR, int ITER>
-__global__ void __launch_bounds__(256)
+// A launch of few rows is bound by the latency of one wavefront's chain, one of many by its
+// instructions: 19 per element where the row fills the lanes' chunks (FULL), 31 before the median
+// clamp, the packed quantiser, the half addition and the exchanges in registers, with the same
+// bytes.  A workgroup is one wavefront, so that rows spread over the compute units: measured
+// against four at 16 / 330 / 2540 / 7930 rows of 768 fp16 3.6 / 3.8 / 6.1 / 10.3 us to
+// 3.8 / 4.1 / 6.1 / 10.4 (before: 4.7 / 5.0 / 7.0 / 12.3).
+template <typename T, typename AccT, int MODE, int LPR, int ITER, bool FULL>
+__global__ void __launch_bounds__(64)
 ln_rows8_kernel(const AccT* __restrict__ gemm_out, T* residual, T* out_t,
                 int8_t* __restrict__ out_q, const T* __restrict__ scale,
                 const T* __restrict__ bias, const T* __restrict__ residual_bias,
@@ -130,12 +136,12 @@ ln_rows8_kernel(const AccT* __restrict__ gemm_out, T* residual, T* out_t,
                 float quant_scale, int is_post_ln, int nparts, long part_stride, int blocked,
                 const int* __restrict__ row_map) {
   constexpr int RPW = kWave / LPR;
-  const int lane = threadIdx.x & 63;
-  const int row = (blockIdx.x * 4 + (threadIdx.x >> 6)) * RPW + lane / LPR;
+  const int lane = threadIdx.x;
+  const int row = blockIdx.x * RPW + lane / LPR;
   int in_row = -1;
   if (MODE == kLnResOut && row_map != nullptr) in_row = row_map[min(row, tokens - 1)];
   // dead rows keep the shuffles convergent
-  ln_rows8_row<T, AccT, MODE, LPR, ITER>(row, row < tokens, lane % LPR, gemm_out, residual, out_t,
+  ln_rows8_row<T, AccT, MODE, LPR, ITER, FULL>(row, row < tokens, lane % LPR, gemm_out, residual, out_t,
                                          out_q, scale, bias, residual_bias, colsum, hidden,
                                          dequant_scale, quant_scale, is_post_ln, nparts,
                                          part_stride, nullptr, 0, blocked, in_row);
@@ -647,11 +653,13 @@ static int launch_ln(const AccT* gemm_out, T* residual, T* out_t, int8_t* out_q,
   }
   if (vec_ok && hidden % 8 == 0) {
     // LPR = 64 when the row fills whole 512-element steps, otherwise two rows per wavefront
-#define LSH_LN8_CASE(LPR, IT)                                                                    \
-  ln_rows8_kernel<T, AccT, MODE, LPR, IT>                                                        \
-      <<<(tokens + 4 * (64 / LPR) - 1) / (4 * (64 / LPR)), 256, 0, stream>>>(                    \
+#define LSH_LN8_RUN(LPR, IT, FULL)                                                               \
+  ln_rows8_kernel<T, AccT, MODE, LPR, IT, FULL>                                                  \
+      <<<(tokens + 64 / LPR - 1) / (64 / LPR), 64, 0, stream>>>(                                 \
           gemm_out, residual, out_t, out_q, scale, bias, residual_bias, colsum, tokens, hidden,  \
           dequant_scale, quant_scale, is_post_ln, nparts, part_stride, blk, row_map)
+#define LSH_LN8_CASE(LPR, IT) \
+  do { if (hidden == LPR * 8 * IT) LSH_LN8_RUN(LPR, IT, true); else LSH_LN8_RUN(LPR, IT, false); } while (0)
     if (hidden <= 256) LSH_LN8_CASE(32, 1);
     else if (hidden <= 512) LSH_LN8_CASE(32, 2);
     else if (hidden <= 768) LSH_LN8_CASE(32, 3);
@@ -659,6 +667,7 @@ static int launch_ln(const AccT* gemm_out, T* residual, T* out_t, int8_t* out_q,
     else if (hidden <= 1536) LSH_LN8_CASE(64, 3);
     else LSH_LN8_CASE(64, 4);
 #undef LSH_LN8_CASE
+#undef LSH_LN8_RUN
     return lsh_check_launch("ln_rows8_kernel");
   }
   if (nparts > 1)

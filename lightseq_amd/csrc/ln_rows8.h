@@ -5,6 +5,7 @@
 // 149-863.
 #pragma once
 #include "ls_device.h"
+#include "tile_common.h"
 
 namespace lsh {
 
@@ -109,22 +110,61 @@ __device__ __forceinline__ void cvt8(const Raw8C& r, float (&o)[8]) {
     o[4 + k] = (float)unpack_i8(r.a.y, k);
   }
 }
+// Sum over the LPR (32 or 64) lanes of a row, every lane active: the additions of the
+// shuffle tree lane ^ 32, 16, 8, 4, 2, 1 in that order, on exchanges that stay in the vector
+// registers (a permute through LDS takes tens of cycles, six in a chain, twice a row).
 template <int LPR>
 __device__ __forceinline__ float row_sum(float v) {
-#pragma unroll
-  for (int m = LPR / 2; m > 0; m >>= 1) v += __shfl_xor(v, m, kWave);
+  // the words of a swap go into scalars first: a bit cast of the element of a vector reads the
+  // vector's first element, whatever the index
+  const uint32_t u = __builtin_bit_cast(uint32_t, v);
+  if constexpr (LPR == 64) {
+    const auto s = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    const uint32_t lo = s[0], hi = s[1];
+    v = __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
+  }
+  const uint32_t w = __builtin_bit_cast(uint32_t, v);
+  const auto s = __builtin_amdgcn_permlane16_swap(w, w, false, false);
+  const uint32_t lo = s[0], hi = s[1];
+  v = __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
+  v += dpp_f<kDppRor8>(v);                         // lane ^ 8
+  v += dpp_f<kDppXor3>(dpp_f<kDppHalfMirror>(v));  // lane ^ 7 ^ 3
+  v += dpp_f<kDppXor2>(v);
+  v += dpp_f<kDppXor1>(v);
   return v;
 }
+typedef _Float16 HalfPair __attribute__((ext_vector_type(2)));
+// keep + bias in the storage type, where keep has just been rounded to it: a half addition
+// (two roundings, to float and to half, of the sum of two halves are one: 24 >= 2 * 11 + 2)
+__device__ __forceinline__ void add8_store(float* p, long i, const float (&keep)[8], const Raw8F& rb) {
+  float b[8], w[8];
+  cvt8(rb, b);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) w[k] = keep[k] + b[k];
+  st8(p, i, w);
+}
+__device__ __forceinline__ void add8_store(__half* p, long i, const float (&keep)[8], const Raw8H& rb) {
+  const uint32_t words[4] = {rb.a.x, rb.a.y, rb.a.z, rb.a.w};
+  uint32_t out[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const HalfPair v = {(_Float16)keep[2 * k], (_Float16)keep[2 * k + 1]};
+    out[k] = __builtin_bit_cast(uint32_t, v + __builtin_bit_cast(HalfPair, words[k]));
+  }
+  *reinterpret_cast<uint4*>(p + i) = make_uint4(out[0], out[1], out[2], out[3]);
+}
+__device__ __forceinline__ void zero8(Raw8F& r) { r.a = r.b = make_float4(0.f, 0.f, 0.f, 0.f); }
+__device__ __forceinline__ void zero8(Raw8H& r) { r.a = make_uint4(0, 0, 0, 0); }
 
 // One row of the 8-wide kernel: `sub` is the lane's index among the LPR lanes of the row,
 // `live` false for a row beyond the tensor (its lanes still take part in the shuffles).
 // gemm_out is read at gemm_out[row * hidden + column] and may point anywhere a flat load
 // reaches (the fused GEMM + LayerNorm kernel passes a tile staged in LDS).
-template <typename T, typename AccT, int MODE, int LPR, int ITER>
+template <typename T, typename AccT, int MODE, int LPR, int ITER, bool FULL = false>
 __device__ __forceinline__ void
 ln_rows8_row(int row, bool live, int sub, const AccT* __restrict__ gemm_out, T* residual, T* out_t,
              int8_t* __restrict__ out_q, const T* __restrict__ scale, const T* __restrict__ bias,
-             const T* __restrict__ residual_bias, const T* __restrict__ colsum, int hidden,
+             const T* __restrict__ residual_bias, const T* __restrict__ colsum, int width,
              float dequant_scale, float quant_scale, int is_post_ln, int nparts, long part_stride,
              const half8_t* pre_res = nullptr, int dead_row = 0, int blocked = 0, int in_row = -1) {
   // pre_res (fp16 only): the lane's ITER residual chunks, already loaded by the caller.
@@ -132,6 +172,9 @@ ln_rows8_row(int row, bool live, int sub, const AccT* __restrict__ gemm_out, T* 
   // hands over a staged tile names a row of the tile.
   // blocked: out_q is a blocked matrix.  in_row: the row of gemm_out and residual that row `row` of
   // out_t is made from, where that is another one (kLnResOut).
+  // FULL: the row fills its lanes' chunks, width == LPR * 8 * ITER.
+  constexpr int kWidth = LPR * 8 * ITER;
+  const int hidden = FULL ? kWidth : width;
   const long base = (long)(live ? (in_row >= 0 ? in_row : row) : dead_row) * hidden;
   const long out_base = (long)row * hidden;
 
@@ -152,7 +195,7 @@ ln_rows8_row(int row, bool live, int sub, const AccT* __restrict__ gemm_out, T* 
   decltype(ld8_raw(gemm_out, 0)) a_raw[ITER];
 #pragma unroll
   for (int it = 0; it < ITER; ++it) {
-    const int e = min((it * LPR + sub) * 8, hidden - 8);
+    const int e = FULL ? (it * LPR + sub) * 8 : min((it * LPR + sub) * 8, hidden - 8);
     g_raw[it] = ld8_raw(scale, e);
     b_raw[it] = ld8_raw(bias, e);
     rb_raw[it] = ld8_raw(rbp, e);
@@ -170,17 +213,11 @@ ln_rows8_row(int row, bool live, int sub, const AccT* __restrict__ gemm_out, T* 
     pin8(r_raw[it]);
     if (MODE != kLnFirst) pin8(a_raw[it]);
   }
-  float gs[ITER][8], bs[ITER][8], rbs[ITER][8];
   float sum = 0.f;
 #pragma unroll
   for (int it = 0; it < ITER; ++it) {
     const int e = (it * LPR + sub) * 8;
-    cvt8(g_raw[it], gs[it]);
-    cvt8(b_raw[it], bs[it]);
-    cvt8(rb_raw[it], rbs[it]);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) rbs[it][k] = has_rb ? rbs[it][k] : 0.f;
-    if (e < hidden && live) {
+    if (FULL || (e < hidden && live)) {
       float r[8];
       if (own_res) {
         cvt8(r_raw[it], r);
@@ -230,7 +267,7 @@ ln_rows8_row(int row, bool live, int sub, const AccT* __restrict__ gemm_out, T* 
 #pragma unroll
   for (int it = 0; it < ITER; ++it) {
     const int e = (it * LPR + sub) * 8;
-    if (e < hidden) {
+    if (FULL || e < hidden) {
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         float t = x[it][k] - mean;
@@ -244,27 +281,34 @@ ln_rows8_row(int row, bool live, int sub, const AccT* __restrict__ gemm_out, T* 
 #pragma unroll
   for (int it = 0; it < ITER; ++it) {
     const int e = (it * LPR + sub) * 8;
-    if (e < hidden) {
-      float o[8];
+    if (FULL || e < hidden) {
+      float g[8], b[8], o[8];
+      cvt8(g_raw[it], g);
+      cvt8(b_raw[it], b);
 #pragma unroll
       for (int k = 0; k < 8; ++k)
-        o[k] = (x[it][k] - mean) * rstd * TT<T>::safe(gs[it][k]) + TT<T>::safe(bs[it][k]);
+        o[k] = (x[it][k] - mean) * rstd * TT<T>::safe(g[k]) + TT<T>::safe(b[k]);
       if (MODE == kLnResOut) {
         st8(out_t, out_base + e, o);
       } else {
         uint2 packed;
-        packed.x = pack4_i8(float2int8(o[0], quant_scale), float2int8(o[1], quant_scale),
-                            float2int8(o[2], quant_scale), float2int8(o[3], quant_scale));
-        packed.y = pack4_i8(float2int8(o[4], quant_scale), float2int8(o[5], quant_scale),
-                            float2int8(o[6], quant_scale), float2int8(o[7], quant_scale));
+        packed.x = float2int8_pack4(o[0], o[1], o[2], o[3], quant_scale);
+        packed.y = float2int8_pack4(o[4], o[5], o[6], o[7], quant_scale);
         *reinterpret_cast<uint2*>(out_q + code_offset(row, e, hidden, blocked)) = packed;
-        float w[8];
+        if (!has_rb) zero8(rb_raw[it]);
+        float keep[8];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          float keep = is_post_ln ? o[k] : x[it][k];
-          w[k] = (MODE == kLnFirst) ? keep + rbs[it][k] : TT<T>::rnd(keep) + rbs[it][k];
+        for (int k = 0; k < 8; ++k) keep[k] = is_post_ln ? o[k] : x[it][k];
+        if (MODE == kLnFirst && sizeof(T) == 2) {
+          // the first norm's sum is a float's, rounded once
+          float rb[8];
+          cvt8(rb_raw[it], rb);
+#pragma unroll
+          for (int k = 0; k < 8; ++k) keep[k] += rb[k];
+          st8(residual, base + e, keep);
+        } else {
+          add8_store(residual, base + e, keep, rb_raw[it]);
         }
-        st8(residual, base + e, w);
       }
     }
   }

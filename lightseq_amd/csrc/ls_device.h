@@ -31,7 +31,10 @@ struct TT<__half> {
   __device__ static float ld(const __half* p, long i) { return __half2float(p[i]); }
   __device__ static void st(__half* p, long i, float v) { p[i] = __float2half_rn(v); }
   __device__ static float rnd(float v) { return __half2float(__float2half_rn(v)); }
-  __device__ static float safe(float v) { return fmaxf(fminf(100000.f, v), -100000.f); }
+  // max(min(100000, v), -100000) as one median: for a number the two agree, and for a NaN the
+  // median is the lesser bound -- negated on both sides, the upper one, as the two steps give.
+  // The signs are operand modifiers of the median and of the instruction that uses its result.
+  __device__ static float safe(float v) { return -__builtin_amdgcn_fmed3f(-v, -100000.f, 100000.f); }
 };
 
 // ---- scalar quantisers: inference/kernels/transformerKernels_int8.cc.cu:14-27
@@ -230,6 +233,8 @@ __device__ __forceinline__ float dpp_f(float x) {
 }
 constexpr int kDppXor1 = 0xB1;         // quad_perm [1,0,3,2]
 constexpr int kDppXor2 = 0x4E;         // quad_perm [2,3,0,1]
+constexpr int kDppXor3 = 0x1B;         // quad_perm [3,2,1,0]
+constexpr int kDppRor8 = 0x128;        // lane l of a row of 16 reads lane l ^ 8
 constexpr int kDppHalfMirror = 0x141;  // lane l of a row of 16 reads lane 7 - l of its half
 constexpr int kDppMirror = 0x140;      // ... lane 15 - l of its row
 __device__ __forceinline__ float lane_read(float v, int l) {
