@@ -19,23 +19,35 @@ constexpr int kPackMaxBatch = 1024;
 constexpr int kItemHeadShift = 16, kItemBlocksShift = 28;  // as in qkv_attn_kernels.hip
 }  // namespace
 
-// One workgroup: a wavefront per sequence finds the last token, then starts by a prefix sum, and
+// One workgroup: a wavefront per sequence finds the last token (COUNT: counts its tokens, what a
+// GPT model takes for the length of a text), then starts by a prefix sum, and
 // the work items of the fused QKV + attention kernel in the order that kernel wants (see
 // qkv_attn_plan_kernel).  Bound by two or three trips to memory.
+template <bool COUNT>
 __global__ void __launch_bounds__(1024)
 enc_pack_plan_kernel(const int* __restrict__ tokens, int padding_id, int* __restrict__ seq,
                      int* __restrict__ items, int batch, int S, int head_num,
-                     unsigned long long* host_rows, unsigned ticket) {
+                     unsigned long long* host_rows, unsigned ticket, int* real_len, float* ppl) {
   __shared__ int len[kPackMaxBatch], order[kPackMaxBatch];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   for (int b = wave; b < batch; b += 16) {
     int last = 0;
     const int* row = tokens + (long)b * S;
 #pragma unroll 4
-    for (int i = lane; i < S; i += 64) last = row[i] != padding_id ? i + 1 : last;
+    for (int i = lane; i < S; i += 64) {
+      const bool token = row[i] != padding_id;
+      last = COUNT ? last + token : token ? i + 1 : last;
+    }
 #pragma unroll
-    for (int m = 32; m > 0; m >>= 1) last = max(last, __shfl_xor(last, m, 64));
+    for (int m = 32; m > 0; m >>= 1) {
+      const int o = __shfl_xor(last, m, 64);
+      last = COUNT ? last + o : max(last, o);
+    }
     if (lane == 0) len[b] = last;
+    if (COUNT && lane == 0) {
+      real_len[b] = last;
+      ppl[b] = 0.f;
+    }
   }
   __syncthreads();
   if (wave == 0) {
@@ -57,6 +69,7 @@ enc_pack_plan_kernel(const int* __restrict__ tokens, int padding_id, int* __rest
       base += __shfl(sum, 63, 64);
     }
     if (lane == 0) {
+      padded &= !COUNT;
       seq[2 * batch] = padded ? base : -1;
       if (host_rows != nullptr)
         __hip_atomic_store(host_rows, (unsigned long long)ticket << 32 | (unsigned)(base + (padded ? 1 : 0)),
@@ -96,8 +109,17 @@ int enc_pack_plan(const int* tokens, int padding_id, const EncPack& pack, int ba
                   int head_num, unsigned long long* host_rows, unsigned ticket, hipStream_t s) {
   if (!tokens || !pack.seq || !pack.row_map || !enc_pack_supported(batch, seq_len, head_num))
     return lsh_fail(LSH_ERR_INVALID, "enc_pack_plan: bad arguments");
-  enc_pack_plan_kernel<<<1, 1024, 0, s>>>(tokens, padding_id, pack.seq, pack.items, batch, seq_len,
-                                          head_num, host_rows, ticket);
+  enc_pack_plan_kernel<false><<<1, 1024, 0, s>>>(tokens, padding_id, pack.seq, pack.items, batch,
+                                                 seq_len, head_num, host_rows, ticket, nullptr, nullptr);
+  return lsh_check_launch("enc_pack_plan_kernel");
+}
+
+int text_pack_plan(const int* tokens, int padding_id, int* seq, int* real_len, float* ppl, int batch,
+                   int seq_len, unsigned long long* host_rows, unsigned ticket, hipStream_t s) {
+  if (!tokens || !seq || !real_len || !ppl || !enc_pack_supported(batch, seq_len, 1))
+    return lsh_fail(LSH_ERR_INVALID, "text_pack_plan: bad arguments");
+  enc_pack_plan_kernel<true><<<1, 1024, 0, s>>>(tokens, padding_id, seq, nullptr, batch, seq_len, 1,
+                                                host_rows, ticket, real_len, ppl);
   return lsh_check_launch("enc_pack_plan_kernel");
 }
 

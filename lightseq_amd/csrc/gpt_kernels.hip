@@ -23,11 +23,18 @@ template <typename T>
 __global__ void __launch_bounds__(256)
 gpt_embedding_kernel(const int8_t* __restrict__ token_emb, const T* __restrict__ pos_emb,
                      const int* __restrict__ token_id, T* __restrict__ output, int padding_id,
-                     int pos_offset, float dequant_scale, int seq_len, int hidden, int vocab) {
+                     int pos_offset, float dequant_scale, int seq_len, int hidden, int vocab,
+                     const int* __restrict__ seq) {
 #pragma clang fp contract(off)
-  const long pos = blockIdx.x;  // batch * seq_len + s
-  const int s = (int)(pos % seq_len);
-  int tid = token_id[pos];
+  const long at = blockIdx.x;  // batch * seq_len + s
+  const int s = (int)(at % seq_len);
+  long pos = at;  // the row it goes to
+  if (seq != nullptr) {
+    const int b = (int)(at / seq_len);
+    if (s >= seq[2 * b + 1]) return;
+    pos = seq[2 * b] + s;
+  }
+  int tid = token_id[at];
   if (tid == padding_id) {
     for (int i = threadIdx.x; i < hidden; i += blockDim.x) TT<T>::st(output, pos * hidden + i, 0.f);
     return;
@@ -89,7 +96,7 @@ template <typename T>
 int gpt_embedding_i8I(int batch_size, int batch_seq_len, int hidden_size, hipStream_t s,
                       const int8_t* token_emb, const T* pos_emb, const int* token_id, T* output,
                       int* real_seq_len, int padding_id, int pos_offset, float dequant_scale,
-                      int vocab_size, int max_step, int* zero_flag) {
+                      int vocab_size, int max_step, int* zero_flag, const int* seq) {
   if (!token_emb || !pos_emb || !token_id || !output || !real_seq_len || batch_size <= 0 ||
       batch_seq_len <= 0 || hidden_size <= 0)
     return lsh_fail(LSH_ERR_INVALID, "ker_gpt_embedding_i8I: bad arguments");
@@ -97,7 +104,7 @@ int gpt_embedding_i8I(int batch_size, int batch_seq_len, int hidden_size, hipStr
     return lsh_fail(LSH_ERR_INVALID, "ker_gpt_embedding_i8I: position outside the table");
   const bool aligned = ((reinterpret_cast<uintptr_t>(token_emb) | reinterpret_cast<uintptr_t>(pos_emb) |
                          reinterpret_cast<uintptr_t>(output)) & 15u) == 0;
-  if (batch_seq_len == 1 && hidden_size % 4 == 0 && aligned) {
+  if (batch_seq_len == 1 && hidden_size % 4 == 0 && aligned && !seq) {
     gpt_embedding_step_kernel<T><<<batch_size, 256, 0, s>>>(
         token_emb, pos_emb, token_id, output, real_seq_len, zero_flag, padding_id, pos_offset,
         dequant_scale, hidden_size, vocab_size);
@@ -107,16 +114,19 @@ int gpt_embedding_i8I(int batch_size, int batch_seq_len, int hidden_size, hipStr
     if (int rc = fill_i32(zero_flag, 0, 1, s)) return rc;
   gpt_embedding_kernel<T><<<batch_size * batch_seq_len, 256, 0, s>>>(
       token_emb, pos_emb, token_id, output, padding_id, pos_offset, dequant_scale, batch_seq_len,
-      hidden_size, vocab_size);
+      hidden_size, vocab_size, seq);
   if (int rc = lsh_check_launch("gpt_embedding_kernel")) return rc;
+  if (seq != nullptr) return LSH_OK;
   gpt_count_tokens_kernel<<<batch_size, 256, 0, s>>>(token_id, real_seq_len, padding_id,
                                                      batch_seq_len);
   return lsh_check_launch("gpt_count_tokens_kernel");
 }
 template int gpt_embedding_i8I<float>(int, int, int, hipStream_t, const int8_t*, const float*,
-                                      const int*, float*, int*, int, int, float, int, int, int*);
+                                      const int*, float*, int*, int, int, float, int, int, int*,
+                                      const int*);
 template int gpt_embedding_i8I<__half>(int, int, int, hipStream_t, const int8_t*, const __half*,
-                                       const int*, __half*, int*, int, int, float, int, int, int*);
+                                       const int*, __half*, int*, int, int, float, int, int, int*,
+                                       const int*);
 
 // ---------------------------------------------------------------------------------
 // prompt pass: int8 QKV GEMM output [tokens, 3H] + bias -> requantised with the cache
@@ -859,13 +869,14 @@ template <bool ALIGNED>
 __global__ void __launch_bounds__(1024)
 ppl_terms_kernel(const int8_t* __restrict__ logits, long ldl, const int* __restrict__ input_ids,
                  const int* __restrict__ real_seq_len, float* __restrict__ terms, int vocab,
-                 int seq_len, float dq) {
+                 int seq_len, float dq, const int* __restrict__ seq) {
   __shared__ float red[16];
   const int b = blockIdx.y, s = blockIdx.x;
   const int len = real_seq_len[b];
   if (s >= len - 1) return;  // (uniform: no term, nothing read by the sum)
   const long tok = (long)b * seq_len + s;
-  const float t = ppl_term<ALIGNED>(logits + tok * ldl, input_ids[tok + 1], len, vocab, dq, red);
+  const long row = seq != nullptr ? seq[2 * b] + s : tok;
+  const float t = ppl_term<ALIGNED>(logits + row * ldl, input_ids[tok + 1], len, vocab, dq, red);
   if (threadIdx.x == 0) terms[tok] = t;
 }
 
@@ -890,7 +901,7 @@ ppl_sum_kernel(const float* __restrict__ terms, const int* __restrict__ real_seq
 
 int ppl_i8I(int batch_size, int batch_seq_len, hipStream_t s, const int8_t* logits,
             const int* input_ids, const int* real_seq_len, float* ppl, int vocab_size,
-            float dequant_scale, float* workspace, int logits_stride) {
+            float dequant_scale, float* workspace, int logits_stride, const int* seq) {
   if (!logits || !input_ids || !real_seq_len || !ppl || batch_size <= 0 || batch_seq_len <= 0 ||
       vocab_size <= 0)
     return lsh_fail(LSH_ERR_INVALID, "ker_ppl_i8I: bad arguments");
@@ -901,16 +912,16 @@ int ppl_i8I(int batch_size, int batch_seq_len, hipStream_t s, const int8_t* logi
     const dim3 grid(batch_seq_len, batch_size);
     if (aligned)
       ppl_terms_kernel<true><<<grid, 1024, 0, s>>>(logits, ldl, input_ids, real_seq_len, workspace,
-                                                   vocab_size, batch_seq_len, dequant_scale);
+                                                   vocab_size, batch_seq_len, dequant_scale, seq);
     else
       ppl_terms_kernel<false><<<grid, 1024, 0, s>>>(logits, ldl, input_ids, real_seq_len, workspace,
-                                                    vocab_size, batch_seq_len, dequant_scale);
+                                                    vocab_size, batch_seq_len, dequant_scale, seq);
     if (int rc = lsh_check_launch("ppl_terms_kernel")) return rc;
     ppl_sum_kernel<<<batch_size, 64, 0, s>>>(workspace, real_seq_len, ppl, batch_seq_len);
     return lsh_check_launch("ppl_sum_kernel");
   }
-  if (logits_stride && logits_stride != vocab_size)
-    return lsh_fail(LSH_ERR_UNSUPPORTED, "ker_ppl_i8I: padded rows need the workspace");
+  if (seq || (logits_stride && logits_stride != vocab_size))
+    return lsh_fail(LSH_ERR_UNSUPPORTED, "ker_ppl_i8I: padded or planned rows need the workspace");
   if (aligned)
     ppl_kernel<true><<<batch_size, 1024, 0, s>>>(logits, input_ids, real_seq_len, ppl, vocab_size,
                                                  batch_seq_len, dequant_scale);

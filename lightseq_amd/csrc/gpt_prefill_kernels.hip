@@ -41,7 +41,8 @@ __global__ void __launch_bounds__(256)
 gpt_arrange_qkv_prefill_i8_kernel(const int8_t* __restrict__ ori, const __half* __restrict__ bias,
                                   int8_t* __restrict__ q_codes, int8_t* __restrict__ k_cache,
                                   int8_t* __restrict__ v_cache, int seq_len, int d, int head_num,
-                                  int groups, int max_step, float ds, float qs) {
+                                  int groups, int max_step, float ds, float qs,
+                                  const int* __restrict__ seq) {
 #pragma clang fp contract(off)
   const int hidden = d * head_num;
   const int grp = blockIdx.x % groups, which = (blockIdx.x / groups) % 3;
@@ -59,22 +60,25 @@ gpt_arrange_qkv_prefill_i8_kernel(const int8_t* __restrict__ ori, const __half* 
       bv[8 + k] = __half2float(b1.v[k]);
     }
   }
-  const int8_t* src = ori + ((long)b * seq_len * 3 + which) * hidden + col;
+  // the rows of sequence b: first and number (a plan has only those that are not padding)
+  const long row0 = seq != nullptr ? seq[2 * b] : (long)b * seq_len;
+  const int n = seq != nullptr ? seq[2 * b + 1] : seq_len;
+  const int8_t* src = ori + (row0 * 3 + which) * hidden + col;
   const long bh = (long)b * head_num + head;
   int8_t* dst = which == 0   ? q_codes + bh * seq_len * d + dim
                 : which == 1 ? k_cache + bh * max_step * d + dim
                              : v_cache + bh * max_step * d + dim;
-  for (int s0 = row; s0 < seq_len; s0 += 32 * UNR) {
+  for (int s0 = row; s0 < n; s0 += 32 * UNR) {
     uint4 w[UNR];
 #pragma unroll
     for (int u = 0; u < UNR; ++u) {
-      const int s = min(s0 + 32 * u, seq_len - 1);
+      const int s = min(s0 + 32 * u, n - 1);
       w[u] = *reinterpret_cast<const uint4*>(src + (long)s * 3 * hidden);
     }
 #pragma unroll
     for (int u = 0; u < UNR; ++u) {
       const int s = s0 + 32 * u;
-      if (s >= seq_len) break;
+      if (s >= n) break;
       const uint32_t wi[4] = {w[u].x, w[u].y, w[u].z, w[u].w};
       uint32_t o[4];
 #pragma unroll
@@ -108,7 +112,7 @@ int gpt_arrange_qkv_prefill_i8(int batch_token_num, int hidden_size, hipStream_t
                                const int8_t* ori_qkv, const __half* qkv_bias, int8_t* q_codes,
                                int8_t* k_cache, int8_t* v_cache, int batch_seq_len,
                                int dim_per_head, int head_num, int max_step, float dequant_scale,
-                               float quant_scale) {
+                               float quant_scale, const int* seq) {
   if (!ori_qkv || !qkv_bias || !q_codes || !k_cache || !v_cache || batch_token_num <= 0 ||
       batch_seq_len <= 0 || batch_token_num % batch_seq_len != 0 || dim_per_head <= 0 ||
       hidden_size != dim_per_head * head_num || batch_seq_len > max_step)
@@ -128,11 +132,11 @@ int gpt_arrange_qkv_prefill_i8(int batch_token_num, int hidden_size, hipStream_t
   if (batch_seq_len > 64)
     gpt_arrange_qkv_prefill_i8_kernel<4><<<batch * 3 * groups, 256, 0, s>>>(
         ori_qkv, qkv_bias, q_codes, k_cache, v_cache, batch_seq_len, dim_per_head, head_num, groups,
-        max_step, dequant_scale, quant_scale);
+        max_step, dequant_scale, quant_scale, seq);
   else
     gpt_arrange_qkv_prefill_i8_kernel<2><<<batch * 3 * groups, 256, 0, s>>>(
         ori_qkv, qkv_bias, q_codes, k_cache, v_cache, batch_seq_len, dim_per_head, head_num, groups,
-        max_step, dequant_scale, quant_scale);
+        max_step, dequant_scale, quant_scale, seq);
   return lsh_check_launch("gpt_arrange_qkv_prefill_i8_kernel");
 }
 
@@ -151,11 +155,11 @@ __global__ void __launch_bounds__(256, 2)
 gpt_prefill_attn_i8_kernel(const int8_t* __restrict__ q_codes, const int8_t* __restrict__ k_cache,
                            const int8_t* __restrict__ v_cache, const int* __restrict__ real_seq_len,
                            int8_t* __restrict__ ctx_q, float quant_scale, float v_quant_scale,
-                           int S, int head_num, int max_step, float alpha, float dq, int BH,
-                           int blocked) {
+                           int seq_len, int head_num, int max_step, float alpha, float dq, int BH,
+                           int blocked, const int* __restrict__ seq) {
   constexpr int D = 64, VSTR = kPfVstr;
   extern __shared__ __align__(16) int8_t smem[];
-  const int nkb_max = (S + 127) / 128;
+  const int nkb_max = (seq_len + 127) / 128;
   int8_t* Ks = smem;
   _Float16* Vt0 = reinterpret_cast<_Float16*>(smem + (size_t)nkb_max * 128 * 64);
   _Float16* tabh = Vt0 + 2 * 64 * VSTR;
@@ -166,8 +170,11 @@ gpt_prefill_attn_i8_kernel(const int8_t* __restrict__ q_codes, const int8_t* __r
   const int qb = nkb_max - 1 - (int)(blockIdx.x / BH), bh = blockIdx.x % BH;
   const int b = bh / head_num, head = bh % head_num;
   const int nkb = qb + 1;  // key blocks 0 .. qb (causal)
+  // rows of a plan: the sequence's positions are its first S only
+  const int S = seq != nullptr ? __builtin_amdgcn_readfirstlane(seq[2 * b + 1]) : seq_len;
+  if (qb * 128 >= S) return;
   const int qi = qb * 128 + wave * 32 + l32;
-  const int8_t* qbase = q_codes + (long)bh * S * D;
+  const int8_t* qbase = q_codes + (long)bh * seq_len * D;
   const int8_t* kbase = k_cache + (long)bh * max_step * D;
   const int8_t* vbase = v_cache + (long)bh * max_step * D;
 
@@ -320,7 +327,7 @@ gpt_prefill_attn_i8_kernel(const int8_t* __restrict__ q_codes, const int8_t* __r
   }
 
   if (qi >= S) return;
-  const long tok = (long)b * S + qi;
+  const long tok = (seq != nullptr ? (long)seq[2 * b] : (long)b * seq_len) + qi;
   const int hidden = head_num * D;
 #pragma unroll
   for (int db = 0; db < D / 32; ++db) {
@@ -341,7 +348,7 @@ int gpt_prefill_attention_i8(const int8_t* q_codes, const int8_t* k_cache, const
                              const int* real_seq_len, int8_t* ctx_q, float quant_scale,
                              float dequant_scale, float v_quant_scale, int batch, int seq_len,
                              int head_num, int dim_per_head, int max_step, hipStream_t s,
-                             bool blocked) {
+                             bool blocked, const int* seq) {
   if (batch <= 0 || seq_len <= 0 || head_num <= 0 || !q_codes || !k_cache || !v_cache ||
       !real_seq_len || !ctx_q || seq_len > max_step || !(v_quant_scale > 0.f))
     return lsh_fail(LSH_ERR_INVALID, "gpt_prefill_attention_i8: bad arguments");
@@ -375,7 +382,7 @@ int gpt_prefill_attention_i8(const int8_t* q_codes, const int8_t* k_cache, const
   const float alpha = __half2float(__float2half_rn(sqrtf(1.f / (float)dim_per_head)));
   gpt_prefill_attn_i8_kernel<<<(int)(BH * nqb), 256, gpt_prefill_lds_bytes(seq_len), s>>>(
       q_codes, k_cache, v_cache, real_seq_len, ctx_q, quant_scale, v_quant_scale, seq_len, head_num,
-      max_step, alpha, dequant_scale, (int)BH, blocked);
+      max_step, alpha, dequant_scale, (int)BH, blocked, seq);
   return lsh_check_launch("gpt_prefill_attn_i8_kernel");
 }
 

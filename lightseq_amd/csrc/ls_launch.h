@@ -192,6 +192,12 @@ bool enc_pack_supported(int batch, int seq_len, int head_num);
 // of rows, for a host that waits for this plan.
 int enc_pack_plan(const int* tokens, int padding_id, const EncPack& pack, int batch, int seq_len,
                   int head_num, unsigned long long* host_rows, unsigned ticket, hipStream_t s);
+// The plan of whole texts for a GPT model: the rows are the first n positions of every text, n the
+// number of its tokens that are not padding (causal: no later position reaches them, and their
+// terms are all a perplexity has).  seq[2 * b], seq[2 * b + 1]: first row and n, real_len[b]: n,
+// ppl[b]: 0.  host_rows: as above.
+int text_pack_plan(const int* tokens, int padding_id, int* seq, int* real_len, float* ppl, int batch,
+                   int seq_len, unsigned long long* host_rows, unsigned ticket, hipStream_t s);
 // launch_enc_emb_i8I into the rows of the plan; pad_mask keeps its [batch, seq_len] form
 int enc_emb_packed(const int8_t* token_emb, const __half* pos_emb, const int* tokens, __half* output,
                    int* pad_mask, int padding_id, const EncPack& pack, int batch, int seq_len,
@@ -464,9 +470,10 @@ template <typename T>
 int gpt_embedding_i8I(int batch_size, int batch_seq_len, int hidden_size, hipStream_t s,
                       const int8_t* token_emb, const T* pos_emb, const int* token_id, T* output,
                       int* real_seq_len, int padding_id, int pos_offset, float dequant_scale,
-                      int vocab_size, int max_step, int* zero_flag = nullptr);
+                      int vocab_size, int max_step, int* zero_flag = nullptr,
+                      const int* seq = nullptr);
 // zero_flag: when given, the int it points to is cleared by the same launch (a generation
-// step's "unfinished" flag)
+// step's "unfinished" flag).  seq: a plan of text_pack_plan, which has also counted the tokens
 int gpt_arrange_qkv_prefill_f16(int batch_token_num, int hidden_size, hipStream_t s,
                                 const int8_t* ori_qkv, const __half* qkv_bias, __half* q_codes,
                                 __half* k_codes, __half* v_deq, int8_t* k_cache, int8_t* v_cache,
@@ -487,12 +494,13 @@ int gpt_arrange_qkv_prefill_i8(int batch_token_num, int hidden_size, hipStream_t
                                const int8_t* ori_qkv, const __half* qkv_bias, int8_t* q_codes,
                                int8_t* k_cache, int8_t* v_cache, int batch_seq_len,
                                int dim_per_head, int head_num, int max_step, float dequant_scale,
-                               float quant_scale);
+                               float quant_scale, const int* seq = nullptr);
+// seq (here and below): the product's / the context's rows are those of a plan of text_pack_plan
 int gpt_prefill_attention_i8(const int8_t* q_codes, const int8_t* k_cache, const int8_t* v_cache,
                              const int* real_seq_len, int8_t* ctx_q, float quant_scale,
                              float dequant_scale, float v_quant_scale, int batch, int seq_len,
                              int head_num, int dim_per_head, int max_step, hipStream_t s,
-                             bool blocked = false);
+                             bool blocked = false, const int* seq = nullptr);
 template <typename T>
 int correlation_softmax_gpt_i32I(int batch_size, int batch_seq_len, int head_num, hipStream_t s,
                                  const int32_t* correlation, T* output, const int* real_seq_len,
@@ -543,9 +551,10 @@ int gpt_greedy_step(const int8_t* logits, int* ids, int* last_ids, int vocab_siz
                     int logits_stride);
 int ppl_i8I(int batch_size, int batch_seq_len, hipStream_t s, const int8_t* logits,
             const int* input_ids, const int* real_seq_len, float* ppl, int vocab_size,
-            float dequant_scale, float* workspace = nullptr, int logits_stride = 0);
+            float dequant_scale, float* workspace = nullptr, int logits_stride = 0,
+            const int* seq = nullptr);
 // workspace: batch * seq_len floats -> one workgroup per position; it also allows rows of logits
-// that lie logits_stride codes apart (0: vocab_size)
+// that lie logits_stride codes apart (0: vocab_size), and those of a plan of text_pack_plan (seq)
 
 // ---- operator kernels of the csrc layer path (layer_ops.hip); clip values are device
 // ---- scalars of type T, dropout ratios must be 0 -------------------------------------

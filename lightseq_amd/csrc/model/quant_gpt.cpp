@@ -39,7 +39,7 @@ void QuantGpt::Infer() {
   if (input_shapes_[0].size() != 2) throw std::runtime_error("token_ids must be 2-D");
   int batch_size = input_shapes_[0][0], seq_len = input_shapes_[0][1];
   if (is_ppl()) {
-    encoder_->run_one_infer(batch_size, seq_len);
+    encoder_->run_one_infer(batch_size, seq_len, host_ids_);
     CHECK_GPU_ERROR(hipStreamSynchronize(stream_));
     set_output_shape(0, {batch_size});
   } else if (tw_._sampling_method == "topk" || tw_._sampling_method == "topp") {
@@ -59,6 +59,7 @@ void QuantGpt::InferHost(const int* ids, int batch, int seq_len, void* host_out,
     h_ids_.upload(ids, n, d_input_.get(), d_input_.size(), stream_);
   set_input_ptr(0, d_input_.get());
   set_input_shape(0, {batch, seq_len});
+  HostIdsScope scope(host_ids_, ids);
   Infer();
 }
 

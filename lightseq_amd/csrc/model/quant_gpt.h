@@ -30,6 +30,7 @@ class QuantGpt : public LSModel {
   // owners first: released after the encoder, also when the constructor throws half way
   StreamOwner stream_;
   HostIds h_ids_;
+  const int* host_ids_ = nullptr;  // the ids of an InferHost() call under way
   DeviceBuffer<int> d_input_, d_sample_id;
   DeviceBuffer<float> d_ppl;
   std::shared_ptr<QuantGptEncoder> encoder_;

@@ -59,6 +59,7 @@ void QuantGptEncoder::init_buffer() {
   const int V = _tw._src_vocab_size;
   const size_t tokens = (size_t)_max_batch_size * _tw._max_step;
   _real_seq_len.alloc(_max_batch_size);
+  _pack_seq.alloc(2 * (size_t)_max_batch_size + 1);
   _ids.alloc(tokens);
   _last_ids.alloc(_max_batch_size);
   _unfinished.alloc(1);
@@ -175,18 +176,48 @@ void QuantGptEncoder::ffn_add_norm(int rows, int8_t* in, int8_t* tmp, bool block
   TAP("res_out", _query[_res].get(), (size_t)rows * H * sizeof(__half));
 }
 
+// A perplexity has no use for the rows of padded positions: where the whole pass can do without
+// them, it computes those of text_pack_plan (0.62 of them with lengths uniform between a quarter
+// and the whole of the longest).  A generation's steps read the caches of all positions.
+bool QuantGptEncoder::packed_route() const {
+  return _ops.blocked && gpt_prefill_i8_enabled() && _tw._hidden_size % 128 == 0 &&
+         gpt_prefill_i8_supported(_batch_seq_len, _tw._head_num, _tw._dim_per_head) &&
+         enc_pack_supported(_batch_size, _batch_seq_len, 1);
+}
+
+// the rows of the plan: counted here, or as the plan counted them (the device embeds and
+// normalises the first layer's rows meanwhile)
+int QuantGptEncoder::count_rows(const int* host_token_ids) const {
+  if (!host_token_ids) return _rows_notice.wait(_stream);
+  int rows = 0;
+  for (int i = 0; i < _batch_size * _batch_seq_len; ++i) rows += host_token_ids[i] != _tw._padding_id;
+  return rows;
+}
+
 // all prompt positions at once (:253-291 / :299-341); leaves the int8 LayerNorm output of
-// the last layer in _buf_a, row-major where the caller picks positions from it
-void QuantGptEncoder::prompt_pass(const int* ids, bool row_major_out) {
-  const int H = _tw._hidden_size, M = _batch_token_num;
+// the last layer in _buf_a, row-major where the caller picks positions from it.  packed: the rows
+// are those of the plan, and _batch_token_num is their number afterwards.
+void QuantGptEncoder::prompt_pass(const int* ids, bool row_major_out, bool packed,
+                                  const int* host_token_ids) {
+  const int H = _tw._hidden_size;
+  int M = _batch_token_num;
+  const int* seq = packed ? _pack_seq.get() : nullptr;
   const float Q = _quant_range;
   _res = 0;
   _tap_step = -2;
-  CHECK_GPU_ERROR(hipMemsetAsync(_real_seq_len.get(), 0, sizeof(int) * _batch_size, _stream));
+  if (packed) {
+    const StepNotice n = host_token_ids ? StepNotice{} : _rows_notice.next(nullptr);
+    LSH_CALL(text_pack_plan(ids, _tw._padding_id, _pack_seq.get(), _real_seq_len.get(), _p_d_ppl,
+                            _batch_size, _batch_seq_len, n.slot, n.tag, _stream));
+  } else {
+    CHECK_GPU_ERROR(hipMemsetAsync(_real_seq_len.get(), 0, sizeof(int) * _batch_size, _stream));
+  }
   LSH_CALL(gpt_embedding_i8I<__half>(_batch_size, _batch_seq_len, H, _stream, _int8_emb.get(),
                                      _pos_emb.get(), ids, _query[_res].get(), _real_seq_len.get(),
                                      _tw._padding_id, 0, _src_emb_clip_max / Q,
-                                     _tw._src_vocab_size, _tw._max_step));
+                                     _tw._src_vocab_size, _tw._max_step, nullptr, seq));
+  // until the number of rows is known, launches cover the most there can be
+  if (packed && host_token_ids) M = _batch_token_num = std::max(1, count_rows(host_token_ids));
   int8_t *a = _buf_a.get(), *b = _buf_b.get();
   __half* qc = _qkv_buf.get();
   __half* kc = qc + _max_batch_dim;
@@ -201,6 +232,8 @@ void QuantGptEncoder::prompt_pass(const int* ids, bool row_major_out) {
       LSH_CALL(norm_layer_resual_i8O<__half>(M, H, _stream, _query[_res].get(), a, w.ln1_scale.get(),
                                              w.ln1_bias.get(), w.b_out.get(), Q / c[4], false,
                                              _ops.blocked));
+    if (packed && !host_token_ids && _layer_id == 0)
+      M = _batch_token_num = std::max(1, count_rows(nullptr));
     _ops.i8o(a, w.w_qkv.get(), b, M, 3 * H, H, c[0] * c[4] / (c[8] * Q), _stream);
     int8_t* k_cache = _self_k_cache.get() + (size_t)_layer_id * _max_batch_dim;
     int8_t* v_cache = _self_v_cache.get() + (size_t)_layer_id * _max_batch_dim;
@@ -208,13 +241,13 @@ void QuantGptEncoder::prompt_pass(const int* ids, bool row_major_out) {
       // int8 end to end: q codes and the caches are all the arrange stage writes, and the
       // attention reads them
       int8_t* q8 = reinterpret_cast<int8_t*>(qc);
-      LSH_CALL(gpt_arrange_qkv_prefill_i8(M, H, _stream, b, w.b_qkv.get(), q8, k_cache, v_cache,
-                                          _batch_seq_len, _tw._dim_per_head, _tw._head_num,
-                                          _tw._max_step, c[8] / Q, Q / c[11]));
+      LSH_CALL(gpt_arrange_qkv_prefill_i8(_batch_size * _batch_seq_len, H, _stream, b,
+                                          w.b_qkv.get(), q8, k_cache, v_cache, _batch_seq_len, _tw._dim_per_head, _tw._head_num,
+                                          _tw._max_step, c[8] / Q, Q / c[11], seq));
       LSH_CALL(gpt_prefill_attention_i8(q8, k_cache, v_cache, _real_seq_len.get(), a, Q / c[5],
                                         c[11] / Q, Q / c[11], _batch_size, _batch_seq_len,
                                         _tw._head_num, _tw._dim_per_head, _tw._max_step, _stream,
-                                        _ops.blocked));
+                                        _ops.blocked, seq));
     } else {
       LSH_CALL(gpt_arrange_qkv_prefill_f16(M, H, _stream, b, w.b_qkv.get(), qc, kc, vd, k_cache,
                                            v_cache, _batch_seq_len, _tw._dim_per_head,
@@ -471,7 +504,7 @@ int QuantGptEncoder::run_one_sample(int batch_size, int batch_seq_len) {
   return _batch_seq_len;
 }
 
-void QuantGptEncoder::run_one_infer(int batch_size, int batch_seq_len) {
+void QuantGptEncoder::run_one_infer(int batch_size, int batch_seq_len, const int* host_token_ids) {
   if (batch_size > _max_batch_size)
     throw std::runtime_error("batch size of input greater than max_batch_size");
   if (batch_seq_len > _tw._max_step)
@@ -483,14 +516,16 @@ void QuantGptEncoder::run_one_infer(int batch_size, int batch_seq_len) {
   _batch_seq_len = batch_seq_len;
   _batch_token_num = batch_size * batch_seq_len;
   const int V = _tw._src_vocab_size;
-  CHECK_GPU_ERROR(hipMemsetAsync(_p_d_ppl, 0, sizeof(float) * batch_size, _stream));
-  prompt_pass(_p_d_token_id, false);
+  const bool packed = packed_route();
+  if (!packed) CHECK_GPU_ERROR(hipMemsetAsync(_p_d_ppl, 0, sizeof(float) * batch_size, _stream));
+  prompt_pass(_p_d_token_id, false, packed, host_token_ids);
   /* compute_ppl (:781-797) */
   logits_product(_buf_a.get(), _batch_token_num);
   // the FFN2 accumulator buffer (tokens * hidden int32, idle by now) holds the per-position terms
   LSH_CALL(ppl_i8I(batch_size, batch_seq_len, _stream, _logits.get(), _p_d_token_id,
                    _real_seq_len.get(), _p_d_ppl, V, _logits_clip_max / _quant_range,
-                   reinterpret_cast<float*>(_int32_ffn_out_buf.get()), _logits_stride));
+                   reinterpret_cast<float*>(_int32_ffn_out_buf.get()), _logits_stride,
+                   packed ? _pack_seq.get() : nullptr));
 }
 
 }  // namespace hip

@@ -30,7 +30,8 @@ class QuantGptEncoder {
   ~QuantGptEncoder();
   void init_buffer();
   std::string check();
-  void run_one_infer(int batch_size, int batch_seq_len);  // perplexity
+  // perplexity; host_token_ids: the ids, where the caller has them in host memory too
+  void run_one_infer(int batch_size, int batch_seq_len, const int* host_token_ids = nullptr);
   int run_one_sample(int batch_size, int batch_seq_len);  // returns the sampled length
   void benchmark_mode(bool is_benchmark) { _is_benchmark = is_benchmark; }
   // Random sampling (topk > 1, topp): restart the per-sequence generator states from `seed`
@@ -60,7 +61,10 @@ class QuantGptEncoder {
   int* _p_d_sample_id;
 
  private:
-  void prompt_pass(const int* ids, bool row_major_out);
+  void prompt_pass(const int* ids, bool row_major_out, bool packed = false,
+                   const int* host_token_ids = nullptr);
+  bool packed_route() const;
+  int count_rows(const int* host_token_ids) const;
   void step_begin(lsh::StepNotice notice);
   bool emb_ln_fused() const;
   void step_layers(int from, int to);
@@ -82,12 +86,13 @@ class QuantGptEncoder {
   bool _use_graphs = false;
   StepGraphs _graphs;
 
-  int _batch_size = 0, _batch_seq_len = 0, _batch_token_num = 0, _batch_max_seq_len = 0;
+  int _batch_size = 0, _batch_seq_len = 0, _batch_max_seq_len = 0;
+  int _batch_token_num = 0;  // rows of the prompt pass
   int _layer_id = 0, _steps_run = 0;
   PhaseEvents _phases;
   long _max_batch_dim;
   int* _h_unfinished = nullptr;  // pinned
-  HostNotice _notice;
+  HostNotice _notice, _rows_notice;
   struct {                       // the step being enqueued
     int8_t *a, *b;               // a: input, then output of a layer
     bool qkv_attn, ln1_blocked, ln_in_product;
@@ -97,6 +102,7 @@ class QuantGptEncoder {
   int _tap_step = -2;  // the cached step being enqueued (tokens sampled so far), -2 outside one
   int _rec_max_steps = 0;
 
+  DeviceBuffer<int> _pack_seq;  // the plan of a perplexity call (text_pack_plan)
   DeviceBuffer<int> _real_seq_len, _ids, _last_ids, _unfinished;
   DeviceBuffer<long long> _sample_state;  // lsh_rng_state_t [max_batch_size]
   // the residual stream; the second one holds a few rows of a step whose layer norms are made by
