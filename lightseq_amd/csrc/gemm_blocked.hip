@@ -166,6 +166,23 @@ int gemm_blk_decself_qkv(const int8_t* A, const int8_t* W, const __half* qkv_bia
   return dispatch_blk<KwI8, EpiDecQkvI8, false>(A, W, epi, step_token_num, 3 * hidden, K, s);
 }
 
+int gemm_blk_prompt_qkv(const int8_t* A, const int8_t* W, const __half* qkv_bias, int8_t* q_codes,
+                        int8_t* k_cache, int8_t* v_cache, int rows, int hidden, int batch, int seq_len,
+                        int head_num, int max_step, const int* row_map, float alpha, float dequant_scale,
+                        float quant_scale, hipStream_t s) {
+  if (!qkv_bias || !q_codes || !k_cache || !v_cache || head_num <= 0 || hidden <= 0 ||
+      hidden % head_num != 0 || batch <= 0 || seq_len <= 0 || seq_len > max_step ||
+      rows > (long)batch * seq_len)
+    return lsh_fail(LSH_ERR_INVALID, "blocked gemm (prompt qkv): bad arguments");
+  const int d = hidden / head_num;
+  if (d % 16 != 0 || hidden >= (1 << 20) || (long)batch * seq_len >= (1 << 22))
+    return lsh_fail(LSH_ERR_UNSUPPORTED, "blocked gemm (prompt qkv): needs dim_per_head % 16 == 0");
+  const EpiPromptQkvI8 epi{q_codes, k_cache, v_cache, qkv_bias, row_map, alpha, dequant_scale, quant_scale,
+                           hidden, head_num, d, max_step, seq_len, 1.0f / (float)hidden,
+                           1.0f / (float)d, 1.0f / (float)seq_len};
+  return dispatch_blk<KwI8, EpiPromptQkvI8, true>(A, W, epi, rows, 3 * hidden, hidden, s);
+}
+
 int gemm_blk_encdec_q(const int8_t* A, const int8_t* W, const __half* q_bias, __half* new_q,
                       int step_token_num, int hidden, int K, int beam_size, int head_num, float alpha,
                       float dequant_scale, hipStream_t s, const LnStep* ln) {

@@ -135,6 +135,68 @@ struct EpiDecQkvI8 {
   static const char* name() { return "EpiDecQkvI8"; }
 };
 
+// QKV product of a GPT prompt pass followed by gpt_arrange_qkv_prefill_i8, with the same bits: code
+// -> code * dq + bias -> requantised with the cache clip -> query codes [batch, head, seq, d], key
+// and value codes into the caches [batch, head, max_step, d].  row_map: the position b * seq + s
+// that a row holds, where the rows are those of a plan.  The stand-alone launch reads and writes
+// all the codes once more and is one of nine launches of a layer: 10.3 us for 3072 rows of 3 x 1024.
+struct EpiPromptQkvI8 {
+  static constexpr bool kTable = false, kBlockedOut = false;
+  int8_t *q, *k, *v;
+  const __half* bias;
+  const int* row_map;
+  float alpha, dequant_scale, quant_scale;
+  int hidden, head_num, dim, max_step, seq;
+  float inv_hidden, inv_dim, inv_seq;
+  struct Col {
+    int8_t* base;
+    int head, steps;
+    half4_t b;
+  };
+  __device__ __forceinline__ Col at(int n) const {
+    const int part = div_by(n, hidden, inv_hidden), i = n - part * hidden;
+    const int head = div_by(i, dim, inv_dim);
+    return Col{(part == 0 ? q : part == 1 ? k : v) + (i - head * dim), head, part == 0 ? seq : max_step, {}};
+  }
+  __device__ __forceinline__ Col column(int n, int) const {
+    Col c = at(n);
+    c.b = *reinterpret_cast<const half4_t*>(bias + n);
+    return c;
+  }
+  __device__ __forceinline__ int8_t* row_ptr(const Col& col, int m) const {
+    const int p = row_map != nullptr ? row_map[m] : m;
+    const int b = div_by(p, seq, inv_seq), s = p - b * seq;
+    return col.base + ((long)(b * head_num + col.head) * col.steps + s) * dim;
+  }
+  __device__ __forceinline__ float value(int acc, __half b) const {
+#pragma clang fp contract(off)
+    return floorf(requant_acc_clamped(acc, alpha)) * dequant_scale + __half2float(b);
+  }
+  __device__ __forceinline__ void store4(int m, int, int, const Col& col, const v4i& c) const {
+    *reinterpret_cast<uint32_t*>(row_ptr(col, m)) =
+        float2int8_pack4(value(c[0], col.b.v[0]), value(c[1], col.b.v[1]), value(c[2], col.b.v[2]),
+                         value(c[3], col.b.v[3]), quant_scale);
+  }
+  // 16 columns of one head (dim % 16 == 0)
+  __device__ __forceinline__ void store16(long m, int n, int, const v16i& c, bool) const {
+    const half8_t b0 = *reinterpret_cast<const half8_t*>(bias + n);
+    const half8_t b1 = *reinterpret_cast<const half8_t*>(bias + n + 8);
+    uint32_t w[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const half8_t& b = j < 2 ? b0 : b1;
+      w[j] = float2int8_pack4(value(c[4 * j], b.v[4 * j & 7]), value(c[4 * j + 1], b.v[(4 * j & 7) + 1]),
+                              value(c[4 * j + 2], b.v[(4 * j & 7) + 2]),
+                              value(c[4 * j + 3], b.v[(4 * j & 7) + 3]), quant_scale);
+    }
+    *reinterpret_cast<uint4*>(row_ptr(at(n), (int)m)) = make_uint4(w[0], w[1], w[2], w[3]);
+  }
+  bool aligned() const {
+    return ((reinterpret_cast<uintptr_t>(bias) | reinterpret_cast<uintptr_t>(q) |
+             reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v)) & 15u) == 0;
+  }
+};
+
 // Decode-step cross-attention query product followed by ker_arrange_encdec_q_i8I
 // (inference/kernels/transformerKernels_int8.cc.cu:1596-1645; call site
 // model/quant_decoder.cc.cu:745-760): code -> half(code * dq) + bias (a half add) -> fp16 q

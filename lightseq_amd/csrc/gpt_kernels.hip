@@ -24,7 +24,7 @@ __global__ void __launch_bounds__(256)
 gpt_embedding_kernel(const int8_t* __restrict__ token_emb, const T* __restrict__ pos_emb,
                      const int* __restrict__ token_id, T* __restrict__ output, int padding_id,
                      int pos_offset, float dequant_scale, int seq_len, int hidden, int vocab,
-                     const int* __restrict__ seq) {
+                     const int* __restrict__ seq, int* __restrict__ row_map) {
 #pragma clang fp contract(off)
   const long at = blockIdx.x;  // batch * seq_len + s
   const int s = (int)(at % seq_len);
@@ -33,6 +33,7 @@ gpt_embedding_kernel(const int8_t* __restrict__ token_emb, const T* __restrict__
     const int b = (int)(at / seq_len);
     if (s >= seq[2 * b + 1]) return;
     pos = seq[2 * b] + s;
+    if (threadIdx.x == 0) row_map[pos] = (int)at;
   }
   int tid = token_id[at];
   if (tid == padding_id) {
@@ -96,8 +97,8 @@ template <typename T>
 int gpt_embedding_i8I(int batch_size, int batch_seq_len, int hidden_size, hipStream_t s,
                       const int8_t* token_emb, const T* pos_emb, const int* token_id, T* output,
                       int* real_seq_len, int padding_id, int pos_offset, float dequant_scale,
-                      int vocab_size, int max_step, int* zero_flag, const int* seq) {
-  if (!token_emb || !pos_emb || !token_id || !output || !real_seq_len || batch_size <= 0 ||
+                      int vocab_size, int max_step, int* zero_flag, const int* seq, int* row_map) {
+  if (!token_emb || !pos_emb || !token_id || !output || !real_seq_len || (!seq != !row_map) || batch_size <= 0 ||
       batch_seq_len <= 0 || hidden_size <= 0)
     return lsh_fail(LSH_ERR_INVALID, "ker_gpt_embedding_i8I: bad arguments");
   if (pos_offset < 0 || (max_step > 0 && pos_offset + batch_seq_len > max_step))
@@ -114,7 +115,7 @@ int gpt_embedding_i8I(int batch_size, int batch_seq_len, int hidden_size, hipStr
     if (int rc = fill_i32(zero_flag, 0, 1, s)) return rc;
   gpt_embedding_kernel<T><<<batch_size * batch_seq_len, 256, 0, s>>>(
       token_emb, pos_emb, token_id, output, padding_id, pos_offset, dequant_scale, batch_seq_len,
-      hidden_size, vocab_size, seq);
+      hidden_size, vocab_size, seq, row_map);
   if (int rc = lsh_check_launch("gpt_embedding_kernel")) return rc;
   if (seq != nullptr) return LSH_OK;
   gpt_count_tokens_kernel<<<batch_size, 256, 0, s>>>(token_id, real_seq_len, padding_id,
@@ -123,10 +124,10 @@ int gpt_embedding_i8I(int batch_size, int batch_seq_len, int hidden_size, hipStr
 }
 template int gpt_embedding_i8I<float>(int, int, int, hipStream_t, const int8_t*, const float*,
                                       const int*, float*, int*, int, int, float, int, int, int*,
-                                      const int*);
+                                      const int*, int*);
 template int gpt_embedding_i8I<__half>(int, int, int, hipStream_t, const int8_t*, const __half*,
                                        const int*, __half*, int*, int, int, float, int, int, int*,
-                                       const int*);
+                                       const int*, int*);
 
 // ---------------------------------------------------------------------------------
 // prompt pass: int8 QKV GEMM output [tokens, 3H] + bias -> requantised with the cache

@@ -41,8 +41,7 @@ __global__ void __launch_bounds__(256)
 gpt_arrange_qkv_prefill_i8_kernel(const int8_t* __restrict__ ori, const __half* __restrict__ bias,
                                   int8_t* __restrict__ q_codes, int8_t* __restrict__ k_cache,
                                   int8_t* __restrict__ v_cache, int seq_len, int d, int head_num,
-                                  int groups, int max_step, float ds, float qs,
-                                  const int* __restrict__ seq) {
+                                  int groups, int max_step, float ds, float qs) {
 #pragma clang fp contract(off)
   const int hidden = d * head_num;
   const int grp = blockIdx.x % groups, which = (blockIdx.x / groups) % 3;
@@ -60,25 +59,22 @@ gpt_arrange_qkv_prefill_i8_kernel(const int8_t* __restrict__ ori, const __half* 
       bv[8 + k] = __half2float(b1.v[k]);
     }
   }
-  // the rows of sequence b: first and number (a plan has only those that are not padding)
-  const long row0 = seq != nullptr ? seq[2 * b] : (long)b * seq_len;
-  const int n = seq != nullptr ? seq[2 * b + 1] : seq_len;
-  const int8_t* src = ori + (row0 * 3 + which) * hidden + col;
+  const int8_t* src = ori + ((long)b * seq_len * 3 + which) * hidden + col;
   const long bh = (long)b * head_num + head;
   int8_t* dst = which == 0   ? q_codes + bh * seq_len * d + dim
                 : which == 1 ? k_cache + bh * max_step * d + dim
                              : v_cache + bh * max_step * d + dim;
-  for (int s0 = row; s0 < n; s0 += 32 * UNR) {
+  for (int s0 = row; s0 < seq_len; s0 += 32 * UNR) {
     uint4 w[UNR];
 #pragma unroll
     for (int u = 0; u < UNR; ++u) {
-      const int s = min(s0 + 32 * u, n - 1);
+      const int s = min(s0 + 32 * u, seq_len - 1);
       w[u] = *reinterpret_cast<const uint4*>(src + (long)s * 3 * hidden);
     }
 #pragma unroll
     for (int u = 0; u < UNR; ++u) {
       const int s = s0 + 32 * u;
-      if (s >= n) break;
+      if (s >= seq_len) break;
       const uint32_t wi[4] = {w[u].x, w[u].y, w[u].z, w[u].w};
       uint32_t o[4];
 #pragma unroll
@@ -112,7 +108,7 @@ int gpt_arrange_qkv_prefill_i8(int batch_token_num, int hidden_size, hipStream_t
                                const int8_t* ori_qkv, const __half* qkv_bias, int8_t* q_codes,
                                int8_t* k_cache, int8_t* v_cache, int batch_seq_len,
                                int dim_per_head, int head_num, int max_step, float dequant_scale,
-                               float quant_scale, const int* seq) {
+                               float quant_scale) {
   if (!ori_qkv || !qkv_bias || !q_codes || !k_cache || !v_cache || batch_token_num <= 0 ||
       batch_seq_len <= 0 || batch_token_num % batch_seq_len != 0 || dim_per_head <= 0 ||
       hidden_size != dim_per_head * head_num || batch_seq_len > max_step)
@@ -132,11 +128,11 @@ int gpt_arrange_qkv_prefill_i8(int batch_token_num, int hidden_size, hipStream_t
   if (batch_seq_len > 64)
     gpt_arrange_qkv_prefill_i8_kernel<4><<<batch * 3 * groups, 256, 0, s>>>(
         ori_qkv, qkv_bias, q_codes, k_cache, v_cache, batch_seq_len, dim_per_head, head_num, groups,
-        max_step, dequant_scale, quant_scale, seq);
+        max_step, dequant_scale, quant_scale);
   else
     gpt_arrange_qkv_prefill_i8_kernel<2><<<batch * 3 * groups, 256, 0, s>>>(
         ori_qkv, qkv_bias, q_codes, k_cache, v_cache, batch_seq_len, dim_per_head, head_num, groups,
-        max_step, dequant_scale, quant_scale, seq);
+        max_step, dequant_scale, quant_scale);
   return lsh_check_launch("gpt_arrange_qkv_prefill_i8_kernel");
 }
 

@@ -319,6 +319,12 @@ int gemm_blk_decself_qkv(const int8_t* A, const int8_t* W, const __half* qkv_bia
                          int8_t* new_k, int8_t* new_v, int step_token_num, int hidden, int K,
                          int head_num, int max_step, int step_id, float alpha, float dequant_scale,
                          float quant_scale, hipStream_t s, const LnStep* ln = nullptr);
+// ... of a prompt pass: gpt_arrange_qkv_prefill_i8 as the epilogue.  row_map: position of each row
+// (text_pack_plan's rows, gpt_embedding_i8I), or null where row i is position i
+int gemm_blk_prompt_qkv(const int8_t* A, const int8_t* W, const __half* qkv_bias, int8_t* q_codes,
+                        int8_t* k_cache, int8_t* v_cache, int rows, int hidden, int batch, int seq_len,
+                        int head_num, int max_step, const int* row_map, float alpha, float dequant_scale,
+                        float quant_scale, hipStream_t s);
 int gemm_blk_encdec_q(const int8_t* A, const int8_t* W, const __half* q_bias, __half* new_q,
                       int step_token_num, int hidden, int K, int beam_size, int head_num, float alpha,
                       float dequant_scale, hipStream_t s, const LnStep* ln = nullptr);
@@ -471,9 +477,10 @@ int gpt_embedding_i8I(int batch_size, int batch_seq_len, int hidden_size, hipStr
                       const int8_t* token_emb, const T* pos_emb, const int* token_id, T* output,
                       int* real_seq_len, int padding_id, int pos_offset, float dequant_scale,
                       int vocab_size, int max_step, int* zero_flag = nullptr,
-                      const int* seq = nullptr);
+                      const int* seq = nullptr, int* row_map = nullptr);
 // zero_flag: when given, the int it points to is cleared by the same launch (a generation
-// step's "unfinished" flag).  seq: a plan of text_pack_plan, which has also counted the tokens
+// step's "unfinished" flag).  seq: a plan of text_pack_plan, which has also counted the
+// tokens; row_map[row] then receives the position batch * seq_len + s that the row holds
 int gpt_arrange_qkv_prefill_f16(int batch_token_num, int hidden_size, hipStream_t s,
                                 const int8_t* ori_qkv, const __half* qkv_bias, __half* q_codes,
                                 __half* k_codes, __half* v_deq, int8_t* k_cache, int8_t* v_cache,
@@ -494,8 +501,8 @@ int gpt_arrange_qkv_prefill_i8(int batch_token_num, int hidden_size, hipStream_t
                                const int8_t* ori_qkv, const __half* qkv_bias, int8_t* q_codes,
                                int8_t* k_cache, int8_t* v_cache, int batch_seq_len,
                                int dim_per_head, int head_num, int max_step, float dequant_scale,
-                               float quant_scale, const int* seq = nullptr);
-// seq (here and below): the product's / the context's rows are those of a plan of text_pack_plan
+                               float quant_scale);
+// seq: the context's rows are those of a plan of text_pack_plan
 int gpt_prefill_attention_i8(const int8_t* q_codes, const int8_t* k_cache, const int8_t* v_cache,
                              const int* real_seq_len, int8_t* ctx_q, float quant_scale,
                              float dequant_scale, float v_quant_scale, int batch, int seq_len,

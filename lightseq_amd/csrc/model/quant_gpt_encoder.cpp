@@ -60,6 +60,7 @@ void QuantGptEncoder::init_buffer() {
   const size_t tokens = (size_t)_max_batch_size * _tw._max_step;
   _real_seq_len.alloc(_max_batch_size);
   _pack_seq.alloc(2 * (size_t)_max_batch_size + 1);
+  _pack_map.alloc(tokens);
   _ids.alloc(tokens);
   _last_ids.alloc(_max_batch_size);
   _unfinished.alloc(1);
@@ -182,7 +183,7 @@ void QuantGptEncoder::ffn_add_norm(int rows, int8_t* in, int8_t* tmp, bool block
 bool QuantGptEncoder::packed_route() const {
   return _ops.blocked && gpt_prefill_i8_enabled() && _tw._hidden_size % 128 == 0 &&
          gpt_prefill_i8_supported(_batch_seq_len, _tw._head_num, _tw._dim_per_head) &&
-         enc_pack_supported(_batch_size, _batch_seq_len, 1);
+         enc_pack_supported(_batch_size, _batch_seq_len, 1);  // (at most 2^20 positions)
 }
 
 // the rows of the plan: counted here, or as the plan counted them (the device embeds and
@@ -215,9 +216,10 @@ void QuantGptEncoder::prompt_pass(const int* ids, bool row_major_out, bool packe
   LSH_CALL(gpt_embedding_i8I<__half>(_batch_size, _batch_seq_len, H, _stream, _int8_emb.get(),
                                      _pos_emb.get(), ids, _query[_res].get(), _real_seq_len.get(),
                                      _tw._padding_id, 0, _src_emb_clip_max / Q,
-                                     _tw._src_vocab_size, _tw._max_step, nullptr, seq));
+                                     _tw._src_vocab_size, _tw._max_step, nullptr, seq, packed ? _pack_map.get() : nullptr));
   // until the number of rows is known, launches cover the most there can be
-  if (packed && host_token_ids) M = _batch_token_num = std::max(1, count_rows(host_token_ids));
+  if (packed && host_token_ids) M = _batch_token_num = count_rows(host_token_ids);
+  if (M == 0) return;  // nothing but padding
   int8_t *a = _buf_a.get(), *b = _buf_b.get();
   __half* qc = _qkv_buf.get();
   __half* kc = qc + _max_batch_dim;
@@ -232,23 +234,34 @@ void QuantGptEncoder::prompt_pass(const int* ids, bool row_major_out, bool packe
       LSH_CALL(norm_layer_resual_i8O<__half>(M, H, _stream, _query[_res].get(), a, w.ln1_scale.get(),
                                              w.ln1_bias.get(), w.b_out.get(), Q / c[4], false,
                                              _ops.blocked));
-    if (packed && !host_token_ids && _layer_id == 0)
-      M = _batch_token_num = std::max(1, count_rows(nullptr));
-    _ops.i8o(a, w.w_qkv.get(), b, M, 3 * H, H, c[0] * c[4] / (c[8] * Q), _stream);
+    if (packed && !host_token_ids && _layer_id == 0) {
+      M = _batch_token_num = count_rows(nullptr);
+      if (M == 0) return;
+    }
+    const float qkv_alpha = c[0] * c[4] / (c[8] * Q);
     int8_t* k_cache = _self_k_cache.get() + (size_t)_layer_id * _max_batch_dim;
     int8_t* v_cache = _self_v_cache.get() + (size_t)_layer_id * _max_batch_dim;
     if (on_codes) {
       // int8 end to end: q codes and the caches are all the arrange stage writes, and the
       // attention reads them
       int8_t* q8 = reinterpret_cast<int8_t*>(qc);
-      LSH_CALL(gpt_arrange_qkv_prefill_i8(_batch_size * _batch_seq_len, H, _stream, b,
-                                          w.b_qkv.get(), q8, k_cache, v_cache, _batch_seq_len, _tw._dim_per_head, _tw._head_num,
-                                          _tw._max_step, c[8] / Q, Q / c[11], seq));
+      if (_ops.blocked && _batch_size * _batch_seq_len < (1 << 22)) {
+        LSH_CALL(gemm_blk_prompt_qkv(a, w.w_qkv.get(), w.b_qkv.get(), q8, k_cache, v_cache, M, H,
+                                     _batch_size, _batch_seq_len, _tw._head_num, _tw._max_step,
+                                     packed ? _pack_map.get() : nullptr, qkv_alpha, c[8] / Q, Q / c[11],
+                                     _stream));
+      } else {
+        _ops.i8o(a, w.w_qkv.get(), b, M, 3 * H, H, qkv_alpha, _stream);
+        LSH_CALL(gpt_arrange_qkv_prefill_i8(M, H, _stream, b, w.b_qkv.get(), q8, k_cache, v_cache,
+                                            _batch_seq_len, _tw._dim_per_head, _tw._head_num,
+                                            _tw._max_step, c[8] / Q, Q / c[11]));
+      }
       LSH_CALL(gpt_prefill_attention_i8(q8, k_cache, v_cache, _real_seq_len.get(), a, Q / c[5],
                                         c[11] / Q, Q / c[11], _batch_size, _batch_seq_len,
                                         _tw._head_num, _tw._dim_per_head, _tw._max_step, _stream,
                                         _ops.blocked, seq));
     } else {
+      _ops.i8o(a, w.w_qkv.get(), b, M, 3 * H, H, qkv_alpha, _stream);
       LSH_CALL(gpt_arrange_qkv_prefill_f16(M, H, _stream, b, w.b_qkv.get(), qc, kc, vd, k_cache,
                                            v_cache, _batch_seq_len, _tw._dim_per_head,
                                            _tw._head_num, _tw._max_step, c[8] / Q, Q / c[11]));
@@ -519,6 +532,7 @@ void QuantGptEncoder::run_one_infer(int batch_size, int batch_seq_len, const int
   const bool packed = packed_route();
   if (!packed) CHECK_GPU_ERROR(hipMemsetAsync(_p_d_ppl, 0, sizeof(float) * batch_size, _stream));
   prompt_pass(_p_d_token_id, false, packed, host_token_ids);
+  if (_batch_token_num == 0) return;  // no text has a term; the results are zero
   /* compute_ppl (:781-797) */
   logits_product(_buf_a.get(), _batch_token_num);
   // the FFN2 accumulator buffer (tokens * hidden int32, idle by now) holds the per-position terms

@@ -102,7 +102,7 @@ class QuantGptEncoder {
   int _tap_step = -2;  // the cached step being enqueued (tokens sampled so far), -2 outside one
   int _rec_max_steps = 0;
 
-  DeviceBuffer<int> _pack_seq;  // the plan of a perplexity call (text_pack_plan)
+  DeviceBuffer<int> _pack_seq, _pack_map;  // the plan of a perplexity call (text_pack_plan)
   DeviceBuffer<int> _real_seq_len, _ids, _last_ids, _unfinished;
   DeviceBuffer<long long> _sample_state;  // lsh_rng_state_t [max_batch_size]
   // the residual stream; the second one holds a few rows of a step whose layer norms are made by
