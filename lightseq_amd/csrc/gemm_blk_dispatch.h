@@ -151,7 +151,8 @@ int dispatch_blk(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K,
 // = K in units of 1000 bytes, are fits to a sweep of hidden 512, 768 and 1024 (K of one and of
 // four times that) over M from 4 to 8192; the smallest one is within 15 % of the fastest there.
 struct SeqTile {
-  int kind;  // 0: a wavefront per 16 x 16, 1: per 32 x 32; 2 - 4: LDS tiles 64 x 64, 128 x 64, 128 x 128
+  int kind;  // 0: a wavefront per 16 x 16, 1: per 32 x 32; 2 - 4: LDS tiles 64 x 64, 128 x 64,
+             // 128 x 128; 5: the last with a third stage
   float us;
 };
 inline SeqTile choose_seq(int M, int N, int K) {
@@ -168,7 +169,10 @@ inline SeqTile choose_seq(int M, int N, int K) {
   if (K % kBK == 0 && K / kBK >= 3 && N % 16 == 0) {
     take(2, lds(tiles(64, 64), 1.9f, 1.4f));
     take(3, lds(tiles(128, 64), 3.7f, 1.8f));
-    take(4, lds(tiles(128, 128), 4.5f, 2.2f));
+    // with no more tiles than compute units a tile has a unit's LDS to itself: 3000 x 1024 x 4096 in
+    // 33.7 us instead of 39.9 (beyond that two tiles a unit are better: 8192 rows 52.0, not 65.8)
+    if (tiles(128, 128) <= 256.f) take(5, lds(tiles(128, 128), 3.85f, 0.f));
+    else take(4, lds(tiles(128, 128), 4.5f, 2.2f));
   }
   return best;
 }
@@ -202,6 +206,7 @@ int dispatch_f16(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K,
       return launch_seq<Epi, 2, 1>(A, W, epi, M, N, K, s);
     case 2: return launch_f16_tile<Epi, 2, 2, 1, 1, 3>(A, W, epi, M, N, K, s);
     case 3: return launch_f16_tile<Epi, 4, 1, 1, 2, 2>(A, W, epi, M, N, K, s);
+    case 5: return launch_f16_tile<Epi, 2, 2, 2, 2, 3>(A, W, epi, M, N, K, s);
     default: return launch_f16_tile<Epi, 2, 2, 2, 2, 2>(A, W, epi, M, N, K, s);
   }
 }

@@ -38,7 +38,7 @@ def test_encoder_layer_edges(batch, seq, hs, nh, ims, pre_ln, act, mask_type):
     assert d.max() < 2e-2 and d.mean() < 1e-3, (d.max(), d.mean())
 
 
-@pytest.mark.parametrize("hs,ims,seq", [(512, 2048, 64), (768, 3072, 37)])
+@pytest.mark.parametrize("hs,ims,seq", [(512, 2048, 64), (768, 3072, 37), (768, 3072, 64), (768, 3072, 128)])
 def test_a_sequence_does_not_depend_on_its_batch(hs, ims, seq):
     from test_oracle_layer_ops import config0
     rng = np.random.default_rng(5)
