@@ -8,6 +8,8 @@
 // Replaces inference/model/quant_bert_encoder.cc.cu:321-347 (two cuBLAS strided
 // batched GEMMs + ker_correlation_softmax_encself + ker_arrange_atten_output_i8O)
 // and inference/kernels/transformerKernels.cc.cu:1119-1172.
+#include <algorithm>
+#include <mutex>
 #include <type_traits>
 
 #include "ls_device.h"
@@ -593,6 +595,361 @@ encself_attn_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
   }
 }
 
+// ---------------------------------------------------------------------------------
+// The same attention (MODE 2 and 3, heads of 64) over two to four blocks of keys, with the same
+// bits.  What bounded the kernel above there was not its arithmetic: 192 workgroups of 200 keys
+// took 38 us, half of it trips to memory one behind the other (every chunk of keys was requested,
+// waited for and stored by itself, and keys were staged again for the second pass), most of
+// the rest a branch and two LDS reads per score for masks that are almost always empty.  Here
+//  * keys, values and masks of the whole sequence are staged once, in fragments' layouts, sixteen
+//    loads of a thread under way together (35 KB of LDS per 128 keys);
+//  * a mask is one addend per key (0, the caller's value, or -inf); a block of 32 keys without any
+//    runs without it, one that is masked throughout or beyond the keys is left out (its
+//    probabilities are exactly zero), and only a mixed one adds;
+//  * waves are as many as there are 32-query tiles to share the staged keys, four where workgroups
+//    are few (then a tile's latency counts).
+// LONGATTN_US
+// ---------------------------------------------------------------------------------
+constexpr int kLongMaxBlocks = 4;
+constexpr size_t long_attn_lds(int nkb) {
+  return (size_t)nkb * (128 * attn_kstr(64) * 2 + 64 * kAttnVstr * 2 + 128 * 4);
+}
+
+template <int MODE>
+__global__ void __launch_bounds__(512, 1)
+long_attn_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
+                 const __half* __restrict__ v, const int* __restrict__ pad_mask,
+                 __half* __restrict__ ctx, int8_t* __restrict__ ctx_q, float quant_scale, int S,
+                 int head_num, float alpha, float dq, int key_len, const int* __restrict__ seq,
+                 const __half* __restrict__ q_cmax, int k_pad) {
+  constexpr int D = 64, KSTR = attn_kstr(D), VSTR = kAttnVstr;
+  constexpr bool LAYER = MODE == kAttnLayer;
+  extern __shared__ __align__(16) int8_t long_smem[];
+  const int bh = blockIdx.y, b = bh / head_num, head = bh % head_num;
+  const int NT = blockDim.x, NW = NT >> 6;
+  const int S0 = S;
+  long row0 = (long)b * S;
+  int nkb = ((LAYER ? key_len : S) + 127) >> 7;
+  _Float16* Ks = reinterpret_cast<_Float16*>(long_smem);
+  _Float16* Vt = Ks + nkb * 128 * KSTR;                       // [key block][64][VSTR]
+  float* madd = reinterpret_cast<float*>(Vt + nkb * 64 * VSTR);
+  if (!LAYER && seq != nullptr) {
+    row0 = seq[2 * b];
+    S = seq[2 * b + 1];
+    const int pad_row = seq[2 * (gridDim.y / head_num)];
+    // the context of the padding's row, once per head
+    if (b == 0 && blockIdx.x == 0 && pad_row >= 0 && threadIdx.x < D / 16)
+      *reinterpret_cast<uint4*>(ctx_q + blocked_offset(pad_row, head * D + threadIdx.x * 16, head_num * D)) =
+          make_uint4(0, 0, 0, 0);
+    if ((int)blockIdx.x * (32 * NW) >= S) return;
+    nkb = (S + 127) >> 7;
+  }
+  int Sk = LAYER ? key_len : S;
+  const bool causal = LAYER && dq != 0.f;
+  if (causal) {  // (as many keys as queries)
+    Sk = min(Sk, ((int)blockIdx.x + 1) * (32 * NW));
+    nkb = (Sk + 127) >> 7;
+  }
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int l32 = lane & 31, g = lane >> 5;
+  const int q0 = (int)blockIdx.x * (32 * NW) + wave * 32, qi = q0 + l32;
+  const int hidden = head_num * D, hidden3 = 3 * hidden;
+  const float kNegInf = -__builtin_inff();
+  const int8_t* codes = reinterpret_cast<const int8_t*>(q) + row0 * hidden3 + head * D;
+  const _Float16* bias = reinterpret_cast<const _Float16*>(k) + head * D;
+  const _Float16* kbase = reinterpret_cast<const _Float16*>(k) + (long)bh * key_len * D;
+  const _Float16* vbase = reinterpret_cast<const _Float16*>(v) + (long)bh * key_len * D;
+
+  // the lane's query: d = ks * 16 + g * 8 .. + 8
+  v8h qreg[D / 16];
+  uint4 wq[2];
+  if constexpr (LAYER) {
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks)
+      qreg[ks] = *reinterpret_cast<const v8h*>(reinterpret_cast<const _Float16*>(q) +
+                                               ((long)bh * S + min(qi, S - 1)) * D + ks * 16 + g * 8);
+  } else {
+#pragma unroll
+    for (int kp = 0; kp < 2; ++kp)
+      wq[kp] = *reinterpret_cast<const uint4*>(codes + (long)min(qi, S - 1) * hidden3 + kp * 32 + g * 16);
+  }
+  const bool q_pad = LAYER ? false : pad_mask[(long)b * S0 + min(qi, S - 1)] != 0;
+  for (int key = tid; key < nkb * 128; key += NT) {
+    float a = 0.f;
+    if constexpr (LAYER) {
+      if (pad_mask != nullptr)
+        a = __half2float(reinterpret_cast<const __half*>(pad_mask)[(long)b * key_len + min(key, Sk - 1)]);
+    } else {
+      a = pad_mask[(long)b * S0 + min(key, Sk - 1)] != 0 ? kNegInf : 0.f;
+    }
+    madd[key] = key < Sk ? a : kNegInf;
+  }
+
+  // Patch p: 4 keys x 8 dimensions of the values, and as many bytes of keys.  Rows past the last
+  // key, up to a whole block of 32, read the last one and become zeros.
+  {
+    const int P = ((Sk + 31) & ~31) * 2;
+    constexpr int KC = LAYER ? 4 : 2, UNR = 2;
+    for (int p0 = tid; p0 < P; p0 += UNR * NT) {
+      uint4 kr[UNR][KC];
+      using VRaw = typename std::conditional<LAYER, uint4, uint2>::type;
+      VRaw vr[UNR][4];
+#pragma unroll
+      for (int u = 0; u < UNR; ++u) {
+        const int p = min(p0 + u * NT, P - 1);
+#pragma unroll
+        for (int j = 0; j < KC; ++j) {
+          const int c = p + j * P;
+          if constexpr (LAYER)
+            kr[u][j] = *reinterpret_cast<const uint4*>(kbase + (long)min(c >> 3, Sk - 1) * D + (c & 7) * 8);
+          else
+            kr[u][j] = *reinterpret_cast<const uint4*>(codes + (long)min(c >> 2, Sk - 1) * hidden3 + hidden +
+                                                       (c & 3) * 16);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int key = min((p >> 3) * 4 + r, Sk - 1);
+          if constexpr (LAYER)
+            vr[u][r] = *reinterpret_cast<const VRaw*>(vbase + (long)key * D + (p & 7) * 8);
+          else
+            vr[u][r] = *reinterpret_cast<const VRaw*>(codes + (long)key * hidden3 + 2 * hidden + (p & 7) * 8);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < UNR; ++u) {
+        const int p = p0 + u * NT;
+        if (p >= P) break;
+#pragma unroll
+        for (int j = 0; j < KC; ++j) {
+          const int c = p + j * P;
+          if constexpr (LAYER) {
+            const int row = c >> 3;
+            *reinterpret_cast<uint4*>(&Ks[row * KSTR + (c & 7) * 8]) = row < Sk ? kr[u][j] : make_uint4(0, 0, 0, 0);
+          } else {
+            const int row = c >> 2;
+            v8h lo, hi;
+            dequant16_bias(kr[u][j], bias + hidden + (c & 3) * 16, dq, lo, hi);
+            if (row >= Sk) lo = hi = (v8h)(_Float16)0;
+            *reinterpret_cast<v8h*>(&Ks[row * KSTR + (c & 3) * 16]) = lo;
+            *reinterpret_cast<v8h*>(&Ks[row * KSTR + (c & 3) * 16 + 8]) = hi;
+          }
+        }
+        const int key = (p >> 3) * 4, ch = p & 7;
+        v8h x[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          if constexpr (LAYER) x[r] = __builtin_bit_cast(v8h, vr[u][r]);
+          else x[r] = dequant8_bias(vr[u][r], bias + 2 * hidden + ch * 8, dq);
+          if (key + r >= Sk) x[r] = (v8h)(_Float16)0;
+        }
+        _Float16* vt = Vt + (key >> 7) * (64 * VSTR) + (key & 127);
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          *reinterpret_cast<v4h*>(&vt[(ch * 8 + e) * VSTR]) = (v4h){x[0][e], x[1][e], x[2][e], x[3][e]};
+      }
+    }
+  }
+  if constexpr (!LAYER) {
+#pragma unroll
+    for (int kp = 0; kp < 2; ++kp) {
+      // lane half g converts chunk kp * 32 + g * 16 .. + 16, then the halves swap their second part
+      v8h lo, hi;
+      dequant16_bias(wq[kp], bias + kp * 32 + g * 16, dq, lo, hi);
+      v8h give = g == 0 ? hi : lo, take;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        reinterpret_cast<int*>(&take)[j] = __shfl_xor(reinterpret_cast<const int*>(&give)[j], 32, 64);
+      qreg[2 * kp] = g == 0 ? lo : take;
+      qreg[2 * kp + 1] = g == 0 ? take : hi;
+    }
+  }
+  __syncthreads();
+  if (q0 >= S) return;  // (the whole wavefront)
+
+  // what the masks of key block kb ask for, per block of 32 keys, the same in every lane
+  struct Blocks { bool live[4], mixed[4]; };
+  auto look = [&](int kb) {
+    Blocks w;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const float a = madd[kb * 128 + h * 64 + lane];
+      const uint64_t some = __ballot(a != 0.f), dead = __ballot(a == kNegInf);
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const int key0 = kb * 128 + h * 64 + s * 32;
+        w.live[2 * h + s] = (uint32_t)(dead >> (32 * s)) != 0xffffffffu && !(causal && key0 > q0 + 31);
+        w.mixed[2 * h + s] = (uint32_t)(some >> (32 * s)) != 0 || (causal && key0 + 31 > q0);
+      }
+    }
+    return w;
+  };
+  auto scores = [&](int kb, int sb, bool mixed, v16f& out) {
+    v16f c;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) c[i] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks) {
+      const v8h a = *reinterpret_cast<const v8h*>(&Ks[(kb * 128 + sb * 32 + l32) * KSTR + ks * 16 + g * 8]);
+      c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qreg[ks], c, 0, 0, 0);
+    }
+    // (a score that is no number counts as masked in the layers)
+    auto value = [&](float t) { return LAYER ? fmaxf(t, kFloatInfNeg) : t; };
+    if (!mixed) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) out[i] = value(round_h(alpha * c[i]));
+    } else {
+      const int key0 = kb * 128 + sb * 32 + 4 * g;
+#pragma unroll
+      for (int f = 0; f < 4; ++f) {
+        const float4 m4 = *reinterpret_cast<const float4*>(&madd[key0 + 8 * f]);
+        const float mm[4] = {m4.x, m4.y, m4.z, m4.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float t = fmaxf(round_h(alpha * c[4 * f + j]) + mm[j], kFloatInfNeg);
+          out[4 * f + j] = (causal && key0 + 8 * f + j > qi) ? kFloatInfNeg : t;
+        }
+      }
+    }
+  };
+
+  // ---- pass 1: maximum and sum of exponentials, a block of 128 keys at a time
+  float m = kFloatInfNeg, sum = 0.f;
+  for (int kb = 0; kb < nkb; ++kb) {
+    const Blocks w = look(kb);
+    v16f sc[4];
+    float bm = kFloatInfNeg;
+#pragma unroll
+    for (int sb = 0; sb < 4; ++sb)
+      if (w.live[sb]) {
+        scores(kb, sb, w.mixed[sb], sc[sb]);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) bm = fmaxf(bm, sc[sb][i]);
+      }
+    bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
+    const float m_new = fmaxf(m, bm);
+    const float mref = m_new == kFloatInfNeg ? 0.f : m_new;
+    float part = 0.f;
+#pragma unroll
+    for (int sb = 0; sb < 4; ++sb)
+      if (w.live[sb]) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) part += __expf(sc[sb][i] - mref);
+      }
+    part += __shfl_xor(part, 32, 64);
+    sum = sum * __expf(m - m_new) + part;
+    m = m_new;
+  }
+
+  // ---- pass 2: probabilities (the correctly rounded quotients, see encself_attn_kernel) x values
+  float rs = __builtin_amdgcn_rcpf(sum);
+  rs = sum > 0.f ? fmaf(fmaf(-sum, rs, 1.f), rs, rs) : 0.f;  // no visible key: all zero
+  const float mref = m == kFloatInfNeg ? 0.f : m;
+  v16f acc[D / 32];
+#pragma unroll
+  for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[db][i] = 0.f;
+  for (int kb = 0; kb < nkb; ++kb) {
+    const Blocks w = look(kb);
+#pragma unroll
+    for (int sb = 0; sb < 4; ++sb) {
+      if (!w.live[sb]) continue;
+      v16f sc;
+      scores(kb, sb, w.mixed[sb], sc);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        v8h pb;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const float e = __expf(sc[8 * t + j] - mref);
+          float qt = e * rs;
+          qt = fmaf(fmaf(-sum, qt, e), rs, qt);
+          qt = fmaf(fmaf(-sum, qt, e), rs, qt);
+          // keep the float quotient a value of its own: folded into the last correction,
+          // the conversion to fp16 would round once instead of twice
+          asm volatile("" : "+v"(qt));
+          pb[j] = (_Float16)qt;
+        }
+#pragma unroll
+        for (int db = 0; db < D / 32; ++db) {
+          const _Float16* vrow = &Vt[kb * (64 * VSTR) + (db * 32 + l32) * VSTR + sb * 32 + 16 * t + 4 * g];
+          const v4h lo = *reinterpret_cast<const v4h*>(vrow);
+          const v4h hi = *reinterpret_cast<const v4h*>(vrow + 8);
+          const v8h a = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+          acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pb, acc[db], 0, 0, 0);
+        }
+      }
+    }
+  }
+
+  if (qi >= S) return;
+  const long tok = row0 + qi;
+  const Quantiser codes_of = Quantiser::of(LAYER && q_cmax != nullptr ? cm(q_cmax) : 1.f);
+#pragma unroll
+  for (int db = 0; db < D / 32; ++db) {
+#pragma unroll
+    for (int vg = 0; vg < 4; ++vg) {
+      const int dd = db * 32 + 8 * vg + 4 * g;
+      float o[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[j] = round_h(acc[db][4 * vg + j]);
+      if (ctx != nullptr) {
+        half4_t t;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) t.v[j] = __float2half_rn(q_pad ? 0.f : o[j]);
+        *reinterpret_cast<half4_t*>(LAYER ? ctx + tok * hidden + head * D + dd
+                                          : ctx + ((long)bh * S + qi) * D + dd) = t;
+      }
+      if (ctx_q != nullptr) {
+        if constexpr (LAYER) {
+          *reinterpret_cast<uint32_t*>(ctx_q + blocked_offset(tok, head * D + dd, k_pad)) =
+              pack4_i8(codes_of.code(o[0]), codes_of.code(o[1]), codes_of.code(o[2]), codes_of.code(o[3]));
+        } else {
+          const uint32_t w4 = float2int8_pack4(o[0], o[1], o[2], o[3], quant_scale);
+          *reinterpret_cast<uint32_t*>(ctx_q + code_offset(tok, head * D + dd, hidden, seq != nullptr)) =
+              q_pad ? 0u : w4;
+        }
+      }
+    }
+  }
+}
+
+template <int MODE>
+static int launch_long_attn(int seq_len, int batch_heads, hipStream_t s, const __half* q, const __half* k,
+                            const __half* v, const int* pad_mask, __half* ctx, int8_t* ctx_q,
+                            float quant_scale, int head_num, float alpha, float dq, int key_len,
+                            const int* seq, const __half* q_cmax, int k_pad) {
+  {
+    // more than the default dynamic LDS limit: raise it once per device
+    static std::mutex mu;
+    static unsigned long long raised = 0;
+    int dev = 0;
+    if (lsh_check_hip(hipGetDevice(&dev), "hipGetDevice")) return LSH_ERR_HIP;
+    std::lock_guard<std::mutex> lock(mu);
+    if (dev >= 64 || !((raised >> dev) & 1)) {
+      if (lsh_check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(long_attn_kernel<MODE>),
+                                            hipFuncAttributeMaxDynamicSharedMemorySize,
+                                            (int)long_attn_lds(kLongMaxBlocks)),
+                        "hipFuncSetAttribute(long_attn_kernel)"))
+        return LSH_ERR_HIP;
+      if (dev < 64) raised |= 1ull << dev;
+    }
+  }
+  // Two blocks of keys leave room for two workgroups of four wavefronts on a compute unit; more
+  // take most of its LDS, and the wavefronts of a chip full of workgroups are then as many as
+  // share them evenly, up to eight.
+  const int tiles = (seq_len + 31) / 32, nkb = (key_len + 127) / 128;
+  int nw = std::min(4, tiles);
+  if (nkb > 2 && (long)batch_heads * ((tiles + 3) / 4) > 256) {
+    const int groups = (tiles + 7) / 8;
+    nw = (tiles + groups - 1) / groups;
+  }
+  long_attn_kernel<MODE><<<dim3((tiles + nw - 1) / nw, batch_heads), 64 * nw, long_attn_lds(nkb), s>>>(
+      q, k, v, pad_mask, ctx, ctx_q, quant_scale, seq_len, head_num, alpha, dq, key_len, seq, q_cmax, k_pad);
+  return LSH_OK;
+}
+
 // 4 wavefronts (128 queries) per workgroup once a sequence has more than 64 queries, so
 // that a (batch, head) pair with up to 128 keys is staged once; 2 wavefronts otherwise.
 template <int MODE>
@@ -602,6 +959,10 @@ static bool launch_attn(int dim_per_head, int seq_len, int batch_heads, hipStrea
                         float dq, int key_len = -1, const int* seq = nullptr,
                         const __half* q_cmax = nullptr, int k_pad = 0) {
   if (key_len < 0) key_len = seq_len;  // self attention: as many keys as queries
+  if constexpr (MODE == kAttnLayer || MODE == kAttnEncI8)
+    if (dim_per_head == 64 && key_len > 128 && key_len <= 128 * kLongMaxBlocks)
+      return launch_long_attn<MODE>(seq_len, batch_heads, s, q, k, v, pad_mask, ctx, ctx_q, quant_scale,
+                                    head_num, alpha, dq, key_len, seq, q_cmax, k_pad) == LSH_OK;
 #define LSH_ATTN(DD, NWV)                                                                      \
   if (key_len <= 128)                                                                          \
     encself_attn_kernel<DD, MODE, NWV, true>                                                   \
