@@ -606,9 +606,10 @@ encself_attn_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
 //  * a mask is one addend per key (0, the caller's value, or -inf); a block of 32 keys without any
 //    runs without it, one that is masked throughout or beyond the keys is left out (its
 //    probabilities are exactly zero), and only a mixed one adds;
-//  * waves are as many as there are 32-query tiles to share the staged keys, four where workgroups
-//    are few (then a tile's latency counts).
-// LONGATTN_US
+//  * a wavefront per tile of 32 queries, up to sixteen to share the staged keys (launch_long_attn);
+//    a plan's longest sequences come first.
+// 96 pairs of 200 keys 38 -> 15.5 us, 288 of 150 59 -> 20, 480 of 250 97 -> 37, 384 packed ones of 96
+// to 384 76 -> 49 (fp16 operands but for the last, int8 codes).
 // ---------------------------------------------------------------------------------
 constexpr int kLongMaxBlocks = 4;
 constexpr size_t long_attn_lds(int nkb) {
@@ -616,16 +617,22 @@ constexpr size_t long_attn_lds(int nkb) {
 }
 
 template <int MODE>
-__global__ void __launch_bounds__(512, 1)
+__global__ void __launch_bounds__(1024, 1)
 long_attn_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
                  const __half* __restrict__ v, const int* __restrict__ pad_mask,
                  __half* __restrict__ ctx, int8_t* __restrict__ ctx_q, float quant_scale, int S,
                  int head_num, float alpha, float dq, int key_len, const int* __restrict__ seq,
-                 const __half* __restrict__ q_cmax, int k_pad) {
+                 const __half* __restrict__ q_cmax, int k_pad, const int* __restrict__ items) {
   constexpr int D = 64, KSTR = attn_kstr(D), VSTR = kAttnVstr;
   constexpr bool LAYER = MODE == kAttnLayer;
   extern __shared__ __align__(16) int8_t long_smem[];
-  const int bh = blockIdx.y, b = bh / head_num, head = bh % head_num;
+  int b = blockIdx.y / head_num, head = blockIdx.y % head_num;
+  if (!LAYER && items != nullptr) {
+    const int item = __builtin_amdgcn_readfirstlane(items[blockIdx.y]);
+    b = item & 0xffff;
+    head = (item >> 16) & 0xfff;
+  }
+  const int bh = b * head_num + head;
   const int NT = blockDim.x, NW = NT >> 6;
   const int S0 = S;
   long row0 = (long)b * S;
@@ -919,7 +926,7 @@ template <int MODE>
 static int launch_long_attn(int seq_len, int batch_heads, hipStream_t s, const __half* q, const __half* k,
                             const __half* v, const int* pad_mask, __half* ctx, int8_t* ctx_q,
                             float quant_scale, int head_num, float alpha, float dq, int key_len,
-                            const int* seq, const __half* q_cmax, int k_pad) {
+                            const int* seq, const __half* q_cmax, int k_pad, const int* items) {
   {
     // more than the default dynamic LDS limit: raise it once per device
     static std::mutex mu;
@@ -936,17 +943,16 @@ static int launch_long_attn(int seq_len, int batch_heads, hipStream_t s, const _
       if (dev < 64) raised |= 1ull << dev;
     }
   }
-  // Two blocks of keys leave room for two workgroups of four wavefronts on a compute unit; more
-  // take most of its LDS, and the wavefronts of a chip full of workgroups are then as many as
-  // share them evenly, up to eight.
+  // As few parts of a sequence's queries as fill the chip (a part stages all keys), of up to 16
+  // tiles: LDS has room for two workgroups of a compute unit with two blocks of keys, for one with
+  // more, and wavefronts that share a workgroup are what hides latency then.
   const int tiles = (seq_len + 31) / 32, nkb = (key_len + 127) / 128;
-  int nw = std::min(4, tiles);
-  if (nkb > 2 && (long)batch_heads * ((tiles + 3) / 4) > 256) {
-    const int groups = (tiles + 7) / 8;
-    nw = (tiles + groups - 1) / groups;
-  }
+  const int room = nkb == 2 ? 512 : 256;
+  const int parts = std::max((tiles + 15) / 16, std::min(room / std::max(batch_heads, 1), (tiles + 3) / 4));
+  const int nw = (tiles + parts - 1) / parts;
   long_attn_kernel<MODE><<<dim3((tiles + nw - 1) / nw, batch_heads), 64 * nw, long_attn_lds(nkb), s>>>(
-      q, k, v, pad_mask, ctx, ctx_q, quant_scale, seq_len, head_num, alpha, dq, key_len, seq, q_cmax, k_pad);
+      q, k, v, pad_mask, ctx, ctx_q, quant_scale, seq_len, head_num, alpha, dq, key_len, seq, q_cmax, k_pad,
+      items);
   return LSH_OK;
 }
 
@@ -957,12 +963,12 @@ static bool launch_attn(int dim_per_head, int seq_len, int batch_heads, hipStrea
                         const __half* q, const __half* k, const __half* v, const int* pad_mask,
                         __half* ctx, int8_t* ctx_q, float quant_scale, int head_num, float alpha,
                         float dq, int key_len = -1, const int* seq = nullptr,
-                        const __half* q_cmax = nullptr, int k_pad = 0) {
+                        const __half* q_cmax = nullptr, int k_pad = 0, const int* items = nullptr) {
   if (key_len < 0) key_len = seq_len;  // self attention: as many keys as queries
   if constexpr (MODE == kAttnLayer || MODE == kAttnEncI8)
     if (dim_per_head == 64 && key_len > 128 && key_len <= 128 * kLongMaxBlocks)
       return launch_long_attn<MODE>(seq_len, batch_heads, s, q, k, v, pad_mask, ctx, ctx_q, quant_scale,
-                                    head_num, alpha, dq, key_len, seq, q_cmax, k_pad) == LSH_OK;
+                                    head_num, alpha, dq, key_len, seq, q_cmax, k_pad, items) == LSH_OK;
 #define LSH_ATTN(DD, NWV)                                                                      \
   if (key_len <= 128)                                                                          \
     encself_attn_kernel<DD, MODE, NWV, true>                                                   \
@@ -1044,7 +1050,7 @@ int encself_attention_packed(const int8_t* qkv, const __half* qkv_bias, float de
   if (!launch_attn<kAttnEncI8>(dim_per_head, seq_len, batch * head_num, s,
                                reinterpret_cast<const __half*>(qkv), qkv_bias, nullptr, pad_mask,
                                nullptr, ctx_q, quant_scale, head_num, alpha, dequant_scale, -1,
-                               pack.seq))
+                               pack.seq, nullptr, 0, pack.items))
     return lsh_fail(LSH_ERR_UNSUPPORTED,
                     "encself_attention_packed: dim_per_head must be 32, 64 or 128");
   return lsh_check_launch("encself_attn_kernel<packed>");

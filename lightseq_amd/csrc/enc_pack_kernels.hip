@@ -22,7 +22,7 @@ constexpr int kItemHeadShift = 16, kItemBlocksShift = 28;  // as in qkv_attn_ker
 // One workgroup: a wavefront per sequence finds the last token (COUNT: counts its tokens, what a
 // GPT model takes for the length of a text), then starts by a prefix sum, and
 // the work items of the fused QKV + attention kernel in the order that kernel wants (see
-// qkv_attn_plan_kernel).  Bound by two or three trips to memory.
+// qkv_attn_plan_kernel; longest sequence first for the attention over more than 128 keys).  Bound by two or three trips to memory.
 template <bool COUNT>
 __global__ void __launch_bounds__(1024)
 enc_pack_plan_kernel(const int* __restrict__ tokens, int padding_id, int* __restrict__ seq,
@@ -86,7 +86,7 @@ enc_pack_plan_kernel(const int* __restrict__ tokens, int padding_id, int* __rest
   const int n = batch * head_num;
   for (int w = tid; w < n; w += 1024) {
     int seq_rank, head;
-    if ((batch & 7) == 0) {
+    if ((batch & 7) == 0 && S <= 128) {
       const int xcd = w & 7, j = w >> 3, per_xcd = n >> 3;
       const int q = j < 32 ? j : per_xcd - 1 - (j - 32);
       seq_rank = xcd + 8 * (q / head_num);

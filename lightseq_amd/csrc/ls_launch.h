@@ -185,7 +185,7 @@ int qkv_attention_i8(const int8_t* x, const int8_t* qkv_weight, const __half* qk
 struct EncPack {
   int* seq;      // [2 * batch + 1]: first row and length of a sequence; the padding's row, or -1
   int* row_map;  // [batch * seq_len]: the row that position (b, s) is computed in
-  int* items;    // [batch * heads]: work items of the fused QKV + attention kernel, or null
+  int* items;    // [batch * heads]: work items of the attention kernels, or null
 };
 bool enc_pack_supported(int batch, int seq_len, int head_num);
 // Fills the plan from the token ids.  host_rows (optional, pinned): receives `ticket` << 32 | number

@@ -249,7 +249,7 @@ void QuantBertEncoder::run_packed(const int* host_token_ids) {
   const int h = _tw._head_num, dph = _tw._dim_per_head, post = _tw._is_post_ln;
   const float Q = _quant_range;
   const bool qkv_fused = qkv_attention_fused_supported(B, S, h, dph);
-  const EncPack pack{_pack_seq.get(), _pack_map.get(), qkv_fused ? _qa_plan.get() : nullptr};
+  const EncPack pack{_pack_seq.get(), _pack_map.get(), _qa_plan.get()};
   LSH_CALL(enc_pack_plan(_p_d_token_id, _tw._padding_id, pack, B, S, h,
                          host_token_ids ? nullptr : _h_pack_rows, ++_pack_ticket, _stream));
   LSH_CALL(enc_emb_packed(_int8_emb.get(), _pos_emb.get(), _p_d_token_id, _residual.get(),
