@@ -82,7 +82,12 @@ __device__ __forceinline__ float act_b(float x) {
   if (ACT == 1) return fmaxf(x, 0.f);
   if (sizeof(T) == 2) {
     const float p3 = TT<T>::rnd(x * TT<T>::rnd(x * x));
-    const float cdf = 0.5f * (1.0f + tanhf(0.7978845608028654f * (x + 0.044715f * p3)));
+    // 0.5 * (1 + tanh(u)) as 1 / (1 + exp(-2u)), two hardware functions: the half it is rounded to
+    // is the same for 65381 of the 65536 halfs x, and for the others (all but two below -2,
+    // where 1 + tanh(u) cancels) the nearer one.  With tanhf the epilogue of the first feed-forward
+    // product took longer than its K loop: 3600 x 3072 x 768 39.5 us, 28.2 now.
+    const float cdf = __builtin_amdgcn_rcpf(
+        1.0f + __builtin_amdgcn_exp2f(-2.f * 0.7978845608028654f * 1.44269504088896340736f * (x + 0.044715f * p3)));
     return TT<T>::rnd(x * TT<T>::rnd(cdf));
   }
   return gelu_tanh(x);
