@@ -193,7 +193,7 @@ class StepTaps {
 // The host's side of StepNotice.  A generation loop has to know after every step whether it goes on;
 // a copy of the word and a stream synchronisation leave the device idle for 25 - 35 us (the
 // wait, then the first launches of the next step).  Instead the loop enqueues the next step's
-// first launches, the first of which publishes the word, and waits for the word alone: the
+// layers, the first launch of which publishes the word, and waits for the word alone: the
 // device works meanwhile.  A step enqueued too far writes nothing that a finished run reads.
 class HostNotice {
  public:
