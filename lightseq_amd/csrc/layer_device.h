@@ -36,29 +36,33 @@ __device__ __forceinline__ float fake_quantize_b(float x, float cmax, int& mask,
 // A quantiser whose scale many elements share: quantize_b and fake_quantize_b bit for bit, the
 // division by the scale made of a correctly rounded reciprocal, taken once, and two residual
 // corrections (Markstein: the quotient is then the correctly rounded one) -- 5 instructions
-// instead of the 12 of a division, in launches that are bound by them.  (A clip value of zero
-// gives other codes than a division by zero does, but what they stand for is zero either way.)
+// instead of the 12 of a division, in launches that are bound by them.
+// The clamp comes first, on the element: an infinite one has no residual (inf - inf), and of an
+// element inside the clip value the quotient is at most 127 in magnitude, whatever its rounding, so
+// that none is needed behind it.  A NaN becomes the lesser bound there, code -127, as it does in
+// quantize_b.  (A clip value of zero gives code 0 where a division by zero gives others; what they
+// stand for is zero either way.)
 struct Quantiser {
-  float scale, inv;
+  float scale, inv, lo, hi;
   static __device__ __forceinline__ Quantiser of(float cmax, bool symmetry = true) {
     float s = cmax / kQ;
     if (!symmetry) s /= 2;
-    return Quantiser{s, 1.0f / s};
+    return Quantiser{s, s != 0.f ? 1.0f / s : 0.f, symmetry ? -cmax : 0.f, cmax};
   }
   __device__ __forceinline__ float quotient(float x) const {
+    x = __builtin_amdgcn_fmed3f(x, lo, hi);
     float q = x * inv;
     q = __builtin_fmaf(__builtin_fmaf(-scale, q, x), inv, q);
     return __builtin_fmaf(__builtin_fmaf(-scale, q, x), inv, q);
   }
   __device__ __forceinline__ float rounded(float x) const {  // -127 .. 127
-    return __builtin_amdgcn_fmed3f(floorf(quotient(x) + 0.5f), -kQ, kQ);
+    return floorf(quotient(x) + 0.5f);
   }
   __device__ __forceinline__ int code(float x) const { return (int)rounded(x); }
   __device__ __forceinline__ float fake(float x) const { return rounded(x) * scale; }
   // the unsigned quantiser (symmetry = false)
   __device__ __forceinline__ float fake_unsigned(float x) const {
-    const float q = __builtin_amdgcn_fmed3f(floorf((quotient(x) - kQ) + 0.5f), -kQ, kQ);
-    return (q + kQ) * scale;
+    return (floorf((quotient(x) - kQ) + 0.5f) + kQ) * scale;
   }
 };
 // kernels.h:497-501

@@ -1,0 +1,79 @@
+"""The quantised layers at the ends of what they accept: elements that are no finite numbers."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import to_dev, to_np
+from test_decoder_layer_gpu import IMS, NH, NLAYER, _case, _make_stack, _release
+from test_layer_ops_gpu import _lo, _make_layer
+
+pytestmark = pytest.mark.gpu
+
+INF = np.float16(np.inf)
+
+
+def _check(got, want, rows):
+    """Outputs of the finite rows, within the bar of the layer tests."""
+    got, want = to_np(got).astype(np.float64)[rows], want.astype(np.float64)[rows]
+    assert np.isfinite(want).all()
+    assert np.isfinite(got).all()
+    d = np.abs(got - want)
+    assert d.max() < 2e-2 and d.mean() < 1e-3, (d.max(), d.mean())
+
+
+@pytest.mark.parametrize("pre_ln,act", [(False, "relu"), (False, "gelu"), (True, "relu"), (True, "gelu")])
+@pytest.mark.parametrize("seq", [17, 150])
+def test_infinite_elements_take_the_outermost_codes(pre_ln, act, seq):
+    """Infinite weights, biases and (where the layer quantises its input itself) inputs have the
+    codes +-127, as the restatement has them: every row but the infinite ones stays what it is.
+    17 keys run the attention kernel of few queries, 150 the one of long sequences."""
+    from test_oracle_layer_ops import config0
+    lo = _lo()
+    rng = np.random.default_rng(seq)
+    batch, hs, nh, ims = 2, 128, 2, 256
+    cfg0 = config0(rng, pre_ln, act, batch, seq, hs, nh, ims)
+    layer, para = _make_layer(cfg0, pre_ln, act, nh, 512, 256)
+    p = lo.split_params(para, hs, ims)  # views
+    p["attn_qkvw"][hs + 3, 5], p["attn_qkvw"][2 * hs + 9, 7] = INF, -INF  # a key's and a value's row
+    p["attn_qkvb"][2 * hs + 11] = -INF  # a column of the context
+    p["attn_ow"][4, 6] = INF
+    p["inter_w"][8, 2], p["inter_b"][10], p["inter_b"][12] = -INF, INF, np.float16(6e4)
+    p["output_w"][1, 3], p["output_w"][2, 10] = INF, -INF
+    with torch.no_grad():
+        layer.para.copy_(to_dev(para))
+    x = cfg0[1].astype(np.float16)
+    rows = np.ones((batch, seq), bool)
+    if not pre_ln:
+        x[0, 4, 5], x[1, 16, 7], x[1, 2, 90] = INF, -INF, INF
+        rows[0, 4] = rows[1, 16] = rows[1, 2] = False
+    with np.errstate(all="ignore"):
+        want = lo.encoder_layer_forward(para, x, np.zeros((batch, seq), np.float16), nh, ims, pre_ln, act)
+    with torch.no_grad():
+        got = layer(to_dev(x), torch.zeros(batch, seq, device="cuda"))
+    _check(got, want, rows)
+
+
+def test_infinite_elements_of_a_decoder_layer():
+    """The same with keys and values that the layer fake-quantises for its cache."""
+    lo = _lo()
+    paras, x, enc, pad, mask = _case(21, 2, 9, 12)
+    for lid, para in enumerate(paras):
+        p = lo.split_decoder_params(para, x.shape[-1], IMS, lid, NLAYER)
+        hs = x.shape[-1]
+        p["attn_qkvb"][hs + 5], p["attn_qkvb"][2 * hs + 6] = INF, -INF
+        p["encdec_attn_qw"][3, 4], p["encdec_attn_ow"][7, 8] = INF, -INF
+        p["output_w"][1, 3] = INF
+        if lid == 0:
+            p["encdec_attn_kvw"][9, 10] = -INF
+    layers = _make_stack(paras, True, "relu", 64, 32)
+    try:
+        with np.errstate(all="ignore"):
+            kv = lo.decoder_encdec_kv(paras[0], enc, NH, IMS, NLAYER)
+        for lid, layer in enumerate(layers):
+            with np.errstate(all="ignore"):
+                want = lo.decoder_layer_forward(paras[lid], lid, NLAYER, x, kv, mask, NH, IMS, True, "relu")
+            with torch.no_grad():
+                got = layer(to_dev(x), to_dev(enc).transpose(0, 1), to_dev(pad))
+            _check(got, want, np.ones(x.shape[:2], bool))
+    finally:
+        _release(layers)
