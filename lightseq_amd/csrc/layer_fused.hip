@@ -87,6 +87,22 @@ __device__ __forceinline__ void unit_halfs(const LayerPrepSection& s, int block)
   }
 }
 
+// eight normalised elements to where they go (`out`, `codes`: null where nobody reads them)
+__device__ __forceinline__ void ln_store(const half8_t& x, const half8_t& g, const half8_t& b, float mean, float rstd,
+                                         const Quantiser& of, __half* out, int8_t* codes) {
+  half8_t o;
+#pragma unroll
+  for (int k = 0; k < 8; ++k)
+    o.v[k] = __float2half_rn((__half2float(x.v[k]) - mean) * rstd * __half2float(g.v[k]) + __half2float(b.v[k]));
+  if (out) *reinterpret_cast<half8_t*>(out) = o;
+  if (codes) {
+    int q[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) q[k] = of.code(__half2float(o.v[k]));
+    *reinterpret_cast<uint2*>(codes) = make_uint2(pack4_i8(q[0], q[1], q[2], q[3]), pack4_i8(q[4], q[5], q[6], q[7]));
+  }
+}
+
 // Layer norm of one row by a wavefront (opb_layer_norm: var = E[x^2] - E[x]^2 + 1e-8), the row kept
 // in registers where it is at most 512 IT elements; the codes of the fp16 result, blocked.
 template <int IT>
@@ -121,19 +137,35 @@ __device__ __forceinline__ void ln_row(const __half* inp, __half* out, int8_t* c
   for (int it = 0; it < IT; ++it) {
     const int e = lane * 8 + it * 512;
     if (e >= hidden) continue;
-    half8_t o;
+    ln_store(raw[it], g[it], b[it], mean, rstd, of, out ? out + base + e : nullptr,
+             codes ? codes + blocked_offset(row, e, k_pad) : nullptr);
+  }
+}
+// Rows that do not fit the registers are read twice, the second time from the cache (in place: a lane
+// writes only what it has read itself).  Same sums in the same order.
+__device__ __forceinline__ void ln_row_long(const __half* inp, __half* out, int8_t* codes, const __half* gamma,
+                                            const __half* beta, const __half* cmax, int row, int hidden,
+                                            int k_pad) {
+  const int lane = threadIdx.x & 63;
+  const long base = (long)row * hidden;
+  float s = 0.f, s2 = 0.f;
+  for (int e = lane * 8; e < hidden; e += 512) {
+    const half8_t raw = *reinterpret_cast<const half8_t*>(inp + base + e);
 #pragma unroll
-    for (int k = 0; k < 8; ++k)
-      o.v[k] = __float2half_rn((__half2float(raw[it].v[k]) - mean) * rstd * __half2float(g[it].v[k]) +
-                               __half2float(b[it].v[k]));
-    if (out) *reinterpret_cast<half8_t*>(out + base + e) = o;
-    if (codes) {
-      int q[8];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) q[k] = of.code(__half2float(o.v[k]));
-      *reinterpret_cast<uint2*>(codes + blocked_offset(row, e, k_pad)) =
-          make_uint2(pack4_i8(q[0], q[1], q[2], q[3]), pack4_i8(q[4], q[5], q[6], q[7]));
+    for (int k = 0; k < 8; ++k) {
+      const float x = __half2float(raw.v[k]);
+      s += x;
+      s2 += x * x;
     }
+  }
+  const float mean = wave_sum(s) / (float)hidden;
+  const float var = wave_sum(s2) / (float)hidden - mean * mean + kLnEps;
+  const float rstd = rsqrtf(var);
+  const Quantiser of = Quantiser::of(codes ? cm(cmax) : 1.f);
+  for (int e = lane * 8; e < hidden; e += 512) {
+    const half8_t raw = *reinterpret_cast<const half8_t*>(inp + base + e);
+    ln_store(raw, *reinterpret_cast<const half8_t*>(gamma + e), *reinterpret_cast<const half8_t*>(beta + e), mean,
+             rstd, of, out ? out + base + e : nullptr, codes ? codes + blocked_offset(row, e, k_pad) : nullptr);
   }
 }
 __device__ __forceinline__ void ln_row_any(const __half* inp, __half* out, int8_t* codes, const __half* gamma,
@@ -142,7 +174,8 @@ __device__ __forceinline__ void ln_row_any(const __half* inp, __half* out, int8_
   if (hidden <= 512) ln_row<1>(inp, out, codes, gamma, beta, cmax, row, hidden, k_pad);
   else if (hidden <= 1024) ln_row<2>(inp, out, codes, gamma, beta, cmax, row, hidden, k_pad);
   else if (hidden <= 2048) ln_row<4>(inp, out, codes, gamma, beta, cmax, row, hidden, k_pad);
-  else ln_row<8>(inp, out, codes, gamma, beta, cmax, row, hidden, k_pad);
+  else if (hidden <= 4096) ln_row<8>(inp, out, codes, gamma, beta, cmax, row, hidden, k_pad);
+  else ln_row_long(inp, out, codes, gamma, beta, cmax, row, hidden, k_pad);
 }
 
 // the additive fp16 mask of the layers, half(value * -1e8), from whatever the caller's mask is made of
@@ -249,7 +282,7 @@ int LayerPrep::halfs(const __half* src, __half* dst, const __half* cmax, int row
 }
 int LayerPrep::norm(const __half* src, int8_t* dst, const __half* gamma, const __half* beta,
                     const __half* cmax, int rows, int hidden, int k_pad) {
-  if (!src || !dst || !gamma || !beta || !cmax || rows <= 0 || hidden <= 0 || hidden % 8 != 0 || hidden > 4096)
+  if (!src || !dst || !gamma || !beta || !cmax || rows <= 0 || hidden <= 0 || hidden % 8 != 0)
     return lsh_fail(LSH_ERR_INVALID, "layer_prep: bad layer norm");
   LayerPrepSection s{};
   s.kind = kPrepNorm;
@@ -305,7 +338,7 @@ int LayerPrep::launch(hipStream_t s) const {
 int layer_norm_codes(const __half* inp, __half* out, int8_t* codes, const __half* gamma, const __half* beta,
                      const __half* cmax, int rows, int hidden, int k_pad, hipStream_t s) {
   if (!inp || (!out && !codes) || !gamma || !beta || (codes && !cmax) || rows <= 0 || hidden <= 0 ||
-      hidden % 8 != 0 || hidden > 4096)
+      hidden % 8 != 0)
     return lsh_fail(LSH_ERR_INVALID, "layer_norm_codes: bad arguments");
   layer_norm_codes_kernel<<<(rows + 3) / 4, 256, 0, s>>>(inp, out, codes, gamma, beta, cmax, rows, hidden,
                                                          k_pad);

@@ -1,4 +1,5 @@
-"""The quantised layers at the ends of what they accept: elements that are no finite numbers."""
+"""The quantised layers at the ends of what they accept: elements that are no finite numbers, rows
+wider than a wavefront's registers."""
 import numpy as np
 import pytest
 import torch
@@ -12,13 +13,13 @@ pytestmark = pytest.mark.gpu
 INF = np.float16(np.inf)
 
 
-def _check(got, want, rows):
+def _check(got, want, rows, bar=2e-2):
     """Outputs of the finite rows, within the bar of the layer tests."""
     got, want = to_np(got).astype(np.float64)[rows], want.astype(np.float64)[rows]
     assert np.isfinite(want).all()
     assert np.isfinite(got).all()
     d = np.abs(got - want)
-    assert d.max() < 2e-2 and d.mean() < 1e-3, (d.max(), d.mean())
+    assert d.max() < bar and d.mean() < 1e-3, (d.max(), d.mean())
 
 
 @pytest.mark.parametrize("pre_ln,act", [(False, "relu"), (False, "gelu"), (True, "relu"), (True, "gelu")])
@@ -77,3 +78,20 @@ def test_infinite_elements_of_a_decoder_layer():
             _check(got, want, np.ones(x.shape[:2], bool))
     finally:
         _release(layers)
+
+
+@pytest.mark.parametrize("hs,nh,pre_ln", [(1536, 24, False), (2080, 65, True), (4096, 32, False), (4128, 129, False),
+                                          (4128, 129, True), (5120, 40, True)])
+def test_wide_layers(hs, nh, pre_ln):
+    """The layer norm by every number of registers a row takes, and by rereading it beyond 4096."""
+    from test_oracle_layer_ops import config0
+    batch, seq, ims = 2, 5, 64
+    cfg0 = config0(np.random.default_rng(hs), pre_ln, "gelu", batch, seq, hs, nh, ims)
+    layer, para = _make_layer(cfg0, pre_ln, "gelu", nh, 16, 8)
+    x = cfg0[1].astype(np.float16)
+    with torch.no_grad():
+        got = layer(to_dev(x), torch.zeros(batch, seq, device="cuda"))
+    want = _lo().encoder_layer_forward(para, x, np.zeros((batch, seq), np.float16), nh, ims, pre_ln, "gelu")
+    # a code of the output projection that another order of sums moves by one is one step of it,
+    # which grows with the width
+    _check(got, want, np.ones((batch, seq), bool), 2e-2 + cfg0[2]["out_out"] / 127)
