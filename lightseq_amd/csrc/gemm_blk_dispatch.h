@@ -43,8 +43,10 @@ int raise_lds(size_t smem) {
   return LSH_OK;
 }
 
+// grid.x: output tiles, which tile_of counts in 24 bits
 template <auto Kern, typename... Args>
 int launch_blk(dim3 grid, int threads, size_t smem, hipStream_t s, Args... args) {
+  if (grid.x >= (1u << 24)) return lsh_fail(LSH_ERR_UNSUPPORTED, "blocked gemm: more than 2^24 output tiles");
   if (int rc = raise_lds<Kern>(smem)) return rc;
   hipEvent_t e0, e1;
   if (gemm_take_timing_events(&e0, &e1))
@@ -98,10 +100,8 @@ inline int check_blk(const int8_t* A, const int8_t* W, bool aligned, int M, int 
     return lsh_fail(LSH_ERR_UNSUPPORTED, "blocked gemm: needs K bytes % 64 == 0 and N % 4 == 0");
   if (((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W)) & 15u) != 0 || !aligned)
     return lsh_fail(LSH_ERR_INVALID, "blocked gemm: operands must be 16-byte aligned");
-  const unsigned long long lim = 0xffffffffull;
-  if ((unsigned long long)(M + 15) / 16 * 16 * K >= lim || (unsigned long long)(N + 15) / 16 * 16 * K >= lim ||
-      (long)((M + 15) / 16) * ((N + 15) / 16) >= (1L << 24))
-    return lsh_fail(LSH_ERR_UNSUPPORTED, "blocked gemm: operand or output too large");
+  if (K >= (1 << 24) || M > 0x7fffff00 || N > 0x7fffff00 || (long)((M + 15) / 16) * ((N + 15) / 16) >= (1L << 31))
+    return lsh_fail(LSH_ERR_UNSUPPORTED, "blocked gemm: operand too large");
   return LSH_OK;
 }
 

@@ -63,7 +63,9 @@ constexpr int kw_lds_bytes() {
 // grid: tiles_m * tiles_n workgroups of 256, times ksplit in y (range y of K stores to rows
 // [y M, (y + 1) M) of the output).  K in bytes, `slices` = the 64-byte slices of a range.
 // D > 1: slices % (4 D) == 0; D == 1: any number.  Preconditions: K % 64 == 0, N % 4 == 0,
-// operands 16-byte aligned, below 2^32 bytes and allocated in whole blocks of 16 rows.
+// operands 16-byte aligned and allocated in whole blocks of 16 rows.  A tile's operands have a
+// 64-bit base and 32-bit offsets, so it is the tile (K below 2^24 bytes) and not the matrix that
+// has to stay below 4 GiB.
 template <typename Tr, typename Epi, int MB, int NB, int D>
 __global__ void __launch_bounds__(256, 2)
 gemm_kw_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, Epi epi, int M, int N,
@@ -104,15 +106,15 @@ gemm_kw_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, Epi e
   const int first = (int)blockIdx.y * slices;
   const int s0 = first + (D > 1 ? wave * (slices / 4) : wave * slices / 4);
   const int ns = D > 1 ? slices / 4 : (wave + 1) * slices / 4 - wave * slices / 4;
-  const int8_t* a_base = A + (long)s0 * 1024;
-  const int8_t* w_base = W + (long)s0 * 1024;
+  const int8_t* a_base = A + (long)m0 * K + (long)s0 * 1024;
+  const int8_t* w_base = W + (long)n0 * K + (long)s0 * 1024;
   uint32_t a_off[MB], w_off[NB];
 #pragma unroll
   for (int i = 0; i < MB; ++i)
-    a_off[i] = (uint32_t)min(m0 + 16 * i, (M - 1) & ~15) * (uint32_t)K + lane * 16;
+    a_off[i] = (uint32_t)min(16 * i, ((M - 1) & ~15) - m0) * (uint32_t)K + lane * 16;
 #pragma unroll
   for (int b = 0; b < NB; ++b)
-    w_off[b] = (uint32_t)min(n0 + 16 * b, (N - 1) & ~15) * (uint32_t)K + lane * 16;
+    w_off[b] = (uint32_t)min(16 * b, ((N - 1) & ~15) - n0) * (uint32_t)K + lane * 16;
   v4i fa[D][MB], fw[D][NB];
   auto load = [&](int u, int s) {
     const int8_t* a = a_base + s * 1024;
@@ -204,17 +206,19 @@ gemm_seq_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, Epi 
   typename Epi::Col col[NB];
 #pragma unroll
   for (int b = 0; b < NB; ++b) col[b] = epi.column(min(n0 + 16 * b + 4 * kq, N - 4), N);
+  const int8_t* a_base = A + (long)m0 * K;
+  const int8_t* w_base = W + (long)n0 * K;
   uint32_t a_off[MB], w_off[NB];
 #pragma unroll
   for (int i = 0; i < MB; ++i)
-    a_off[i] = (uint32_t)min(m0 + 16 * i, (M - 1) & ~15) * (uint32_t)K + lane * 16;
+    a_off[i] = (uint32_t)min(16 * i, ((M - 1) & ~15) - m0) * (uint32_t)K + lane * 16;
 #pragma unroll
   for (int b = 0; b < NB; ++b)
-    w_off[b] = (uint32_t)min(n0 + 16 * b, (N - 1) & ~15) * (uint32_t)K + lane * 16;
+    w_off[b] = (uint32_t)min(16 * b, ((N - 1) & ~15) - n0) * (uint32_t)K + lane * 16;
   v4i fa[D][MB], fw[D][NB];
   auto load = [&](int u, int s) {
-    const int8_t* a = A + s * 1024;
-    const int8_t* w = W + s * 1024;
+    const int8_t* a = a_base + s * 1024;
+    const int8_t* w = w_base + s * 1024;
 #pragma unroll
     for (int b = 0; b < NB; ++b) fw[u][b] = *reinterpret_cast<const v4i*>(w + w_off[b]);
 #pragma unroll

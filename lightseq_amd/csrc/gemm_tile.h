@@ -219,9 +219,10 @@ __device__ __forceinline__ void tile_of(int t, int nblk, int tiles_m, int tiles_
 // into the stage that the second-to-last step frees, while the last step is multiplied.
 // Every wavefront of the workgroup must call it (it holds workgroup barriers: tile_gemm_barriers
 // of them); the caller separates two calls by a barrier of its own.
-// Preconditions: K % 128 == 0, K / 128 >= NST, N % 16 == 0, 32-bit operand offsets, operands
-// 16-byte aligned.  A_FROM_L2: the rows of A were written by other compute units of this XCD
-// during this launch (read past the vector cache).  BLOCKED: both operands in the blocked layout.
+// Preconditions: K % 128 == 0, K / 128 >= NST, N % 16 == 0, operands 16-byte aligned and below 2^32
+// bytes (BLOCKED: K below 2^24, the offsets count from the tile).  A_FROM_L2: the rows of A were
+// written by other compute units of this XCD during this launch (read past the vector cache).
+// BLOCKED: both operands in the blocked layout, row0 a multiple of 16.
 // ---------------------------------------------------------------------------------
 template <typename Epi, typename = void>
 struct EpiHasClips : std::false_type {};
@@ -276,6 +277,11 @@ __device__ __forceinline__ void tile_gemm(const int8_t* __restrict__ A,
   const int wm = wave / WGN, wn = wave % WGN, l32 = lane & 31, g = lane >> 5;
   const int nk = K / kBK;
 
+  const int8_t *a_tile = A, *w_tile = W;
+  if (BLOCKED) {
+    a_tile += (long)row0 * K;
+    w_tile += (long)tn * TN * K;
+  }
   uint32_t a_src[NA], w_src[NW];
 #pragma unroll
   for (int i = 0; i < NA; ++i) {
@@ -286,7 +292,7 @@ __device__ __forceinline__ void tile_gemm(const int8_t* __restrict__ A,
       // one 1-KB block of 16 rows x 64 bytes per load, as it lies in memory: it is in fragment
       // order already, and 16 lanes of a fragment read are 256 contiguous bytes of LDS
       const int q = wave + NWV * i;
-      a_src[i] = (uint32_t)min((row0 >> 4) + (q >> 1), (row_end - 1) >> 4) * 16u * (uint32_t)K +
+      a_src[i] = (uint32_t)min(q >> 1, ((row_end - 1) >> 4) - (row0 >> 4)) * 16u * (uint32_t)K +
                  (q & 1) * 1024 + lane * 16;
     }
   }
@@ -299,7 +305,7 @@ __device__ __forceinline__ void tile_gemm(const int8_t* __restrict__ A,
       // the two halves of an odd block's rows change places: 16 lanes in sigma order read eight
       // rows of an even and the same eight of the odd block, which must not share their banks
       const int q = wave + NWV * i;
-      w_src[i] = (uint32_t)min(tn * (TN / 16) + (q >> 1), (N - 1) >> 4) * 16u * (uint32_t)K +
+      w_src[i] = (uint32_t)min(q >> 1, ((N - 1) >> 4) - tn * (TN / 16)) * 16u * (uint32_t)K +
                  (q & 1) * 1024 + (lane ^ ((q >> 1) & 1) * 8) * 16;
     }
   }
@@ -322,12 +328,12 @@ __device__ __forceinline__ void tile_gemm(const int8_t* __restrict__ A,
     const uint32_t base = lds0 + slot * STAGE;
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
-      if (A_FROM_L2) dma1_l2(A + kt * KSTEP, a_src[i], base + (wave + NWV * i) * 1024);
-      else dma1(A + kt * KSTEP, a_src[i], base + (wave + NWV * i) * 1024);
+      if (A_FROM_L2) dma1_l2(a_tile + kt * KSTEP, a_src[i], base + (wave + NWV * i) * 1024);
+      else dma1(a_tile + kt * KSTEP, a_src[i], base + (wave + NWV * i) * 1024);
     }
 #pragma unroll
     for (int i = 0; i < NW; ++i)
-      dma1(W + kt * KSTEP, w_src[i], base + TM * kBK + (wave + NWV * i) * 1024);
+      dma1(w_tile + kt * KSTEP, w_src[i], base + TM * kBK + (wave + NWV * i) * 1024);
   };
   // LDS byte offset of this lane's fragment chunk for K slice 0; slice ks is at (offset ^ (ks << 5)):
   // chunk index 2 * ks + g, swizzled by the row key, and 2 * ks only touches bits 1-2 of it
