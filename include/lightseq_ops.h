@@ -330,7 +330,7 @@ int ls_destroy_layer(const char* layer_name, int layer_id);
  * padding) of element type mask_type -- 0: the additive fp16 mask of the fw functions; 1: float,
  * 2: fp16, 3: 8-bit (bool), 4: int32, 5: int64.  enc_output of the decoder layer: token s of
  * sentence b at b * enc_stride_batch + s * enc_stride_seq (elements, multiples of 8; hidden values
- * contiguous); layer 0 reads it where it makes the cross-attention keys and values (step <= 0).
+ * contiguous, the first 16-byte aligned); layer 0 reads it where it makes the cross-attention keys and values (step <= 0).
  * The five cache pointers are those of ls_transformer_decoder_layer_fw_fp16. */
 int ls_encoder_layer_call_fp16(int layer_id, const void* weights, const void* input, const void* padding_mask,
                                int mask_type, void* output, int batch_size, int seq_len,

@@ -12,6 +12,10 @@
 // same codes multiplied in int8 give exact sums at half the bytes, but those differ from the
 // sums of the fp16-rounded values by about one unit of fp16, which after a few layers has moved
 // enough codes by one to be seen (4 % of a six-layer output).
+//
+// aligned() of these epilogues has nothing to ask: a layer call takes parameters, residual and output
+// at any address, as the streaming kernels did (vector accesses to global memory need no
+// alignment here); the operands are the layer's own buffers, which check_blk looks at.
 #include "gemm_blk_dispatch.h"
 #include "gemm_dec_epi.h"
 #include "layer_device.h"

@@ -221,6 +221,9 @@ void TransformerDecoderLayer<T>::Forward(const T* dec_input_ptr, const T* enc_ou
   if (makes_encdec_kv()) {
     // :236-262: fake-quantised weights, the encoder output as it is
     if (!enc_output_ptr) throw std::runtime_error("Forward: null encoder output");
+    if (reinterpret_cast<uintptr_t>(enc_output_ptr) % 16 != 0 || (_batch_size > 1 && enc_stride_b % 8 != 0) ||
+        (_src_seq_len > 1 && enc_stride_s % 8 != 0))
+      throw std::runtime_error("Forward: the encoder output must be 16-byte aligned, its strides multiples of 8");
     if (!_encdec_attn_kvw_ptr)
       throw std::runtime_error("Forward: layer 0 holds no cross-attention k/v weights");
     const size_t enc_elems = (((size_t)_max_batch_tokens + 15) & ~(size_t)15) * _kh;

@@ -354,9 +354,10 @@ class LSTransformerDecoderLayer(nn.Module):
         # and in the first one; it reads the encoder output where it lies
         enc = encoder_out
         if cfg.layer_id == 0 and step <= 0:
-            if (enc.dtype != torch.half or enc.stride(2) != 1 or enc.stride(0) % 8 or enc.stride(1) % 8
-                    or enc.data_ptr() % 16):
-                enc = enc.to(torch.half).contiguous()
+            if (enc.dtype != torch.half or enc.stride(2) != 1 or (src_len > 1 and enc.stride(0) % 8)
+                    or (batch > 1 and enc.stride(1) % 8) or enc.data_ptr() % 16):
+                # (memory of its own: for a contiguous view contiguous() would be the view)
+                enc = torch.empty(enc.shape, dtype=torch.half, device=enc.device).copy_(enc)
         output = torch.empty_like(decoder_states)
         pointers = [ptr(t) for t in cache_list] if cache_list is not None else [None] * 5
         training = self.training and cache is None

@@ -1,5 +1,5 @@
 """The quantised layers at the ends of what they accept: elements that are no finite numbers, rows
-wider than a wavefront's registers."""
+wider than a wavefront's registers, encoder outputs at odd places."""
 import numpy as np
 import pytest
 import torch
@@ -95,3 +95,49 @@ def test_wide_layers(hs, nh, pre_ln):
     # a code of the output projection that another order of sums moves by one is one step of it,
     # which grows with the width
     _check(got, want, np.ones((batch, seq), bool), 2e-2 + cfg0[2]["out_out"] / 127)
+
+
+def test_encoder_output_at_any_place():
+    """A view that is not 16-byte aligned, or whose strides are no multiples of 8, gives the bits of
+    an aligned tensor (a stride that a single sentence or token does not use says nothing);
+    the C call refuses what its contract excludes."""
+    from lightseq_amd import lib
+    for batch, src in ((2, 12), (1, 12), (2, 1)):
+        paras, x, enc, pad, mask = _case(7, batch, 9, src)
+        layers = _make_stack(paras, True, "relu", 64, 32)
+        layer, hs = layers[0], x.shape[-1]
+        try:
+            xd, padd = to_dev(x), to_dev(pad)
+            aligned = to_dev(np.ascontiguousarray(enc.transpose(1, 0, 2)))
+            n = aligned.numel()
+            odd = torch.empty(n + 8, dtype=torch.half, device="cuda")[3:n + 3].view(aligned.shape).copy_(aligned)
+            assert odd.is_contiguous() and odd.data_ptr() % 16 == 6
+            wide = torch.empty(src, batch, hs + 4, dtype=torch.half, device="cuda")[..., :hs].copy_(aligned)
+            places = [odd, wide]
+            if batch == 1:
+                places.append(aligned.as_strided(aligned.shape, (hs, 7, 1)))
+            if src == 1:
+                places.append(aligned.as_strided(aligned.shape, (7, hs, 1)))
+            with torch.no_grad():
+                want = layer(xd, aligned, padd)
+                for place in places:
+                    assert torch.equal(layer(xd, place, padd), want)
+            out = torch.empty_like(xd)
+
+            def call(address, stride_b, stride_s):
+                lib.call("ls_decoder_layer_call_fp16", 0, lib.ptr(layer.para), lib.ptr(xd), address, stride_b,
+                         stride_s, lib.ptr(padd), 1, lib.ptr(out), batch, 9, src, -1, *[None] * 5, 0, 1,
+                         lib.current_stream())
+
+            refused = [(odd.data_ptr(), hs, batch * hs)]
+            if batch > 1:
+                refused.append((aligned.data_ptr(), 4, batch * hs))
+            if src > 1:
+                refused.append((aligned.data_ptr(), hs, 4))
+            for args in refused:
+                with pytest.raises(lib.LSHError, match="16-byte aligned"):
+                    call(*args)
+            call(aligned.data_ptr(), hs, batch * hs)
+            assert torch.equal(out, want)
+        finally:
+            _release(layers)
