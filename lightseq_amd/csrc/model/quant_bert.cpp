@@ -58,11 +58,26 @@ void QuantBert::infer(void* host_out, bool host_f16) {
   set_output_shape(0, {batch_size, seq_len, tw_._hidden_size});
 }
 
+// Where the GPU sees `bytes` bytes of the caller's memory.  A kernel writes there: memory that was not
+// allocated as pinned would be a fault, so it is asked for first.
+static void* device_view(void* p, size_t bytes) {
+  hipPointerAttribute_t first{}, last{};
+  const bool known = hipPointerGetAttributes(&first, p) == hipSuccess &&
+                     hipPointerGetAttributes(&last, static_cast<char*>(p) + bytes - 1) == hipSuccess;
+  if (!known) (void)hipGetLastError();
+  if (!known || first.type == hipMemoryTypeUnregistered || !first.devicePointer ||
+      static_cast<char*>(last.devicePointer) != static_cast<char*>(first.devicePointer) + bytes - 1)
+    throw std::runtime_error("host_out is not pinned host memory of the size of the output");
+  return first.devicePointer;
+}
+
 void QuantBert::InferHost(const int* ids, int batch, int seq_len, void* host_out, bool host_f16) {
   // more ids than the input holds: Infer() names the limit that was passed
   const size_t n = (size_t)std::max(batch, 0) * (size_t)std::max(seq_len, 0);
-  if (ids && n > 0 && n <= d_input_.size())
+  if (ids && n > 0 && n <= d_input_.size()) {
+    if (host_out) host_out = device_view(host_out, n * tw_._hidden_size * (host_f16 ? sizeof(__half) : sizeof(float)));
     h_ids_.upload(ids, n, d_input_.get(), d_input_.size(), stream_);
+  }
   set_input_ptr(0, d_input_.get());
   set_input_shape(0, {batch, seq_len});
   HostIdsScope scope(host_ids_, ids);
