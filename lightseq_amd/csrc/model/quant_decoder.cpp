@@ -259,11 +259,6 @@ void QuantDecoder::run_one_infer(int batch_size, int batch_seq_len) {
   const int limit = _batch_max_decode_length - 1;
   if (!_is_benchmark && !_use_graphs && !_rec_logits && !_rec_alive && !step_taps.any() &&
       emb_ln_fused()) {
-    // Whether a step is needed is known while the device works at its layers.  All of them are
-    // enqueued before the host waits: it enqueues a launch in 2.5 us where the device takes 3.3,
-    // so what it is ahead when the word comes is what covers its hiccups of 100 us and more.
-    // 16 x 64 tokens, beam 4: 32.4 ms with one layer, 31.4 with four, 30.9 with the six.  A run
-    // that stops early pays for the layers of one step.
     const int L = _tw._n_dec_layer;
     for (_cur_step = 0; _cur_step < limit; _cur_step++) {
       if (_cur_step == 0) {
@@ -279,9 +274,12 @@ void QuantDecoder::run_one_infer(int batch_size, int batch_seq_len) {
       }
       ++_cur_step;
       step_begin(_notice.next(search ? _num_finished.get() : _sample_unfinished.get()));
-      step_layers(0, L);
+      const int ahead = layers_ahead(_cur_step, L);
+      step_layers(0, ahead);
+      const bool stop = finished(search, _notice.wait(_stream));
+      if (!stop) step_layers(ahead, L);
       --_cur_step;
-      if (finished(search, _notice.wait(_stream))) break;
+      if (stop) break;
     }
   } else {
     for (_cur_step = 0; _cur_step < limit; _cur_step++) {

@@ -475,16 +475,10 @@ int QuantGptEncoder::run_one_sample(int batch_size, int batch_seq_len) {
     count_token();
     const int L = _tw._n_enc_layer;
     if (!_is_benchmark && !_use_graphs && !_rec_logits && emb_ln_fused()) {
-      // Whether a step is needed is known while the device works at its layers.  Three quarters of
-      // them are enqueued before the host waits for the word: it enqueues a launch in 2.5 us where
-      // the device takes 3.4, so what it is ahead when the word comes is what covers its hiccups
-      // of 100 us and more.  GPT-2-medium, 128 tokens after 45: 66.6 ms with 2 layers of the 24,
-      // 63.7 with 12, 60.6 with 18, 62.2 with all; 16 sequences after 512: 96.1, 94.1, 90.3, 90.6.
-      // A run that stops early pays for these layers once.
-      const int ahead = L - L / 4;
       _phases.mark(1, _stream);
       while (_batch_seq_len < _batch_max_seq_len) {
         step_begin(_notice.next(_unfinished.get()));
+        const int ahead = layers_ahead(loop_steps + 1, L);
         step_layers(0, ahead);
         if (_notice.wait(_stream) == 0) break;
         ++loop_steps;
