@@ -266,7 +266,10 @@ gemm_seq_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, Epi 
 // third when every compute unit works), each further one s0 + s1 k, with the table epilogue
 // `table` more per tile.  The constants are a fit to a sweep of every tile over M from 16 to 7680
 // and the four products of a layer at hidden 768 and 1024 (K from 768 to 4096); over that sweep
-// the tile with the smallest estimate is 2 % slower than the fastest on average.
+// the tile with the smallest estimate is 2 % slower than the fastest on average.  (All tiles slow
+// down alike when more than half of the compute units work, up to half as much again with long K,
+// so that what is left out there does not change the choice: the LDS tiles over eight products
+// and M from 256 to 8192, 1.6 % on average and 7 % at the 95th percentile.)
 // ---------------------------------------------------------------------------------
 struct TileCost {
   int tm, tn;
@@ -277,9 +280,7 @@ inline float tile_us(const TileCost& c, int M, int N, int K, int ksplit, int cus
       (long)((M + c.tm - 1) / c.tm) * ((N + c.tn - 1) / c.tn) * ksplit;
   const float per = (float)((tiles + cus - 1) / cus), k = K / 1024.f;
   const float busy = tiles < cus ? (float)tiles / cus : 1.f;
-  float first = c.a + c.b * k * (1.f + 0.35f * busy);
-  // tiles that have a compute unit to themselves take longer once nearly all of them do
-  if (c.tm == 256 && c.tn < 256 && tiles <= cus && busy > 0.8f) first += 4.f;
+  const float first = c.a + c.b * k * (1.f + 0.35f * busy);
   return first + (per - 1.f) * (c.s0 + c.s1 * k) + (table ? per * c.table : 0.f);
 }
 constexpr TileCost kKwCost[] = {{16, 16, 2.3f, 0.2f, 0.05f, 0.2f, 0.03f},
