@@ -947,7 +947,7 @@ static int launch_long_attn(int seq_len, int batch_heads, hipStream_t s, const _
   // tiles: LDS has room for two workgroups of a compute unit with two blocks of keys, for one with
   // more, and wavefronts that share a workgroup are what hides latency then.
   const int tiles = (seq_len + 31) / 32, nkb = (key_len + 127) / 128;
-  const int room = nkb == 2 ? 512 : 256;
+  const int room = (nkb == 2 ? 2 : 1) * cu_count();
   const int parts = std::max((tiles + 15) / 16, std::min(room / std::max(batch_heads, 1), (tiles + 3) / 4));
   const int nw = (tiles + parts - 1) / parts;
   long_attn_kernel<MODE><<<dim3((tiles + nw - 1) / nw, batch_heads), 64 * nw, long_attn_lds(nkb), s>>>(

@@ -149,29 +149,33 @@ int dispatch_blk(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K,
 
 // fp16 products: every output one chain in ascending K (gemm_seq_kernel).  The estimates, in us with k
 // = K in units of 1000 bytes, are fits to a sweep of hidden 512, 768 and 1024 (K of one and of
-// four times that) over M from 4 to 8192; the smallest one is within 15 % of the fastest there.
+// four times that) over M from 4 to 8192 on 256 compute units; the smallest one is within 15 % of
+// the fastest there.  What a launch takes beyond one round of the chip goes by the tiles per
+// compute unit.
 struct SeqTile {
   int kind;  // 0: a wavefront per 16 x 16, 1: per 32 x 32; 2 - 4: LDS tiles 64 x 64, 128 x 64,
              // 128 x 128; 5: the last with a third stage
   float us;
 };
-inline SeqTile choose_seq(int M, int N, int K) {
+inline SeqTile choose_seq(int M, int N, int K, int cus) {
   const float k = (float)K / 1000.f;
-  auto tiles = [&](int tm, int tn) { return (float)((long)((M + tm - 1) / tm) * ((N + tn - 1) / tn)); };
-  auto lds = [&](float t, float first, float more) {
-    return 2.f + first * k + (t > 256.f ? (t / 256.f - 1.f) * (1.f + more * k) : 0.f);
+  auto tiles = [&](int tm, int tn) {  // per compute unit
+    return (float)((long)((M + tm - 1) / tm) * ((N + tn - 1) / tn)) / (float)cus;
   };
-  SeqTile best{0, std::max(std::max(2.8f, 0.9f + 0.5f * k), 2.f + 0.00095f * tiles(16, 16) * k)};
+  auto lds = [&](float t, float first, float more) {
+    return 2.f + first * k + (t > 1.f ? (t - 1.f) * (1.f + more * k) : 0.f);
+  };
+  SeqTile best{0, std::max(std::max(2.8f, 0.9f + 0.5f * k), 2.f + 0.2432f * tiles(16, 16) * k)};
   auto take = [&](int kind, float us) {
     if (us < best.us) best = SeqTile{kind, us};
   };
-  take(1, std::max(1.f + 1.2f * k, 2.f + 0.0022f * tiles(32, 32) * k));
+  take(1, std::max(1.f + 1.2f * k, 2.f + 0.5632f * tiles(32, 32) * k));
   if (K % kBK == 0 && K / kBK >= 3 && N % 16 == 0) {
     take(2, lds(tiles(64, 64), 1.9f, 1.4f));
     take(3, lds(tiles(128, 64), 3.7f, 1.8f));
     // with no more tiles than compute units a tile has a unit's LDS to itself: 3000 x 1024 x 4096 in
     // 33.7 us instead of 39.9 (beyond that two tiles a unit are better: 8192 rows 52.0, not 65.8)
-    if (tiles(128, 128) <= 256.f) take(5, lds(tiles(128, 128), 3.85f, 0.f));
+    if (tiles(128, 128) <= 1.f) take(5, lds(tiles(128, 128), 3.85f, 0.f));
     else take(4, lds(tiles(128, 128), 4.5f, 2.2f));
   }
   return best;
@@ -196,7 +200,7 @@ template <typename Epi>
 int dispatch_f16(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K, hipStream_t s) {
   if (int rc = check_blk(A, W, epi.aligned(), M, N, K)) return rc;
   const int slices = K / 64;
-  switch (choose_seq(M, N, K).kind) {
+  switch (choose_seq(M, N, K, cu_count()).kind) {
     case 0:
       if (slices % 16 == 0) return launch_seq<Epi, 1, 16>(A, W, epi, M, N, K, s);
       if (slices % 8 == 0) return launch_seq<Epi, 1, 8>(A, W, epi, M, N, K, s);
