@@ -7,8 +7,10 @@ valid lengths uniform in [32, 128] with right padding, token ids uniform over a
 30522 vocabulary, random-init weights ~N(0, 0.02) quantised per tensor -- run
 through the drop-in entry point ``QuantBert(path, max_batch)`` / ``LSModel::Infer``.
 A step is one ``Infer()`` over one batch whose token ids are already resident in
-HBM.  ``value`` = batch * seq_len * steps / wall time of the timed steps (padded
-tokens counted, as the reference's b32 x s128 figures do).
+HBM.  ``value`` = batch * seq_len * steps / wall time of the timed steps: positions of the
+padded batch, as the reference's b32 x s128 figures count them, although the rows of padding are
+left out of the computation.  ``config`` says so (``value_counts``) and how many of the positions
+are tokens (``valid_tokens``; ``valid_tokens_per_s`` is the rate that counts only those).
 
 The JSON line also carries
   roofline       the dominant kernel launch (by total time) among the int8 GEMM sites
@@ -263,8 +265,8 @@ def gemm_microbench(reps=40):
             "int8 out (requantising epilogue)": lambda: K.gemm_i8_i8o(a, w, c8, M, N, Kd, alpha),
             "int8 out, bias+GELU+requant fused": lambda: K.gemm_i8_bias_gelu_i8o(
                 a, w, c8, bias, M, N, Kd, alpha, clip_out / 127, 127 / clip_act),
-            "int8 out, bias+GELU+requant fused through the per-column table (what the models run; "
-            "same bytes)": lambda: K.gemm_i8_lut_i8o(a, w, c8, lut, M, N, Kd, alpha),
+            "int8 out, bias+GELU+requant fused through the per-column table (row-major operands; the "
+            "models run the same epilogue on blocked ones)": lambda: K.gemm_i8_lut_i8o(a, w, c8, lut, M, N, Kd, alpha),
         }
         res = {}
         for name, fn in cases.items():
@@ -508,6 +510,9 @@ def bench_bert(args):
                                "FFN 3072 GELU, batch 32 x seq 128, valid lengths U[32,128] right-padded, "
                                "vocab 30522, random-init N(0,0.02) weights quantised per tensor",
                    "batch": BATCH, "seq_len": SEQ, "valid_tokens": int(lens.sum()),
+                   "value_counts": "positions of the padded batch (batch * seq_len a step); rows of "
+                                   "padding are not computed",
+                   "valid_tokens_per_s": float(lens.sum()) * args.steps / dt,
                    "entry_point": "QuantBert / LSModel::Infer"},
         "roofline": roofline,
     }

@@ -54,6 +54,31 @@ def test_infinite_elements_take_the_outermost_codes(pre_ln, act, seq):
     _check(got, want, rows)
 
 
+@pytest.mark.parametrize("act", ["relu", "gelu"])
+def test_a_nan_has_the_code_of_minus_infinity(act):
+    """Input or weight: the lesser bound, so that rows without one have the same bits either way."""
+    from test_oracle_layer_ops import config0
+    lo = _lo()
+    batch, seq, hs, nh, ims = 2, 17, 128, 2, 256
+    layer, para = _make_layer(config0(np.random.default_rng(4), False, act, batch, seq, hs, nh, ims), False, act, nh,
+                              512, 256)
+    x = config0(np.random.default_rng(5), False, act, batch, seq, hs, nh, ims)[1].astype(np.float16)
+    outs = []
+    for value in (np.float16(np.nan), -INF):
+        q = para.copy()
+        p = lo.split_params(q, hs, ims)
+        p["attn_qkvw"][hs + 3, 5] = p["attn_ow"][4, 6] = p["inter_w"][8, 2] = p["output_w"][1, 3] = value
+        y = x.copy()
+        y[0, 4, 5] = y[1, 16, 7] = value
+        with torch.no_grad():
+            layer.para.copy_(to_dev(q))
+            outs.append(to_np(layer(to_dev(y), torch.zeros(batch, seq, device="cuda"))))
+    rows = np.ones((batch, seq), bool)
+    rows[0, 4] = rows[1, 16] = False
+    assert np.isfinite(outs[0][rows]).all() and not np.isfinite(outs[0][~rows]).any()
+    np.testing.assert_array_equal(outs[0][rows], outs[1][rows])
+
+
 def test_infinite_elements_of_a_decoder_layer():
     """The same with keys and values that the layer fake-quantises for its cache."""
     lo = _lo()
