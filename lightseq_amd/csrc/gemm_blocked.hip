@@ -1,4 +1,4 @@
-// int8 and fp16 products on blocked operands (tile_common.h names the layout): what the models and
+// int8 and fp16 products on blocked operands (blocked_offset in ls_device.h is the layout): what the models and
 // layers run.  Weights are blocked once at load; activations are written blocked by the kernel
 // that produces them (layer norm, attention, the table epilogue), so no product waits for a
 // rearrangement.

@@ -1,9 +1,9 @@
 // fp16 GEMM with fp32 accumulation on v_mfma_f32_32x32x16_f16:
 //   C[M,N] = A[M,K] * W[N,K]^T, both operands K-contiguous, C row-major.
 //
-// Used once per translation request to project the encoder output onto the keys and
-// values of every decoder layer (inference/model/quant_decoder.cc.cu:489-501), so it
-// is written for simplicity: a workgroup of 4 wavefronts owns a 64 x 128 tile, each
+// Projects the encoder output onto the keys and values of every decoder layer, once per
+// translation request (inference/model/quant_decoder.cc.cu:489-501), where the widths do not
+// block (gemm_blk_kv_f16 otherwise), so it is written for simplicity: a workgroup of 4 wavefronts owns a 64 x 128 tile, each
 // wavefront a 64 x 32 slice of it, and the MFMA operands are loaded straight from
 // global memory (one 16-byte row fragment per lane and k-step; rows beyond the
 // matrix are clamped for the loads and masked for the stores).

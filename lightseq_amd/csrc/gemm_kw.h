@@ -4,7 +4,7 @@
 //
 //   C[M,N] = epilogue( sum_k A[M,k] * W[N,k] )      int8 x int8 -> int32 or fp16 x fp16 -> fp32
 //
-// Blocked operands (tile_common.h): 16 rows x 64 bytes of K are 1 KB in the order in which the
+// Blocked operands (blocked_offset in ls_device.h): 16 rows x 64 bytes of K are 1 KB in the order in which the
 // lanes of a wavefront hold an MFMA fragment, so a fragment is one load instruction over eight
 // whole 128-byte lines.  From row-major operands the same instruction touches 16 rows, and the
 // address unit takes about 55 clocks for it instead of 17: 525 x 768 x 3072 (int32 out) takes
