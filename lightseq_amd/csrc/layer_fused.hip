@@ -15,8 +15,9 @@ namespace {
 // pass quantises the weights (2 bytes read and 1 written per parameter: 10 MB for a
 // Transformer-base layer).  As one launch per matrix that was 4 us each, six to nine times per
 // layer; the sections below -- weights, the input, the mask, the copy of a decoding step's caches
-// -- do not depend on one another, so they are ranges of workgroups of one grid and the
-// launch lasts as long as the memory takes: Transformer-base encoder layer 4.9 us in all.
+// -- do not depend on one another, so they are ranges of workgroups of one grid: by the kernel
+// trace 8.0 us for a Transformer-base encoder layer (10 MB) and 18 us for a step of a
+// Transformer-big decoder layer (64 MB with its caches, 3.6 TB/s).
 //
 // Sections that write blocked matrices work on units of 16 rows x 512 columns: a wavefront reads
 // 128-byte pieces of 16 rows and writes 1 KB, the 16 rows x 64 bytes block; what a unit reads is
