@@ -142,8 +142,8 @@ int gemm_blk_preferred_ksplit(int M, int N, int K) {
 int gemm_blk_lut(const int8_t* A, const int8_t* W, int8_t* C, const int8_t* lut, int M, int N, int K,
                  float alpha, hipStream_t s, const LnStep* ln) {
   if (!lut) return lsh_fail(LSH_ERR_INVALID, "blocked gemm (table epilogue): null table");
-  if (N % 64 != 0)
-    return lsh_fail(LSH_ERR_UNSUPPORTED, "blocked gemm (table epilogue): the output needs N % 64 == 0");
+  if (N % 64 != 0 || N >= (1 << 24))  // (table offsets of 32 bits)
+    return lsh_fail(LSH_ERR_UNSUPPORTED, "blocked gemm (table epilogue): the output needs N % 64 == 0 and N < 2^24");
   if (ln) return launch_ln_gemm<EpiLutBlk, false>(*ln, W, EpiLutBlk{C, lut, alpha}, M, N, K, s);
   return dispatch_blk<KwI8, EpiLutBlk, true>(A, W, EpiLutBlk{C, lut, alpha}, M, N, K, s);
 }
