@@ -619,10 +619,10 @@ constexpr size_t long_attn_lds(int nkb) {
 template <int MODE>
 __global__ void __launch_bounds__(1024, 1)
 long_attn_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
-                 const __half* __restrict__ v, const int* __restrict__ pad_mask,
-                 __half* __restrict__ ctx, int8_t* __restrict__ ctx_q, float quant_scale, int S,
-                 int head_num, float alpha, float dq, int key_len, const int* __restrict__ seq,
-                 const __half* __restrict__ q_cmax, int k_pad, const int* __restrict__ items) {
+                 const __half* __restrict__ v, const int* __restrict__ items, const int* __restrict__ seq, int S,
+                 int head_num, int key_len, const int* __restrict__ pad_mask, __half* __restrict__ ctx,
+                 int8_t* __restrict__ ctx_q, float quant_scale, float alpha, float dq,
+                 const __half* __restrict__ q_cmax, int k_pad) {
   constexpr int D = 64, KSTR = attn_kstr(D), VSTR = kAttnVstr;
   constexpr bool LAYER = MODE == kAttnLayer;
   extern __shared__ __align__(16) int8_t long_smem[];
@@ -951,8 +951,8 @@ static int launch_long_attn(int seq_len, int batch_heads, hipStream_t s, const _
   const int parts = std::max((tiles + 15) / 16, std::min(room / std::max(batch_heads, 1), (tiles + 3) / 4));
   const int nw = (tiles + parts - 1) / parts;
   long_attn_kernel<MODE><<<dim3((tiles + nw - 1) / nw, batch_heads), 64 * nw, long_attn_lds(nkb), s>>>(
-      q, k, v, pad_mask, ctx, ctx_q, quant_scale, seq_len, head_num, alpha, dq, key_len, seq, q_cmax, k_pad,
-      items);
+      q, k, v, items, seq, seq_len, head_num, key_len, pad_mask, ctx, ctx_q, quant_scale, alpha, dq, q_cmax,
+      k_pad);
   return LSH_OK;
 }
 
@@ -1129,9 +1129,9 @@ int layer_cross_attention_f16(const __half* q, const __half* k, const __half* v,
 template <int D, int NKB>
 __global__ void __launch_bounds__(64)
 layer_attn_few_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
-                      const __half* __restrict__ v, const __half* __restrict__ add_mask,
-                      int8_t* __restrict__ codes, const __half* __restrict__ q_cmax, int k_pad, int q_blocks,
-                      int q_len, int head_num, int key_len, float alpha, int causal) {
+                      const __half* __restrict__ v, const __half* __restrict__ add_mask, int q_blocks, int q_len,
+                      int head_num, int key_len, float alpha, int causal, int8_t* __restrict__ codes,
+                      const __half* __restrict__ q_cmax, int k_pad) {
   constexpr int CH = D / 8, VS = 36;  // 16-byte chunks of a row; halfs per dimension in LDS
   constexpr int VP = 8 * CH / 64 > 0 ? 8 * CH / 64 : 1;  // patches of 4 keys x 8 dims per lane and block
   __shared__ __align__(16) _Float16 Vt[D * VS];
@@ -1274,9 +1274,9 @@ static void launch_attn_few(const __half* q, const __half* k, const __half* v, c
                             int key_len, float alpha, bool causal, hipStream_t s) {
   const int q_blocks = (q_len + 31) / 32;
 #define LSH_FEW(NKB)                                                                                    \
-  layer_attn_few_kernel<D, NKB><<<pairs * q_blocks, 64, 0, s>>>(q, k, v, add_mask, codes, cmax, k_pad,  \
-                                                                q_blocks, q_len, head_num, key_len,     \
-                                                                alpha, causal ? 1 : 0)
+  layer_attn_few_kernel<D, NKB><<<pairs * q_blocks, 64, 0, s>>>(q, k, v, add_mask, q_blocks, q_len,     \
+                                                                head_num, key_len, alpha,               \
+                                                                causal ? 1 : 0, codes, cmax, k_pad)
   if (key_len <= 32) LSH_FEW(1);
   else if (key_len <= 64) LSH_FEW(2);
   else if (key_len <= 96) LSH_FEW(3);

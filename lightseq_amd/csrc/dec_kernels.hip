@@ -664,9 +664,9 @@ struct EncdecQProd {
 template <int D, int UN, bool QPROD = false, int LN_ROWS = 0>
 __global__ void __launch_bounds__(QPROD ? 512 : 256)
 encdec_attn_short_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
-                         const __half* __restrict__ v, const int* __restrict__ pad_mask,
-                         __half* __restrict__ ctx, int8_t* __restrict__ ctx_q, float quant_scale,
-                         int beam_size, int head_num, int seq_len, float alpha_h, int blocked,
+                         const __half* __restrict__ v, const int* __restrict__ pad_mask, int beam_size,
+                         int head_num, int seq_len, float alpha_h, __half* __restrict__ ctx,
+                         int8_t* __restrict__ ctx_q, float quant_scale, int blocked,
                          EncdecQProd qp = EncdecQProd{}) {
 #pragma clang fp contract(off)
   constexpr int CH = D / 8;     // lanes per row
@@ -882,8 +882,8 @@ int encdec_q_attention_f16(const int8_t* x, const int8_t* q_weight, const __half
   const int un = (batch_seq_len + 7) / 8;
 #define LSH_ENCDEC_Q_LN(UN, LN)                                                              \
   encdec_attn_short_kernel<64, UN, true, LN><<<grid, 512, 0, s>>>(                               \
-      nullptr, k, v, pad_mask, nullptr, ctx_q, quant_scale, beam_size, head_num, batch_seq_len, \
-      alpha_h, blocked, qp)
+      nullptr, k, v, pad_mask, beam_size, head_num, batch_seq_len, alpha_h, nullptr, ctx_q,     \
+      quant_scale, blocked, qp)
 #define LSH_ENCDEC_Q(UN)                                 \
   if (!ln) LSH_ENCDEC_Q_LN(UN, 0);                       \
   else if (beam_size == 1) LSH_ENCDEC_Q_LN(UN, 1);       \
@@ -922,9 +922,9 @@ int encdec_attention_f16(const __half* q, const __half* k, const __half* v, cons
     const int kpw = 512 / dim_per_head;  // rows per load instruction of a wavefront
     const int un = (batch_seq_len + kpw - 1) / kpw;
 #define LSH_ENCDEC_SHORT(D, UN)                                                                   \
-  encdec_attn_short_kernel<D, UN><<<grid, 256, 0, s>>>(q, k, v, pad_mask, ctx, ctx_q, quant_scale, \
-                                                       beam_size, head_num, batch_seq_len, alpha_h, \
-                                                       blocked)
+  encdec_attn_short_kernel<D, UN><<<grid, 256, 0, s>>>(q, k, v, pad_mask, beam_size, head_num,     \
+                                                       batch_seq_len, alpha_h, ctx, ctx_q,          \
+                                                       quant_scale, blocked)
 #define LSH_ENCDEC_SHORT_D(D)                \
   if (un <= 4) LSH_ENCDEC_SHORT(D, 4);       \
   else if (un <= 8) LSH_ENCDEC_SHORT(D, 8);  \

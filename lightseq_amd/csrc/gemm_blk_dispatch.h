@@ -14,8 +14,8 @@ namespace lsh {
 // one output tile per workgroup, both operands blocked
 template <typename Tr, typename Epi, int WGM, int WGN, int MB, int NB, int NST>
 __global__ void __launch_bounds__(64 * WGM * WGN)
-gemm_blk_tile_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, Epi epi, int M,
-                     int N, int K, int tiles_m, int tiles_n) {
+gemm_blk_tile_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, int M, int N, int K,
+                     int tiles_m, int tiles_n, Epi epi) {
   extern __shared__ __align__(16) int8_t smem[];
   asm volatile("" : "+s"(tiles_m) : "s"(A), "s"(W));
   constexpr int TM = WGM * MB * 32;
@@ -64,7 +64,7 @@ int launch_kw(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K, in
   constexpr size_t smem = kw_lds_bytes<Epi, MB, NB>();
   const int slices = K / 64 / ksplit;
 #define LSH_KW(D)                                                                                   \
-  return launch_blk<gemm_kw_kernel<Tr, Epi, MB, NB, D>>(grid, 256, smem, s, A, W, epi, M, N, K, slices, tm, tn)
+  return launch_blk<gemm_kw_kernel<Tr, Epi, MB, NB, D>>(grid, 256, smem, s, A, W, M, N, K, slices, tm, tn, epi)
   if (slices % 16 == 0) LSH_KW(4);
   if (slices % 12 == 0) LSH_KW(3);
   if (slices % 8 == 0) LSH_KW(2);
@@ -120,23 +120,23 @@ int dispatch_blk(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K,
         const int tm = (M + t.tm - 1) / t.tm, tn = (N + t.tn - 1) / t.tn;
         const dim3 grid(tm * tn);
         if (t.tn == 256)
-          return launch_blk<gemm_blk_tile_kernel<Tr, Epi, 2, 4, 4, 2, 2>>(grid, 512, 2 * 512 * kBK, s, A, W, epi, M, N,
-                                                                      K, tm, tn);
+          return launch_blk<gemm_blk_tile_kernel<Tr, Epi, 2, 4, 4, 2, 2>>(grid, 512, 2 * 512 * kBK, s, A, W, M, N, K, tm,
+                                                                      tn, epi);
         if (t.tn == 192)
-          return launch_blk<gemm_blk_tile_kernel<Tr, Epi, 4, 2, 2, 3, 2>>(grid, 512, 2 * 448 * kBK, s, A, W, epi, M, N,
-                                                                      K, tm, tn);
+          return launch_blk<gemm_blk_tile_kernel<Tr, Epi, 4, 2, 2, 3, 2>>(grid, 512, 2 * 448 * kBK, s, A, W, M, N, K, tm,
+                                                                      tn, epi);
         if (t.tm == 256)
-          return launch_blk<gemm_blk_tile_kernel<Tr, Epi, 4, 2, 2, 2, 3>>(grid, 512, 3 * 384 * kBK, s, A, W, epi, M, N,
-                                                                      K, tm, tn);
+          return launch_blk<gemm_blk_tile_kernel<Tr, Epi, 4, 2, 2, 2, 3>>(grid, 512, 3 * 384 * kBK, s, A, W, M, N, K, tm,
+                                                                      tn, epi);
         if (t.tn == 128)
-          return launch_blk<gemm_blk_tile_kernel<Tr, Epi, 2, 2, 2, 2, 2>>(grid, 256, 2 * 256 * kBK, s, A, W, epi, M, N,
-                                                                      K, tm, tn);
+          return launch_blk<gemm_blk_tile_kernel<Tr, Epi, 2, 2, 2, 2, 2>>(grid, 256, 2 * 256 * kBK, s, A, W, M, N, K, tm,
+                                                                      tn, epi);
         // long K loops: a third stage instead of a third workgroup per compute unit
         if (K >= 2048)
-          return launch_blk<gemm_blk_tile_kernel<Tr, Epi, 4, 1, 1, 2, 3>>(grid, 256, 3 * 192 * kBK, s, A, W, epi, M, N,
-                                                                      K, tm, tn);
-        return launch_blk<gemm_blk_tile_kernel<Tr, Epi, 4, 1, 1, 2, 2>>(grid, 256, 2 * 192 * kBK, s, A, W, epi, M, N, K,
-                                                                    tm, tn);
+          return launch_blk<gemm_blk_tile_kernel<Tr, Epi, 4, 1, 1, 2, 3>>(grid, 256, 3 * 192 * kBK, s, A, W, M, N, K, tm,
+                                                                      tn, epi);
+        return launch_blk<gemm_blk_tile_kernel<Tr, Epi, 4, 1, 1, 2, 2>>(grid, 256, 2 * 192 * kBK, s, A, W, M, N, K, tm,
+                                                                      tn, epi);
       }
     }
   }
@@ -184,15 +184,15 @@ inline SeqTile choose_seq(int M, int N, int K, int cus) {
 template <typename Epi, int MB, int D>
 int launch_seq(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K, hipStream_t s) {
   const int tm = (M + 16 * MB - 1) / (16 * MB), tn = (N + 16 * MB - 1) / (16 * MB);
-  return launch_blk<gemm_seq_kernel<KwF16, Epi, 1, 1, MB, MB, D>>(dim3(tm * tn), 64, 0, s, A, W, epi, M, N, K,
-                                                                  K / 64, tm, tn);
+  return launch_blk<gemm_seq_kernel<KwF16, Epi, 1, 1, MB, MB, D>>(dim3(tm * tn), 64, 0, s, A, W, M, N, K,
+                                                                  K / 64, tm, tn, epi);
 }
 template <typename Epi, int WGM, int WGN, int MB, int NB, int NST>
 int launch_f16_tile(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K, hipStream_t s) {
   constexpr int TM = WGM * MB * 32, TN = WGN * NB * 32;
   const int tm = (M + TM - 1) / TM, tn = (N + TN - 1) / TN;
   return launch_blk<gemm_blk_tile_kernel<KwF16, Epi, WGM, WGN, MB, NB, NST>>(
-      dim3(tm * tn), 64 * WGM * WGN, NST * (TM + TN) * kBK, s, A, W, epi, M, N, K, tm, tn);
+      dim3(tm * tn), 64 * WGM * WGN, NST * (TM + TN) * kBK, s, A, W, M, N, K, tm, tn, epi);
 }
 
 // K in bytes

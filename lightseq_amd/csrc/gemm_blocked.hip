@@ -17,7 +17,7 @@ namespace lsh {
 // us per generation step of a GPT-2 medium shape, batch 1: 573 -> 457.
 template <typename Epi, bool I32, int ROWS, int D>
 __global__ void __launch_bounds__(256)
-ln_gemm_kernel(const LnStep ln, const int8_t* __restrict__ W, Epi epi, int M, int N, int K) {
+ln_gemm_kernel(const int8_t* __restrict__ W, int M, int N, int K, const LnStep ln, Epi epi) {
   extern __shared__ __align__(16) int8_t smem[];
   __shared__ __align__(16) float red_ln[2 * ROWS * 4];
   int8_t* codes = smem;           // [16 rows, K] blocked
@@ -72,10 +72,10 @@ int launch_ln_rows(const LnStep& ln, const int8_t* W, Epi epi, int M, int N, int
   const dim3 grid((N + 15) / 16);
   const size_t smem = 16 * (size_t)K + 4 * 68 * 16 + (Epi::kTable ? 16 * 256 : 0);
   switch (K >> 8) {
-    case 1: return launch_blk<ln_gemm_kernel<Epi, I32, ROWS, 1>>(grid, 256, smem, s, ln, W, epi, M, N, K);
-    case 2: return launch_blk<ln_gemm_kernel<Epi, I32, ROWS, 2>>(grid, 256, smem, s, ln, W, epi, M, N, K);
-    case 3: return launch_blk<ln_gemm_kernel<Epi, I32, ROWS, 3>>(grid, 256, smem, s, ln, W, epi, M, N, K);
-    default: return launch_blk<ln_gemm_kernel<Epi, I32, ROWS, 4>>(grid, 256, smem, s, ln, W, epi, M, N, K);
+    case 1: return launch_blk<ln_gemm_kernel<Epi, I32, ROWS, 1>>(grid, 256, smem, s, W, M, N, K, ln, epi);
+    case 2: return launch_blk<ln_gemm_kernel<Epi, I32, ROWS, 2>>(grid, 256, smem, s, W, M, N, K, ln, epi);
+    case 3: return launch_blk<ln_gemm_kernel<Epi, I32, ROWS, 3>>(grid, 256, smem, s, W, M, N, K, ln, epi);
+    default: return launch_blk<ln_gemm_kernel<Epi, I32, ROWS, 4>>(grid, 256, smem, s, W, M, N, K, ln, epi);
   }
 }
 template <typename Epi, bool I32>

@@ -68,8 +68,8 @@ constexpr int kw_lds_bytes() {
 // has to stay below 4 GiB.
 template <typename Tr, typename Epi, int MB, int NB, int D>
 __global__ void __launch_bounds__(256, 2)
-gemm_kw_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, Epi epi, int M, int N,
-               int K, int slices, int tiles_m, int tiles_n) {
+gemm_kw_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, int M, int N, int K, int slices,
+               int tiles_m, int tiles_n, Epi epi) {
   typedef typename Tr::Acc Acc;
   extern __shared__ __align__(16) int8_t smem[];
   constexpr int QN = 4 * NB;  // column quads of a tile
@@ -193,8 +193,8 @@ gemm_kw_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, Epi e
 // ---------------------------------------------------------------------------------
 template <typename Tr, typename Epi, int WM, int WN, int MB, int NB, int D>
 __global__ void __launch_bounds__(64 * WM * WN)
-gemm_seq_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, Epi epi, int M, int N, int K,
-                int slices, int tiles_m, int tiles_n) {
+gemm_seq_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, int M, int N, int K, int slices,
+                int tiles_m, int tiles_n, Epi epi) {
   typedef typename Tr::Acc Acc;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);

@@ -421,9 +421,12 @@ __device__ __forceinline__ void tile_gemm(const int8_t* __restrict__ A,
   for (int t = 0; t < NST - 1; ++t) {
     slices(smem + slot * STAGE);
     __builtin_amdgcn_s_waitcnt(0xC07F);
-    if (NST - 2 - t == 0) wait_vmcnt<0>();
-    else if (NST - 2 - t == 1) wait_vmcnt<PER>();
-    else wait_vmcnt<2 * PER>();
+    switch (NST - 2 - t) {  // stages that may still be on their way
+      case 0: wait_vmcnt<0>(); break;
+      case 1: wait_vmcnt<PER>(); break;
+      case 2: wait_vmcnt<2 * PER>(); break;
+      default: wait_vmcnt<3 * PER>();
+    }
     __builtin_amdgcn_s_barrier();
     if (LUT && t == NST - 2) {
       // the slot of the second-to-last step is free: the tile's table rows go there

@@ -129,11 +129,10 @@ ln_rows_kernel(const AccT* __restrict__ gemm_out, T* residual, T* out_t,
 // 3.8 / 4.1 / 6.1 / 10.4 (before: 4.7 / 5.0 / 7.0 / 12.3).
 template <typename T, typename AccT, int MODE, int LPR, int ITER, bool FULL>
 __global__ void __launch_bounds__(64)
-ln_rows8_kernel(const AccT* __restrict__ gemm_out, T* residual, T* out_t,
-                int8_t* __restrict__ out_q, const T* __restrict__ scale,
+ln_rows8_kernel(const AccT* __restrict__ gemm_out, T* residual, const T* __restrict__ scale,
                 const T* __restrict__ bias, const T* __restrict__ residual_bias,
-                const T* __restrict__ colsum, int tokens, int hidden, float dequant_scale,
-                float quant_scale, int is_post_ln, int nparts, long part_stride, int blocked,
+                const T* __restrict__ colsum, int tokens, int hidden, T* out_t, int8_t* __restrict__ out_q,
+                float dequant_scale, float quant_scale, int is_post_ln, int nparts, long part_stride, int blocked,
                 const int* __restrict__ row_map) {
   constexpr int RPW = kWave / LPR;
   const int lane = threadIdx.x;
@@ -374,11 +373,10 @@ ln_row_wg_finish(const float (&x)[4], bool on, int e, long base, const float (&g
 // 16 lanes and the four rows of a wavefront pairwise; the wavefronts in ascending order.
 template <typename T, typename AccT, int MODE>
 __global__ void __launch_bounds__(256)
-ln_row_wg_kernel(const AccT* __restrict__ gemm_out, T* residual, T* out_t,
-                 int8_t* __restrict__ out_q, const T* __restrict__ scale,
+ln_row_wg_kernel(const AccT* __restrict__ gemm_out, T* residual, const T* __restrict__ scale,
                  const T* __restrict__ bias, const T* __restrict__ residual_bias,
-                 const T* __restrict__ colsum, int hidden, float dequant_scale,
-                 float quant_scale, int is_post_ln, int nparts, long part_stride, int blocked) {
+                 const T* __restrict__ colsum, int hidden, int nparts, long part_stride, T* out_t,
+                 int8_t* __restrict__ out_q, float dequant_scale, float quant_scale, int is_post_ln, int blocked) {
   __shared__ float red[2][4];
   const int e0 = (int)threadIdx.x * 4;
   const bool on = e0 < hidden;
@@ -652,8 +650,8 @@ static int launch_ln(const AccT* gemm_out, T* residual, T* out_t, int8_t* out_q,
   if (vec_ok && hidden <= 1024 && g_ln_few_rows && !row_map) {
     const int tpr = ((hidden / 4 + 63) / 64) * 64;  // threads of a row: whole wavefronts
     ln_row_wg_kernel<T, AccT, MODE><<<tokens, tpr, 0, stream>>>(
-        gemm_out, residual, out_t, out_q, scale, bias, residual_bias, colsum, hidden,
-        dequant_scale, quant_scale, is_post_ln, nparts, part_stride, blk);
+        gemm_out, residual, scale, bias, residual_bias, colsum, hidden, nparts, part_stride, out_t, out_q,
+        dequant_scale, quant_scale, is_post_ln, blk);
     return lsh_check_launch("ln_row_wg_kernel");
   }
   if (vec_ok && hidden % 8 == 0) {
@@ -661,7 +659,7 @@ static int launch_ln(const AccT* gemm_out, T* residual, T* out_t, int8_t* out_q,
 #define LSH_LN8_RUN(LPR, IT, FULL)                                                               \
   ln_rows8_kernel<T, AccT, MODE, LPR, IT, FULL>                                                  \
       <<<(tokens + 64 / LPR - 1) / (64 / LPR), 64, 0, stream>>>(                                 \
-          gemm_out, residual, out_t, out_q, scale, bias, residual_bias, colsum, tokens, hidden,  \
+          gemm_out, residual, scale, bias, residual_bias, colsum, tokens, hidden, out_t, out_q,  \
           dequant_scale, quant_scale, is_post_ln, nparts, part_stride, blk, row_map)
 #define LSH_LN8_CASE(LPR, IT) \
   do { if (hidden == LPR * 8 * IT) LSH_LN8_RUN(LPR, IT, true); else LSH_LN8_RUN(LPR, IT, false); } while (0)

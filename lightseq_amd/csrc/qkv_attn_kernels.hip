@@ -45,10 +45,9 @@ constexpr int kQaItemHeadShift = 16, kQaItemBlocksShift = 28;
 template <bool PK>
 __global__ void __launch_bounds__(256, 2)
 qkv_attn_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W,
-                const _Float16* __restrict__ bias, const int* __restrict__ pad_mask,
-                const int* __restrict__ plan, int8_t* __restrict__ ctx_q, float requant_alpha,
-                float dq, float quant_scale, float alpha, int S, int batch, int head_num, int K,
-                const int* __restrict__ seq) {
+                const int* __restrict__ plan, const int* __restrict__ seq, int S, int batch, int head_num, int K,
+                const _Float16* __restrict__ bias, const int* __restrict__ pad_mask, int8_t* __restrict__ ctx_q,
+                float requant_alpha, float dq, float quant_scale, float alpha) {
   constexpr int D = kQaD, WGN = 2, MB = 2, NB = 3, NWV = 4, TM = kQaTM, TN = kQaTN;
   constexpr int STAGE = kQaStage, NST = kQaNst;
   constexpr int NA = TM / 8 / NWV, NW = TN / 8 / NWV;  // 1-KB loads per wavefront
@@ -453,10 +452,9 @@ static int launch_qkv_attention(const int8_t* x, const int8_t* qkv_weight, const
   if (plan != nullptr && !qkv_attention_plan_supported(batch, seq_len, head_num))
     return lsh_fail(LSH_ERR_INVALID, "qkv_attention_i8: this shape has no plan");
   hipExtLaunchKernelGGL(qkv_attn_kernel<PK>, dim3(batch * head_num), dim3(256), smem, s, e0, e1, 0, x,
-                        qkv_weight, reinterpret_cast<const _Float16*>(qkv_bias), pad_mask, plan,
-                        ctx_q,
-                        requant_alpha, dequant_scale, quant_scale, alpha, seq_len, batch, head_num,
-                        hidden, seq);
+                        qkv_weight, plan, seq, seq_len, batch, head_num, hidden,
+                        reinterpret_cast<const _Float16*>(qkv_bias), pad_mask, ctx_q, requant_alpha, dequant_scale,
+                        quant_scale, alpha);
   return lsh_check_launch("qkv_attn_kernel");
 }
 
