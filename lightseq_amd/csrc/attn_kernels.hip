@@ -584,7 +584,7 @@ encself_attn_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
       if (MODE == kAttnLayer) {
         if (ctx_q != nullptr)
           *reinterpret_cast<uint32_t*>(ctx_q + blocked_offset(tok, head * D + dd, k_pad)) =
-              pack4_i8(codes_of.code(o[0]), codes_of.code(o[1]), codes_of.code(o[2]), codes_of.code(o[3]));
+              codes_of.pack4(o[0], o[1], o[2], o[3]);
       } else if (ctx_q != nullptr) {
         // a padded query gives zeros, whose code is 0
         const uint32_t w4 = float2int8_pack4(o[0], o[1], o[2], o[3], quant_scale);
@@ -911,7 +911,7 @@ long_attn_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
       if (ctx_q != nullptr) {
         if constexpr (LAYER) {
           *reinterpret_cast<uint32_t*>(ctx_q + blocked_offset(tok, head * D + dd, k_pad)) =
-              pack4_i8(codes_of.code(o[0]), codes_of.code(o[1]), codes_of.code(o[2]), codes_of.code(o[3]));
+              codes_of.pack4(o[0], o[1], o[2], o[3]);
         } else {
           const uint32_t w4 = float2int8_pack4(o[0], o[1], o[2], o[3], quant_scale);
           *reinterpret_cast<uint32_t*>(ctx_q + code_offset(tok, head * D + dd, hidden, seq != nullptr)) =
@@ -1260,11 +1260,9 @@ layer_attn_few_kernel(const __half* __restrict__ q, const __half* __restrict__ k
 #pragma unroll
     for (int vg = 0; vg < 4; ++vg) {
       const int dd = db * 32 + 8 * vg + 4 * g;
-      int c[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) c[j] = codes_of.code(round_h(acc[db][4 * vg + j]));
       *reinterpret_cast<uint32_t*>(codes + blocked_offset(row, head * D + dd, k_pad)) =
-          pack4_i8(c[0], c[1], c[2], c[3]);
+          codes_of.pack4(round_h(acc[db][4 * vg]), round_h(acc[db][4 * vg + 1]), round_h(acc[db][4 * vg + 2]),
+                         round_h(acc[db][4 * vg + 3]));
     }
 }
 

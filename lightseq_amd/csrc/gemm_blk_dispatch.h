@@ -72,22 +72,35 @@ int launch_kw(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K, in
 #undef LSH_KW
 }
 
-// The LDS tile kernel: 8 wavefronts for the tall tiles, 4 for 128 x 128 and 128 x 64 (two or three
+template <typename Tr, typename Epi, int WGM, int WGN, int MB, int NB, int NST>
+int launch_tile(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K, hipStream_t s) {
+  constexpr int TM = WGM * MB * 32, TN = WGN * NB * 32;
+  const int tm = (M + TM - 1) / TM, tn = (N + TN - 1) / TN;
+  return launch_blk<gemm_blk_tile_kernel<Tr, Epi, WGM, WGN, MB, NB, NST>>(
+      dim3(tm * tn), 64 * WGM * WGN, (tile_lds_bytes<Epi, WGM, WGN, MB, NB, NST>()), s, A, W, M, N, K, tm, tn, epi);
+}
+
+// The LDS tile kernel: 8 wavefronts for tiles from 128 x 128 up, 4 for the small ones (several
 // workgroups then share a compute unit and one's epilogue runs under the other's K loop).
-constexpr TileCost kLdsCost[] = {{128, 64, 2.5f, 2.45f, 0.2f, 2.6f, 0.6f},
-                                 {128, 128, 2.9f, 3.6f, 0.6f, 4.9f, 0.9f},
-                                 {256, 128, 3.1f, 5.4f, 1.5f, 9.0f, 1.3f},
-                                 {256, 192, 3.6f, 7.1f, 3.0f, 9.5f, 1.7f},
-                                 {256, 256, 4.1f, 9.2f, 4.0f, 12.0f, 2.4f}};
+constexpr TileCost kLdsCost[] = {{64, 64, 2.2f, 1.54f, 0.22f, 1.13f, 0.27f, 0.69f},
+                                 {128, 64, 2.55f, 2.32f, 0.2f, 1.85f, 0.46f, 1.4f},
+                                 {128, 128, 2.5f, 3.36f, 1.07f, 2.7f, 0.52f, 2.55f},
+                                 {256, 128, 3.0f, 5.5f, 2.7f, 6.1f, 0.93f, 4.85f},
+                                 {256, 192, 3.65f, 7.3f, 2.35f, 9.25f, 1.5f, 7.25f},
+                                 {256, 256, 4.35f, 9.3f, 0.f, 14.2f, 2.2f, 8.95f}};
+// (its third stage costs the 128 x 64 tile its third workgroup per compute unit)
+constexpr int kLongK = 2048;
+constexpr TileCost kLongKCost{128, 64, 2.55f, 2.32f, 0.2f, 2.35f, 0.46f, 1.4f};
 struct LdsTile {
   int tm = 0, tn = 0;
   float us = 0;
 };
-inline LdsTile choose_lds_tile(int M, int N, int K, int cus, bool table) {
+inline LdsTile choose_lds_tile(int M, int N, int K, int cus, EpilogueCost epi) {
   LdsTile best;
   if (K % kBK != 0 || K / kBK < 3 || N % 16 != 0) return best;
   for (const auto& c : kLdsCost) {
-    const float us = tile_us(c, M, N, K, 1, cus, table);
+    const bool long_k = K >= kLongK && c.tm == 128 && c.tn == 64;
+    const float us = tile_us(long_k ? kLongKCost : c, M, N, K, 1, cus, epi);
     if (best.tm == 0 || us < best.us) best = LdsTile{c.tm, c.tn, us};
   }
   return best;
@@ -112,31 +125,24 @@ int dispatch_blk(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K,
   if (ksplit < 1 || K % (64 * ksplit) != 0)
     return lsh_fail(LSH_ERR_INVALID, "blocked gemm: K does not split into whole 64-byte slices");
   const int cus = cu_count();
-  const KwTile kw = kw_choose_tile(M, N, K / ksplit, ksplit, cus, Epi::kTable);
+  constexpr EpilogueCost cost = epilogue_cost<Epi>();
+  const KwTile kw = kw_choose_tile(M, N, K / ksplit, ksplit, cus, cost);
   if constexpr (TILES) {
     if (ksplit == 1) {
-      const LdsTile t = choose_lds_tile(M, N, K, cus, Epi::kTable);
+      const LdsTile t = choose_lds_tile(M, N, K, cus, cost);
       if (t.tm != 0 && t.us < kw.us) {
-        const int tm = (M + t.tm - 1) / t.tm, tn = (N + t.tn - 1) / t.tn;
-        const dim3 grid(tm * tn);
-        if (t.tn == 256)
-          return launch_blk<gemm_blk_tile_kernel<Tr, Epi, 2, 4, 4, 2, 2>>(grid, 512, 2 * 512 * kBK, s, A, W, M, N, K, tm,
-                                                                      tn, epi);
-        if (t.tn == 192)
-          return launch_blk<gemm_blk_tile_kernel<Tr, Epi, 4, 2, 2, 3, 2>>(grid, 512, 2 * 448 * kBK, s, A, W, M, N, K, tm,
-                                                                      tn, epi);
-        if (t.tm == 256)
-          return launch_blk<gemm_blk_tile_kernel<Tr, Epi, 4, 2, 2, 2, 3>>(grid, 512, 3 * 384 * kBK, s, A, W, M, N, K, tm,
-                                                                      tn, epi);
-        if (t.tn == 128)
-          return launch_blk<gemm_blk_tile_kernel<Tr, Epi, 2, 2, 2, 2, 2>>(grid, 256, 2 * 256 * kBK, s, A, W, M, N, K, tm,
-                                                                      tn, epi);
+        if (t.tn == 256) return launch_tile<Tr, Epi, 2, 4, 4, 2, 2>(A, W, epi, M, N, K, s);
+        if (t.tn == 192) return launch_tile<Tr, Epi, 4, 2, 2, 3, 2>(A, W, epi, M, N, K, s);
+        if (t.tm == 256) return launch_tile<Tr, Epi, 4, 2, 2, 2, 3>(A, W, epi, M, N, K, s);
+        // where a tile has a compute unit to itself the ring may fill its LDS: 2348 x 1024 x 1024 in 6.6
+        // instead of 6.9 us (with two tiles a unit 2348 x 3072 x 1024 takes 12.1, not 10.4)
+        if (t.tn == 128 && K >= 4 * kBK && (long)((M + 127) / 128) * ((N + 127) / 128) <= cus)
+          return launch_tile<Tr, Epi, 4, 2, 1, 2, 4>(A, W, epi, M, N, K, s);
+        if (t.tn == 128) return launch_tile<Tr, Epi, 4, 2, 1, 2, 2>(A, W, epi, M, N, K, s);
+        if (t.tm == 64) return launch_tile<Tr, Epi, 2, 2, 1, 1, 3>(A, W, epi, M, N, K, s);
         // long K loops: a third stage instead of a third workgroup per compute unit
-        if (K >= 2048)
-          return launch_blk<gemm_blk_tile_kernel<Tr, Epi, 4, 1, 1, 2, 3>>(grid, 256, 3 * 192 * kBK, s, A, W, M, N, K, tm,
-                                                                      tn, epi);
-        return launch_blk<gemm_blk_tile_kernel<Tr, Epi, 4, 1, 1, 2, 2>>(grid, 256, 2 * 192 * kBK, s, A, W, M, N, K, tm,
-                                                                      tn, epi);
+        if (K >= kLongK) return launch_tile<Tr, Epi, 4, 1, 1, 2, 3>(A, W, epi, M, N, K, s);
+        return launch_tile<Tr, Epi, 2, 2, 2, 1, 2>(A, W, epi, M, N, K, s);
       }
     }
   }
@@ -187,14 +193,6 @@ int launch_seq(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K, h
   return launch_blk<gemm_seq_kernel<KwF16, Epi, 1, 1, MB, MB, D>>(dim3(tm * tn), 64, 0, s, A, W, M, N, K,
                                                                   K / 64, tm, tn, epi);
 }
-template <typename Epi, int WGM, int WGN, int MB, int NB, int NST>
-int launch_f16_tile(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K, hipStream_t s) {
-  constexpr int TM = WGM * MB * 32, TN = WGN * NB * 32;
-  const int tm = (M + TM - 1) / TM, tn = (N + TN - 1) / TN;
-  return launch_blk<gemm_blk_tile_kernel<KwF16, Epi, WGM, WGN, MB, NB, NST>>(
-      dim3(tm * tn), 64 * WGM * WGN, NST * (TM + TN) * kBK, s, A, W, M, N, K, tm, tn, epi);
-}
-
 // K in bytes
 template <typename Epi>
 int dispatch_f16(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K, hipStream_t s) {
@@ -208,10 +206,10 @@ int dispatch_f16(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K,
     case 1:
       if (slices % 4 == 0) return launch_seq<Epi, 2, 4>(A, W, epi, M, N, K, s);
       return launch_seq<Epi, 2, 1>(A, W, epi, M, N, K, s);
-    case 2: return launch_f16_tile<Epi, 2, 2, 1, 1, 3>(A, W, epi, M, N, K, s);
-    case 3: return launch_f16_tile<Epi, 4, 1, 1, 2, 2>(A, W, epi, M, N, K, s);
-    case 5: return launch_f16_tile<Epi, 2, 2, 2, 2, 3>(A, W, epi, M, N, K, s);
-    default: return launch_f16_tile<Epi, 2, 2, 2, 2, 2>(A, W, epi, M, N, K, s);
+    case 2: return launch_tile<KwF16, Epi, 2, 2, 1, 1, 3>(A, W, epi, M, N, K, s);
+    case 3: return launch_tile<KwF16, Epi, 4, 1, 1, 2, 2>(A, W, epi, M, N, K, s);
+    case 5: return launch_tile<KwF16, Epi, 2, 2, 2, 2, 3>(A, W, epi, M, N, K, s);
+    default: return launch_tile<KwF16, Epi, 2, 2, 2, 2, 2>(A, W, epi, M, N, K, s);
   }
 }
 

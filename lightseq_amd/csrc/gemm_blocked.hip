@@ -105,8 +105,9 @@ bool ln_step_supported(int rows, int hidden) {
 }
 
 const char* gemm_blk_kernel_name(int M, int N, int K, bool table) {
-  const LdsTile t = choose_lds_tile(M, N, K, cu_count(), table);
-  return t.tm != 0 && t.us < kw_choose_tile(M, N, K, 1, cu_count(), table).us ? "gemm_blk_tile_kernel"
+  const EpilogueCost epi = table ? EpilogueCost::kTable : EpilogueCost::kPlain;
+  const LdsTile t = choose_lds_tile(M, N, K, cu_count(), epi);
+  return t.tm != 0 && t.us < kw_choose_tile(M, N, K, 1, cu_count(), epi).us ? "gemm_blk_tile_kernel"
                                                                               : "gemm_kw_kernel";
 }
 
@@ -127,10 +128,10 @@ int gemm_blk_i32o(const int8_t* A, const int8_t* W, int32_t* C, int M, int N, in
 int gemm_blk_preferred_ksplit(int M, int N, int K) {
   int best = 1;
   if (M > kKwColdRows) return best;
-  float best_us = kw_choose_tile(M, N, K, 1, cu_count(), false).us;
+  float best_us = kw_choose_tile(M, N, K, 1, cu_count(), EpilogueCost::kPlain).us;
   for (int ks = 2; ks <= 4; ++ks) {
     if (K % (512 * ks) != 0) continue;
-    const float us = kw_choose_tile(M, N, K / ks, ks, cu_count(), false).us + 0.1f * ks;
+    const float us = kw_choose_tile(M, N, K / ks, ks, cu_count(), EpilogueCost::kPlain).us + 0.1f * ks;
     if (us < best_us) {
       best = ks;
       best_us = us;

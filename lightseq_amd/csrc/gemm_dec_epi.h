@@ -141,7 +141,7 @@ struct EpiDecQkvI8 {
 // that a row holds, where the rows are those of a plan.  The stand-alone launch reads and writes
 // all the codes once more and is one of nine launches of a layer: 10.3 us for 3072 rows of 3 x 1024.
 struct EpiPromptQkvI8 {
-  static constexpr bool kTable = false, kBlockedOut = false;
+  static constexpr bool kTable = false, kBlockedOut = false, kStaged = true, kFetch = true;
   int8_t *q, *k, *v;
   const __half* bias;
   const int* row_map;
@@ -153,18 +153,14 @@ struct EpiPromptQkvI8 {
     int head, steps;
     half4_t b;
   };
-  __device__ __forceinline__ Col at(int n) const {
+  __device__ __forceinline__ Col column(int n, int) const {
     const int part = div_by(n, hidden, inv_hidden), i = n - part * hidden;
     const int head = div_by(i, dim, inv_dim);
-    return Col{(part == 0 ? q : part == 1 ? k : v) + (i - head * dim), head, part == 0 ? seq : max_step, {}};
+    return Col{(part == 0 ? q : part == 1 ? k : v) + (i - head * dim), head, part == 0 ? seq : max_step,
+               *reinterpret_cast<const half4_t*>(bias + n)};
   }
-  __device__ __forceinline__ Col column(int n, int) const {
-    Col c = at(n);
-    c.b = *reinterpret_cast<const half4_t*>(bias + n);
-    return c;
-  }
-  __device__ __forceinline__ int8_t* row_ptr(const Col& col, int m) const {
-    const int p = row_map != nullptr ? row_map[m] : m;
+  __device__ __forceinline__ int fetch(int m, int, int) const { return row_map != nullptr ? row_map[m] : m; }
+  __device__ __forceinline__ int8_t* row_ptr(const Col& col, int p) const {
     const int b = div_by(p, seq, inv_seq), s = p - b * seq;
     return col.base + ((long)(b * head_num + col.head) * col.steps + s) * dim;
   }
@@ -172,24 +168,10 @@ struct EpiPromptQkvI8 {
 #pragma clang fp contract(off)
     return floorf(requant_acc_clamped(acc, alpha)) * dequant_scale + __half2float(b);
   }
-  __device__ __forceinline__ void store4(int m, int, int, const Col& col, const v4i& c) const {
-    *reinterpret_cast<uint32_t*>(row_ptr(col, m)) =
+  __device__ __forceinline__ void store4(int, int, int, const Col& col, const v4i& c, int p) const {
+    *reinterpret_cast<uint32_t*>(row_ptr(col, p)) =
         float2int8_pack4(value(c[0], col.b.v[0]), value(c[1], col.b.v[1]), value(c[2], col.b.v[2]),
                          value(c[3], col.b.v[3]), quant_scale);
-  }
-  // 16 columns of one head (dim % 16 == 0)
-  __device__ __forceinline__ void store16(long m, int n, int, const v16i& c, bool) const {
-    const half8_t b0 = *reinterpret_cast<const half8_t*>(bias + n);
-    const half8_t b1 = *reinterpret_cast<const half8_t*>(bias + n + 8);
-    uint32_t w[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const half8_t& b = j < 2 ? b0 : b1;
-      w[j] = float2int8_pack4(value(c[4 * j], b.v[4 * j & 7]), value(c[4 * j + 1], b.v[(4 * j & 7) + 1]),
-                              value(c[4 * j + 2], b.v[(4 * j & 7) + 2]),
-                              value(c[4 * j + 3], b.v[(4 * j & 7) + 3]), quant_scale);
-    }
-    *reinterpret_cast<uint4*>(row_ptr(at(n), (int)m)) = make_uint4(w[0], w[1], w[2], w[3]);
   }
   bool aligned() const {
     return ((reinterpret_cast<uintptr_t>(bias) | reinterpret_cast<uintptr_t>(q) |

@@ -26,8 +26,6 @@
 
 namespace lsh {
 
-typedef float v4f __attribute__((ext_vector_type(4)));
-
 struct KwI8 {
   typedef v16i Acc16;  // of the LDS tile loop: sixteen neighbouring columns
   typedef v4i Acc;  // four neighbouring columns of one row
@@ -101,6 +99,9 @@ gemm_kw_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, int M
   const int n = n0 + 4 * quad;
   const typename Epi::Col col = epi.column(min(n, N - 4), N);
   const auto raw = epi_request(epi);
+  decltype(epi_fetch(epi, 0, 0, 0)) fetched[PER];
+#pragma unroll
+  for (int j = 0; j < PER; ++j) fetched[j] = epi_fetch(epi, min(m0 + row0 + j * ROWS, M - 1), min(n, N - 4), N);
 
   // this wavefront's slices
   const int first = (int)blockIdx.y * slices;
@@ -177,7 +178,7 @@ gemm_kw_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, int M
                     (red[2 * MB * NB * 68 + cell] + red[3 * MB * NB * 68 + cell]);
       const int mo = m + (int)blockIdx.y * M;
       if constexpr (Epi::kTable) fin.store4(mo, n, N, col, c, tab + 4 * quad * 256);
-      else fin.store4(mo, n, N, col, c);
+      else epi_store4(fin, mo, n, N, col, c, fetched[j]);
     }
   }
 }
@@ -206,6 +207,12 @@ gemm_seq_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, int 
   typename Epi::Col col[NB];
 #pragma unroll
   for (int b = 0; b < NB; ++b) col[b] = epi.column(min(n0 + 16 * b + 4 * kq, N - 4), N);
+  decltype(epi_fetch(epi, 0, 0, 0)) fetched[MB][NB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+      fetched[i][b] = epi_fetch(epi, min(m0 + 16 * i + l16, M - 1), min(n0 + 16 * b + 4 * kq, N - 4), N);
   const int8_t* a_base = A + (long)m0 * K;
   const int8_t* w_base = W + (long)n0 * K;
   uint32_t a_off[MB], w_off[NB];
@@ -255,7 +262,7 @@ gemm_seq_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, int 
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
       const int n = n0 + 16 * b + 4 * kq;
-      if (n < N) epi.store4(m, n, N, col[b], acc[i][b]);
+      if (n < N) epi_store4(epi, m, n, N, col[b], acc[i][b], fetched[i][b]);
     }
   }
 }
@@ -263,30 +270,36 @@ gemm_seq_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, int 
 // ---------------------------------------------------------------------------------
 // host side: the estimated duration of a launch.  Its length is that of the compute unit with the
 // most tiles: the first tile takes a + b k microseconds (k: K in units of 1024 bytes; b grows by a
-// third when every compute unit works), each further one s0 + s1 k, with the table epilogue
-// `table` more per tile.  The constants are a fit to a sweep of every tile over M from 16 to 7680
-// and the four products of a layer at hidden 768 and 1024 (K from 768 to 4096); over that sweep
-// the tile with the smallest estimate is 2 % slower than the fastest on average.  (All tiles slow
-// down alike when more than half of the compute units work, up to half as much again with long K,
-// so that what is left out there does not change the choice: the LDS tiles over eight products
-// and M from 256 to 8192, 1.6 % on average and 7 % at the 95th percentile.)
+// third when every compute unit works), each further one s0 + s1 k, and every one `table` more with
+// the table epilogue, `arith` more with an epilogue that dequantises, adds and rounds to fp16.
+// The constants are fits to a sweep of every tile over eight epilogues, hidden 512, 768 and 1024
+// and 24 M from 16 to 7926: the tile with the smallest estimate is 1 to 2 % slower than the fastest
+// on average, 5 to 8 % at the 95th percentile.  (One set of constants for all epilogues, fitted to
+// the plain ones, was 5 % off for those and 5 to 12 % for the others.)
 // ---------------------------------------------------------------------------------
+enum class EpilogueCost { kPlain, kTable, kArith };
+template <typename Epi>
+constexpr EpilogueCost epilogue_cost() {
+  return Epi::kTable ? EpilogueCost::kTable
+                     : EpiStaged<Epi>::value || EpiHasClips<Epi>::value ? EpilogueCost::kArith : EpilogueCost::kPlain;
+}
 struct TileCost {
   int tm, tn;
-  float a, b, s0, s1, table;
+  float a, b, s0, s1, table, arith;
 };
-inline float tile_us(const TileCost& c, int M, int N, int K, int ksplit, int cus, bool table) {
+inline float tile_us(const TileCost& c, int M, int N, int K, int ksplit, int cus, EpilogueCost epi) {
   const long tiles =
       (long)((M + c.tm - 1) / c.tm) * ((N + c.tn - 1) / c.tn) * ksplit;
   const float per = (float)((tiles + cus - 1) / cus), k = K / 1024.f;
   const float busy = tiles < cus ? (float)tiles / cus : 1.f;
   const float first = c.a + c.b * k * (1.f + 0.35f * busy);
-  return first + (per - 1.f) * (c.s0 + c.s1 * k) + (table ? per * c.table : 0.f);
+  const float each = epi == EpilogueCost::kTable ? c.table : epi == EpilogueCost::kArith ? c.arith : 0.f;
+  return first + (per - 1.f) * (c.s0 + c.s1 * k) + per * each;
 }
-constexpr TileCost kKwCost[] = {{16, 16, 2.3f, 0.2f, 0.05f, 0.2f, 0.03f},
-                                {32, 32, 2.3f, 0.3f, 0.1f, 0.6f, 0.12f},
-                                {64, 32, 2.65f, 0.6f, 0.25f, 0.9f, 0.35f},
-                                {64, 64, 3.0f, 0.9f, 0.8f, 1.15f, 2.0f}};
+constexpr TileCost kKwCost[] = {{16, 16, 2.4f, 0.15f, 0.f, 0.25f, 0.04f, 0.1f},
+                                {32, 32, 2.5f, 0.39f, 0.02f, 0.54f, 0.1f, 0.15f},
+                                {64, 32, 2.55f, 0.66f, 0.12f, 0.79f, 0.2f, 0.29f},
+                                {64, 64, 2.8f, 1.0f, 0.65f, 0.98f, 0.79f, 0.61f}};
 struct KwTile {
   int mb, nb;
   float us;
@@ -302,10 +315,10 @@ inline TileCost kw_cold_cost(TileCost c) {
   return c;
 }
 // K: the bytes of one of `ksplit` ranges
-inline KwTile kw_choose_tile(int M, int N, int K, int ksplit, int cus, bool table) {
+inline KwTile kw_choose_tile(int M, int N, int K, int ksplit, int cus, EpilogueCost epi) {
   KwTile best{0, 0, 0.f};
   for (const auto& c : kKwCost) {
-    const float us = tile_us(M <= kKwColdRows ? kw_cold_cost(c) : c, M, N, K, ksplit, cus, table);
+    const float us = tile_us(M <= kKwColdRows ? kw_cold_cost(c) : c, M, N, K, ksplit, cus, epi);
     if (best.mb == 0 || us < best.us) best = KwTile{c.tm / 16, c.tn / 16, us};
   }
   return best;

@@ -34,9 +34,11 @@ __device__ __forceinline__ float fake_quantize_b(float x, float cmax, int& mask,
   return symmetry ? q * scale : (q + kQ) * scale;
 }
 // A quantiser whose scale many elements share: quantize_b and fake_quantize_b bit for bit, the
-// division by the scale made of a correctly rounded reciprocal, taken once, and two residual
-// corrections (Markstein: the quotient is then the correctly rounded one) -- 5 instructions
-// instead of the 12 of a division, in launches that are bound by them.
+// division by the scale made of a correctly rounded reciprocal, taken once, and a residual
+// correction -- 3 instructions instead of the 12 of a division, in launches that are bound by them.
+// Elements and clip values are halfs, so that the codes can be compared one by one: over all finite
+// clip values and all halfs (2 x 10^9 pairs, both quantisers) they are those of the division, as
+// with a second correction; without any 27265 differ.
 // The clamp comes first, on the element: an infinite one has no residual (inf - inf), and of an
 // element inside the clip value the quotient is at most 127 in magnitude, whatever its rounding, so
 // that none is needed behind it.  A NaN becomes the lesser bound there, code -127, as it does in
@@ -51,14 +53,16 @@ struct Quantiser {
   }
   __device__ __forceinline__ float quotient(float x) const {
     x = __builtin_amdgcn_fmed3f(x, lo, hi);
-    float q = x * inv;
-    q = __builtin_fmaf(__builtin_fmaf(-scale, q, x), inv, q);
+    const float q = x * inv;
     return __builtin_fmaf(__builtin_fmaf(-scale, q, x), inv, q);
   }
   __device__ __forceinline__ float rounded(float x) const {  // -127 .. 127
     return floorf(quotient(x) + 0.5f);
   }
-  __device__ __forceinline__ int code(float x) const { return (int)rounded(x); }
+  // four codes of one word: the conversion floors and writes its byte
+  __device__ __forceinline__ uint32_t pack4(float x0, float x1, float x2, float x3) const {
+    return floor_pack4_i8(quotient(x0) + 0.5f, quotient(x1) + 0.5f, quotient(x2) + 0.5f, quotient(x3) + 0.5f);
+  }
   __device__ __forceinline__ float fake(float x) const { return rounded(x) * scale; }
   // the unsigned quantiser (symmetry = false)
   __device__ __forceinline__ float fake_unsigned(float x) const {

@@ -30,6 +30,13 @@ __device__ __forceinline__ const __half* unit_row(const LayerPrepSection& s, int
   return s.src + (long)(r / s.n1) * s.stride0 + (long)(r % s.n1) * s.stride1;
 }
 
+__device__ __forceinline__ uint2 codes8(const Quantiser& of, const half8_t& x) {
+  float f[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) f[e] = __half2float(x.v[e]);
+  return make_uint2(of.pack4(f[0], f[1], f[2], f[3]), of.pack4(f[4], f[5], f[6], f[7]));
+}
+
 __device__ __forceinline__ void unit_codes(const LayerPrepSection& s, int block) {
   const int per_row = (s.K + kUnitK - 1) / kUnitK;
   const int rb = block / per_row, kc = block - rb * per_row;
@@ -51,12 +58,10 @@ __device__ __forceinline__ void unit_codes(const LayerPrepSection& s, int block)
     uint32_t w[4];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      int q[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) q[e] = of.code(__half2float(x[i][h].v[e]));
+      const uint2 q = codes8(of, x[i][h]);
       const bool on = row < s.rows && k + h * 8 < s.K;
-      w[2 * h] = on ? pack4_i8(q[0], q[1], q[2], q[3]) : 0u;
-      w[2 * h + 1] = on ? pack4_i8(q[4], q[5], q[6], q[7]) : 0u;
+      w[2 * h] = on ? q.x : 0u;
+      w[2 * h + 1] = on ? q.y : 0u;
     }
     *reinterpret_cast<uint4*>(static_cast<int8_t*>(s.dst) + blocked_offset(row, k, s.k_pad)) =
         make_uint4(w[0], w[1], w[2], w[3]);
@@ -96,12 +101,7 @@ __device__ __forceinline__ void ln_store(const half8_t& x, const half8_t& g, con
   for (int k = 0; k < 8; ++k)
     o.v[k] = __float2half_rn((__half2float(x.v[k]) - mean) * rstd * __half2float(g.v[k]) + __half2float(b.v[k]));
   if (out) *reinterpret_cast<half8_t*>(out) = o;
-  if (codes) {
-    int q[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) q[k] = of.code(__half2float(o.v[k]));
-    *reinterpret_cast<uint2*>(codes) = make_uint2(pack4_i8(q[0], q[1], q[2], q[3]), pack4_i8(q[4], q[5], q[6], q[7]));
-  }
+  if (codes) *reinterpret_cast<uint2*>(codes) = codes8(of, o);
 }
 
 // Layer norm of one row by a wavefront (opb_layer_norm: var = E[x^2] - E[x]^2 + 1e-8), the row kept

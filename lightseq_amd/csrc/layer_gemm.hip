@@ -33,7 +33,7 @@ __device__ __forceinline__ half4_t pack_half4(float a, float b, float c, float d
   return o;
 }
 
-// eight halfs as one 16-byte access: an LDS tile's lane holds sixteen neighbouring columns
+// eight halfs as one 16-byte access
 __device__ __forceinline__ half8_t ld8(const __half* p) { return *reinterpret_cast<const half8_t*>(p); }
 __device__ __forceinline__ void st8(void* p, const half8_t& x) { *reinterpret_cast<half8_t*>(p) = x; }
 
@@ -68,7 +68,7 @@ struct HeadPart {
 // (opb_quant_bias_add_transform_20314); cache_cmax: fake-quantised like a cache entry
 template <bool CACHE>
 struct EpiHeads {
-  static constexpr bool kTable = false, kBlockedOut = false, kClips = true;
+  static constexpr bool kTable = false, kBlockedOut = false, kClips = true, kStaged = true;
   HeadPart p0, p1, p2;
   const __half *bias, *cache_cmax;
   ProductClips clips;
@@ -115,24 +115,12 @@ struct EpiHeads {
     for (int k = 0; k < 4; ++k) x[k] = last(clips.value(c[k], __half2float(col.b.v[k])));
     *reinterpret_cast<half4_t*>(row_ptr(col, m)) = pack_half4(x[0], x[1], x[2], x[3]);
   }
-  __device__ __forceinline__ void store16(long m, int n, int N, const v16i& c, bool) const {
-    const Col col = column(n, N);
-    __half* p = row_ptr(col, (int)m);
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const half8_t b = ld8(bias + n + 8 * h);
-      half8_t x;
-#pragma unroll
-      for (int k = 0; k < 8; ++k) x.v[k] = __float2half_rn(last(clips.value(c[8 * h + k], __half2float(b.v[k]))));
-      st8(p + 8 * h, x);
-    }
-  }
   bool aligned() const { return true; }
 };
 
 // (dequantised code + bias) + residual (opb_quant_dropout_res_bias)
 struct EpiResidual {
-  static constexpr bool kTable = false, kBlockedOut = false, kClips = true;
+  static constexpr bool kTable = false, kBlockedOut = false, kClips = true, kStaged = true, kFetch = true;
   __half* out;
   const __half *bias, *residual;
   ProductClips clips;
@@ -148,26 +136,15 @@ struct EpiResidual {
   __device__ __forceinline__ Col column(int n, int) const {
     return Col{*reinterpret_cast<const half4_t*>(bias + n)};
   }
-  __device__ __forceinline__ void store4(int m, int n, int N, const Col& col, const v4i& c) const {
-    const long at = (long)m * N + n;
-    const half4_t r = *reinterpret_cast<const half4_t*>(residual + at);
+  __device__ __forceinline__ half4_t fetch(int m, int n, int N) const {
+    return *reinterpret_cast<const half4_t*>(residual + (long)m * N + n);
+  }
+  __device__ __forceinline__ void store4(int m, int n, int N, const Col& col, const v4i& c, const half4_t& r) const {
     float x[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k)
       x[k] = clips.value(c[k], __half2float(col.b.v[k])) + __half2float(r.v[k]);
-    *reinterpret_cast<half4_t*>(out + at) = pack_half4(x[0], x[1], x[2], x[3]);
-  }
-  __device__ __forceinline__ void store16(long m, int n, int N, const v16i& c, bool) const {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const long at = m * N + n + 8 * h;
-      const half8_t b = ld8(bias + n + 8 * h), r = ld8(residual + at);
-      half8_t x;
-#pragma unroll
-      for (int k = 0; k < 8; ++k)
-        x.v[k] = __float2half_rn(clips.value(c[8 * h + k], __half2float(b.v[k])) + __half2float(r.v[k]));
-      st8(out + at, x);
-    }
+    *reinterpret_cast<half4_t*>(out + (long)m * N + n) = pack_half4(x[0], x[1], x[2], x[3]);
   }
   bool aligned() const { return true; }
 };
@@ -176,7 +153,7 @@ struct EpiResidual {
 // (opb_quant_dropout_act_bias; in_cmax: that product's input clip)
 template <bool RELU>
 struct EpiAct {
-  static constexpr bool kTable = false, kBlockedOut = true, kClips = true;
+  static constexpr bool kTable = false, kBlockedOut = true, kClips = true, kColumn16 = true;
   __half* out;
   int out_k;  // bytes of a row of `out`
   const __half *bias, *in_cmax;
@@ -211,13 +188,16 @@ struct EpiAct {
     *reinterpret_cast<half4_t*>(reinterpret_cast<char*>(out) + blocked_offset(m, 2 * n, out_k)) =
         four(col.b, c[0], c[1], c[2], c[3]);
   }
-  __device__ __forceinline__ void store16(long m, int n, int, const v16i& c, bool) const {
+  struct Col16 {
+    half8_t b[2];
+  };
+  __device__ __forceinline__ Col16 column16(int n) const { return Col16{{ld8(bias + n), ld8(bias + n + 8)}}; }
+  __device__ __forceinline__ void store16(long m, int n, int, const v16i& c, const Col16& col) const {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const half8_t b = ld8(bias + n + 8 * h);
       half8_t x;
 #pragma unroll
-      for (int k = 0; k < 8; ++k) x.v[k] = __float2half_rn(value(c[8 * h + k], b.v[k]));
+      for (int k = 0; k < 8; ++k) x.v[k] = __float2half_rn(value(c[8 * h + k], col.b[h].v[k]));
       st8(reinterpret_cast<char*>(out) + blocked_offset(m, 2 * (n + 8 * h), out_k), x);
     }
   }
@@ -227,7 +207,7 @@ struct EpiAct {
 // second feed-forward product, fp16: (product, rounded as it was stored, + bias) + residual
 // (opb_dropout_res_bias)
 struct EpiFfn2 {
-  static constexpr bool kTable = false, kBlockedOut = false;
+  static constexpr bool kTable = false, kBlockedOut = false, kStaged = true, kFetch = true;
   __half* out;
   const __half *bias, *residual;
   struct Col {
@@ -236,27 +216,15 @@ struct EpiFfn2 {
   __device__ __forceinline__ Col column(int n, int) const {
     return Col{*reinterpret_cast<const half4_t*>(bias + n)};
   }
-  __device__ __forceinline__ void store4(int m, int n, int N, const Col& col, const v4f& c) const {
-    const long at = (long)m * N + n;
-    const half4_t r = *reinterpret_cast<const half4_t*>(residual + at);
+  __device__ __forceinline__ half4_t fetch(int m, int n, int N) const {
+    return *reinterpret_cast<const half4_t*>(residual + (long)m * N + n);
+  }
+  __device__ __forceinline__ void store4(int m, int n, int N, const Col& col, const v4f& c, const half4_t& r) const {
     float x[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k)
       x[k] = TT<__half>::rnd(TT<__half>::rnd(c[k]) + __half2float(col.b.v[k])) + __half2float(r.v[k]);
-    *reinterpret_cast<half4_t*>(out + at) = pack_half4(x[0], x[1], x[2], x[3]);
-  }
-  __device__ __forceinline__ void store16(long m, int n, int N, const v16f& c, bool) const {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const long at = m * N + n + 8 * h;
-      const half8_t b = ld8(bias + n + 8 * h), r = ld8(residual + at);
-      half8_t x;
-#pragma unroll
-      for (int k = 0; k < 8; ++k)
-        x.v[k] = __float2half_rn(TT<__half>::rnd(TT<__half>::rnd(c[8 * h + k]) + __half2float(b.v[k])) +
-                                 __half2float(r.v[k]));
-      st8(out + at, x);
-    }
+    *reinterpret_cast<half4_t*>(out + (long)m * N + n) = pack_half4(x[0], x[1], x[2], x[3]);
   }
   bool aligned() const { return true; }
 };
@@ -265,7 +233,7 @@ struct EpiFfn2 {
 // [b][head][s][d] of each layer, bias added in fp16 (opb_bias_add_transform_20314,
 // arrange_encdec_kv)
 struct EpiKv {
-  static constexpr bool kTable = false, kBlockedOut = false;
+  static constexpr bool kTable = false, kBlockedOut = false, kStaged = true;
   __half *k, *v;
   long layer_stride;
   const __half* bias;
@@ -292,18 +260,6 @@ struct EpiKv {
   }
   __device__ __forceinline__ void store4(int m, int, int, const Col& col, const v4f& c) const {
     *reinterpret_cast<half4_t*>(row_ptr(col, m)) = four(col.b, c[0], c[1], c[2], c[3]);
-  }
-  __device__ __forceinline__ void store16(long m, int n, int N, const v16f& c, bool) const {
-    __half* p = row_ptr(column(n, N), (int)m);
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const half8_t b = ld8(bias + n + 8 * h);
-      half8_t x;
-#pragma unroll
-      for (int k = 0; k < 8; ++k)
-        x.v[k] = __float2half_rn(TT<__half>::rnd(c[8 * h + k]) + __half2float(b.v[k]));
-      st8(p + 8 * h, x);
-    }
   }
   bool aligned() const { return true; }
 };

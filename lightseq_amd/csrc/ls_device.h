@@ -73,10 +73,9 @@ __device__ __forceinline__ int requant_acc_fast(int acc, float alpha) {
   asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(q) : "v"(requant_acc_clamped(acc, alpha)));
   return q;
 }
-// four accumulators -> four codes in one word; the conversion writes its low byte in place
-__device__ __forceinline__ uint32_t requant_acc_pack4(int a0, int a1, int a2, int a3, float alpha) {
-  const float y0 = requant_acc_clamped(a0, alpha), y1 = requant_acc_clamped(a1, alpha);
-  const float y2 = requant_acc_clamped(a2, alpha), y3 = requant_acc_clamped(a3, alpha);
+// the floors of four floats between -128 and 128 as the bytes of one word; the conversion writes its
+// low byte in place
+__device__ __forceinline__ uint32_t floor_pack4_i8(float y0, float y1, float y2, float y3) {
   uint32_t p;
   asm("v_cvt_flr_i32_f32_sdwa %0, %1 dst_sel:BYTE_0 dst_unused:UNUSED_PAD src0_sel:DWORD"
       : "=v"(p)
@@ -91,6 +90,12 @@ __device__ __forceinline__ uint32_t requant_acc_pack4(int a0, int a1, int a2, in
       : "+v"(p)
       : "v"(y3));
   return p;
+}
+// four accumulators -> four codes in one word
+__device__ __forceinline__ uint32_t requant_acc_pack4(int a0, int a1, int a2, int a3, float alpha) {
+  const float y0 = requant_acc_clamped(a0, alpha), y1 = requant_acc_clamped(a1, alpha);
+  const float y2 = requant_acc_clamped(a2, alpha), y3 = requant_acc_clamped(a3, alpha);
+  return floor_pack4_i8(y0, y1, y2, y3);
 }
 // inference/kernels/common.h:17-23
 __device__ __forceinline__ float gelu_tanh(float x) {

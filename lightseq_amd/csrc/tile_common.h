@@ -122,20 +122,7 @@ __device__ __forceinline__ uint32_t float2int8_pack4(float x0, float x1, float x
   const float y1 = __builtin_amdgcn_fmed3f(x1 * quant_scale + 0.5f, -127.f, 127.5f);
   const float y2 = __builtin_amdgcn_fmed3f(x2 * quant_scale + 0.5f, -127.f, 127.5f);
   const float y3 = __builtin_amdgcn_fmed3f(x3 * quant_scale + 0.5f, -127.f, 127.5f);
-  uint32_t p;
-  asm("v_cvt_flr_i32_f32_sdwa %0, %1 dst_sel:BYTE_0 dst_unused:UNUSED_PAD src0_sel:DWORD"
-      : "=v"(p)
-      : "v"(y0));
-  asm("v_cvt_flr_i32_f32_sdwa %0, %1 dst_sel:BYTE_1 dst_unused:UNUSED_PRESERVE src0_sel:DWORD"
-      : "+v"(p)
-      : "v"(y1));
-  asm("v_cvt_flr_i32_f32_sdwa %0, %1 dst_sel:BYTE_2 dst_unused:UNUSED_PRESERVE src0_sel:DWORD"
-      : "+v"(p)
-      : "v"(y2));
-  asm("v_cvt_flr_i32_f32_sdwa %0, %1 dst_sel:BYTE_3 dst_unused:UNUSED_PRESERVE src0_sel:DWORD"
-      : "+v"(p)
-      : "v"(y3));
-  return p;
+  return floor_pack4_i8(y0, y1, y2, y3);
 }
 
 

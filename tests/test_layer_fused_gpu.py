@@ -38,7 +38,8 @@ def test_encoder_layer_edges(batch, seq, hs, nh, ims, pre_ln, act, mask_type):
     assert d.max() < 2e-2 and d.mean() < 1e-3, (d.max(), d.mean())
 
 
-@pytest.mark.parametrize("hs,ims,seq", [(512, 2048, 64), (768, 3072, 37), (768, 3072, 64), (768, 3072, 128)])
+@pytest.mark.parametrize("hs,ims,seq", [(512, 2048, 64), (768, 3072, 37), (768, 3072, 64), (768, 3072, 128),
+                                        (1024, 4096, 61)])
 def test_a_sequence_does_not_depend_on_its_batch(hs, ims, seq):
     from test_oracle_layer_ops import config0
     rng = np.random.default_rng(5)
@@ -50,6 +51,36 @@ def test_a_sequence_does_not_depend_on_its_batch(hs, ims, seq):
         full = layer(x, pad)
         for n in (1, 3, 9, 20):
             assert torch.equal(layer(x[:n].contiguous(), pad[:n].contiguous()), full[:n])
+
+
+@pytest.mark.parametrize("hs,nh,trg,src", [(512, 8, 61, 20), (1024, 16, 31, 64)])
+def test_a_target_does_not_depend_on_its_batch(hs, nh, trg, src):
+    """The same of a decoder layer: products into heads and caches, residuals, keys and values of the
+    encoder output, by tiles of 16 x 16 to 256 x 256 with remainders in rows."""
+    from lightseq_amd import layers as L
+    L.LSTransformerDecoderLayer.new_stack()
+    torch.manual_seed(7)
+    cfg = L.LSTransformerDecoderLayer.get_config(
+        max_batch_tokens=80 * max(trg, src), max_seq_len=64, hidden_size=hs, intermediate_size=4 * hs, nhead=nh,
+        attn_prob_dropout_ratio=0.0, activation_dropout_ratio=0.0, hidden_dropout_ratio=0.0, pre_layer_norm=True,
+        fp16=True, local_rank=0, nlayer=1, activation_fn="relu")
+    layer = L.LSTransformerDecoderLayer(cfg).half().to(DEV).eval()
+    layer.enable_quant()
+    at = layer.para_offset[18]
+    n = layer.para_offset[19] - at
+    with torch.no_grad():
+        layer.para[at:at + n] = torch.tensor([4.0, 0.15, 6.0], dtype=torch.half, device=DEV).repeat(n // 3)
+    try:
+        x = torch.randn(80, trg, hs, device=DEV).half()
+        enc = torch.randn(src, 80, hs, device=DEV).half()
+        pad = torch.zeros(80, src, device=DEV)
+        with torch.no_grad():
+            full = layer(x, enc, pad)
+            for b in (1, 2, 7, 16, 33):
+                got = layer(x[:b].contiguous(), enc[:, :b].contiguous(), pad[:b].contiguous())
+                assert torch.equal(got, full[:b]), b
+    finally:
+        _release([layer])
 
 
 @pytest.mark.parametrize("trg,src,pre_ln", [(1, 1, False), (33, 64, True), (64, 33, False)])
