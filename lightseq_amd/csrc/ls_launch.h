@@ -37,6 +37,11 @@ int fill_i32(int* p, int value, int n, hipStream_t s);
 // copies to or from pinned host memory made by a kernel: n 4-byte words / n fp16 values as floats
 int copy_words(const void* in, void* out, long n, hipStream_t s);
 int widen_f16(const __half* in, float* out, long n, hipStream_t s);
+// an encoder's result [batch, S, hidden] to pinned host memory, as floats or fp16: `row` at the positions
+// from lens[b] on of sequence b (beside work of another stream) / the others, `seq` as in an EncPack
+int host_padding(const __half* row, const int* lens, void* out, bool f16, int batch, int S, int hidden,
+                 hipStream_t s);
+int host_tokens(const __half* in, const int* seq, void* out, bool f16, int batch, int S, int hidden, hipStream_t s);
 int stored_u8_to_i8(const uint8_t* input, int8_t* output, int rows, int cols, bool transpose,
                     hipStream_t s);
 template <typename T>

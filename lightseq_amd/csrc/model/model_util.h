@@ -94,6 +94,24 @@ class HostIds {
   int* p_ = nullptr;
 };
 
+// Pinned ints that kernels read.
+class PinnedInts {
+ public:
+  PinnedInts() = default;
+  PinnedInts(const PinnedInts&) = delete;
+  PinnedInts& operator=(const PinnedInts&) = delete;
+  ~PinnedInts() {
+    if (p_) (void)hipHostFree(p_);
+  }
+  void alloc(size_t n) {
+    if (!p_) CHECK_GPU_ERROR(hipHostMalloc(reinterpret_cast<void**>(&p_), n * sizeof(int)));
+  }
+  int* get() const { return p_; }
+
+ private:
+  int* p_ = nullptr;
+};
+
 // A pointer that is set for the length of a call.
 class HostIdsScope {
  public:

@@ -26,9 +26,11 @@ class QuantBert : public LSModel {
 
  private:
   void infer(void* host_out, bool host_f16);
+  bool pads_first(int batch, int seq_len, bool host_f16);
   // owners first: released after the encoder, also when the constructor throws half way
-  StreamOwner stream_;
+  StreamOwner stream_, side_stream_;
   HostIds h_ids_;
+  PinnedInts h_lens_;  // tokens of each sequence of the call under way
   const int* host_ids_ = nullptr;  // the ids of an InferHost() call under way
   DeviceBuffer<int> d_input_, d_padding_mask_;
   DeviceBuffer<__half> d_encoder_output_;

@@ -315,7 +315,7 @@ void QuantBertEncoder::run_packed(const int* host_token_ids) {
   }
 }
 
-void QuantBertEncoder::run_one_infer(int batch_size, int batch_seq_len, const int* host_token_ids) {
+void QuantBertEncoder::set_batch(int batch_size, int batch_seq_len) {
   if (batch_size > _max_batch_size)
     throw std::runtime_error("batch size of input greater than max_batch_size");
   if (batch_seq_len > _tw._max_step)
@@ -324,6 +324,23 @@ void QuantBertEncoder::run_one_infer(int batch_size, int batch_seq_len, const in
   _batch_size = batch_size;
   _batch_seq_len = batch_seq_len;
   _batch_token_num = batch_size * batch_seq_len;
+}
+
+void QuantBertEncoder::make_padding_row() {
+  set_batch(1, 1);
+  if (!packed_route()) return;
+  const int id = _tw._padding_id;
+  CHECK_GPU_ERROR(hipMemcpyAsync(const_cast<int*>(_p_d_token_id), &id, sizeof(int), hipMemcpyHostToDevice, _stream));
+  run_packed(&id);
+  _padding_row.alloc(_tw._hidden_size);
+  CHECK_GPU_ERROR(hipMemcpyAsync(_padding_row.get(), _p_d_output, _tw._hidden_size * sizeof(__half),
+                                 hipMemcpyDeviceToDevice, _stream));
+  CHECK_GPU_ERROR(hipStreamSynchronize(_stream));
+  _padding_row_valid = true;
+}
+
+void QuantBertEncoder::run_one_infer(int batch_size, int batch_seq_len, const int* host_token_ids) {
+  set_batch(batch_size, batch_seq_len);
   if (packed_route()) {
     _seg_active = false;
     run_packed(host_token_ids);

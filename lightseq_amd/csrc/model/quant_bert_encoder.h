@@ -30,6 +30,18 @@ class QuantBertEncoder {
   // waits for workgroups of its own launch gave up; the encoder has switched that route off).
   bool finish_infer();
 
+  // What every position behind the end of its sequence holds after the stack: the row of a padding
+  // token, a constant of the weights like the activation tables (embedding zero, context zero).
+  // make_padding_row(): one pass of the stack over a single such token, when the model is loaded.
+  void make_padding_row();
+  // null where a call of that shape does not run the route that has such a row
+  const __half* padding_row(int batch_size, int batch_seq_len) {
+    set_batch(batch_size, batch_seq_len);
+    return _padding_row_valid && packed_route() ? _padding_row.get() : nullptr;
+  }
+  // start and length of each sequence, as the last call of that route left them
+  const int* sequences() const { return _pack_seq.get(); }
+
   // Debug taps (all optional, device pointers owned by the caller): copies of the
   // intermediates of layer `tap_layer`, for parity bisection.
   struct Taps {
@@ -65,6 +77,7 @@ class QuantBertEncoder {
   void ffn_add_norm();
   // the route of every call without taps: blocked operands, no rows for padding
   bool packed_route() const;
+  void set_batch(int batch_size, int batch_seq_len);
   void run_packed(const int* host_token_ids);
   int packed_rows(const int* host_token_ids);
   void ensure_row_major_weights();
@@ -103,6 +116,8 @@ class QuantBertEncoder {
   // packed route
   bool _blockable = false;  // widths that block (multiples of 64)
   DeviceBuffer<int> _pack_seq, _pack_map;
+  DeviceBuffer<__half> _padding_row;
+  bool _padding_row_valid = false;
   DeviceBuffer<__half> _residual;  // residual stream of the packed rows
   unsigned long long* _h_pack_rows = nullptr;  // pinned: ticket << 32 | rows of the plan
   unsigned _pack_ticket = 0;

@@ -281,6 +281,75 @@ int widen_f16(const __half* in, float* out, long n, hipStream_t s) {
   return lsh_check_launch("widen_f16_kernel");
 }
 
+// An encoder's result [batch, S, hidden] in pinned host memory, in two launches.  All positions behind
+// the ends of their sequences hold one row, which is known before the call (see EncPack): what the
+// link needs for them (0.37 of the bytes with lengths uniform between a quarter and the whole of S)
+// passes while the stack computes, the rest after it.
+// The first launch runs beside the stack's.  Ordinary stores would stay in the L2 as dirty lines and
+// every kernel boundary of the other stream would wait until they are out (14 MB by 8 to 2048
+// workgroups: a 10 us kernel beside it ends after 250 us), so these write through, and a wavefront
+// waits for each: 64 wavefronts keep the link busy (14 MB in 270 us) and the kernel beside them
+// ends after 25 us.
+template <typename Out>
+__device__ __forceinline__ uint4 out_piece(const __half* row, int piece) {
+  uint4 o;
+  if constexpr (sizeof(Out) == 4) {
+    const half4_t h = *reinterpret_cast<const half4_t*>(row + piece * 4);
+    const float4 f = make_float4(__half2float(h.v[0]), __half2float(h.v[1]), __half2float(h.v[2]), __half2float(h.v[3]));
+    __builtin_memcpy(&o, &f, sizeof(o));
+  } else {
+    o = *reinterpret_cast<const uint4*>(row + piece * 8);
+  }
+  return o;
+}
+template <typename Out>
+__global__ void __launch_bounds__(256)
+host_padding_kernel(const __half* __restrict__ row, const int* __restrict__ lens, uint4* __restrict__ out, int batch,
+                    int S, int pieces) {
+  typedef int v4 __attribute__((ext_vector_type(4)));
+  for (int c = threadIdx.x; c < pieces; c += blockDim.x) {
+    const v4 v = __builtin_bit_cast(v4, out_piece<Out>(row, c));
+    for (int b = 0; b < batch; ++b)
+      for (int p = lens[b] + blockIdx.x; p < S; p += gridDim.x)
+        asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_waitcnt vmcnt(0)" ::"v"(
+                         out + ((long)b * S + p) * pieces + c),
+                     "v"(v)
+                     : "memory");
+  }
+}
+template <typename Out>
+__global__ void __launch_bounds__(256)
+host_tokens_kernel(const __half* __restrict__ in, const int* __restrict__ seq, uint4* __restrict__ out, int batch,
+                   int S, int pieces) {
+  for (int p = blockIdx.x; p < batch * S; p += gridDim.x) {
+    const int b = p / S;
+    if (p - b * S >= seq[2 * b + 1]) continue;
+    const __half* row = in + (long)p * pieces * (16 / sizeof(Out));
+    for (int c = threadIdx.x; c < pieces; c += 256) out[(long)p * pieces + c] = out_piece<Out>(row, c);
+  }
+}
+int host_padding(const __half* row, const int* lens, void* out, bool f16, int batch, int S, int hidden,
+                 hipStream_t s) {
+  if (!row || !lens || !out || !al16(row) || !al16(out) || batch <= 0 || S <= 0 || hidden <= 0 || hidden % 8 != 0)
+    return lsh_fail(LSH_ERR_INVALID, "host_padding: bad arguments");
+  const int pieces = hidden / (f16 ? 8 : 4), waves = std::min((pieces + 63) / 64, 4);
+  const int blocks = (64 + waves - 1) / waves;
+  if (f16) host_padding_kernel<__half><<<blocks, 64 * waves, 0, s>>>(row, lens, static_cast<uint4*>(out), batch, S, pieces);
+  else host_padding_kernel<float><<<blocks, 64 * waves, 0, s>>>(row, lens, static_cast<uint4*>(out), batch, S, pieces);
+  return lsh_check_launch("host_padding_kernel");
+}
+int host_tokens(const __half* in, const int* seq, void* out, bool f16, int batch, int S, int hidden, hipStream_t s) {
+  if (!in || !seq || !out || !al16(in) || !al16(out) || batch <= 0 || S <= 0 || (long)batch * S >= (1L << 31) ||
+      hidden <= 0 || hidden % 8 != 0)
+    return lsh_fail(LSH_ERR_INVALID, "host_tokens: bad arguments");
+  const int blocks = std::min(batch * S, 2048);
+  if (f16)
+    host_tokens_kernel<__half><<<blocks, 256, 0, s>>>(in, seq, static_cast<uint4*>(out), batch, S, hidden / 8);
+  else
+    host_tokens_kernel<float><<<blocks, 256, 0, s>>>(in, seq, static_cast<uint4*>(out), batch, S, hidden / 4);
+  return lsh_check_launch("host_tokens_kernel");
+}
+
 #define LSH_INST(T)                                                                          \
   template int quantize_tensor<T>(const T*, int8_t*, long, float, hipStream_t);              \
   template int dequantize_tensor<T>(const int32_t*, T*, long, float, hipStream_t);           \

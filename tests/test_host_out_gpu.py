@@ -29,3 +29,47 @@ def test_ordinary_memory_is_refused(tmp_path):
             np.testing.assert_array_equal(pinned, want.astype(dtype))
     finally:
         model.close()
+
+
+def _ragged(lens, seq, pad, rng):
+    ids = rng.integers(1, 90, size=(len(lens), seq), dtype=np.int32)
+    for b, n in enumerate(lens):
+        ids[b, n:] = pad
+        if n > 3:
+            ids[b, 1] = pad  # padding inside a sequence is one of its rows
+    return ids
+
+
+@pytest.mark.parametrize("name,lens,seq", [
+    ("bert_base", [384] * 3 + [1, 0, 200, 383, 64, 97], 384),  # 1.1 MB of padding and more: sent ahead
+    ("bert_base", [128, 20, 3] + [90] * 29, 128),
+    ("bert_base", [0, 0, 0], 512),
+    ("bert_base", [512, 171], 512),  # one position of padding short of 1 MiB in floats
+    ("bert_base", [512, 170], 512),
+])
+def test_padding_sent_ahead_is_the_padding_of_the_stack(tmp_path_factory, name, lens, seq):
+    """Result by host memory against the one that stays on the device, in both formats."""
+    from lightseq_amd import inference, synthetic
+    cfg = dict(synthetic.bert_config(name), n_layer=2, vocab=128)
+    path = os.path.join(str(tmp_path_factory.mktemp("pads")), "m.pb")
+    synthetic.write_quant_bert(path, cfg, seed=3)
+    model = inference.QuantBert(path, 32)
+    try:
+        ids = _ragged(lens, seq, cfg["padding_id"], np.random.default_rng(seq))
+        dev = torch.from_numpy(ids).cuda()
+        out = torch.zeros(len(lens), seq, cfg["hidden"], dtype=torch.half, device="cuda")
+        model.infer(ids[:1])  # another shape first
+        got32, got16 = model.infer(ids).copy(), model.infer_fp16(ids).copy()
+        plain = inference.LSModel("QuantBert", path, 32)
+        try:
+            plain.set_input_ptr(0, dev.data_ptr())
+            plain.set_input_shape(0, dev.shape)
+            plain.set_output_ptr(0, out.data_ptr())
+            plain.infer_device()
+            want = out.cpu().numpy()
+        finally:
+            plain.close()
+        np.testing.assert_array_equal(got16, want)
+        np.testing.assert_array_equal(got32, want.astype(np.float32))
+    finally:
+        model.close()
