@@ -77,20 +77,20 @@ int launch_tile(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K, 
   constexpr int TM = WGM * MB * 32, TN = WGN * NB * 32;
   const int tm = (M + TM - 1) / TM, tn = (N + TN - 1) / TN;
   return launch_blk<gemm_blk_tile_kernel<Tr, Epi, WGM, WGN, MB, NB, NST>>(
-      dim3(tm * tn), 64 * WGM * WGN, (tile_lds_bytes<Epi, WGM, WGN, MB, NB, NST>()), s, A, W, M, N, K, tm, tn, epi);
+      dim3(tm * tn), 64 * WGM * WGN, NST * (TM + TN) * kBK, s, A, W, M, N, K, tm, tn, epi);
 }
 
 // The LDS tile kernel: 8 wavefronts for tiles from 128 x 128 up, 4 for the small ones (several
 // workgroups then share a compute unit and one's epilogue runs under the other's K loop).
-constexpr TileCost kLdsCost[] = {{64, 64, 2.2f, 1.54f, 0.22f, 1.13f, 0.27f, 0.69f},
-                                 {128, 64, 2.55f, 2.32f, 0.2f, 1.85f, 0.46f, 1.4f},
-                                 {128, 128, 2.5f, 3.36f, 1.07f, 2.7f, 0.52f, 2.55f},
-                                 {256, 128, 3.0f, 5.5f, 2.7f, 6.1f, 0.93f, 4.85f},
-                                 {256, 192, 3.65f, 7.3f, 2.35f, 9.25f, 1.5f, 7.25f},
-                                 {256, 256, 4.35f, 9.3f, 0.f, 14.2f, 2.2f, 8.95f}};
+constexpr TileCost kLdsCost[] = {{64, 64, 2.2f, 1.54f, 0.22f, 1.13f, 0.27f, 0.56f},
+                                 {128, 64, 2.55f, 2.32f, 0.2f, 1.85f, 0.46f, 1.1f},
+                                 {128, 128, 2.5f, 3.36f, 1.07f, 2.7f, 0.52f, 2.2f},
+                                 {256, 128, 3.0f, 5.5f, 2.7f, 6.1f, 0.93f, 3.9f},
+                                 {256, 192, 3.65f, 7.3f, 2.35f, 9.25f, 1.5f, 5.95f},
+                                 {256, 256, 4.35f, 9.3f, 0.f, 14.2f, 2.2f, 7.4f}};
 // (its third stage costs the 128 x 64 tile its third workgroup per compute unit)
 constexpr int kLongK = 2048;
-constexpr TileCost kLongKCost{128, 64, 2.55f, 2.32f, 0.2f, 2.35f, 0.46f, 1.4f};
+constexpr TileCost kLongKCost{128, 64, 2.55f, 2.32f, 0.2f, 2.35f, 0.46f, 1.1f};
 struct LdsTile {
   int tm = 0, tn = 0;
   float us = 0;

@@ -141,7 +141,7 @@ struct EpiDecQkvI8 {
 // that a row holds, where the rows are those of a plan.  The stand-alone launch reads and writes
 // all the codes once more and is one of nine launches of a layer: 10.3 us for 3072 rows of 3 x 1024.
 struct EpiPromptQkvI8 {
-  static constexpr bool kTable = false, kBlockedOut = false, kStaged = true, kFetch = true;
+  static constexpr bool kTable = false, kBlockedOut = false, kColumn16 = true, kFetch = true, kFetch16 = true;
   int8_t *q, *k, *v;
   const __half* bias;
   const int* row_map;
@@ -172,6 +172,26 @@ struct EpiPromptQkvI8 {
     *reinterpret_cast<uint32_t*>(row_ptr(col, p)) =
         float2int8_pack4(value(c[0], col.b.v[0]), value(c[1], col.b.v[1]), value(c[2], col.b.v[2]),
                          value(c[3], col.b.v[3]), quant_scale);
+  }
+  // 16 columns of one head (dim % 16 == 0)
+  struct Col16 {
+    half8_t b[2];
+  };
+  __device__ __forceinline__ Col16 column16(int n) const {
+    return Col16{{*reinterpret_cast<const half8_t*>(bias + n), *reinterpret_cast<const half8_t*>(bias + n + 8)}};
+  }
+  __device__ __forceinline__ int fetch16(int m, int, int) const { return fetch(m, 0, 0); }
+  __device__ __forceinline__ void store16(long, int n, int, const v16i& c, const Col16& col, int p) const {
+    uint32_t w[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const __half* b = &col.b[j >> 1].v[4 * (j & 1)];
+      w[j] = float2int8_pack4(value(c[4 * j], b[0]), value(c[4 * j + 1], b[1]), value(c[4 * j + 2], b[2]),
+                              value(c[4 * j + 3], b[3]), quant_scale);
+    }
+    const int part = div_by(n, hidden, inv_hidden), i = n - part * hidden, head = div_by(i, dim, inv_dim);
+    const Col at{(part == 0 ? q : part == 1 ? k : v) + (i - head * dim), head, part == 0 ? seq : max_step, {}};
+    *reinterpret_cast<uint4*>(row_ptr(at, p)) = make_uint4(w[0], w[1], w[2], w[3]);
   }
   bool aligned() const {
     return ((reinterpret_cast<uintptr_t>(bias) | reinterpret_cast<uintptr_t>(q) |

@@ -281,7 +281,7 @@ enum class EpilogueCost { kPlain, kTable, kArith };
 template <typename Epi>
 constexpr EpilogueCost epilogue_cost() {
   return Epi::kTable ? EpilogueCost::kTable
-                     : EpiStaged<Epi>::value || EpiHasClips<Epi>::value ? EpilogueCost::kArith : EpilogueCost::kPlain;
+                     : EpiHasColumn16<Epi>::value ? EpilogueCost::kArith : EpilogueCost::kPlain;
 }
 struct TileCost {
   int tm, tn;
@@ -307,7 +307,13 @@ struct KwTile {
 // Few rows: a generation step, whose weights come from the memory and not from the L2.  A compute
 // unit draws about 37 KB/us of them (16 x 1024 x 4096: 64 KB of weights per tile 4.6 us, 16 KB
 // 3.5 us), so a tile's weights are priced at that rate where it is more than the fitted slope.
+// The other constants are those of an earlier fit: the sweep's small launches find their weights in
+// the caches.
 constexpr int kKwColdRows = 64;
+constexpr TileCost kKwColdCost[] = {{16, 16, 2.3f, 0.2f, 0.05f, 0.2f, 0.03f, 0.1f},
+                                    {32, 32, 2.3f, 0.3f, 0.1f, 0.6f, 0.12f, 0.15f},
+                                    {64, 32, 2.65f, 0.6f, 0.25f, 0.9f, 0.35f, 0.3f},
+                                    {64, 64, 3.0f, 0.9f, 0.8f, 1.15f, 2.0f, 0.6f}};
 inline TileCost kw_cold_cost(TileCost c) {
   const float slope = (float)c.tn / 36.f;  // us per 1024 bytes of K
   c.b = c.b * 1.35f < slope ? slope / 1.35f : c.b;
@@ -317,8 +323,9 @@ inline TileCost kw_cold_cost(TileCost c) {
 // K: the bytes of one of `ksplit` ranges
 inline KwTile kw_choose_tile(int M, int N, int K, int ksplit, int cus, EpilogueCost epi) {
   KwTile best{0, 0, 0.f};
-  for (const auto& c : kKwCost) {
-    const float us = tile_us(M <= kKwColdRows ? kw_cold_cost(c) : c, M, N, K, ksplit, cus, epi);
+  for (int i = 0; i < 4; ++i) {
+    const TileCost c = M <= kKwColdRows ? kw_cold_cost(kKwColdCost[i]) : kKwCost[i];
+    const float us = tile_us(c, M, N, K, ksplit, cus, epi);
     if (best.mb == 0 || us < best.us) best = KwTile{c.tm / 16, c.tn / 16, us};
   }
   return best;

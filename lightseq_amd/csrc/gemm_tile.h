@@ -261,23 +261,11 @@ __device__ __forceinline__ void epi_store4(const Epi& e, int m, int n, int N, co
   if constexpr (EpiHasFetch<Epi>::value) e.store4(m, n, N, col, c, x);
   else e.store4(m, n, N, col, c);
 }
-// kStaged (optional): an LDS tile ends in store4 on rows laid out in LDS, not in store16 on
-// accumulators.  There a lane holds 16 columns of one row and its neighbours other rows, so a store
-// instruction of a row-major output touches 32 lines for 1 KB, and what the epilogue reads per
-// column is asked for when it is needed; here 16 lanes hold 64 columns of a row, whose column
-// values arrived during the K loop.  976 x 3072 x 1024 into heads, tiles of 64 x 64: 16.2 us with
-// store16, 9.9 so; of 128 x 128: 13.5 and 11.2.
-template <typename Epi, typename = void>
-struct EpiStaged : std::false_type {};
-template <typename Epi>
-struct EpiStaged<Epi, std::enable_if_t<Epi::kStaged>> : std::true_type {};
-template <typename Epi, int WGM, int WGN, int MB, int NB, int NST>
-constexpr int tile_lds_bytes() {
-  constexpr int ring = NST * (WGM * MB + WGN * NB) * 32 * kBK;
-  constexpr int rows = WGM * 32 * (WGN * NB * 32 * 4 + 16);
-  return EpiStaged<Epi>::value && rows > ring ? rows : ring;
-}
-// kColumn16 (optional): what store16 needs of the columns n .. n + 15, requested ahead of the K loop
+// kColumn16, kFetch16 (optional): what store16 needs of the columns n .. n + 15, and of row m or of its
+// 16 elements, requested ahead of the K loop and handed to it.  An epilogue that asks for them when
+// it needs them waits for one memory trip after another: 976 x 3072 x 1024 into heads 13.5 us so,
+// 9.2 with both requested (and 9.9 with the rows laid out in LDS and stored 64 columns at a time,
+// the accumulators' layout being no friend of whole lines).
 template <typename Epi, typename = void>
 struct EpiHasColumn16 : std::false_type {};
 template <typename Epi>
@@ -287,12 +275,15 @@ __device__ __forceinline__ auto epi_column16(const Epi& e, int n) {
   if constexpr (EpiHasColumn16<Epi>::value) return e.column16(n);
   else return EpiNoFetch{};
 }
+template <typename Epi, typename = void>
+struct EpiHasFetch16 : std::false_type {};
 template <typename Epi>
-__device__ __forceinline__ auto epi_column4(const Epi& e, int n, int N) {
-  if constexpr (EpiStaged<Epi>::value) return e.column(n, N);
+struct EpiHasFetch16<Epi, std::enable_if_t<Epi::kFetch16>> : std::true_type {};
+template <typename Epi>
+__device__ __forceinline__ auto epi_fetch16(const Epi& e, int m, int n, int N) {
+  if constexpr (EpiHasFetch16<Epi>::value) return e.fetch16(m, n, N);
   else return EpiNoFetch{};
 }
-
 // 32 x 32 products over 32 bytes of K: int8, or fp16 (the lanes hold the operands alike)
 __device__ __forceinline__ v16i mma32(const v4i& w, const v4i& a, const v16i& c) {
   return __builtin_amdgcn_mfma_i32_32x32x32_i8(w, a, c, 0, 0, 0);
@@ -312,7 +303,7 @@ __device__ __forceinline__ void tile_gemm(const int8_t* __restrict__ A,
                                           const int8_t* __restrict__ W, const Epi& epi_arg, int row0,
                                           int row_end, int N, int K, int tn, int8_t* smem) {
   const auto raw = epi_request(epi_arg);
-  constexpr bool LUT = is_lut<Epi>, STAGED = EpiStaged<Epi>::value;
+  constexpr bool LUT = is_lut<Epi>;
   // The operand order of the MFMA decides what a lane's 16 accumulators are: weight rows first,
   // 16 adjacent columns of one output row (one 16-byte store of int8 codes); activations first,
   // 16 rows of one column -- the layout for int32 output, whose stores then cover whole lines.
@@ -330,16 +321,22 @@ __device__ __forceinline__ void tile_gemm(const int8_t* __restrict__ A,
   const int wm = wave / WGN, wn = wave % WGN, l32 = lane & 31, g = lane >> 5;
   const int nk = K / kBK;
 
-  // per column: of 64-column groups where rows are staged, of this lane's 16 columns otherwise
-  constexpr int CG = STAGED ? TN / 64 : 1;
-  static_assert(!STAGED || TN % 64 == 0, "staged rows: groups of 64 columns");
-  decltype(epi_column4(epi_arg, 0, 0)) col4[CG];
   decltype(epi_column16(epi_arg, 0)) col16[NB];
+  decltype(epi_fetch16(epi_arg, 0, 0, 0)) x16[MB][NB];
+  auto first_col = [&](int j) { return min(tn * TN + wn * (NB * 32) + j * 32 + 16 * g, N - 16); };
+  auto fetch16 = [&]() {
 #pragma unroll
-  for (int cg = 0; cg < CG; ++cg) col4[cg] = epi_column4(epi_arg, min(tn * TN + cg * 64 + (tid & 15) * 4, N - 4), N);
+    for (int i = 0; i < MB; ++i)
 #pragma unroll
-  for (int j = 0; j < NB; ++j)
-    col16[j] = epi_column16(epi_arg, min(tn * TN + wn * (NB * 32) + j * 32 + 16 * g, N - 16));
+      for (int j = 0; j < NB; ++j)
+        x16[i][j] =
+            epi_fetch16(epi_arg, min(row0 + wm * (MB * 32) + i * 32 + l32, row_end - 1), first_col(j), N);
+  };
+#pragma unroll
+  for (int j = 0; j < NB; ++j) col16[j] = epi_column16(epi_arg, first_col(j));
+  // (wavefronts of more than four blocks have no registers left for residuals until the loop is over)
+  constexpr bool FETCH_AHEAD = MB * NB <= 4;
+  if (FETCH_AHEAD) fetch16();
 
   const int8_t *a_tile = A, *w_tile = W;
   if (BLOCKED) {
@@ -535,44 +532,7 @@ __device__ __forceinline__ void tile_gemm(const int8_t* __restrict__ A,
       }
     return;
   }
-  if constexpr (STAGED) {
-    // 32 rows of every wavefront at a time, as many rows of TN accumulators (16 bytes apart in banks)
-    typedef typename std::conditional<std::is_same<Acc16, v16i>::value, v4i, v4f>::type Acc4;
-    constexpr int LD = TN * 4 + 16, RPP = NWV * 4, PASS = WGM * 32 / RPP;
-    const int quad = tid & 15, first = tid >> 4;
-#pragma unroll
-    for (int i = 0; i < MB; ++i) {
-      auto row_of = [&](int p) {
-        const int lr = first + p * RPP;
-        return row0 + (lr >> 5) * (MB * 32) + i * 32 + (lr & 31);
-      };
-      decltype(epi_fetch(epi, 0, 0, 0)) x[PASS][CG];
-#pragma unroll
-      for (int p = 0; p < PASS; ++p)
-#pragma unroll
-        for (int cg = 0; cg < CG; ++cg)
-          x[p][cg] = epi_fetch(epi, min(row_of(p), row_end - 1), min(tn * TN + cg * 64 + quad * 4, N - 4), N);
-      __syncthreads();
-#pragma unroll
-      for (int j = 0; j < NB; ++j)
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          *reinterpret_cast<Acc4*>(smem + (wm * 32 + l32) * LD + (wn * (NB * 32) + j * 32 + 16 * g + 4 * q) * 4) =
-              Acc4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-      __syncthreads();
-#pragma unroll
-      for (int p = 0; p < PASS; ++p) {
-        const int m = row_of(p);
-#pragma unroll
-        for (int cg = 0; cg < CG; ++cg) {
-          const int nl = cg * 64 + quad * 4;
-          const Acc4 c = *reinterpret_cast<const Acc4*>(smem + (first + p * RPP) * LD + nl * 4);
-          if (m < row_end && tn * TN + nl < N) epi_store4(epi, m, tn * TN + nl, N, col4[cg], c, x[p][cg]);
-        }
-      }
-    }
-    return;
-  }
+  if (!FETCH_AHEAD) fetch16();
   const int8_t* tab = smem + tab_slot * STAGE;
 #pragma unroll
   for (int i = 0; i < MB; ++i) {
@@ -584,8 +544,9 @@ __device__ __forceinline__ void tile_gemm(const int8_t* __restrict__ A,
         const int n = tn * TN + nl;
         if (n < N) {
           if constexpr (LUT) epi.store16_lds(m, n, N, acc[i][j], true, tab, nl);
+          else if constexpr (EpiHasFetch16<Epi>::value) epi.store16(m, n, N, acc[i][j], col16[j], x16[i][j]);
           else if constexpr (EpiHasColumn16<Epi>::value) epi.store16(m, n, N, acc[i][j], col16[j]);
-          else if constexpr (!STAGED) epi.store16(m, n, N, acc[i][j], true);
+          else epi.store16(m, n, N, acc[i][j], true);
         }
       }
     }

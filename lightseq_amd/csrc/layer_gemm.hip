@@ -33,9 +33,13 @@ __device__ __forceinline__ half4_t pack_half4(float a, float b, float c, float d
   return o;
 }
 
-// eight halfs as one 16-byte access
+// eight halfs as one 16-byte access; an LDS tile's lane holds sixteen neighbouring columns
 __device__ __forceinline__ half8_t ld8(const __half* p) { return *reinterpret_cast<const half8_t*>(p); }
 __device__ __forceinline__ void st8(void* p, const half8_t& x) { *reinterpret_cast<half8_t*>(p) = x; }
+struct Half16 {
+  half8_t h[2];
+};
+__device__ __forceinline__ Half16 ld16(const __half* p) { return Half16{{ld8(p), ld8(p + 8)}}; }
 
 // clip values {input, weight, output} of an int8 product
 struct ProductClips {
@@ -68,7 +72,7 @@ struct HeadPart {
 // (opb_quant_bias_add_transform_20314); cache_cmax: fake-quantised like a cache entry
 template <bool CACHE>
 struct EpiHeads {
-  static constexpr bool kTable = false, kBlockedOut = false, kClips = true, kStaged = true;
+  static constexpr bool kTable = false, kBlockedOut = false, kClips = true, kColumn16 = true, kFetch16 = true;
   HeadPart p0, p1, p2;
   const __half *bias, *cache_cmax;
   ProductClips clips;
@@ -115,12 +119,39 @@ struct EpiHeads {
     for (int k = 0; k < 4; ++k) x[k] = last(clips.value(c[k], __half2float(col.b.v[k])));
     *reinterpret_cast<half4_t*>(row_ptr(col, m)) = pack_half4(x[0], x[1], x[2], x[3]);
   }
+  struct Col16 {
+    Half16 b;
+    __half* base;
+    int head, len;
+  };
+  __device__ __forceinline__ Col16 column16(int n) const {
+    const Col c = column(n, 0);
+    return Col16{ld16(bias + n), c.base + c.off, c.head, c.len};
+  }
+  struct Row16 {
+    int b, s;
+  };
+  __device__ __forceinline__ Row16 fetch16(int m, int, int) const {
+    const int b = div_by(m, seq, inv_seq);
+    return Row16{b, m - b * seq};
+  }
+  __device__ __forceinline__ void store16(long, int, int, const v16i& c, const Col16& col, const Row16& r) const {
+    __half* p = col.base + ((long)(r.b * heads + col.head) * col.len + r.s) * dim;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      half8_t x;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) x.v[k] = __float2half_rn(last(clips.value(c[8 * h + k], __half2float(col.b.h[h].v[k]))));
+      st8(p + 8 * h, x);
+    }
+  }
   bool aligned() const { return true; }
 };
 
 // (dequantised code + bias) + residual (opb_quant_dropout_res_bias)
 struct EpiResidual {
-  static constexpr bool kTable = false, kBlockedOut = false, kClips = true, kStaged = true, kFetch = true;
+  static constexpr bool kTable = false, kBlockedOut = false, kClips = true, kFetch = true, kColumn16 = true,
+                        kFetch16 = true;
   __half* out;
   const __half *bias, *residual;
   ProductClips clips;
@@ -145,6 +176,18 @@ struct EpiResidual {
     for (int k = 0; k < 4; ++k)
       x[k] = clips.value(c[k], __half2float(col.b.v[k])) + __half2float(r.v[k]);
     *reinterpret_cast<half4_t*>(out + (long)m * N + n) = pack_half4(x[0], x[1], x[2], x[3]);
+  }
+  __device__ __forceinline__ Half16 column16(int n) const { return ld16(bias + n); }
+  __device__ __forceinline__ Half16 fetch16(int m, int n, int N) const { return ld16(residual + (long)m * N + n); }
+  __device__ __forceinline__ void store16(long m, int n, int N, const v16i& c, const Half16& b, const Half16& r) const {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      half8_t x;
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        x.v[k] = __float2half_rn(clips.value(c[8 * h + k], __half2float(b.h[h].v[k])) + __half2float(r.h[h].v[k]));
+      st8(out + m * N + n + 8 * h, x);
+    }
   }
   bool aligned() const { return true; }
 };
@@ -188,16 +231,13 @@ struct EpiAct {
     *reinterpret_cast<half4_t*>(reinterpret_cast<char*>(out) + blocked_offset(m, 2 * n, out_k)) =
         four(col.b, c[0], c[1], c[2], c[3]);
   }
-  struct Col16 {
-    half8_t b[2];
-  };
-  __device__ __forceinline__ Col16 column16(int n) const { return Col16{{ld8(bias + n), ld8(bias + n + 8)}}; }
-  __device__ __forceinline__ void store16(long m, int n, int, const v16i& c, const Col16& col) const {
+  __device__ __forceinline__ Half16 column16(int n) const { return ld16(bias + n); }
+  __device__ __forceinline__ void store16(long m, int n, int, const v16i& c, const Half16& b) const {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       half8_t x;
 #pragma unroll
-      for (int k = 0; k < 8; ++k) x.v[k] = __float2half_rn(value(c[8 * h + k], col.b[h].v[k]));
+      for (int k = 0; k < 8; ++k) x.v[k] = __float2half_rn(value(c[8 * h + k], b.h[h].v[k]));
       st8(reinterpret_cast<char*>(out) + blocked_offset(m, 2 * (n + 8 * h), out_k), x);
     }
   }
@@ -207,7 +247,7 @@ struct EpiAct {
 // second feed-forward product, fp16: (product, rounded as it was stored, + bias) + residual
 // (opb_dropout_res_bias)
 struct EpiFfn2 {
-  static constexpr bool kTable = false, kBlockedOut = false, kStaged = true, kFetch = true;
+  static constexpr bool kTable = false, kBlockedOut = false, kFetch = true, kColumn16 = true, kFetch16 = true;
   __half* out;
   const __half *bias, *residual;
   struct Col {
@@ -226,6 +266,19 @@ struct EpiFfn2 {
       x[k] = TT<__half>::rnd(TT<__half>::rnd(c[k]) + __half2float(col.b.v[k])) + __half2float(r.v[k]);
     *reinterpret_cast<half4_t*>(out + (long)m * N + n) = pack_half4(x[0], x[1], x[2], x[3]);
   }
+  __device__ __forceinline__ Half16 column16(int n) const { return ld16(bias + n); }
+  __device__ __forceinline__ Half16 fetch16(int m, int n, int N) const { return ld16(residual + (long)m * N + n); }
+  __device__ __forceinline__ void store16(long m, int n, int N, const v16f& c, const Half16& b, const Half16& r) const {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      half8_t x;
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        x.v[k] = __float2half_rn(TT<__half>::rnd(TT<__half>::rnd(c[8 * h + k]) + __half2float(b.h[h].v[k])) +
+                                 __half2float(r.h[h].v[k]));
+      st8(out + m * N + n + 8 * h, x);
+    }
+  }
   bool aligned() const { return true; }
 };
 
@@ -233,7 +286,7 @@ struct EpiFfn2 {
 // [b][head][s][d] of each layer, bias added in fp16 (opb_bias_add_transform_20314,
 // arrange_encdec_kv)
 struct EpiKv {
-  static constexpr bool kTable = false, kBlockedOut = false, kStaged = true;
+  static constexpr bool kTable = false, kBlockedOut = false, kColumn16 = true, kFetch16 = true;
   __half *k, *v;
   long layer_stride;
   const __half* bias;
@@ -260,6 +313,33 @@ struct EpiKv {
   }
   __device__ __forceinline__ void store4(int m, int, int, const Col& col, const v4f& c) const {
     *reinterpret_cast<half4_t*>(row_ptr(col, m)) = four(col.b, c[0], c[1], c[2], c[3]);
+  }
+  struct Col16 {
+    Half16 b;
+    __half* base;
+    int head;
+  };
+  __device__ __forceinline__ Col16 column16(int n) const {
+    const Col c = column(n, 0);
+    return Col16{ld16(bias + n), c.base, c.head};
+  }
+  struct Row16 {
+    int b, s;
+  };
+  __device__ __forceinline__ Row16 fetch16(int m, int, int) const {
+    const int b = div_by(m, seq, inv_seq);
+    return Row16{b, m - b * seq};
+  }
+  __device__ __forceinline__ void store16(long, int, int, const v16f& c, const Col16& col, const Row16& r) const {
+    __half* p = col.base + ((long)(r.b * heads + col.head) * seq + r.s) * dim;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      half8_t x;
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        x.v[k] = __float2half_rn(TT<__half>::rnd(c[8 * h + k]) + __half2float(col.b.h[h].v[k]));
+      st8(p + 8 * h, x);
+    }
   }
   bool aligned() const { return true; }
 };
