@@ -13,7 +13,7 @@
 #include <type_traits>
 
 #include "ls_device.h"
-#include "layer_device.h"
+#include "layer_prep.h"
 #include "ls_launch.h"
 #include "tile_common.h"
 
@@ -1130,13 +1130,19 @@ template <int D, int NKB>
 __global__ void __launch_bounds__(64)
 layer_attn_few_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
                       const __half* __restrict__ v, const __half* __restrict__ add_mask, int q_blocks, int q_len,
-                      int head_num, int key_len, float alpha, int causal, int8_t* __restrict__ codes,
-                      const __half* __restrict__ q_cmax, int k_pad) {
+                      int head_num, int key_len, int attn_blocks, float alpha, int causal,
+                      int8_t* __restrict__ codes, const __half* __restrict__ q_cmax, int k_pad,
+                      const LayerRide also) {
   constexpr int CH = D / 8, VS = 36;  // 16-byte chunks of a row; halfs per dimension in LDS
   constexpr int VP = 8 * CH / 64 > 0 ? 8 * CH / 64 : 1;  // patches of 4 keys x 8 dims per lane and block
   __shared__ __align__(16) _Float16 Vt[D * VS];
   __shared__ __align__(16) float addm[NKB * 32];
   const int lane = threadIdx.x;
+  if ((int)blockIdx.x >= attn_blocks) {
+    const int w = (int)blockIdx.x - attn_blocks;
+    ride_unit(also, w >> 2, w & 3);
+    return;
+  }
   const int bh = (int)blockIdx.x / q_blocks, q0 = ((int)blockIdx.x - bh * q_blocks) * 32;
   const int b = bh / head_num, head = bh - b * head_num;
   const int l32 = lane & 31, g = lane >> 5;
@@ -1269,12 +1275,12 @@ layer_attn_few_kernel(const __half* __restrict__ q, const __half* __restrict__ k
 template <int D>
 static void launch_attn_few(const __half* q, const __half* k, const __half* v, const __half* add_mask,
                             int8_t* codes, const __half* cmax, int k_pad, int pairs, int q_len, int head_num,
-                            int key_len, float alpha, bool causal, hipStream_t s) {
+                            int key_len, float alpha, bool causal, hipStream_t s, const LayerRide& ride) {
   const int q_blocks = (q_len + 31) / 32;
 #define LSH_FEW(NKB)                                                                                    \
-  layer_attn_few_kernel<D, NKB><<<pairs * q_blocks, 64, 0, s>>>(q, k, v, add_mask, q_blocks, q_len,     \
-                                                                head_num, key_len, alpha,               \
-                                                                causal ? 1 : 0, codes, cmax, k_pad)
+  layer_attn_few_kernel<D, NKB><<<pairs * q_blocks + 4 * ride.blocks, 64, 0, s>>>(                      \
+      q, k, v, add_mask, q_blocks, q_len, head_num, key_len, pairs * q_blocks, alpha, causal ? 1 : 0,   \
+      codes, cmax, k_pad, ride)
   if (key_len <= 32) LSH_FEW(1);
   else if (key_len <= 64) LSH_FEW(2);
   else if (key_len <= 96) LSH_FEW(3);
@@ -1283,10 +1289,19 @@ static void launch_attn_few(const __half* q, const __half* k, const __half* v, c
 }
 
 constexpr int kAttnFewQueries = 128;
+// Few queries: the fragments of a pair's keys and values fit a wavefront's registers up to 128 keys
+// of 64 dimensions (64 of 128).
+static bool few_queries(int seq_len, int key_len, long pairs, int dim_per_head) {
+  return seq_len <= kAttnFewQueries && pairs < (1L << 30) && key_len <= 128 && key_len * dim_per_head <= 128 * 64;
+}
+bool layer_attention_takes_riders(int seq_len, int key_len, long batch_heads, int dim_per_head) {
+  return few_queries(seq_len, key_len, batch_heads, dim_per_head);
+}
 
 int layer_attention_codes(const __half* q, const __half* k, const __half* v, const __half* add_mask,
                           int8_t* codes, const __half* cmax, int k_pad, int batch, int seq_len, int key_len,
-                          int head_num, int dim_per_head, bool mask_future, hipStream_t s) {
+                          int head_num, int dim_per_head, bool mask_future, hipStream_t s,
+                          const LayerPrep* also) {
   if (batch <= 0 || seq_len <= 0 || key_len <= 0 || head_num <= 0 || !q || !k || !v || !codes || !cmax ||
       k_pad % 64 != 0 || k_pad < head_num * dim_per_head || (mask_future && seq_len != key_len))
     return lsh_fail(LSH_ERR_INVALID, "layer_attention_codes: bad arguments");
@@ -1297,23 +1312,25 @@ int layer_attention_codes(const __half* q, const __half* k, const __half* v, con
     return lsh_fail(LSH_ERR_INVALID, "layer_attention: pointers must be 16-byte aligned");
   const float alpha = __half2float(
       __float2half_rn(1.0f / __half2float(__float2half_rn(sqrtf((float)dim_per_head)))));
-  // Few queries: the fragments of a pair's keys and values fit a wavefront's registers up to 128 keys
-  // of 64 dimensions (64 of 128).
   const long pairs = (long)batch * head_num;
-  if (seq_len <= kAttnFewQueries && pairs < (1L << 30) && key_len * dim_per_head <= 128 * 64 && key_len <= 128) {
+  LayerRide ride{};
+  if (also)
+    if (int rc = also->ride(&ride)) return rc;
+  if (few_queries(seq_len, key_len, pairs, dim_per_head)) {
     if (dim_per_head == 32)
       launch_attn_few<32>(q, k, v, add_mask, codes, cmax, k_pad, (int)pairs, seq_len, head_num, key_len, alpha,
-                          mask_future, s);
+                          mask_future, s, ride);
     else if (dim_per_head == 64)
       launch_attn_few<64>(q, k, v, add_mask, codes, cmax, k_pad, (int)pairs, seq_len, head_num, key_len, alpha,
-                          mask_future, s);
+                          mask_future, s, ride);
     else if (dim_per_head == 128)
       launch_attn_few<128>(q, k, v, add_mask, codes, cmax, k_pad, (int)pairs, seq_len, head_num, key_len, alpha,
-                           mask_future, s);
+                           mask_future, s, ride);
     else
       return lsh_fail(LSH_ERR_UNSUPPORTED, "layer_attention: dim_per_head must be 32, 64 or 128");
     return lsh_check_launch("layer_attn_few_kernel");
   }
+  if (ride.blocks > 0) return lsh_fail(LSH_ERR_UNSUPPORTED, "layer_attention: no riders in this form");
   if (!launch_attn<kAttnLayer>(dim_per_head, seq_len, batch * head_num, s, q, k, v,
                                reinterpret_cast<const int*>(add_mask), nullptr, codes, 0.f, head_num, alpha,
                                mask_future ? 1.f : 0.f, key_len, nullptr, cmax, k_pad))

@@ -1,7 +1,7 @@
 // What a quantised layer needs ahead of and between its products (layer_gemm.hip), in as few
 // launches as there are dependencies: one that prepares everything the forward pass starts from,
 // and the layer norm between two products.
-#include "layer_device.h"
+#include "layer_prep.h"
 #include "ls_launch.h"
 
 #include <algorithm>
@@ -18,81 +18,6 @@ namespace {
 // -- do not depend on one another, so they are ranges of workgroups of one grid: by the kernel
 // trace 8.0 us for a Transformer-base encoder layer (10 MB) and 18 us for a step of a
 // Transformer-big decoder layer (64 MB with its caches, 3.6 TB/s).
-//
-// Sections that write blocked matrices work on units of 16 rows x 512 columns: a wavefront reads
-// 128-byte pieces of 16 rows and writes 1 KB, the 16 rows x 64 bytes block; what a unit reads is
-// requested before any of it is converted.
-constexpr int kUnitK = 512;
-
-__device__ __forceinline__ const __half* unit_row(const LayerPrepSection& s, int row) {
-  const int r = min(row, s.rows - 1);
-  if (s.n1 == 1) return s.src + (long)r * s.stride0;
-  return s.src + (long)(r / s.n1) * s.stride0 + (long)(r % s.n1) * s.stride1;
-}
-
-__device__ __forceinline__ uint2 codes8(const Quantiser& of, const half8_t& x) {
-  float f[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) f[e] = __half2float(x.v[e]);
-  return make_uint2(of.pack4(f[0], f[1], f[2], f[3]), of.pack4(f[4], f[5], f[6], f[7]));
-}
-
-__device__ __forceinline__ void unit_codes(const LayerPrepSection& s, int block) {
-  const int per_row = (s.K + kUnitK - 1) / kUnitK;
-  const int rb = block / per_row, kc = block - rb * per_row;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int row = rb * 16 + (lane & 15);
-  const int k0 = kc * kUnitK + wave * 64 + (lane >> 4) * 16;
-  const __half* src = unit_row(s, row);
-  half8_t x[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-      x[i][h] = *reinterpret_cast<const half8_t*>(src + min(k0 + i * 256 + h * 8, s.K - 8));  // K % 8 == 0
-  const Quantiser of = Quantiser::of(cm(s.cmax));
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int k = k0 + i * 256;
-    if (k >= s.k_pad) break;
-    uint32_t w[4];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const uint2 q = codes8(of, x[i][h]);
-      const bool on = row < s.rows && k + h * 8 < s.K;
-      w[2 * h] = on ? q.x : 0u;
-      w[2 * h + 1] = on ? q.y : 0u;
-    }
-    *reinterpret_cast<uint4*>(static_cast<int8_t*>(s.dst) + blocked_offset(row, k, s.k_pad)) =
-        make_uint4(w[0], w[1], w[2], w[3]);
-  }
-}
-
-// fp16 -> blocked fp16 (64 bytes of K are 32 halfs), fake-quantised where `cmax` is set
-__device__ __forceinline__ void unit_halfs(const LayerPrepSection& s, int block) {
-  const int per_row = (s.K + kUnitK - 1) / kUnitK;
-  const int rb = block / per_row, kc = block - rb * per_row;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int row = rb * 16 + (lane & 15);
-  const int k0 = kc * kUnitK + wave * 32 + (lane >> 4) * 8;
-  const __half* src = unit_row(s, row);
-  half8_t x[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) x[i] = *reinterpret_cast<const half8_t*>(src + min(k0 + i * 128, s.K - 8));
-  const Quantiser of = Quantiser::of(s.cmax ? cm(s.cmax) : 1.f);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int k = k0 + i * 128;
-    if (k >= s.k_pad) break;
-    if (s.cmax) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) x[i].v[e] = __float2half_rn(of.fake(__half2float(x[i].v[e])));
-    }
-    if (row >= s.rows || k >= s.K) x[i] = half8_t{};
-    *reinterpret_cast<half8_t*>(static_cast<char*>(s.dst) + blocked_offset(row, 2 * k, 2 * s.k_pad)) = x[i];
-  }
-}
-
 // eight normalised elements to where they go (`out`, `codes`: null where nobody reads them)
 __device__ __forceinline__ void ln_store(const half8_t& x, const half8_t& g, const half8_t& b, float mean, float rstd,
                                          const Quantiser& of, __half* out, int8_t* codes) {
@@ -204,8 +129,8 @@ layer_prep_kernel(const LayerPrepArgs a) {
   const int block = (int)blockIdx.x - first;
   const LayerPrepSection& s = a.s[i];
   switch (s.kind) {
-    case kPrepCodes: unit_codes(s, block); break;
-    case kPrepHalfs: unit_halfs(s, block); break;
+    case kPrepCodes: unit_codes(s, block, (int)(threadIdx.x >> 6)); break;
+    case kPrepHalfs: unit_halfs(s, block, (int)(threadIdx.x >> 6)); break;
     case kPrepNorm: {
       const int row = block * 4 + (int)(threadIdx.x >> 6);
       if (row < s.rows)
@@ -232,9 +157,10 @@ layer_prep_kernel(const LayerPrepArgs a) {
 __global__ void __launch_bounds__(256)
 layer_norm_codes_kernel(const __half* inp, __half* out, int8_t* codes, const __half* __restrict__ gamma,
                         const __half* __restrict__ beta, const __half* __restrict__ cmax, int rows,
-                        int hidden, int k_pad) {
-  const int row = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
-  if (row < rows) ln_row_any(inp, out, codes, gamma, beta, cmax, row, hidden, k_pad);
+                        int hidden, int k_pad, const LayerRide also) {
+  const int row = blockIdx.x * 4 + (int)(threadIdx.x >> 6), blocks = (rows + 3) >> 2;
+  if ((int)blockIdx.x >= blocks) ride_unit(also, (int)blockIdx.x - blocks, (int)(threadIdx.x >> 6));
+  else if (row < rows) ln_row_any(inp, out, codes, gamma, beta, cmax, row, hidden, k_pad);
 }
 
 }  // namespace
@@ -323,6 +249,21 @@ int LayerPrep::grow(const __half* src, __half* dst, int rows, int K, long dst_st
   s.stride1 = dst_stride;
   return add(s);
 }
+int LayerPrep::ride(LayerRide* out) const {
+  LayerRide r{};
+  if (_args.n > kLayerRideMost) return lsh_fail(LSH_ERR_UNSUPPORTED, "layer_prep: too many sections to ride");
+  for (int i = 0; i < kLayerRideMost; ++i) {
+    r.first[i] = i < _args.n ? r.blocks : 0x7fffffff;
+    if (i >= _args.n) continue;
+    if (_args.s[i].kind != kPrepCodes && _args.s[i].kind != kPrepHalfs)
+      return lsh_fail(LSH_ERR_UNSUPPORTED, "layer_prep: only matrices ride");
+    r.s[i] = _args.s[i];
+    r.blocks += _args.s[i].blocks;
+  }
+  if (r.blocks >= (1 << 26)) return lsh_fail(LSH_ERR_UNSUPPORTED, "layer_prep: too many workgroups");
+  *out = r;
+  return LSH_OK;
+}
 int LayerPrep::launch(hipStream_t s) const {
   LayerPrepArgs args = _args;
   long blocks = 0;
@@ -337,12 +278,15 @@ int LayerPrep::launch(hipStream_t s) const {
 }
 
 int layer_norm_codes(const __half* inp, __half* out, int8_t* codes, const __half* gamma, const __half* beta,
-                     const __half* cmax, int rows, int hidden, int k_pad, hipStream_t s) {
+                     const __half* cmax, int rows, int hidden, int k_pad, hipStream_t s, const LayerPrep* also) {
+  LayerRide ride{};
+  if (also)
+    if (int rc = also->ride(&ride)) return rc;
   if (!inp || (!out && !codes) || !gamma || !beta || (codes && !cmax) || rows <= 0 || hidden <= 0 ||
       hidden % 8 != 0)
     return lsh_fail(LSH_ERR_INVALID, "layer_norm_codes: bad arguments");
-  layer_norm_codes_kernel<<<(rows + 3) / 4, 256, 0, s>>>(inp, out, codes, gamma, beta, cmax, rows, hidden,
-                                                         k_pad);
+  layer_norm_codes_kernel<<<(rows + 3) / 4 + ride.blocks, 256, 0, s>>>(inp, out, codes, gamma, beta, cmax, rows,
+                                                                       hidden, k_pad, ride);
   return lsh_check_launch("layer_norm_codes_kernel");
 }
 

@@ -196,13 +196,20 @@ void TransformerDecoderLayer<T>::Forward(const T* dec_input_ptr, const T* enc_ou
   const bool relu = _activation_fn == "relu";
   const int src_tok = _batch_size * _src_seq_len;
 
-  LayerPrep prep;
+  const int self_batch = _predict ? _batch_size * _trg_seq_len : _batch_size;
+  const int from_len = _predict ? 1 : _trg_seq_len, to_len = _predict ? _step + 1 : _trg_seq_len;
+  // what the first product reads, and what rides in later launches ahead of its reader
+  LayerPrep prep, with_self, with_norm, with_cross, with_norm2;
+  const bool self_riders = layer_attention_takes_riders(from_len, to_len, (long)self_batch * _heads, hd);
+  const bool cross_riders = layer_attention_takes_riders(_trg_seq_len, _src_seq_len, (long)_batch_size * _heads, hd);
+  LayerPrep& early = self_riders ? with_self : prep;
   LSH_CALL(prep.codes(_attn_qkvw_ptr, _wqkv.get(), _attn_qkv_cmax_ptr + 1, 3 * hs, hs, _kh));
-  LSH_CALL(prep.codes(_attn_ow_ptr, _wself_out.get(), _attn_out_cmax_ptr + 1, hs, hs, _kh));
-  LSH_CALL(prep.codes(_encdec_attn_qw_ptr, _wq.get(), _encdec_qkv_cmax_ptr + 1, hs, hs, _kh));
-  LSH_CALL(prep.codes(_encdec_attn_ow_ptr, _wcross_out.get(), _encdec_out_cmax_ptr + 1, hs, hs, _kh));
-  LSH_CALL(prep.codes(_inter_w_ptr, _winter.get(), _inter_cmax_ptr + 1, ims, hs, _kh));
-  LSH_CALL(prep.halfs(_output_w_ptr, _woutput.get(), _output_cmax_ptr + 1, hs, ims, _ki, 1, ims, 0));
+  LSH_CALL(early.codes(_attn_ow_ptr, _wself_out.get(), _attn_out_cmax_ptr + 1, hs, hs, _kh));
+  LSH_CALL(early.codes(_encdec_attn_qw_ptr, _wq.get(), _encdec_qkv_cmax_ptr + 1, hs, hs, _kh));
+  LSH_CALL(with_norm.codes(_encdec_attn_ow_ptr, _wcross_out.get(), _encdec_out_cmax_ptr + 1, hs, hs, _kh));
+  LSH_CALL((cross_riders ? with_cross : with_norm)
+               .codes(_inter_w_ptr, _winter.get(), _inter_cmax_ptr + 1, ims, hs, _kh));
+  LSH_CALL(with_norm2.halfs(_output_w_ptr, _woutput.get(), _output_cmax_ptr + 1, hs, ims, _ki, 1, ims, 0));
   if (_is_pre_ln)
     LSH_CALL(prep.norm(dec_input_ptr, _qin.get(), _attn_nw_ptr, _attn_nb_ptr, _attn_qkv_cmax_ptr, tok, hs, _kh));
   else
@@ -212,7 +219,6 @@ void TransformerDecoderLayer<T>::Forward(const T* dec_input_ptr, const T* enc_ou
     LSH_CALL(prep.mask(enc_mask_ptr, mask_kind, _mask.get(), src_tok));
     mask = _mask.get();
   }
-  const int self_batch = _predict ? _batch_size * _trg_seq_len : _batch_size;
   if (_predict && _step > 0)  // :173-180: new cache = previous cache ++ this step's k / v
     for (int i = 0; i < 2; ++i)
       LSH_CALL(prep.grow(cache[2 + i], cache[i], self_batch * _heads, _step * hd, (long)(_step + 1) * hd));
@@ -249,7 +255,6 @@ void TransformerDecoderLayer<T>::Forward(const T* dec_input_ptr, const T* enc_ou
 
   // self attention (:91-233); k and v leave the product as the cache will hold them: fake-quantised
   // (:134-138)
-  const int from_len = _predict ? 1 : _trg_seq_len, to_len = _predict ? _step + 1 : _trg_seq_len;
   const size_t batch_dim = (size_t)tok * hs;
   T* q = _qkv.get();
   T* const self[3] = {q, _predict ? cache[0] : q + batch_dim, _predict ? cache[1] : q + 2 * batch_dim};
@@ -258,7 +263,8 @@ void TransformerDecoderLayer<T>::Forward(const T* dec_input_ptr, const T* enc_ou
   LSH_CALL(layer_gemm_heads(_qin.get(), _wqkv.get(), tok, 3, hs, _kh, _attn_qkvb_ptr, _attn_qkv_cmax_ptr,
                             _attn_qkv_cache_cmax_ptr, from_len, _heads, self, len, at, _stream));
   LSH_CALL(layer_attention_codes(self[0], self[1], self[2], nullptr, _qin.get(), _attn_out_cmax_ptr, _kh,
-                                 self_batch, from_len, to_len, _heads, hd, !_predict, _stream));
+                                 self_batch, from_len, to_len, _heads, hd, !_predict, _stream,
+                                 self_riders ? &with_self : nullptr));
   LSH_CALL(layer_gemm_residual(_qin.get(), _wself_out.get(), tok, hs, _kh, _attn_ob_ptr, _attn_out_cmax_ptr,
                                dec_input_ptr, _encdec_inp.get(), _stream));
 
@@ -268,14 +274,15 @@ void TransformerDecoderLayer<T>::Forward(const T* dec_input_ptr, const T* enc_ou
   LSH_CALL(layer_norm_codes(x, _is_pre_ln ? nullptr : x, _qin.get(),
                             _is_pre_ln ? _encdec_attn_nw_ptr : _attn_nw_ptr,
                             _is_pre_ln ? _encdec_attn_nb_ptr : _attn_nb_ptr, _encdec_qkv_cmax_ptr, tok, hs,
-                            _kh, _stream));
+                            _kh, _stream, &with_norm));
   T* const cross[1] = {q};
   LSH_CALL(layer_gemm_heads(_qin.get(), _wq.get(), tok, 1, hs, _kh, _encdec_attn_qb_ptr,
                             _encdec_qkv_cmax_ptr, nullptr, _trg_seq_len, _heads, cross, &_trg_seq_len, at,
                             _stream));
   const T* k = kv + (size_t)_layer_id * 2 * src_dim;
   LSH_CALL(layer_attention_codes(q, k, k + src_dim, mask, _qin.get(), _encdec_out_cmax_ptr, _kh, _batch_size,
-                                 _trg_seq_len, _src_seq_len, _heads, hd, false, _stream));
+                                 _trg_seq_len, _src_seq_len, _heads, hd, false, _stream,
+                                 cross_riders ? &with_cross : nullptr));
   LSH_CALL(layer_gemm_residual(_qin.get(), _wcross_out.get(), tok, hs, _kh, _encdec_attn_ob_ptr,
                                _encdec_out_cmax_ptr, x, _ffn_inp.get(), _stream));
 
@@ -284,7 +291,7 @@ void TransformerDecoderLayer<T>::Forward(const T* dec_input_ptr, const T* enc_ou
   LSH_CALL(layer_norm_codes(x, _is_pre_ln ? nullptr : x, _qin.get(),
                             _is_pre_ln ? _ffn_nw_ptr : _encdec_attn_nw_ptr,
                             _is_pre_ln ? _ffn_nb_ptr : _encdec_attn_nb_ptr, _inter_cmax_ptr, tok, hs, _kh,
-                            _stream));
+                            _stream, &with_norm2));
   LSH_CALL(layer_gemm_act(_qin.get(), _winter.get(), tok, ims, _kh, _inter_b_ptr, _inter_cmax_ptr,
                           _output_cmax_ptr, relu, _act.get(), _ki, _stream));
   LSH_CALL(layer_gemm_ffn2(_act.get(), _woutput.get(), tok, hs, _ki, _output_b_ptr, x, dec_output_ptr,

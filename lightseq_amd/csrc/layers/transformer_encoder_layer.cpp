@@ -128,11 +128,14 @@ void TransformerEncoderLayer<T>::Forward(const T* input_ptr, const void* input_m
   const int tok = _batch_tokens, hs = _hidden_size, ims = _intermediate_size, hd = hs / _heads;
   const bool relu = _activation_fn == "relu";
 
-  LayerPrep prep;
+  // what the first product reads, and what rides in later launches ahead of its reader
+  LayerPrep prep, with_attn, with_norm;
+  const bool riders = layer_attention_takes_riders(_seq_len, _seq_len, (long)_batch_size * _heads, hd);
+  LayerPrep& later = riders ? with_attn : prep;
   LSH_CALL(prep.codes(_attn_qkvw_ptr, _wqkv.get(), _attn_qkv_cmax_ptr + 1, 3 * hs, hs, _kh));
-  LSH_CALL(prep.codes(_attn_ow_ptr, _wout.get(), _attn_out_cmax_ptr + 1, hs, hs, _kh));
-  LSH_CALL(prep.codes(_inter_w_ptr, _winter.get(), _inter_cmax_ptr + 1, ims, hs, _kh));
-  LSH_CALL(prep.halfs(_output_w_ptr, _woutput.get(), _output_cmax_ptr + 1, hs, ims, _ki, 1, ims, 0));
+  LSH_CALL(later.codes(_attn_ow_ptr, _wout.get(), _attn_out_cmax_ptr + 1, hs, hs, _kh));
+  LSH_CALL(later.codes(_inter_w_ptr, _winter.get(), _inter_cmax_ptr + 1, ims, hs, _kh));
+  LSH_CALL(with_norm.halfs(_output_w_ptr, _woutput.get(), _output_cmax_ptr + 1, hs, ims, _ki, 1, ims, 0));
   if (_is_pre_ln)
     LSH_CALL(prep.norm(input_ptr, _qin.get(), _attn_nw_ptr, _attn_nb_ptr, _attn_qkv_cmax_ptr, tok, hs, _kh));
   else
@@ -152,7 +155,8 @@ void TransformerEncoderLayer<T>::Forward(const T* input_ptr, const void* input_m
                             _mask_future_tokens ? _attn_qkv_cache_cmax_ptr : nullptr, _seq_len, _heads,
                             heads, len, at, _stream));
   LSH_CALL(layer_attention_codes(heads[0], heads[1], heads[2], mask, _qin.get(), _attn_out_cmax_ptr, _kh,
-                                 _batch_size, _seq_len, _seq_len, _heads, hd, _mask_future_tokens, _stream));
+                                 _batch_size, _seq_len, _seq_len, _heads, hd, _mask_future_tokens, _stream,
+                                 riders ? &with_attn : nullptr));
   LSH_CALL(layer_gemm_residual(_qin.get(), _wout.get(), tok, hs, _kh, _attn_ob_ptr, _attn_out_cmax_ptr,
                                input_ptr, _ffn_inp.get(), _stream));
 
@@ -160,7 +164,7 @@ void TransformerEncoderLayer<T>::Forward(const T* input_ptr, const void* input_m
   // The norm between the halves closes the first (post) or opens the second (pre).
   LSH_CALL(layer_norm_codes(_ffn_inp.get(), _is_pre_ln ? nullptr : _ffn_inp.get(), _qin.get(),
                             _is_pre_ln ? _ffn_nw_ptr : _attn_nw_ptr, _is_pre_ln ? _ffn_nb_ptr : _attn_nb_ptr,
-                            _inter_cmax_ptr, tok, hs, _kh, _stream));
+                            _inter_cmax_ptr, tok, hs, _kh, _stream, &with_norm));
   LSH_CALL(layer_gemm_act(_qin.get(), _winter.get(), tok, ims, _kh, _inter_b_ptr, _inter_cmax_ptr,
                           _output_cmax_ptr, relu, _act.get(), _ki, _stream));
   LSH_CALL(layer_gemm_ffn2(_act.get(), _woutput.get(), tok, hs, _ki, _output_b_ptr, _ffn_inp.get(), out_ptr,

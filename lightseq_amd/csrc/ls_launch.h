@@ -679,6 +679,12 @@ struct LayerPrepArgs {
   int n;
   LayerPrepSection s[kLayerPrepMost];
 };
+// a few matrices of it as spare workgroups (256 threads, or four times as many wavefronts) of another launch
+constexpr int kLayerRideMost = 3;
+struct LayerRide {
+  int blocks, first[kLayerRideMost];
+  LayerPrepSection s[kLayerRideMost];
+};
 // Everything a layer's forward pass starts from, collected and done in one launch.
 class LayerPrep {
  public:
@@ -695,6 +701,7 @@ class LayerPrep {
   // rows of K elements to the beginning of rows of dst_stride elements
   int grow(const __half* src, __half* dst, int rows, int K, long dst_stride);
   int launch(hipStream_t s) const;
+  int ride(LayerRide* out) const;
 
  private:
   int add(const LayerPrepSection& s);
@@ -702,10 +709,14 @@ class LayerPrep {
 };
 // layer norm of fp16 rows to fp16 (out may be inp, or null) and / or to blocked codes
 int layer_norm_codes(const __half* inp, __half* out, int8_t* codes, const __half* gamma, const __half* beta,
-                     const __half* cmax, int rows, int hidden, int k_pad, hipStream_t s);
+                     const __half* cmax, int rows, int hidden, int k_pad, hipStream_t s,
+                     const LayerPrep* also = nullptr);
 // the layers' attention, its context as blocked codes [batch * seq_len, k_pad] (cmax: device scalar)
 int layer_attention_codes(const __half* q, const __half* k, const __half* v, const __half* add_mask,
                           int8_t* codes, const __half* cmax, int k_pad, int batch, int seq_len, int key_len,
-                          int head_num, int dim_per_head, bool mask_future, hipStream_t s);
+                          int head_num, int dim_per_head, bool mask_future, hipStream_t s,
+                          const LayerPrep* also = nullptr);
+// whether matrices can ride in that launch (`also`)
+bool layer_attention_takes_riders(int seq_len, int key_len, long batch_heads, int dim_per_head);
 
 }  // namespace lsh
