@@ -674,11 +674,6 @@ struct LayerPrepSection {
   int rows, K, k_pad, n1;
   long stride0, stride1;
 };
-struct LayerPrepArgs {
-  int first[kLayerPrepMost];  // first workgroup of each section
-  int n;
-  LayerPrepSection s[kLayerPrepMost];
-};
 // a few matrices of it as spare workgroups (256 threads, or four times as many wavefronts) of another launch
 constexpr int kLayerRideMost = 3;
 struct LayerRide {
@@ -705,7 +700,8 @@ class LayerPrep {
 
  private:
   int add(const LayerPrepSection& s);
-  LayerPrepArgs _args{};
+  int _n = 0;
+  LayerPrepSection _s[kLayerPrepMost];
 };
 // layer norm of fp16 rows to fp16 (out may be inp, or null) and / or to blocked codes
 int layer_norm_codes(const __half* inp, __half* out, int8_t* codes, const __half* gamma, const __half* beta,

@@ -229,7 +229,9 @@ def ptr(x):
 
 
 def current_stream():
-    return torch.cuda.current_stream().cuda_stream
+    """Handle of torch's current stream on the current device (as torch.cuda.current_stream() gives it,
+    without the 3 us that its Stream object takes: a fourth of what a layer call costs Python)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def call(name, *args):
