@@ -336,16 +336,17 @@ __device__ __forceinline__ void decself_attend_row_once_body(uint4 qv, const uin
       *reinterpret_cast<float4*>(p + k) = make_float4(acc[k], acc[k + 1], acc[k + 2], acc[k + 3]);
   }
   __syncthreads();
-  const int tid = wid * 64 + lane;
-  if (tid < D) {
+  // (a group of one wavefront has more dimensions of a 128-wide head than lanes)
+#pragma unroll
+  for (int dim = wid * 64 + lane; dim < D; dim += 64 * NWV) {
     float t[4 * NWV];  // pairwise tree over the partial sums
 #pragma unroll
-    for (int i = 0; i < 4 * NWV; ++i) t[i] = part[i * D + tid];
+    for (int i = 0; i < 4 * NWV; ++i) t[i] = part[i * D + dim];
 #pragma unroll
     for (int st = 1; st < 4 * NWV; st *= 2)
 #pragma unroll
       for (int i = 0; i < 4 * NWV; i += 2 * st) t[i] += t[i + st];
-    if (live) out[(tid >> 4) * out_chunk + (tid & 15)] = (int8_t)float2int8(t[0], quant_scale);
+    if (live) out[(dim >> 4) * out_chunk + (dim & 15)] = (int8_t)float2int8(t[0], quant_scale);
   }
 }
 
