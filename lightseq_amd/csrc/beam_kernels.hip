@@ -860,22 +860,41 @@ beam_topk_part_kernel(const int8_t* __restrict__ logits, long ldl, const T* __re
 // and applies ker_refresh_result to them (inference/kernels/transformerKernels.cc.cu:
 // 1398-1463): new sequences, summed log-probabilities of live beams, scores of
 // finished ones, the finished count (added to *num_finished, which the top-k kernel ahead of
-// it cleared), plus the parent table for the cache reorder.
+// it cleared), plus the parent table for the cache reorder, or (beam_from) the table that stands in
+// its place: a beam inherits its parent's entries for the steps so far, and the parent itself is
+// the entry of this one.  The reorder of 64 rows x 16 heads x 64 steps of 6 layers takes 19 us of a
+// 260 us step, the table a few bytes of this launch.
 __global__ void __launch_bounds__(64)
 beam_merge_kernel(const float* __restrict__ top_score, const int* __restrict__ top_idx,
                   const int* __restrict__ old_alive_seq, int* __restrict__ new_alive_seq,
                   float* __restrict__ seq_probs, float* __restrict__ seq_score,
                   int* __restrict__ parent, int* __restrict__ num_finished, int batch,
                   int beam_size, int vocab, int max_step, int cur_step, float length_norm,
-                  int end_id, int parts) {
+                  int end_id, int parts, const int8_t* __restrict__ beam_from,
+                  int8_t* __restrict__ new_beam_from, int beam_stride) {
 #pragma clang fp contract(off)
   // grid: a workgroup of one wavefront per sentence (16 sentences as the 16 wavefronts of one
   // workgroup took turns on one compute unit's SIMDs: four times the time per instruction)
   __shared__ int seq_lds[1][512];  // the sentence's old sequences (beam_size * max_step <= 512)
+  __shared__ int from_lds[128];    // ... and its rows of the beam table, where the sequences fit
   const int lane = threadIdx.x & 63, wid = 0;
   const int nw = gridDim.x;
   const int ncand = beam_size * beam_size * parts;  // proposals of a sentence
   int finished = 0;
+  // row j of the new beam table from row `par` of the old one, four steps a lane
+  auto inherit = [&](const int* old_words, int b, int j, int par) {
+    int* to = reinterpret_cast<int*>(new_beam_from + ((long)b * beam_size + j) * beam_stride);
+    for (int w = lane; 4 * w <= cur_step; w += 64) {
+      const int old = old_words[w];
+      unsigned o = 0;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int from = 4 * w + k == cur_step ? 0 : unpack_i8((uint32_t)old, k);
+        o |= (unsigned)((from + par - j) & 255) << (8 * k);
+      }
+      to[w] = (int)o;
+    }
+  };
   // applies one pick (ker_refresh_result): the new sequence, then probability or score
   auto apply = [&](int b, int j, float score, int idx) {
     // a sentence always has at least beam_size proposals; guard the indices anyway
@@ -887,6 +906,10 @@ beam_merge_kernel(const float* __restrict__ top_score, const int* __restrict__ t
     int* to = new_alive_seq + ((long)b * beam_size + j) * max_step;
     for (int t = lane; t < max_step; t += 64)
       to[t] = t > cur_step + 1 ? end_id : (t == cur_step + 1 ? can_vocab : from[t]);
+    if (beam_from) {
+      const int par = can_vocab != end_id ? can_beam : j;  // a finished beam keeps what it has
+      inherit(reinterpret_cast<const int*>(beam_from + ((long)b * beam_size + par) * beam_stride), b, j, par);
+    }
     if (lane == 0) {
       if (can_vocab != end_id) {
         seq_probs[b * beam_size + j] = (score - (float)b * kMinLogProb) / length_norm;
@@ -920,7 +943,14 @@ beam_merge_kernel(const float* __restrict__ top_score, const int* __restrict__ t
       const int* ci = top_idx + (long)b * ncand;
       // the sentence's old sequences are requested together with the proposals and parked in
       // LDS: the new sequences then cost no second trip to memory after the picks are known
-      int olds[8];
+      int olds[8], oldf[2];
+      const int from_words = beam_size * beam_stride / 4;
+      const bool from_staged = beam_from != nullptr && from_words <= 128;
+      const int* from_old = reinterpret_cast<const int*>(beam_from + (long)b * beam_size * beam_stride);
+      if (from_staged) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) oldf[u] = from_old[min(lane + 64 * u, from_words - 1)];
+      }
       if (staged) {
 #pragma unroll
         for (int u = 0; u < 8; ++u)
@@ -954,6 +984,12 @@ beam_merge_kernel(const float* __restrict__ top_score, const int* __restrict__ t
       if (staged) {
 #pragma unroll
         for (int u = 0; u < 8; ++u) seq_lds[wid][lane + 64 * u] = olds[u];
+      }
+      if (from_staged) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) from_lds[lane + 64 * u] = oldf[u];
+      }
+      if (staged || from_staged) {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -972,6 +1008,10 @@ beam_merge_kernel(const float* __restrict__ top_score, const int* __restrict__ t
         for (int t = lane; t < max_step; t += 64) {
           const int old = staged ? seq_lds[wid][can_beam * max_step + t] : from[t];
           to[t] = t > cur_step + 1 ? end_id : (t == cur_step + 1 ? can_vocab : old);
+        }
+        if (beam_from) {
+          const int par = can_vocab != end_id ? can_beam : j;
+          inherit((from_staged ? from_lds : from_old) + par * (beam_stride / 4), b, j, par);
         }
       }
       if (lane < beam_size) {
@@ -1037,7 +1077,8 @@ int beam_search_step_i8I(const int8_t* logits, const T* logit_bias, float* seq_p
                          float* top_score, int* top_idx, int* parent, int* num_finished,
                          float dequant_scale, int vocab_size, int max_step, float length_norm,
                          int cur_step, int batch_size, int beam_size, int end_id, hipStream_t s,
-                         float* part_ws, size_t part_ws_words, int logits_stride) {
+                         float* part_ws, size_t part_ws_words, int logits_stride,
+                         const int8_t* beam_from, int8_t* new_beam_from, int beam_stride) {
   if (!logits || !logit_bias || !seq_probs || !seq_score || !old_alive_seq || !new_alive_seq ||
       !top_score || !top_idx || !parent || !num_finished || vocab_size <= 0 || batch_size <= 0 ||
       max_step <= 0 || cur_step < 0 || cur_step + 1 >= max_step)
@@ -1046,6 +1087,10 @@ int beam_search_step_i8I(const int8_t* logits, const T* logit_bias, float* seq_p
     return lsh_fail(LSH_ERR_INVALID, "wrong beam_size, should be 1, 2, 4, 8, 16 or 32");
   if (old_alive_seq == new_alive_seq)
     return lsh_fail(LSH_ERR_INVALID, "beam_search_step: the sequence buffers must differ");
+  if ((beam_from != nullptr) != (new_beam_from != nullptr) ||
+      (beam_from && (beam_from == new_beam_from || beam_stride % 4 != 0 || beam_stride < max_step ||
+                     ((reinterpret_cast<uintptr_t>(beam_from) | reinterpret_cast<uintptr_t>(new_beam_from)) & 3u) != 0)))
+    return lsh_fail(LSH_ERR_INVALID, "beam_search_step: bad beam tables");
   if ((long)beam_size * vocab_size > 0x7ffffffe)
     return lsh_fail(LSH_ERR_UNSUPPORTED, "beam_search_step: beam_size * vocab_size overflows");
   const long ldl = logits_stride ? logits_stride : vocab_size;
@@ -1084,15 +1129,17 @@ int beam_search_step_i8I(const int8_t* logits, const T* logit_bias, float* seq_p
   beam_merge_kernel<<<batch_size < 1024 ? batch_size : 1024, 64, 0, s>>>(top_score, top_idx, old_alive_seq, new_alive_seq,
                                        seq_probs, seq_score, parent, num_finished, batch_size,
                                        beam_size, vocab_size, max_step, cur_step, length_norm,
-                                       end_id, parts);
+                                       end_id, parts, beam_from, new_beam_from, beam_stride);
   return lsh_check_launch("beam_merge_kernel");
 }
 template int beam_search_step_i8I<float>(const int8_t*, const float*, float*, float*, const int*,
                                          int*, float*, int*, int*, int*, float, int, int, float,
-                                         int, int, int, int, hipStream_t, float*, size_t, int);
+                                         int, int, int, int, hipStream_t, float*, size_t, int,
+                                         const int8_t*, int8_t*, int);
 template int beam_search_step_i8I<__half>(const int8_t*, const __half*, float*, float*, const int*,
                                           int*, float*, int*, int*, int*, float, int, int, float,
-                                          int, int, int, int, hipStream_t, float*, size_t, int);
+                                          int, int, int, int, hipStream_t, float*, size_t, int,
+                                         const int8_t*, int8_t*, int);
 
 // ---------------------------------------------------------------------------------
 // The search step for callers that cannot allocate device memory (code under HIP graph

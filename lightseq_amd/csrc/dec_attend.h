@@ -48,16 +48,34 @@ __host__ __device__ constexpr long decself_group_floats(int step_num) {
   return rounds > one ? rounds : one;
 }
 
-// q: the D query codes; kb / vb: the pair's cache rows [max_step][D]; out: where the D context
+// Where step j of a pair's cache lies, in bytes from the pair's own rows [max_step][D]: in its place, or
+// (beam search without moving cache rows) in the rows of the beam of the same sentence that
+// computed it, `beam`[j] rows of the batch away; `last` is the step at hand, the pair's own.
+template <int D>
+struct RowsInPlace {
+  __device__ __forceinline__ long offset(int j) const { return (long)j * D; }
+};
+template <int D>
+struct RowsByBeam {
+  const int8_t* beam;
+  int last;
+  long row_bytes;  // of one row of the batch: heads * max_step * D
+  __device__ __forceinline__ long offset(int j) const {
+    const int b = beam[max(min(j, last - 1), 0)];
+    return (j < last ? b : 0) * row_bytes + (long)j * D;
+  }
+};
+
+// q: the D query codes; kb / vb: the pair's own cache rows; out: where the D context
 // codes go (nothing is stored unless `live`), 16 codes together and `out_chunk` bytes from one 16 to
 // the next (16: row-major, 256: a blocked matrix, see blocked_offset).  lds: decself_group_floats() floats of the group.
 // wid: wavefront within the group, lane: lane within the wavefront.
-template <int D, int NWV, int UN>
+template <int D, int NWV, int UN, typename Rows>
 __device__ __forceinline__ void decself_attend_row_rounds(const int8_t* q, const int8_t* kb,
-                                                          const int8_t* vb, int8_t* out, bool live,
-                                                   int out_chunk, int step_num, float attn_scale,
-                                                   float dq, float quant_scale, float* lds, int wid,
-                                                   int lane) {
+                                                          const int8_t* vb, const Rows& rows, int8_t* out,
+                                                          bool live, int out_chunk, int step_num,
+                                                          float attn_scale, float dq, float quant_scale,
+                                                          float* lds, int wid, int lane) {
 #pragma clang fp contract(off)
   constexpr int CH = D / 16;    // lanes per cache row
   constexpr int KPW = 64 / CH;  // rows per wavefront per load
@@ -82,7 +100,7 @@ __device__ __forceinline__ void decself_attend_row_rounds(const int8_t* q, const
     for (int u = 0; u < UN; ++u) {
       const int j = base + u * NWV * KPW + grp;
       // clamped instead of predicated: unconditional loads stay back to back
-      kv[u] = *reinterpret_cast<const uint4*>(kb + (long)min(j, step_num - 1) * D + c * 16);
+      kv[u] = *reinterpret_cast<const uint4*>(kb + rows.offset(min(j, step_num - 1)) + c * 16);
     }
     // The first round of value loads is requested right behind the first round of keys, before
     // any key is used: the two memory round trips of a short cache run side by side instead of
@@ -91,7 +109,7 @@ __device__ __forceinline__ void decself_attend_row_rounds(const int8_t* q, const
 #pragma unroll
       for (int u = 0; u < UN; ++u) {
         const int j = wid * KPW + u * NWV * KPW + grp;
-        vv0[u] = *reinterpret_cast<const uint4*>(vb + (long)min(j, step_num - 1) * D + c * 16);
+        vv0[u] = *reinterpret_cast<const uint4*>(vb + rows.offset(min(j, step_num - 1)) + c * 16);
       }
     }
 #pragma unroll
@@ -134,7 +152,7 @@ __device__ __forceinline__ void decself_attend_row_rounds(const int8_t* q, const
       if (base == wid * KPW)
         vv[u] = vv0[u];
       else
-        vv[u] = *reinterpret_cast<const uint4*>(vb + (long)min(j, step_num - 1) * D + c * 16);
+        vv[u] = *reinterpret_cast<const uint4*>(vb + rows.offset(min(j, step_num - 1)) + c * 16);
     }
 #pragma unroll
     for (int u = 0; u < UN; ++u) {
@@ -212,35 +230,35 @@ __device__ __forceinline__ void decself_attend_row_once_body(uint4 qv, const uin
 // The cache rows of a lane for the register-resident form: lane (grp, c) of wavefront wid holds
 // bytes [16 c, 16 c + 16) of rows (u NWV + wid) KPW + grp, u < UN (clamped to the last row,
 // not predicated: unconditional loads stay back to back).
-template <int D, int NWV, int UN>
-__device__ __forceinline__ void decself_attend_load_rows(const int8_t* kb, const int8_t* vb,
+template <int D, int NWV, int UN, typename Rows>
+__device__ __forceinline__ void decself_attend_load_rows(const int8_t* kb, const int8_t* vb, const Rows& rows,
                                                          int step_num, int wid, int lane,
                                                          uint4 (&kv)[UN], uint4 (&vv)[UN]) {
   constexpr int CH = D / 16, KPW = 64 / CH;
   const int c = lane % CH, grp = lane / CH;
+  long off[UN];
 #pragma unroll
   for (int u = 0; u < UN; ++u) {
     const int j = (u * NWV + wid) * KPW + grp;
-    kv[u] = *reinterpret_cast<const uint4*>(kb + (long)min(j, step_num - 1) * D + c * 16);
+    off[u] = rows.offset(min(j, step_num - 1)) + c * 16;
   }
 #pragma unroll
-  for (int u = 0; u < UN; ++u) {
-    const int j = (u * NWV + wid) * KPW + grp;
-    vv[u] = *reinterpret_cast<const uint4*>(vb + (long)min(j, step_num - 1) * D + c * 16);
-  }
+  for (int u = 0; u < UN; ++u) kv[u] = *reinterpret_cast<const uint4*>(kb + off[u]);
+#pragma unroll
+  for (int u = 0; u < UN; ++u) vv[u] = *reinterpret_cast<const uint4*>(vb + off[u]);
 }
 
-template <int D, int NWV, int UN>
+template <int D, int NWV, int UN, typename Rows>
 __device__ __forceinline__ void decself_attend_row_once(const int8_t* q, const int8_t* kb,
-                                                        const int8_t* vb, int8_t* out, bool live,
-                                                        int out_chunk, int step_num,
+                                                        const int8_t* vb, const Rows& rows, int8_t* out,
+                                                        bool live, int out_chunk, int step_num,
                                                         float attn_scale, float dq,
                                                         float quant_scale, float* lds, int wid,
                                                         int lane) {
   constexpr int CH = D / 16;
   const uint4 qv = *reinterpret_cast<const uint4*>(q + (lane % CH) * 16);
   uint4 kv[UN], vv[UN];
-  decself_attend_load_rows<D, NWV, UN>(kb, vb, step_num, wid, lane, kv, vv);
+  decself_attend_load_rows<D, NWV, UN>(kb, vb, rows, step_num, wid, lane, kv, vv);
   decself_attend_row_once_body<D, NWV, UN>(qv, kv, vv, out, live, out_chunk, step_num, attn_scale, dq,
                                            quant_scale, lds, wid, lane);
 }
@@ -352,17 +370,17 @@ __device__ __forceinline__ void decself_attend_row_once_body(uint4 qv, const uin
 
 // The group's attention: one round where the cache fits it, otherwise rounds through LDS.  The
 // choice follows the cache length only, so a row's result does not depend on its batch.
-template <int D, int NWV, int UN>
+template <int D, int NWV, int UN, typename Rows>
 __device__ __forceinline__ void decself_attend_row(const int8_t* q, const int8_t* kb,
-                                                   const int8_t* vb, int8_t* out, bool live,
+                                                   const int8_t* vb, const Rows& rows, int8_t* out, bool live,
                                                    int out_chunk, int step_num, float attn_scale,
                                                    float dq, float quant_scale, float* lds, int wid,
                                                    int lane) {
   if (step_num <= UN * NWV * (64 / (D / 16)))
-    decself_attend_row_once<D, NWV, UN>(q, kb, vb, out, live, out_chunk, step_num, attn_scale, dq,
+    decself_attend_row_once<D, NWV, UN>(q, kb, vb, rows, out, live, out_chunk, step_num, attn_scale, dq,
                                         quant_scale, lds, wid, lane);
   else
-    decself_attend_row_rounds<D, NWV, UN>(q, kb, vb, out, live, out_chunk, step_num, attn_scale, dq,
+    decself_attend_row_rounds<D, NWV, UN>(q, kb, vb, rows, out, live, out_chunk, step_num, attn_scale, dq,
                                           quant_scale, lds, wid, lane);
 }
 

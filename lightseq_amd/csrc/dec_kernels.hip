@@ -203,12 +203,22 @@ decself_attn_kernel(int32_t* __restrict__ scores, const int8_t* __restrict__ q,
 // across lanes (shuffles) and wavefronts (LDS): a tree instead of the ascending-step order
 // of the kernel above, so a context code can differ by one from it where the float sum
 // lands next to a rounding boundary.  Requires d in {32, 64, 128} and 16-byte aligned rows.
-template <int D, int NWV, int UN>
+// BY_BEAM: the steps of a row's cache lie where a beam table says (CacheBeams).
+template <int D, bool BY_BEAM>
+__device__ __forceinline__ auto cache_rows(const int8_t* beam_from, int beam_stride, long row, int step_num,
+                                           int head_num, int max_step) {
+  if constexpr (BY_BEAM)
+    return RowsByBeam<D>{beam_from + row * beam_stride, step_num - 1, (long)head_num * max_step * D};
+  else
+    return RowsInPlace<D>{};
+}
+
+template <int D, int NWV, int UN, bool BY_BEAM>
 __global__ void __launch_bounds__(64 * NWV)
 decself_attn_wg_kernel(const int8_t* __restrict__ q, const int8_t* __restrict__ k_cache,
-                       const int8_t* __restrict__ v_cache, int8_t* __restrict__ new_v,
-                       int step_num, int max_step, int head_num, float attn_scale, float dq,
-                       float quant_scale, int blocked) {
+                       const int8_t* __restrict__ v_cache, const int8_t* __restrict__ beam_from,
+                       int step_num, int max_step, int head_num, int beam_stride, int8_t* __restrict__ new_v,
+                       float attn_scale, float dq, float quant_scale, int blocked) {
   extern __shared__ __align__(16) float lds_f[];
   // grid: x = head, y = row (no division before the first load)
   const int head = (int)blockIdx.x;
@@ -216,6 +226,7 @@ decself_attn_wg_kernel(const int8_t* __restrict__ q, const int8_t* __restrict__ 
   const long bh = row * head_num + head;
   decself_attend_row<D, NWV, UN>(q + bh * D, k_cache + bh * (long)max_step * D,
                                  v_cache + bh * (long)max_step * D,
+                                 cache_rows<D, BY_BEAM>(beam_from, beam_stride, row, step_num, head_num, max_step),
                                  new_v + code_offset(row, head * D, head_num * D, blocked), true,
                                  blocked ? 256 : 16, step_num, attn_scale, dq, quant_scale, lds_f, threadIdx.x >> 6,
                                  threadIdx.x & 63);
@@ -224,12 +235,12 @@ decself_attn_wg_kernel(const int8_t* __restrict__ q, const int8_t* __restrict__ 
 // Short caches (one wavefront's loads cover them: at most 8 * 1024 / D steps): four (row, head)
 // pairs per workgroup, one wavefront each, so that a step's attention is one round of the
 // chip instead of four (1024 pairs at batch 16 x beam 4 x 16 heads).
-template <int D, int UN>
+template <int D, int UN, bool BY_BEAM>
 __global__ void __launch_bounds__(256)
 decself_attn_pack_kernel(const int8_t* __restrict__ q, const int8_t* __restrict__ k_cache,
-                         const int8_t* __restrict__ v_cache, int8_t* __restrict__ new_v,
-                         long bh_total, int step_num, int max_step, int head_num, float attn_scale,
-                         float dq, float quant_scale, int blocked) {
+                         const int8_t* __restrict__ v_cache, const int8_t* __restrict__ beam_from,
+                         long bh_total, int step_num, int max_step, int head_num, int beam_stride,
+                         int8_t* __restrict__ new_v, float attn_scale, float dq, float quant_scale, int blocked) {
   extern __shared__ __align__(16) float lds_f[];
   const int wave = threadIdx.x >> 6;
   const long bh_raw = (long)blockIdx.x * 4 + wave;
@@ -237,12 +248,12 @@ decself_attn_pack_kernel(const int8_t* __restrict__ q, const int8_t* __restrict_
   const long bh = live ? bh_raw : bh_total - 1;
   // new_v is [rows, heads * D]: row-major, a pair's D codes sit at bh * D of it
   long at = bh * D;
-  if (blocked) {
-    const int row = (int)(bh / head_num);
-    at = blocked_offset(row, ((int)bh - row * head_num) * D, head_num * D);
-  }
+  const int row = blocked || BY_BEAM ? (int)(bh / head_num) : 0;
+  if (blocked) at = blocked_offset(row, ((int)bh - row * head_num) * D, head_num * D);
   decself_attend_row_once<D, 1, UN>(q + bh * D, k_cache + bh * (long)max_step * D,
-                                    v_cache + bh * (long)max_step * D, new_v + at, live,
+                                    v_cache + bh * (long)max_step * D,
+                                    cache_rows<D, BY_BEAM>(beam_from, beam_stride, row, step_num, head_num, max_step),
+                                    new_v + at, live,
                                     blocked ? 256 : 16, step_num, attn_scale, dq, quant_scale,
                                     lds_f + wave * decself_group_floats<D, 1>(step_num), 0,
                                     threadIdx.x & 63);
@@ -286,9 +297,11 @@ int fuse_softmax_new_value_i32I_i8O(const int32_t* correlation, const int8_t* v,
 int decself_attention_i8(const int8_t* q, const int8_t* k_cache, const int8_t* v_cache,
                          int8_t* new_v, int batch_head_num, int step_num, int max_step,
                          int head_num, int dim_per_head, float attn_scale, float dequant_scale,
-                         float quant_scale, hipStream_t s, bool blocked) {
+                         float quant_scale, hipStream_t s, bool blocked, const CacheBeams* beams) {
   if (!q || !k_cache || !v_cache || !new_v)
     return lsh_fail(LSH_ERR_INVALID, "decself_attention: null pointer");
+  if (beams && (!beams->from || beams->stride < max_step))
+    return lsh_fail(LSH_ERR_INVALID, "decself_attention: bad beam table");
   if (blocked && (dim_per_head % 16 != 0 || head_num * dim_per_head % 64 != 0))
     return lsh_fail(LSH_ERR_UNSUPPORTED, "decself_attention: blocked output of this width");
   if (int rc = decself_check(batch_head_num, step_num, max_step, head_num, dim_per_head)) return rc;
@@ -304,34 +317,37 @@ int decself_attention_i8(const int8_t* q, const int8_t* k_cache, const int8_t* v
     // never fills are code to fetch and clamped loads to wait for.
     const bool wide = step_num > 256;
     const dim3 grid(head_num, batch_head_num / head_num);
+    const CacheBeams by = beams ? *beams : CacheBeams{};
     const int kpw = 1024 / dim_per_head;  // cached steps per load instruction of a wavefront
     if (step_num <= 8 * kpw) {
+#define LSH_DECSELF_PACK_RUN(D, UN, BY)                                                          \
+  decself_attn_pack_kernel<D, UN, BY>                                                            \
+      <<<(batch_head_num + 3) / 4, 256, 4 * decself_group_floats<D, 1>(step_num) * sizeof(float), \
+         s>>>(q, k_cache, v_cache, by.from, batch_head_num, step_num, max_step, head_num,        \
+              by.stride, new_v, attn_scale, dequant_scale, quant_scale, blocked)
 #define LSH_DECSELF_PACK(D)                                                                      \
-  if (step_num <= 4 * kpw)                                                                       \
-    decself_attn_pack_kernel<D, 4>                                                               \
-        <<<(batch_head_num + 3) / 4, 256, 4 * decself_group_floats<D, 1>(step_num) * sizeof(float), \
-           s>>>(q, k_cache, v_cache, new_v, batch_head_num, step_num, max_step, head_num,        \
-                attn_scale, dequant_scale, quant_scale, blocked);                                                     \
-  else                                                                                           \
-    decself_attn_pack_kernel<D, 8>                                                               \
-        <<<(batch_head_num + 3) / 4, 256, 4 * decself_group_floats<D, 1>(step_num) * sizeof(float), \
-           s>>>(q, k_cache, v_cache, new_v, batch_head_num, step_num, max_step, head_num,        \
-                attn_scale, dequant_scale, quant_scale, blocked)
+  if (step_num <= 4 * kpw && beams) LSH_DECSELF_PACK_RUN(D, 4, true);                            \
+  else if (step_num <= 4 * kpw) LSH_DECSELF_PACK_RUN(D, 4, false);                               \
+  else if (beams) LSH_DECSELF_PACK_RUN(D, 8, true);                                              \
+  else LSH_DECSELF_PACK_RUN(D, 8, false)
       if (dim_per_head == 32) { LSH_DECSELF_PACK(32); }
       else if (dim_per_head == 64) { LSH_DECSELF_PACK(64); }
       else { LSH_DECSELF_PACK(128); }
 #undef LSH_DECSELF_PACK
+#undef LSH_DECSELF_PACK_RUN
       return lsh_check_launch("decself_attn_pack_kernel");
     }
     // loads per lane of the 8-wavefront form: as many as the cache needs (a slot beyond the cache
     // is a clamped load and a dead row of arithmetic; the lanes' rows and the order of their
     // sums do not depend on it, so neither do the bits)
     const int un8 = (step_num + 8 * kpw - 1) / (8 * kpw);
+#define LSH_DECSELF_RUN(D, NWV, UN, BY)                                                         \
+  decself_attn_wg_kernel<D, NWV, UN, BY>                                                        \
+      <<<grid, 64 * NWV, decself_group_floats<D, NWV>(step_num) * sizeof(float), s>>>(          \
+          q, k_cache, v_cache, by.from, step_num, max_step, head_num, by.stride, new_v,         \
+          attn_scale, dequant_scale, quant_scale, blocked)
 #define LSH_DECSELF_WIDE(D, UN)                                                                 \
-  decself_attn_wg_kernel<D, 8, UN>                                                              \
-      <<<grid, 512, decself_group_floats<D, 8>(step_num) * sizeof(float), s>>>(                 \
-          q, k_cache, v_cache, new_v, step_num, max_step, head_num, attn_scale, dequant_scale,  \
-          quant_scale, blocked)
+  do { if (beams) LSH_DECSELF_RUN(D, 8, UN, true); else LSH_DECSELF_RUN(D, 8, UN, false); } while (0)
 #define LSH_DECSELF(D)                                                                          \
   if (wide) {                                                                                   \
     if (un8 <= 3) LSH_DECSELF_WIDE(D, 3);                                                       \
@@ -339,18 +355,19 @@ int decself_attention_i8(const int8_t* q, const int8_t* k_cache, const int8_t* v
     else if (un8 == 5) LSH_DECSELF_WIDE(D, 5);                                                  \
     else if (un8 == 6) LSH_DECSELF_WIDE(D, 6);                                                  \
     else LSH_DECSELF_WIDE(D, 8);                                                                \
-  } else /* 8192 / D < step_num <= 256 */                                                         \
-    decself_attn_wg_kernel<D, 4, 4>                                                             \
-        <<<grid, 256, decself_group_floats<D, 4>(step_num) * sizeof(float), s>>>(               \
-        q, k_cache, v_cache, new_v, step_num, max_step, head_num, attn_scale, dequant_scale,    \
-        quant_scale, blocked)
+  } else if (beams) /* 8192 / D < step_num <= 256 */                                            \
+    LSH_DECSELF_RUN(D, 4, 4, true);                                                             \
+  else                                                                                          \
+    LSH_DECSELF_RUN(D, 4, 4, false)
     if (dim_per_head == 32) { LSH_DECSELF(32); }
     else if (dim_per_head == 64) { LSH_DECSELF(64); }
     else { LSH_DECSELF(128); }
 #undef LSH_DECSELF
 #undef LSH_DECSELF_WIDE
+#undef LSH_DECSELF_RUN
     return lsh_check_launch("decself_attn_wg_kernel");
   }
+  if (beams) return lsh_fail(LSH_ERR_UNSUPPORTED, "decself_attention: beam table with this head size or alignment");
   decself_attn_kernel<2><<<(batch_head_num + 3) / 4, 256, decself_lds(step_num), s>>>(
       nullptr, q, k_cache, v_cache, new_v, batch_head_num, step_num, max_step, head_num,
       dim_per_head, attn_scale, dequant_scale, quant_scale, blocked);

@@ -138,7 +138,7 @@ decself_qkv_attn_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__
     const int row = min(row0 + g, rows - 1);
     const long bh = (long)row * head_num + head;
     decself_attend_row<D, NWV, UN>(new_q + bh * D, k_cache + bh * (long)max_step * D,
-                                   v_cache + bh * (long)max_step * D,
+                                   v_cache + bh * (long)max_step * D, RowsInPlace<D>{},
                                    ctx + code_offset(row, head * D, hidden, blocked_ctx), row0 + g < rows,
                                    blocked_ctx ? 256 : 16, step_num, attn_scale, cache_dequant_scale, ctx_quant_scale,
                                    lds_f + g * gfl, wid, lane);
@@ -184,7 +184,7 @@ decself_qkv_attn_early_kernel(const int8_t* __restrict__ x, const int8_t* __rest
 
   // ---- 0. the row's cache: requested before anything else ----
   uint4 kv[UN], vv[UN];
-  decself_attend_load_rows<D, NWV, UN>(kb, vb, step_num, wave, lane, kv, vv);
+  decself_attend_load_rows<D, NWV, UN>(kb, vb, RowsInPlace<D>{}, step_num, wave, lane, kv, vv);
   // (and the bias of the element this thread finishes in the epilogue)
   const __half bias_h = bias[(long)(min(tid, COLS - 1) >> 6) * hidden + head * D + (tid & 63)];
 

@@ -399,10 +399,19 @@ int fuse_softmax_new_value_i32I_i8O(const int32_t* correlation, const int8_t* v,
                                     int dim_per_head, float attn_scale, float dequant_scale,
                                     float quant_scale, hipStream_t s);
 // (blocked: the context codes are written as a blocked matrix)
+// Beam search without moving the rows of the caches: step t of the history of row r lies in the rows of
+// row r + from[r * stride + t], the row that computed it.  The search step keeps the table
+// (beam_search_step_i8I); the step at hand is always a row's own.
+struct CacheBeams {
+  const int8_t* from = nullptr;
+  int stride = 0;
+};
+// beams: heads of 32, 64 or 128 and 16-byte aligned operands only
 int decself_attention_i8(const int8_t* q, const int8_t* k_cache, const int8_t* v_cache,
                          int8_t* new_v, int batch_head_num, int step_num, int max_step,
                          int head_num, int dim_per_head, float attn_scale, float dequant_scale,
-                         float quant_scale, hipStream_t s, bool blocked = false);
+                         float quant_scale, hipStream_t s, bool blocked = false,
+                         const CacheBeams* beams = nullptr);
 template <typename T>
 int arrange_encdec_q_i8I(int step_token_num, int hidden_size, hipStream_t s, const int8_t* ori_q,
                          const T* q_bias, T* new_q, int beam_size, int dim_per_head, int head_num,
@@ -464,7 +473,11 @@ int beam_search_step_i8I(const int8_t* logits, const T* logit_bias, float* seq_p
                          float* top_score, int* top_idx, int* parent, int* num_finished,
                          float dequant_scale, int vocab_size, int max_step, float length_norm,
                          int cur_step, int batch_size, int beam_size, int end_id, hipStream_t s,
-                         float* part_ws = nullptr, size_t part_ws_words = 0, int logits_stride = 0);
+                         float* part_ws = nullptr, size_t part_ws_words = 0, int logits_stride = 0,
+                         const int8_t* beam_from = nullptr, int8_t* new_beam_from = nullptr,
+                         int beam_stride = 0);
+// (beam_from, new_beam_from: the CacheBeams table before and after the step, rows of beam_stride bytes,
+// a multiple of 4 and at least max_step)
 // 4-byte words of the optional workspace `part_ws` with which the per-row top-k of the step is
 // dealt to several workgroups per row (0: this shape runs one workgroup per row either way)
 size_t beam_search_step_workspace_words(int batch_size, int beam_size, int vocab_size);

@@ -104,6 +104,8 @@ void QuantDecoder::init_buffer() {
     _alive_seq[i].alloc(start_id_vec.size());
     _alive_seq[i].upload(start_id_vec.data(), start_id_vec.size(), _stream);
   }
+  _beam_stride = (_tw._max_step + 3) & ~3;
+  for (auto& b : _beam_from) b.alloc((size_t)rows * _beam_stride);
   _alive_seq_probs.alloc(rows);
   _alive_seq_score_own.alloc(rows);
   CHECK_GPU_ERROR(hipMemsetAsync(_alive_seq_score_own.get(), 0, rows * sizeof(float), _stream));
@@ -247,6 +249,9 @@ void QuantDecoder::run_one_infer(int batch_size, int batch_seq_len) {
   // steps go), so that a step's launches are the same from call to call
   _alive_cur = 0;
   _cache_cur = 0;
+  const int d = _tw._dim_per_head;
+  _by_beam = !_is_sampling && (d == 32 || d == 64 || d == 128) && _step_token_num <= 65535 && !step_taps.any() &&
+             !_rec_logits && !_rec_alive && !decself_qkv_attention_enabled();
 
   _phases.mark(0, _stream);
   project_encoder_output();
@@ -343,7 +348,7 @@ bool QuantDecoder::run_step() {
   // two sequence / cache buffers is current: one graph per such key.  A sampling step clears
   // its flag with a memset and runs eagerly.
   const uint64_t key = ((uint64_t)_batch_size << 40) | ((uint64_t)_batch_seq_len << 24) |
-                       ((uint64_t)_cur_step << 8) | (uint64_t)(_alive_cur << 1 | _cache_cur);
+                       ((uint64_t)_cur_step << 8) | (uint64_t)(_by_beam << 2 | _alive_cur << 1 | _cache_cur);
   _graphs.run(key, _stream,
               _use_graphs && !_is_sampling && !_rec_logits && !_rec_alive && !step_taps.any(),
               [&] {
@@ -361,7 +366,7 @@ void QuantDecoder::step_done(bool search) {
   ++_steps_run;
   if (!search) return;
   _alive_cur ^= 1;
-  if (_cur_step > 0) _cache_cur ^= 1;
+  if (_cur_step > 0 && !_by_beam) _cache_cur ^= 1;
 }
 
 // the one device-to-host word of a step: all beams finished -> stop early
@@ -384,7 +389,7 @@ void QuantDecoder::step_begin(StepNotice notice) {
   // The opt-in launch reads row-major operands.  With taps set the two launches run, so that q
   // and the caches are copied before the attention as the tap names promise; the bytes are the
   // same either way.
-  _qkv_attn = !step_taps.any() && decself_qkv_attention_enabled() && _tw._dim_per_head == 64 &&
+  _qkv_attn = !_by_beam && !step_taps.any() && decself_qkv_attention_enabled() && _tw._dim_per_head == 64 &&
               decself_qkv_attention_supported(_step_token_num, _tw._hidden_size, _tw._head_num,
                                               _tw._max_step);
   // few rows: the layer norms inside the stack are made by the products that read them; that in
@@ -500,9 +505,11 @@ void QuantDecoder::self_attention() {
     TAP("self_k_cache", k_cache, mh * _tw._max_step);
     TAP("self_v_cache", v_cache, mh * _tw._max_step);
     // int8 q.K -> softmax -> new value, one kernel
+    const CacheBeams beams{_beam_from[_alive_cur].get(), _beam_stride};
     LSH_CALL(decself_attention_i8(_buf_q.get(), k_cache, v_cache, _buf_b.get(), M * _tw._head_num,
                                   _cur_step + 1, _tw._max_step, _tw._head_num, _tw._dim_per_head,
-                                  attn_scale, c[18] / Q, Q / c[7], _stream, _ops.blocked));
+                                  attn_scale, c[18] / Q, Q / c[7], _stream, _ops.blocked,
+                                  _by_beam ? &beams : nullptr));
   }
   TAP_CODES("self_ctx_q", _buf_b.get(), H);
   _ops.i8o(_buf_b.get(), w.w_self_out.get(), _buf_a.get(), M, H, H, c[1] * c[7] / (c[13] * Q),
@@ -687,7 +694,9 @@ void QuantDecoder::beam_search() {
       alive_new, _top_score.get(), _top_idx.get(), _parent.get(), _num_finished.get(),
       _logits_clip_max / _quant_range, _tw._trg_vocab_size, _tw._max_step,
       _h_length_norm[_cur_step], _cur_step, _batch_size, _tw._beam_size, _tw._end_id, _stream,
-      _topk_part_ws.get(), _topk_part_ws.size(), _logits_stride));
+      _topk_part_ws.get(), _topk_part_ws.size(), _logits_stride,
+      _by_beam ? _beam_from[_alive_cur].get() : nullptr, _by_beam ? _beam_from[_alive_cur ^ 1].get() : nullptr,
+      _beam_stride));
   if (_rec_alive && _cur_step < _rec_max_steps)
     CHECK_GPU_ERROR(hipMemcpyAsync(
         _rec_alive + (size_t)_cur_step * _step_token_num * _tw._max_step, alive_new,
@@ -695,7 +704,7 @@ void QuantDecoder::beam_search() {
 
   /* ---refresh cache: k, v for decoder self attention--- (also on a step that turns out to be
    * the last one: the early-stop test reads the finished count after the step) */
-  if (_cur_step > 0) {
+  if (_cur_step > 0 && !_by_beam) {
     LSH_CALL(refresh_cache_by_parent_i8(
         _tw._n_dec_layer, _step_token_num, _stream, _parent.get(),
         _self_k_cache[_cache_cur].get(), _self_v_cache[_cache_cur].get(),

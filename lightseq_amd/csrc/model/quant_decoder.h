@@ -119,6 +119,12 @@ class QuantDecoder {
   int _cache_cur = 0;
   DeviceBuffer<int> _alive_seq[2];
   int _alive_cur = 0;
+  // Where the beams' cached steps lie (lsh::CacheBeams), double-buffered with the sequences.  With it
+  // the caches stay in the first buffers and no row of them is ever moved; runs that record
+  // or tap steps, other head sizes and the opt-in launch move rows, as the tap names promise.
+  DeviceBuffer<int8_t> _beam_from[2];
+  int _beam_stride = 0;
+  bool _by_beam = false;
   DeviceBuffer<float> _alive_seq_probs, _alive_seq_score_own, _top_score, _topk_part_ws;
   DeviceBuffer<int> _top_idx, _parent, _num_finished;
   DeviceBuffer<int> _sample_unfinished;           // the flag of a sampling step
