@@ -8,6 +8,7 @@
 // step is reproducible bit for bit.
 #include "dec_attend.h"
 #include "ln_step.h"
+#include "out_product.h"
 #include "ls_device.h"
 #include "ls_launch.h"
 
@@ -669,6 +670,8 @@ encdec_attn_vec_kernel(const __half* __restrict__ q, const __half* __restrict__ 
 // LN_ROWS > 0 (beam_size <= LN_ROWS): the product wavefronts also make the sentence's rows, by the
 // layer norm that precedes the product (ln_step.h; `x` is not read).  A workgroup normalises its
 // own sentence's beams only, so this holds for any batch; the launch it replaces took 3 us.
+// OUT (with LN_ROWS): the layer norm reads the sums of the self attention's out-projection, and all
+// eight wavefronts go on with that of this attention (out_product.h; ctx_q is not written).
 struct EncdecQProd {
   const int8_t* x;
   const int8_t* W;
@@ -676,9 +679,11 @@ struct EncdecQProd {
   int hidden;
   float alpha, dequant_scale;
   LnStep ln;
+  const int8_t* W_out;  // OUT only
+  int32_t *out_acc, *next_acc;
 };
 
-template <int D, int UN, bool QPROD = false, int LN_ROWS = 0>
+template <int D, int UN, bool QPROD = false, int LN_ROWS = 0, int OUT = 0>
 __global__ void __launch_bounds__(QPROD ? 512 : 256)
 encdec_attn_short_kernel(const __half* __restrict__ q, const __half* __restrict__ k,
                          const __half* __restrict__ v, const int* __restrict__ pad_mask, int beam_size,
@@ -692,9 +697,12 @@ encdec_attn_short_kernel(const __half* __restrict__ q, const __half* __restrict_
   __shared__ __align__(16) __half q_lds[QPROD ? 4 * D : 8];
   __shared__ __align__(16) int8_t codes[LN_ROWS ? 16 * 1024 : 16];
   __shared__ __align__(16) float red_ln[LN_ROWS ? 2 * LN_ROWS * 4 : 4];
+  __shared__ __align__(16) int8_t ctx_lds[OUT ? 4 * D : 16];
+  OutFragments<OUT ? OUT : 1> out_w;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   // grid: x = head, y = sentence, z = groups of 4 beams; wavefront = beam
-  const int head = (int)blockIdx.x, beam = (int)blockIdx.z * 4 + wid;
+  const int head = (int)blockIdx.x, beam = (OUT ? 0 : (int)blockIdx.z * 4) + wid;
+  const int out_first = ((int)blockIdx.z * 8 + __builtin_amdgcn_readfirstlane(wid)) * OUT;
   const long b = blockIdx.y;
   const bool alive = beam < beam_size;
   const int bm = alive ? beam : beam_size - 1;
@@ -723,7 +731,7 @@ encdec_attn_short_kernel(const __half* __restrict__ q, const __half* __restrict_
       const int8_t* wp = qp.W + code_offset((long)head * D + pw * 16 + m, kq * 16, qp.hidden, blocked);
       const int slice = blocked ? 1024 : 64;  // from one 64-byte slice of a row to the next
       const uint2 braw = *reinterpret_cast<const uint2*>(qp.bias + head * D + pw * 16 + 4 * kq);
-      LnStepRows<false, LN_ROWS ? LN_ROWS : 1> ln;
+      LnStepRows<OUT ? 1 : 0, LN_ROWS ? LN_ROWS : 1> ln;
       if constexpr (LN_ROWS) {
         ln.load(qp.ln, (int)threadIdx.x - 256, b * beam_size, beam_size, qp.hidden);
         __builtin_amdgcn_sched_barrier(0);
@@ -731,10 +739,11 @@ encdec_attn_short_kernel(const __half* __restrict__ q, const __half* __restrict_
       v4i xf[16], wf[16];
 #pragma unroll
       for (int sl = 0; sl < 16; ++sl) wf[sl] = *reinterpret_cast<const v4i*>(wp + min(sl, KS - 1) * slice);
+      if constexpr (OUT) out_w.request(qp.W_out, head, head_num, out_first, lane);
       if constexpr (LN_ROWS) {
         __builtin_amdgcn_sched_barrier(0);
         ln.finish(qp.ln, (int)threadIdx.x - 256, b * beam_size, beam_size, qp.hidden, codes, red_ln,
-                  head == 0);
+                  head == 0 && (!OUT || blockIdx.z == 0));
         __syncthreads();
         xp = codes + lane * 16;
       }
@@ -763,7 +772,15 @@ encdec_attn_short_kernel(const __half* __restrict__ q, const __half* __restrict_
       }
       __syncthreads();
       if constexpr (LN_ROWS)
-        if (head == 0) ln.store(qp.ln, (int)threadIdx.x - 256, b * beam_size, beam_size, qp.hidden);
+        if (head == 0 && (!OUT || blockIdx.z == 0)) ln.store(qp.ln, (int)threadIdx.x - 256, b * beam_size, beam_size, qp.hidden);
+      if constexpr (OUT) {
+        // the sentence's share of the next launch's sums: 64 columns
+        if (blockIdx.z == 0 && pw < beam_size)
+          qp.next_acc[(b * beam_size + pw) * qp.hidden + head * D + lane] = 0;
+        __syncthreads();
+        out_w.template add<4>(ctx_lds, qp.out_acc + b * beam_size * qp.hidden, beam_size, qp.hidden, out_first,
+                              lane);
+      }
       return;
     }
   }
@@ -780,6 +797,10 @@ encdec_attn_short_kernel(const __half* __restrict__ q, const __half* __restrict_
   for (int u = 0; u < UN; ++u) {
     const int j = min(u * KPW + grp, seq_len - 1);
     vv[u].u = *reinterpret_cast<const uint4*>(vb + (long)j * D);
+  }
+  if constexpr (OUT) {
+    __builtin_amdgcn_sched_barrier(0);
+    out_w.request(qp.W_out, head, head_num, out_first, lane);
   }
   if constexpr (LN_ROWS) {  // the layer norm's barriers
     __syncthreads();
@@ -847,6 +868,15 @@ encdec_attn_short_kernel(const __half* __restrict__ q, const __half* __restrict_
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  if constexpr (OUT) {
+    static_assert(D == 64, "a lane per dimension");
+    const float t = (part[lane] + part[D + lane]) + (part[2 * D + lane] + part[3 * D + lane]);
+    ctx_lds[wid * D + lane] = (int8_t)float2int8(TT<__half>::rnd(t), quant_scale);
+    __syncthreads();
+    out_w.template add<4>(ctx_lds, qp.out_acc + b * beam_size * qp.hidden, beam_size, qp.hidden, out_first,
+                          lane);
+    return;
+  }
   if (!alive) return;
   const long row = b * beam_size + beam;
   for (int dd = lane; dd < D; dd += 64) {
@@ -866,12 +896,16 @@ bool encdec_q_attention_supported(int beam_size, int head_num, int hidden, int b
          hidden <= 1024 && batch_seq_len >= 1 && batch_seq_len <= 16 * 8;
 }
 
+bool encdec_q_attention_out_supported(int batch_size, int head_num, int hidden) {
+  return hidden == head_num * 64 && hidden <= 1024 && hidden % 256 == 0 && batch_size * head_num <= cu_count();
+}
+
 int encdec_q_attention_f16(const int8_t* x, const int8_t* q_weight, const __half* q_bias,
                            const __half* k, const __half* v, const int* pad_mask, int8_t* ctx_q,
                            float quant_scale, int batch_size, int beam_size, int head_num,
                            int batch_seq_len, int hidden, float alpha, float dequant_scale,
-                           hipStream_t s, bool blocked, const LnStep* ln) {
-  if ((!x && !ln) || !q_weight || !q_bias || !k || !v || !pad_mask || !ctx_q || batch_size <= 0)
+                           hipStream_t s, bool blocked, const LnStep* ln, const OutSums* out) {
+  if ((!x && !ln) || !q_weight || !q_bias || !k || !v || !pad_mask || !(ctx_q || out) || batch_size <= 0)
     return lsh_fail(LSH_ERR_INVALID, "encdec_q_attention: bad arguments");
   if (!encdec_q_attention_supported(beam_size, head_num, hidden, batch_seq_len) ||
       batch_size > 65535 ||
@@ -882,34 +916,52 @@ int encdec_q_attention_f16(const int8_t* x, const int8_t* q_weight, const __half
                     "encdec_q_attention: needs heads of 64, hidden <= 1024, at most 4 beams, a "
                     "source of at most 128 tokens, 16-byte aligned operands");
   const long rows = (long)batch_size * beam_size;
-  if (!ln && x < ctx_q + rows * hidden && ctx_q < x + rows * hidden)
+  if (!ln && ctx_q && x < ctx_q + rows * hidden && ctx_q < x + rows * hidden)
     return lsh_fail(LSH_ERR_INVALID, "encdec_q_attention: ctx_q overlaps x");
   const float alpha_h = __half2float(__float2half_rn(sqrtf(1.f / 64.f)));
-  const dim3 grid(head_num, batch_size, 1);
+  const int share = out ? min(out_product_share(batch_size * head_num), 4) : 1;  // (8: see OutFragments)
+  const dim3 grid(head_num, batch_size, share);
   if (ln) {
     const uintptr_t all = reinterpret_cast<uintptr_t>(ln->acc) | reinterpret_cast<uintptr_t>(ln->res_in) |
                           reinterpret_cast<uintptr_t>(ln->res_out) | reinterpret_cast<uintptr_t>(ln->scale) |
                           reinterpret_cast<uintptr_t>(ln->bias) | reinterpret_cast<uintptr_t>(ln->res_bias) |
                           reinterpret_cast<uintptr_t>(ln->colsum);
-    if (!blocked || hidden % 256 != 0 || ln->planes != 0 || !ln->acc || !ln->res_in || !ln->res_out ||
+    if (!blocked || hidden % 256 != 0 || ln->planes != (out ? 1 : 0) ||
+        (ln->requant != 0.f) != (out != nullptr) || !ln->acc || !ln->res_in || !ln->res_out ||
         ln->res_in == ln->res_out || !ln->scale || !ln->bias || (all & 15u) != 0)
       return lsh_fail(LSH_ERR_UNSUPPORTED, "encdec_q_attention: layer norm not covered");
   }
-  const EncdecQProd qp{x, q_weight, q_bias, hidden, alpha, dequant_scale, ln ? *ln : LnStep{}};
+  if (out) {
+    if (!ln || !out->W || !out->acc || !out->next_acc || out->acc == out->next_acc || ln->acc == out->acc ||
+        ln->acc == out->next_acc || !encdec_q_attention_out_supported(batch_size, head_num, hidden) ||
+        ((reinterpret_cast<uintptr_t>(out->W) | reinterpret_cast<uintptr_t>(out->acc) |
+          reinterpret_cast<uintptr_t>(out->next_acc)) & 15u) != 0)
+      return lsh_fail(LSH_ERR_UNSUPPORTED, "encdec_q_attention: out-projection not covered");
+  }
+  const EncdecQProd qp{x, q_weight, q_bias, hidden, alpha, dequant_scale, ln ? *ln : LnStep{},
+                       out ? out->W : nullptr, out ? out->acc : nullptr, out ? out->next_acc : nullptr};
   const int un = (batch_seq_len + 7) / 8;
-#define LSH_ENCDEC_Q_LN(UN, LN)                                                              \
-  encdec_attn_short_kernel<64, UN, true, LN><<<grid, 512, 0, s>>>(                               \
+#define LSH_ENCDEC_Q_LN(UN, LN, OUT)                                                         \
+  encdec_attn_short_kernel<64, UN, true, LN, OUT><<<grid, 512, 0, s>>>(                          \
       nullptr, k, v, pad_mask, beam_size, head_num, batch_seq_len, alpha_h, nullptr, ctx_q,     \
       quant_scale, blocked, qp)
+#define LSH_ENCDEC_Q_ROWS(UN, OUT)                       \
+  do {                                                   \
+    if (beam_size == 1) LSH_ENCDEC_Q_LN(UN, 1, OUT);     \
+    else if (beam_size == 2) LSH_ENCDEC_Q_LN(UN, 2, OUT); \
+    else LSH_ENCDEC_Q_LN(UN, 4, OUT);                    \
+  } while (0)
 #define LSH_ENCDEC_Q(UN)                                 \
-  if (!ln) LSH_ENCDEC_Q_LN(UN, 0);                       \
-  else if (beam_size == 1) LSH_ENCDEC_Q_LN(UN, 1);       \
-  else if (beam_size == 2) LSH_ENCDEC_Q_LN(UN, 2);       \
-  else LSH_ENCDEC_Q_LN(UN, 4)
+  if (!ln) LSH_ENCDEC_Q_LN(UN, 0, 0);                    \
+  else if (!out) LSH_ENCDEC_Q_ROWS(UN, 0);               \
+  else if (share == 4) LSH_ENCDEC_Q_ROWS(UN, 2);         \
+  else if (share == 2) LSH_ENCDEC_Q_ROWS(UN, 4);         \
+  else LSH_ENCDEC_Q_ROWS(UN, 8)
   if (un <= 4) { LSH_ENCDEC_Q(4); }
   else if (un <= 8) { LSH_ENCDEC_Q(8); }
   else { LSH_ENCDEC_Q(16); }
 #undef LSH_ENCDEC_Q
+#undef LSH_ENCDEC_Q_ROWS
 #undef LSH_ENCDEC_Q_LN
   return lsh_check_launch("encdec_attn_short_kernel<q product>");
 }

@@ -15,7 +15,7 @@ namespace lsh {
 // a quarter of K per wavefront (D slices), its weights requested right behind the inputs of
 // the layer norm and in flight while it runs.  Everything after the codes is gemm_kw_kernel's.
 // us per generation step of a GPT-2 medium shape, batch 1: 573 -> 457.
-template <typename Epi, bool I32, int ROWS, int D>
+template <typename Epi, int PLANES, int ROWS, int D>
 __global__ void __launch_bounds__(256)
 ln_gemm_kernel(const int8_t* __restrict__ W, int M, int N, int K, const LnStep ln, Epi epi) {
   extern __shared__ __align__(16) int8_t smem[];
@@ -29,7 +29,7 @@ ln_gemm_kernel(const int8_t* __restrict__ W, int M, int N, int K, const LnStep l
   const int n0 = blockIdx.x * 16;
   // every argument in one batch of scalar loads
   asm volatile("" ::"s"(W), "s"(M), "s"(N), "s"(K), "s"(epi.alpha));
-  LnStepRows<I32, ROWS, D> rows;
+  LnStepRows<PLANES, ROWS, D> rows;
   rows.load(ln, tid, 0, M, K);
   __builtin_amdgcn_sched_barrier(0);
   const int8_t* wp = W + ((long)blockIdx.x * (K >> 6) + wave * D) * 1024 + lane * 16;
@@ -67,20 +67,20 @@ ln_gemm_kernel(const int8_t* __restrict__ W, int M, int N, int K, const LnStep l
 
 namespace {
 
-template <typename Epi, bool I32, int ROWS>
+template <typename Epi, int PLANES, int ROWS>
 int launch_ln_rows(const LnStep& ln, const int8_t* W, Epi epi, int M, int N, int K, hipStream_t s) {
   const dim3 grid((N + 15) / 16);
   const size_t smem = 16 * (size_t)K + 4 * 68 * 16 + (Epi::kTable ? 16 * 256 : 0);
   switch (K >> 8) {
-    case 1: return launch_blk<ln_gemm_kernel<Epi, I32, ROWS, 1>>(grid, 256, smem, s, W, M, N, K, ln, epi);
-    case 2: return launch_blk<ln_gemm_kernel<Epi, I32, ROWS, 2>>(grid, 256, smem, s, W, M, N, K, ln, epi);
-    case 3: return launch_blk<ln_gemm_kernel<Epi, I32, ROWS, 3>>(grid, 256, smem, s, W, M, N, K, ln, epi);
-    default: return launch_blk<ln_gemm_kernel<Epi, I32, ROWS, 4>>(grid, 256, smem, s, W, M, N, K, ln, epi);
+    case 1: return launch_blk<ln_gemm_kernel<Epi, PLANES, ROWS, 1>>(grid, 256, smem, s, W, M, N, K, ln, epi);
+    case 2: return launch_blk<ln_gemm_kernel<Epi, PLANES, ROWS, 2>>(grid, 256, smem, s, W, M, N, K, ln, epi);
+    case 3: return launch_blk<ln_gemm_kernel<Epi, PLANES, ROWS, 3>>(grid, 256, smem, s, W, M, N, K, ln, epi);
+    default: return launch_blk<ln_gemm_kernel<Epi, PLANES, ROWS, 4>>(grid, 256, smem, s, W, M, N, K, ln, epi);
   }
 }
-template <typename Epi, bool I32>
-int launch_ln_gemm(const LnStep& ln, const int8_t* W, Epi epi, int M, int N, int K, hipStream_t s) {
-  if (!ln_step_supported(M, K) || N % 4 != 0 || ln.planes > 4 || (ln.planes != 0) != I32)
+template <typename Epi, int PLANES>
+int launch_ln_planes(const LnStep& ln, const int8_t* W, Epi epi, int M, int N, int K, hipStream_t s) {
+  if (!ln_step_supported(M, K) || N % 4 != 0 || ln.planes > 4)
     return lsh_fail(LSH_ERR_UNSUPPORTED, "layer norm + product: shape not covered");
   if (!ln.acc || !ln.res_in || !ln.res_out || ln.res_in == ln.res_out || !ln.scale || !ln.bias || !W ||
       !epi.aligned())
@@ -91,9 +91,19 @@ int launch_ln_gemm(const LnStep& ln, const int8_t* W, Epi epi, int M, int N, int
                         reinterpret_cast<uintptr_t>(ln.colsum) | reinterpret_cast<uintptr_t>(W);
   if ((all & 15u) != 0 || ln.plane_stride % 4 != 0)
     return lsh_fail(LSH_ERR_INVALID, "layer norm + product: operands must be 16-byte aligned");
-  if (M == 1) return launch_ln_rows<Epi, I32, 1>(ln, W, epi, M, N, K, s);
-  if (M == 2) return launch_ln_rows<Epi, I32, 2>(ln, W, epi, M, N, K, s);
-  return launch_ln_rows<Epi, I32, 4>(ln, W, epi, M, N, K, s);
+  if (M == 1) return launch_ln_rows<Epi, PLANES, 1>(ln, W, epi, M, N, K, s);
+  if (M == 2) return launch_ln_rows<Epi, PLANES, 2>(ln, W, epi, M, N, K, s);
+  return launch_ln_rows<Epi, PLANES, 4>(ln, W, epi, M, N, K, s);
+}
+// FROM_FFN: behind a second feed-forward product, whose planes are sums; otherwise behind an
+// out-projection, which leaves codes or (with the attention, out_product.h) sums to requantise
+template <typename Epi, bool FROM_FFN>
+int launch_ln_gemm(const LnStep& ln, const int8_t* W, Epi epi, int M, int N, int K, hipStream_t s) {
+  if (FROM_FFN != (ln.planes != 0 && ln.requant == 0.f) || (ln.requant != 0.f && ln.planes != 1))
+    return lsh_fail(LSH_ERR_UNSUPPORTED, "layer norm + product: operand not covered");
+  if constexpr (FROM_FFN) return launch_ln_planes<Epi, 4>(ln, W, epi, M, N, K, s);
+  else if (ln.planes) return launch_ln_planes<Epi, 1>(ln, W, epi, M, N, K, s);
+  else return launch_ln_planes<Epi, 0>(ln, W, epi, M, N, K, s);
 }
 
 }  // namespace

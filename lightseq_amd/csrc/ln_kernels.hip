@@ -376,7 +376,8 @@ __global__ void __launch_bounds__(256)
 ln_row_wg_kernel(const AccT* __restrict__ gemm_out, T* residual, const T* __restrict__ scale,
                  const T* __restrict__ bias, const T* __restrict__ residual_bias,
                  const T* __restrict__ colsum, int hidden, int nparts, long part_stride, T* out_t,
-                 int8_t* __restrict__ out_q, float dequant_scale, float quant_scale, int is_post_ln, int blocked) {
+                 int8_t* __restrict__ out_q, float dequant_scale, float quant_scale, int is_post_ln, int blocked,
+                 float requant) {
   __shared__ float red[2][4];
   const int e0 = (int)threadIdx.x * 4;
   const bool on = e0 < hidden;
@@ -420,6 +421,10 @@ ln_row_wg_kernel(const AccT* __restrict__ gemm_out, T* residual, const T* __rest
         acc.x += t.x; acc.y += t.y; acc.z += t.z; acc.w += t.w;
       }
       a[0] = (float)acc.x; a[1] = (float)acc.y; a[2] = (float)acc.z; a[3] = (float)acc.w;
+      if (requant != 0.f) {  // (uniform)
+        a[0] = (float)requant_acc_fast(acc.x, requant); a[1] = (float)requant_acc_fast(acc.y, requant);
+        a[2] = (float)requant_acc_fast(acc.z, requant); a[3] = (float)requant_acc_fast(acc.w, requant);
+      }
     } else {
       ld4_acc(gemm_out, base + e, a);
       pin4(g_raw, b_raw, rb_raw, c_raw);
@@ -635,7 +640,7 @@ static int launch_ln(const AccT* gemm_out, T* residual, T* out_t, int8_t* out_q,
                      const T* bias, const T* residual_bias, const T* colsum, int tokens,
                      int hidden, float dequant_scale, float quant_scale, int is_post_ln,
                      hipStream_t stream, int nparts = 1, long part_stride = 0, bool blocked = false,
-                     const int* row_map = nullptr) {
+                     const int* row_map = nullptr, float requant = 0.f) {
   if (tokens <= 0 || hidden <= 0) return lsh_fail(LSH_ERR_INVALID, "layer norm: empty shape");
   if (nparts < 1 || (nparts > 1 && (sizeof(AccT) != 4 || part_stride % 4 != 0)))
     return lsh_fail(LSH_ERR_INVALID, "layer norm: bad accumulator planes");
@@ -651,9 +656,11 @@ static int launch_ln(const AccT* gemm_out, T* residual, T* out_t, int8_t* out_q,
     const int tpr = ((hidden / 4 + 63) / 64) * 64;  // threads of a row: whole wavefronts
     ln_row_wg_kernel<T, AccT, MODE><<<tokens, tpr, 0, stream>>>(
         gemm_out, residual, scale, bias, residual_bias, colsum, hidden, nparts, part_stride, out_t, out_q,
-        dequant_scale, quant_scale, is_post_ln, blk);
+        dequant_scale, quant_scale, is_post_ln, blk, requant);
     return lsh_check_launch("ln_row_wg_kernel");
   }
+  if (requant != 0.f)
+    return lsh_fail(LSH_ERR_UNSUPPORTED, "layer norm: sums to requantise go to the row kernel");
   if (vec_ok && hidden % 8 == 0) {
     // LPR = 64 when the row fills whole 512-element steps, otherwise two rows per wavefront
 #define LSH_LN8_RUN(LPR, IT, FULL)                                                               \
@@ -763,13 +770,15 @@ int residual_bias_ln_i8O(const AccT* input, const T* scale, const T* bias, const
                          int8_t* output, T* residual, int batch_tokens, int hidden_size,
                          float dequant_scale, float quant_scale, hipStream_t stream,
                          bool is_post_ln, const T* colsum, int nparts, long part_stride,
-                         bool blocked) {
+                         bool blocked, float requant) {
+  if (requant != 0.f && (sizeof(AccT) != 4 || nparts != 1))
+    return lsh_fail(LSH_ERR_INVALID, "ker_residual_bias_ln_*_i8O: only one plane of sums is requantised");
   if (!input || !output || !scale || !bias || !residual)
     return lsh_fail(LSH_ERR_INVALID, "ker_residual_bias_ln_*_i8O: null pointer");
   return launch_ln<T, AccT, kLnResQuant>(input, residual, nullptr, output, scale, bias,
                                          residual_bias, colsum, batch_tokens, hidden_size,
                                          dequant_scale, quant_scale, is_post_ln, stream, nparts,
-                                         part_stride, blocked);
+                                         part_stride, blocked, nullptr, requant);
 }
 
 template <typename T>
@@ -791,10 +800,10 @@ int residual_bias_ln_i32I(const int32_t* input, const T* scale, const T* bias, c
                                         const T*, float, bool, bool);                            \
   template int residual_bias_ln_i8O<T, int8_t>(const int8_t*, const T*, const T*, const T*,      \
                                                int8_t*, T*, int, int, float, float, hipStream_t, \
-                                               bool, const T*, int, long, bool);                 \
+                                               bool, const T*, int, long, bool, float);          \
   template int residual_bias_ln_i8O<T, int32_t>(const int32_t*, const T*, const T*, const T*,    \
                                                 int8_t*, T*, int, int, float, float,             \
-                                                hipStream_t, bool, const T*, int, long, bool);   \
+                                                hipStream_t, bool, const T*, int, long, bool, float); \
   template int residual_bias_ln_i32I<T>(const int32_t*, const T*, const T*, const T*, T*, int,   \
                                         int, float, hipStream_t, const T*, int, long, const int*);
 LSH_INST(float)

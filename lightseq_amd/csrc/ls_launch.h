@@ -94,7 +94,8 @@ int residual_bias_ln_i8O(const AccT* input, const T* scale, const T* bias, const
                          int8_t* output, T* residual, int batch_tokens, int hidden_size,
                          float dequant_scale, float quant_scale, hipStream_t stream,
                          bool is_post_ln, const T* colsum, int nparts = 1, long part_stride = 0,
-                         bool blocked = false);
+                         bool blocked = false, float requant = 0.f);
+// (requant != 0: int32 sums that become the int8 codes of that scale first; row kernel only)
 // row_map (optional): row r of output is made from row row_map[r] of input and residual
 template <typename T>
 int residual_bias_ln_i32I(const int32_t* input, const T* scale, const T* bias, const T* residual,
@@ -305,7 +306,9 @@ int gemm_blk_preferred_ksplit(int M, int N, int K);
 // reads its codes instead of a launch of its own (ln_step.h): the same codes and the same
 // residual stream, which goes to another buffer because other workgroups still read res_in.
 struct LnStep {
-  const void* acc;    // planes == 0: int8 [rows, hidden]; else int32 planes of [rows, hidden]
+  // planes == 0: int8 [rows, hidden]; else int32 planes of [rows, hidden]; requant != 0: one plane of sums
+  // that are requantised first, to the codes the product's epilogue would have left
+  const void* acc;
   int planes;         // at most 4
   long plane_stride;  // elements
   const __half* res_in;
@@ -313,6 +316,7 @@ struct LnStep {
   const __half *scale, *bias, *res_bias, *colsum;  // the last two may be null
   float dequant_scale, quant_scale;
   int is_post_ln;
+  float requant = 0.f;
 };
 // rows and widths for which a product takes an LnStep instead of A
 bool ln_step_supported(int rows, int hidden);
@@ -412,6 +416,15 @@ int decself_attention_i8(const int8_t* q, const int8_t* k_cache, const int8_t* v
                          int head_num, int dim_per_head, float attn_scale, float dequant_scale,
                          float quant_scale, hipStream_t s, bool blocked = false,
                          const CacheBeams* beams = nullptr);
+// The same attention with the out-projection that follows it: context codes times W (blocked [hidden,
+// hidden]) added to the int32 sums acc [rows, hidden], which start from zero; next_acc is cleared.
+// Heads of 64, at most 16 and an even number of them, caches of up to 1024 steps, as many (row,
+// head) pairs as one round of the chip takes.
+bool decself_attention_out_supported(int rows, int head_num, int dim_per_head, int step_num);
+int decself_attention_out_i8(const int8_t* q, const int8_t* k_cache, const int8_t* v_cache, const int8_t* W,
+                             int32_t* acc, int32_t* next_acc, int rows, int step_num, int max_step, int head_num,
+                             float attn_scale, float dequant_scale, float quant_scale, hipStream_t s,
+                             const CacheBeams* beams = nullptr);
 template <typename T>
 int arrange_encdec_q_i8I(int step_token_num, int hidden_size, hipStream_t s, const int8_t* ori_q,
                          const T* q_bias, T* new_q, int beam_size, int dim_per_head, int head_num,
@@ -429,12 +442,21 @@ int encdec_attention_f16(const __half* q, const __half* k, const __half* v, cons
                          hipStream_t s, bool blocked = false);
 // blocked: x, q_weight and ctx_q are blocked matrices; ln (with blocked, hidden % 256 == 0): the rows
 // are made by this layer norm, x is not read
+// out: ctx_q is not written; the context codes go through the out-projection behind (blocked W), its
+// int32 sums [rows, hidden] are added to acc, which starts from zero, and next_acc is cleared; the layer
+// norm then reads sums too (LnStep::requant).  Hidden a multiple of 256, one round of the chip.
+struct OutSums {
+  const int8_t* W;
+  int32_t *acc, *next_acc;
+};
+bool encdec_q_attention_out_supported(int batch_size, int head_num, int hidden);
 bool encdec_q_attention_supported(int beam_size, int head_num, int hidden, int batch_seq_len);
 int encdec_q_attention_f16(const int8_t* x, const int8_t* q_weight, const __half* q_bias,
                            const __half* k, const __half* v, const int* pad_mask, int8_t* ctx_q,
                            float quant_scale, int batch_size, int beam_size, int head_num,
                            int batch_seq_len, int hidden, float alpha, float dequant_scale,
-                           hipStream_t s, bool blocked = false, const LnStep* ln = nullptr);
+                           hipStream_t s, bool blocked = false, const LnStep* ln = nullptr,
+                           const OutSums* out = nullptr);
 
 // ---- beam search (beam_kernels.hip) -------------------------------------------------------
 template <typename T>

@@ -434,6 +434,28 @@ inline DeviceBuffer<int8_t> block_weight_padded(const DeviceBuffer<int8_t>& w, i
   return b;
 }
 
+// The int32 sums of the out-projections that attention launches add to: three buffers of [rows, hidden]
+// that take turns.  A launch adds to the current one and clears that of the launch behind it; a run
+// clears all three before its first step.  A step's first turn follows from its index alone, as a
+// graph replay needs.
+class OutSumsRing {
+ public:
+  void alloc(size_t most) { _buf.alloc(3 * most); }
+  void begin_run(size_t n, hipStream_t s) {
+    _n = n;
+    LSH_CALL(lsh::fill_i32(_buf.get(), 0, (int)(3 * n), s));
+  }
+  void begin_step(int launches_before) { _turn = launches_before % 3; }
+  int32_t* sums() const { return _buf.get() + (size_t)_turn * _n; }
+  int32_t* next_sums() const { return _buf.get() + (size_t)((_turn + 1) % 3) * _n; }
+  void launched() { _turn = (_turn + 1) % 3; }
+
+ private:
+  DeviceBuffer<int32_t> _buf;
+  size_t _n = 0;
+  int _turn = 0;
+};
+
 // The products of a layer stack whose int8 matrices are all blocked (hidden and inner size
 // multiples of 64) or all row-major.
 struct LayerProducts {

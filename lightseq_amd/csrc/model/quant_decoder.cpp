@@ -93,6 +93,7 @@ void QuantDecoder::init_buffer() {
   _logits.alloc(rows * (size_t)_logits_stride);
   // up to 8 accumulator planes of the split-K second FFN product
   _int32_ffn_out_buf.alloc(rows * H * 8);
+  _out_sums.alloc((size_t)rows * H);
   for (int i = 0; i < 2; ++i) {
     _self_k_cache[i].alloc((size_t)L * _layer_size_self_k);
     _self_v_cache[i].alloc((size_t)L * _layer_size_self_k);
@@ -252,6 +253,8 @@ void QuantDecoder::run_one_infer(int batch_size, int batch_seq_len) {
   const int d = _tw._dim_per_head;
   _by_beam = !_is_sampling && (d == 32 || d == 64 || d == 128) && _step_token_num <= 65535 && !step_taps.any() &&
              !_rec_logits && !_rec_alive && !decself_qkv_attention_enabled();
+  _out_run = out_run();
+  if (_out_run) _out_sums.begin_run((size_t)_step_token_num * _tw._hidden_size, _stream);
 
   _phases.mark(0, _stream);
   project_encoder_output();
@@ -344,11 +347,11 @@ void QuantDecoder::project_encoder_output() {
 
 bool QuantDecoder::run_step() {
   const bool search = step_runs_beam_search();
-  // The launches of a step depend on the shapes of the call, the step index and which of the
+  // The launches of a step depend on the shapes of the call, its routes, the step index and which of the
   // two sequence / cache buffers is current: one graph per such key.  A sampling step clears
   // its flag with a memset and runs eagerly.
   const uint64_t key = ((uint64_t)_batch_size << 40) | ((uint64_t)_batch_seq_len << 24) |
-                       ((uint64_t)_cur_step << 8) | (uint64_t)(_by_beam << 2 | _alive_cur << 1 | _cache_cur);
+                       ((uint64_t)_cur_step << 8) | (uint64_t)(_out_run << 3 | _by_beam << 2 | _alive_cur << 1 | _cache_cur);
   _graphs.run(key, _stream,
               _use_graphs && !_is_sampling && !_rec_logits && !_rec_alive && !step_taps.any(),
               [&] {
@@ -389,13 +392,16 @@ void QuantDecoder::step_begin(StepNotice notice) {
   // The opt-in launch reads row-major operands.  With taps set the two launches run, so that q
   // and the caches are copied before the attention as the tap names promise; the bytes are the
   // same either way.
-  _qkv_attn = !_by_beam && !step_taps.any() && decself_qkv_attention_enabled() && _tw._dim_per_head == 64 &&
+  _qkv_attn = !_by_beam && !_out_run && !step_taps.any() && decself_qkv_attention_enabled() && _tw._dim_per_head == 64 &&
               decself_qkv_attention_supported(_step_token_num, _tw._hidden_size, _tw._head_num,
                                               _tw._max_step);
   // few rows: the layer norms inside the stack are made by the products that read them; that in
   // front of the cross attention by its launch, whatever the number of rows
   _ln_in_product = !step_taps.any() && !_qkv_attn && _ops.ln_in_product(_step_token_num, _tw._hidden_size);
   _ln_in_encdec = !step_taps.any() && _ops.blocked && _tw._hidden_size % 256 == 0;
+  _out_step = _out_run && decself_attention_out_supported(_step_token_num, _tw._head_num, _tw._dim_per_head,
+                                                          _cur_step + 1);
+  _out_sums.begin_step(_cur_step * _tw._n_dec_layer * (encdec_out() ? 2 : 1));
   _res = 0;
   embedding(notice);
 }
@@ -506,26 +512,43 @@ void QuantDecoder::self_attention() {
     TAP("self_v_cache", v_cache, mh * _tw._max_step);
     // int8 q.K -> softmax -> new value, one kernel
     const CacheBeams beams{_beam_from[_alive_cur].get(), _beam_stride};
-    LSH_CALL(decself_attention_i8(_buf_q.get(), k_cache, v_cache, _buf_b.get(), M * _tw._head_num,
+    if (_out_step)  // ... with the out-projection behind it; the layer norm requantises its sums
+      LSH_CALL(decself_attention_out_i8(_buf_q.get(), k_cache, v_cache, w.w_self_out.get(), _out_sums.sums(),
+                                        _out_sums.next_sums(), M, _cur_step + 1, _tw._max_step, _tw._head_num,
+                                        attn_scale, c[18] / Q, Q / c[7], _stream, _by_beam ? &beams : nullptr));
+    else
+      LSH_CALL(decself_attention_i8(_buf_q.get(), k_cache, v_cache, _buf_b.get(), M * _tw._head_num,
                                   _cur_step + 1, _tw._max_step, _tw._head_num, _tw._dim_per_head,
                                   attn_scale, c[18] / Q, Q / c[7], _stream, _ops.blocked,
                                   _by_beam ? &beams : nullptr));
   }
-  TAP_CODES("self_ctx_q", _buf_b.get(), H);
-  _ops.i8o(_buf_b.get(), w.w_self_out.get(), _buf_a.get(), M, H, H, c[1] * c[7] / (c[13] * Q),
-           _stream);
-  TAP("self_out_q", _buf_a.get(), mh);
+  const float out_alpha = c[1] * c[7] / (c[13] * Q);
+  const int32_t* sums = _out_sums.sums();
+  if (_out_step) {
+    _out_sums.launched();
+  } else {
+    TAP_CODES("self_ctx_q", _buf_b.get(), H);
+    _ops.i8o(_buf_b.get(), w.w_self_out.get(), _buf_a.get(), M, H, H, out_alpha, _stream);
+    TAP("self_out_q", _buf_a.get(), mh);
+  }
   if (encdec_q_fused() ? _ln_in_encdec : _ln_in_product && _tw._dim_per_head % 16 == 0) {
     _ln = LnStep{_buf_a.get(), 0, 0, _cur_step_query[_res].get(), _cur_step_query[_res ^ 1].get(),
                  w.encdec_ln_scale.get(), w.encdec_ln_bias.get(), w.b_encdec_out.get(), nullptr,
                  c[13] / Q, Q / c[8], _tw._is_post_ln};
+    if (_out_step) _ln.acc = sums, _ln.planes = 1, _ln.requant = out_alpha;
     _res ^= 1;
     return;
   }
-  LSH_CALL((residual_bias_ln_i8O<__half, int8_t>(
-      _buf_a.get(), w.encdec_ln_scale.get(), w.encdec_ln_bias.get(), w.b_encdec_out.get(),
-      _buf_b.get(), _cur_step_query[_res].get(), M, H, c[13] / Q, Q / c[8], _stream, _tw._is_post_ln,
-      nullptr, 1, 0, _ops.blocked)));
+  if (_out_step)
+    LSH_CALL((residual_bias_ln_i8O<__half, int32_t>(
+        sums, w.encdec_ln_scale.get(), w.encdec_ln_bias.get(), w.b_encdec_out.get(), _buf_b.get(),
+        _cur_step_query[_res].get(), M, H, c[13] / Q, Q / c[8], _stream, _tw._is_post_ln, nullptr, 1, 0,
+        _ops.blocked, out_alpha)));
+  else
+    LSH_CALL((residual_bias_ln_i8O<__half, int8_t>(
+        _buf_a.get(), w.encdec_ln_scale.get(), w.encdec_ln_bias.get(), w.b_encdec_out.get(),
+        _buf_b.get(), _cur_step_query[_res].get(), M, H, c[13] / Q, Q / c[8], _stream, _tw._is_post_ln,
+        nullptr, 1, 0, _ops.blocked)));
   TAP_CODES("encdec_ln_q", _buf_b.get(), H);
   TAP("res_self", _cur_step_query[_res].get(), mh * sizeof(__half));
 }
@@ -535,6 +558,31 @@ void QuantDecoder::self_attention() {
 bool QuantDecoder::encdec_q_fused() const {
   return !step_taps.any() && _tw._dim_per_head == 64 &&
          encdec_q_attention_supported(_tw._beam_size, _tw._head_num, _tw._hidden_size, _batch_seq_len);
+}
+
+// The cross attention's out-projection goes with the self attention's: the launch of short sources,
+// with the layer norm in it (so a run's steps have one launch with sums a layer, or two).
+bool QuantDecoder::encdec_out() const {
+  return _out_run && encdec_q_fused() &&
+         encdec_q_attention_out_supported(_batch_size, _tw._head_num, _tw._hidden_size);
+}
+
+// Decided once a run: a step that left the sums' turn out would leave the next one's buffer uncleared.
+// (A run whose caches outgrow the launch goes on without it: it never comes back.)
+bool QuantDecoder::out_run() const {
+  if (!_ops.blocked || _layers.empty() || step_taps.any() || decself_qkv_attention_enabled() ||
+      !decself_attention_out_supported(_step_token_num, _tw._head_num, _tw._dim_per_head, 1))
+    return false;
+  // the launch of a short source with the layer norm in it reads sums only with its own out-projection
+  if (encdec_q_fused() && _tw._hidden_size % 256 == 0 &&
+      !encdec_q_attention_out_supported(_batch_size, _tw._head_num, _tw._hidden_size))
+    return false;
+  for (int l = 0; l < _tw._n_dec_layer; ++l) {
+    const float* c = &_dec_clip_max[l * 19];
+    if (c[1] * c[7] / (c[13] * _quant_range) == 0.f || c[3] * c[9] / (c[15] * _quant_range) == 0.f)
+      return false;  // no code but zero: LnStep's "none"
+  }
+  return true;
 }
 
 void QuantDecoder::encdec_attention() {
@@ -548,14 +596,20 @@ void QuantDecoder::encdec_attention() {
     // the context goes to the second part of _buf_a because other workgroups still read the
     // rows (_buf_b, or the first part)
     int8_t* ctx_q = _buf_a.get() + _ops.rows(M) * H;
+    const bool out = _out_step && encdec_out();
+    const OutSums sums{w.w_encdec_out.get(), _out_sums.sums(), _out_sums.next_sums()};
     LSH_CALL(encdec_q_attention_f16(
         _buf_b.get(), w.w_encdec_q.get(), w.b_encdec_q.get(),
         _encdec_k.get() + (size_t)_layer_id * _layer_size_encdec_k,
         _encdec_v.get() + (size_t)_layer_id * _layer_size_encdec_k, _p_d_padding_mask, ctx_q,
         Q / c[9], _batch_size, _tw._beam_size, _tw._head_num, _batch_seq_len, H,
-        c[2] * c[8] / (c[14] * Q), c[14] / Q, _stream, _ops.blocked, _ln_in_encdec ? &_ln : nullptr));
-    _ops.i8o(ctx_q, w.w_encdec_out.get(), _buf_a.get(), M, H, H, c[3] * c[9] / (c[15] * Q), _stream);
-    encdec_norm();
+        c[2] * c[8] / (c[14] * Q), c[14] / Q, _stream, _ops.blocked, _ln_in_encdec ? &_ln : nullptr,
+        out ? &sums : nullptr));
+    if (out)
+      _out_sums.launched();
+    else
+      _ops.i8o(ctx_q, w.w_encdec_out.get(), _buf_a.get(), M, H, H, c[3] * c[9] / (c[15] * Q), _stream);
+    encdec_norm(out ? sums.acc : nullptr);
     return;
   }
   // q product; its epilogue is ker_arrange_encdec_q_i8I (fp16 q [batch, heads, beam, d])
@@ -584,27 +638,35 @@ void QuantDecoder::encdec_attention() {
   TAP_CODES("encdec_ctx_q", _buf_b.get(), H);
   _ops.i8o(_buf_b.get(), w.w_encdec_out.get(), _buf_a.get(), M, H, H, c[3] * c[9] / (c[15] * Q),
            _stream);
-  encdec_norm();
+  encdec_norm(nullptr);
 }
 
-// the layer norm behind the cross attention
-void QuantDecoder::encdec_norm() {
+// the layer norm behind the cross attention; sums: of the out-projection, codes in _buf_a otherwise
+void QuantDecoder::encdec_norm(const int32_t* sums) {
   const int H = _tw._hidden_size, M = _step_token_num;
   const Layer& w = _layers[_layer_id];
   const float* c = &_dec_clip_max[_layer_id * 19];
   const float Q = _quant_range;
-  TAP("encdec_out_q", _buf_a.get(), (size_t)M * H);
+  const float out_alpha = c[3] * c[9] / (c[15] * Q);
+  if (!sums) TAP("encdec_out_q", _buf_a.get(), (size_t)M * H);
   if (_ln_in_product) {
     _ln = LnStep{_buf_a.get(), 0, 0, _cur_step_query[_res].get(), _cur_step_query[_res ^ 1].get(),
                  w.ffn_ln_scale.get(), w.ffn_ln_bias.get(), w.b_ffn2.get(), nullptr, c[15] / Q,
                  Q / c[10], _tw._is_post_ln};
+    if (sums) _ln.acc = sums, _ln.planes = 1, _ln.requant = out_alpha;
     _res ^= 1;
     return;
   }
-  LSH_CALL((residual_bias_ln_i8O<__half, int8_t>(
-      _buf_a.get(), w.ffn_ln_scale.get(), w.ffn_ln_bias.get(), w.b_ffn2.get(), _buf_b.get(),
-      _cur_step_query[_res].get(), M, H, c[15] / Q, Q / c[10], _stream, _tw._is_post_ln, nullptr, 1, 0,
-      _ops.blocked)));
+  if (sums)
+    LSH_CALL((residual_bias_ln_i8O<__half, int32_t>(
+        sums, w.ffn_ln_scale.get(), w.ffn_ln_bias.get(), w.b_ffn2.get(), _buf_b.get(),
+        _cur_step_query[_res].get(), M, H, c[15] / Q, Q / c[10], _stream, _tw._is_post_ln, nullptr, 1, 0,
+        _ops.blocked, out_alpha)));
+  else
+    LSH_CALL((residual_bias_ln_i8O<__half, int8_t>(
+        _buf_a.get(), w.ffn_ln_scale.get(), w.ffn_ln_bias.get(), w.b_ffn2.get(), _buf_b.get(),
+        _cur_step_query[_res].get(), M, H, c[15] / Q, Q / c[10], _stream, _tw._is_post_ln, nullptr, 1, 0,
+        _ops.blocked)));
   TAP_CODES("ffn_ln_q", _buf_b.get(), H);
   TAP("res_encdec", _cur_step_query[_res].get(), (size_t)M * H * sizeof(__half));
 }

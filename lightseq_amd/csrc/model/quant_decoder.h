@@ -68,9 +68,11 @@ class QuantDecoder {
   void embedding(lsh::StepNotice notice);
   bool emb_ln_fused() const;
   void self_attention();
+  bool out_run() const;
+  bool encdec_out() const;
   bool encdec_q_fused() const;
   void encdec_attention();
-  void encdec_norm();
+  void encdec_norm(const int32_t* sums);
   void ffn_add_norm();
   void step_begin(lsh::StepNotice notice);
   void step_layers(int from, int to);
@@ -115,6 +117,9 @@ class QuantDecoder {
   DeviceBuffer<__half> _query_buf1;
   DeviceBuffer<int8_t> _buf_a, _buf_b, _buf_q, _logits;
   DeviceBuffer<int32_t> _int32_ffn_out_buf;
+  OutSumsRing _out_sums;
+  // this run's attention launches go through the out-projections while the cache length lets them
+  bool _out_run = false, _out_step = false;
   DeviceBuffer<int8_t> _self_k_cache[2], _self_v_cache[2];  // [n_layer][rows*max_step*H]
   int _cache_cur = 0;
   DeviceBuffer<int> _alive_seq[2];

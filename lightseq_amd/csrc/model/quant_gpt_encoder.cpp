@@ -82,6 +82,7 @@ void QuantGptEncoder::init_buffer() {
   _logits.alloc((_tw._sampling_method == "ppl" ? tokens : (size_t)_max_batch_size) * _logits_stride);
   // room for the accumulator planes of the split-K second FFN product
   _int32_ffn_out_buf.alloc(std::max(tokens * H * 4, (size_t)64 * H * 8));
+  _out_sums.alloc((size_t)_max_batch_size * H);
   _self_k_cache.alloc((size_t)L * _max_batch_dim);
   _self_v_cache.alloc((size_t)L * _max_batch_dim);
   CHECK_GPU_ERROR(hipMemsetAsync(_self_k_cache.get(), 0, _self_k_cache.size(), _stream));
@@ -291,12 +292,15 @@ void QuantGptEncoder::step_begin(StepNotice notice) {
   _step.b = _buf_b.get();
   _tap_step = _steps_run;
   // the opt-in launch of the QKV product and the attention reads row-major operands
-  _step.qkv_attn = !step_taps.any() && decself_qkv_attention_enabled() && _tw._dim_per_head == 64 &&
+  _step.qkv_attn = !_out_run && !step_taps.any() && decself_qkv_attention_enabled() && _tw._dim_per_head == 64 &&
                    decself_qkv_attention_supported(B, H, _tw._head_num, _tw._max_step);
   _step.ln1_blocked = _ops.blocked && !_step.qkv_attn;
   // few rows: the layer norms between two layers and between the two halves of a layer are made
   // by the products that read them
   _step.ln_in_product = !step_taps.any() && !_step.qkv_attn && _ops.ln_in_product(B, H);
+  _step.out_in_attention =
+      _out_run && decself_attention_out_supported(B, _tw._head_num, _tw._dim_per_head, _batch_seq_len);
+  _out_sums.begin_step(_batch_seq_len * _tw._n_enc_layer);
   _res = 0;
   if (emb_ln_fused()) {
     const Layer& w0 = _layers[0];
@@ -321,13 +325,26 @@ bool QuantGptEncoder::emb_ln_fused() const {
          _tw._n_enc_layer > 0;
 }
 
+// Decided once a run: a step that left the sums' turn out would leave the next one's buffer uncleared.
+// (A run whose caches outgrow the launch goes on without it: it never comes back.)
+bool QuantGptEncoder::out_run() const {
+  if (!_ops.blocked || step_taps.any() || decself_qkv_attention_enabled() ||
+      !decself_attention_out_supported(_batch_size, _tw._head_num, _tw._dim_per_head, _batch_seq_len + 1))
+    return false;
+  for (int l = 0; l < _tw._n_enc_layer; ++l) {
+    const float* c = &_enc_clip_max[l * 12];
+    if (c[1] * c[5] / (c[9] * _quant_range) == 0.f) return false;  // no code but zero: LnStep's "none"
+  }
+  return true;
+}
+
 void QuantGptEncoder::step_layers(int from, int to) {
   LnFewRowsScope few_rows;
   const int H = _tw._hidden_size, B = _batch_size;
   const float Q = _quant_range;
   int8_t *&a = _step.a, *&b = _step.b;
   const bool qkv_attn = _step.qkv_attn, ln1_blocked = _step.ln1_blocked,
-             ln_in_product = _step.ln_in_product;
+             ln_in_product = _step.ln_in_product, out = _step.out_in_attention;
   LnStep ln{}, &ln_next = _step.ln_next;
   const size_t bh = (size_t)B * H;
   for (_layer_id = from; _layer_id < to; _layer_id++) {
@@ -359,25 +376,43 @@ void QuantGptEncoder::step_layers(int from, int to) {
       TAP("self_q", _buf_q.get(), bh);
       TAP("k_cache", k_cache, bh * _tw._max_step);
       TAP("v_cache", v_cache, bh * _tw._max_step);
-      LSH_CALL(decself_attention_i8(_buf_q.get(), k_cache, v_cache, b, B * _tw._head_num,
-                                    _batch_seq_len, _tw._max_step, _tw._head_num,
-                                    _tw._dim_per_head, _atten_scaler, c[11] / Q, Q / c[5], _stream,
-                                    _ops.blocked));
+      if (!out)
+        LSH_CALL(decself_attention_i8(_buf_q.get(), k_cache, v_cache, b, B * _tw._head_num,
+                                      _batch_seq_len, _tw._max_step, _tw._head_num,
+                                      _tw._dim_per_head, _atten_scaler, c[11] / Q, Q / c[5], _stream,
+                                      _ops.blocked));
     }
-    TAP_CODES("ctx_q", b, B, H);
-    _ops.i8o(b, w.w_out.get(), a, B, H, H, c[1] * c[5] / (c[9] * Q), _stream);
-    TAP("out_q", a, bh);
+    const float out_alpha = c[1] * c[5] / (c[9] * Q);
+    const int32_t* sums = _out_sums.sums();
+    if (out) {
+      // the attention and the out-projection in one launch; the layer norm requantises its sums
+      LSH_CALL(decself_attention_out_i8(_buf_q.get(), k_cache, v_cache, w.w_out.get(), _out_sums.sums(),
+                                        _out_sums.next_sums(), B, _batch_seq_len, _tw._max_step, _tw._head_num,
+                                        _atten_scaler, c[11] / Q, Q / c[5], _stream));
+      _out_sums.launched();
+    } else {
+      TAP_CODES("ctx_q", b, B, H);
+      _ops.i8o(b, w.w_out.get(), a, B, H, H, out_alpha, _stream);
+      TAP("out_q", a, bh);
+    }
     if (ln_in_product) {
       ln = LnStep{a, 0, 0, _query[_res].get(), _query[_res ^ 1].get(), w.ln2_scale.get(),
                   w.ln2_bias.get(), w.b_ffn2.get(), nullptr, c[9] / Q, Q / c[6], 0};
+      if (out) ln.acc = sums, ln.planes = 1, ln.requant = out_alpha;
       _res ^= 1;
       ffn_add_norm(B, a, b, true, &ln, &ln_next);
       continue;
     }
-    LSH_CALL((residual_bias_ln_i8O<__half, int8_t>(a, w.ln2_scale.get(), w.ln2_bias.get(),
-                                                   w.b_ffn2.get(), b, _query[_res].get(), B, H,
-                                                   c[9] / Q, Q / c[6], _stream, false, nullptr, 1,
-                                                   0, _ops.blocked)));
+    if (out)
+      LSH_CALL((residual_bias_ln_i8O<__half, int32_t>(sums, w.ln2_scale.get(), w.ln2_bias.get(),
+                                                      w.b_ffn2.get(), b, _query[_res].get(), B, H,
+                                                      c[9] / Q, Q / c[6], _stream, false, nullptr, 1,
+                                                      0, _ops.blocked, out_alpha)));
+    else
+      LSH_CALL((residual_bias_ln_i8O<__half, int8_t>(a, w.ln2_scale.get(), w.ln2_bias.get(),
+                                                     w.b_ffn2.get(), b, _query[_res].get(), B, H,
+                                                     c[9] / Q, Q / c[6], _stream, false, nullptr, 1,
+                                                     0, _ops.blocked)));
     TAP_CODES("ln2_q", b, B, H);
     TAP("res_attn", _query[_res].get(), bh * sizeof(__half));
     ffn_add_norm(B, b, a, _layer_id == _tw._n_enc_layer - 1 ? _ops.blocked : ln1_blocked, nullptr,
@@ -454,6 +489,7 @@ int QuantGptEncoder::run_one_sample(int batch_size, int batch_seq_len) {
   _batch_max_seq_len = std::min(_tw._max_step, batch_seq_len + _tw._extra_decode_length);
   _steps_run = 0;
   const int H = _tw._hidden_size;
+  _out_run = out_run();
 
   _phases.mark(0, _stream);
   // ids [batch, max_step] <- prompt
@@ -474,6 +510,7 @@ int QuantGptEncoder::run_one_sample(int batch_size, int batch_seq_len) {
     enqueue_sampling(_hid_last[_ops.blocked].get(), true);
     count_token();
     const int L = _tw._n_enc_layer;
+    if (_out_run) _out_sums.begin_run((size_t)batch_size * H, _stream);
     if (!_is_benchmark && !_use_graphs && !_rec_logits && emb_ln_fused()) {
       _phases.mark(1, _stream);
       while (_batch_seq_len < _batch_max_seq_len) {
@@ -491,8 +528,8 @@ int QuantGptEncoder::run_one_sample(int batch_size, int batch_seq_len) {
       _phases.mark(1, _stream);
       while (go_on && _batch_seq_len < _batch_max_seq_len) {
         ++loop_steps;
-        // the launches of a step depend on the batch size and the position only
-        const uint64_t key = ((uint64_t)_batch_size << 32) | (uint32_t)_batch_seq_len;
+        // the launches of a step depend on the batch size, the position and the run's route only
+        const uint64_t key = ((uint64_t)_batch_size << 32) | ((uint64_t)_out_run << 31) | (uint32_t)_batch_seq_len;
         _graphs.run(key, _stream, _use_graphs && !_rec_logits && !step_taps.any(), [&] {
           step_begin(StepNotice{});
           step_layers(0, L);

@@ -68,6 +68,7 @@ class QuantGptEncoder {
   void step_begin(lsh::StepNotice notice);
   bool emb_ln_fused() const;
   void step_layers(int from, int to);
+  bool out_run() const;
   void ffn_add_norm(int rows, int8_t* in, int8_t* tmp, bool blocked_out, const lsh::LnStep* ln_in,
                     lsh::LnStep* ln_out);
   void logits_product(const int8_t* hidden, int rows);
@@ -95,7 +96,7 @@ class QuantGptEncoder {
   HostNotice _notice, _rows_notice;
   struct {                       // the step being enqueued
     int8_t *a, *b;               // a: input, then output of a layer
-    bool qkv_attn, ln1_blocked, ln_in_product;
+    bool qkv_attn, ln1_blocked, ln_in_product, out_in_attention;
     lsh::LnStep ln_next;         // what the next layer's first product makes for itself
   } _step{};
   int8_t* _rec_logits = nullptr;
@@ -113,6 +114,8 @@ class QuantGptEncoder {
   DeviceBuffer<int8_t> _buf_a, _buf_b, _buf_q, _logits;
   DeviceBuffer<int8_t> _hid_last[2];  // row-major, and as the logits product reads it
   DeviceBuffer<int32_t> _int32_ffn_out_buf;
+  OutSumsRing _out_sums;
+  bool _out_run = false;  // this run's attention launches go through the out-projection while they can
   DeviceBuffer<int8_t> _self_k_cache, _self_v_cache;  // [n_layer][max_batch_dim]
   DeviceBuffer<int8_t> _int8_emb, _emb_blk;           // [vocab, H]; blocked, padded
   LayerProducts _ops;
