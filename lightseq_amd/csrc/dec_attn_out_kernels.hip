@@ -14,7 +14,7 @@ __global__ void __launch_bounds__(512)
 decself_out_kernel(const int8_t* __restrict__ q, const int8_t* __restrict__ k_cache,
                    const int8_t* __restrict__ v_cache, const int8_t* __restrict__ beam_from, int step_num,
                    int max_step, int head_num, int beam_stride, const int8_t* __restrict__ W, int32_t* acc,
-                   int32_t* next_acc, int rows, float attn_scale, float dq, float quant_scale) {
+                   int32_t* next_acc, int32_t* ffn_acc, int rows, float attn_scale, float dq, float quant_scale) {
   constexpr int D = 64, CH = D / 16, ATTEND = ROWS == 4 ? 4 : NWV;
   extern __shared__ __align__(16) float lds_f[];
   __shared__ __align__(16) int8_t ctx[ROWS * D];
@@ -48,11 +48,14 @@ decself_out_kernel(const int8_t* __restrict__ q, const int8_t* __restrict__ k_ca
     __syncthreads();
     __syncthreads();
   }
-  // the workgroup's share of the next launch's sums: its rows, 64 columns
+  // the workgroup's share of the next launch's sums and the feed-forward block's: its rows, 64 columns
   if (blockIdx.z == 0 && (int)threadIdx.x < ROWS * 16) {
     const int r = row0 + ((int)threadIdx.x >> 4);
-    if (r < rows)
-      *reinterpret_cast<int4*>(next_acc + (long)r * hidden + head * D + (threadIdx.x & 15) * 4) = make_int4(0, 0, 0, 0);
+    const long at = (long)r * hidden + head * D + (threadIdx.x & 15) * 4;
+    if (r < rows) {
+      *reinterpret_cast<int4*>(next_acc + at) = make_int4(0, 0, 0, 0);
+      *reinterpret_cast<int4*>(ffn_acc + at) = make_int4(0, 0, 0, 0);
+    }
   }
   __syncthreads();
   out.template add<ROWS>(ctx, acc + (long)row0 * hidden, rows - row0, hidden, first, lane);
@@ -68,25 +71,25 @@ bool decself_attention_out_supported(int rows, int head_num, int dim_per_head, i
 }
 
 int decself_attention_out_i8(const int8_t* q, const int8_t* k_cache, const int8_t* v_cache, const int8_t* W,
-                             int32_t* acc, int32_t* next_acc, int rows, int step_num, int max_step, int head_num,
-                             float attn_scale, float dequant_scale, float quant_scale, hipStream_t s,
+                             int32_t* acc, int32_t* next_acc, int32_t* ffn_acc, int rows, int step_num, int max_step,
+                             int head_num, float attn_scale, float dequant_scale, float quant_scale, hipStream_t s,
                              const CacheBeams* beams) {
-  if (!q || !k_cache || !v_cache || !W || !acc || !next_acc || acc == next_acc || step_num > max_step ||
+  if (!q || !k_cache || !v_cache || !W || !acc || !next_acc || !ffn_acc || acc == next_acc || acc == ffn_acc || step_num > max_step ||
       (beams && (!beams->from || beams->stride < max_step)))
     return lsh_fail(LSH_ERR_INVALID, "decself_attention_out: bad arguments");
   if (!decself_attention_out_supported(rows, head_num, 64, step_num) || rows > 65535 || max_step > 4096)
     return lsh_fail(LSH_ERR_UNSUPPORTED, "decself_attention_out: shape not covered");
   if (((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k_cache) |
         reinterpret_cast<uintptr_t>(v_cache) | reinterpret_cast<uintptr_t>(W) | reinterpret_cast<uintptr_t>(acc) |
-        reinterpret_cast<uintptr_t>(next_acc)) & 15u) != 0)
+        reinterpret_cast<uintptr_t>(next_acc) | reinterpret_cast<uintptr_t>(ffn_acc)) & 15u) != 0)
     return lsh_fail(LSH_ERR_INVALID, "decself_attention_out: operands must be 16-byte aligned");
   const CacheBeams by = beams ? *beams : CacheBeams{};
 #define LSH_OUT_RUN(NWV, UN, ROWS, N, BY)                                                                      \
   decself_out_kernel<NWV, UN, ROWS, N, BY>                                                                     \
       <<<dim3(head_num, (rows + ROWS - 1) / ROWS, 8 / N), 512,                                                  \
          ROWS * decself_group_floats<64, NWV>(step_num) * sizeof(float), s>>>(                                 \
-          q, k_cache, v_cache, by.from, step_num, max_step, head_num, by.stride, W, acc, next_acc, rows,       \
-          attn_scale, dequant_scale, quant_scale)
+          q, k_cache, v_cache, by.from, step_num, max_step, head_num, by.stride, W, acc, next_acc, ffn_acc,    \
+          rows, attn_scale, dequant_scale, quant_scale)
 #define LSH_OUT_BY(NWV, UN, ROWS, N) \
   do { if (beams) LSH_OUT_RUN(NWV, UN, ROWS, N, true); else LSH_OUT_RUN(NWV, UN, ROWS, N, false); } while (0)
 #define LSH_OUT(NWV, UN, ROWS)                                               \

@@ -731,7 +731,7 @@ encdec_attn_short_kernel(const __half* __restrict__ q, const __half* __restrict_
       const int8_t* wp = qp.W + code_offset((long)head * D + pw * 16 + m, kq * 16, qp.hidden, blocked);
       const int slice = blocked ? 1024 : 64;  // from one 64-byte slice of a row to the next
       const uint2 braw = *reinterpret_cast<const uint2*>(qp.bias + head * D + pw * 16 + 4 * kq);
-      LnStepRows<OUT ? 1 : 0, LN_ROWS ? LN_ROWS : 1> ln;
+      LnStepRows<OUT ? kLnRequant : 0, LN_ROWS ? LN_ROWS : 1> ln;
       if constexpr (LN_ROWS) {
         ln.load(qp.ln, (int)threadIdx.x - 256, b * beam_size, beam_size, qp.hidden);
         __builtin_amdgcn_sched_barrier(0);

@@ -129,9 +129,13 @@ enc_emb_packed_kernel(const int8_t* __restrict__ token_emb, const __half* __rest
                       const int* __restrict__ tokens, __half* __restrict__ output,
                       int* __restrict__ pad_mask, const int* __restrict__ seq,
                       int* __restrict__ row_map, int pad_id, int batch, int S, int hidden, float scale,
-                      int vocab) {
+                      int vocab, int32_t* clear) {
   const int dim = threadIdx.x * 8, pos = blockIdx.x, b = blockIdx.y;
   const long at = (long)b * S + pos;
+  if (clear != nullptr && dim < hidden) {
+    int4* p = reinterpret_cast<int4*>(clear + at * hidden + dim);
+    p[0] = p[1] = make_int4(0, 0, 0, 0);
+  }
   int token = tokens[at];
   const int start = seq[2 * b], len = seq[2 * b + 1], pad_row = seq[2 * batch];
   const bool pad = token == pad_id;
@@ -164,7 +168,8 @@ enc_emb_packed_kernel(const int8_t* __restrict__ token_emb, const __half* __rest
 
 int enc_emb_packed(const int8_t* token_emb, const __half* pos_emb, const int* tokens, __half* output,
                    int* pad_mask, int padding_id, const EncPack& pack, int batch, int seq_len,
-                   int hidden, hipStream_t s, float dequant_scale, bool scaled, int vocab_size) {
+                   int hidden, hipStream_t s, float dequant_scale, bool scaled, int vocab_size,
+                   int32_t* clear) {
   if (!token_emb || !pos_emb || !tokens || !output || !pad_mask || !pack.seq || !pack.row_map ||
       batch <= 0 || seq_len <= 0 || hidden <= 0 || hidden % 8 != 0 || hidden > 8192)
     return lsh_fail(LSH_ERR_INVALID, "enc_emb_packed: bad arguments");
@@ -174,7 +179,7 @@ int enc_emb_packed(const int8_t* token_emb, const __half* pos_emb, const int* to
   enc_emb_packed_kernel<<<dim3(seq_len, batch), threads, 0, s>>>(token_emb, pos_emb, tokens, output,
                                                                  pad_mask, pack.seq, pack.row_map,
                                                                  padding_id, batch, seq_len, hidden,
-                                                                 scale, vocab_size);
+                                                                 scale, vocab_size, clear);
   return lsh_check_launch("enc_emb_packed_kernel");
 }
 

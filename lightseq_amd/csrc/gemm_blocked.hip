@@ -101,9 +101,12 @@ template <typename Epi, bool FROM_FFN>
 int launch_ln_gemm(const LnStep& ln, const int8_t* W, Epi epi, int M, int N, int K, hipStream_t s) {
   if (FROM_FFN != (ln.planes != 0 && ln.requant == 0.f) || (ln.requant != 0.f && ln.planes != 1))
     return lsh_fail(LSH_ERR_UNSUPPORTED, "layer norm + product: operand not covered");
-  if constexpr (FROM_FFN) return launch_ln_planes<Epi, 4>(ln, W, epi, M, N, K, s);
-  else if (ln.planes) return launch_ln_planes<Epi, 1>(ln, W, epi, M, N, K, s);
-  else return launch_ln_planes<Epi, 0>(ln, W, epi, M, N, K, s);
+  if constexpr (FROM_FFN)
+    return ln.planes == 1 ? launch_ln_planes<Epi, 1>(ln, W, epi, M, N, K, s)
+                          : launch_ln_planes<Epi, 4>(ln, W, epi, M, N, K, s);
+  else
+    return ln.planes ? launch_ln_planes<Epi, kLnRequant>(ln, W, epi, M, N, K, s)
+                     : launch_ln_planes<Epi, 0>(ln, W, epi, M, N, K, s);
 }
 
 }  // namespace
@@ -129,6 +132,10 @@ int gemm_blk_i8o(const int8_t* A, const int8_t* W, int8_t* C, int M, int N, int 
 int gemm_blk_i32o(const int8_t* A, const int8_t* W, int32_t* C, int M, int N, int K, int ksplit,
                   hipStream_t s) {
   return dispatch_blk<KwI8, EpiI32, true>(A, W, EpiI32{C}, M, N, K, s, ksplit);
+}
+
+int gemm_blk_i32_add(const int8_t* A, const int8_t* W, int32_t* C, int M, int N, int K, int ksplit, hipStream_t s) {
+  return dispatch_blk<KwI8, EpiI32Add, false>(A, W, EpiI32Add{EpiI32{C}}, M, N, K, s, ksplit);
 }
 
 // Ranges of K (int32 planes, summed by the layer norm that reads them) for the few rows of a

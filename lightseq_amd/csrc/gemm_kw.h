@@ -24,6 +24,8 @@
 #pragma once
 #include "gemm_tile.h"
 
+#include <type_traits>
+
 namespace lsh {
 
 struct KwI8 {
@@ -51,6 +53,11 @@ struct KwF16 {
 // table of column n (kw_table_index says where a code is).
 // kBlockedOut: the output is a blocked int8 matrix; the lanes of a wavefront then take the 256
 // bytes that 16 rows of one 16-column chunk are.
+// kAddRanges (optional): the ranges of K add to the same elements instead of storing to planes.
+template <typename Epi, typename = void>
+constexpr bool kEpiAddsRanges = false;
+template <typename Epi>
+constexpr bool kEpiAddsRanges<Epi, std::void_t<decltype(Epi::kAddRanges)>> = Epi::kAddRanges;
 // bytes of LDS: partial sums (a 16 x 16 block padded to 68 16-byte cells, so that the lanes that
 // read neighbouring columns hit different banks) and the table rows
 template <typename Epi, int MB, int NB>
@@ -176,7 +183,7 @@ gemm_kw_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, int M
       const int cell = ((row >> 4) * NB + (quad >> 2)) * 68 + (quad & 3) * 17 + (row & 15);
       const Acc c = (red[cell] + red[MB * NB * 68 + cell]) +
                     (red[2 * MB * NB * 68 + cell] + red[3 * MB * NB * 68 + cell]);
-      const int mo = m + (int)blockIdx.y * M;
+      const int mo = kEpiAddsRanges<Epi> ? m : m + (int)blockIdx.y * M;
       if constexpr (Epi::kTable) fin.store4(mo, n, N, col, c, tab + 4 * quad * 256);
       else epi_store4(fin, mo, n, N, col, c, fetched[j]);
     }

@@ -60,6 +60,20 @@ struct EpiI32 {
   static const char* name() { return "EpiI32"; }
 };
 
+// int32 sums that start from zero and to which ranges of K add: exact in any order, and a reader has one
+// plane to fetch instead of four.  That counts where every workgroup of the next product makes the
+// layer norm (4 rows, us with planes and with sums: that product 5.2 and 4.5, this one, 4 x 1024 x 4096,
+// 2.8 and 3.0) and where planes were no choice (16 x 768 x 3072: 3.4 in one range, 3.0).  In front
+// of a layer norm of its own it costs more than it saves: 16 rows 3.3 and 3.5, 64 rows 3.7 and 5.3.
+struct EpiI32Add : EpiI32 {
+  static constexpr bool kAddRanges = true;
+  __device__ __forceinline__ void store4(int m, int n, int N, Col, const v4i& c) const {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      __hip_atomic_fetch_add(C + (long)m * N + n + i, c[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+};
+
 __device__ __forceinline__ void store16_i8(int8_t* p, int n, int N, const int (&q)[16], bool full) {
   if (full) {
     uint4 o;

@@ -127,23 +127,23 @@ ln_rows_kernel(const AccT* __restrict__ gemm_out, T* residual, T* out_t,
 // bytes.  A workgroup is one wavefront, so that rows spread over the compute units: measured
 // against four at 16 / 330 / 2540 / 7930 rows of 768 fp16 3.6 / 3.8 / 6.1 / 10.3 us to
 // 3.8 / 4.1 / 6.1 / 10.4 (before: 4.7 / 5.0 / 7.0 / 12.3).
-template <typename T, typename AccT, int MODE, int LPR, int ITER, bool FULL>
+template <typename T, typename AccT, int MODE, int LPR, int ITER, bool FULL, bool REQ>
 __global__ void __launch_bounds__(64)
 ln_rows8_kernel(const AccT* __restrict__ gemm_out, T* residual, const T* __restrict__ scale,
                 const T* __restrict__ bias, const T* __restrict__ residual_bias,
                 const T* __restrict__ colsum, int tokens, int hidden, T* out_t, int8_t* __restrict__ out_q,
                 float dequant_scale, float quant_scale, int is_post_ln, int nparts, long part_stride, int blocked,
-                const int* __restrict__ row_map) {
+                const int* __restrict__ row_map, float requant) {
   constexpr int RPW = kWave / LPR;
   const int lane = threadIdx.x;
   const int row = blockIdx.x * RPW + lane / LPR;
   int in_row = -1;
   if (MODE == kLnResOut && row_map != nullptr) in_row = row_map[min(row, tokens - 1)];
   // dead rows keep the shuffles convergent
-  ln_rows8_row<T, AccT, MODE, LPR, ITER, FULL>(row, row < tokens, lane % LPR, gemm_out, residual, out_t,
+  ln_rows8_row<T, AccT, MODE, LPR, ITER, FULL, REQ>(row, row < tokens, lane % LPR, gemm_out, residual, out_t,
                                          out_q, scale, bias, residual_bias, colsum, hidden,
                                          dequant_scale, quant_scale, is_post_ln, nparts,
-                                         part_stride, nullptr, 0, blocked, in_row);
+                                         part_stride, nullptr, 0, blocked, in_row, requant);
 }
 
 // ---------------------------------------------------------------------------------
@@ -371,7 +371,7 @@ ln_row_wg_finish(const float (&x)[4], bool on, int e, long base, const float (&g
 // permutes, and one barrier per reduction.
 // Order of a row sum: (x0 + x1) + (x2 + x3) per lane; lanes of a quad, the quads of a row of
 // 16 lanes and the four rows of a wavefront pairwise; the wavefronts in ascending order.
-template <typename T, typename AccT, int MODE>
+template <typename T, typename AccT, int MODE, bool REQ>
 __global__ void __launch_bounds__(256)
 ln_row_wg_kernel(const AccT* __restrict__ gemm_out, T* residual, const T* __restrict__ scale,
                  const T* __restrict__ bias, const T* __restrict__ residual_bias,
@@ -420,11 +420,11 @@ ln_row_wg_kernel(const AccT* __restrict__ gemm_out, T* residual, const T* __rest
         const int4 t = *reinterpret_cast<const int4*>(gemm_out + (long)p * part_stride + base + e);
         acc.x += t.x; acc.y += t.y; acc.z += t.z; acc.w += t.w;
       }
-      a[0] = (float)acc.x; a[1] = (float)acc.y; a[2] = (float)acc.z; a[3] = (float)acc.w;
-      if (requant != 0.f) {  // (uniform)
-        a[0] = (float)requant_acc_fast(acc.x, requant); a[1] = (float)requant_acc_fast(acc.y, requant);
-        a[2] = (float)requant_acc_fast(acc.z, requant); a[3] = (float)requant_acc_fast(acc.w, requant);
+      if constexpr (REQ) {
+        acc.x = requant_acc_fast(acc.x, requant); acc.y = requant_acc_fast(acc.y, requant);
+        acc.z = requant_acc_fast(acc.z, requant); acc.w = requant_acc_fast(acc.w, requant);
       }
+      a[0] = (float)acc.x; a[1] = (float)acc.y; a[2] = (float)acc.z; a[3] = (float)acc.w;
     } else {
       ld4_acc(gemm_out, base + e, a);
       pin4(g_raw, b_raw, rb_raw, c_raw);
@@ -654,20 +654,24 @@ static int launch_ln(const AccT* gemm_out, T* residual, T* out_t, int8_t* out_q,
   const int blk = blocked ? 1 : 0;
   if (vec_ok && hidden <= 1024 && g_ln_few_rows && !row_map) {
     const int tpr = ((hidden / 4 + 63) / 64) * 64;  // threads of a row: whole wavefronts
-    ln_row_wg_kernel<T, AccT, MODE><<<tokens, tpr, 0, stream>>>(
+    constexpr bool CAN_REQ = sizeof(AccT) == 4 && MODE == kLnResQuant;
+    const auto kernel = CAN_REQ && requant != 0.f ? ln_row_wg_kernel<T, AccT, MODE, CAN_REQ>
+                                                  : ln_row_wg_kernel<T, AccT, MODE, false>;
+    kernel<<<tokens, tpr, 0, stream>>>(
         gemm_out, residual, scale, bias, residual_bias, colsum, hidden, nparts, part_stride, out_t, out_q,
         dequant_scale, quant_scale, is_post_ln, blk, requant);
     return lsh_check_launch("ln_row_wg_kernel");
   }
-  if (requant != 0.f)
-    return lsh_fail(LSH_ERR_UNSUPPORTED, "layer norm: sums to requantise go to the row kernel");
   if (vec_ok && hidden % 8 == 0) {
     // LPR = 64 when the row fills whole 512-element steps, otherwise two rows per wavefront
-#define LSH_LN8_RUN(LPR, IT, FULL)                                                               \
-  ln_rows8_kernel<T, AccT, MODE, LPR, IT, FULL>                                                  \
+    constexpr bool CAN_REQ = sizeof(AccT) == 4 && MODE == kLnResQuant;
+#define LSH_LN8_REQ(LPR, IT, FULL, REQ)                                                          \
+  ln_rows8_kernel<T, AccT, MODE, LPR, IT, FULL, REQ>                                             \
       <<<(tokens + 64 / LPR - 1) / (64 / LPR), 64, 0, stream>>>(                                 \
           gemm_out, residual, scale, bias, residual_bias, colsum, tokens, hidden, out_t, out_q,  \
-          dequant_scale, quant_scale, is_post_ln, nparts, part_stride, blk, row_map)
+          dequant_scale, quant_scale, is_post_ln, nparts, part_stride, blk, row_map, requant)
+#define LSH_LN8_RUN(LPR, IT, FULL) \
+  do { if (CAN_REQ && requant != 0.f) LSH_LN8_REQ(LPR, IT, FULL, CAN_REQ); else LSH_LN8_REQ(LPR, IT, FULL, false); } while (0)
 #define LSH_LN8_CASE(LPR, IT) \
   do { if (hidden == LPR * 8 * IT) LSH_LN8_RUN(LPR, IT, true); else LSH_LN8_RUN(LPR, IT, false); } while (0)
     if (hidden <= 256) LSH_LN8_CASE(32, 1);
@@ -678,8 +682,11 @@ static int launch_ln(const AccT* gemm_out, T* residual, T* out_t, int8_t* out_q,
     else LSH_LN8_CASE(64, 4);
 #undef LSH_LN8_CASE
 #undef LSH_LN8_RUN
+#undef LSH_LN8_REQ
     return lsh_check_launch("ln_rows8_kernel");
   }
+  if (requant != 0.f)
+    return lsh_fail(LSH_ERR_UNSUPPORTED, "layer norm: sums to requantise need hidden % 8 == 0");
   if (nparts > 1)
     return lsh_fail(LSH_ERR_UNSUPPORTED, "layer norm: accumulator planes need hidden % 8 == 0");
   if (!vec_ok) {

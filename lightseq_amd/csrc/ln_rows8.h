@@ -160,18 +160,20 @@ __device__ __forceinline__ void zero8(Raw8H& r) { r.a = make_uint4(0, 0, 0, 0); 
 // `live` false for a row beyond the tensor (its lanes still take part in the shuffles).
 // gemm_out is read at gemm_out[row * hidden + column] and may point anywhere a flat load
 // reaches (the fused GEMM + LayerNorm kernel passes a tile staged in LDS).
-template <typename T, typename AccT, int MODE, int LPR, int ITER, bool FULL = false>
+template <typename T, typename AccT, int MODE, int LPR, int ITER, bool FULL = false, bool REQ = false>
 __device__ __forceinline__ void
 ln_rows8_row(int row, bool live, int sub, const AccT* __restrict__ gemm_out, T* residual, T* out_t,
              int8_t* __restrict__ out_q, const T* __restrict__ scale, const T* __restrict__ bias,
              const T* __restrict__ residual_bias, const T* __restrict__ colsum, int width,
              float dequant_scale, float quant_scale, int is_post_ln, int nparts, long part_stride,
-             const half8_t* pre_res = nullptr, int dead_row = 0, int blocked = 0, int in_row = -1) {
+             const half8_t* pre_res = nullptr, int dead_row = 0, int blocked = 0, int in_row = -1,
+             float requant = 0.f) {
   // pre_res (fp16 only): the lane's ITER residual chunks, already loaded by the caller.
   // dead_row: the row whose addresses a lane without a row reads (and drops); a caller that
   // hands over a staged tile names a row of the tile.
   // blocked: out_q is a blocked matrix.  in_row: the row of gemm_out and residual that row `row` of
   // out_t is made from, where that is another one (kLnResOut).
+  // REQ: int32 sums that become int8 codes of the scale `requant` first.
   // FULL: the row fills its lanes' chunks, width == LPR * 8 * ITER.
   constexpr int kWidth = LPR * 8 * ITER;
   const int hidden = FULL ? kWidth : width;
@@ -242,7 +244,7 @@ ln_rows8_row(int row, bool live, int sub, const AccT* __restrict__ gemm_out, T* 
             for (int k = 0; k < 8; ++k) acc[k] += more[k];
           }
 #pragma unroll
-          for (int k = 0; k < 8; ++k) a[k] = (float)acc[k];
+          for (int k = 0; k < 8; ++k) a[k] = (float)(REQ ? requant_acc_fast(acc[k], requant) : acc[k]);
         } else {
           cvt8(a_raw[it], a);
         }

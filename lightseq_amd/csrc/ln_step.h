@@ -16,15 +16,17 @@
 
 namespace lsh {
 
+constexpr int kLnRequant = -1;
+
 // ROWS rows (those from `rows` on repeat the last one and leave nothing) on 256 threads, hidden a
 // multiple of 256 up to 1024: 256 D, or not known at compile time (D = 0).  PLANES: 0 int8 codes,
-// 4 up to four int32 planes, 1 one plane of sums that are requantised first.
+// 1 one int32 plane, 4 up to four, kLnRequant one plane of sums that are requantised first (p.requant).
 template <int PLANES, int ROWS, int D = 0>
 struct LnStepRows {
-  static_assert(PLANES == 0 || PLANES == 1 || PLANES == 4, "codes, sums or planes");
   static constexpr bool I32 = PLANES != 0;
+  static constexpr int NP = PLANES == kLnRequant ? 1 : PLANES;
   Raw4H g, b, rb, cs, r[ROWS];
-  int4 m[ROWS][PLANES ? PLANES : 1];
+  int4 m[ROWS][I32 ? NP : 1];
   uint32_t w[ROWS];
 
   // requests everything; t: thread of the 256
@@ -42,7 +44,7 @@ struct LnStepRows {
       r[i] = ld4_raw(p.res_in, at);
       if constexpr (I32) {
 #pragma unroll
-        for (int u = 0; u < PLANES; ++u)
+        for (int u = 0; u < NP; ++u)
           m[i][u] = *reinterpret_cast<const int4*>(static_cast<const int32_t*>(p.acc) +
                                                    min(u, p.planes - 1) * p.plane_stride + at);
       } else {
@@ -92,17 +94,16 @@ struct LnStepRows {
       if constexpr (I32) {
         int4 acc = m[i][0];
 #pragma unroll
-        for (int u = 1; u < PLANES; ++u)
+        for (int u = 1; u < NP; ++u)
           if (u < p.planes) {
             acc.x += m[i][u].x; acc.y += m[i][u].y;
             acc.z += m[i][u].z; acc.w += m[i][u].w;
           }
-        if constexpr (PLANES == 1) {
-          a[0] = (float)requant_acc_fast(acc.x, p.requant); a[1] = (float)requant_acc_fast(acc.y, p.requant);
-          a[2] = (float)requant_acc_fast(acc.z, p.requant); a[3] = (float)requant_acc_fast(acc.w, p.requant);
-        } else {
-          a[0] = (float)acc.x; a[1] = (float)acc.y; a[2] = (float)acc.z; a[3] = (float)acc.w;
+        if constexpr (PLANES == kLnRequant) {
+          acc.x = requant_acc_fast(acc.x, p.requant); acc.y = requant_acc_fast(acc.y, p.requant);
+          acc.z = requant_acc_fast(acc.z, p.requant); acc.w = requant_acc_fast(acc.w, p.requant);
         }
+        a[0] = (float)acc.x; a[1] = (float)acc.y; a[2] = (float)acc.z; a[3] = (float)acc.w;
       } else {
 #pragma unroll
         for (int k = 0; k < 4; ++k) a[k] = (float)unpack_i8(w[i], k);

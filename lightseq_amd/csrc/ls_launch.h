@@ -95,7 +95,7 @@ int residual_bias_ln_i8O(const AccT* input, const T* scale, const T* bias, const
                          float dequant_scale, float quant_scale, hipStream_t stream,
                          bool is_post_ln, const T* colsum, int nparts = 1, long part_stride = 0,
                          bool blocked = false, float requant = 0.f);
-// (requant != 0: int32 sums that become the int8 codes of that scale first; row kernel only)
+// (requant != 0: int32 sums that become the int8 codes of that scale first; widths that are multiples of 8)
 // row_map (optional): row r of output is made from row row_map[r] of input and residual
 template <typename T>
 int residual_bias_ln_i32I(const int32_t* input, const T* scale, const T* bias, const T* residual,
@@ -205,9 +205,11 @@ int enc_pack_plan(const int* tokens, int padding_id, const EncPack& pack, int ba
 int text_pack_plan(const int* tokens, int padding_id, int* seq, int* real_len, float* ppl, int batch,
                    int seq_len, unsigned long long* host_rows, unsigned ticket, hipStream_t s);
 // launch_enc_emb_i8I into the rows of the plan; pad_mask keeps its [batch, seq_len] form
+// (clear: int32 [batch * seq_len, hidden] to start from zero, optional)
 int enc_emb_packed(const int8_t* token_emb, const __half* pos_emb, const int* tokens, __half* output,
                    int* pad_mask, int padding_id, const EncPack& pack, int batch, int seq_len,
-                   int hidden, hipStream_t s, float dequant_scale, bool scaled, int vocab_size);
+                   int hidden, hipStream_t s, float dequant_scale, bool scaled, int vocab_size,
+                   int32_t* clear = nullptr);
 // qkv_attention_i8 on packed rows with blocked x, qkv_weight and ctx_q
 int qkv_attention_packed(const int8_t* x, const int8_t* qkv_weight, const __half* qkv_bias,
                          const int* pad_mask, int8_t* ctx_q, float requant_alpha,
@@ -218,6 +220,15 @@ int encself_attention_packed(const int8_t* qkv, const __half* qkv_bias, float de
                              const int* pad_mask, int8_t* ctx_q, float quant_scale, int batch,
                              int seq_len, int head_num, int dim_per_head, hipStream_t s,
                              const EncPack& pack);
+
+// The same for a batch of few tokens, from row-major QKV codes through the out-projection (blocked W): int32
+// sums [rows, hidden] are added to acc, which starts from zero; `clear` is (clear_rows rows).
+// Heads of 64, at most 16 and an even number of them, at most kEncOutPositions positions in all.
+constexpr int kEncOutPositions = 96;
+bool enc_attention_out_supported(int batch, int seq_len, int head_num, int dim_per_head);
+int enc_attention_out(const int8_t* qkv, const __half* qkv_bias, float dequant_scale, const int* pad_mask,
+                      const int8_t* W, int32_t* acc, int32_t* clear, int clear_rows, float quant_scale, int batch,
+                      int seq_len, int head_num, hipStream_t s, const EncPack& pack);
 
 // The plan of such launches (batch * head_num ints, made once per padding mask): workgroups take
 // their (sequence, head) pairs longest sequence first, paired on a compute unit with the
@@ -301,6 +312,8 @@ int gemm_blk_i8o(const int8_t* A, const int8_t* W, int8_t* C, int M, int N, int 
 int gemm_blk_i32o(const int8_t* A, const int8_t* W, int32_t* C, int M, int N, int K, int ksplit,
                   hipStream_t s);
 int gemm_blk_preferred_ksplit(int M, int N, int K);
+// the ranges of K added to C, which starts from zero
+int gemm_blk_i32_add(const int8_t* A, const int8_t* W, int32_t* C, int M, int N, int K, int ksplit, hipStream_t s);
 
 // residual_bias_ln_i8O of a few rows, made by the product (or the cross-attention launch) that
 // reads its codes instead of a launch of its own (ln_step.h): the same codes and the same
@@ -417,13 +430,14 @@ int decself_attention_i8(const int8_t* q, const int8_t* k_cache, const int8_t* v
                          float quant_scale, hipStream_t s, bool blocked = false,
                          const CacheBeams* beams = nullptr);
 // The same attention with the out-projection that follows it: context codes times W (blocked [hidden,
-// hidden]) added to the int32 sums acc [rows, hidden], which start from zero; next_acc is cleared.
+// hidden]) added to the int32 sums acc [rows, hidden], which start from zero; next_acc is cleared, and so
+// are ffn_acc's sums, which the second feed-forward product behind adds to.
 // Heads of 64, at most 16 and an even number of them, caches of up to 1024 steps, as many (row,
 // head) pairs as one round of the chip takes.
 bool decself_attention_out_supported(int rows, int head_num, int dim_per_head, int step_num);
 int decself_attention_out_i8(const int8_t* q, const int8_t* k_cache, const int8_t* v_cache, const int8_t* W,
-                             int32_t* acc, int32_t* next_acc, int rows, int step_num, int max_step, int head_num,
-                             float attn_scale, float dequant_scale, float quant_scale, hipStream_t s,
+                             int32_t* acc, int32_t* next_acc, int32_t* ffn_acc, int rows, int step_num, int max_step,
+                             int head_num, float attn_scale, float dequant_scale, float quant_scale, hipStream_t s,
                              const CacheBeams* beams = nullptr);
 template <typename T>
 int arrange_encdec_q_i8I(int step_token_num, int hidden_size, hipStream_t s, const int8_t* ori_q,

@@ -440,7 +440,7 @@ inline DeviceBuffer<int8_t> block_weight_padded(const DeviceBuffer<int8_t>& w, i
 // graph replay needs.
 class OutSumsRing {
  public:
-  void alloc(size_t most) { _buf.alloc(3 * most); }
+  void alloc(size_t most) { _buf.alloc(4 * most); }
   void begin_run(size_t n, hipStream_t s) {
     _n = n;
     LSH_CALL(lsh::fill_i32(_buf.get(), 0, (int)(3 * n), s));
@@ -448,6 +448,8 @@ class OutSumsRing {
   void begin_step(int launches_before) { _turn = launches_before % 3; }
   int32_t* sums() const { return _buf.get() + (size_t)_turn * _n; }
   int32_t* next_sums() const { return _buf.get() + (size_t)((_turn + 1) % 3) * _n; }
+  // the second feed-forward product's, which every launch of a self attention clears
+  int32_t* ffn_sums() const { return _buf.get() + 3 * _n; }
   void launched() { _turn = (_turn + 1) % 3; }
 
  private:
@@ -480,6 +482,15 @@ struct LayerProducts {
            float alpha, hipStream_t s, const lsh::LnStep* ln = nullptr) const {
     LSH_CALL(blocked ? lsh::gemm_blk_lut(x, w, out, table, m, n, k, alpha, s, ln)
                      : lsh::gemm_i8_lut_i8o(x, w, out, table, m, n, k, alpha, s));
+  }
+  // the product as sums of `cleared` where splitting K pays (one plane in any case), else planes of `out`
+  int i32_sums(const int8_t* x, const int8_t* w, int32_t* out, int32_t* cleared, const int32_t** acc, int m,
+               int n, int k, int max_planes, hipStream_t s) const {
+    const int ranges = blocked && cleared ? lsh::gemm_blk_preferred_ksplit(m, n, k) : 1;
+    *acc = ranges > 1 ? cleared : out;
+    if (ranges <= 1) return i32o(x, w, out, m, n, k, max_planes, s);
+    LSH_CALL(lsh::gemm_blk_i32_add(x, w, cleared, m, n, k, ranges, s));
+    return 1;
   }
   // int32 accumulators in up to max_planes planes of [m, n]; returns their number
   int i32o(const int8_t* x, const int8_t* w, int32_t* out, int m, int n, int k, int max_planes,

@@ -58,6 +58,7 @@ void QuantBertEncoder::init_buffer() {
   // room for the accumulator planes of a split-K second FFN product (up to 4 at encoder
   // sizes, up to 8 for the few rows of a decode step)
   _int32_ffn_out_buf.alloc(std::max((size_t)tokens * H * 4, (size_t)64 * H * 8));
+  _out_sums.alloc(3 * (size_t)kEncOutPositions * H);
   _qa_plan.alloc((size_t)_max_batch_size * _tw._head_num);
   _seg_sync.alloc(ffn_segment_sync_words());
   CHECK_GPU_ERROR(hipMemsetAsync(_seg_sync.get(), 0, _seg_sync.size() * sizeof(unsigned), _stream));
@@ -244,17 +245,30 @@ int QuantBertEncoder::packed_rows(const int* host_token_ids) {
   return (int)(unsigned)*p;
 }
 
+// A batch of so few tokens that the fused launch of QKV product and attention waits for single compute
+// units to read the weights (enc_attn_out_kernels.hip); the same bytes.
+bool QuantBertEncoder::attention_out_route() const {
+  if (!enc_attention_out_supported(_batch_size, _batch_seq_len, _tw._head_num, _tw._dim_per_head)) return false;
+  for (int l = 0; l < _tw._n_enc_layer; ++l) {
+    const float* c = &_enc_clip_max[l * _tw._clip_stride];
+    if (c[1] * c[5] / (c[9] * _quant_range) == 0.f) return false;  // no code but zero: the layer norm's "none"
+  }
+  return true;
+}
+
 void QuantBertEncoder::run_packed(const int* host_token_ids) {
   const int H = _tw._hidden_size, I = _tw._inner_size, B = _batch_size, S = _batch_seq_len;
   const int h = _tw._head_num, dph = _tw._dim_per_head, post = _tw._is_post_ln;
   const float Q = _quant_range;
   const bool qkv_fused = qkv_attention_fused_supported(B, S, h, dph);
+  const bool out_fused = attention_out_route();
   const EncPack pack{_pack_seq.get(), _pack_map.get(), _qa_plan.get()};
   LSH_CALL(enc_pack_plan(_p_d_token_id, _tw._padding_id, pack, B, S, h,
                          host_token_ids ? nullptr : _h_pack_rows, ++_pack_ticket, _stream));
   LSH_CALL(enc_emb_packed(_int8_emb.get(), _pos_emb.get(), _p_d_token_id, _residual.get(),
                           _p_d_padding_mask, _tw._padding_id, pack, B, S, H, _stream,
-                          _src_emb_clip_max / Q, _tw._scale_embedding, _tw._src_vocab_size));
+                          _src_emb_clip_max / Q, _tw._scale_embedding, _tw._src_vocab_size,
+                          out_fused ? out_sums(0) : nullptr));
   int8_t *a = _int8_ffn_in_buf.get(), *b = _int8_ffn_out_buf.get();
   __half* res = _residual.get();
   // until the number of rows is known, launches cover the most there can be
@@ -274,7 +288,19 @@ void QuantBertEncoder::run_packed(const int* host_token_ids) {
     // QKV product and attention: one kernel per (sequence, head) for short sequences, else the
     // product's codes and an attention that dequantises them
     int8_t* ctx = b;
-    if (qkv_fused) {
+    const float out_alpha = c[1] * c[5] / (c[9] * Q);
+    const int32_t* sums = nullptr;
+    if (out_fused) {
+      // few tokens: the product over the whole chip, then attention and out-projection in one launch
+      int32_t* cur = out_sums(_layer_id);
+      prof_begin(0, M, 3 * H, H, "blocked");
+      LSH_CALL(gemm_blk_i8o(a, w.qkv_blk.get(), b, M, 3 * H, H, c[0] * c[4] / (c[8] * Q), _stream));
+      // (clears the next layer's sums and the feed-forward block's, which lie side by side)
+      LSH_CALL(enc_attention_out(b, w.b_qkv.get(), c[8] / Q, _p_d_padding_mask, w.out_blk.get(), cur,
+                                 std::min(out_sums(_layer_id + 1), ffn_sums()), 2 * B * S, Q / c[5], B, S, h,
+                                 _stream, pack));
+      sums = cur;
+    } else if (qkv_fused) {
       prof_begin(0, _batch_token_num, 3 * H, H, "fused_qkv_attn");
       LSH_CALL(qkv_attention_packed(a, w.qkv_blk.get(), w.b_qkv.get(), _p_d_padding_mask, ctx,
                                     c[0] * c[4] / (c[8] * Q), c[8] / Q, Q / c[5], B, S, h, dph, _stream,
@@ -288,28 +314,37 @@ void QuantBertEncoder::run_packed(const int* host_token_ids) {
                                         h, dph, _stream, pack));
     }
     // `a` holds the context
-    prof_begin(1, rows(), H, H, "blocked");
-    LSH_CALL(gemm_blk_i8o(a, w.out_blk.get(), b, M, H, H, c[1] * c[5] / (c[9] * Q), _stream));
-    LSH_CALL((residual_bias_ln_i8O<__half, int8_t>(b, w.ln2_scale.get(), w.ln2_bias.get(), w.b_ffn2.get(),
-                                                   a, res, M, H, c[9] / Q, Q / c[6], _stream, post, nullptr,
-                                                   1, 0, true)));
+    if (sums) {
+      LSH_CALL((residual_bias_ln_i8O<__half, int32_t>(sums, w.ln2_scale.get(), w.ln2_bias.get(),
+                                                      w.b_ffn2.get(), a, res, rows(), H, c[9] / Q, Q / c[6],
+                                                      _stream, post, nullptr, 1, 0, true, out_alpha)));
+    } else {
+      prof_begin(1, rows(), H, H, "blocked");
+      LSH_CALL(gemm_blk_i8o(a, w.out_blk.get(), b, M, H, H, out_alpha, _stream));
+      LSH_CALL((residual_bias_ln_i8O<__half, int8_t>(b, w.ln2_scale.get(), w.ln2_bias.get(), w.b_ffn2.get(),
+                                                     a, res, M, H, c[9] / Q, Q / c[6], _stream, post, nullptr,
+                                                     1, 0, true)));
+    }
     prof_begin(2, M, I, H, "blocked");
     LSH_CALL(gemm_blk_lut(a, w.ffn1_blk.get(), b, w.ffn1_act_lut.get(), M, I, H,
                           c[2] * c[6] / (c[10] * Q), _stream));
     prof_begin(3, M, H, I, "blocked");
-    LSH_CALL(gemm_blk_i32o(b, w.ffn2_blk.get(), _int32_ffn_out_buf.get(), M, H, I, 1, _stream));
+    const int ranges = sums && M <= 16 ? gemm_blk_preferred_ksplit(M, H, I) : 1;  // (see EpiI32Add)
+    const int32_t* ffn2 = ranges > 1 ? ffn_sums() : _int32_ffn_out_buf.get();
+    if (ranges > 1) LSH_CALL(gemm_blk_i32_add(b, w.ffn2_blk.get(), ffn_sums(), M, H, I, ranges, _stream));
+    else LSH_CALL(gemm_blk_i32o(b, w.ffn2_blk.get(), _int32_ffn_out_buf.get(), M, H, I, 1, _stream));
     const float dequant_scale = _tw._use_gelu ? c[3] * c[7] / (Q * Q) : c[3] * c[7] / (2 * Q * Q);
     const __half* colsum = w.ffn2_colsum.get();  // nullptr for GELU models
     if (_layer_id == _tw._n_enc_layer - 1) {
       // every position of the padded shape from the row it was computed in
-      LSH_CALL(residual_bias_ln_i32I<__half>(_int32_ffn_out_buf.get(), _final_ln_scale.get(),
+      LSH_CALL(residual_bias_ln_i32I<__half>(ffn2, _final_ln_scale.get(),
                                              _final_ln_bias.get(), res, _p_d_output, _batch_token_num, H,
                                              dequant_scale, _stream, colsum, 1, 0, pack.row_map));
     } else {
       const Layer& nx = _layers[_layer_id + 1];
       const float clip_next = _enc_clip_max[(_layer_id + 1) * _tw._clip_stride + 4];
       LSH_CALL((residual_bias_ln_i8O<__half, int32_t>(
-          _int32_ffn_out_buf.get(), nx.ln1_scale.get(), nx.ln1_bias.get(), nx.b_out.get(), a, res, M, H,
+          ffn2, nx.ln1_scale.get(), nx.ln1_bias.get(), nx.b_out.get(), a, res, M, H,
           dequant_scale, Q / clip_next, _stream, post, colsum, 1, 0, true)));
     }
   }

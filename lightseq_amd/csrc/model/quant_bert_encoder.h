@@ -76,6 +76,12 @@ class QuantBertEncoder {
   void self_attention();
   void ffn_add_norm();
   // the route of every call without taps: blocked operands, no rows for padding
+  bool attention_out_route() const;
+  // the sums of a layer's out-projection, two buffers that take turns, and between them those of its
+  // second feed-forward product: a layer's attention launch clears the other one and these
+  int32_t* out_sums(int layer) const { return _out_sums.get() + (layer & 1) * 2 * sums_size(); }
+  int32_t* ffn_sums() const { return _out_sums.get() + sums_size(); }
+  size_t sums_size() const { return (size_t)_batch_token_num * _tw._hidden_size; }
   bool packed_route() const;
   void set_batch(int batch_size, int batch_seq_len);
   void run_packed(const int* host_token_ids);
@@ -110,6 +116,7 @@ class QuantBertEncoder {
   // activations
   DeviceBuffer<__half> _qkv_buf;  // q | k | v, each max_batch_dim
   DeviceBuffer<int8_t> _int8_ffn_in_buf, _int8_ffn_out_buf;
+  DeviceBuffer<int32_t> _out_sums;
   DeviceBuffer<int32_t> _int32_ffn_out_buf;
   DeviceBuffer<int> _qa_plan;      // plan of the fused QKV + attention launches of a call
   const int* _qa_plan_cur = nullptr;  // ... when this call has one

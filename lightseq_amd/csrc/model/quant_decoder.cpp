@@ -514,7 +514,7 @@ void QuantDecoder::self_attention() {
     const CacheBeams beams{_beam_from[_alive_cur].get(), _beam_stride};
     if (_out_step)  // ... with the out-projection behind it; the layer norm requantises its sums
       LSH_CALL(decself_attention_out_i8(_buf_q.get(), k_cache, v_cache, w.w_self_out.get(), _out_sums.sums(),
-                                        _out_sums.next_sums(), M, _cur_step + 1, _tw._max_step, _tw._head_num,
+                                        _out_sums.next_sums(), _out_sums.ffn_sums(), M, _cur_step + 1, _tw._max_step, _tw._head_num,
                                         attn_scale, c[18] / Q, Q / c[7], _stream, _by_beam ? &beams : nullptr));
     else
       LSH_CALL(decself_attention_i8(_buf_q.get(), k_cache, v_cache, _buf_b.get(), M * _tw._head_num,
@@ -685,9 +685,11 @@ void QuantDecoder::ffn_add_norm() {
   TAP_CODES("ffn1_act_q", act, I);
   // a tapped accumulator is one plane (the planes of a split product sum to it exactly)
   const bool tap_acc = step_taps.wants(_layer_id, _cur_step, "ffn2_acc");
-  const int nparts = _ops.i32o(act, w.w_ffn2.get(), _int32_ffn_out_buf.get(), M, H, I,
-                               tap_acc ? 1 : 8, _stream);
-  TAP("ffn2_acc", _int32_ffn_out_buf.get(), (size_t)M * H * sizeof(int32_t));
+  const int32_t* acc;
+  const int nparts = _ops.i32_sums(act, w.w_ffn2.get(), _int32_ffn_out_buf.get(),
+                                   _out_step && _ln_in_product ? _out_sums.ffn_sums() : nullptr, &acc, M, H, I, tap_acc ? 1 : 8,
+                                   _stream);
+  TAP("ffn2_acc", acc, (size_t)M * H * sizeof(int32_t));
 
   const float dequant_scale =
       _tw._use_gelu ? c[5] * c[11] / (Q * Q) : c[5] * c[11] / (2 * Q * Q);
@@ -706,14 +708,14 @@ void QuantDecoder::ffn_add_norm() {
     clip_max = _dec_clip_max[(_layer_id + 1) * 19 + 6];
   }
   if (_ln_in_product && _layer_id != _tw._n_dec_layer - 1) {
-    _ln = LnStep{_int32_ffn_out_buf.get(), nparts, (long)M * H, _cur_step_query[_res].get(),
+    _ln = LnStep{acc, nparts, (long)M * H, _cur_step_query[_res].get(),
                  _cur_step_query[_res ^ 1].get(), scale_ptr, bias_ptr, res_bias_ptr,
                  w.ffn2_colsum.get(), dequant_scale, Q / clip_max, _tw._is_post_ln};
     _res ^= 1;
     return;
   }
   LSH_CALL((residual_bias_ln_i8O<__half, int32_t>(
-      _int32_ffn_out_buf.get(), scale_ptr, bias_ptr, res_bias_ptr, _buf_a.get(),
+      acc, scale_ptr, bias_ptr, res_bias_ptr, _buf_a.get(),
       _cur_step_query[_res].get(), M, H, dequant_scale, Q / clip_max, _stream, _tw._is_post_ln,
       w.ffn2_colsum.get(), nparts, (long)M * H,
       _ops.blocked && (!_qkv_attn || _layer_id == _tw._n_dec_layer - 1))));

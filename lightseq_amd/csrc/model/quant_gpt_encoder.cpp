@@ -136,7 +136,7 @@ void QuantGptEncoder::init_buffer() {
   step_taps.copy_codes(_layer_id, _tap_step, name, ptr, rows, cols, _ops.blocked, _stream)
 
 void QuantGptEncoder::ffn_add_norm(int rows, int8_t* in, int8_t* tmp, bool blocked_out,
-                                   const LnStep* ln_in, LnStep* ln_out) {
+                                   const LnStep* ln_in, LnStep* ln_out, int32_t* ffn_sums) {
   const int H = _tw._hidden_size, I = _tw._inner_size;
   const Layer& w = _layers[_layer_id];
   const float* c = &_enc_clip_max[_layer_id * 12];
@@ -146,9 +146,10 @@ void QuantGptEncoder::ffn_add_norm(int rows, int8_t* in, int8_t* tmp, bool block
   TAP_CODES("act_q", tmp, rows, I);
   // a tapped accumulator is one plane (the planes of a split product sum to it exactly)
   const bool tap_acc = step_taps.wants(_layer_id, _tap_step, "ffn2_acc");
-  const int nparts = _ops.i32o(tmp, w.w_ffn2.get(), _int32_ffn_out_buf.get(), rows, H, I,
-                               tap_acc ? 1 : rows <= 64 ? 8 : 4, _stream);
-  TAP("ffn2_acc", _int32_ffn_out_buf.get(), (size_t)rows * H * sizeof(int32_t));
+  const int32_t* acc;
+  const int nparts = _ops.i32_sums(tmp, w.w_ffn2.get(), _int32_ffn_out_buf.get(), ffn_sums, &acc, rows, H, I,
+                                   tap_acc ? 1 : rows <= 64 ? 8 : 4, _stream);
+  TAP("ffn2_acc", acc, (size_t)rows * H * sizeof(int32_t));
   const float dequant_scale = c[3] * c[7] / (Q * Q);
   const __half *scale_ptr, *bias_ptr, *res_bias_ptr;
   float clip_max;
@@ -165,14 +166,14 @@ void QuantGptEncoder::ffn_add_norm(int rows, int8_t* in, int8_t* tmp, bool block
     clip_max = _enc_clip_max[(_layer_id + 1) * 12 + 4];
   }
   if (ln_out && _layer_id != _tw._n_enc_layer - 1) {
-    *ln_out = LnStep{_int32_ffn_out_buf.get(), nparts, (long)rows * H, _query[_res].get(),
+    *ln_out = LnStep{acc, nparts, (long)rows * H, _query[_res].get(),
                      _query[_res ^ 1].get(), scale_ptr, bias_ptr, res_bias_ptr, nullptr, dequant_scale,
                      Q / clip_max, 0};
     _res ^= 1;
     return;
   }
   LSH_CALL((residual_bias_ln_i8O<__half, int32_t>(
-      _int32_ffn_out_buf.get(), scale_ptr, bias_ptr, res_bias_ptr, in, _query[_res].get(), rows, H,
+      acc, scale_ptr, bias_ptr, res_bias_ptr, in, _query[_res].get(), rows, H,
       dequant_scale, Q / clip_max, _stream, false, nullptr, nparts, (long)rows * H, blocked_out)));
   TAP_CODES("next_ln_q", in, rows, H);
   TAP("res_out", _query[_res].get(), (size_t)rows * H * sizeof(__half));
@@ -387,7 +388,7 @@ void QuantGptEncoder::step_layers(int from, int to) {
     if (out) {
       // the attention and the out-projection in one launch; the layer norm requantises its sums
       LSH_CALL(decself_attention_out_i8(_buf_q.get(), k_cache, v_cache, w.w_out.get(), _out_sums.sums(),
-                                        _out_sums.next_sums(), B, _batch_seq_len, _tw._max_step, _tw._head_num,
+                                        _out_sums.next_sums(), _out_sums.ffn_sums(), B, _batch_seq_len, _tw._max_step, _tw._head_num,
                                         _atten_scaler, c[11] / Q, Q / c[5], _stream));
       _out_sums.launched();
     } else {
@@ -400,7 +401,7 @@ void QuantGptEncoder::step_layers(int from, int to) {
                   w.ln2_bias.get(), w.b_ffn2.get(), nullptr, c[9] / Q, Q / c[6], 0};
       if (out) ln.acc = sums, ln.planes = 1, ln.requant = out_alpha;
       _res ^= 1;
-      ffn_add_norm(B, a, b, true, &ln, &ln_next);
+      ffn_add_norm(B, a, b, true, &ln, &ln_next, out ? _out_sums.ffn_sums() : nullptr);
       continue;
     }
     if (out)

@@ -70,7 +70,7 @@ class QuantGptEncoder {
   void step_layers(int from, int to);
   bool out_run() const;
   void ffn_add_norm(int rows, int8_t* in, int8_t* tmp, bool blocked_out, const lsh::LnStep* ln_in,
-                    lsh::LnStep* ln_out);
+                    lsh::LnStep* ln_out, int32_t* ffn_sums = nullptr);
   void logits_product(const int8_t* hidden, int rows);
   void enqueue_sampling(const int8_t* hidden, bool clear_flag);
   void count_token();

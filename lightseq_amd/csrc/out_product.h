@@ -72,6 +72,27 @@ struct OutFragments {
       }
     }
   }
+  // any number of rows, 16 at a time (those from `rows` on of the last 16 need not hold anything)
+  __device__ __forceinline__ void add_rows(const int8_t* ctx, int32_t* acc, int rows, int hidden, int first,
+                                           int lane) {
+    const int l16 = lane & 15, kq = lane >> 4;
+#pragma unroll
+    for (int f = 0; f < N; ++f) asm volatile("" : "+v"(w[f]));
+    for (int r0 = 0; r0 < rows; r0 += 16) {
+      const v4i a = *reinterpret_cast<const v4i*>(ctx + (r0 + l16) * 64 + kq * 16);
+#pragma unroll
+      for (int f = 0; f < N; ++f) {
+        // a lane holds column l16 of the block for rows 4 kq + 0 .. 3: an instruction adds to 64
+        // consecutive bytes of four rows
+        const v4i c = KwI8::mma(a, w[f], (v4i)0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if ((first + f) * 16 < hidden && r0 + 4 * kq + i < rows)
+            __hip_atomic_fetch_add(acc + (long)(r0 + 4 * kq + i) * hidden + (first + f) * 16 + l16, c[i],
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+  }
 };
 
 // how many workgroups share a head's columns where `groups` would hold all of them

@@ -89,3 +89,38 @@ def test_decoder_steps(tmp_path, batch, beam, hidden, seq, extra, gelu, post):
     ids, _ = synthetic.make_token_ids(dict(vocab=cfg["src_vocab"], padding_id=cfg["padding_id"]), batch,
                                       seq, seed=batch)
     _same("QuantTransformer", path, cfg, ids)
+
+
+# batches of few positions and beyond the limit: a workgroup's share of the columns (8 .. 1 blocks of 16 a wavefront),
+# one to three blocks of 32 tokens, sequences of nothing but padding, holes
+@pytest.mark.parametrize("hidden,lens,seq,holes", [
+    (128, [1], 1, []), (256, [17, 3], 17, []), (768, [16], 16, []), (768, [5], 40, []), (1024, [33, 0, 40], 40, [(0, 2)]),
+    (512, [64, 63], 64, [(1, 7)]), (768, [96], 96, []), (768, [97], 97, []), (1024, [128], 128, [(0, 64)]), (768, [0, 0], 20, []),
+    (768, [3, 9, 11, 2, 7] * 2, 12, []), (1024, [1, 2, 0, 4] * 8, 4, []), (384, [65], 70, []),
+])
+@pytest.mark.parametrize("post", [False, True])
+def test_encoder(tmp_path, hidden, lens, seq, holes, post):
+    from lightseq_amd import inference, synthetic
+    cfg = dict(synthetic.bert_config("tiny"), n_layer=3, hidden=hidden, inner=2 * hidden, head_num=hidden // 64,
+               vocab=300, max_step=128, is_post_ln=post)
+    path = os.path.join(str(tmp_path), "m.pb")
+    synthetic.write_quant_bert(path, cfg, seed=3)
+    ids = np.random.default_rng(seq).integers(1, cfg["vocab"], size=(len(lens), seq), dtype=np.int32)
+    ids[np.arange(seq)[None, :] >= np.asarray(lens)[:, None]] = cfg["padding_id"]
+    for b, s in holes:
+        ids[b, s] = cfg["padding_id"]
+    model = inference.QuantBert(path, len(lens))
+    try:
+        got = [model.infer_fp16(ids) for _ in range(2)]
+        d_ids = torch.from_numpy(ids).to(DEV)
+        model.set_input_ptr(0, d_ids.data_ptr())
+        model.set_input_shape(0, ids.shape)
+        model.infer_device()
+        got.append(model._download(0).cpu().numpy())
+        tap = torch.zeros(ids.size * hidden, dtype=torch.int8, device=DEV)
+        model.set_tap(0, "ctx_q", tap)  # the route with products of their own
+        want = model.infer_fp16(ids)
+        for g in got:
+            np.testing.assert_array_equal(g.view(np.uint16), want.view(np.uint16))
+    finally:
+        model.close()
