@@ -576,71 +576,143 @@ int sample_state_setup(void* state, int n, unsigned long long seed, hipStream_t 
   return lsh_check_launch("sample_state_setup_kernel");
 }
 
-// The 16 consecutive ids a thread reads per piece belong to 16 classes that do not change from
-// piece to piece (16 * 1024 is a multiple of 1024), so a thread reduces in registers and
-// touches LDS 16 times at the end.  f(e, v, c): slot e of the thread, id v, code c.
-template <typename F>
-__device__ __forceinline__ void sample_scan_row(const int8_t* __restrict__ lr, int vocab, F f) {
-  const int a = (int)(reinterpret_cast<uintptr_t>(lr) & 15u);
-  const int8_t* base = lr - a;
-  const int pieces = (vocab + a + 15) >> 4;
-  for (int p = threadIdx.x; p < pieces; p += kSampleThreads) {
-    const int v0 = p * 16 - a;
-    if (v0 >= 0 && v0 + 16 <= vocab) {
-      const uint4 w = *reinterpret_cast<const uint4*>(base + (long)p * 16);
-      const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+// The row as the threads read it: 16 consecutive ids a piece, four pieces of a thread in flight and,
+// up to 65536 ids, kept for the second pass.  They belong to 16 classes that do not change from
+// piece to piece (16 * 1024 is a multiple of 1024), the same ones for the threads of a lane in all
+// sixteen wavefronts.
+struct SampleRow {
+  static constexpr int kPieces = 4;
+  const int8_t* base;  // 16-byte aligned, `a` bytes before the row
+  int a, vocab, pieces;
+  uint32_t w[kPieces][4];
+
+  __device__ __forceinline__ SampleRow(const int8_t* __restrict__ lr, int vocab_)
+      : a((int)(reinterpret_cast<uintptr_t>(lr) & 15u)), vocab(vocab_) {
+    base = lr - a;
+    pieces = (vocab + a + 15) >> 4;
+  }
+  __device__ __forceinline__ int piece(int chunk, int i) const {
+    return (chunk * kPieces + i) * kSampleThreads + (int)threadIdx.x;
+  }
+  __device__ __forceinline__ int chunks() const {
+    return (pieces + kPieces * kSampleThreads - 1) / (kPieces * kSampleThreads);
+  }
+  // the pieces that lie in the row
+  __device__ __forceinline__ int whole0() const { return a ? 1 : 0; }
+  __device__ __forceinline__ int whole1() const { return (vocab + a) >> 4; }
+  // the first and the last piece where the row has a part of them: positions outside hold the lowest code
+  __device__ __forceinline__ void edges(uint4* lds) const {
+    const int t = threadIdx.x;
+    if (t >= 32) return;
+    const int v = (t < 16 ? 0 : (pieces - 1) * 16) - a + (t & 15);
+    reinterpret_cast<int8_t*>(lds)[t] = v >= 0 && v < vocab ? base[v + a] : (int8_t)-128;
+  }
+  __device__ __forceinline__ void load(int chunk) {
 #pragma unroll
-      for (int e = 0; e < 16; ++e) f(e, v0 + e, unpack_i8(ws[e >> 2], e & 3));
-    } else {
-#pragma unroll
-      for (int e = 0; e < 16; ++e)
-        if (v0 + e >= 0 && v0 + e < vocab) f(e, v0 + e, (int)lr[v0 + e]);
+    for (int i = 0; i < kPieces; ++i) {
+      const int p = piece(chunk, i);
+      uint4 v = make_uint4(0x80808080u, 0x80808080u, 0x80808080u, 0x80808080u);
+      if (p >= whole0() && p < whole1()) v = *reinterpret_cast<const uint4*>(base + (long)p * 16);
+      w[i][0] = v.x; w[i][1] = v.y; w[i][2] = v.z; w[i][3] = v.w;
     }
   }
+  // (behind a barrier behind edges())
+  __device__ __forceinline__ void patch(int chunk, const uint4* lds) {
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) {
+      const int p = piece(chunk, i);
+      if (p < pieces && (p < whole0() || p >= whole1())) {
+        const uint4 v = lds[p == 0 ? 0 : 1];
+        w[i][0] = v.x; w[i][1] = v.y; w[i][2] = v.z; w[i][3] = v.w;
+      }
+    }
+  }
+};
+
+typedef short short2v __attribute__((ext_vector_type(2)));
+// four int8 codes a word: the larger ones
+__device__ __forceinline__ uint32_t max4_i8(uint32_t x, uint32_t y) {
+  const short2v ox = __builtin_bit_cast(short2v, x & 0xff00ff00u), oy = __builtin_bit_cast(short2v, y & 0xff00ff00u);
+  const short2v ex = __builtin_bit_cast(short2v, (x << 8) & 0xff00ff00u),
+                ey = __builtin_bit_cast(short2v, (y << 8) & 0xff00ff00u);
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(ox, oy)) |
+         (__builtin_bit_cast(uint32_t, __builtin_elementwise_max(ex, ey)) >> 8);
+}
+template <int N>
+__device__ __forceinline__ int row_ror_max_i(int v) {
+  return max(v, __builtin_amdgcn_update_dpp(0, v, 0x120 + N, 0xf, 0xf, false));
+}
+// maximum of 32 lanes
+__device__ __forceinline__ int max32(int v) {
+  v = row_ror_max_i<8>(row_ror_max_i<4>(row_ror_max_i<2>(row_ror_max_i<1>(v))));
+  return max(v, __shfl_xor(v, 16, 64));
 }
 
 // One row; every thread returns the sampled id.  k > 1: top-k, k == 0: top-p with p.
-__device__ int sample_row(const int8_t* __restrict__ lr, int vocab, int k, float p, float scale,
+// One workgroup reads 50 KB at GPT-2's vocabulary and exchanges a few numbers, so what counts is the
+// chain: all loads of a thread at once, maxima of the wavefronts meet in LDS without atomics, thresholds by
+// permutations in every wavefront, the second pass from registers (top-k of 4: 14.9 -> 7.5 us).
+__device__ __forceinline__ int sample_row(const int8_t* __restrict__ lr, int vocab, int k, float p, float scale,
                           SampleState* st, SampleShared& sh) {
   const int t = threadIdx.x;
-  const int a = (int)(reinterpret_cast<uintptr_t>(lr) & 15u);
-  const int cls0 = (16 * t - a) & (kSampleThreads - 1);  // class of the thread's slot 0
-  sh.cls[t] = -129;
-  if (t < 260) sh.hist[t] = 0;
-  if (t == 0) sh.x = sample_draw_uniform(st);
-  __syncthreads();
-  {
-    int m[16];
+  SampleRow row(lr, vocab);
+  const int chunks = row.chunks();
+  uint32_t m[4] = {0x80808080u, 0x80808080u, 0x80808080u, 0x80808080u};  // maxima of the 16 slots
+  SampleState state{};
+  row.edges(sh.edge);
+  for (int c = 0; c < chunks; ++c) {
+    row.load(c);
+    if (c == 0) {
+      sh.cls[t] = 0;
+      if (t < 260) sh.hist[t] = 0;
+      if (t == kSampleThreads - 1) state = *st;
+      __syncthreads();
+    }
+    row.patch(c, sh.edge);
 #pragma unroll
-    for (int e = 0; e < 16; ++e) m[e] = -129;
-    sample_scan_row(lr, vocab, [&](int e, int, int c) { m[e] = max(m[e], c); });
+    for (int i = 0; i < SampleRow::kPieces; ++i)
 #pragma unroll
-    for (int e = 0; e < 16; ++e)
-      if (m[e] > -129) atomicMax(&sh.cls[(cls0 + e) & (kSampleThreads - 1)], m[e]);
+      for (int q = 0; q < 4; ++q) m[q] = max4_i8(m[q], row.w[i][q]);
+  }
+  sh.slots[t] = make_uint4(m[0], m[1], m[2], m[3]);
+  if (t == kSampleThreads - 1) {
+    sh.x = sample_uniform(state);
+    st->draws = state.draws + 1;
   }
   __syncthreads();
-  const int cm = sh.cls[t];
-  const int gmax = (int)block_max((float)cm, sh.red);
+  int cm = -128;
+  {
+    const int8_t* slot = reinterpret_cast<const int8_t*>(sh.slots) + ((t + row.a) & (kSampleThreads - 1));
+#pragma unroll
+    for (int w = 0; w < 16; ++w) cm = max(cm, (int)slot[w * 1024]);
+  }
+  if (t >= vocab) cm = -129;  // an empty class
+  {
+    const int g = max32(cm);
+    if ((t & 31) == 0) sh.group[t >> 5] = g;
+  }
+  __syncthreads();
+  const int gm = sh.group[t & 31];
+  const int gmax = max32(gm);
   const float mx = (float)gmax * scale;
+  int thr;
   if (k > 0) {
-    // rough k-th largest class maximum
-    if (t < 32) {
-      int w = sh.cls[32 * t];
-      for (int l = 1; l < 32; ++l) w = max(w, sh.cls[32 * t + l]);
-      sh.hist[t] = w;
-    }
-    __syncthreads();
-    if (t == 0) {
-      int best = 127;
-      for (int g = 0; g < k; ++g) {
-        int w = sh.hist[g];
-        for (int j = g + k; j < 32; j += k) w = max(w, sh.hist[j]);
-        best = min(best, w);
-      }
-      sh.thr = best;
-    }
+    // rough k-th largest class maximum: the smallest of the k largest of the groups that agree modulo k
+    thr = gm;
+    for (int d = 16; d >= k; d >>= 1) thr = max(thr, __shfl_xor(thr, d, 64));
+    for (int d = min(k, 32) >> 1; d > 0; d >>= 1) thr = min(thr, __shfl_xor(thr, d, 64));
   } else {
-    // classes per maximum code, exp of every code, then one thread walks the codes downwards
+    // classes per maximum code, exp of every code, then one thread walks the codes downwards, in the
+    // reference's order but sixteen reads at a time (a top-p step of 50257 ids 34.0 -> 18.3 us, with the rest)
+    constexpr int kWalk = 16;
+    auto codes_below = [&](int c0, int (&n)[kWalk], float (&e)[kWalk]) {  // c0, c0 - 1, ...; none below -128
+#pragma unroll
+      for (int i = 0; i < kWalk; ++i) {
+        const int at = max(c0 - i + 129, 0);
+        n[i] = sh.hist[at] & (at > 0 ? -1 : 0);  // (read in any case: no branches)
+        e[i] = sh.pf[at];
+      }
+    };
     atomicAdd(&sh.hist[cm + 129], 1);
     if (t < 257)
       sh.pf[t] = expf(fmaxf((float)(t - 129) * scale - mx, kLogitThreshMin));  // t = code + 129
@@ -648,41 +720,65 @@ __device__ int sample_row(const int8_t* __restrict__ lr, int vocab, int k, float
     if (t == 0) {
       // an empty class holds -inf in the reference: exp(-64) each
       float total = (float)sh.hist[0] * expf(kLogitThreshMin);
-      for (int c = gmax; c >= -128; --c) total += (float)sh.hist[c + 129] * sh.pf[c + 129];
+      for (int c0 = gmax; c0 >= -128; c0 -= kWalk) {
+        int n[kWalk];
+        float e[kWalk];
+        codes_below(c0, n, e);
+#pragma unroll
+        for (int i = 0; i < kWalk; ++i) total += (float)n[i] * e[i];
+      }
       const float limit = p * total;
       float pre = 0.f;
-      int thr = gmax;
-      for (int c = gmax; c >= -128; --c) {
-        const int n = sh.hist[c + 129];
-        if (n == 0) continue;
-        if (pre + sh.pf[c + 129] > limit) break;
-        thr = c;
-        pre += (float)n * sh.pf[c + 129];
+      int last = gmax;
+      bool inside = true;
+      for (int c0 = gmax; c0 >= -128 && inside; c0 -= kWalk) {
+        int n[kWalk];
+        float e[kWalk];
+        codes_below(c0, n, e);
+#pragma unroll
+        for (int i = 0; i < kWalk; ++i) {
+          const bool some = n[i] != 0;
+          inside &= !(some & (pre + e[i] > limit));
+          const float with = pre + (float)n[i] * e[i];
+          last = inside & some ? c0 - i : last;
+          pre = inside & some ? with : pre;
+        }
       }
-      sh.thr = thr;
+      sh.thr = last;
+    }
+    __syncthreads();
+    thr = sh.thr;
+  }
+  // candidate keys: (rank << 20) | (2^20 - 1 - id); 0 = none.  rank: 1 where the exp is clamped (all
+  // such ids tie: the first one wins), code + 130 else, where the first id of the largest code wins.
+  // sh.cls is [slot % 16][slot / 16] here, so that the lanes of an atomic hit different banks.
+  for (int ch = 0; ch < chunks; ++ch) {
+    if (chunks > 1) {
+      row.load(ch);
+      row.patch(ch, sh.edge);
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int top = unpack_i8(m[e >> 2], e & 3);
+      if (top < thr) continue;
+      const bool clamped = (float)top * scale - mx < kLogitThreshMin;
+      const int from = clamped ? thr : top;
+      int id = vocab;
+#pragma unroll
+      for (int i = SampleRow::kPieces - 1; i >= 0; --i) {
+        const int v = row.piece(ch, i) * 16 - row.a + e;
+        // (positions outside the row hold the lowest code)
+        const bool hit = (unpack_i8(row.w[i][e >> 2], e & 3) >= from) &
+                         ((from > -128) | ((unsigned)v < (unsigned)vocab));
+        id = hit ? v : id;
+      }
+      if (id < vocab)
+        atomicMax(&sh.cls[e * 64 + (t & 63)], ((clamped ? 1 : top + 130) << kSampleIdBits) | (kSampleIdMask - id));
     }
   }
   __syncthreads();
-  const int thr = sh.thr;
-  sh.cls[t] = 0;  // candidate keys: (rank << 20) | (2^20 - 1 - id); 0 = none
-  __syncthreads();
-  {
-    // rank: 1 where the exp is clamped (all such ids tie: the first one wins), code + 130 else
-    int key[16];
-#pragma unroll
-    for (int e = 0; e < 16; ++e) key[e] = 0;
-    sample_scan_row(lr, vocab, [&](int e, int v, int c) {
-      if (c >= thr) {
-        const bool clamped = (float)c * scale - mx < kLogitThreshMin;
-        key[e] = max(key[e], ((clamped ? 1 : c + 130) << kSampleIdBits) | (kSampleIdMask - v));
-      }
-    });
-#pragma unroll
-    for (int e = 0; e < 16; ++e)
-      if (key[e] != 0) atomicMax(&sh.cls[(cls0 + e) & (kSampleThreads - 1)], key[e]);
-  }
-  __syncthreads();
-  const int key = sh.cls[t];
+  const int slot = (t + row.a) & (kSampleThreads - 1);
+  const int key = sh.cls[(slot & 15) * 64 + (slot >> 4)];
   const int rank = key >> kSampleIdBits;
   const int my_id = key == 0 ? vocab : kSampleIdMask - (key & kSampleIdMask);
   const float ex = key == 0 ? 0.f

@@ -35,11 +35,14 @@ __device__ __forceinline__ uint32_t philox4x32_10_word0(uint32_t c0, uint32_t c1
 constexpr int kSampleThreads = 1024;
 constexpr int kSampleIdBits = 20, kSampleIdMask = (1 << kSampleIdBits) - 1;
 
-struct SampleShared {
-  int cls[kSampleThreads];   // class maxima (codes; -129 = empty), then candidate keys
+struct alignas(16) SampleShared {
+  int cls[kSampleThreads];   // class maxima of float logits, then candidate keys
+  uint4 slots[kSampleThreads];  // maxima of the threads' 16 slots (codes)
+  uint4 edge[2];             // pieces that the row has a part of
+  int group[32];             // maxima of 32 classes each
   float pf[kSampleThreads];  // exps (top-p), then wavefront prefix totals
   int hist[260];             // classes per maximum code (top-p)
-  float red[16];
+  alignas(16) float red[16];
   int thr, tok;
   float x;
 };
@@ -47,12 +50,44 @@ struct SampleShared {
 // The next uniform number in (0, 1] of one sequence (called by one thread): word 0 of
 // Philox4x32-10 with key = seed and counter = (draws, 0, row, 0), mapped as curand_uniform maps
 // 32 bits; advances the state.
-__device__ __forceinline__ float sample_draw_uniform(SampleState* st) {
-  const SampleState s = *st;
+__device__ __forceinline__ float sample_uniform(const SampleState& s) {
   const uint32_t w = philox4x32_10_word0(s.draws, 0u, s.row, 0u, (uint32_t)s.seed,
                                          (uint32_t)(s.seed >> 32));
-  st->draws = s.draws + 1;
   return (float)w * 2.3283064365386963e-10f + 1.1641532182693481e-10f;
+}
+__device__ __forceinline__ float sample_draw_uniform(SampleState* st) {
+  const SampleState s = *st;
+  st->draws = s.draws + 1;
+  return sample_uniform(s);
+}
+
+// block_sum and block_max of sixteen wavefronts: their sixteen values are read together instead of one
+// after the other, and added in the same order.
+__device__ __forceinline__ void sample_all(float v, float* red, float (&o)[16]) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  __syncthreads();  // protect `red` from a previous use
+  if (lane == 0) red[wid] = v;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float4 q = reinterpret_cast<const float4*>(red)[i];
+    o[4 * i] = q.x; o[4 * i + 1] = q.y; o[4 * i + 2] = q.z; o[4 * i + 3] = q.w;
+  }
+}
+__device__ __forceinline__ float sample_sum(float v, float* red) {
+  float o[16], r = 0.f;
+  sample_all(wave_sum(v), red, o);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) r += o[i];
+  return r;
+}
+__device__ __forceinline__ float sample_max(float v, float* red) {
+  float o[16];
+  sample_all(wave_max_dpp(v), red, o);
+  float r = o[0];
+#pragma unroll
+  for (int i = 1; i < 16; ++i) r = fmaxf(r, o[i]);
+  return r;
 }
 
 // Thread t holds at most one candidate: its exp `ex` (0 = none) and id `my_id`; sh.x holds the
@@ -60,7 +95,7 @@ __device__ __forceinline__ float sample_draw_uniform(SampleState* st) {
 // prefix reaches x (gptKernels_int8.cc.cu:347-395); every thread returns the chosen id.
 __device__ __forceinline__ int sample_pick(float ex, int my_id, SampleShared& sh) {
   const int t = threadIdx.x;
-  const float prob = ex / block_sum(ex, sh.red);
+  const float prob = ex / sample_sum(ex, sh.red);
   // inclusive prefix in thread order: within the wavefront, then the totals of the wavefronts before
   float pre = prob;
   const int lane = t & 63, wid = t >> 6;
@@ -72,13 +107,14 @@ __device__ __forceinline__ int sample_pick(float ex, int my_id, SampleShared& sh
   __syncthreads();
   if (lane == 63) sh.pf[wid] = pre;
   __syncthreads();
-  for (int w = 0; w < wid; ++w) pre += sh.pf[w];
+#pragma unroll
+  for (int w = 0; w < 16; ++w) pre = w < wid ? pre + sh.pf[w] : pre;
   const float x = sh.x;
-  int pick = kSampleThreads - (int)block_max((float)(x > pre ? 0 : kSampleThreads - t), sh.red);
+  int pick = kSampleThreads - (int)sample_max((float)(x > pre ? 0 : kSampleThreads - t), sh.red);
   if (pick == kSampleThreads) {
     // rounding left the last prefix below x: the lowest thread of the largest probability
-    const float pmax = block_max(prob, sh.red);
-    pick = kSampleThreads - (int)block_max((float)(prob == pmax ? kSampleThreads - t : 0), sh.red);
+    const float pmax = sample_max(prob, sh.red);
+    pick = kSampleThreads - (int)sample_max((float)(prob == pmax ? kSampleThreads - t : 0), sh.red);
   }
   if (t == pick) sh.tok = my_id;
   __syncthreads();
