@@ -7,6 +7,7 @@
 #include <hip/hip_ext.h>
 
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 
 namespace lsh {
@@ -160,7 +161,7 @@ int dispatch_blk(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K,
 // compute unit.
 struct SeqTile {
   int kind;  // 0: a wavefront per 16 x 16, 1: per 32 x 32; 2 - 4: LDS tiles 64 x 64, 128 x 64,
-             // 128 x 128; 5: the last with a third stage
+             // 128 x 128; 5: the last with a third stage; 6, 7: 256 x 192, 256 x 256
   float us;
 };
 inline SeqTile choose_seq(int M, int N, int K, int cus) {
@@ -183,6 +184,16 @@ inline SeqTile choose_seq(int M, int N, int K, int cus) {
     // 33.7 us instead of 39.9 (beyond that two tiles a unit are better: 8192 rows 52.0, not 65.8)
     if (tiles(128, 128) <= 1.f) take(5, lds(tiles(128, 128), 3.85f, 0.f));
     else take(4, lds(tiles(128, 128), 4.5f, 2.2f));
+    if (best.kind == 4) {
+      // Several rounds of the chip: the larger tiles where theirs come out even, priced in whole rounds
+      // (fits to the projections of keys and values, N = 6144 to 12288, M from 500 to 8000, to 5 %; us with
+      // 128 x 128 and now: 976 x 12288 x 2048 28.8 and 25.8, 1200 x 12288 x 2048 36.1 and 30.8, 4096 x 12288
+      // x 2048 103 and 95, 976 x 9216 x 1536 22.8 and 19.5).  3 % less at least, or the smaller tile stays.
+      auto rounds = [&](int tm, int tn) { return std::ceil(tiles(tm, tn)); };
+      const float small = 2.f + k + rounds(128, 128) * (1.65f + 3.22f * k);
+      const float wide = rounds(256, 192) * (6.2f + 9.2f * k), square = rounds(256, 256) * (8.9f + 10.4f * k);
+      if (std::min(wide, square) < 0.97f * small) best.kind = wide <= square ? 6 : 7;
+    }
   }
   return best;
 }
@@ -209,6 +220,8 @@ int dispatch_f16(const int8_t* A, const int8_t* W, Epi epi, int M, int N, int K,
     case 2: return launch_tile<KwF16, Epi, 2, 2, 1, 1, 3>(A, W, epi, M, N, K, s);
     case 3: return launch_tile<KwF16, Epi, 4, 1, 1, 2, 2>(A, W, epi, M, N, K, s);
     case 5: return launch_tile<KwF16, Epi, 2, 2, 2, 2, 3>(A, W, epi, M, N, K, s);
+    case 6: return launch_tile<KwF16, Epi, 4, 2, 2, 3, 2>(A, W, epi, M, N, K, s);
+    case 7: return launch_tile<KwF16, Epi, 2, 4, 4, 2, 2>(A, W, epi, M, N, K, s);
     default: return launch_tile<KwF16, Epi, 2, 2, 2, 2, 2>(A, W, epi, M, N, K, s);
   }
 }

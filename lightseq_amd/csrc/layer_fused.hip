@@ -16,9 +16,10 @@ namespace {
 // pass quantises the weights (2 bytes read and 1 written per parameter: 10 MB for a
 // Transformer-base layer).  As one launch per matrix that was 4 us each, six to nine times per
 // layer; the sections below -- weights, the input, the mask, the copy of a decoding step's caches
-// -- do not depend on one another, so they are ranges of workgroups of one grid: by the kernel
-// trace 8.0 us for a Transformer-base encoder layer (10 MB) and 18 us for a step of a
-// Transformer-big decoder layer (64 MB with its caches, 3.6 TB/s).
+// -- do not depend on one another, so they are ranges of workgroups of one grid (all of them, by the
+// kernel trace: 8.0 us for a Transformer-base encoder layer, 10 MB, and 18 us for a step of a
+// Transformer-big decoder layer, 64 MB with its caches, 3.6 TB/s).  Weights that only later products
+// read ride in the launches between (layer_prep.h); the rest takes 4.0 and 9.5 us.
 // eight normalised elements to where they go (`out`, `codes`: null where nobody reads them)
 __device__ __forceinline__ void ln_store(const half8_t& x, const half8_t& g, const half8_t& b, float mean, float rstd,
                                          const Quantiser& of, __half* out, int8_t* codes) {
