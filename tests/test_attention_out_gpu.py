@@ -19,7 +19,7 @@ def _run(kind, path, cfg, ids, tapped):
     model = getattr(inference, kind)(path, ids.shape[0])
     rows = ids.shape[0] * cfg.get("beam_size", 1)
     vocab = cfg.get("trg_vocab", cfg.get("vocab"))
-    most = cfg["extra_decode_length"] + 2 + (0 if kind == "QuantGpt" else ids.shape[1])
+    most = cfg["max_step"] if kind != "QuantGpt" else cfg["extra_decode_length"] + 2
     call = (lambda: (model.sample(ids),)) if kind == "QuantGpt" else (lambda: model.infer(ids))
     try:
         model.benchmark_mode(True)
@@ -46,12 +46,12 @@ def _run(kind, path, cfg, ids, tapped):
         model.close()
 
 
-def _same(kind, path, cfg, ids):
+def _same(kind, path, cfg, ids, first=None):
     want, want_logits = _run(kind, path, cfg, ids, True)
     got, got_logits = _run(kind, path, cfg, ids, False)
     np.testing.assert_array_equal(want_logits, got_logits)
     assert want_logits.any()
-    for run in got:
+    for run in got[:first]:
         for a, b in zip(want[0], run):
             np.testing.assert_array_equal(a, b)
 
@@ -89,6 +89,18 @@ def test_decoder_steps(tmp_path, batch, beam, hidden, seq, extra, gelu, post):
     ids, _ = synthetic.make_token_ids(dict(vocab=cfg["src_vocab"], padding_id=cfg["padding_id"]), batch,
                                       seq, seed=batch)
     _same("QuantTransformer", path, cfg, ids)
+
+
+@pytest.mark.parametrize("method", ["topk", "topp", "topk_greedy"])
+def test_decoder_steps_that_sample(tmp_path, method):
+    from lightseq_amd import synthetic
+    cfg = synthetic.transformer_config("tiny")
+    cfg.update(hidden=512, inner=256, head_num=8, sampling_method=method, topk=4, topp=0.8, beam_size=4,
+               max_step=64, extra_decode_length=20)
+    path = os.path.join(str(tmp_path), "qt.pb")
+    synthetic.write_quant_transformer(path, cfg, seed=6, w_std=0.2)
+    ids = np.random.default_rng(5).integers(4, cfg["src_vocab"], size=(3, 11), dtype=np.int32)
+    _same("QuantTransformer", path, cfg, ids, first=1)  # (later calls draw other numbers)
 
 
 # batches of few positions and beyond the limit: a workgroup's share of the columns (8 .. 1 blocks of 16 a wavefront),
