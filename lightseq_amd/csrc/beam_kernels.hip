@@ -715,32 +715,45 @@ beam_topk_reg_kernel(const int8_t* __restrict__ logits, long ldl, const T* __res
 // computes the row's maximum and sum of exponentials itself, from all of the row (the one-pass
 // sums of beam_topk_reg_kernel in another order; a separate statistics launch ahead of it cost
 // more than the repeated arithmetic), then the scores of its own part's ids and the part's
-// best beam_size by the same 64-bit keys.
+// best beam_size by the same order (score, then the lower id).
 // The merge then reads P * beam_size proposals per row instead of beam_size: a row's best
 // beam_size by (score, id) are among the union of its parts' best beam_size by (score, id), so
 // the beams chosen are the same.
+// thread t owns ids lo + 16 t .. + 15 of every part: 512 threads, one 16-byte piece each (two
+// wavefronts per SIMD take turns; with 32 ids per thread and one wavefront per SIMD every dependent
+// instruction waits out its latency and the kernel takes twice as long).  Pieces as raw words, so that all
+// of a thread's are requested before the first is converted; one beyond the row is the row's last.
 template <typename T>
-__device__ __forceinline__ void beam_part_load(const int8_t* __restrict__ lr,
-                                               const T* __restrict__ logit_bias, int lo, int hi,
-                                               float dq, float (&lg)[16]) {
+struct BeamPiece {
+  static constexpr int BW = 16 * sizeof(T) / 16;  // 16-byte words of bias
+  uint4 w, b[BW];
+  __device__ __forceinline__ void request(const int8_t* __restrict__ lr, const T* __restrict__ logit_bias, int v0) {
+    w = *reinterpret_cast<const uint4*>(lr + v0);
+#pragma unroll
+    for (int i = 0; i < BW; ++i) b[i] = *reinterpret_cast<const uint4*>(logit_bias + v0 + i * (16 / BW));
+  }
+  __device__ __forceinline__ void pin() {
+    asm volatile("" : "+v"(w.x), "+v"(w.y), "+v"(w.z), "+v"(w.w));
+#pragma unroll
+    for (int i = 0; i < BW; ++i) asm volatile("" : "+v"(b[i].x), "+v"(b[i].y), "+v"(b[i].z), "+v"(b[i].w));
+  }
+  __device__ __forceinline__ void logits(float dq, float (&lg)[16]) const {
 #pragma clang fp contract(off)
-  // thread t owns ids lo + 16 t .. + 15: 512 threads, one 16-byte piece each (two wavefronts
-  // per SIMD take turns; with 32 ids per thread and one wavefront per SIMD every dependent
-  // instruction waits out its latency and the kernel takes twice as long)
-  const int v0 = lo + 16 * (int)threadIdx.x;
-  if (v0 < hi) {
-    const uint4 w = *reinterpret_cast<const uint4*>(lr + v0);
-    float b[16];
-    ld4(logit_bias, v0, *reinterpret_cast<float(*)[4]>(b));
-    ld4(logit_bias, v0 + 4, *reinterpret_cast<float(*)[4]>(b + 4));
-    ld4(logit_bias, v0 + 8, *reinterpret_cast<float(*)[4]>(b + 8));
-    ld4(logit_bias, v0 + 12, *reinterpret_cast<float(*)[4]>(b + 12));
     const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+    T bias[16];
+    __builtin_memcpy(bias, b, sizeof(bias));
 #pragma unroll
-    for (int e = 0; e < 16; ++e) lg[e] = (float)unpack_i8(ws[e >> 2], e & 3) * dq + b[e];
-  } else {
+    for (int e = 0; e < 16; ++e) lg[e] = (float)unpack_i8(ws[e >> 2], e & 3) * dq + (float)bias[e];
+  }
+};
+// eight wavefronts' values, read together
+__device__ __forceinline__ void beam_part_all(float v, float* red, float (&o)[8]) {
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
 #pragma unroll
-    for (int e = 0; e < 16; ++e) lg[e] = 0.f;
+  for (int i = 0; i < 2; ++i) {
+    const float4 q = reinterpret_cast<const float4*>(red)[i];
+    o[4 * i] = q.x; o[4 * i + 1] = q.y; o[4 * i + 2] = q.z; o[4 * i + 3] = q.w;
   }
 }
 
@@ -756,14 +769,31 @@ beam_topk_part_kernel(const int8_t* __restrict__ logits, long ldl, const T* __re
 #pragma clang fp contract(off)
   // the merge that follows adds its finished beams to the count: it starts at zero
   if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *num_finished = 0;
-  __shared__ unsigned long long wbest[2][8];
-  __shared__ float red_max[16], red_sum[16];
+  __shared__ __align__(16) uint2 wbest[2][8];
+  __shared__ __align__(16) float red_max[8], red_sum[8];
   const int part = blockIdx.x, row = blockIdx.y, P = gridDim.x, t = threadIdx.x;
   const int lane = t & 63, wid = t >> 6;
   const int batch_id = row / beam_size, beam_id = row % beam_size;
   float* os = top_score + ((long)row * P + part) * beam_size;
   int* oi = top_idx + ((long)row * P + part) * beam_size;
-  if (cur_step != 0 && alive_seq[(long)row * max_step + cur_step] == end_id) {
+  const int lo = part * kBeamPartIds, hi = min(lo + kBeamPartIds, vocab);
+  // the row's maximum and sum of exponentials: every workgroup of the row reads all of it (the
+  // other parts' logits come from L2), so no workgroup waits for another.  One trip to memory: with a
+  // branch around each part's loads there were six.  32000 ids, us a launch of 4 and of 64 rows: 13.0 and
+  // 13.1, now 11.0 and 11.2, a third of it from the selection on 32-bit numbers below.
+  BeamPiece<T> piece[4], own;
+  const int8_t* lr = logits + row * ldl;
+#pragma unroll
+  for (int p = 0; p < 4; ++p) piece[p].request(lr, logit_bias, min(p * kBeamPartIds + 16 * t, vocab - 16));
+  own.request(lr, logit_bias, min(lo + 16 * t, vocab - 16));
+  int last = alive_seq[(long)row * max_step + cur_step];
+  float prob = seq_probs[row];
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int p = 0; p < 4; ++p) piece[p].pin();
+  own.pin();
+  asm volatile("" : "+v"(last), "+v"(prob));
+  if (cur_step != 0 && last == end_id) {
     // a finished beam proposes itself once (part 0, slot 0)
     if (t < beam_size) {
       const bool self = part == 0 && t == 0;
@@ -772,22 +802,19 @@ beam_topk_part_kernel(const int8_t* __restrict__ logits, long ldl, const T* __re
     }
     return;
   }
-  const int lo = part * kBeamPartIds, hi = min(lo + kBeamPartIds, vocab);
-  // the row's maximum and sum of exponentials: every workgroup of the row reads all of it (the
-  // other parts' logits come from L2), so no workgroup waits for another
   float all[4][16];
-#pragma unroll
-  for (int p = 0; p < 4; ++p)
-    beam_part_load(logits + row * ldl, logit_bias, p * kBeamPartIds,
-                   min((p + 1) * kBeamPartIds, vocab), dq, all[p]);
   float tmax = kFloatInfNeg;
 #pragma unroll
-  for (int p = 0; p < 4; ++p)
-    if (p * kBeamPartIds + 16 * t < vocab) {
+  for (int p = 0; p < 4; ++p) {
+    piece[p].logits(dq, all[p]);
+    // (a piece beyond the row repeats its last)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) tmax = fmaxf(tmax, all[p][i]);
-    }
-  const float max_logit = block_max_dpp(tmax, red_max);
+    for (int i = 0; i < 16; ++i) tmax = fmaxf(tmax, all[p][i]);
+  }
+  float of[8];
+  beam_part_all(wave_max_dpp(tmax), red_max, of);
+  const float max_logit = fmaxf(fmaxf(fmaxf(of[0], of[1]), fmaxf(of[2], of[3])),
+                                fmaxf(fmaxf(of[4], of[5]), fmaxf(of[6], of[7])));
   float se = 0.f;
 #pragma unroll
   for (int p = 0; p < 4; ++p)
@@ -795,62 +822,72 @@ beam_topk_part_kernel(const int8_t* __restrict__ logits, long ldl, const T* __re
 #pragma unroll
       for (int i = 0; i < 16; ++i) se += __expf(fmaxf(all[p][i] - max_logit, kLogitThreshMin));
     }
-  const float sum_exp = block_sum_dpp(se, red_sum);
+  beam_part_all(wave_sum_dpp(se), red_sum, of);
+  float sum_exp = of[0];
+#pragma unroll
+  for (int i = 1; i < 8; ++i) sum_exp += of[i];
+  const float base = prob - logf(sum_exp) - max_logit;
   float lg[16];
+  own.logits(dq, lg);
+  // The scores as numbers in their order (0: none; a thread's ids are all of the part or none).  Of equal
+  // ones the lowest id comes first: a thread's, a wavefront's and the workgroup's ids ascend, so the
+  // first of them is it, and no 64-bit key has to be compared.
+  const bool live = lo + 16 * t < hi;
+  unsigned order[16];
 #pragma unroll
-  for (int i = 0; i < 16; ++i)
-    lg[i] = part == 0 ? all[0][i] : part == 1 ? all[1][i] : part == 2 ? all[2][i] : all[3][i];
-  const float base = seq_probs[row] - logf(sum_exp) - max_logit;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) lg[i] = cand_score(lg[i], base, length_norm, batch_id);
-  auto id_of = [&](int i) { return lo + 16 * t + i; };
-  auto key_of = [&](int i) -> unsigned long long {
-    const int id = id_of(i);
-    if (id >= hi) return 0ull;
-    unsigned u = __builtin_bit_cast(unsigned, lg[i] + 0.f);  // -0 -> +0
+  for (int i = 0; i < 16; ++i) {
+    unsigned u = __builtin_bit_cast(unsigned, cand_score(lg[i], base, length_norm, batch_id) + 0.f);  // -0 -> +0
     u ^= (u >> 31) ? 0xffffffffu : 0x80000000u;
-    return ((unsigned long long)u << 32) | (unsigned)(0x7fffffff - id);
-  };
-  auto my_best_below = [&](unsigned long long bound) {
-    unsigned long long best = 0ull;
+    order[i] = live ? max(u, 1u) : 0u;
+  }
+  unsigned mine = 0u;
+  int my_i = 0;
+  auto find_mine = [&]() {
+    mine = order[0];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const unsigned long long c = key_of(i);
-      if (c < bound && c > best) best = c;
-    }
-    return best;
+    for (int i = 1; i < 16; ++i) mine = max(mine, order[i]);
+    my_i = 0;
+#pragma unroll
+    for (int i = 15; i >= 0; --i) my_i = order[i] == mine ? i : my_i;
   };
-  auto umax64 = [](unsigned long long a, unsigned long long b) { return a > b ? a : b; };
-  auto dpp64 = [](unsigned long long x, auto ctrl) {
-    const unsigned l = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)x, decltype(ctrl)::value, 0xf, 0xf, false);
-    const unsigned h = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(x >> 32), decltype(ctrl)::value, 0xf, 0xf, false);
-    return ((unsigned long long)h << 32) | l;
+  find_mine();
+  auto dpp = [](unsigned x, auto ctrl) {
+    return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, decltype(ctrl)::value, 0xf, 0xf, false);
   };
-  auto lane64 = [](unsigned long long x, int l) {
-    const unsigned lo32 = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)x, l);
-    const unsigned hi32 = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(x >> 32), l);
-    return ((unsigned long long)hi32 << 32) | lo32;
-  };
-  unsigned long long mine = my_best_below(~0ull);
   for (int k = 0; k < beam_size; ++k) {
-    unsigned long long best = mine;
-    best = umax64(best, dpp64(best, std::integral_constant<int, kDppXor1>()));
-    best = umax64(best, dpp64(best, std::integral_constant<int, kDppXor2>()));
-    best = umax64(best, dpp64(best, std::integral_constant<int, kDppHalfMirror>()));
-    best = umax64(best, dpp64(best, std::integral_constant<int, kDppMirror>()));
-    best = umax64(umax64(lane64(best, 0), lane64(best, 16)), umax64(lane64(best, 32), lane64(best, 48)));
-    unsigned long long* wb = wbest[k & 1];
-    if (lane == 0) wb[wid] = best;
+    unsigned m = mine;
+    m = max(m, dpp(m, std::integral_constant<int, kDppXor1>()));
+    m = max(m, dpp(m, std::integral_constant<int, kDppXor2>()));
+    m = max(m, dpp(m, std::integral_constant<int, kDppHalfMirror>()));
+    m = max(m, dpp(m, std::integral_constant<int, kDppMirror>()));
+    auto lane_u = [&](int l) { return (unsigned)__builtin_amdgcn_readlane((int)m, l); };
+    m = max(max(lane_u(0), lane_u(16)), max(lane_u(32), lane_u(48)));
+    const int first = __builtin_ctzll(__ballot(mine == m));
+    const int at = (wid * 64 + first) * 16 + __builtin_amdgcn_readlane(my_i, first);  // id within the part
+    uint2* wb = wbest[k & 1];
+    if (lane == 0) wb[wid] = make_uint2(m, (unsigned)at);
     __syncthreads();
-    best = umax64(umax64(umax64(wb[0], wb[1]), umax64(wb[2], wb[3])),
-                  umax64(umax64(wb[4], wb[5]), umax64(wb[6], wb[7])));
-    if (t == 0) {
-      unsigned u = (unsigned)(best >> 32);
-      u ^= (u >> 31) ? 0x80000000u : 0xffffffffu;
-      os[k] = best == 0ull ? -INFINITY : __builtin_bit_cast(float, u);
-      oi[k] = best == 0ull ? kNoCand : beam_id * vocab + (0x7fffffff - (int)(unsigned)best);
+    unsigned w_u[8], w_at[8];
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const uint4 q = reinterpret_cast<const uint4*>(wb)[w];
+      w_u[2 * w] = q.x; w_at[2 * w] = q.y; w_u[2 * w + 1] = q.z; w_at[2 * w + 1] = q.w;
     }
-    if (best == mine && best != 0ull) mine = my_best_below(best);
+    unsigned best = w_u[0], best_at = 0u;
+#pragma unroll
+    for (int w = 1; w < 8; ++w) best = max(best, w_u[w]);
+#pragma unroll
+    for (int w = 7; w >= 0; --w) best_at = w_u[w] == best ? w_at[w] : best_at;
+    if (t == 0) {
+      const unsigned u = best ^ ((best >> 31) ? 0x80000000u : 0xffffffffu);
+      os[k] = best == 0u ? -INFINITY : __builtin_bit_cast(float, u);
+      oi[k] = best == 0u ? kNoCand : beam_id * vocab + lo + (int)best_at;
+    }
+    if (best != 0u && best_at >> 4 == (unsigned)t) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) order[i] = (int)(best_at & 15u) == i ? 0u : order[i];
+      find_mine();
+    }
   }
 }
 
